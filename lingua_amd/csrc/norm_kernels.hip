@@ -16,7 +16,8 @@
 // order of the fp32 sum of squares, which differs from ATen's reduction, so y
 // can differ from the eager result in the last bf16 bit of an element now and
 // then (the tests bound it: at most one bf16 ulp, > 99.5 % identical).
-// One 256-thread workgroup per row, as the long-row cast kernel.
+// Two layouts, as in the row-wise casts: a wavefront per row for short rows, a
+// 256-thread workgroup per row for the longer ones.
 #include "l8_common.h"
 
 namespace l8 {
@@ -38,58 +39,185 @@ L8_DEV float wave_sum_f32(float v) {
   return (a + b) + (c + d);
 }
 
+// The weights of a lane's columns, kept in registers for all rows it sees: packed pairs as they are in memory (bf16),
+// or one register each (fp32).  Zero beyond column C.
+template <int N, bool W_F32>
+struct NormWeights {
+  uint32_t reg[N * (W_F32 ? 8 : 4)];
+  template <typename ColOf>
+  L8_DEV void load(const void *w, int C, ColOf col_of) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int c = col_of(j);
+#pragma unroll
+      for (int e = 0; e < (W_F32 ? 8 : 4); ++e) {
+        uint32_t v = 0;
+        // a bf16 weight may start at any even address: the copy states two-byte alignment
+        if (c < C) {
+          if (W_F32) v = ((const uint32_t *)w)[c + e];
+          else __builtin_memcpy(&v, (const uint16_t *)w + c + 2 * e, 4);
+        }
+        reg[j * (W_F32 ? 8 : 4) + e] = v;
+      }
+    }
+  }
+  L8_DEV float get(int j, int e) const {
+    if (W_F32) return __uint_as_float(reg[j * 8 + e]);
+    const uint32_t p = reg[j * 4 + (e >> 1)];
+    return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
+  }
+};
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// row r of x; zeros beyond column C and for a row at or beyond R (no branch around a load)
+template <int N, typename ColOf>
+L8_DEV void load_norm_row(v4i (&buf)[N], const uint16_t *x, int64_t r, int64_t R, int64_t ldx, int C, ColOf col_of) {
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(x + (r < R ? r : 0) * ldx, r < R ? (uint32_t)C * 2u : 0u);
+#pragma unroll
+  for (int j = 0; j < N; ++j) buf[j] = load16_nt(rs, (uint32_t)col_of(j) * 2u, 0);
+}
+L8_DEV void store16_nt(__amdgpu_buffer_rsrc_t rs, uint32_t voff, v4i data) {
+  __builtin_amdgcn_raw_buffer_store_b128(data, rs, (int)voff, 0, 2 /* non-temporal */);
+}
+L8_DEV void store8_nt(__amdgpu_buffer_rsrc_t rs, uint32_t voff, v2i data) {
+  __builtin_amdgcn_raw_buffer_store_b64(data, rs, (int)voff, 0, 2 /* non-temporal */);
+}
+#endif
+
+// Short rows (C <= NCH * 512): one wavefront owns a row, so neither the sum of squares nor the row amax crosses waves
+// and there is no barrier; the next row is requested before the current one is touched (loads through descriptors
+// without branches, as in the row-wise cast).  HBM-bound: 5 bytes per element.
+template <int NCH, bool COLMAX, bool W_F32>
+__global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_wave_kernel(
+    const uint16_t *__restrict__ x, const void *__restrict__ w, int64_t R, int C, int64_t ldx, float eps,
+    uint16_t *__restrict__ y, int64_t ldy, uint8_t *__restrict__ q, int64_t ldq, float *__restrict__ scale,
+    float *__restrict__ rstd, uint16_t *__restrict__ col_partials, int scale_rule) {
+#if defined(__HIP_DEVICE_COMPILE__)  // buffer descriptors exist in the device pass only
+  extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];  // [C] bf16 when COLMAX
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto col_of = [&](int j) { return j * 512 + lane * 8; };
+  uint32_t cmax[COLMAX ? NCH * 4 : 1];
+  if (COLMAX) {
+#pragma unroll
+    for (int i = 0; i < NCH * 4; ++i) cmax[i] = 0;
+  }
+  NormWeights<NCH, W_F32> wt;
+  wt.load(w, C, [&](int j) { return col_of(j); });
+  const float inv_c = 1.0f / (float)C;
+  const int64_t stride = (int64_t)gridDim.x * kNormWaves;
+  int64_t r = (int64_t)blockIdx.x * kNormWaves + wave;
+  v4i cur[NCH], nxt[NCH];
+  load_norm_row<NCH>(cur, x, r, R, ldx, C, [&](int j) { return col_of(j); });
+  while (r < R) {
+    const int64_t rn = r + stride;
+    load_norm_row<NCH>(nxt, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float lo = __uint_as_float((uint32_t)cur[j][k] << 16), hi = __uint_as_float((uint32_t)cur[j][k] & 0xffff0000u);
+        ss += lo * lo;
+        ss += hi * hi;
+      }
+    ss = wave_sum_f32(ss);
+    const float rinv = 1.0f / sqrtf(ss * inv_c + eps);
+    const __amdgpu_buffer_rsrc_t rsY = make_rsrc(y + r * ldy, (uint32_t)C * 2u);
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      v4i yv;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float lo = __uint_as_float((uint32_t)cur[j][k] << 16), hi = __uint_as_float((uint32_t)cur[j][k] & 0xffff0000u);
+        const uint32_t ylo = bf16_rne_bits((lo * rinv) * wt.get(j, 2 * k));
+        const uint32_t yhi = bf16_rne_bits((hi * rinv) * wt.get(j, 2 * k + 1));
+        yv[k] = (int)(ylo | (yhi << 16));
+        m = pk_absmax_u16(m, (uint32_t)yv[k]);
+        if (COLMAX) cmax[j * 4 + k] = pk_absmax_u16(cmax[j * 4 + k], (uint32_t)yv[k]);
+      }
+      store16_nt(rsY, (uint32_t)col_of(j) * 2u, yv);
+      cur[j] = yv;  // the row of y replaces the row of x in registers
+    }
+    const uint32_t amax_bits = wave_max_u32(max(m & 0xffffu, m >> 16));
+    const RowScale rs = row_scale(amax_bits, scale_rule);
+    if (lane == 0) {
+      if (rstd) rstd[r] = rinv;
+      if (scale) scale[r] = rs.s;
+    }
+    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(q ? q + r * ldq : nullptr, q ? (uint32_t)C : 0u);
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) store8_nt(rsQ, (uint32_t)col_of(j), cvt8(cur[j], rs.recip));
+    if (q && !rs.finite) {  // a non-finite amax: the bytes are redone from this lane's own y with the integer conversion
+      asm volatile("" ::: "memory");
+#pragma unroll 1
+      for (int c = lane * 8; c < C; c += 512) *(v2i *)(q + r * ldq + c) = cvt8_slow(*(const v4i *)(y + r * ldy + c), rs.recip);
+    }
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) cur[j] = nxt[j];
+    r = rn;
+  }
+  if (COLMAX) {  // the waves' column maxima meet in LDS, one wave after the other, and leave as this workgroup's row
+    v4i *lds4 = (v4i *)dyn_lds;
+    for (int wv = 0; wv < kNormWaves; ++wv) {
+      if (wave == wv) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j) {
+          const int c = col_of(j);
+          if (c < C) {
+            v4i mine = {(int)cmax[j * 4], (int)cmax[j * 4 + 1], (int)cmax[j * 4 + 2], (int)cmax[j * 4 + 3]};
+            if (wv > 0) {
+              const v4i old = lds4[c / 8];
+#pragma unroll
+              for (int k = 0; k < 4; ++k) mine[k] = (int)pk_absmax_u16((uint32_t)old[k], (uint32_t)mine[k]);
+            }
+            if (wv == kNormWaves - 1) *(v4i *)(col_partials + (int64_t)blockIdx.x * C + c) = mine;
+            else lds4[c / 8] = mine;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+#endif
+}
+
+// Longer rows: one workgroup per row (a wave-per-row kernel would need more than 256 registers), the next row requested
+// ahead of the two barriers of the current one.
 template <int NCHW, bool COLMAX, bool W_F32>
 __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_kernel(
     const uint16_t *__restrict__ x, const void *__restrict__ w, int64_t R, int C, int64_t ldx, float eps,
     uint16_t *__restrict__ y, int64_t ldy, uint8_t *__restrict__ q, int64_t ldq, float *__restrict__ scale,
     float *__restrict__ rstd, uint16_t *__restrict__ col_partials, int scale_rule) {
+#if defined(__HIP_DEVICE_COMPILE__)  // buffer descriptors exist in the device pass only
   __shared__ float red_ss[2][kNormWaves];
   __shared__ uint32_t red_mx[2][kNormWaves];
-  extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
-  constexpr bool CLDS = COLMAX && colmax_in_lds<NCHW, 1>();
-  v4i *lds_cm = (v4i *)dyn_lds;  // [C / 8]
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   auto col_of = [&](int j) { return (j * kNormWaves + wave) * 512 + lane * 8; };
-  uint32_t cmax[(COLMAX && !CLDS) ? NCHW * 4 : 1];
+  uint32_t cmax[COLMAX ? NCHW * 4 : 1];
   if (COLMAX) {
 #pragma unroll
-    for (int j = 0; j < NCHW; ++j) {
-      if (CLDS) {
-        if (col_of(j) < C) lds_cm[col_of(j) / 8] = v4i{0, 0, 0, 0};
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k) cmax[j * 4 + k] = 0;
-      }
-    }
+    for (int i = 0; i < NCHW * 4; ++i) cmax[i] = 0;
   }
-  // the weights of this thread's columns stay in registers for all its rows
-  float wf[NCHW][8];
-#pragma unroll
-  for (int j = 0; j < NCHW; ++j) {
-    const int c = col_of(j);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      if (c < C) wf[j][e] = W_F32 ? ((const float *)w)[c + e] : bf16_bits_to_f32(((const uint16_t *)w)[c + e]);
-      else wf[j][e] = 0.0f;
-    }
-  }
+  NormWeights<NCHW, W_F32> wt;  // of this thread's columns, in registers for all its rows
+  wt.load(w, C, [&](int j) { return col_of(j); });
   const float inv_c = 1.0f / (float)C;
+  v4i cur[NCHW], nxt[NCHW];
+  load_norm_row<NCHW>(cur, x, blockIdx.x, R, ldx, C, [&](int j) { return col_of(j); });
   int it = 0;
   for (int64_t r = blockIdx.x; r < R; r += gridDim.x, ++it) {
-    v4i xv[NCHW];
+    load_norm_row<NCHW>(nxt, x, r + gridDim.x, R, ldx, C, [&](int j) { return col_of(j); });
     float ss = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NCHW; ++j) {
-      const int c = col_of(j);
-      xv[j] = c < C ? __builtin_nontemporal_load((const v4i *)(x + r * ldx + c)) : v4i{0, 0, 0, 0};
+    for (int j = 0; j < NCHW; ++j)
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float lo = __uint_as_float((uint32_t)xv[j][k] << 16), hi = __uint_as_float((uint32_t)xv[j][k] & 0xffff0000u);
+        const float lo = __uint_as_float((uint32_t)cur[j][k] << 16), hi = __uint_as_float((uint32_t)cur[j][k] & 0xffff0000u);
         ss += lo * lo;
         ss += hi * hi;
       }
-    }
     ss = wave_sum_f32(ss);
     if (lane == 0) red_ss[it & 1][wave] = ss;
     __syncthreads();
@@ -99,28 +227,22 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_kernel(
     const float rinv = 1.0f / sqrtf(tot * inv_c + eps);
     if (threadIdx.x == 0 && rstd) rstd[r] = rinv;
 
+    const __amdgpu_buffer_rsrc_t rsY = make_rsrc(y + r * ldy, (uint32_t)C * 2u);
     uint32_t m = 0;
 #pragma unroll
     for (int j = 0; j < NCHW; ++j) {
       v4i yv;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float lo = __uint_as_float((uint32_t)xv[j][k] << 16), hi = __uint_as_float((uint32_t)xv[j][k] & 0xffff0000u);
-        const uint32_t ylo = bf16_rne_bits((lo * rinv) * wf[j][2 * k]);
-        const uint32_t yhi = bf16_rne_bits((hi * rinv) * wf[j][2 * k + 1]);
+        const float lo = __uint_as_float((uint32_t)cur[j][k] << 16), hi = __uint_as_float((uint32_t)cur[j][k] & 0xffff0000u);
+        const uint32_t ylo = bf16_rne_bits((lo * rinv) * wt.get(j, 2 * k));
+        const uint32_t yhi = bf16_rne_bits((hi * rinv) * wt.get(j, 2 * k + 1));
         yv[k] = (int)(ylo | (yhi << 16));
         m = pk_absmax_u16(m, (uint32_t)yv[k]);
-        if (COLMAX && !CLDS) cmax[j * 4 + k] = pk_absmax_u16(cmax[j * 4 + k], (uint32_t)yv[k]);
+        if (COLMAX) cmax[j * 4 + k] = pk_absmax_u16(cmax[j * 4 + k], (uint32_t)yv[k]);
       }
-      const int c = col_of(j);
-      if (CLDS && c < C) {
-        v4i old = lds_cm[c / 8];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) old[k] = (int)pk_absmax_u16((uint32_t)old[k], (uint32_t)yv[k]);
-        lds_cm[c / 8] = old;
-      }
-      if (c < C) __builtin_nontemporal_store(yv, (v4i *)(y + r * ldy + c));
-      xv[j] = yv;  // the row of y replaces the row of x in registers
+      store16_nt(rsY, (uint32_t)col_of(j) * 2u, yv);
+      cur[j] = yv;  // the row of y replaces the row of x in registers
     }
     m = wave_max_u32(max(m & 0xffffu, m >> 16));
     if (lane == 0) red_mx[it & 1][wave] = m;
@@ -130,17 +252,17 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_kernel(
     for (int wv = 0; wv < kNormWaves; ++wv) amax_bits = max(amax_bits, red_mx[it & 1][wv]);
     const RowScale rs = row_scale(amax_bits, scale_rule);
     if (threadIdx.x == 0 && scale) scale[r] = rs.s;
-    if (q) {
-      uint8_t *qrow = q + r * ldq;
+    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(q ? q + r * ldq : nullptr, q ? (uint32_t)C : 0u);
 #pragma unroll
-      for (int j = 0; j < NCHW; ++j) {
-        const int c = col_of(j);
-        if (c < C) {
-          if (rs.finite) __builtin_nontemporal_store(cvt8(xv[j], rs.recip), (v2i *)(qrow + c));
-          else *(v2i *)(qrow + c) = cvt8_slow(xv[j], rs.recip);
-        }
-      }
+    for (int j = 0; j < NCHW; ++j) store8_nt(rsQ, (uint32_t)col_of(j), cvt8(cur[j], rs.recip));
+    if (q && !rs.finite) {  // as in the kernel above: redone from this thread's own y
+      asm volatile("" ::: "memory");
+#pragma unroll 1
+      for (int c = threadIdx.x * 8; c < C; c += kNormBlock * 8)
+        *(v2i *)(q + r * ldq + c) = cvt8_slow(*(const v4i *)(y + r * ldy + c), rs.recip);
     }
+#pragma unroll
+    for (int j = 0; j < NCHW; ++j) cur[j] = nxt[j];
   }
   if (COLMAX) {
 #pragma unroll
@@ -148,9 +270,10 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_kernel(
       const int c = col_of(j);
       if (c < C)
         *(v4i *)(col_partials + (int64_t)blockIdx.x * C + c) =
-            CLDS ? lds_cm[c / 8] : v4i{(int)cmax[j * 4], (int)cmax[j * 4 + 1], (int)cmax[j * 4 + 2], (int)cmax[j * 4 + 3]};
+            v4i{(int)cmax[j * 4], (int)cmax[j * 4 + 1], (int)cmax[j * 4 + 2], (int)cmax[j * 4 + 3]};
     }
   }
+#endif
 }
 
 // Backward of the norm: with xhat = x * r and gh = gy * w,
@@ -165,49 +288,46 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
     const uint16_t *__restrict__ gy, const uint16_t *__restrict__ x, const void *__restrict__ w,
     const float *__restrict__ rstd, int64_t R, int C, int64_t ldg, int64_t ldx, uint16_t *__restrict__ gx, int64_t ldgx,
     float *__restrict__ gw_partials) {
+#if defined(__HIP_DEVICE_COMPILE__)
   __shared__ float red[2][kNormWaves];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   auto col_of = [&](int j) { return (j * kNormWaves + wave) * 512 + lane * 8; };
-  float wf[NCHW][8], gwacc[NCHW][8];
+  NormWeights<NCHW, W_F32> wt;
+  wt.load(w, C, [&](int j) { return col_of(j); });
+  float gwacc[NCHW][8];
 #pragma unroll
-  for (int j = 0; j < NCHW; ++j) {
-    const int c = col_of(j);
+  for (int j = 0; j < NCHW; ++j)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      gwacc[j][e] = 0.0f;
-      if (c < C) wf[j][e] = W_F32 ? ((const float *)w)[c + e] : bf16_bits_to_f32(((const uint16_t *)w)[c + e]);
-      else wf[j][e] = 0.0f;
-    }
-  }
+    for (int e = 0; e < 8; ++e) gwacc[j][e] = 0.0f;
   const float inv_c = 1.0f / (float)C;
+  v4i xc[NCHW], gc[NCHW], xn[NCHW], gn[NCHW];
+  float rinv = rstd[blockIdx.x];  // the grid is never larger than R
+  load_norm_row<NCHW>(xc, x, blockIdx.x, R, ldx, C, [&](int j) { return col_of(j); });
+  load_norm_row<NCHW>(gc, gy, blockIdx.x, R, ldg, C, [&](int j) { return col_of(j); });
   int it = 0;
   for (int64_t r = blockIdx.x; r < R; r += gridDim.x, ++it) {
-    const float rinv = rstd[r];
-    float xh[NCHW][8], gh[NCHW][8];
+    const int64_t rn = r + gridDim.x;
+    const float rinv_n = rstd[rn < R ? rn : r];
+    load_norm_row<NCHW>(xn, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
+    load_norm_row<NCHW>(gn, gy, rn, R, ldg, C, [&](int j) { return col_of(j); });
+    auto xhat = [&](int j, int e) {
+      const uint32_t p = (uint32_t)xc[j][e >> 1];
+      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16)) * rinv;
+    };
+    auto grad = [&](int j, int e) {
+      const uint32_t p = (uint32_t)gc[j][e >> 1];
+      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
+    };
     float dot = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NCHW; ++j) {
-      const int c = col_of(j);
-      v4i xv = {0, 0, 0, 0}, gv = {0, 0, 0, 0};
-      if (c < C) {
-        xv = __builtin_nontemporal_load((const v4i *)(x + r * ldx + c));
-        gv = __builtin_nontemporal_load((const v4i *)(gy + r * ldg + c));
-      }
+    for (int j = 0; j < NCHW; ++j)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-          const int e = 2 * k + half;
-          const float xe = __uint_as_float(half ? ((uint32_t)xv[k] & 0xffff0000u) : ((uint32_t)xv[k] << 16));
-          const float ge = __uint_as_float(half ? ((uint32_t)gv[k] & 0xffff0000u) : ((uint32_t)gv[k] << 16));
-          xh[j][e] = xe * rinv;
-          gh[j][e] = ge * wf[j][e];
-          gwacc[j][e] += ge * xh[j][e];
-          dot += gh[j][e] * xh[j][e];
-        }
+      for (int e = 0; e < 8; ++e) {
+        const float ge = grad(j, e), xh = xhat(j, e);
+        gwacc[j][e] += ge * xh;
+        dot += (ge * wt.get(j, e)) * xh;
       }
-    }
     dot = wave_sum_f32(dot);
     if (lane == 0) red[it & 1][wave] = dot;
     __syncthreads();
@@ -215,20 +335,24 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
 #pragma unroll
     for (int wv = 0; wv < kNormWaves; ++wv) tot += red[it & 1][wv];
     const float c1 = tot * inv_c;
+    const __amdgpu_buffer_rsrc_t rsG = make_rsrc(gx + r * ldgx, (uint32_t)C * 2u);
 #pragma unroll
     for (int j = 0; j < NCHW; ++j) {
-      const int c = col_of(j);
-      if (c < C) {
-        v4i out;
+      v4i out;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t lo = bf16_rne_bits((gh[j][2 * k] - xh[j][2 * k] * c1) * rinv);
-          const uint32_t hi = bf16_rne_bits((gh[j][2 * k + 1] - xh[j][2 * k + 1] * c1) * rinv);
-          out[k] = (int)(lo | (hi << 16));
-        }
-        __builtin_nontemporal_store(out, (v4i *)(gx + r * ldgx + c));
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t lo = bf16_rne_bits((grad(j, 2 * k) * wt.get(j, 2 * k) - xhat(j, 2 * k) * c1) * rinv);
+        const uint32_t hi = bf16_rne_bits((grad(j, 2 * k + 1) * wt.get(j, 2 * k + 1) - xhat(j, 2 * k + 1) * c1) * rinv);
+        out[k] = (int)(lo | (hi << 16));
       }
+      store16_nt(rsG, (uint32_t)col_of(j) * 2u, out);
     }
+#pragma unroll
+    for (int j = 0; j < NCHW; ++j) {
+      xc[j] = xn[j];
+      gc[j] = gn[j];
+    }
+    rinv = rinv_n;
   }
 #pragma unroll
   for (int j = 0; j < NCHW; ++j) {
@@ -239,25 +363,132 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
       *(v4f *)(dst + 4) = v4f{gwacc[j][4], gwacc[j][5], gwacc[j][6], gwacc[j][7]};
     }
   }
+#endif
 }
 
-// gw[c] = sum over the partial rows.  A workgroup owns 32 columns; thread (tx, ty)
-// adds slots ty, ty+8, ... of column tx, then the eight sums are added in order of ty.
-__global__ __launch_bounds__(256) void rmsnorm_gw_fold_kernel(const float *__restrict__ partials, int n_slots, int C,
-                                                              float *__restrict__ gw) {
-  __shared__ float part[8][32];
-  const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const int c = blockIdx.x * 32 + tx;
-  float s = 0.0f;
-  if (c < C)
-    for (int sl = ty; sl < n_slots; sl += 8) s += partials[(int64_t)sl * C + c];
-  part[ty][tx] = s;
-  __syncthreads();
-  if (ty == 0 && c < C) {
-    float t = part[0][tx];
+// Short rows: a wavefront per row, the next row's gy and x requested ahead; the row products for gw are accumulated per
+// lane over all rows of the wave and meet in LDS at the end, wave after wave (a fixed order).
+template <int NCH, bool W_F32>
+__global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_wave_kernel(
+    const uint16_t *__restrict__ gy, const uint16_t *__restrict__ x, const void *__restrict__ w,
+    const float *__restrict__ rstd, int64_t R, int C, int64_t ldg, int64_t ldx, uint16_t *__restrict__ gx, int64_t ldgx,
+    float *__restrict__ gw_partials) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];  // [C] floats
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  auto col_of = [&](int j) { return j * 512 + lane * 8; };
+  NormWeights<NCH, W_F32> wt;
+  wt.load(w, C, [&](int j) { return col_of(j); });
+  float gwacc[NCH][8];
 #pragma unroll
-    for (int k = 1; k < 8; ++k) t += part[k][tx];
-    gw[c] = t;
+  for (int j = 0; j < NCH; ++j)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) gwacc[j][e] = 0.0f;
+  const float inv_c = 1.0f / (float)C;
+  const int64_t stride = (int64_t)gridDim.x * kNormWaves;
+  int64_t r = (int64_t)blockIdx.x * kNormWaves + wave;
+  v4i xc[NCH], gc[NCH], xn[NCH], gn[NCH];
+  float rinv = r < R ? rstd[r] : 0.0f, rinv_n = 0.0f;
+  load_norm_row<NCH>(xc, x, r, R, ldx, C, [&](int j) { return col_of(j); });
+  load_norm_row<NCH>(gc, gy, r, R, ldg, C, [&](int j) { return col_of(j); });
+  while (r < R) {
+    const int64_t rn = r + stride;
+    rinv_n = rstd[rn < R ? rn : r];
+    load_norm_row<NCH>(xn, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
+    load_norm_row<NCH>(gn, gy, rn, R, ldg, C, [&](int j) { return col_of(j); });
+    auto xhat = [&](int j, int e) {
+      const uint32_t p = (uint32_t)xc[j][e >> 1];
+      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16)) * rinv;
+    };
+    auto grad = [&](int j, int e) {
+      const uint32_t p = (uint32_t)gc[j][e >> 1];
+      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
+    };
+    float dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float ge = grad(j, e), xh = xhat(j, e);
+        gwacc[j][e] += ge * xh;
+        dot += (ge * wt.get(j, e)) * xh;
+      }
+    const float c1 = wave_sum_f32(dot) * inv_c;
+    const __amdgpu_buffer_rsrc_t rsG = make_rsrc(gx + r * ldgx, (uint32_t)C * 2u);
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      v4i out;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t lo = bf16_rne_bits((grad(j, 2 * k) * wt.get(j, 2 * k) - xhat(j, 2 * k) * c1) * rinv);
+        const uint32_t hi = bf16_rne_bits((grad(j, 2 * k + 1) * wt.get(j, 2 * k + 1) - xhat(j, 2 * k + 1) * c1) * rinv);
+        out[k] = (int)(lo | (hi << 16));
+      }
+      store16_nt(rsG, (uint32_t)col_of(j) * 2u, out);
+    }
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      xc[j] = xn[j];
+      gc[j] = gn[j];
+    }
+    rinv = rinv_n;
+    r = rn;
+  }
+  v4f *lds4 = (v4f *)dyn_lds;
+  for (int wv = 0; wv < kNormWaves; ++wv) {
+    if (wave == wv) {
+#pragma unroll
+      for (int j = 0; j < NCH; ++j) {
+        const int c = col_of(j);
+        if (c < C) {
+#pragma unroll
+          for (int half = 0; half < 2; ++half) {
+            v4f mine = {gwacc[j][4 * half], gwacc[j][4 * half + 1], gwacc[j][4 * half + 2], gwacc[j][4 * half + 3]};
+            if (wv > 0) mine = lds4[c / 4 + half] + mine;
+            if (wv == kNormWaves - 1) *(v4f *)(gw_partials + (int64_t)blockIdx.x * C + c + 4 * half) = mine;
+            else lds4[c / 4 + half] = mine;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+#endif
+}
+
+// gw[c] = sum over the partial rows, in a fixed order.  A workgroup owns 32 columns -- one 128-byte line of every
+// partial row -- and its 1024 threads read 16 bytes each from 128 rows at a time, so that the few hundred rows are a
+// handful of loads per thread, all in flight together (with eight rows at a time the loads came one after the other:
+// 20 us for 512 rows of 2048 columns, now 4.8); the row groups then meet in LDS.
+constexpr int kGwCols = 32, kGwThreads = 1024, kGwGroups = kGwThreads / 8;
+__global__ __launch_bounds__(kGwThreads) void rmsnorm_gw_fold_kernel(const float *__restrict__ partials, int n_slots, int C,
+                                                                     float *__restrict__ gw) {
+  __shared__ v4f red[kGwGroups][8];
+  __shared__ float red2[8][kGwCols];
+  const int cc = threadIdx.x & 7, sg = threadIdx.x >> 3;
+  const int col = blockIdx.x * kGwCols + cc * 4;
+  v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (col < C) {
+#pragma unroll 4
+    for (int sl = sg; sl < n_slots; sl += kGwGroups) s += *(const v4f *)(partials + (int64_t)sl * C + col);
+  }
+  red[sg][cc] = s;
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int c = threadIdx.x & 31, part = threadIdx.x >> 5;
+    float t = 0.0f;
+#pragma unroll
+    for (int g = 0; g < kGwGroups / 8; ++g) t += reinterpret_cast<const float *>(&red[part * (kGwGroups / 8) + g][0])[c];
+    red2[part][c] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < kGwCols) {
+    float t = red2[0][threadIdx.x];
+#pragma unroll
+    for (int part = 1; part < 8; ++part) t += red2[part][threadIdx.x];
+    const int c = blockIdx.x * kGwCols + threadIdx.x;
+    if (c < C) gw[c] = t;
   }
 }
 
@@ -268,35 +499,48 @@ static int64_t norm_blocks(int64_t R) {
 
 constexpr int64_t kNormMaxC = 4 * kNormWaves * 512;  // 8192: the weights of a thread's columns live in registers
 
-template <int NCHW, bool W_F32>
+// Which layout: a wavefront per row up to 2048 columns, a workgroup per row beyond (up to 8192), where a wave's row,
+// the row requested ahead, the weights and the column maxima or gw sums no longer fit 256 registers.  Inside a 1B-sized
+// step, [16384,2048], us: forward 59 (a workgroup per row, each row requested when its turn comes) -> 49 (next row
+// requested ahead) -> 34 (a wavefront per row: 168 MB at 4.9 TB/s); backward 45 -> 37 -> 35 (201 MB at 5.7 TB/s); the
+// fold of gw 20 -> 4.8.  [4093,4096], workgroup per row with the next row ahead: forward 25.5 -> 20.5, backward
+// 23.8 -> 20.5, fold 17.6 -> 4.9.  Four workgroups per compute unit instead of two: forward +-4 %, backward 7 % slower.
+// workgroups of the wavefront-per-row kernels (never more than norm_blocks(R), which the workspaces are sized for)
+static int64_t norm_wave_blocks(int64_t R) { return norm_blocks((R + kNormWaves - 1) / kNormWaves); }
+
+// N = chunks of 512 columns per wave (WAVE) or of 2048 per workgroup
+template <bool WAVE, int N, bool W_F32>
 static int launch_norm(const void *x, const void *w, int64_t R, int64_t C, int64_t ldx, float eps, void *y, int64_t ldy,
                        void *q, int64_t ldq, float *scale, float *rstd, float *col_amax, void *ws, hipStream_t st) {
-  const int64_t blocks = norm_blocks(R);
-  if (col_amax) {
-    const size_t lds = colmax_in_lds<NCHW, 1>() ? (size_t)C * 2 : 0;
-    hipLaunchKernelGGL((rmsnorm_cast_rowwise_kernel<NCHW, true, W_F32>), dim3((unsigned)blocks), dim3(kNormBlock), lds, st,
-                       (const uint16_t *)x, w, R, (int)C, ldx, eps, (uint16_t *)y, ldy, (uint8_t *)q, ldq, scale, rstd,
-                       (uint16_t *)ws, l8::scale_rule());
-    L8_HIP(hipGetLastError());
-    return fold_colmax(ws, blocks, C, col_amax, st);
+  const int64_t blocks = WAVE ? norm_wave_blocks(R) : norm_blocks(R);
+  auto go = [&](auto kernel, size_t lds) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kNormBlock), lds, st, (const uint16_t *)x, w, R, (int)C, ldx, eps,
+                       (uint16_t *)y, ldy, (uint8_t *)q, ldq, scale, rstd, (uint16_t *)ws, l8::scale_rule());
+  };
+  if constexpr (WAVE) {
+    if (col_amax) go(rmsnorm_cast_rowwise_wave_kernel<N, true, W_F32>, (size_t)C * 2);
+    else go(rmsnorm_cast_rowwise_wave_kernel<N, false, W_F32>, 0);
+  } else {
+    if (col_amax) go(rmsnorm_cast_rowwise_kernel<N, true, W_F32>, 0);
+    else go(rmsnorm_cast_rowwise_kernel<N, false, W_F32>, 0);
   }
-  hipLaunchKernelGGL((rmsnorm_cast_rowwise_kernel<NCHW, false, W_F32>), dim3((unsigned)blocks), dim3(kNormBlock), 0, st,
-                     (const uint16_t *)x, w, R, (int)C, ldx, eps, (uint16_t *)y, ldy, (uint8_t *)q, ldq, scale, rstd,
-                     (uint16_t *)nullptr, l8::scale_rule());
   L8_HIP(hipGetLastError());
-  return L8_OK;
+  return col_amax ? fold_colmax(ws, blocks, C, col_amax, st) : L8_OK;
 }
 
-template <int NCHW, bool W_F32>
+template <bool WAVE, int N, bool W_F32>
 static int launch_norm_bwd(const void *gy, const void *x, const void *w, const float *rstd, int64_t R, int64_t C,
                            int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, float *gw, void *ws, hipStream_t st) {
-  const int64_t blocks = norm_blocks(R);
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<NCHW, W_F32>), dim3((unsigned)blocks), dim3(kNormBlock), 0, st,
-                     (const uint16_t *)gy, (const uint16_t *)x, w, rstd, R, (int)C, ldg, ldx, (uint16_t *)gx, ldgx,
-                     (float *)ws);
+  const int64_t blocks = WAVE ? norm_wave_blocks(R) : norm_blocks(R);
+  auto go = [&](auto kernel, size_t lds) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kNormBlock), lds, st, (const uint16_t *)gy, (const uint16_t *)x, w,
+                       rstd, R, (int)C, ldg, ldx, (uint16_t *)gx, ldgx, (float *)ws);
+  };
+  if constexpr (WAVE) go(rmsnorm_bwd_wave_kernel<N, W_F32>, (size_t)C * 4);
+  else go(rmsnorm_bwd_kernel<N, W_F32>, 0);
   L8_HIP(hipGetLastError());
-  hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + 31) / 32)), dim3(256), 0, st, (const float *)ws,
-                     (int)blocks, (int)C, gw);
+  hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + kGwCols - 1) / kGwCols)), dim3(kGwThreads), 0, st,
+                     (const float *)ws, (int)blocks, (int)C, gw);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
@@ -317,7 +561,7 @@ extern "C" int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int 
   if (C == 0) return L8_OK;
   L8_REQUIRE(gw, "l8_rmsnorm_bwd: null pointer");
   if (R == 0) {  // no rows: gw = 0, written by the fold kernel over zero partial rows
-    hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + 31) / 32)), dim3(256), 0, (hipStream_t)stream,
+    hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + kGwCols - 1) / kGwCols)), dim3(kGwThreads), 0, (hipStream_t)stream,
                        (const float *)nullptr, 0, (int)C, gw);
     L8_HIP(hipGetLastError());
     return L8_OK;
@@ -332,13 +576,13 @@ extern "C" int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int 
   L8_REQUIRE(workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0,
              "l8_rmsnorm_bwd: needs a 16-byte aligned workspace of %lld bytes", (long long)need);
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nchw = ((C + 511) / 512 + kNormWaves - 1) / kNormWaves;
-#define L8_NORM_BWD(N)                                                                                               \
-  return w_is_f32 ? launch_norm_bwd<N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)             \
-                  : launch_norm_bwd<N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)
-  if (nchw <= 1) L8_NORM_BWD(1);
-  if (nchw <= 2) L8_NORM_BWD(2);
-  L8_NORM_BWD(4);
+#define L8_NORM_BWD(WAVE, N)                                                                                              \
+  return w_is_f32 ? launch_norm_bwd<WAVE, N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)            \
+                  : launch_norm_bwd<WAVE, N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)
+  const int64_t nch = (C + 511) / 512, nchw = (nch + kNormWaves - 1) / kNormWaves;
+  if (nch <= 4) L8_NORM_BWD(true, 4);
+  if (nchw <= 2) L8_NORM_BWD(false, 2);
+  L8_NORM_BWD(false, 4);
 #undef L8_NORM_BWD
 }
 
@@ -366,12 +610,12 @@ extern "C" int l8_rmsnorm_cast_rowwise(const void *x, const void *w, int w_is_f3
                "l8_rmsnorm_cast_rowwise: col_amax needs a 16-byte aligned workspace of %lld bytes", (long long)need);
   }
   hipStream_t st = (hipStream_t)stream;
-  const int64_t nchw = ((C + 511) / 512 + kNormWaves - 1) / kNormWaves;
-#define L8_NORM(N)                                                                                                        \
-  return w_is_f32 ? launch_norm<N, true>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)      \
-                  : launch_norm<N, false>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)
-  if (nchw <= 1) L8_NORM(1);
-  if (nchw <= 2) L8_NORM(2);
-  L8_NORM(4);
+#define L8_NORM(WAVE, N)                                                                                                        \
+  return w_is_f32 ? launch_norm<WAVE, N, true>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)      \
+                  : launch_norm<WAVE, N, false>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)
+  const int64_t nch = (C + 511) / 512, nchw = (nch + kNormWaves - 1) / kNormWaves;
+  if (nch <= 4) L8_NORM(true, 4);
+  if (nchw <= 2) L8_NORM(false, 2);
+  L8_NORM(false, 4);
 #undef L8_NORM
 }

@@ -83,6 +83,29 @@ def test_zero_rows_and_nonfinite():
     assert torch.equal(q0.view(torch.uint8), q.view(torch.uint8)) and torch.equal(s0.view(torch.int32), s.view(torch.int32))
 
 
+@pytest.mark.parametrize("shape", [(2, 2040), (3, 2048), (5, 2056), (2051, 16), (2051, 2056), (2, 4104)])
+def test_either_side_of_the_layout_line(shape):
+    """A wavefront per row up to 2048 columns, a workgroup per row beyond; more rows than one pass of the grid; rows
+    whose amax is not finite take the integer conversion.  Bounds as in the tests above."""
+    from lingua_amd import ops
+    x = seeded_bf16(shape, std=2.0, seed=shape[0] + shape[1])
+    x[0, -1], x[-1, 0] = float("inf"), float("nan")
+    gy = seeded_bf16(shape, std=0.05, seed=shape[0] + shape[1] + 1)
+    w = (1.0 + 0.1 * torch.randn(shape[1], generator=torch.Generator().manual_seed(3))).to(torch.bfloat16)
+    col = torch.zeros(shape[1], dtype=torch.float32, device="cuda")
+    y, q, s, rstd = ops.rmsnorm_cast_rowwise(x.cuda(), w.cuda(), EPS, col_amax=col)
+    q0, s0, _ = ops.cast_rowwise(y)
+    assert torch.equal(q0.view(torch.uint8), q.view(torch.uint8)) and torch.equal(s0.view(torch.int32), s.view(torch.int32))
+    assert torch.equal(ops.col_amax(y).view(torch.int32), col.view(torch.int32))
+    check_y(y[1:-1], rt.rmsnorm(x, w, EPS)[1:-1]) if shape[0] > 2 else None
+    x[0, -1], x[-1, 0] = 1.0, 1.0
+    xa, wa = x.clone().requires_grad_(True), w.clone().float().requires_grad_(True)
+    rt.rmsnorm(xa, wa, EPS).backward(gy)
+    _, _, _, rstd = ops.rmsnorm_cast_rowwise(x.cuda(), w.cuda(), EPS, want_q=False)
+    gx, gw = ops.rmsnorm_bwd(gy.cuda(), x.cuda(), w.cuda(), rstd)
+    assert rel_l2(gx, xa.grad) <= 1e-3 and rel_l2(gw, wa.grad) <= 1e-4
+
+
 def test_argument_errors():
     from lingua_amd import ops
     x = seeded_bf16((4, 64)).cuda()
