@@ -247,6 +247,42 @@ const char *l8_gemm_algo_name(int algo);
  * per-kernel figures and must name the kernel that ran.  No counterpart in the reference. */
 int l8_gemm_pick(int64_t M, int64_t N, int64_t K);
 
+/* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
+ * Exactly the sequence l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt with its temporaries in `workspace`.  Every
+ * member is eight bytes wide and in this order (a caller without C fills an array).
+ *   x [M,K] bf16 (ldx), w [N,K] bf16 (ldw); bias bf16 [N] or NULL; y bf16 [M,N] (ldy)
+ *   qx e4m3fn [M,K] dense + sx fp32 [M]: where the quantised x is wanted, NULL = in the workspace; with x_ready they
+ *      hold it already and x is not read
+ *   qw e4m3fn [N,K] dense + sw fp32 [N], w_ready: the same for the weight
+ *   col_amax_x fp32 [K] or NULL: column amaxes of x (not with x_ready);  amax_w bf16 [N] or NULL: row amaxes of w (not with
+ *      w_ready)
+ *   algo  as in l8_gemm_nt (0 = library default)
+ *   workspace  device scratch, 256-byte aligned, at least l8_linear_fwd_workspace(args) bytes (which depends on the shape and
+ *      on which members are NULL, not on the other pointers' values) */
+typedef struct {
+  const void *x;
+  int64_t M, K, ldx;
+  const void *w;
+  int64_t N, ldw;
+  const void *bias;
+  void *y;
+  int64_t ldy;
+  void *qx;
+  float *sx;
+  float *col_amax_x;
+  int64_t x_ready;
+  void *qw;
+  float *sw;
+  void *amax_w;
+  int64_t w_ready;
+  int64_t algo;
+  void *workspace;
+  int64_t workspace_bytes;
+  void *stream;
+} l8_linear_fwd_args;
+int64_t l8_linear_fwd_workspace(const l8_linear_fwd_args *args);
+int l8_linear_fwd(const l8_linear_fwd_args *args);
+
 #ifdef __cplusplus
 }
 #endif

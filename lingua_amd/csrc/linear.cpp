@@ -1,0 +1,75 @@
+// One call per pass of a linear: the casts and the product of lingua/float8.py:85-96 enqueued by one entry, their
+// temporaries in one workspace.  A caller in an interpreted language pays for one crossing and one allocation where it
+// paid for one per kernel; with a few tokens that was most of the time.  Same kernels, same order, same results as the
+// entries called one by one.
+#include "l8_common.h"
+
+namespace l8 {
+
+// Hands out 256-byte aligned pieces of a workspace; with a null base it only adds sizes up.
+struct Pieces {
+  uint8_t *base;
+  int64_t used = 0;
+  void *take(int64_t bytes) {
+    uint8_t *p = base ? base + used : nullptr;
+    used += (bytes + 255) / 256 * 256;
+    return p;
+  }
+};
+
+struct LinearFwd {
+  void *qx, *qw, *col_ws;
+  float *sx, *sw;
+  int64_t col_ws_bytes;
+};
+
+static LinearFwd plan(const l8_linear_fwd_args &a, Pieces &ws) {
+  LinearFwd t{};
+  t.qx = a.qx ? a.qx : ws.take(a.M * a.K);
+  t.sx = a.qx ? a.sx : (float *)ws.take(a.M * 4);
+  t.qw = a.qw ? a.qw : ws.take(a.N * a.K);
+  t.sw = a.qw ? a.sw : (float *)ws.take(a.N * 4);
+  t.col_ws_bytes = a.col_amax_x ? l8_cast_rowwise_workspace(a.M, a.K) : 0;
+  t.col_ws = t.col_ws_bytes ? ws.take(t.col_ws_bytes) : nullptr;
+  return t;
+}
+
+}  // namespace l8
+
+using namespace l8;
+
+static int check_fwd(const l8_linear_fwd_args *a) {
+  L8_REQUIRE(a != nullptr, "l8_linear_fwd: null arguments");
+  L8_REQUIRE(a->M >= 0 && a->N >= 0 && a->K >= 0, "l8_linear_fwd: negative shape");
+  L8_REQUIRE((a->qx != nullptr) == (a->sx != nullptr) && (a->qw != nullptr) == (a->sw != nullptr),
+             "l8_linear_fwd: a quantised operand comes with its scales");
+  L8_REQUIRE(!a->x_ready || (a->qx && !a->col_amax_x), "l8_linear_fwd: x_ready without qx, or with col_amax_x");
+  L8_REQUIRE(!a->w_ready || (a->qw && !a->amax_w), "l8_linear_fwd: w_ready without qw, or with amax_w");
+  return L8_OK;
+}
+
+extern "C" int64_t l8_linear_fwd_workspace(const l8_linear_fwd_args *a) {
+  if (check_fwd(a) != L8_OK) return L8_EINVAL;
+  Pieces ws{nullptr};
+  plan(*a, ws);
+  return ws.used;
+}
+
+extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
+  int rc = check_fwd(a);
+  if (rc != L8_OK) return rc;
+  Pieces ws{(uint8_t *)a->workspace};
+  const LinearFwd t = plan(*a, ws);
+  L8_REQUIRE(ws.used <= a->workspace_bytes && ((uintptr_t)a->workspace % 256) == 0,
+             "l8_linear_fwd: needs a 256-byte aligned workspace of %lld bytes", (long long)ws.used);
+  if (!a->x_ready) {
+    rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, a->K, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
+    if (rc != L8_OK) return rc;
+  }
+  if (!a->w_ready) {
+    rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);
+    if (rc != L8_OK) return rc;
+  }
+  return l8_gemm_nt(t.qx, t.qw, a->M, a->N, a->K, a->K, a->K, t.sx, L8_SCALE_ROW, t.sw, L8_SCALE_ROW, a->bias, a->y, a->ldy,
+                    (int)a->algo, a->stream);
+}

@@ -171,16 +171,16 @@ class _LastCast:
 
     @staticmethod
     def _slot(t):
-        return (t.device.index, torch.cuda.current_stream(t.device).cuda_stream)
+        index = t.device.index
+        return (index, ops.current_stream_ptr(index))
 
     @staticmethod
     def _key(t):
-        return (t.data_ptr(), tuple(t.shape), tuple(t.stride()), t.dtype, t.device, t._version,
-                torch.cuda.current_stream(t.device).cuda_stream)
+        return (t.data_ptr(), t.shape, t.stride(), t.dtype, t.device, t._version, ops.current_stream_ptr(t.device.index))
 
     def get(self, t, user):
         # inference tensors have no version counter: nothing would show a write, so they are never shared
-        if t.is_inference():
+        if not self.entries or t.is_inference():
             return None
         entry = self.entries.get(self._slot(t))
         if entry is None or user in entry[3] or entry[0] != self._key(t):
@@ -203,6 +203,8 @@ class _LastCast:
 
     def clear(self, like=None):
         """Drops the entry of the device and current stream of ``like``, or every entry (``like=None``)."""
+        if not self.entries:
+            return
         if like is None:
             self.entries.clear()
         elif like.is_cuda:
@@ -306,9 +308,7 @@ def get_scale_rule() -> str:
     return ops.get_scale_rule()
 
 
-def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
-    """Forward of lingua/float8.py:85-96 on 2-D bf16 operands.  Returns ``(out, amax_b_t, a_col_amax | None)``:
-    the two extra tensors are what backward needs beyond ``a`` and ``b_t``."""
+def _check_operands(a, b_t):
     if a.dtype != torch.bfloat16 or b_t.dtype != torch.bfloat16:
         raise RuntimeError(f"Fp8LinearFn: bf16 input and weight required, got {a.dtype} and {b_t.dtype}")
     if not a.is_cuda or a.device != b_t.device:
@@ -318,6 +318,12 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
         # what torch._scaled_mm tells the reference at lingua/float8.py:65 (both of mat2's dimensions must be
         # divisible by 16); here the forward product could run, but dgrad reduces over out_features
         raise RuntimeError(f"Fp8LinearFn: in_features ({a.shape[-1]}) and out_features ({b_t.shape[0]}) must be multiples of 16")
+
+
+def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
+    """Forward of lingua/float8.py:85-96 on 2-D bf16 operands.  Returns ``(out, amax_b_t, a_col_amax | None)``:
+    the two extra tensors are what backward needs beyond ``a`` and ``b_t``."""
+    _check_operands(a, b_t)
     # column amaxes of `a` fall out of the row-wise pass; wgrad wants them
     _bwd_cast.clear(a)
     hit = _fwd_cast.get(a, b_t.data_ptr()) if config.share_input_casts else None
@@ -333,6 +339,35 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
     qb, sb, amax_b_t = weight_cast_rowwise(b_t)
     out = ops.gemm_nt(qa, qb, sa, sb, bias, algo=gemm_algo)
     return out, amax_b_t, a_col_amax
+
+
+# Up to this many tokens an inference pass quantises its activation once per linear: the cast costs its launch, and the
+# memo that lets linears share it costs the host as much.
+_UNSHARED_TOKENS = 64
+
+
+def linear_infer(a, b_t, bias):
+    """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
+    both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same kernels and results as ``linear_forward``."""
+    if ops.kernel_timer is not None or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
+        return linear_forward(a.flatten(end_dim=-2), b_t, bias, False, config.gemm_algo)[0].unflatten(0, a.shape[:-1])
+    shape = a.shape
+    if a.dim() != 2:
+        a = a.flatten(end_dim=-2)
+    _check_operands(a, b_t)
+    _bwd_cast.clear(a)
+    tokens = a.shape[0]
+    out = a.new_empty(shape[:-1] + b_t.shape[:1])
+    x_cast = hit = None
+    if config.share_input_casts:
+        x_cast = hit = _fwd_cast.get(a, b_t.data_ptr())
+        if hit is None and tokens > _UNSHARED_TOKENS:
+            x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
+    w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
+    ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, w_cast, w_cast is not None, None, config.gemm_algo)
+    if hit is None and x_cast is not None:
+        _fwd_cast.put(a, (*x_cast, None), b_t.data_ptr())
+    return out
 
 
 def input_cast_for_wgrad(a, a_col_amax, user):
@@ -437,11 +472,14 @@ class Fp8LinearFn(torch.autograd.Function):
 
 class Fp8Linear(torch.nn.Linear):
     def forward(self, input: torch.Tensor) -> torch.Tensor:
+        weight, bias = self.weight, self.bias
         if config.use_custom_ops:
             from .custom_ops import fp8_linear
-            out = fp8_linear(input.flatten(end_dim=-2), self.weight, self.bias)
+            out = fp8_linear(input.flatten(end_dim=-2), weight, bias)
+        elif torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
+            out = Fp8LinearFn.apply(input.flatten(end_dim=-2), weight, bias)
         else:
-            out = Fp8LinearFn.apply(input.flatten(end_dim=-2), self.weight, self.bias)
+            return linear_infer(input, weight, bias)
         out = out.unflatten(0, input.shape[:-1])
         return out
 

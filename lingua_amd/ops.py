@@ -4,6 +4,7 @@
 All inputs are CUDA (HIP) tensors on a gfx950 device.  Outputs are returned as
 ``torch.float8_e4m3fn`` / ``torch.float32`` / ``torch.bfloat16`` tensors.
 """
+import struct
 from typing import Optional, Tuple
 
 import torch
@@ -50,13 +51,18 @@ class _timed:
         return False
 
 
+# Raw handle of the calling thread's current stream on a device.  The public property builds a Python Stream object on
+# every call (2 us, as much as a launch); this is what PyTorch's own generated code calls.
+current_stream_ptr = torch._C._cuda_getCurrentRawStream
+
+
 def _prep(t: torch.Tensor, what: str):
     """Checks that `t` lives on a gfx950 GPU and returns the raw handle of the calling thread's current stream
     on that GPU.  The process's current device is left alone."""
     if not t.is_cuda:
         raise RuntimeError(f"{what}: expected a GPU tensor, got device {t.device} (there is no CPU path)")
     _lib.require_device(t.device.index)
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return current_stream_ptr(t.device.index)
 
 
 def _wrote_into(t: torch.Tensor) -> None:
@@ -291,6 +297,46 @@ def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tens
     if user_out:
         _wrote_into(out)
     return out
+
+
+_FWD = struct.Struct("22q")   # l8_linear_fwd_args: eight bytes per member
+
+
+def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y: torch.Tensor, x_cast=None, x_ready: bool = False,
+               col_amax: Optional[torch.Tensor] = None, w_cast=None, w_ready: bool = False, amax_w: Optional[torch.Tensor] = None,
+               algo: int = 0) -> None:
+    """y [M,N] (dense) = x @ w.T + bias with row-wise casts of both, in one call of the library: the same kernels as
+    ``cast_rowwise``, ``cast_rowwise``, ``gemm_nt``.  ``x_cast`` / ``w_cast`` = (q, scale), dense: where the quantised
+    operand goes (None: a temporary), or with ``x_ready`` / ``w_ready`` where it comes from."""
+    st = _prep(x, "linear_fwd")
+    x, w = _rows_2d(x, torch.bfloat16, "linear_fwd(x)"), _rows_2d(w, torch.bfloat16, "linear_fwd(w)")
+    M, K = x.shape
+    N = w.shape[0]
+    if w.shape[1] != K:
+        raise RuntimeError(f"linear_fwd: reduction dims differ ({K} vs {w.shape[1]})")
+    if bias is not None:
+        if bias.dtype != torch.bfloat16 or bias.numel() != N:
+            raise RuntimeError("linear_fwd: bias must be bf16 with N elements")
+        bias = bias.contiguous()
+    if M == 0 or N == 0:
+        return
+    lib = _lib.load()
+    members = [x.data_ptr(), M, K, _ld(x), w.data_ptr(), N, _ld(w), 0 if bias is None else bias.data_ptr(), y.data_ptr(), N,
+               x_cast[0].data_ptr() if x_cast else 0, x_cast[1].data_ptr() if x_cast else 0,
+               0 if col_amax is None else col_amax.data_ptr(), x_ready,
+               w_cast[0].data_ptr() if w_cast else 0, w_cast[1].data_ptr() if w_cast else 0,
+               0 if amax_w is None else amax_w.data_ptr(), w_ready, algo, 0, 0, st]
+    need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))
+    if need > 0:
+        ws = x.new_empty(need, dtype=torch.uint8)
+        members[19], members[20] = ws.data_ptr(), need
+    dev = x.device.index
+    if torch._C._cuda_getDevice() == dev:
+        code = lib.l8_linear_fwd(_FWD.pack(*members))
+    else:
+        with torch.cuda.device(dev):
+            code = lib.l8_linear_fwd(_FWD.pack(*members))
+    _lib.check(code, "l8_linear_fwd")
 
 
 def gemm_pick(M: int, N: int, K: int) -> Tuple[int, str]:

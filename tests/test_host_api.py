@@ -56,6 +56,29 @@ def test_argument_validation_happens_before_launch():
     assert lib.l8_gemm_nt(None, None, 0, 4, 16, 16, 16, None, 1, None, 1, None, None, 4, 0, None) == 0
 
 
+def test_linear_call_validates_its_arguments_on_the_host():
+    """l8_linear_fwd takes a struct of eight-byte members; what it cannot serve is refused before any launch, and the
+    workspace it asks for covers exactly the members that are left to it."""
+    lib = _lib.load()
+    fake = 1 << 20
+    base = dict(x=fake, M=32, K=64, ldx=64, w=fake, N=48, ldw=64, bias=0, y=fake, ldy=48, qx=0, sx=0, col=0, x_ready=0, qw=0,
+                sw=0, amax_w=0, w_ready=0, algo=0, ws=0, ws_bytes=0, stream=0)
+
+    def pack(**kw):
+        return ops._FWD.pack(*dict(base, **kw).values())
+
+    full = lib.l8_linear_fwd_workspace(pack())
+    assert full >= 32 * 64 + 32 * 4 + 48 * 64 + 48 * 4
+    assert lib.l8_linear_fwd_workspace(pack(qw=fake, sw=fake, w_ready=1)) < full
+    assert lib.l8_linear_fwd_workspace(pack(qx=fake, sx=fake)) < full
+    assert lib.l8_linear_fwd_workspace(pack(col=fake)) > full
+    assert lib.l8_linear_fwd(pack()) == -1 and "workspace" in _lib.last_error()
+    assert lib.l8_linear_fwd(pack(M=-1)) == -1 and lib.l8_linear_fwd_workspace(pack(M=-1)) == -1
+    assert lib.l8_linear_fwd(pack(x_ready=1)) == -1 and "x_ready" in _lib.last_error()
+    assert lib.l8_linear_fwd(pack(w_ready=1)) == -1 and "w_ready" in _lib.last_error()
+    assert lib.l8_linear_fwd(pack(qx=fake)) == -1 and lib.l8_linear_fwd(None) == -1
+
+
 def test_no_cpu_path():
     x = torch.zeros(4, 16, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="no CPU path"):
