@@ -51,6 +51,7 @@
 #include <type_traits>
 
 #include "l8_common.h"
+#include "skinny.h"
 
 namespace l8 {
 
@@ -1260,6 +1261,7 @@ template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, 8>(const GemmArgs);
 
+constexpr int kSkinnyAlgo = 17;  // position in the list below
 static const Algo kAlgos[] = {
     L8_ALGO_LIST(L8_ALGO_ROW)
     /* 11, 12: persistent 256x256 tiles, 4 waves, one panel stream across tiles, C stored from the accumulators */
@@ -1279,6 +1281,8 @@ static const Algo kAlgos[] = {
        algo 12 at K = 4096 and 2-4 % behind it at K >= 8192 (1.5 x the LDS reads); a product with a bias takes the
        plain kernel (the bias instantiation would not fit the 256 registers of a wave without spills) */
     {"stream_mt4x2w_2x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, 8>, 256, 256, 512, 5 * 256 * 128, true, nullptr, nullptr},
+    /* 17: at most 64 tokens: 16 rows of B and all of A per workgroup, K split over its waves (skinny_kernels.hip) */
+    {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr},
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
 
@@ -1300,11 +1304,15 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // large problems: the persistent kernel (measured 2-11 % ahead of the plain ones on every shape with at
   // least one 256x256 tile per compute unit; groups of 4 tile rows ahead of groups of 8 by 1-3 %), also when
   // the big tiles leave up to 7/16 of the compute units idle (measured with K = 2048 .. 16384: 144 to 240
-  // tiles on 256 compute units run 10-25 % faster than with 128x128 tiles, 128 tiles and fewer 15-45 % slower);
-  // problems that would leave more of the chip idle with big tiles: 128x128 tiles
+  // tiles on 256 compute units run 10-25 % faster than with 128x128 tiles, 128 tiles and fewer 15-45 % slower)
   (void)K;
-  const int64_t big_tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  if (big_tiles * 16 >= (int64_t)num_cus() * 9) return 12;
+  const int64_t cus = num_cus();
+  auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  if (tiles(256, 256) * 16 >= cus * 9) return 12;
+  // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against 128 x 128 tiles: [20,2048].
+  // [2048,2048] 4.2 / 11.6, [64,11008].[4096,11008] 18.9 / 65, [32,4096].[11008,4096] 14.6 / 28.5, [64,8192].[8192,8192]
+  // 25.3 / 51, [64,4096].[11008,4096] 19.7 / 28.6.
+  if (M <= kSkinnyMaxM) return kSkinnyAlgo;
   return 2;
 }
 
@@ -1382,6 +1390,12 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
                     (sb_mode != L8_SCALE_ROW || ((uintptr_t)sb % 16) == 0) &&
                     (bias == nullptr || (((uintptr_t)bias % 8) == 0 && kAlgos[algo - 1].fn_bias != nullptr));
     if (!ok) algo = pick_plain_big(K);
+  }
+  if (algo == kSkinnyAlgo) {
+    if (skinny_serves(M, N, K, lda, ldb, 1))
+      return skinny_linear(SkinnyArgs{A, B, (int)M, (int)N, (int)K, lda, ldb, sa, sb, sa_mode == L8_SCALE_ROW, sb_mode == L8_SCALE_ROW,
+                                      (const uint16_t *)bias, (uint16_t *)C, ldc, 0}, false, (hipStream_t)stream);
+    algo = 2;
   }
   const Algo &al = kAlgos[algo - 1];
   // 32-bit in-tile byte offsets: (tile rows) * ld + K must stay below 2^31

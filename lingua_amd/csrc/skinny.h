@@ -1,0 +1,27 @@
+// Products of a few tokens with a whole weight (skinny_kernels.hip): what the dispatch in the other files needs of them.
+#pragma once
+#include "l8_common.h"
+
+namespace l8 {
+
+struct SkinnyArgs {
+  const void *x, *w;    // x fp8; w fp8, or bf16 where the kernel quantises it
+  int M, N, K;
+  int64_t ldx, ldw;     // in elements
+  const float *sx, *sw; // sw unused where the kernel quantises the weight
+  int sx_row, sw_row;
+  const uint16_t *bias;
+  uint16_t *y;
+  int64_t ldy;
+  int scale_rule;
+};
+
+constexpr int kSkinnyMaxM = 64;
+// longest row that is quantised in registers: 12 steps of 128 elements for each of eight waves (192 registers)
+constexpr int kSkinnyMaxQuantSteps = 12, kSkinnyMaxQuantK = kSkinnyMaxQuantSteps * 128 * 8;
+
+// can the kernels serve the problem (w_bytes: 1 = fp8 weight, 2 = bf16 weight that is quantised on the way)
+bool skinny_serves(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int w_bytes);
+int skinny_linear(const SkinnyArgs &p, bool w_is_bf16, hipStream_t st);
+
+}  // namespace l8

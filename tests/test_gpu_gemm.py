@@ -42,6 +42,31 @@ def test_exact_small_integer_operands(algo):
         assert torch.equal(out.cpu().double(), want), (algo, M, N, K)
 
 
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 48, 49, 64])
+def test_few_tokens_exact_on_integers_and_within_tolerance_of_the_oracle(M):
+    """At most 64 tokens (the default's choice; 65 take a tile kernel): token tiles of 16 full and ragged, weight rows
+    that do not fill a tile of 16, reductions shorter than one step of 128, ragged, and longer than the eight waves'
+    first round of steps; scalar scales and a bias.  Integers in -1 .. 1 sum exactly whatever the order."""
+    from lingua_amd import ops
+    assert ops.gemm_pick(M, 2048, 2048)[1].startswith("skinny") and not ops.gemm_pick(65, 2048, 2048)[1].startswith("skinny")
+    g = torch.Generator().manual_seed(700 + M)
+    for (N, K) in [(1, 16), (16, 128), (17, 144), (33, 1040), (100, 2064), (520, 4112)]:
+        A = torch.randint(-1, 2, (M, K), generator=g).float()
+        B = torch.randint(-1, 2, (N, K), generator=g).float()
+        sa = torch.tensor([2.0 ** (i % 5 - 2) for i in range(M)]).reshape(M, 1)
+        sb = torch.tensor([2.0 ** (i % 3) for i in range(N)]).reshape(N, 1)
+        out = ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa.cuda(), sb.cuda())
+        assert torch.equal(out.cpu().double(), (A.double() @ B.double().t()) * sa.double() * sb.double().t()), (M, N, K)
+        qa, qb = random_fp8_bytes((M, K), g), random_fp8_bytes((N, K), g)
+        bias = (torch.randn(N, generator=g) * 50).to(torch.bfloat16)
+        for sa_, sb_, b_ in ((sa, sb, bias), (sa[:1], sb, None), (sa, sb[:1], bias)):
+            out = ops.gemm_nt(qa.cuda().view(torch.float8_e4m3fn), qb.cuda().view(torch.float8_e4m3fn), sa_.cuda(), sb_.cuda(),
+                              b_.cuda() if b_ is not None else None)
+            # about 3 % of the products of random bytes round to the other neighbour (the matrix instruction's own sum,
+            # whatever the kernel); where one of few outputs dominates the norm, its step is up to 2^-8 of it
+            assert rel_l2(out, oracle.gemm_nt(qa, qb, sa_, sb_, b_)) <= (TOL if M * N >= 5000 else 2.0 ** -8), (M, N, K)
+
+
 @pytest.mark.parametrize("algo", [0, 1, 2, 3, 11, 15])
 def test_k_indexing_with_one_hot_operands(algo):
     # B[n] is one-hot at k = pi(n): C[m,n] = A[m, pi(n)] exactly, for any K (tails included)
