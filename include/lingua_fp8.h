@@ -248,8 +248,9 @@ const char *l8_gemm_algo_name(int algo);
 int l8_gemm_pick(int64_t M, int64_t N, int64_t K);
 
 /* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
- * Exactly the sequence l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt with its temporaries in `workspace`.  Every
- * member is eight bytes wide and in this order (a caller without C fills an array).
+ * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; with a few
+ * tokens, and neither qw nor amax_w asked for, the weight is quantised inside the product.  Every member is eight bytes
+ * wide and in this order (a caller without C fills an array).
  *   x [M,K] bf16 (ldx), w [N,K] bf16 (ldw); bias bf16 [N] or NULL; y bf16 [M,N] (ldy)
  *   qx e4m3fn [M,K] dense + sx fp32 [M]: where the quantised x is wanted, NULL = in the workspace; with x_ready they
  *      hold it already and x is not read

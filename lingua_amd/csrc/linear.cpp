@@ -1,8 +1,8 @@
 // One call per pass of a linear: the casts and the product of lingua/float8.py:85-96 enqueued by one entry, their
 // temporaries in one workspace.  A caller in an interpreted language pays for one crossing and one allocation where it
-// paid for one per kernel; with a few tokens that was most of the time.  Same kernels, same order, same results as the
-// entries called one by one.
+// paid for one per kernel; with a few tokens that was most of the time.  Same results as the entries called one by one.
 #include "l8_common.h"
+#include "skinny.h"
 
 namespace l8 {
 
@@ -21,14 +21,21 @@ struct LinearFwd {
   void *qx, *qw, *col_ws;
   float *sx, *sw;
   int64_t col_ws_bytes;
+  bool w_on_the_way;  // the weight is quantised inside the product
 };
 
 static LinearFwd plan(const l8_linear_fwd_args &a, Pieces &ws) {
   LinearFwd t{};
   t.qx = a.qx ? a.qx : ws.take(a.M * a.K);
   t.sx = a.qx ? a.sx : (float *)ws.take(a.M * 4);
-  t.qw = a.qw ? a.qw : ws.take(a.N * a.K);
-  t.sw = a.qw ? a.sw : (float *)ws.take(a.N * 4);
+  // A few tokens and nobody who wants the weight's bytes or amaxes: one pass over the weight instead of three (read,
+  // written, read).  us, weights cold, cast + product / one kernel: [1,4096].[11008,4096] 44 / 20.8, [7,4096].[4096,4096]
+  // 25 / 10.4, [8,2048].[8192,2048] 20 / 12, [64,4096].[11008,4096] 54 / 28.
+  t.w_on_the_way = !a.qw && !a.amax_w && a.algo == 0 && skinny_serves(a.M, a.N, a.K, a.K, a.ldw, 2);
+  if (!t.w_on_the_way) {
+    t.qw = a.qw ? a.qw : ws.take(a.N * a.K);
+    t.sw = a.qw ? a.sw : (float *)ws.take(a.N * 4);
+  }
   t.col_ws_bytes = a.col_amax_x ? l8_cast_rowwise_workspace(a.M, a.K) : 0;
   t.col_ws = t.col_ws_bytes ? ws.take(t.col_ws_bytes) : nullptr;
   return t;
@@ -65,6 +72,12 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
   if (!a->x_ready) {
     rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, a->K, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
     if (rc != L8_OK) return rc;
+  }
+  if (t.w_on_the_way) {
+    L8_REQUIRE(a->w && a->y && a->K > 0 && a->K % 16 == 0 && a->ldw % 8 == 0 && a->ldw >= a->K && ((uintptr_t)a->w % 16) == 0 && a->ldy >= a->N,
+               "l8_linear_fwd: K=%lld must be a multiple of 16, ldw=%lld of 8 and >= K, w 16-byte aligned, ldy >= N", (long long)a->K, (long long)a->ldw);
+    return skinny_linear(SkinnyArgs{t.qx, a->w, (int)a->M, (int)a->N, (int)a->K, a->K, a->ldw, t.sx, nullptr, 1, 0,
+                                    (const uint16_t *)a->bias, (uint16_t *)a->y, a->ldy, scale_rule()}, true, (hipStream_t)a->stream);
   }
   if (!a->w_ready) {
     rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);

@@ -65,3 +65,27 @@ def test_linears_share_an_activation_and_see_it_change():
             x.mul_(3.0)
             assert rel_l2(w3(x), oracle.linear_forward(x.cpu(), w3.weight.detach().cpu())) <= 1e-3
         float8.clear_cast_memos()
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
+@pytest.mark.parametrize("K", [16, 272, 4096, 4112, 8192, 8208, 12288, 12304])
+def test_weight_quantised_inside_the_product(M, K):
+    """Few tokens: the weight's row amaxes, scales and bytes are made between its only read and the product.  Rows of
+    every register budget (4096, 8192, 12288 columns) and past the last; zero rows, rows with an infinity or a NaN (their
+    outputs are NaN), a weight with a padded row stride; the same bits as the casts and the product one by one."""
+    from lingua_amd import ops
+    N = 52
+    x = seeded_bf16((M, K), seed=M + K).cuda()
+    w = torch.zeros((N, K + 8), dtype=torch.bfloat16)[:, :K]
+    w.copy_(seeded_bf16((N, K), 0.02, seed=K))
+    w[1] = 0.0
+    w[7, K - 1], w[20, 0] = float("nan"), float("inf")
+    bias = seeded_bf16((N,), seed=2).cuda()
+    w = w.cuda()
+    qx, sx, _ = ops.cast_rowwise(x)
+    qw, sw, _ = ops.cast_rowwise(w)
+    want = ops.gemm_nt(qx, qw, sx, sw, bias)
+    got = torch.empty_like(want)
+    ops.linear_fwd(x, w, bias, got)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and bool(torch.isnan(want[:, [7, 20]]).all())
+    assert torch.equal(torch.nan_to_num(got.float()), torch.nan_to_num(want.float()))
