@@ -1241,9 +1241,18 @@ struct Algo {
   X(2, 2, 4, 4, 5, 16, 0) /* 9: algo 1 with groups of 16                      */ \
   X(2, 4, 4, 2, 5, 8, 0)  /* 10: algo 3 with taller groups                    */
 
+// 18 .. 21: small problems, one workgroup per compute unit or fewer: a ring of 9 slots (3.5 K tiles ahead instead of 1.5;
+// a second workgroup has no use for the LDS) and smaller tiles where 128 x 128 ones would be too few
+#define L8_SMALL_ALGO_LIST(X)                         \
+  X(2, 2, 2, 2, 9, 4, 0) /* 18: 128x128            */ \
+  X(2, 2, 1, 2, 9, 4, 0) /* 19: 64x128             */ \
+  X(2, 2, 2, 1, 9, 4, 0) /* 20: 128x64             */ \
+  X(2, 2, 1, 1, 9, 4, 0) /* 21: 64x64              */
+
 #define L8_INSTANTIATE(WM, WN, TM, TN, R, GM, PF) \
   template __global__ void gemm_nt_kernel<WM, WN, TM, TN, R, GM, PF>(const GemmArgs);
 L8_ALGO_LIST(L8_INSTANTIATE)
+L8_SMALL_ALGO_LIST(L8_INSTANTIATE)
 
 #define L8_MAX2(a, b) ((a) > (b) ? (a) : (b))
 #define L8_ALGO_ROW(WM, WN, TM, TN, R, GM, PF)                                                                \
@@ -1283,6 +1292,7 @@ static const Algo kAlgos[] = {
     {"stream_mt4x2w_2x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, 8>, 256, 256, 512, 5 * 256 * 128, true, nullptr, nullptr},
     /* 17: at most 64 tokens: 16 rows of B and all of A per workgroup, K split over its waves (skinny_kernels.hip) */
     {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr},
+    L8_SMALL_ALGO_LIST(L8_ALGO_ROW)
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
 
@@ -1309,11 +1319,22 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(256, 256) * 16 >= cus * 9) return 12;
-  // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against 128 x 128 tiles: [20,2048].
-  // [2048,2048] 4.2 / 11.6, [64,11008].[4096,11008] 18.9 / 65, [32,4096].[11008,4096] 14.6 / 28.5, [64,8192].[8192,8192]
-  // 25.3 / 51, [64,4096].[11008,4096] 19.7 / 28.6.
-  if (M <= kSkinnyMaxM) return kSkinnyAlgo;
-  return 2;
+  // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against the best tile: [20,2048].
+  // [2048,2048] 4.2 / 7.5, [64,11008].[4096,11008] 18.9 / 28.8, [32,4096].[11008,4096] 14.6 / 13.5; from 48 tokens on
+  // the 64 x 64 tiles win where there are enough of them ([48,4096].[11008,4096] 17.6 / 14.0, [40,4096].[8192,4096]
+  // 12.2 / 12.1, [64,8192].[8192,8192] 25.3 / 23.5).
+  if (M <= 32 || (M <= kSkinnyMaxM && tiles(64, 64) * 16 < cus * 7)) return kSkinnyAlgo;
+  // Otherwise the smallest tile that gives no compute unit a second workgroup: these kernels are bound by their LDS
+  // traffic and by what a K tile costs whatever its size, so more units at work are worth more than the larger tile's
+  // economy.  us, 128 x 128 with two workgroups per unit (configuration 2) / chosen: [200,4096].[4096,4096] 19.1 / 11.9
+  // (64 x 64), [333,8192].[2048,8192] 32.8 / 19.5 (64 x 64), [1021,2048].[2048,2048] 12.3 / 9.3 (64 x 128),
+  // [512,4096].[4096,4096] 19.7 / 14.7 (128 x 64), [700,11008].[4096,11008] 67.2 / 49.5 (128 x 128, 9 slots),
+  // [2048,16384].[2048,16384] 86.8 / 72.1 (the same).
+  if (tiles(64, 64) <= cus) return 21;
+  if (tiles(64, 128) <= cus) return 19;
+  if (tiles(128, 64) <= cus) return 20;
+  if (tiles(128, 128) <= cus) return 18;
+  return 2;  // two 128 x 128 workgroups share a unit: [1500,1440].[3008,1440] 16.3, 20.9 with nine slots
 }
 
 // Host arithmetic only: the tile configuration `algo = 0` resolves to for this problem on the current device when

@@ -67,6 +67,33 @@ def test_few_tokens_exact_on_integers_and_within_tolerance_of_the_oracle(M):
             assert rel_l2(out, oracle.gemm_nt(qa, qb, sa_, sb_, b_)) <= (TOL if M * N >= 5000 else 2.0 ** -8), (M, N, K)
 
 
+@pytest.mark.parametrize("algo,tile", [(18, (128, 128)), (19, (64, 128)), (20, (128, 64)), (21, (64, 64))])
+def test_small_tiles_exact_on_integers_at_their_edges(algo, tile):
+    """The configurations for problems of at most one workgroup per compute unit: tiles full, one short and one over,
+    reductions from a ring that is never filled (K = 16) to one that wraps several times."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(800 + algo)
+    bm, bn = tile
+    for (M, N, K) in [(bm, bn, 16), (bm - 1, bn + 1, 128), (bm + 1, bn - 1, 400), (3 * bm, 2 * bn, 1152), (2 * bm + 5, bn + 8, 2064)]:
+        A = torch.randint(-1, 2, (M, K), generator=g).float()
+        B = torch.randint(-1, 2, (N, K), generator=g).float()
+        sa = torch.tensor([2.0 ** (i % 5 - 2) for i in range(M)]).reshape(M, 1)
+        bias = torch.randint(-8, 9, (N,), generator=g).to(torch.bfloat16)
+        out = ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa.cuda(), torch.ones(1, 1).cuda(), bias.cuda(), algo=algo)
+        want = ((A.double() @ B.double().t()) * sa.double() + bias.double()).to(torch.bfloat16)
+        assert torch.equal(out.cpu(), want), (algo, M, N, K)
+
+
+@pytest.mark.parametrize("mnk,name", [((200, 4096, 4096), "1x1t"), ((1021, 2048, 2048), "1x2t"), ((512, 4096, 4096), "1x2t"),
+                                      ((2176, 960, 256), "2x1t"), ((2048, 2048, 4096), "2x2t_r9"), ((1500, 3008, 1440), "2x2t_r5"),
+                                      ((64, 11008, 4096), "1x1t"), ((16384, 2048, 2048), "stream")])
+def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
+    from lingua_amd import ops
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are for 256 compute units")
+    assert name in ops.gemm_pick(*mnk)[1]
+
+
 @pytest.mark.parametrize("algo", [0, 1, 2, 3, 11, 15])
 def test_k_indexing_with_one_hot_operands(algo):
     # B[n] is one-hot at k = pi(n): C[m,n] = A[m, pi(n)] exactly, for any K (tails included)
