@@ -634,9 +634,13 @@ static int64_t rowwise_blocks(int64_t R, int64_t C, bool colmax) {
     return blocks < cap ? blocks : cap;
   }
   if ((nch + kRowWaves - 1) / kRowWaves <= 16) {
-    // without column maxima four workgroups per unit: [32768,8192] behind its producer 123 us, 130 with eight, 124 with two
-    // (a row requested ahead does what more workgroups would); the weight [4096,11008] 23.5 / 25.0 / 23.6
-    const int64_t cap = cus * (colmax ? 2 : 4);
+    // Workgroups per unit, each with a row in registers and a row requested ahead: enough rows in flight to cover the
+    // memory's latency, no more than it wants (and, with column maxima, few partial rows to write and fold).  us, row
+    // amaxes alone / cast / with column maxima: [16384,4608] 2 per unit 48.7 / 54.2 / 58.0, 4: 31.9 / 40.3 / 45.7,
+    // 6: 28.5 / 41.2, 8: 32.5 / 44.0, with column maxima 3: 48.6; [32768,8192] 2: 102 / 127 / 133, 4: 85 / 130 / 143,
+    // 8: 92 / 137, with column maxima 3: 138; behind its producer the cast of [32768,8192] takes 124 / 123 / 130 with 2 / 4 / 8.
+    const bool short_row = nch <= 3 * kRowWaves;
+    const int64_t cap = cus * (colmax ? (short_row ? 3 : 2) : (short_row ? 6 : 4));
     return R < cap ? R : cap;
   }
   return 0;
@@ -716,6 +720,7 @@ static int cast_rowwise_impl(const char *what, const void *x, int64_t R, int64_t
   if (nch <= 8) return launch_rowwise<8>(x, R, C, ldx, q, ldq, scale, amax, col_amax, ws, st);
   // longer rows: one workgroup per row, nchw = chunks per lane
   const int64_t nchw = (nch + kRowWaves - 1) / kRowWaves;
+  if (nchw <= 3) return launch_rowwise_wg<3>(x, R, C, ldx, q, ldq, scale, amax, col_amax, ws, st);
   if (nchw <= 4) return launch_rowwise_wg<4>(x, R, C, ldx, q, ldq, scale, amax, col_amax, ws, st);
   if (nchw <= 6) return launch_rowwise_wg<6>(x, R, C, ldx, q, ldq, scale, amax, col_amax, ws, st);
   if (nchw <= 8) return launch_rowwise_wg<8>(x, R, C, ldx, q, ldq, scale, amax, col_amax, ws, st);

@@ -67,6 +67,14 @@ def test_rowwise_shapes(shape, with_col):
     check_rowwise(x, with_col)
 
 
+@pytest.mark.parametrize("shape", [(2, 4096), (3, 4104), (2, 6144), (1600, 4616), (3, 6152), (2, 8192), (1030, 8200)])
+@pytest.mark.parametrize("with_col", [False, True])
+def test_rowwise_either_side_of_the_layout_lines(shape, with_col):
+    """A wavefront per row up to 4096 columns, then a workgroup per row with three, four, six ... chunks per lane; more
+    rows than one pass of the grid."""
+    check_rowwise(seeded_bf16(shape, seed=shape[0] + shape[1]), with_col)
+
+
 def test_rowwise_config1_inputs():
     check_rowwise(seeded_bf16((4096, 2048), 1.0, seed=0), with_col=True)
     check_rowwise(seeded_bf16((2048, 2048), 0.02, seed=1))
