@@ -247,6 +247,12 @@ const char *l8_gemm_algo_name(int algo);
  * per-kernel figures and must name the kernel that ran.  No counterpart in the reference. */
 int l8_gemm_pick(int64_t M, int64_t N, int64_t K);
 
+/* C += product: C = bf16( f32(bf16(product * scales)) + f32(C) ), what l8_gemm_nt into a temporary followed by an
+ * elementwise bf16 add would leave, without the two passes of that add.  Serves the sum of the input gradients of linears
+ * on one activation (autograd adds them, lingua/float8.py:119 once per linear).  Arguments as in l8_gemm_nt, no bias. */
+int l8_gemm_nt_add(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                   const float *sa, int sa_mode, const float *sb, int sb_mode, void *C, int64_t ldc, int algo, void *stream);
+
 /* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
  * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; with a few
  * tokens, and neither qw nor amax_w asked for, the weight is quantised inside the product.  Every member is eight bytes

@@ -63,6 +63,7 @@ struct GemmArgs {
   int sa_row, sb_row;
   const uint16_t *bias;
   uint16_t *C;
+  int add;  // C = bf16(bf16(product) + C) instead of C = bf16(product): a sum of gradients without a pass of its own
   int tiles_m, tiles_n;
   uint64_t *dbg;  // L8_GEMM_PROF builds only
   // persistent kernels, optional (null = every tile is computed by one workgroup): workspace for tiles whose
@@ -119,6 +120,22 @@ L8_DEV void store16_aux(v4i data, __amdgpu_buffer_rsrc_t rs, uint32_t voff, int 
 // and at its end, and shader-clock cycles spent in the K loops and in the C-tile stores.
 #ifndef L8_GEMM_PROF
 #define L8_GEMM_PROF 0
+#endif
+
+#if defined(__HIP_DEVICE_COMPILE__)
+// Eight bf16 plus eight bf16, each sum rounded to nearest even: what PyTorch's add makes of two bf16 tensors.
+L8_DEV v4i add_bf16x8(v4i a, v4i b) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  v4i r;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float lo = __uint_as_float((uint32_t)a[k] << 16) + __uint_as_float((uint32_t)b[k] << 16);
+    const float hi = __uint_as_float((uint32_t)a[k] & 0xffff0000u) + __uint_as_float((uint32_t)b[k] & 0xffff0000u);
+    const bf2 p = {(__bf16)lo, (__bf16)hi};
+    r[k] = __builtin_bit_cast(int, p);
+  }
+  return r;
+}
 #endif
 
 // s_waitcnt for vmcnt <= n and lgkmcnt == 0 (expcnt untouched)
@@ -486,6 +503,14 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
     // that the C tile on its way out does not push the operand panels out of the L2
     uint16_t *dst = p.C + (int64_t)(m0 + row0) * p.ldc + n0 + col;
     const uint32_t at = lds0 + row0 * C_ROW + col * 2;
+    if (p.add) {
+#pragma unroll 8
+      for (int it = 0; it < ITERS; ++it) {
+        v4i *at_c = (v4i *)(dst + (int64_t)it * ROWS_PER_IT * p.ldc);
+        __builtin_nontemporal_store(add_bf16x8(*reinterpret_cast<lds_v4i_ptr>(at + it * (ROWS_PER_IT * C_ROW)), __builtin_nontemporal_load(at_c)), at_c);
+      }
+      return;
+    }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it)
       __builtin_nontemporal_store(*reinterpret_cast<lds_v4i_ptr>(at + it * (ROWS_PER_IT * C_ROW)),
@@ -499,11 +524,14 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
       if (m < p.M && n < p.N) {
         uint16_t *dst = p.C + (int64_t)m * p.ldc + n;
         if (c_vec && n + 8 <= p.N) {
-          __builtin_nontemporal_store(v, (v4i *)dst);
+          __builtin_nontemporal_store(p.add ? add_bf16x8(v, *(const v4i *)dst) : v, (v4i *)dst);
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
-            if (n + e < p.N) dst[e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+            if (n + e < p.N) {
+              const uint32_t h = ((uint32_t)v[e >> 1] >> (16 * (e & 1))) & 0xffffu;
+              dst[e] = p.add ? (uint16_t)bf16_rne_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(dst[e])) : (uint16_t)h;
+            }
         }
       }
     }
@@ -539,7 +567,10 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
 // so the workgroups resident on an XCD always work on W consecutive tiles of
 // the grouped order and share their panels in that XCD's L2.
 // ---------------------------------------------------------------------------
-template <int GROUP_M, bool HAS_BIAS, bool SK = false, int NW = 4>
+// ADD: the bf16 tile is added to what C holds (two gradients of one activation) in the epilogue.  The C values are
+// requested C_AHEAD row groups before they are used: the counter retires in order, so the wait for them is also one for the
+// stores issued before they were requested, and those have had that long.
+template <int GROUP_M, bool HAS_BIAS, bool SK = false, int NW = 4, bool ADD = false>
 __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // NW = 4: one wave per SIMD, 128x128 per wave (the least LDS traffic per flop); NW = 8: two waves per SIMD,
@@ -887,6 +918,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
 #pragma unroll
       for (int g = 0; g < P_AHEAD; ++g) request_parts(g, pbuf[g]);
     }
+    // (the values of C that an ADD tile is added to, two 16-byte pieces per lane and row group)
+    constexpr int C_AHEAD = 4;
+    [[maybe_unused]] v4i cbuf[C_AHEAD + 1][2];
     [[maybe_unused]] uint64_t tq0 = 0, tq1 = 0, tq2 = 0;
     if (L8_GEMM_PROF) {
       tq0 = __builtin_readcyclecounter();
@@ -900,6 +934,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     // store nothing (N % 8 == 0 here: a lane pair is in or out as a whole).
     const int par = l31 >> 4;
     const uint32_t c_voff = (n0 + lane_col < p.N) ? (uint32_t)((4 * h + par) * ldc2 + lane_col * 2) : kOOB;
+    [[maybe_unused]] auto request_c = [&](int g, v4i (&dst)[2]) {
+      const int row = wm * WROWS + (g >> 2) * 32 + 8 * (g & 3);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) dst[i] = __builtin_amdgcn_raw_buffer_load_b128(rsC, c_voff, (row + 2 * i) * ldc2, 2 /* streaming */);
+    };
+    if constexpr (ADD) {
+#pragma unroll
+      for (int g = 0; g < C_AHEAD; ++g) request_c(g, cbuf[g]);
+    }
     if (L8_GEMM_PROF) {
       __builtin_amdgcn_s_waitcnt(0x0070);  // the scales
       tq2 = __builtin_readcyclecounter();
@@ -914,6 +957,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
         float(&sa_cur)[4] = sa_grp[g & 1];
         if constexpr (PARTS) {
           if (g + P_AHEAD < TM * 4) request_parts(g + P_AHEAD, pbuf[(g + P_AHEAD) % (P_AHEAD + 1)]);
+        }
+        if constexpr (ADD) {
+          if (g + C_AHEAD < TM * 4) request_c(g + C_AHEAD, cbuf[(g + C_AHEAD) % (C_AHEAD + 1)]);
         }
         if (g + 1 < TM * 4) {
           request_row_scales(g + 1, sa_grp[(g + 1) & 1]);
@@ -945,7 +991,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
           // even rows of its second
           const auto s0 = __builtin_amdgcn_permlane16_swap((unsigned)o[0][0], (unsigned)o[1][0], false, false);
           const auto s1 = __builtin_amdgcn_permlane16_swap((unsigned)o[0][1], (unsigned)o[1][1], false, false);
-          const v4i out = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+          v4i out = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
+          if constexpr (ADD) out = add_bf16x8(out, cbuf[g % (C_AHEAD + 1)][e2 / 2]);
           if (L8_GEMM_DIAG != 3 && !(L8_GEMM_DIAG == 8 && (qd & 1)))  // experiments: no stores (3), half of them (8)
             store16(out, rsC, c_voff, (row + e2) * ldc2, 2 /* streaming */);
           // one row pair at a time: left free, the scheduler reads a hundred accumulator registers ahead and the
@@ -1225,6 +1272,7 @@ struct Algo {
   int bm, bn, threads, lds;
   bool persistent;   // one workgroup per compute unit walks a list of tiles
   gemm_fn fn_bias;   // persistent kernels: the instantiation that adds a bias (the plain kernels branch inside)
+  gemm_fn fn_add;    // persistent kernels: the instantiation that adds to C (bias-free), or null (the plain kernels branch inside)
   gemm_fn fn_sk;     // persistent kernels: the instantiation that can share a tile's K range out (bias-free), or null
 };
 
@@ -1257,13 +1305,14 @@ L8_SMALL_ALGO_LIST(L8_INSTANTIATE)
 #define L8_MAX2(a, b) ((a) > (b) ? (a) : (b))
 #define L8_ALGO_ROW(WM, WN, TM, TN, R, GM, PF)                                                                \
   {"mt" #WM "x" #WN "w_" #TM "x" #TN "t_r" #R "_g" #GM "_pf" #PF, gemm_nt_kernel<WM, WN, TM, TN, R, GM, PF>, \
-   WM * TM * 32, WN * TN * 32, WM * WN * 64, R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr},
+   WM * TM * 32, WN * TN * 32, WM * WN * 64, R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr, nullptr},
 
 template __global__ void gemm_nt_stream_kernel<8, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<8, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, 4, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
@@ -1274,24 +1323,25 @@ constexpr int kSkinnyAlgo = 17;  // position in the list below
 static const Algo kAlgos[] = {
     L8_ALGO_LIST(L8_ALGO_ROW)
     /* 11, 12: persistent 256x256 tiles, 4 waves, one panel stream across tiles, C stored from the accumulators */
-    {"stream_mt2x2w_4x4t_r5_g8", gemm_nt_stream_kernel<8, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<8, true>, nullptr},
-    {"stream_mt2x2w_4x4t_r5_g4", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g8", gemm_nt_stream_kernel<8, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<8, true>, nullptr, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g4", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>,
+     gemm_nt_stream_kernel<4, false, false, 4, true>, nullptr},
     /* 13, 14: other shapes of the block of tiles resident on an XCD (2 x 16 and 16 x 2 instead of 4 x 8: 18 panels
        shared by 32 tiles instead of 12), kept for the traffic comparison */
-    {"stream_mt2x2w_4x4t_r5_g2", gemm_nt_stream_kernel<2, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<2, true>, nullptr},
-    {"stream_mt2x2w_4x4t_r5_g16", gemm_nt_stream_kernel<16, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<16, true>, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g2", gemm_nt_stream_kernel<2, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<2, true>, nullptr, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g16", gemm_nt_stream_kernel<16, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<16, true>, nullptr, nullptr},
     /* 15: algo 12 that may share the K range of the last round's tiles out between workgroups (l8_gemm_nt_ws with
        a workspace; without one it is algo 12).  Measured neutral on the shapes it applies to: the part is
        power-limited, and the compute units that the plain split leaves idle in the last round let the busy ones
        clock higher, which recovers most of what the idle ones lose. */
     {"stream_mt2x2w_4x4t_r5_g4_sk", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>,
-     gemm_nt_stream_kernel<4, false, true>},
+     gemm_nt_stream_kernel<4, false, false, 4, true>, gemm_nt_stream_kernel<4, false, true>},
     /* 16: algo 12 with eight waves (two per SIMD, 64x128 each), kept for the comparison: measured 1-2 % ahead of
        algo 12 at K = 4096 and 2-4 % behind it at K >= 8192 (1.5 x the LDS reads); a product with a bias takes the
        plain kernel (the bias instantiation would not fit the 256 registers of a wave without spills) */
-    {"stream_mt4x2w_2x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, 8>, 256, 256, 512, 5 * 256 * 128, true, nullptr, nullptr},
+    {"stream_mt4x2w_2x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, 8>, 256, 256, 512, 5 * 256 * 128, true, nullptr, nullptr, nullptr},
     /* 17: at most 64 tokens: 16 rows of B and all of A per workgroup, K split over its waves (skinny_kernels.hip) */
-    {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr},
+    {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr, nullptr},
     L8_SMALL_ALGO_LIST(L8_ALGO_ROW)
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
@@ -1386,7 +1436,7 @@ extern "C" int l8_gemm_shares_k(int64_t M, int64_t N, int64_t K, int compute_uni
 
 static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                         const float *sa, int sa_mode, const float *sb, int sb_mode, const void *bias, void *C,
-                        int64_t ldc, int algo, void *workspace, int64_t workspace_bytes, void *stream) {
+                        int64_t ldc, int add, int algo, void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(M >= 0 && N >= 0 && K >= 0, "l8_gemm_nt: negative shape");
   if (M == 0 || N == 0) return L8_OK;
   L8_REQUIRE(A && B && C && sa && sb, "l8_gemm_nt: null pointer");
@@ -1409,13 +1459,14 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
                     M < (1LL << 29) && N < (1LL << 29) &&
                     (sa_mode != L8_SCALE_ROW || ((uintptr_t)sa % 16) == 0) &&
                     (sb_mode != L8_SCALE_ROW || ((uintptr_t)sb % 16) == 0) &&
-                    (bias == nullptr || (((uintptr_t)bias % 8) == 0 && kAlgos[algo - 1].fn_bias != nullptr));
+                    (bias == nullptr || (((uintptr_t)bias % 8) == 0 && kAlgos[algo - 1].fn_bias != nullptr)) &&
+                    (!add || kAlgos[algo - 1].fn_add != nullptr);
     if (!ok) algo = pick_plain_big(K);
   }
   if (algo == kSkinnyAlgo) {
     if (skinny_serves(M, N, K, lda, ldb, 1))
       return skinny_linear(SkinnyArgs{A, B, (int)M, (int)N, (int)K, lda, ldb, sa, sb, sa_mode == L8_SCALE_ROW, sb_mode == L8_SCALE_ROW,
-                                      (const uint16_t *)bias, (uint16_t *)C, ldc, 0}, false, (hipStream_t)stream);
+                                      (const uint16_t *)bias, (uint16_t *)C, ldc, 0, add}, false, (hipStream_t)stream);
     algo = 2;
   }
   const Algo &al = kAlgos[algo - 1];
@@ -1436,6 +1487,7 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
   p.sa_row = sa_mode == L8_SCALE_ROW;
   p.sb_row = sb_mode == L8_SCALE_ROW;
   p.bias = (const uint16_t *)bias;
+  p.add = add;
   p.sk_flags = nullptr;
   p.sk_partials = nullptr;
   p.sk_epoch = 0;
@@ -1455,6 +1507,7 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
   if (slot < 0 || !attr_done[slot][algo - 1]) {
     L8_HIP(hipFuncSetAttribute((const void *)al.fn, hipFuncAttributeMaxDynamicSharedMemorySize, al.lds));
     if (al.fn_bias) L8_HIP(hipFuncSetAttribute((const void *)al.fn_bias, hipFuncAttributeMaxDynamicSharedMemorySize, al.lds));
+    if (al.fn_add) L8_HIP(hipFuncSetAttribute((const void *)al.fn_add, hipFuncAttributeMaxDynamicSharedMemorySize, al.lds));
     if (al.fn_sk) L8_HIP(hipFuncSetAttribute((const void *)al.fn_sk, hipFuncAttributeMaxDynamicSharedMemorySize, al.lds));
     if (slot >= 0) attr_done[slot][algo - 1] = true;
   }
@@ -1466,8 +1519,8 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
     grid = want < cus8 ? want : cus8;
     if (grid < 8) grid = 8;
   }
-  gemm_fn fn = (al.fn_bias && p.bias) ? al.fn_bias : al.fn;
-  if (al.fn_sk && !p.bias && workspace != nullptr && grid <= kSkMaxGrid && workspace_bytes >= kSkFlagBytes + grid * kSkTileBytes) {
+  gemm_fn fn = (al.fn_add && add) ? al.fn_add : (al.fn_bias && p.bias) ? al.fn_bias : al.fn;
+  if (al.fn_sk && !p.bias && !add && workspace != nullptr && grid <= kSkMaxGrid && workspace_bytes >= kSkFlagBytes + grid * kSkTileBytes) {
     // the kernel decides per XCD (their tile counts differ by at most one) with the same test
     const int64_t W = grid / 8, KT = (K + 127) / 128, q = nblocks / 8;
     bool use = sk_pays(q, W, KT) || (nblocks % 8 != 0 && sk_pays(q + 1, W, KT));
@@ -1500,12 +1553,18 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
 extern "C" int l8_gemm_nt(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                           const float *sa, int sa_mode, const float *sb, int sb_mode, const void *bias, void *C,
                           int64_t ldc, int algo, void *stream) {
-  return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, bias, C, ldc, algo, nullptr, 0, stream);
+  return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, bias, C, ldc, 0, algo, nullptr, 0, stream);
+}
+
+extern "C" int l8_gemm_nt_add(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                              const float *sa, int sa_mode, const float *sb, int sb_mode, void *C, int64_t ldc, int algo,
+                              void *stream) {
+  return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, nullptr, C, ldc, 1, algo, nullptr, 0, stream);
 }
 
 extern "C" int l8_gemm_nt_ws(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                              const float *sa, int sa_mode, const float *sb, int sb_mode, const void *bias, void *C,
                              int64_t ldc, int algo, void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(workspace == nullptr || ((uintptr_t)workspace % 16) == 0, "l8_gemm_nt_ws: workspace must be 16-byte aligned");
-  return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, bias, C, ldc, algo, workspace, workspace_bytes, stream);
+  return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, bias, C, ldc, 0, algo, workspace, workspace_bytes, stream);
 }

@@ -77,7 +77,7 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
     L8_REQUIRE(a->w && a->y && a->K > 0 && a->K % 16 == 0 && a->ldw % 8 == 0 && a->ldw >= a->K && ((uintptr_t)a->w % 16) == 0 && a->ldy >= a->N,
                "l8_linear_fwd: K=%lld must be a multiple of 16, ldw=%lld of 8 and >= K, w 16-byte aligned, ldy >= N", (long long)a->K, (long long)a->ldw);
     return skinny_linear(SkinnyArgs{t.qx, a->w, (int)a->M, (int)a->N, (int)a->K, a->K, a->ldw, t.sx, nullptr, 1, 0,
-                                    (const uint16_t *)a->bias, (uint16_t *)a->y, a->ldy, scale_rule()}, true, (hipStream_t)a->stream);
+                                    (const uint16_t *)a->bias, (uint16_t *)a->y, a->ldy, scale_rule(), 0}, true, (hipStream_t)a->stream);
   }
   if (!a->w_ready) {
     rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);

@@ -14,6 +14,7 @@ struct SkinnyArgs {
   uint16_t *y;
   int64_t ldy;
   int scale_rule;
+  int add;              // y = bf16(bf16(product) + y)
 };
 
 constexpr int kSkinnyMaxM = 64;

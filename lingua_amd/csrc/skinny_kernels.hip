@@ -190,6 +190,11 @@ __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && MT > 2) ? 2 : 4)) void 
     if (p.bias) v[e] += bf16_bits_to_f32(p.bias[ne]);
   }
   uint16_t *dst = p.y + (int64_t)m * p.ldy + n;
+  if (p.add) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < p.N) v[e] = bf16_round(v[e]) + bf16_bits_to_f32(dst[e]);
+  }
   if (n + 4 <= p.N && (((uintptr_t)dst) & 7) == 0) {
     *(v2i *)dst = v2i{(int)(bf16_rne_bits(v[0]) | (bf16_rne_bits(v[1]) << 16)), (int)(bf16_rne_bits(v[2]) | (bf16_rne_bits(v[3]) << 16))};
   } else {

@@ -383,10 +383,10 @@ def input_cast_for_wgrad(a, a_col_amax, user):
 
 
 def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b: bool, need_bias: bool,
-                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None):
+                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None, grad_a=None):
     """Backward of lingua/float8.py:99-131 (fp8 wgrad optional).  Returns ``(grad_a, grad_b, grad_bias)`` with
     ``None`` where not needed.  ``a_tcast`` = ``(qat [K,M], sat [K,1])`` made in forward stands in for ``a``
-    (then ``a`` may be None; fp8 wgrad only)."""
+    (then ``a`` may be None; fp8 wgrad only).  ``grad_a``: a gradient of ``a`` that this one is added to, in place."""
     if grad_out.dtype != torch.bfloat16:
         raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {grad_out.dtype}")
     fp8_wgrad = fp8_wgrad and need_b
@@ -402,9 +402,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
         g_col_amax = torch.empty(grad_out.shape[1], dtype=torch.float32, device=grad_out.device) if fp8_wgrad else None
         qg, sg, _ = ops.cast_rowwise(grad_out, col_amax=g_col_amax)
         qb, sb = weight_cast_tensorwise_t(b_t, amax_b_t)
-        grad_a = ops.gemm_nt(qg, qb, sg, sb, None, algo=gemm_algo)
-    else:
-        grad_a = None
+        grad_a = ops.gemm_nt(qg, qb, sg, sb, None, algo=gemm_algo, out=grad_a, add=grad_a is not None)
 
     if need_b:
         if fp8_wgrad:

@@ -265,8 +265,10 @@ def release_gemm_workspaces() -> None:
 
 
 def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tensor,
-            bias: Optional[torch.Tensor] = None, algo: int = 0, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """bf16( (qa @ qb^T) * sa * sb^T + bias ).  qa [M,K], qb [N,K] fp8; sa [M,1]|[1,1], sb [N,1]|[1,1] fp32."""
+            bias: Optional[torch.Tensor] = None, algo: int = 0, out: Optional[torch.Tensor] = None,
+            add: bool = False) -> torch.Tensor:
+    """bf16( (qa @ qb^T) * sa * sb^T + bias ).  qa [M,K], qb [N,K] fp8; sa [M,1]|[1,1], sb [N,1]|[1,1] fp32.
+    ``add``: ``out`` += that product, both in bf16 (the bits of ``out.add_(product)``); no bias then."""
     qa = _rows_2d(qa, torch.float8_e4m3fn, "gemm_nt(A)")
     qb = _rows_2d(qb, torch.float8_e4m3fn, "gemm_nt(B)")
     st = _prep(qa, "gemm_nt")
@@ -284,15 +286,25 @@ def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tens
             raise RuntimeError("gemm_nt: bias must be bf16 with N elements")
         bias = bias.contiguous()
     user_out = out is not None
+    if add and (not user_out or bias is not None):
+        raise RuntimeError("gemm_nt: add needs out and takes no bias")
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=qa.device)
     elif out.dtype != torch.bfloat16 or out.shape != (M, N) or out.stride(1) != 1:
         raise RuntimeError("gemm_nt: out must be bf16 [M,N] with unit column stride")
+    ldc = _ld(out) if M > 1 else max(N, 1)
+    if add:
+        with _timed("gemm_nt", 2 * M * N * K, qa.device):
+            code = _lib.load().l8_gemm_nt_add(qa.data_ptr(), qb.data_ptr(), M, N, K, _ld(qa), _ld(qb), sa.data_ptr(), sa_mode,
+                                              sb.data_ptr(), sb_mode, out.data_ptr(), ldc, algo, st)
+        _lib.check(code, "l8_gemm_nt_add")
+        _wrote_into(out)
+        return out
     ws_ptr, ws_bytes = _gemm_workspace(qa.device, st, algo)
     with _timed("gemm_nt", 2 * M * N * K, qa.device):
         code = _lib.load().l8_gemm_nt_ws(qa.data_ptr(), qb.data_ptr(), M, N, K, _ld(qa), _ld(qb), sa.data_ptr(), sa_mode,
                                          sb.data_ptr(), sb_mode, bias.data_ptr() if bias is not None else None,
-                                         out.data_ptr(), _ld(out) if M > 1 else max(N, 1), algo, ws_ptr, ws_bytes, st)
+                                         out.data_ptr(), ldc, algo, ws_ptr, ws_bytes, st)
     _lib.check(code, "l8_gemm_nt_ws")
     if user_out:
         _wrote_into(out)

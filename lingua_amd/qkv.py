@@ -78,11 +78,8 @@ class Fp8QKVFn(torch.autograd.Function):
         for i, g in enumerate(grads):
             if g is None or not (ctx.need[0] or ctx.need[1 + i]):
                 continue
-            ga, gb, _ = f8.linear_backward(g.contiguous(), x, ws[i], amaxes[i], x_col, ctx.need[0], ctx.need[1 + i], False,
-                                           ctx.fp8_wgrad, ctx.gemm_algo)
-            gws[i] = gb
-            if ga is not None:
-                gx = ga if gx is None else gx.add_(ga)
+            gx, gws[i], _ = f8.linear_backward(g.contiguous(), x, ws[i], amaxes[i], x_col, ctx.need[0], ctx.need[1 + i], False,
+                                               ctx.fp8_wgrad, ctx.gemm_algo, grad_a=gx)
         return (gx, *gws)
 
 

@@ -105,7 +105,7 @@ class Fp8SwiGLUFn(torch.autograd.Function):
             qw1t, sw1t = f8.weight_cast_tensorwise_t(w1, amax_w1)
             gx = ops.gemm_nt(qg1, qw1t, sg1, sw1t, None, algo=algo)
             qw3t, sw3t = f8.weight_cast_tensorwise_t(w3, amax_w3)
-            gx += ops.gemm_nt(qg3, qw3t, sg3, sw3t, None, algo=algo)
+            ops.gemm_nt(qg3, qw3t, sg3, sw3t, None, algo=algo, out=gx, add=True)
         del qg1, qg3
         if need_w1 or need_w3:
             if fp8_wgrad:

@@ -94,6 +94,27 @@ def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
     assert name in ops.gemm_pick(*mnk)[1]
 
 
+@pytest.mark.parametrize("algo,mnk", [(0, (40, 52, 272)), (2, (130, 200, 144)), (2, (256, 256, 128)), (12, (256, 256, 128)),
+                                      (12, (300, 520, 400)), (12, (4136, 4104, 272)), (11, (520, 264, 144)), (17, (33, 50, 1040)),
+                                      (18, (128, 128, 256)), (21, (65, 70, 128))])
+def test_product_added_to_what_the_output_holds(algo, mnk):
+    """add=True leaves the bits of out.add_(product): every kernel's epilogue (interior and ragged tiles, a workgroup's
+    second tile, a configuration without an add of its own), an output with a row stride, nothing written beside it."""
+    from lingua_amd import ops
+    M, N, K = mnk
+    g = torch.Generator().manual_seed(900 + algo + M)
+    qa, qb = (random_fp8_bytes(s, g).cuda().view(torch.float8_e4m3fn) for s in ((M, K), (N, K)))
+    sa, sb = (torch.rand(M, 1, generator=g) + 0.5).cuda(), (torch.rand(1, 1, generator=g) + 0.5).cuda()
+    for sb_ in (sb, sb.expand(N, 1).contiguous()):
+        buf = (torch.randn(M, N + 16, generator=g) * 1e4).to(torch.bfloat16).cuda()
+        want = buf.clone()
+        want[:, 8:8 + N] += ops.gemm_nt(qa, qb, sa, sb_, algo=algo)
+        ops.gemm_nt(qa, qb, sa, sb_, algo=algo, out=buf[:, 8:8 + N], add=True)
+        assert torch.equal(buf.view(torch.int16), want.view(torch.int16))
+    with pytest.raises(RuntimeError, match="add needs out"):
+        ops.gemm_nt(qa, qb, sa, sb, algo=algo, add=True)
+
+
 @pytest.mark.parametrize("algo", [0, 1, 2, 3, 11, 15])
 def test_k_indexing_with_one_hot_operands(algo):
     # B[n] is one-hot at k = pi(n): C[m,n] = A[m, pi(n)] exactly, for any K (tails included)
