@@ -1319,7 +1319,7 @@ template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, 8>(const GemmArgs);
 
-constexpr int kSkinnyAlgo = 17;  // position in the list below
+static_assert(kSkinnyAlgo == 17, "position in the list below");
 static const Algo kAlgos[] = {
     L8_ALGO_LIST(L8_ALGO_ROW)
     /* 11, 12: persistent 256x256 tiles, 4 waves, one panel stream across tiles, C stored from the accumulators */
@@ -1466,7 +1466,7 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
   if (algo == kSkinnyAlgo) {
     if (skinny_serves(M, N, K, lda, ldb, 1))
       return skinny_linear(SkinnyArgs{A, B, (int)M, (int)N, (int)K, lda, ldb, sa, sb, sa_mode == L8_SCALE_ROW, sb_mode == L8_SCALE_ROW,
-                                      (const uint16_t *)bias, (uint16_t *)C, ldc, 0, add}, false, (hipStream_t)stream);
+                                      (const uint16_t *)bias, (uint16_t *)C, ldc, 0, add}, false, false, (hipStream_t)stream);
     algo = 2;
   }
   const Algo &al = kAlgos[algo - 1];

@@ -21,17 +21,22 @@ struct LinearFwd {
   void *qx, *qw, *col_ws;
   float *sx, *sw;
   int64_t col_ws_bytes;
-  bool w_on_the_way;  // the weight is quantised inside the product
+  bool w_on_the_way, x_on_the_way;  // quantised inside the product
 };
 
 static LinearFwd plan(const l8_linear_fwd_args &a, Pieces &ws) {
   LinearFwd t{};
-  t.qx = a.qx ? a.qx : ws.take(a.M * a.K);
-  t.sx = a.qx ? a.sx : (float *)ws.take(a.M * 4);
   // A few tokens and nobody who wants the weight's bytes or amaxes: one pass over the weight instead of three (read,
   // written, read).  us, weights cold, cast + product / one kernel: [1,4096].[11008,4096] 44 / 20.8, [7,4096].[4096,4096]
   // 25 / 10.4, [8,2048].[8192,2048] 20 / 12, [64,4096].[11008,4096] 54 / 28.
   t.w_on_the_way = !a.qw && !a.amax_w && a.algo == 0 && skinny_serves(a.M, a.N, a.K, a.K, a.ldw, 2);
+  const int w_bytes = t.w_on_the_way ? 2 : 1;
+  t.x_on_the_way = !a.qx && !a.col_amax_x && a.algo == 0 && a.K > 0 && skinny_quantises_x(a.M, a.N, a.K, a.ldx, w_bytes) &&
+                   (t.w_on_the_way || (skinny_serves(a.M, a.N, a.K, a.ldx, a.K, 1) && l8_gemm_pick(a.M, a.N, a.K) == kSkinnyAlgo));
+  if (!t.x_on_the_way) {
+    t.qx = a.qx ? a.qx : ws.take(a.M * a.K);
+    t.sx = a.qx ? a.sx : (float *)ws.take(a.M * 4);
+  }
   if (!t.w_on_the_way) {
     t.qw = a.qw ? a.qw : ws.take(a.N * a.K);
     t.sw = a.qw ? a.sw : (float *)ws.take(a.N * 4);
@@ -69,20 +74,27 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
   const LinearFwd t = plan(*a, ws);
   L8_REQUIRE(ws.used <= a->workspace_bytes && ((uintptr_t)a->workspace % 256) == 0,
              "l8_linear_fwd: needs a 256-byte aligned workspace of %lld bytes", (long long)ws.used);
-  if (!a->x_ready) {
+  if (!a->x_ready && !t.x_on_the_way) {
     rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, a->K, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
     if (rc != L8_OK) return rc;
   }
-  if (t.w_on_the_way) {
+  if (t.x_on_the_way || t.w_on_the_way) {
     L8_REQUIRE(a->w && a->y && a->K > 0 && a->K % 16 == 0 && a->ldw % 8 == 0 && a->ldw >= a->K && ((uintptr_t)a->w % 16) == 0 && a->ldy >= a->N,
                "l8_linear_fwd: K=%lld must be a multiple of 16, ldw=%lld of 8 and >= K, w 16-byte aligned, ldy >= N", (long long)a->K, (long long)a->ldw);
-    return skinny_linear(SkinnyArgs{t.qx, a->w, (int)a->M, (int)a->N, (int)a->K, a->K, a->ldw, t.sx, nullptr, 1, 0,
-                                    (const uint16_t *)a->bias, (uint16_t *)a->y, a->ldy, scale_rule(), 0}, true, (hipStream_t)a->stream);
+    if (t.x_on_the_way)
+      L8_REQUIRE(a->x && a->ldx % 8 == 0 && a->ldx >= a->K && ((uintptr_t)a->x % 16) == 0,
+                 "l8_linear_fwd: x must be 16-byte aligned, ldx=%lld a multiple of 8 and >= K", (long long)a->ldx);
+    if (!t.w_on_the_way) L8_REQUIRE(((uintptr_t)t.qw % 16) == 0, "l8_linear_fwd: qw must be 16-byte aligned");
   }
-  if (!a->w_ready) {
+  if (!t.w_on_the_way && !a->w_ready) {
     rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);
     if (rc != L8_OK) return rc;
   }
+  if (t.x_on_the_way || t.w_on_the_way)
+    return skinny_linear(SkinnyArgs{t.x_on_the_way ? a->x : t.qx, t.w_on_the_way ? a->w : t.qw, (int)a->M, (int)a->N, (int)a->K,
+                                    t.x_on_the_way ? a->ldx : a->K, t.w_on_the_way ? a->ldw : a->K, t.sx, t.sw, 1, 1,
+                                    (const uint16_t *)a->bias, (uint16_t *)a->y, a->ldy, scale_rule(), 0},
+                         t.w_on_the_way, t.x_on_the_way, (hipStream_t)a->stream);
   return l8_gemm_nt(t.qx, t.qw, a->M, a->N, a->K, a->K, a->K, t.sx, L8_SCALE_ROW, t.sw, L8_SCALE_ROW, a->bias, a->y, a->ldy,
                     (int)a->algo, a->stream);
 }

@@ -89,3 +89,29 @@ def test_weight_quantised_inside_the_product(M, K):
     ops.linear_fwd(x, w, bias, got)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and bool(torch.isnan(want[:, [7, 20]]).all())
     assert torch.equal(torch.nan_to_num(got.float()), torch.nan_to_num(want.float()))
+
+
+@pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("K", [16, 1040, 2048, 2064, 4096, 4112])
+@pytest.mark.parametrize("kept", [True, False])
+def test_tokens_quantised_inside_the_product(M, K, kept):
+    """A handful of tokens: every workgroup quantises them for itself, the weight kept quantised or not.  Rows of both
+    register budgets and past the last, padded row strides, a zero row, rows with an infinity or a NaN (NaN outputs);
+    the same bits as the casts and the product one by one."""
+    from lingua_amd import ops
+    N = 84
+    x = torch.zeros((M, K + 8), dtype=torch.bfloat16)[:, :K]
+    x.copy_(seeded_bf16((M, K), seed=M + K))
+    if M > 2:
+        x[1] = 0.0
+    if M > 4:
+        x[2, K - 1], x[M - 1, 0] = float("nan"), float("-inf")
+    x, w = x.cuda(), seeded_bf16((N, K), 0.02, seed=K).cuda()
+    bias = seeded_bf16((N,), seed=2).cuda()
+    qx, sx, _ = ops.cast_rowwise(x)
+    qw, sw, _ = ops.cast_rowwise(w)
+    want = ops.gemm_nt(qx, qw, sx, sw, bias)
+    got = torch.empty_like(want)
+    ops.linear_fwd(x, w, bias, got, w_cast=(qw, sw) if kept else None, w_ready=kept)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and (M <= 4 or bool(torch.isnan(want[[2, M - 1]]).all()))
+    assert torch.equal(torch.nan_to_num(got.float()), torch.nan_to_num(want.float()))
