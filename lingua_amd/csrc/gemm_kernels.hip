@@ -142,8 +142,10 @@ L8_DEV v4i add_bf16x8(v4i a, v4i b) {
 #define L8_WAIT_VM_LGKM0(n) \
   __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (0x7 << 4) | (0x0 << 8) | ((((n) >> 4) & 0x3) << 14))
 
-template <int WM, int WN, int TM, int TN, int R, int GROUP_M, int PF>
-__global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) {
+// KS > 1: KS groups of WM x WN waves, each with a ring of its own, take K tiles in turn (group g the tiles g, g + KS, ..)
+// and add their accumulators at the end, in the order of the groups.
+template <int WM, int WN, int TM, int TN, int R, int GROUP_M, int PF, int KS = 1>
+__global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr int BM = WM * TM * 32, BN = WN * TN * 32, BK = 128;
   constexpr int NW = WM * WN;
@@ -163,7 +165,8 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int group = KS > 1 ? wave_all / NW : 0, wave = KS > 1 ? wave_all % NW : wave_all;
   const int wm = wave / WN, wn = wave % WN;
 
   // ---- XCD-aware, grouped workgroup -> tile mapping ----
@@ -228,8 +231,8 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
   }
   const int chunk_even = (lpos ^ lrow) * 16, chunk_odd = (lpos ^ lrow ^ 1) * 16;  // byte offset in the row, by parity of g
 
-  const int KT = (p.K + BK - 1) / BK;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
+  const int KT = (p.K + BK * KS - 1) / (BK * KS);  // trips
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem + group * (R * UNIT);
   auto wrap = [](int slot) { return slot >= R ? slot - R : slot; };  // slot in [0, 2R)
   // Units are issued in the order A(0), B(0), A(1), B(1), ...; unit u lives in
   // ring slot u % R (the callers keep the slot numbers as running scalars).
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
   // tile kt (A or B panel) into ring slot `slot`: first the L2 touches, then
   // the 1 KiB panel loads.
   auto load_one = [&](bool is_b, int kt, int slot, int i) {
-    const int k0 = kt * BK;
+    const int k0 = (kt * KS + group) * BK;
     const uint32_t m_even = (k0 + chunk_even < p.K) ? 0u : kOOB, m_odd = (k0 + chunk_odd < p.K) ? 0u : kOOB;
     if (!is_b) {
       const uint32_t dst = lds0 + slot * UNIT + wave * (NA * 1024);
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
       // overwritten by the panel loads that follow (a wave's loads return in order)
       if (i < PFA)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, reinterpret_cast<lds_ptr_t>(dst), 4,
-                                                 pfa_voff[i < PFA ? i : 0] | ((k0 + PF * BK < p.K) ? 0u : kOOB), k0 + PF * BK, 0, 0);
+                                                 pfa_voff[i < PFA ? i : 0] | ((k0 + PF * KS * BK < p.K) ? 0u : kOOB), k0 + PF * KS * BK, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsA, reinterpret_cast<lds_ptr_t>(dst + (i - PFA) * 1024), 16,
                                                  a_voff[(i - PFA) & 1] | (((i - PFA) & 1) ? m_odd : m_even),
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
       const uint32_t dst = lds0 + slot * UNIT + wave * (NB * 1024);
       if (i < PFB)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, reinterpret_cast<lds_ptr_t>(dst), 4,
-                                                 pfb_voff[i < PFB ? i : 0] | ((k0 + PF * BK < p.K) ? 0u : kOOB), k0 + PF * BK, 0, 0);
+                                                 pfb_voff[i < PFB ? i : 0] | ((k0 + PF * KS * BK < p.K) ? 0u : kOOB), k0 + PF * KS * BK, 0, 0);
       else
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, reinterpret_cast<lds_ptr_t>(dst + (i - PFB) * 1024), 16,
                                                  b_voff[(i - PFB) & 1] | (((i - PFB) & 1) ? m_odd : m_even),
@@ -425,6 +428,41 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
   // before the ring is reused as the staging area of the C tile
   L8_WAIT_VM_LGKM0(0);
   __builtin_amdgcn_s_barrier();
+  if constexpr (KS > 1) {
+    // every group's ring is idle: the others leave their sums in theirs, the first group adds them to its own
+    static_assert(BM * BN * 4 <= R * UNIT, "a group's sums must fit in its ring");
+    typedef __attribute__((address_space(3))) v4f *lds_v4f_ptr;
+    constexpr int PIECE = NW * 64 * 16;
+    const uint32_t mine = lds0 + (wave * 64 + lane) * 16;
+    if (group > 0) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int qd = 0; qd < 4; ++qd)
+            *reinterpret_cast<lds_v4f_ptr>(mine + ((tn * TM + tm) * 4 + qd) * PIECE) =
+                v4f{acc[tn][tm][qd * 4], acc[tn][tm][qd * 4 + 1], acc[tn][tm][qd * 4 + 2], acc[tn][tm][qd * 4 + 3]};
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (group == 0) {
+#pragma unroll
+      for (int g = 1; g < KS; ++g)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int qd = 0; qd < 4; ++qd) {
+              const v4f t = *reinterpret_cast<lds_v4f_ptr>(mine + g * (R * UNIT) + ((tn * TM + tm) * 4 + qd) * PIECE);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[tn][tm][qd * 4 + e] += t[e];
+            }
+    }
+  }
 
   // lane (l31, h) of tile (tn, tm) holds m = l31 and, in accumulator quad qd,
   // n = 8*qd + 4*h + {0..3}.  After the half-wave swap, lanes with h == 0 hold
@@ -487,10 +525,13 @@ __global__ __launch_bounds__(WM *WN * 64) void gemm_nt_kernel(const GemmArgs p) 
     }
   }
   };
-  if (p.bias) convert_and_stage(std::true_type{});
-  else convert_and_stage(std::false_type{});
+  if (group == 0) {
+    if (p.bias) convert_and_stage(std::true_type{});
+    else convert_and_stage(std::false_type{});
+  }
   __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's part of the tile is in LDS
   __builtin_amdgcn_s_barrier();
+  if (group > 0) return;
   // 16-byte chunk c of the tile: row c / CPR, columns 8 * (c % CPR) .. +7
   constexpr int CPR = BN / 8, CHUNKS = BM * CPR;
   static_assert(CHUNKS % (NW * 64) == 0, "whole wave stores");
@@ -1289,23 +1330,38 @@ struct Algo {
   X(2, 2, 4, 4, 5, 16, 0) /* 9: algo 1 with groups of 16                      */ \
   X(2, 4, 4, 2, 5, 8, 0)  /* 10: algo 3 with taller groups                    */
 
-// 18 .. 21: small problems, one workgroup per compute unit or fewer: a ring of 9 slots (3.5 K tiles ahead instead of 1.5;
+// 18 .. 20: small problems, one workgroup per compute unit or fewer: a ring of 9 slots (3.5 K tiles ahead instead of 1.5;
 // a second workgroup has no use for the LDS) and smaller tiles where 128 x 128 ones would be too few
 #define L8_SMALL_ALGO_LIST(X)                         \
   X(2, 2, 2, 2, 9, 4, 0) /* 18: 128x128            */ \
   X(2, 2, 1, 2, 9, 4, 0) /* 19: 64x128             */ \
-  X(2, 2, 2, 1, 9, 4, 0) /* 20: 128x64             */ \
-  X(2, 2, 1, 1, 9, 4, 0) /* 21: 64x64              */
+  X(2, 2, 2, 1, 9, 4, 0) /* 20: 128x64             */
+
+// X(WM, WN, TM, TN, R, GROUP_M, KS): the smallest tiles, K tiles dealt to two groups of waves with a ring each.  A trip
+// costs them 310 ns whatever they load (wait, barrier, LDS reads, one or two matrix instructions in a row; a ring of 13 or
+// 19 slots changed nothing), so two trips run side by side.  us, weight just written, one group / two / four:
+// [333,8192].[2048,8192] 19.5 / 14.6 / 16.7, [100,11008].[4096,11008] 24.9 / 18.7 / 22.2, [200,4096].[4096,4096] 11.2 / 8.9 /
+// 9.3.  Larger tiles gain nothing: 128x128 [700,11008].[4096,11008] 39.2 / 39.7, 64x128 [1021,2048].[2048,2048] cold 9.3 / 9.9.
+#define L8_SPLIT_ALGO_LIST(X)                         \
+  X(2, 2, 1, 1, 9, 4, 2) /* 21: 64x64              */ \
+  X(1, 2, 1, 1, 9, 4, 2) /* 22: 32x64              */
 
 #define L8_INSTANTIATE(WM, WN, TM, TN, R, GM, PF) \
   template __global__ void gemm_nt_kernel<WM, WN, TM, TN, R, GM, PF>(const GemmArgs);
 L8_ALGO_LIST(L8_INSTANTIATE)
 L8_SMALL_ALGO_LIST(L8_INSTANTIATE)
+#define L8_SPLIT_INSTANTIATE(WM, WN, TM, TN, R, GM, KS) \
+  template __global__ void gemm_nt_kernel<WM, WN, TM, TN, R, GM, 0, KS>(const GemmArgs);
+L8_SPLIT_ALGO_LIST(L8_SPLIT_INSTANTIATE)
 
 #define L8_MAX2(a, b) ((a) > (b) ? (a) : (b))
 #define L8_ALGO_ROW(WM, WN, TM, TN, R, GM, PF)                                                                \
   {"mt" #WM "x" #WN "w_" #TM "x" #TN "t_r" #R "_g" #GM "_pf" #PF, gemm_nt_kernel<WM, WN, TM, TN, R, GM, PF>, \
    WM * TM * 32, WN * TN * 32, WM * WN * 64, R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr, nullptr},
+
+#define L8_SPLIT_ALGO_ROW(WM, WN, TM, TN, R, GM, KS)                                                               \
+  {"mt" #WM "x" #WN "w_" #TM "x" #TN "t_r" #R "_g" #GM "_ks" #KS, gemm_nt_kernel<WM, WN, TM, TN, R, GM, 0, KS>, \
+   WM * TM * 32, WN * TN * 32, WM * WN * KS * 64, KS * R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr, nullptr},
 
 template __global__ void gemm_nt_stream_kernel<8, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<8, true>(const GemmArgs);
@@ -1343,6 +1399,7 @@ static const Algo kAlgos[] = {
     /* 17: at most 64 tokens: 16 rows of B and all of A per workgroup, K split over its waves (skinny_kernels.hip) */
     {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr, nullptr},
     L8_SMALL_ALGO_LIST(L8_ALGO_ROW)
+    L8_SPLIT_ALGO_LIST(L8_SPLIT_ALGO_ROW)
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
 
@@ -1365,7 +1422,6 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // least one 256x256 tile per compute unit; groups of 4 tile rows ahead of groups of 8 by 1-3 %), also when
   // the big tiles leave up to 7/16 of the compute units idle (measured with K = 2048 .. 16384: 144 to 240
   // tiles on 256 compute units run 10-25 % faster than with 128x128 tiles, 128 tiles and fewer 15-45 % slower)
-  (void)K;
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   if (tiles(256, 256) * 16 >= cus * 9) return 12;
@@ -1373,11 +1429,16 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // [2048,2048] 4.2 / 7.5, [64,11008].[4096,11008] 18.9 / 28.8, [32,4096].[11008,4096] 14.6 / 13.5; from 48 tokens on
   // the 64 x 64 tiles win where there are enough of them ([48,4096].[11008,4096] 17.6 / 14.0, [40,4096].[8192,4096]
   // 12.2 / 12.1, [64,8192].[8192,8192] 25.3 / 23.5).
+  // With 9/16 of the units at work on 32 x 64 tiles, more than one tile of 16 tokens or rows beyond 4096 make the skinny
+  // kernels the slower ones (every workgroup reads all of x): [32,4096].[11008,4096] 14.4 / 13.0, [32,5120].[14336,5120]
+  // 24.6 / 17.1, [16,5120].[9216,5120] 15.8 / 13.7, but [16,4096].[11008,4096] 10.9 / 12.5, [32,4096].[8192,4096] 10.6 / 11.8.
+  const int64_t wide = tiles(32, 64);
+  if (M > 8 && M <= 32 && (M > 16 || K > 4096) && wide * 16 >= cus * 9 && wide <= cus) return 22;
   if (M <= 32 || (M <= kSkinnyMaxM && tiles(64, 64) * 16 < cus * 7)) return kSkinnyAlgo;
   // Otherwise the smallest tile that gives no compute unit a second workgroup: these kernels are bound by their LDS
   // traffic and by what a K tile costs whatever its size, so more units at work are worth more than the larger tile's
-  // economy.  us, 128 x 128 with two workgroups per unit (configuration 2) / chosen: [200,4096].[4096,4096] 19.1 / 11.9
-  // (64 x 64), [333,8192].[2048,8192] 32.8 / 19.5 (64 x 64), [1021,2048].[2048,2048] 12.3 / 9.3 (64 x 128),
+  // economy.  us, 128 x 128 with two workgroups per unit (configuration 2) / chosen: [200,4096].[4096,4096] 19.1 / 8.9
+  // (64 x 64), [333,8192].[2048,8192] 32.8 / 14.6 (64 x 64), [1021,2048].[2048,2048] 12.3 / 9.3 (64 x 128),
   // [512,4096].[4096,4096] 19.7 / 14.7 (128 x 64), [700,11008].[4096,11008] 67.2 / 49.5 (128 x 128, 9 slots),
   // [2048,16384].[2048,16384] 86.8 / 72.1 (the same).
   if (tiles(64, 64) <= cus) return 21;

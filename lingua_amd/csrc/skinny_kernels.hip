@@ -282,11 +282,11 @@ bool skinny_quantises_x(int64_t M, int64_t N, int64_t K, int64_t ldx, int w_byte
          (w_bytes == 1 || K <= 2 * kSkStep * kSkWaves || (N + 15) / 16 <= num_cus());
 }
 
-// How many steps a wave requests together (U): all of them where it has two, else four while the registers last.  us,
-// weights cold: [1,2048].[2048,2048] U = 2 / 4 3.4 / 3.9; [7,4096].[4096,4096] 5.8 / 5.4; [1,4096].[11008,4096] 10.6 / 9.3
-// (4.8 TB/s; 19.4 with 128 x 128 tiles); [32,4096].[11008,4096] 15.1 / 15.5 (19.6 with tiles), [32,11008].[4096,11008]
-// 15.3 / 15.1 (43.9); four token tiles U = 1 / 2: [64,4096].[11008,4096] 19.8 / 20.7 (19.6), [64,14336].[4096,14336]
-// 23.6 / 24.3 (57.4).
+// How many steps a wave requests together (U): all of them where it has two, else four while the registers last, one with
+// more tokens.  us, weights cold: [1,2048].[2048,2048] U = 2 / 4 3.4 / 3.9; [7,4096].[4096,4096] 5.8 / 5.4; [1,4096].
+// [11008,4096] 10.6 / 9.3 (4.8 TB/s; 19.4 with 128 x 128 tiles); two token tiles U = 1 / 2 / 4: [32,11008].[4096,11008]
+// 14.0 / 14.8 / 14.9 (43.9 with tiles), [32,4096].[4096,4096] 7.1 / 7.2 / 6.7, [17,2048].[8192,2048] 6.1 / 5.8 / 7.4; four
+// token tiles U = 1 / 2: [64,4096].[11008,4096] 19.8 / 20.7 (19.6), [64,14336].[4096,14336] 23.6 / 24.3 (57.4).
 int skinny_linear(const SkinnyArgs &p, bool w_is_bf16, bool x_is_bf16, hipStream_t st) {
   const int mt = (p.M + 15) / 16;
   const int steps = (p.K + kSkStep * kSkWaves - 1) / (kSkStep * kSkWaves);  // of a wave
@@ -305,7 +305,7 @@ int skinny_linear(const SkinnyArgs &p, bool w_is_bf16, bool x_is_bf16, hipStream
 #undef L8_SKINNY_Q
   }
   if (mt == 1) return steps <= 2 ? skinny_go<1, 2, 0, 0>(p, st) : skinny_go<1, 4, 0, 0>(p, st);
-  if (mt == 2) return skinny_go<2, 2, 0, 0>(p, st);
+  if (mt == 2) return steps <= 2 ? skinny_go<2, 2, 0, 0>(p, st) : skinny_go<2, 1, 0, 0>(p, st);
   if (mt == 3) return skinny_go<3, 1, 0, 0>(p, st);
   return skinny_go<4, 1, 0, 0>(p, st);
 }

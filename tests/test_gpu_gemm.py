@@ -67,10 +67,11 @@ def test_few_tokens_exact_on_integers_and_within_tolerance_of_the_oracle(M):
             assert rel_l2(out, oracle.gemm_nt(qa, qb, sa_, sb_, b_)) <= (TOL if M * N >= 5000 else 2.0 ** -8), (M, N, K)
 
 
-@pytest.mark.parametrize("algo,tile", [(18, (128, 128)), (19, (64, 128)), (20, (128, 64)), (21, (64, 64))])
+@pytest.mark.parametrize("algo,tile", [(18, (128, 128)), (19, (64, 128)), (20, (128, 64)), (21, (64, 64)), (22, (32, 64))])
 def test_small_tiles_exact_on_integers_at_their_edges(algo, tile):
     """The configurations for problems of at most one workgroup per compute unit: tiles full, one short and one over,
-    reductions from a ring that is never filled (K = 16) to one that wraps several times."""
+    reductions from a ring that is never filled (K = 16; a second group of waves without a K tile) to one that wraps
+    several times."""
     from lingua_amd import ops
     g = torch.Generator().manual_seed(800 + algo)
     bm, bn = tile
@@ -86,7 +87,8 @@ def test_small_tiles_exact_on_integers_at_their_edges(algo, tile):
 
 @pytest.mark.parametrize("mnk,name", [((200, 4096, 4096), "1x1t"), ((1021, 2048, 2048), "1x2t"), ((512, 4096, 4096), "1x2t"),
                                       ((2176, 960, 256), "2x1t"), ((2048, 2048, 4096), "2x2t_r9"), ((1500, 3008, 1440), "2x2t_r5"),
-                                      ((64, 11008, 4096), "1x1t"), ((16384, 2048, 2048), "stream")])
+                                      ((64, 11008, 4096), "mt2x2w_1x1t"), ((32, 11008, 4096), "mt1x2w_1x1t"), ((16, 11008, 4096), "skinny"),
+                                      ((9, 9216, 5120), "mt1x2w_1x1t"), ((8, 9216, 5120), "skinny"), ((32, 16448, 4096), "skinny"), ((16384, 2048, 2048), "stream")])
 def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
     from lingua_amd import ops
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
@@ -96,7 +98,7 @@ def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
 
 @pytest.mark.parametrize("algo,mnk", [(0, (40, 52, 272)), (2, (130, 200, 144)), (2, (256, 256, 128)), (12, (256, 256, 128)),
                                       (12, (300, 520, 400)), (12, (4136, 4104, 272)), (11, (520, 264, 144)), (17, (33, 50, 1040)),
-                                      (18, (128, 128, 256)), (21, (65, 70, 128))])
+                                      (18, (128, 128, 256)), (21, (65, 70, 128)), (22, (32, 64, 400))])
 def test_product_added_to_what_the_output_holds(algo, mnk):
     """add=True leaves the bits of out.add_(product): every kernel's epilogue (interior and ragged tiles, a workgroup's
     second tile, a configuration without an add of its own), an output with a row stride, nothing written beside it."""
