@@ -124,6 +124,13 @@ int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t ldx,
                        const void *amax, int amax_dtype, int transpose,
                        void *q, int64_t ldq, float *scale, void *stream);
 
+/* The transposed tensor-wise cast with the amax still to be found among amax_rows (bf16 [n], the row amaxes of x): equals
+ * l8_amax_reduce followed by l8_cast_tensorwise with transpose != 0, in one launch.
+ * Requires n % 8 == 0, n <= 16384 and 16-byte aligned amax_rows beside what l8_cast_tensorwise does. */
+int l8_cast_tensorwise_t_rows(const void *x, int64_t R, int64_t C, int64_t ldx,
+                              const void *amax_rows, int64_t n,
+                              void *q, int64_t ldq, float *scale, void *stream);
+
 /* Column-wise (token-dimension) scale -> cast, written transposed:
  * equals scale(x.t().contiguous(), its row amax) (lingua/float8.py:43-47 applied to
  * the operand layout an fp8 wgrad needs; the reference computes wgrad in bf16 at :123).
@@ -133,6 +140,12 @@ int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t ldx,
 int l8_cast_colwise_transposed(const void *x, int64_t R, int64_t C, int64_t ldx,
                                const float *col_amax,
                                void *q, int64_t ldq, float *scale, void *stream);
+
+/* The same with columns R .. Rp - 1 of q (Rp <= ldq) filled with zeros: a product that reduces over Rp rows is the one
+ * over R. */
+int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t C, int64_t ldx,
+                                   const float *col_amax,
+                                   void *q, int64_t ldq, int64_t Rp, float *scale, void *stream);
 
 /* Scaled fp8 product, both operands reduction-contiguous ("NT"):
  *   C[m,n] = bf16( (sum_k A[m,k]*B[n,k]) * sa[m or 0] * sb[n or 0] + bias[n] )

@@ -31,7 +31,9 @@ SIGNATURES = {
     "l8_col_amax": [_p, _i64, _i64, _i64, _p, _p],
     "l8_amax_reduce": [_p, _i64, _p, _p],
     "l8_cast_tensorwise": [_p, _i64, _i64, _i64, _p, _int, _int, _p, _i64, _p, _p],
+    "l8_cast_tensorwise_t_rows": [_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p],
     "l8_cast_colwise_transposed": [_p, _i64, _i64, _i64, _p, _p, _i64, _p, _p],
+    "l8_cast_colwise_transposed_pad": [_p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p],
     "l8_gemm_nt": [_p, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _p, _p, _i64, _int, _p],
     "l8_gemm_nt_ws": [_p, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _p, _p, _i64, _int, _p, _i64, _p],
     "l8_gemm_nt_add": [_p, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _p, _i64, _int, _p],

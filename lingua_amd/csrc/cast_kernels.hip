@@ -466,16 +466,27 @@ struct TransposeTile {
 };
 constexpr int kMaxTileRows = 256;                 // no tile is taller (bounds the row stride the host accepts)
 
-template <bool PER_COL, int TC, int TU>
+// Where the scale comes from: one amax, a column amax each, or one amax that every workgroup finds among the row amaxes
+// (a few kilobytes from the L2 under the tile's loads, where a reduction of its own is a launch).  Weights inside a forward
+// + backward, us, reduction + cast / this: [2048,2048] 4.7 + 4.7 / 5.2, [4096,14336] 4.8 + 33.6 / 34.7, [14336,4096]
+// 7.5 + 34.0 / 36.8.
+enum class AmaxFrom { kScalar, kColumns, kRows };
+constexpr int64_t kMaxAmaxRows = 16384;           // longest list that every workgroup reads
+
+// Columns R .. Rp - 1 of q are zeros: what a reduction over the tokens pads them to.  The rows are whole 16-byte pieces
+// then, also for an odd number of tokens: [4093,14336] 36.1 -> 33.9 us, [4093,4096] 13.6 -> 12.4, and no fill in front (5).
+template <AmaxFrom FROM, int TC, int TU>
 __global__ __launch_bounds__(256) void cast_transposed_kernel(
     const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, const void *__restrict__ amax_scalar, int amax_f32,
-    const uint32_t *__restrict__ col_amax, uint8_t *__restrict__ q, int64_t ldq, float *__restrict__ scale,
-    int vec_store, int scale_rule) {
+    const uint32_t *__restrict__ col_amax, const uint16_t *__restrict__ amax_rows, int n_amax, uint8_t *__restrict__ q,
+    int64_t ldq, int64_t Rp, float *__restrict__ scale, int vec_store, int scale_rule) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only
   using T = TransposeTile<TC, TU>;
+  constexpr bool PER_COL = FROM == AmaxFrom::kColumns, ROWS = FROM == AmaxFrom::kRows;
   constexpr int kTC = T::kTC, kCCH = T::kCCH, kRG = T::kRG, kTU = T::kTU, kTR = T::kTR, kTStride = T::kTStride;
   __shared__ __attribute__((aligned(16))) uint8_t tile[kTC * kTStride];
   __shared__ float recips[kTC];
+  __shared__ uint32_t wave_amax[4];
   const int t = threadIdx.x;
   // Workgroup w takes column block w % nct and row tile (w / nct + w % nct) % nrt:
   // a diagonal walk.  The workgroups resident at one time then touch addresses
@@ -485,7 +496,7 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
   // tiles (long runs in the output rows) and each row tile through consecutive
   // column blocks (wide bands of the input rows).
   const int nct = (C + kTC - 1) / kTC;
-  const int64_t nrt = (R + kTR - 1) / kTR;
+  const int64_t nrt = (Rp + kTR - 1) / kTR;
   const int cb = (int)(blockIdx.x % nct);
   const int64_t rt = (blockIdx.x / nct + cb) % nrt;
   const int64_t r0 = rt * kTR;
@@ -498,8 +509,20 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
   // scale(s) first, the tile right behind it.  The counter of outstanding loads retires in order, so the wait for
   // the amax leaves the tile's loads in flight, and the division and the reciprocal run under them.  (With a branch
   // around each load the compiler waited for all of them after the fifth and again before the division.)
-  uint32_t amax_lo, amax_hi = 0;
-  if (PER_COL) {
+  uint32_t amax_lo = 0, amax_hi = 0;
+  v4i listed[ROWS ? 4 : 1];
+  if constexpr (ROWS) {
+    const __amdgpu_buffer_rsrc_t rsList = make_rsrc(amax_rows, (uint32_t)n_amax * 2u);  // zeros beyond the list
+    for (int i0 = t * 8;; i0 += 4 * 256 * 8) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) listed[k] = __builtin_amdgcn_raw_buffer_load_b128(rsList, (i0 + k * 256 * 8) * 2, 0, 0);
+      if (i0 - t * 8 + 4 * 256 * 8 >= n_amax) break;  // the last four stay in flight under the tile's loads
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) amax_lo = pk_absmax_u16(amax_lo, (uint32_t)listed[k][w]);
+    }
+  } else if (PER_COL) {
     const __amdgpu_buffer_rsrc_t rsAmax = make_rsrc(col_amax, (uint32_t)C * 4u);
     amax_lo = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rsAmax, (c0 + t % kTC) * 4, 0, 0);  // zero beyond column C
   } else {
@@ -517,7 +540,7 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
   // dword).  The host keeps kTR * ldx * 2 below 2^30.
   const int64_t rows_left = R - r0;
   const uint32_t row_bytes = (uint32_t)ldx * 2u;
-  const uint32_t tile_bytes = (uint32_t)((rows_left < kTR ? (int)rows_left : kTR) - 1) * row_bytes + (uint32_t)C * 2u;
+  const uint32_t tile_bytes = rows_left <= 0 ? 0u : (uint32_t)((rows_left < kTR ? (int)rows_left : kTR) - 1) * row_bytes + (uint32_t)C * 2u;
   const __amdgpu_buffer_rsrc_t rsX = make_rsrc(x + r0 * ldx, tile_bytes);
   const uint32_t voff = (c < C ? (uint32_t)c * 2u : tile_bytes) + (uint32_t)(rg * 4) * row_bytes;
   v4i in[kTU][4];
@@ -538,6 +561,16 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
       recips[t] = rc;
     }
     __syncthreads();
+  }
+  if constexpr (ROWS) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) amax_lo = pk_absmax_u16(amax_lo, (uint32_t)listed[k][w]);
+    const uint32_t m = wave_max_u32(max(amax_lo & 0xffffu, amax_lo >> 16));
+    if ((t & 63) == 0) wave_amax[t >> 6] = m;
+    __syncthreads();
+    amax_lo = max(max(wave_amax[0], wave_amax[1]), max(wave_amax[2], wave_amax[3]));
   }
   float rcp[8];
   bool finite = true;
@@ -589,8 +622,7 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
       uint32_t packed = 0;
       for (int i = 0; i < 4; ++i) {
         const int64_t r = r0 + (u * kRG + rg) * 4 + i;
-        const uint32_t h = (r < R && c + j < C) ? x[r * ldx + c + j] : 0u;
-        packed |= e4m3fn_from_f32_slow(bf16_bits_to_f32(h) * rc) << (8 * i);
+        if (r < R && c + j < C) packed |= e4m3fn_from_f32_slow(bf16_bits_to_f32(x[r * ldx + c + j]) * rc) << (8 * i);
       }
       *(uint32_t *)(tile + (cc * 8 + j) * kTStride + (u * kRG + rg) * 4) = packed;
     }
@@ -605,14 +637,14 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
     const int seg = idx % SEGS;
     const int col = c0 + oc;
     const int64_t r = r0 + seg * 16;
-    if (col < C && r < R) {
+    if (col < C && r < Rp) {
       const v4i v = *(const v4i *)(tile + oc * kTStride + seg * 16);
       uint8_t *dst = q + (int64_t)col * ldq + r;
-      if (vec_store && r + 16 <= R) {
+      if (vec_store && r + 16 <= Rp) {
         *(v4i *)dst = v;  // not a streaming store: see the note on the tile shapes
       } else {
         const uint8_t *src = tile + oc * kTStride + seg * 16;
-        for (int b = 0; b < 16 && r + b < R; ++b) dst[b] = src[b];
+        for (int b = 0; b < 16 && r + b < Rp; ++b) dst[b] = src[b];
       }
     }
   }
@@ -853,36 +885,56 @@ extern "C" int l8_amax_reduce(const void *amax, int64_t n, void *amax_out, void 
   return L8_OK;
 }
 
+// What a transposed cast is asked for: one of amax (bf16 or fp32 scalar), col_amax and amax_rows is set.
+struct TransposedCast {
+  const void *x;
+  int64_t R, C, ldx;
+  const void *amax;
+  int amax_f32;
+  const float *col_amax;
+  const void *amax_rows;
+  int64_t n_amax;
+  void *q;
+  int64_t ldq, Rp;
+  float *scale;
+};
+
 template <int TC, int TU>
-static int launch_transposed_tile(bool per_col, const void *x, int64_t R, int64_t C, int64_t ldx, const void *amax,
-                                  int amax_f32, const float *col_amax, void *q, int64_t ldq, float *scale, hipStream_t st) {
+static int launch_transposed_tile(const TransposedCast &a, hipStream_t st) {
   using T = TransposeTile<TC, TU>;
   static_assert(T::kTR <= kMaxTileRows, "the row-stride limit assumes no taller tile");
-  const int64_t gx = ((C + T::kTC - 1) / T::kTC) * ((R + T::kTR - 1) / T::kTR);
-  L8_REQUIRE(gx < (1LL << 31), "transposed cast: shape too large (%lld x %lld)", (long long)R, (long long)C);
-  const int vec = (ldq % 16 == 0 && aligned(q, 16)) ? 1 : 0;
-  if (per_col)
-    hipLaunchKernelGGL((cast_transposed_kernel<true, TC, TU>), dim3((unsigned)gx), dim3(256), 0, st,
-                       (const uint16_t *)x, R, (int)C, ldx, (const void *)nullptr, 0, (const uint32_t *)col_amax,
-                       (uint8_t *)q, ldq, scale, vec, l8::scale_rule());
-  else
-    hipLaunchKernelGGL((cast_transposed_kernel<false, TC, TU>), dim3((unsigned)gx), dim3(256), 0, st,
-                       (const uint16_t *)x, R, (int)C, ldx, amax, amax_f32, (const uint32_t *)nullptr,
-                       (uint8_t *)q, ldq, scale, vec, l8::scale_rule());
+  const int64_t gx = ((a.C + T::kTC - 1) / T::kTC) * ((a.Rp + T::kTR - 1) / T::kTR);
+  L8_REQUIRE(gx < (1LL << 31), "transposed cast: shape too large (%lld x %lld)", (long long)a.R, (long long)a.C);
+  const int vec = (a.ldq % 16 == 0 && aligned(a.q, 16)) ? 1 : 0;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gx), dim3(256), 0, st, (const uint16_t *)a.x, a.R, (int)a.C, a.ldx, a.amax, a.amax_f32,
+                       (const uint32_t *)a.col_amax, (const uint16_t *)a.amax_rows, (int)a.n_amax, (uint8_t *)a.q, a.ldq, a.Rp, a.scale,
+                       vec, l8::scale_rule());
+  };
+  if (a.col_amax) go(cast_transposed_kernel<AmaxFrom::kColumns, TC, TU>);
+  else if (a.amax_rows) go(cast_transposed_kernel<AmaxFrom::kRows, TC, TU>);
+  else go(cast_transposed_kernel<AmaxFrom::kScalar, TC, TU>);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
 
-static int launch_transposed(bool per_col, const void *x, int64_t R, int64_t C, int64_t ldx, const void *amax,
-                             int amax_f32, const float *col_amax, void *q, int64_t ldq, float *scale, hipStream_t st) {
+static int launch_transposed(const TransposedCast &a, hipStream_t st) {
   // a tile's rows within 1 GiB: then no sum of a lane's offset (up to twice the tile) and a row's scalar offset wraps
-  L8_REQUIRE((int64_t)kMaxTileRows * ldx * 2 < (1LL << 30), "transposed cast: row stride too large (%lld elements)", (long long)ldx);
-  const int64_t tiles128 = ((C + 127) / 128) * ((R + 127) / 128);
+  L8_REQUIRE((int64_t)kMaxTileRows * a.ldx * 2 < (1LL << 30), "transposed cast: row stride too large (%lld elements)", (long long)a.ldx);
+  const int64_t tiles128 = ((a.C + 127) / 128) * ((a.R + 127) / 128);
   if (tiles128 < 4 * (int64_t)num_cus())  // too few 128 x 128 tiles for four workgroups per compute unit
-    return launch_transposed_tile<64, 1>(per_col, x, R, C, ldx, amax, amax_f32, col_amax, q, ldq, scale, st);
-  if (R >= 16384 && C >= 8192)  // the large activations: see the note on the tile shapes
-    return launch_transposed_tile<128, 4>(per_col, x, R, C, ldx, amax, amax_f32, col_amax, q, ldq, scale, st);
-  return launch_transposed_tile<128, 2>(per_col, x, R, C, ldx, amax, amax_f32, col_amax, q, ldq, scale, st);
+    return launch_transposed_tile<64, 1>(a, st);
+  if (a.R >= 16384 && a.C >= 8192)  // the large activations: see the note on the tile shapes
+    return launch_transposed_tile<128, 4>(a, st);
+  return launch_transposed_tile<128, 2>(a, st);
+}
+
+static int check_transposed(const char *what, const TransposedCast &a) {
+  L8_REQUIRE(a.x && a.q, "%s: null pointer", what);
+  L8_REQUIRE(a.C % 8 == 0 && a.ldx % 8 == 0 && a.ldx >= a.C && aligned(a.x, 16), "%s: C, ldx multiples of 8 and x 16-byte aligned required", what);
+  L8_REQUIRE(a.C < (1LL << 31), "%s: C too large", what);
+  L8_REQUIRE(a.Rp >= a.R && a.ldq >= a.Rp, "%s: transposed output needs ldq >= R and its padding", what);
+  return L8_OK;
 }
 
 extern "C" int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t ldx, const void *amax, int amax_dtype,
@@ -898,7 +950,7 @@ extern "C" int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t l
   hipStream_t st = (hipStream_t)stream;
   if (transpose) {
     L8_REQUIRE(ldq >= R, "l8_cast_tensorwise: transposed output needs ldq >= R");
-    return launch_transposed(false, x, R, C, ldx, amax, amax_dtype, nullptr, q, ldq, scale, st);
+    return launch_transposed(TransposedCast{x, R, C, ldx, amax, amax_dtype, nullptr, nullptr, 0, q, ldq, R, scale}, st);
   }
   L8_REQUIRE(ldq >= C && ldq % 8 == 0 && aligned(q, 8), "l8_cast_tensorwise: q must be 8-byte aligned with ldq %% 8 == 0, ldq >= C");
   const int64_t total = R * (C / 8);
@@ -911,15 +963,36 @@ extern "C" int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t l
   return L8_OK;
 }
 
+// The weight of dgrad with the row amaxes that forward left: bf16 amax_rows[n], as l8_amax_reduce and l8_cast_tensorwise
+// would take it.
+extern "C" int l8_cast_tensorwise_t_rows(const void *x, int64_t R, int64_t C, int64_t ldx, const void *amax_rows, int64_t n, void *q,
+                                         int64_t ldq, float *scale, void *stream) {
+  L8_REQUIRE(R >= 0 && C >= 0, "l8_cast_tensorwise_t_rows: negative shape");
+  L8_REQUIRE(amax_rows && scale && n >= 8 && n <= kMaxAmaxRows && n % 8 == 0 && aligned(amax_rows, 16),
+             "l8_cast_tensorwise_t_rows: 16-byte aligned amaxes, a multiple of 8 of them and at most %lld, required", (long long)kMaxAmaxRows);
+  if (R == 0 || C == 0) return L8_OK;
+  const TransposedCast a{x, R, C, ldx, nullptr, 0, nullptr, amax_rows, n, q, ldq, R, scale};
+  const int rc = check_transposed("l8_cast_tensorwise_t_rows", a);
+  return rc == L8_OK ? launch_transposed(a, (hipStream_t)stream) : rc;
+}
+
+static int cast_colwise(const char *what, const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax, void *q,
+                        int64_t ldq, int64_t Rp, float *scale, void *stream) {
+  L8_REQUIRE(R >= 0 && C >= 0, "%s: negative shape", what);
+  if (C == 0) return L8_OK;
+  L8_REQUIRE(col_amax && scale, "%s: col_amax and scale must be non-null", what);
+  L8_REQUIRE(R > 0, "%s: R must be positive when C > 0", what);
+  const TransposedCast a{x, R, C, ldx, nullptr, 0, col_amax, nullptr, 0, q, ldq, Rp, scale};
+  const int rc = check_transposed(what, a);
+  return rc == L8_OK ? launch_transposed(a, (hipStream_t)stream) : rc;
+}
+
 extern "C" int l8_cast_colwise_transposed(const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax,
                                           void *q, int64_t ldq, float *scale, void *stream) {
-  L8_REQUIRE(R >= 0 && C >= 0, "l8_cast_colwise_transposed: negative shape");
-  if (C == 0) return L8_OK;
-  L8_REQUIRE(col_amax && scale, "l8_cast_colwise_transposed: col_amax and scale must be non-null");
-  L8_REQUIRE(R > 0, "l8_cast_colwise_transposed: R must be positive when C > 0");
-  L8_REQUIRE(x && q, "l8_cast_colwise_transposed: null pointer");
-  L8_REQUIRE(C % 8 == 0 && ldx % 8 == 0 && ldx >= C && aligned(x, 16), "l8_cast_colwise_transposed: C, ldx multiples of 8 and x 16-byte aligned required");
-  L8_REQUIRE(ldq >= R, "l8_cast_colwise_transposed: ldq >= R required");
-  L8_REQUIRE(C < (1LL << 31), "l8_cast_colwise_transposed: C too large");
-  return launch_transposed(true, x, R, C, ldx, nullptr, 0, col_amax, q, ldq, scale, (hipStream_t)stream);
+  return cast_colwise("l8_cast_colwise_transposed", x, R, C, ldx, col_amax, q, ldq, R, scale, stream);
+}
+
+extern "C" int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax,
+                                              void *q, int64_t ldq, int64_t Rp, float *scale, void *stream) {
+  return cast_colwise("l8_cast_colwise_transposed_pad", x, R, C, ldx, col_amax, q, ldq, Rp, scale, stream);
 }

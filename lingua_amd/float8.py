@@ -258,7 +258,7 @@ class _WeightCasts:
         slot = self._slot(w) if config.cache_weight_casts else None
         if slot is not None and "tw" in slot:
             return slot["tw"]
-        value = ops.cast_tensorwise(w, ops.amax_reduce(amax_rows), transpose=True)
+        value = ops.cast_tensorwise_t_rows(w, amax_rows)
         if slot is not None:
             slot["tw"] = value
         return value

@@ -197,6 +197,28 @@ def cast_tensorwise(x: torch.Tensor, amax: torch.Tensor, transpose: bool = False
     return q, scale
 
 
+# Longest list of row amaxes that the transposed cast reduces itself; see l8_cast_tensorwise_t_rows.
+_MAX_AMAX_ROWS = 16384
+
+
+def cast_tensorwise_t_rows(x: torch.Tensor, amax_rows: torch.Tensor):
+    """``cast_tensorwise(x, amax_reduce(amax_rows), transpose=True)``, in one launch where the list allows it."""
+    x = _rows_2d(x, torch.bfloat16, "cast_tensorwise_t_rows")
+    n = amax_rows.numel()
+    if (amax_rows.dtype != torch.bfloat16 or amax_rows.device != x.device or not amax_rows.is_contiguous() or n % 8 or
+            not 0 < n <= _MAX_AMAX_ROWS or amax_rows.data_ptr() % 16):
+        return cast_tensorwise(x, amax_reduce(amax_rows), transpose=True)
+    st = _prep(x, "cast_tensorwise_t_rows")
+    R, C = x.shape
+    q = torch.empty((C, R), dtype=torch.float8_e4m3fn, device=x.device)
+    scale = torch.empty((1, 1), dtype=torch.float32, device=x.device)
+    with _timed("cast_tensorwise_t", R * C * 3 + 2 * n + 4, x.device):
+        code = _lib.load().l8_cast_tensorwise_t_rows(x.data_ptr(), R, C, _ld(x), amax_rows.data_ptr(), n, q.data_ptr(), max(R, 1),
+                                                     scale.data_ptr(), st)
+    _lib.check(code, "l8_cast_tensorwise_t_rows")
+    return q, scale
+
+
 def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to: int = 16):
     """scale(x.t().contiguous(), its row amax): returns (q [C,Rp] fp8, scale [C,1] fp32).
 
@@ -215,13 +237,11 @@ def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to:
         return q, (torch.clamp(col_amax_f32, min=1e-12) / 448.0).reshape(C, 1)
     Rp = (R + pad_to - 1) // pad_to * pad_to
     q = torch.empty((C, Rp), dtype=torch.float8_e4m3fn, device=x.device)
-    if Rp != R:
-        q.view(torch.uint8)[:, R:].zero_()   # the kernel writes columns 0 .. R-1; only the padding is filled here
     scale = torch.empty((C, 1), dtype=torch.float32, device=x.device)
     with _timed("cast_colwise_t", R * C * 3 + 4 * C, x.device):
-        code = _lib.load().l8_cast_colwise_transposed(x.data_ptr(), R, C, _ld(x), col_amax_f32.data_ptr(),
-                                                      q.data_ptr(), max(Rp, 1), scale.data_ptr(), st)
-    _lib.check(code, "l8_cast_colwise_transposed")
+        code = _lib.load().l8_cast_colwise_transposed_pad(x.data_ptr(), R, C, _ld(x), col_amax_f32.data_ptr(),
+                                                          q.data_ptr(), max(Rp, 1), Rp, scale.data_ptr(), st)
+    _lib.check(code, "l8_cast_colwise_transposed_pad")
     return q, scale
 
 

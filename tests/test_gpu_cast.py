@@ -413,3 +413,36 @@ def test_casts_under_the_gpu_division_rule_equal_pytorchs_own_gpu_ops(shape, gpu
         q_t, s_t = rt.scale(xt if transpose else xd, amax)
         cols = shape[0] if transpose else shape[1]
         assert bits_equal(q[:, :cols].contiguous().view(torch.uint8), q_t.view(torch.uint8)) and bits_equal(s.reshape(-1), s_t.reshape(-1))
+
+
+@pytest.mark.parametrize("N,K", [(8, 16), (16, 272), (2048, 72), (2056, 2048), (8192, 136), (8200, 64), (16384, 8), (16392, 64)])
+def test_transposed_cast_finds_the_amax_among_the_row_amaxes(N, K):
+    """The dgrad weight quantised straight from its row amaxes: lists of one to eight loads per thread and past the last
+    length, the largest amax in the first and last row, an infinity and a NaN; the bytes of reduction + cast."""
+    from lingua_amd import ops
+    w = seeded_bf16((N, K), 0.02, seed=N).cuda()
+    for row, value in ((0, 3.0), (N - 1, -5.0), (N // 2, float("inf")), (N - 3, float("nan"))):
+        w[row, K - 1] = value
+        amax = ops.cast_rowwise(w, want_q=False)[2]
+        q, s = ops.cast_tensorwise_t_rows(w, amax)
+        wq, ws = ops.cast_tensorwise(w, ops.amax_reduce(amax), transpose=True)
+        assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8)), (N, K, value)
+        assert torch.equal(s.view(torch.int32), ws.view(torch.int32)), (N, K, value)
+
+
+@pytest.mark.parametrize("R", [1, 15, 16, 17, 63, 65, 127, 129, 1021])
+@pytest.mark.parametrize("pad_to", [16, 48, 512])
+def test_transposed_cast_pads_with_zeros(R, pad_to):
+    """Columns beyond the rows of x are zeros -- also under a column whose amax is infinite or NaN, and in tiles that hold
+    nothing else -- and the rest is what the unpadded cast writes."""
+    from lingua_amd import ops
+    for C in (8, 200):
+        x = seeded_bf16((R, C), seed=R + C)
+        x[R - 1, 3], x[0, C - 1] = float("inf"), float("nan")
+        xd = x.cuda()
+        torch.full((C * (R + pad_to),), 0x55, dtype=torch.uint8, device="cuda")  # what the allocator hands out next is not zero
+        q, s = ops.cast_colwise_transposed(xd, ops.col_amax(xd), pad_to=pad_to)
+        wq, ws = oracle.cast_colwise_transposed(x)
+        assert q.shape == (C, (R + pad_to - 1) // pad_to * pad_to)
+        assert torch.equal(q.cpu().view(torch.uint8)[:, :R], wq) and not q.view(torch.uint8)[:, R:].any()
+        assert torch.equal(s.cpu().reshape(-1).view(torch.int32), ws.reshape(-1).view(torch.int32))
