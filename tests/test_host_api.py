@@ -61,17 +61,20 @@ def test_linear_call_validates_its_arguments_on_the_host():
     workspace it asks for covers exactly the members that are left to it."""
     lib = _lib.load()
     fake = 1 << 20
-    base = dict(x=fake, M=32, K=64, ldx=64, w=fake, N=48, ldw=64, bias=0, y=fake, ldy=48, qx=0, sx=0, col=0, x_ready=0, qw=0,
+    base = dict(x=fake, M=80, K=64, ldx=64, w=fake, N=48, ldw=64, bias=0, y=fake, ldy=48, qx=0, sx=0, col=0, x_ready=0, qw=0,
                 sw=0, amax_w=0, w_ready=0, algo=0, ws=0, ws_bytes=0, stream=0)
 
     def pack(**kw):
         return ops._FWD.pack(*dict(base, **kw).values())
 
     full = lib.l8_linear_fwd_workspace(pack())
-    assert full >= 32 * 64 + 32 * 4 + 48 * 64 + 48 * 4
+    assert full >= 80 * 64 + 80 * 4 + 48 * 64 + 48 * 4
     assert lib.l8_linear_fwd_workspace(pack(qw=fake, sw=fake, w_ready=1)) < full
     assert lib.l8_linear_fwd_workspace(pack(qx=fake, sx=fake)) < full
     assert lib.l8_linear_fwd_workspace(pack(col=fake)) > full
+    # up to 64 tokens the weight is quantised inside the product, up to 8 the tokens too: nothing to put anywhere
+    assert 32 * 64 + 32 * 4 <= lib.l8_linear_fwd_workspace(pack(M=32)) < lib.l8_linear_fwd_workspace(pack(M=32, amax_w=fake))
+    assert lib.l8_linear_fwd_workspace(pack(M=8)) == 0 < lib.l8_linear_fwd_workspace(pack(M=9))
     assert lib.l8_linear_fwd(pack()) == -1 and "workspace" in _lib.last_error()
     assert lib.l8_linear_fwd(pack(M=-1)) == -1 and lib.l8_linear_fwd_workspace(pack(M=-1)) == -1
     assert lib.l8_linear_fwd(pack(x_ready=1)) == -1 and "x_ready" in _lib.last_error()
