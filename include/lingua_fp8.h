@@ -73,6 +73,18 @@ int l8_get_scale_rule(void);
 int l8_cast_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx,
                     void *q, int64_t ldq, float *scale, void *amax, float *col_amax,
                     void *workspace, int64_t workspace_bytes, void *stream);
+
+/* The same for n operands of one width C, without column amaxes: one launch for up to three of them where C <= 16384, else
+ * as n calls.  Every operand needs x, q and scale; amax may be NULL. */
+typedef struct {
+  const void *x;
+  int64_t R, ldx;
+  void *q;
+  int64_t ldq;
+  float *scale;
+  void *amax;
+} l8_cast_rowwise_item;
+int l8_cast_rowwise_many(const l8_cast_rowwise_item *items, int64_t n, int64_t C, void *stream);
 int64_t l8_cast_rowwise_workspace(int64_t R, int64_t C);
 
 /* l8_cast_rowwise for callers that cannot allocate device memory (code under HIP graph capture, tight

@@ -6,6 +6,7 @@
 // read + 1 byte written; every kernel here reads each input byte from HBM once.
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "l8_common.h"
 
@@ -36,10 +37,49 @@ L8_DEV void load_row(v4i (&buf)[NCH], const uint16_t *x, int64_t r, int64_t R, i
 }
 #endif
 
-template <int NCH, bool COLMAX>
+// Several operands of one width as one list of rows: row r of the launch is row r - first of the operand that holds it.
+// What a linear quantises together (activation and weight, the weights of projections that share an input) takes one
+// launch, whose rows are in flight together, instead of one per operand that each fill and drain the chip.  us, one by one /
+// together: [4096,2048] and [2048,2048] 6.6 + 6.2 / 10.9, [333,2048] and [8192,2048] 3.5 + 13.8 / 13.4, three [2048,2048]
+// weights 5.2 + 4.9 + 4.9 / 9.0.
+constexpr int kMaxRowOperands = 3;
+constexpr int64_t kMaxRowwiseManyColumns = 8 * 4 * 512;  // eight chunks per lane of a workgroup
+struct RowOperand {
+  const uint16_t *x;
+  int64_t first, ldx;  // first row in the list; the operands are in order
+  uint8_t *q;
+  int64_t ldq;
+  float *scale;
+  uint16_t *amax;
+};
+struct RowOperands {
+  RowOperand op[kMaxRowOperands];  // unused ones start beyond the last row
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+L8_DEV RowOperand operand_of(const RowOperands &list, int64_t r) {
+  RowOperand o = list.op[0];
+#pragma unroll
+  for (int i = 1; i < kMaxRowOperands; ++i) {  // member by member: a copy of the whole would live in scratch memory
+    const RowOperand &t = list.op[i];
+    const bool here = r >= t.first;
+    o.x = here ? t.x : o.x;
+    o.first = here ? t.first : o.first;
+    o.ldx = here ? t.ldx : o.ldx;
+    o.q = here ? t.q : o.q;
+    o.ldq = here ? t.ldq : o.ldq;
+    o.scale = here ? t.scale : o.scale;
+    o.amax = here ? t.amax : o.amax;
+  }
+  return o;
+}
+#endif
+
+// MANY: the operands come from `list`, R counts the rows of all of them and x .. amax_out are not used.
+template <int NCH, bool COLMAX, bool MANY = false>
 __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
     const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint8_t *__restrict__ q, int64_t ldq,
-    float *__restrict__ scale, uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule) {
+    float *__restrict__ scale, uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule,
+    const std::conditional_t<MANY, RowOperands, int> list) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer descriptors exist in the device pass only
   extern __shared__ uint32_t lds_colmax[];  // [C/2] packed bf16 pairs when COLMAX
   // the next row is prefetched into a second register set unless that would
@@ -49,6 +89,15 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register: the row descriptors hang on it
   const int64_t wave_stride = (int64_t)gridDim.x * kRowWaves;
   int64_t r = (int64_t)blockIdx.x * kRowWaves + wave;
+  auto load = [&](auto &buf, int64_t row) {
+    constexpr int N = sizeof(buf) / sizeof(buf[0]);
+    if constexpr (MANY) {
+      const RowOperand op = operand_of(list, row);
+      load_row<N>(buf, op.x - op.first * op.ldx, row, R, op.ldx, C, lane);
+    } else {
+      load_row<N>(buf, x, row, R, ldx, C, lane);
+    }
+  };
 
   uint32_t cmax[COLMAX ? NCH * 4 : 1];
   if (COLMAX) {
@@ -57,11 +106,11 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
   }
 
   v4i cur[NCH];
-  load_row<NCH>(cur, x, r, R, ldx, C, lane);
+  load(cur, r);
   while (r < R) {
     const int64_t rn = r + wave_stride;
     v4i nxt[PREFETCH ? NCH : 1];
-    if (PREFETCH) load_row<PREFETCH ? NCH : 1>(nxt, x, rn, R, ldx, C, lane);
+    if (PREFETCH) load(nxt, rn);
 
     // row amax on packed pairs
     uint32_t m = 0;
@@ -84,26 +133,36 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
       s = __uint_as_float(0x7fc00000u);  // NaN amax -> NaN scale
     }
     const float recip = recip_exact(s);
-    if (lane == 0) {
+    const uint16_t *xrow = x + r * ldx;
+    uint8_t *qrow = q ? q + r * ldq : nullptr;
+    if constexpr (MANY) {
+      const RowOperand cur_op = operand_of(list, r);
+      const int64_t ro = r - cur_op.first;
+      xrow = cur_op.x + ro * cur_op.ldx;
+      qrow = cur_op.q + ro * cur_op.ldq;
+      if (lane == 0) {
+        cur_op.scale[ro] = s;
+        if (cur_op.amax) cur_op.amax[ro] = (uint16_t)amax_bits;
+      }
+    } else if (lane == 0) {
       if (scale) scale[r] = s;
       if (amax_out) amax_out[r] = (uint16_t)amax_bits;
     }
-    uint8_t *qrow = q ? q + r * ldq : nullptr;
-    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(qrow, q ? (uint32_t)C : 0u);  // stores beyond column C, or without q, are dropped
+    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(qrow, MANY || q ? (uint32_t)C : 0u);  // stores beyond column C, or without q, are dropped
 #pragma unroll
     for (int j = 0; j < NCH; ++j) store8(rsQ, (uint32_t)(j * 512 + lane * 8), cvt8(cur[j], recip));
-    if (q && !finite) {
+    if ((MANY || q) && !finite) {
       // a row with a non-finite amax: redone from memory with the integer conversion, replacing the bytes above (one
       // small loop beside the common path instead of NCH unrolled copies of that conversion inside it)
 #pragma unroll 1
-      for (int c = lane * 8; c < C; c += 512) *(v2i *)(qrow + c) = cvt8_slow(*(const v4i *)(x + r * ldx + c), recip);
+      for (int c = lane * 8; c < C; c += 512) *(v2i *)(qrow + c) = cvt8_slow(*(const v4i *)(xrow + c), recip);
     }
     if (PREFETCH) {
 #pragma unroll
       for (int j = 0; j < NCH; ++j) cur[j] = nxt[PREFETCH ? j : 0];
     } else {
       __builtin_amdgcn_sched_barrier(0);  // the row registers are reused: do not start the loads early
-      load_row<NCH>(cur, x, rn, R, ldx, C, lane);
+      load(cur, rn);
     }
     r = rn;
   }
@@ -142,17 +201,23 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
 // many workgroups fit a CU.  The row amax crosses waves through LDS with one
 // barrier per row (double-buffered).  Column maxima of different waves cover
 // disjoint columns and are merged into the global array directly.
-template <int NCHW, bool COLMAX>
+template <int NCHW, bool COLMAX, bool MANY = false>
 __global__ __launch_bounds__(kRowBlock, (NCHW <= 4 ? 4 : (NCHW <= 8 ? 2 : 1))) void cast_rowwise_wg_kernel(
     const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint8_t *__restrict__ q, int64_t ldq,
-    float *__restrict__ scale, uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule) {
+    float *__restrict__ scale, uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule,
+    const std::conditional_t<MANY, RowOperands, int> list) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer descriptors exist in the device pass only
   __shared__ uint32_t red[2][kRowWaves];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   auto col_of = [&](int j) { return (j * kRowWaves + wave) * 512 + lane * 8; };
   auto load = [&](v4i (&buf)[NCHW], int64_t r) {  // zeros beyond column C and for a row beyond R, as in load_row
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(x + (r < R ? r : 0) * ldx, r < R ? (uint32_t)C * 2u : 0u);
+    const uint16_t *row = x + (r < R ? r : 0) * ldx;
+    if constexpr (MANY) {
+      const RowOperand op = operand_of(list, r);
+      row = op.x + (r < R ? r - op.first : 0) * op.ldx;
+    }
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(row, r < R ? (uint32_t)C * 2u : 0u);
 #pragma unroll
     for (int j = 0; j < NCHW; ++j) buf[j] = load16_nt(rs, (uint32_t)col_of(j) * 2u, 0);
   };
@@ -190,18 +255,28 @@ __global__ __launch_bounds__(kRowBlock, (NCHW <= 4 ? 4 : (NCHW <= 8 ? 2 : 1))) v
     if (finite) s = scale_from_amax(bf16_bits_to_f32(amax_bits), scale_rule);
     else s = __uint_as_float(amax_bits == 0x7f80u ? 0x7f800000u : 0x7fc00000u);
     const float recip = recip_exact(s);
-    if (threadIdx.x == 0) {
+    const uint16_t *xrow = x + r * ldx;
+    uint8_t *qrow = q ? q + r * ldq : nullptr;
+    if constexpr (MANY) {
+      const RowOperand cur_op = operand_of(list, r);
+      const int64_t ro = r - cur_op.first;
+      xrow = cur_op.x + ro * cur_op.ldx;
+      qrow = cur_op.q + ro * cur_op.ldq;
+      if (threadIdx.x == 0) {
+        cur_op.scale[ro] = s;
+        if (cur_op.amax) cur_op.amax[ro] = (uint16_t)amax_bits;
+      }
+    } else if (threadIdx.x == 0) {
       if (scale) scale[r] = s;
       if (amax_out) amax_out[r] = (uint16_t)amax_bits;
     }
-    uint8_t *qrow = q ? q + r * ldq : nullptr;
-    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(qrow, q ? (uint32_t)C : 0u);  // stores beyond column C, or without q, are dropped
+    const __amdgpu_buffer_rsrc_t rsQ = make_rsrc(qrow, MANY || q ? (uint32_t)C : 0u);  // stores beyond column C, or without q, are dropped
 #pragma unroll
     for (int j = 0; j < NCHW; ++j) store8(rsQ, (uint32_t)col_of(j), cvt8(cur[j], recip));
-    if (q && !finite) {  // non-finite amax: redone from memory with the integer conversion, as in cast_rowwise_kernel
+    if ((MANY || q) && !finite) {  // non-finite amax: redone from memory with the integer conversion, as in cast_rowwise_kernel
 #pragma unroll 1
       for (int c = threadIdx.x * 8; c < C; c += kRowBlock * 8)
-        *(v2i *)(qrow + c) = cvt8_slow(*(const v4i *)(x + r * ldx + c), recip);
+        *(v2i *)(qrow + c) = cvt8_slow(*(const v4i *)(xrow + c), recip);
     }
 #pragma unroll
     for (int j = 0; j < NCHW; ++j) cur[j] = nxt[j];
@@ -698,12 +773,12 @@ static int launch_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx, void
   if (col_amax) {
     const size_t lds = (size_t)C * sizeof(uint16_t);
     hipLaunchKernelGGL((cast_rowwise_kernel<NCH, true>), dim3((unsigned)blocks), dim3(kRowBlock), lds, st,
-                       (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule());
+                       (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule(), 0);
     L8_HIP(hipGetLastError());
     return fold_colmax(ws, blocks, C, col_amax, st);
   }
   hipLaunchKernelGGL((cast_rowwise_kernel<NCH, false>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
-                     (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule());
+                     (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule(), 0);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
@@ -714,12 +789,40 @@ static int launch_rowwise_wg(const void *x, int64_t R, int64_t C, int64_t ldx, v
   const int64_t blocks = rowwise_blocks(R, C, col_amax != nullptr);
   if (col_amax) {
     hipLaunchKernelGGL((cast_rowwise_wg_kernel<NCHW, true>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
-                       (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule());
+                       (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule(), 0);
     L8_HIP(hipGetLastError());
     return fold_colmax(ws, blocks, C, col_amax, st);
   }
   hipLaunchKernelGGL((cast_rowwise_wg_kernel<NCHW, false>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
-                     (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule());
+                     (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule(), 0);
+  L8_HIP(hipGetLastError());
+  return L8_OK;
+}
+
+static int cast_rowwise_many(const l8_cast_rowwise_item *items, int n, int64_t C, hipStream_t st) {
+  RowOperands list{};
+  int64_t rows = 0;
+  for (int i = 0; i < kMaxRowOperands; ++i) {
+    if (i < n) {
+      const l8_cast_rowwise_item &t = items[i];
+      list.op[i] = {(const uint16_t *)t.x, rows, t.ldx, (uint8_t *)t.q, t.ldq, t.scale, (uint16_t *)t.amax};
+      rows += t.R;
+    } else {
+      list.op[i].first = INT64_MAX;
+    }
+  }
+  const unsigned blocks = (unsigned)rowwise_blocks(rows, C, false);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kRowBlock), 0, st, nullptr, rows, (int)C, 0, nullptr, 0, nullptr, nullptr, nullptr,
+                       l8::scale_rule(), list);
+  };
+  const int64_t nch = (C + 511) / 512, nchw = (nch + kRowWaves - 1) / kRowWaves;
+  if (nch <= 4) go(cast_rowwise_kernel<4, false, true>);
+  else if (nch <= 8) go(cast_rowwise_kernel<8, false, true>);
+  else if (nchw <= 3) go(cast_rowwise_wg_kernel<3, false, true>);
+  else if (nchw <= 4) go(cast_rowwise_wg_kernel<4, false, true>);
+  else if (nchw <= 6) go(cast_rowwise_wg_kernel<6, false, true>);
+  else go(cast_rowwise_wg_kernel<8, false, true>);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
@@ -728,6 +831,23 @@ static int launch_rowwise_wg(const void *x, int64_t R, int64_t C, int64_t ldx, v
 
 using namespace l8;
 
+// Can an operand with these pointers and strides be one of several (the checks of cast_rowwise_impl, as an answer)?
+static bool many_serves(const l8_cast_rowwise_item &t, int64_t C) {
+  return t.R > 0 && t.x && t.q && t.scale && t.ldx % 8 == 0 && t.ldx >= C && aligned(t.x, 16) && t.ldq % 8 == 0 && t.ldq >= C && aligned(t.q, 8);
+}
+
+extern "C" int l8_cast_rowwise_many(const l8_cast_rowwise_item *items, int64_t n, int64_t C, void *stream) {
+  L8_REQUIRE(items && n >= 0 && C >= 0, "l8_cast_rowwise_many: null items, or a negative count");
+  bool together = n > 1 && n <= kMaxRowOperands && C > 0 && C % 8 == 0 && C <= kMaxRowwiseManyColumns;
+  for (int64_t i = 0; i < n && together; ++i) together = many_serves(items[i], C);
+  if (together) return cast_rowwise_many(items, (int)n, C, (hipStream_t)stream);
+  for (int64_t i = 0; i < n; ++i) {
+    const l8_cast_rowwise_item &t = items[i];
+    const int rc = l8_cast_rowwise(t.x, t.R, C, t.ldx, t.q, t.ldq, t.scale, t.amax, nullptr, nullptr, 0, stream);
+    if (rc != L8_OK) return rc;
+  }
+  return L8_OK;
+}
 
 extern "C" int64_t l8_cast_rowwise_workspace(int64_t R, int64_t C) {
   if (R <= 0 || C <= 0) return 0;

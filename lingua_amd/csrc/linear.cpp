@@ -74,7 +74,13 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
   const LinearFwd t = plan(*a, ws);
   L8_REQUIRE(ws.used <= a->workspace_bytes && ((uintptr_t)a->workspace % 256) == 0,
              "l8_linear_fwd: needs a 256-byte aligned workspace of %lld bytes", (long long)ws.used);
-  if (!a->x_ready && !t.x_on_the_way) {
+  const bool cast_x = !a->x_ready && !t.x_on_the_way, cast_w = !t.w_on_the_way && !a->w_ready;
+  const bool together = cast_x && cast_w && !a->col_amax_x;
+  if (together) {
+    const l8_cast_rowwise_item items[2] = {{a->x, a->M, a->ldx, t.qx, a->K, t.sx, nullptr}, {a->w, a->N, a->ldw, t.qw, a->K, t.sw, a->amax_w}};
+    rc = l8_cast_rowwise_many(items, 2, a->K, a->stream);
+    if (rc != L8_OK) return rc;
+  } else if (cast_x) {
     rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, a->K, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
     if (rc != L8_OK) return rc;
   }
@@ -86,7 +92,7 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
                  "l8_linear_fwd: x must be 16-byte aligned, ldx=%lld a multiple of 8 and >= K", (long long)a->ldx);
     if (!t.w_on_the_way) L8_REQUIRE(((uintptr_t)t.qw % 16) == 0, "l8_linear_fwd: qw must be 16-byte aligned");
   }
-  if (!t.w_on_the_way && !a->w_ready) {
+  if (cast_w && !together) {
     rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);
     if (rc != L8_OK) return rc;
   }

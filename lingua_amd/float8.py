@@ -275,6 +275,13 @@ def weight_cast_rowwise(w):
     return _weight_casts.rowwise(w)
 
 
+def weight_casts_rowwise(ws):
+    """``weight_cast_rowwise`` of weights of one width that are quantised together."""
+    if config.cache_weight_casts:
+        return [_weight_casts.rowwise(w) for w in ws]
+    return ops.cast_rowwise_many(ws)
+
+
 def weight_cast_tensorwise_t(w, amax_rows):
     """``(q [K,N], scale [1,1])`` of a weight [N,K], tensor-wise from its saved row amaxes and written
     transposed (the dgrad operand, lingua/float8.py:111-118)."""

@@ -127,6 +127,40 @@ def cast_rowwise(x: torch.Tensor, col_amax: Optional[torch.Tensor] = None, want_
     return q, scale, amax
 
 
+def cast_rowwise_many(xs, out=None):
+    """``cast_rowwise`` of several tensors of one width, in one launch where the library can.  ``out``: (q [sum of rows, C]
+    fp8, scale [sum of rows, 1] fp32), dense, that receives the results one below the other.  Returns a list of (q, scale,
+    amax) per tensor."""
+    xs = [_rows_2d(x, torch.bfloat16, "cast_rowwise_many") for x in xs]
+    dev, C = xs[0].device, xs[0].shape[1]
+    st = _prep(xs[0], "cast_rowwise_many")
+    rows = [x.shape[0] for x in xs]
+    if any(x.shape[1] != C or x.device != dev for x in xs):
+        raise RuntimeError("cast_rowwise_many: tensors of one width on one device required")
+    if out is not None:
+        q_all, s_all = out
+        if (q_all.dtype != torch.float8_e4m3fn or tuple(q_all.shape) != (sum(rows), C) or not q_all.is_contiguous() or q_all.device != dev or
+                s_all.dtype != torch.float32 or tuple(s_all.shape) != (sum(rows), 1) or not s_all.is_contiguous() or s_all.device != dev):
+            raise RuntimeError("cast_rowwise_many: out must be dense e4m3fn [rows,C] and fp32 [rows,1] tensors on the inputs' device")
+        qs, ss = q_all.split(rows), s_all.split(rows)
+    else:
+        qs = [torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=dev) for x in xs]
+        ss = [torch.empty((n, 1), dtype=torch.float32, device=dev) for n in rows]
+    if kernel_timer is not None:  # per-kernel figures are of the casts one by one
+        return [cast_rowwise(x, out_q=q, out_scale=s) for x, q, s in zip(xs, qs, ss)]
+    amaxes = [torch.empty((n, 1), dtype=torch.bfloat16, device=dev) for n in rows]
+    items = []
+    for x, q, s, a in zip(xs, qs, ss, amaxes):
+        items += [x.data_ptr(), x.shape[0], _ld(x), q.data_ptr(), C, s.data_ptr(), a.data_ptr()]
+    with _timed("cast_rowwise_many", sum(rows) * (3 * C + 4), dev):
+        code = _lib.load().l8_cast_rowwise_many(struct.pack(f"{len(items)}q", *items), len(xs), C, st)
+    _lib.check(code, "l8_cast_rowwise_many")
+    if out is not None:
+        _wrote_into(q_all)
+        _wrote_into(s_all)
+    return list(zip(qs, ss, amaxes))
+
+
 AMAX_BF16, AMAX_F32 = 0, 1
 
 

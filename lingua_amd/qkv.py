@@ -54,11 +54,7 @@ class Fp8QKVFn(torch.autograd.Function):
         sizes = [w.shape[0] for w in ws]
         qw = torch.empty((sum(sizes), K), dtype=torch.float8_e4m3fn, device=x.device)
         sw = torch.empty((sum(sizes), 1), dtype=torch.float32, device=x.device)
-        amaxes, o = [], 0
-        for w, n in zip(ws, sizes):
-            _, _, amax_w = ops.cast_rowwise(w, out_q=qw[o:o + n], out_scale=sw[o:o + n])
-            amaxes.append(amax_w)
-            o += n
+        amaxes = [amax for _, _, amax in ops.cast_rowwise_many(ws, out=(qw, sw))]
         y = ops.gemm_nt(qx, qw, sx, sw, None, algo=cfg.gemm_algo)
         ctx.fp8_wgrad, ctx.gemm_algo, ctx.has_col = cfg.fp8_wgrad, cfg.gemm_algo, x_col is not None
         ctx.need = (x.requires_grad,) + tuple(w.requires_grad for w in ws)

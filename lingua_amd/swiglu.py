@@ -48,8 +48,7 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         else:
             x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_x_col else None
             qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col)
-        q1, s1, amax_w1 = f8.weight_cast_rowwise(w1)
-        q3, s3, amax_w3 = f8.weight_cast_rowwise(w3)
+        (q1, s1, amax_w1), (q3, s3, amax_w3) = f8.weight_casts_rowwise((w1, w3))
         h1 = ops.gemm_nt(qx, q1, sx, s1, None, algo=algo)
         h3 = ops.gemm_nt(qx, q3, sx, s3, None, algo=algo)
         del qx, q1, q3

@@ -446,3 +446,30 @@ def test_transposed_cast_pads_with_zeros(R, pad_to):
         assert q.shape == (C, (R + pad_to - 1) // pad_to * pad_to)
         assert torch.equal(q.cpu().view(torch.uint8)[:, :R], wq) and not q.view(torch.uint8)[:, R:].any()
         assert torch.equal(s.cpu().reshape(-1).view(torch.int32), ws.reshape(-1).view(torch.int32))
+
+
+@pytest.mark.parametrize("C", [16, 520, 2048, 2056, 4104, 8192, 8200, 16384, 16392])
+@pytest.mark.parametrize("rows", [(1, 1), (3, 4097), (70, 1, 9), (4100, 2, 5), (5, 6, 7, 8), (3, 0, 2)])
+def test_several_operands_in_one_launch(C, rows):
+    """Rows of every kernel, the first and last row of an operand next to each other in the list, more operands than a
+    launch takes, an empty one, a padded row stride, zero rows and rows with an infinity or a NaN: the bytes, scales and
+    amaxes of one call per operand."""
+    from lingua_amd import ops
+    if max(rows) * C > 1 << 25:
+        rows = tuple(min(n, 600) for n in rows)
+    xs = []
+    for i, n in enumerate(rows):
+        x = torch.zeros((n, C + 8), dtype=torch.bfloat16, device="cuda")[:, :C]
+        x.copy_(torch.randn(n, C, generator=torch.Generator(device="cuda").manual_seed(i), device="cuda") * 10.0 ** (i - 1))
+        if n > 2:
+            x[n - 1] = 0.0
+            x[0, C - 1], x[1, 0] = float("inf"), float("nan")
+        xs.append(x)
+    want = [ops.cast_rowwise(x) for x in xs]
+    out = (torch.full((sum(rows), C), 0x55, dtype=torch.uint8, device="cuda").view(torch.float8_e4m3fn),
+           torch.zeros((sum(rows), 1), device="cuda"))
+    for got in (ops.cast_rowwise_many(xs), ops.cast_rowwise_many(xs, out=out)):
+        for (q, s, a), (wq, ws, wa) in zip(got, want):
+            assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8))
+            assert torch.equal(s.view(torch.int32), ws.view(torch.int32)) and torch.equal(a.view(torch.int16), wa.view(torch.int16))
+    assert torch.equal(out[0].view(torch.uint8), torch.cat([w[0].view(torch.uint8) for w in want]))
