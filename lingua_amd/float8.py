@@ -40,6 +40,7 @@ from dataclasses import dataclass
 from typing import Callable, Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import ops
 
@@ -475,13 +476,21 @@ class Fp8LinearFn(torch.autograd.Function):
                                ctx.bias_requires_grad, ctx.fp8_wgrad, ctx.gemm_algo, a_tcast)
 
 
+def _plain_call():
+    """No transform or tracer sees the call: under forward-mode AD, functorch, TorchScript tracing or compilation the
+    autograd function has to, which refuses, records or breaks the graph where the bare kernels would go unnoticed."""
+    return (forward_ad._current_level < 0 and not torch._C._are_functorch_transforms_active() and
+            torch._C._get_tracing_state() is None and not torch.compiler.is_compiling())
+
+
 class Fp8Linear(torch.nn.Linear):
     def forward(self, input: torch.Tensor) -> torch.Tensor:
         weight, bias = self.weight, self.bias
         if config.use_custom_ops:
             from .custom_ops import fp8_linear
             out = fp8_linear(input.flatten(end_dim=-2), weight, bias)
-        elif torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad)):
+        elif (torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad))
+              or not _plain_call()):
             out = Fp8LinearFn.apply(input.flatten(end_dim=-2), weight, bias)
         else:
             return linear_infer(input, weight, bias)

@@ -333,6 +333,27 @@ def test_linear_refuses_operands_it_cannot_serve_before_any_gpu_work():
         Fp8LinearFn.apply(meta_x, torch.zeros(48, 40, dtype=torch.bfloat16, device="meta"), None)
 
 
+def test_transforms_and_tracers_still_see_the_autograd_function(monkeypatch):
+    """A forward without gradients takes one bare library call, whose result has no tangent, no batch dimension and no
+    place in a trace: forward-mode AD and functorch are refused as before, a trace holds the function and not its result."""
+    from lingua_amd import float8
+    lin = Fp8Linear(32, 48, bias=False, dtype=torch.bfloat16).requires_grad_(False)
+    x = torch.randn(8, 32).to(torch.bfloat16)
+    bare = []
+    monkeypatch.setattr(float8, "linear_infer", lambda a, w, b: bare.append(1) or a @ w.t())
+    monkeypatch.setattr(float8, "linear_forward", lambda a, w, *rest: (a @ w.t(), w.abs().amax(1, keepdim=True), None))
+    lin(x)
+    assert bare == [1]
+    with torch.autograd.forward_ad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+        lin(torch.autograd.forward_ad.make_dual(x, x))
+    for transform in (torch.func.vmap(lin), torch.func.grad(lambda t: lin(t).sum())):
+        with pytest.raises(RuntimeError, match="functorch"):
+            transform(x.unsqueeze(0))
+    traced = torch.jit.trace(lin, x, check_trace=False)
+    assert torch.equal(traced(2 * x), 2 * (x @ lin.weight.t()))
+    assert bare == [1]
+
+
 def test_a_named_library_that_is_not_there_fails_loudly():
     """LINGUA_FP8_LIB points lingua_amd at another build of the library (a tuning variant); a path that does not exist
     is an error that names the path, never a silent return to the shipped library."""
