@@ -278,6 +278,20 @@ int l8_gemm_pick(int64_t M, int64_t N, int64_t K);
 int l8_gemm_nt_add(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                    const float *sa, int sa_mode, const float *sb, int sb_mode, void *C, int64_t ldc, int algo, void *stream);
 
+/* C_i [M_i,N] = bf16(A_i [M_i,K] . B^T * sa_i * sb) for n products with one B: the weight gradients of linears on one
+ * activation (lingua/float8.py:123 once per linear).  One launch for two or three of them where that takes fewer rounds of
+ * tiles over the chip, else as n calls of l8_gemm_nt.  sa_i fp32 [M_i]; lda and ldc are those of every A_i and C_i. */
+typedef struct {
+  const void *A;
+  int64_t M;
+  const float *sa;
+  void *C;
+} l8_gemm_part;
+int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                     const float *sb, int sb_mode, int64_t ldc, int algo, void *stream);
+/* Host arithmetic only: would l8_gemm_nt_multi launch these once (aligned operands, n = 2 or 3 assumed; reads M alone)? */
+int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t K);
+
 /* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
  * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; with a few
  * tokens, and neither qw nor amax_w asked for, the weight is quantised inside the product.  Every member is eight bytes

@@ -72,6 +72,14 @@ struct GemmArgs {
   float *sk_partials;
   uint32_t sk_epoch;  // value that marks a flag as set in THIS launch (never 0; flags are never cleared)
   int sk_wait_limit;  // polls of a flag before the waiting workgroup gives up and poisons its tile
+  // MULTI kernels: products with the same B, one below the other.  A, sa, C and M above are the first one's; a further one
+  // starts at tile row first / 256 of the launch, an unused one beyond the last.
+  struct Part {
+    const uint8_t *A;
+    const float *sa;
+    uint16_t *C;
+    int first, M;
+  } part[2];
 };
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -611,7 +619,11 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // ADD: the bf16 tile is added to what C holds (two gradients of one activation) in the epilogue.  The C values are
 // requested C_AHEAD row groups before they are used: the counter retires in order, so the wait for them is also one for the
 // stores issued before they were requested, and those have had that long.
-template <int GROUP_M, bool HAS_BIAS, bool SK = false, int NW = 4, bool ADD = false>
+//
+// MULTI: up to three products with one B (the weight gradients of linears on one activation) as one list of tiles.  On its
+// own [2048,16384].[2048,16384]^T has 64 tiles of 256 x 256, too few for this kernel, and [11008,4096] leaves a third of the
+// units without work in its last round; together they fill the rounds.
+template <int GROUP_M, bool HAS_BIAS, bool SK = false, int NW = 4, bool ADD = false, bool MULTI = false>
 __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // NW = 4: one wave per SIMD, 128x128 per wave (the least LDS traffic per flop); NW = 8: two waves per SIMD,
@@ -751,6 +763,24 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
   auto wrap = [](int slot) { return slot >= R ? slot - R : slot; };
 
+  // the product that the tile row at m0 belongs to (m0 becomes its row inside that product)
+  auto part_of = [&](int &m0) {
+    GemmArgs::Part t = {p.A, p.sa, p.C, 0, p.M};
+    if constexpr (MULTI) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const bool here = m0 >= p.part[i].first;
+        t.A = here ? p.part[i].A : t.A;
+        t.sa = here ? p.part[i].sa : t.sa;
+        t.C = here ? p.part[i].C : t.C;
+        t.first = here ? p.part[i].first : t.first;
+        t.M = here ? p.part[i].M : t.M;
+      }
+      m0 -= t.first;
+    }
+    return t;
+  };
+
   // loader cursor: the K tile whose panels are requested next (two K tiles ahead of the one being multiplied)
   int ld_seg = 0, ld_kt = 0;
   [[maybe_unused]] int ld_ke = KT;  // SK: the loader's piece ends here
@@ -767,9 +797,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
         ld_kt = piece_kb;
         ld_ke = piece_ke;
       }
-      const int64_t a_left = (int64_t)(p.M - m0 - 1) * p.lda + p.K;
+      const GemmArgs::Part t = part_of(m0);
+      const int64_t a_left = (int64_t)(t.M - m0 - 1) * p.lda + p.K;
       const int64_t b_left = (int64_t)(p.N - n0 - 1) * p.ldb + p.K;
-      ld_rsA = make_rsrc(p.A + (int64_t)m0 * p.lda, a_left < 0x7fffffff ? (uint32_t)a_left : 0x7fffffffu);
+      ld_rsA = make_rsrc(t.A + (int64_t)m0 * p.lda, a_left < 0x7fffffff ? (uint32_t)a_left : 0x7fffffffu);
       ld_rsB = make_rsrc(p.B + (int64_t)n0 * p.ldb, b_left < 0x7fffffff ? (uint32_t)b_left : 0x7fffffffu);
     } else {  // past the last tile: every load is out of range and fills its LDS bytes with zeros
       ld_rsA = make_rsrc(p.A, 0);
@@ -867,7 +898,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
   [[maybe_unused]] const __amdgpu_buffer_rsrc_t rsBias = make_rsrc(HAS_BIAS ? (const void *)p.bias : (const void *)p.sb, (uint32_t)p.N * 2u);
   // a scale that is one number for the whole operand is read once (read per tile, between the stores of one tile
   // and the K loop of the next, it was a vector load whose result was copied at once: a wait for every store)
-  const int sa_one = p.sa_row ? 0 : __builtin_amdgcn_readfirstlane(__float_as_int(p.sa[0]));
+  const int sa_one = MULTI || p.sa_row ? 0 : __builtin_amdgcn_readfirstlane(__float_as_int(p.sa[0]));
   const int sb_one = p.sb_row ? 0 : __builtin_amdgcn_readfirstlane(__float_as_int(p.sb[0]));
   auto load_scales = [&](int m0, int n0) {
     // lane-derived values are formed afresh from an opaque copy of the lane number wherever a tile's prologue or
@@ -876,9 +907,14 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     asm volatile("" : "+v"(l));
     const int l31 = l & 31;
     const int cg = 2 * (l31 & 15) + (l31 >> 4);  // this lane's group of four output columns (of its wave's 32)
-    if (p.sa_row) {
-      seg_sa[0] = __builtin_amdgcn_raw_buffer_load_b32(rsSa, (wm * WROWS + l) * 4, m0 * 4, 0);
-      if constexpr (TM == 4) seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rsSa, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
+    if (MULTI || p.sa_row) {
+      __amdgpu_buffer_rsrc_t rs = rsSa;
+      if constexpr (MULTI) {
+        const GemmArgs::Part t = part_of(m0);
+        rs = make_rsrc(t.sa, (uint32_t)t.M * 4u);
+      }
+      seg_sa[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + l) * 4, m0 * 4, 0);
+      if constexpr (TM == 4) seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
     } else {
       seg_sa[0] = seg_sa[1] = sa_one;
     }
@@ -914,8 +950,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     const int l31 = l & 31, h = l >> 5;
     int lane_col = wn * 128 + 8 * (l31 & 15);  // first of the eight columns this lane stores
     asm volatile("" : "+v"(lane_col));
-    const int64_t c_left = ((int64_t)(p.M - m0 - 1) * p.ldc + (p.N - n0)) * 2;
-    const __amdgpu_buffer_rsrc_t rsC = make_rsrc(p.C + (int64_t)m0 * p.ldc + n0, c_left < 0x7fffffff ? (uint32_t)c_left : 0x7fffffffu);
+    const GemmArgs::Part t = part_of(m0);
+    const int64_t c_left = ((int64_t)(t.M - m0 - 1) * p.ldc + (p.N - n0)) * 2;
+    const __amdgpu_buffer_rsrc_t rsC = make_rsrc(t.C + (int64_t)m0 * p.ldc + n0, c_left < 0x7fffffff ? (uint32_t)c_left : 0x7fffffffu);
     float sbv[4];
     [[maybe_unused]] float bv[4];
 #pragma unroll
@@ -1369,6 +1406,7 @@ template __global__ void gemm_nt_stream_kernel<4, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, 4, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, 4, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
@@ -1495,6 +1533,13 @@ extern "C" int l8_gemm_shares_k(int64_t M, int64_t N, int64_t K, int compute_uni
   return (int)((sk_pays(q + 1, W, KT) ? rem : 0) + (sk_pays(q, W, KT) ? 8 - rem : 0));
 }
 
+// one workgroup per compute unit, a multiple of 8 of them (the hardware deals workgroups to the 8 XCDs in turn)
+static int64_t persistent_grid(int64_t nblocks) {
+  const int64_t cus8 = (num_cus() / 8) * 8, want = (nblocks + 7) / 8 * 8;
+  const int64_t grid = want < cus8 ? want : cus8;
+  return grid < 8 ? 8 : grid;
+}
+
 static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                         const float *sa, int sa_mode, const float *sb, int sb_mode, const void *bias, void *C,
                         int64_t ldc, int add, int algo, void *workspace, int64_t workspace_bytes, void *stream) {
@@ -1572,14 +1617,7 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
     if (al.fn_sk) L8_HIP(hipFuncSetAttribute((const void *)al.fn_sk, hipFuncAttributeMaxDynamicSharedMemorySize, al.lds));
     if (slot >= 0) attr_done[slot][algo - 1] = true;
   }
-  int64_t grid = nblocks;
-  if (al.persistent) {
-    // one workgroup per compute unit, a multiple of 8 of them (the hardware deals workgroups to the 8 XCDs in turn)
-    const int64_t cus8 = (num_cus() / 8) * 8;
-    const int64_t want = (nblocks + 7) / 8 * 8;
-    grid = want < cus8 ? want : cus8;
-    if (grid < 8) grid = 8;
-  }
+  const int64_t grid = al.persistent ? persistent_grid(nblocks) : nblocks;
   gemm_fn fn = (al.fn_add && add) ? al.fn_add : (al.fn_bias && p.bias) ? al.fn_bias : al.fn;
   if (al.fn_sk && !p.bias && !add && workspace != nullptr && grid <= kSkMaxGrid && workspace_bytes >= kSkFlagBytes + grid * kSkTileBytes) {
     // the kernel decides per XCD (their tile counts differ by at most one) with the same test
@@ -1628,4 +1666,76 @@ extern "C" int l8_gemm_nt_ws(const void *A, const void *B, int64_t M, int64_t N,
                              int64_t ldc, int algo, void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(workspace == nullptr || ((uintptr_t)workspace % 16) == 0, "l8_gemm_nt_ws: workspace must be 16-byte aligned");
   return gemm_nt_impl(A, B, M, N, K, lda, ldb, sa, sa_mode, sb, sb_mode, bias, C, ldc, 0, algo, workspace, workspace_bytes, stream);
+}
+
+// Do products of M[i] rows with one B of N rows run faster as one launch of the persistent kernel?  Bound by the matrix cores
+// of the units that have a tile: apart, each product leaves units without one (in its last round, or in all of it on the
+// smaller tiles); together they do so once.  us, apart / together, 256 units:
+//   3 x [2048,K].[2048,K]^T, 192 tiles: K = 256 18.6 / 10.9, 1024 25.4 / 18.1, 4096 57.8 / 42.3, 16384 192.5 / 145.7 (2.83 PFLOP/s)
+//   [2048 + 512 + 512], 96 tiles: 256 14.9 / 9.6, 1024 19.6 / 15.6, 4096 40.1 / 38.5, but 16384 119.0 / 122.5
+//   3 x [1408,..], 108 tiles: 4096 43.1 / 38.2, 16384 142.0 / 124.3;  3 x [1280,..], 75: 131.3 / 121.9;  3 x [1024,..], 48: 80.7 / 120.9
+//   2 x [2816,..].[1024,..], 88 tiles: 1024 16.3 / 15.0, 4096 36.3 / 37.1;  2 x [2048,..], 64 tiles: 29.4 / 36.2
+//   whole rounds: 3 x [4096,4096].[4096,4096] 152.5 / 142.4, 2 x [14336,4096].[4096,4096] 353 / 328, 2 x [11008,4096].[4096,4096] 272 / 267
+// so from 3/8 of a tile per unit on, a little more where the reduction is long.
+extern "C" int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t K) {
+  int64_t tiles = 0;
+  for (int64_t i = 0; i < n; ++i) tiles += ((parts[i].M + 255) / 256) * ((N + 255) / 256);
+  return tiles * 32 >= (int64_t)num_cus() * (K > 4096 ? 13 : 12);
+}
+
+extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_t N, int64_t K, int64_t lda, int64_t ldb,
+                                const float *sb, int sb_mode, int64_t ldc, int algo, void *stream) {
+  L8_REQUIRE(n >= 0 && (n == 0 || parts), "l8_gemm_nt_multi: null list or negative count");
+  bool one = algo == 0 && n >= 2 && n <= 3 && B && sb && N > 0 && N < (1LL << 29) && K > 0 && K % 16 == 0 && K < (1LL << 31) && N % 8 == 0 &&
+             ldc % 8 == 0 && ldc >= N && ldc < (1LL << 22) && lda % 16 == 0 && ldb % 16 == 0 && lda >= K && ldb >= K &&
+             256 * lda + K < (1LL << 31) && 256 * ldb + K < (1LL << 31) && ((uintptr_t)B % 16) == 0 &&
+             (sb_mode == L8_SCALE_SCALAR || (sb_mode == L8_SCALE_ROW && ((uintptr_t)sb % 16) == 0));
+  int64_t tile_rows = 0;
+  for (int64_t i = 0; one && i < n; ++i) {
+    const l8_gemm_part &t = parts[i];
+    one = t.A && t.C && t.sa && t.M > 0 && t.M < (1LL << 28) && ((uintptr_t)t.A % 16) == 0 && ((uintptr_t)t.C % 16) == 0 && ((uintptr_t)t.sa % 16) == 0;
+    tile_rows += (t.M + 255) / 256;
+  }
+  one = one && tile_rows * ((N + 255) / 256) < (1LL << 31) && l8_gemm_multi_pays(parts, n, N, K);
+  if (!one) {
+    for (int64_t i = 0; i < n; ++i) {
+      const l8_gemm_part &t = parts[i];
+      const int rc = gemm_nt_impl(t.A, B, t.M, N, K, lda, ldb, t.sa, L8_SCALE_ROW, sb, sb_mode, nullptr, t.C, ldc, 0, algo, nullptr, 0, stream);
+      if (rc != L8_OK) return rc;
+    }
+    return L8_OK;
+  }
+  constexpr int kLds = 5 * 256 * 128;
+  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, 4, false, true>;
+  GemmArgs p{};
+  p.A = (const uint8_t *)parts[0].A;
+  p.B = (const uint8_t *)B;
+  p.M = (int)parts[0].M;
+  p.N = (int)N;
+  p.K = (int)K;
+  p.lda = lda;
+  p.ldb = ldb;
+  p.ldc = ldc;
+  p.sa = parts[0].sa;
+  p.sb = sb;
+  p.sa_row = 1;
+  p.sb_row = sb_mode == L8_SCALE_ROW;
+  p.C = (uint16_t *)parts[0].C;
+  p.tiles_m = (int)tile_rows;
+  p.tiles_n = (int)((N + 255) / 256);
+  int64_t first = 0;
+  for (int i = 0; i < 2; ++i) {
+    first += (parts[i].M + 255) / 256 * 256;
+    if (i + 1 < n) p.part[i] = {(const uint8_t *)parts[i + 1].A, parts[i + 1].sa, (uint16_t *)parts[i + 1].C, (int)first, (int)parts[i + 1].M};
+    else p.part[i] = {p.A, p.sa, p.C, 0x7fffffff, p.M};
+  }
+  static std::atomic<bool> attr_done[kMaxDev] = {};  // idempotent; a race only repeats the call
+  const int slot = device_slot();
+  if (slot < 0 || !attr_done[slot]) {
+    L8_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
+    if (slot >= 0) attr_done[slot] = true;
+  }
+  hipLaunchKernelGGL(fn, dim3((unsigned)persistent_grid((int64_t)p.tiles_m * p.tiles_n)), dim3(256), kLds, (hipStream_t)stream, p);
+  L8_HIP(hipGetLastError());
+  return L8_OK;
 }

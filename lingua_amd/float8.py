@@ -391,10 +391,12 @@ def input_cast_for_wgrad(a, a_col_amax, user):
 
 
 def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b: bool, need_bias: bool,
-                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None, grad_a=None):
+                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None, grad_a=None, wgrad_later=None):
     """Backward of lingua/float8.py:99-131 (fp8 wgrad optional).  Returns ``(grad_a, grad_b, grad_bias)`` with
     ``None`` where not needed.  ``a_tcast`` = ``(qat [K,M], sat [K,1])`` made in forward stands in for ``a``
-    (then ``a`` may be None; fp8 wgrad only).  ``grad_a``: a gradient of ``a`` that this one is added to, in place."""
+    (then ``a`` may be None; fp8 wgrad only).  ``grad_a``: a gradient of ``a`` that this one is added to, in place.
+    ``wgrad_later``: a list that receives the operands ``(qgt, sgt, qat, sat)`` of the fp8 wgrad product in the place of
+    ``grad_b``, which then is ``None``."""
     if grad_out.dtype != torch.bfloat16:
         raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {grad_out.dtype}")
     fp8_wgrad = fp8_wgrad and need_b
@@ -428,7 +430,11 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
                 qat, sat = ops.cast_colwise_transposed(a, a_col_amax)
                 if config.share_input_casts:
                     _bwd_cast.put(a, (qat, sat), b_t.data_ptr())
-            grad_b = ops.gemm_nt(qgt, qat, sgt, sat, None, algo=gemm_algo)
+            if wgrad_later is not None:
+                wgrad_later.append((qgt, sgt, qat, sat))
+                grad_b = None
+            else:
+                grad_b = ops.gemm_nt(qgt, qat, sgt, sat, None, algo=gemm_algo)
         else:
             grad_b = grad_out.t() @ a
     else:

@@ -10,9 +10,10 @@ into row slices of it) and a single GEMM produces ``[T, Nq+Nk+Nv]``, of which
 the three linears return column slices.  Same recipe, same scales (every weight
 row keeps its own), so the same bits as three separate products.
 
-Backward stays per linear (lingua/float8.py:99-131): the three dgrads have
-different row scales and cannot be one product; the three wgrads share the
-token-dimension copy of ``x`` through the memo of ``lingua_amd.float8``.
+Backward stays per linear (lingua/float8.py:99-131) but for its launches: the
+three dgrads have different row scales and are added up by their epilogues, the
+three wgrads share the token-dimension copy of ``x`` and run as one list of
+tiles.
 
 Nothing changes in the attention module or in the state dict: ``wq`` computes
 all three products when it is called and keeps the other two for ``wk`` and
@@ -70,12 +71,19 @@ class Fp8QKVFn(torch.autograd.Function):
         saved = ctx.saved_tensors
         x, ws, amaxes = saved[0], saved[1:4], saved[4:7]
         x_col = saved[7] if ctx.has_col else None
-        gx, gws = None, [None, None, None]
+        gx, gws, later, which = None, [None, None, None], [], []
         for i, g in enumerate(grads):
             if g is None or not (ctx.need[0] or ctx.need[1 + i]):
                 continue
+            # the wgrads share the quantised x and wait for one launch
             gx, gws[i], _ = f8.linear_backward(g.contiguous(), x, ws[i], amaxes[i], x_col, ctx.need[0], ctx.need[1 + i], False,
-                                               ctx.fp8_wgrad, ctx.gemm_algo, grad_a=gx)
+                                               ctx.fp8_wgrad, ctx.gemm_algo, a_tcast=later[0][2:] if later else None, grad_a=gx,
+                                               wgrad_later=later)
+            which += [i] * (len(later) - len(which))
+        if later:
+            qgts, sgts, (qat, *_), (sat, *_) = zip(*later)
+            for i, gw in zip(which, ops.gemm_nt_multi(qgts, qat, sgts, sat, algo=ctx.gemm_algo)):
+                gws[i] = gw
         return (gx, *gws)
 
 

@@ -111,10 +111,15 @@ class Fp8SwiGLUFn(torch.autograd.Function):
                 if x_col is None:
                     x_col = ops.col_amax(x)
                 qxt, sxt = ops.cast_colwise_transposed(x, x_col)   # shared by both wgrads
-                if need_w1:
+                if need_w1 and need_w3:
+                    q1, s1 = ops.cast_colwise_transposed(g1, g1_col)
+                    del g1
+                    q3, s3 = ops.cast_colwise_transposed(g3, g3_col)
+                    gw1, gw3 = ops.gemm_nt_multi((q1, q3), qxt, (s1, s3), sxt, algo=algo)
+                elif need_w1:
                     qgt, sgt = ops.cast_colwise_transposed(g1, g1_col)
                     gw1 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
-                if need_w3:
+                else:
                     qgt, sgt = ops.cast_colwise_transposed(g3, g3_col)
                     gw3 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
             else:

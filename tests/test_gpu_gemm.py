@@ -96,6 +96,29 @@ def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
     assert name in ops.gemm_pick(*mnk)[1]
 
 
+@pytest.mark.parametrize("rows,N,K,together", [((2008, 2048, 520), 2048, 272, True), ((2500, 2500), 2056, 16, True), ((1536, 1500), 2048, 400, True),
+                                               ((2817, 2900, 3070), 2200, 1040, True), ((256, 8), 512, 144, False),
+                                               ((1536, 1500), 2048, 4112, False),
+                                               ((2048, 2048, 2048), 2052, 128, None), ((2048, 0, 2048), 2048, 128, None)])
+def test_products_with_one_operand_in_one_launch(rows, N, K, together):
+    """Every product has the bits it has alone, in one launch or in several: last tile rows that are short, of different
+    lengths, one row alone in a tile; short column tiles; K tiles that are short, fewer than the ring; a workgroup's second
+    tile in another product than its first; outputs (N % 8) and lists (an empty product) that cannot go together."""
+    import struct
+    from lingua_amd import _lib, ops
+    if together is not None and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        parts = [v for m in rows for v in (0, m, 0, 0)]
+        assert _lib.load().l8_gemm_multi_pays(struct.pack(f"{len(parts)}q", *parts), len(rows), N, K) == together
+    g = torch.Generator().manual_seed(950 + N)
+    qb = random_fp8_bytes((N, K), g).cuda().view(torch.float8_e4m3fn)
+    sb = (torch.rand(N, 1, generator=g) + 0.5).cuda()
+    qas = [random_fp8_bytes((m, K), g).cuda().view(torch.float8_e4m3fn) for m in rows]
+    sas = [(torch.rand(m, 1, generator=g) + 0.5).cuda() for m in rows]
+    for qa, sa, out in zip(qas, sas, ops.gemm_nt_multi(qas, qb, sas, sb)):
+        want = ops.gemm_nt(qa, qb, sa, sb, algo=12 if together else 0)
+        assert out.shape == want.shape and torch.equal(out.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("algo,mnk", [(0, (40, 52, 272)), (2, (130, 200, 144)), (2, (256, 256, 128)), (12, (256, 256, 128)),
                                       (12, (300, 520, 400)), (12, (4136, 4104, 272)), (11, (520, 264, 144)), (17, (33, 50, 1040)),
                                       (18, (128, 128, 256)), (21, (65, 70, 128)), (22, (32, 64, 400))])
