@@ -188,12 +188,4 @@ L8_DEV void store8(__amdgpu_buffer_rsrc_t rs, uint32_t voff, v2i data) {
 }
 #endif
 
-// Workgroup-per-row kernels that produce their row on the fly (fused gate, fused
-// norm) keep column maxima in registers (packed pairs, NCHW * 4 dwords per
-// tensor) while that fits the 256-register budget of two workgroups per CU,
-// else in a dynamic LDS array of one bf16 per column and tensor; either way
-// every column belongs to exactly one thread, so no synchronisation is involved.
-template <int NCHW, int TENSORS>
-constexpr bool colmax_in_lds() { return NCHW * 4 * TENSORS > 32; }
-
 }  // namespace l8

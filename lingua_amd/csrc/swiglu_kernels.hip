@@ -18,9 +18,20 @@
 // last bits of the fp32 sigmoid: at most two bf16 ulps apart, identical for
 // more than 99.5 % of the elements (the bound the tests state); amax, scale
 // and e4m3 bytes are then exact functions of the bf16 values produced here.
-// One 256-thread workgroup per row (wave
-// w owns the 512-column chunks w, w+4, ...), the layout of the long-row kernel
-// of cast_kernels.hip; the amax -> scale -> cast stage is shared with it.
+// One workgroup per row (wave w of W owns the 512-column chunks w, w+W, ...),
+// the layout of the long-row kernel of cast_kernels.hip; the amax -> scale ->
+// cast stage is shared with it.
+//
+// Bound by memory: 5 (+ 2 with h) bytes per element forward, 12 backward.  What
+// reaches its rate is loads in flight, so a lane holds few chunks and a long row
+// takes more waves rather than more registers per lane: four up to 4096 columns,
+// eight up to 16384 forward (2 to 4 chunks) and up to 12288 backward (2 or 3),
+// sixteen with 2 chunks beyond.  With more than four the column maxima live in
+// LDS.  us inside a forward + backward, four waves / this: [16384,8192] forward
+// 162.5 / 156.7 (6.0 TB/s), backward 292 / 262 (6.1 TB/s); [4093,14336] forward
+// 82.6 / 76.9, backward (a two-pass kernel before) 149.7 / 124.7 (5.6 TB/s).
+// Alone, with the folds of the column maxima: backward [16384,5632] 235 / 205,
+// [16384,8704] 354 / 309, [16384,11008] 430 / 424, [16384,16384] 710 / 601.
 #include "l8_common.h"
 
 namespace l8 {
@@ -66,18 +77,18 @@ L8_DEV void gate_bwd2(uint32_t d, uint32_t a, uint32_t b, uint32_t &g1, uint32_t
   g3 = g3l | (g3h << 16);
 }
 
-template <int NCHW, bool COLMAX>
-__global__ __launch_bounds__(kGateBlock, 2) void swiglu_cast_rowwise_kernel(
+template <int NCHW, bool COLMAX, int WAVES = kGateWaves>
+__global__ __launch_bounds__(WAVES * 64, WAVES == kGateWaves ? 2 : 4) void swiglu_cast_rowwise_kernel(
     const uint16_t *__restrict__ h1, const uint16_t *__restrict__ h3, int64_t R, int C, int64_t ld1, int64_t ld3,
     uint16_t *__restrict__ hout, int64_t ldh, uint8_t *__restrict__ q, int64_t ldq, float *__restrict__ scale,
     uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule) {
-  __shared__ uint32_t red[2][kGateWaves];
+  __shared__ uint32_t red[2][WAVES];
   extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
-  constexpr bool CLDS = COLMAX && colmax_in_lds<NCHW, 1>();
+  constexpr bool CLDS = COLMAX && WAVES > kGateWaves;  // column maxima in LDS instead of registers
   v4i *lds_cm = (v4i *)dyn_lds;  // [C / 8]
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  auto col_of = [&](int j) { return (j * kGateWaves + wave) * 512 + lane * 8; };
+  auto col_of = [&](int j) { return (j * WAVES + wave) * 512 + lane * 8; };
   uint32_t cmax[(COLMAX && !CLDS) ? NCHW * 4 : 1];
   if (COLMAX) {
 #pragma unroll
@@ -127,7 +138,7 @@ __global__ __launch_bounds__(kGateBlock, 2) void swiglu_cast_rowwise_kernel(
     __syncthreads();
     uint32_t amax_bits = 0;
 #pragma unroll
-    for (int w = 0; w < kGateWaves; ++w) amax_bits = max(amax_bits, red[it & 1][w]);
+    for (int w = 0; w < WAVES; ++w) amax_bits = max(amax_bits, red[it & 1][w]);
     const RowScale rs = row_scale(amax_bits, scale_rule);
     if (threadIdx.x == 0) {
       if (scale) scale[r] = rs.s;
@@ -156,19 +167,19 @@ __global__ __launch_bounds__(kGateBlock, 2) void swiglu_cast_rowwise_kernel(
   }
 }
 
-template <int NCHW, bool COLMAX>
-__global__ __launch_bounds__(kGateBlock, 2) void swiglu_bwd_cast_rowwise_kernel(
+template <int NCHW, bool COLMAX, int WAVES = kGateWaves>
+__global__ __launch_bounds__(WAVES * 64, WAVES == kGateWaves ? 2 : 4) void swiglu_bwd_cast_rowwise_kernel(
     const uint16_t *__restrict__ dh, const uint16_t *__restrict__ h1, const uint16_t *__restrict__ h3, int64_t R, int C,
     int64_t lddh, int64_t ld1, int64_t ld3, uint16_t *__restrict__ g1out, uint16_t *__restrict__ g3out, int64_t ldg,
     uint8_t *__restrict__ q1, uint8_t *__restrict__ q3, int64_t ldq, float *__restrict__ scale1,
     float *__restrict__ scale3, uint16_t *__restrict__ col_partials1, uint16_t *__restrict__ col_partials3, int scale_rule) {
-  __shared__ uint32_t red[2][2][kGateWaves];
+  __shared__ uint32_t red[2][2][WAVES];
   extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];
-  constexpr bool CLDS = COLMAX && colmax_in_lds<NCHW, 2>();
+  constexpr bool CLDS = COLMAX && WAVES > kGateWaves;  // column maxima in LDS instead of registers
   v4i *lds_cm1 = (v4i *)dyn_lds, *lds_cm3 = lds_cm1 + C / 8;  // [C / 8] each
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
-  auto col_of = [&](int j) { return (j * kGateWaves + wave) * 512 + lane * 8; };
+  auto col_of = [&](int j) { return (j * WAVES + wave) * 512 + lane * 8; };
   uint32_t cmax1[(COLMAX && !CLDS) ? NCHW * 4 : 1], cmax3[(COLMAX && !CLDS) ? NCHW * 4 : 1];
   if (COLMAX) {
 #pragma unroll
@@ -231,7 +242,7 @@ __global__ __launch_bounds__(kGateBlock, 2) void swiglu_bwd_cast_rowwise_kernel(
     __syncthreads();
     uint32_t bits1 = 0, bits3 = 0;
 #pragma unroll
-    for (int w = 0; w < kGateWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       bits1 = max(bits1, red[it & 1][0][w]);
       bits3 = max(bits3, red[it & 1][1][w]);
     }
@@ -266,8 +277,7 @@ __global__ __launch_bounds__(kGateBlock, 2) void swiglu_bwd_cast_rowwise_kernel(
   }
 }
 
-// Wide rows (ffn dimensions beyond what a 256-thread workgroup holds in
-// registers without spilling): 1024 threads per row, two passes.  Pass 1
+// Wide rows (beyond 16384 columns, more than a workgroup holds in registers): 1024 threads per row, two passes.  Pass 1
 // computes the gate, stores the bf16 result and reduces the row amax; pass 2
 // reads the thread's own bf16 values back (they are still in L2) and casts.
 // Column maxima live in LDS (one bf16 per column and tensor, each owned by one
@@ -487,48 +497,41 @@ static int launch_bwd_wide(const void *dh, const void *h1, const void *h3, int64
   return L8_OK;
 }
 
-template <int NCHW>
+template <int NCHW, int WAVES = kGateWaves>
 static int launch_fwd(const void *h1, const void *h3, int64_t R, int64_t C, int64_t ld1, int64_t ld3, void *h, int64_t ldh,
                       void *q, int64_t ldq, float *scale, void *amax, float *col_amax, void *ws, hipStream_t st) {
   const int64_t blocks = gate_blocks(R);
   if (col_amax) {
-    const size_t lds = colmax_in_lds<NCHW, 1>() ? (size_t)C * 2 : 0;
-    if (lds > 48 * 1024) {  // above the default limit for dynamic LDS; idempotent
-      static bool raised[kMaxDev] = {};
-      const int slot = device_slot();
-      if (slot < 0 || !raised[slot])
-        L8_HIP(hipFuncSetAttribute((const void *)swiglu_cast_rowwise_kernel<NCHW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
-      if (slot >= 0) raised[slot] = true;
-    }
-    hipLaunchKernelGGL((swiglu_cast_rowwise_kernel<NCHW, true>), dim3((unsigned)blocks), dim3(kGateBlock), lds, st,
+    const size_t lds = (WAVES > kGateWaves) ? (size_t)C * 2 : 0;
+    hipLaunchKernelGGL((swiglu_cast_rowwise_kernel<NCHW, true, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), lds, st,
                        (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, ld1, ld3, (uint16_t *)h, ldh, (uint8_t *)q, ldq,
                        scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule());
     L8_HIP(hipGetLastError());
     return fold_colmax(ws, blocks, C, col_amax, st);
   }
-  hipLaunchKernelGGL((swiglu_cast_rowwise_kernel<NCHW, false>), dim3((unsigned)blocks), dim3(kGateBlock), 0, st,
+  hipLaunchKernelGGL((swiglu_cast_rowwise_kernel<NCHW, false, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), 0, st,
                      (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, ld1, ld3, (uint16_t *)h, ldh, (uint8_t *)q, ldq,
                      scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule());
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
 
-template <int NCHW>
+template <int NCHW, int WAVES = kGateWaves>
 static int launch_bwd(const void *dh, const void *h1, const void *h3, int64_t R, int64_t C, int64_t lddh, int64_t ld1,
                       int64_t ld3, void *g1, void *g3, int64_t ldg, void *q1, void *q3, int64_t ldq, float *s1, float *s3,
                       float *ca1, float *ca3, void *ws, hipStream_t st) {
   const int64_t blocks = gate_blocks(R);
   if (ca1) {
     uint16_t *w1 = (uint16_t *)ws, *w3 = w1 + blocks * C;
-    const size_t lds = colmax_in_lds<NCHW, 2>() ? (size_t)C * 4 : 0;
+    const size_t lds = (WAVES > kGateWaves) ? (size_t)C * 4 : 0;
     if (lds > 48 * 1024) {  // above the default limit for dynamic LDS; idempotent
       static bool raised[kMaxDev] = {};
       const int slot = device_slot();
       if (slot < 0 || !raised[slot])
-        L8_HIP(hipFuncSetAttribute((const void *)swiglu_bwd_cast_rowwise_kernel<NCHW, true>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
+        L8_HIP(hipFuncSetAttribute((const void *)swiglu_bwd_cast_rowwise_kernel<NCHW, true, WAVES>, hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024));
       if (slot >= 0) raised[slot] = true;
     }
-    hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_kernel<NCHW, true>), dim3((unsigned)blocks), dim3(kGateBlock), lds, st,
+    hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_kernel<NCHW, true, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), lds, st,
                        (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,
                        (uint16_t *)g1, (uint16_t *)g3, ldg, (uint8_t *)q1, (uint8_t *)q3, ldq, s1, s3, w1, w3, l8::scale_rule());
     L8_HIP(hipGetLastError());
@@ -536,7 +539,7 @@ static int launch_bwd(const void *dh, const void *h1, const void *h3, int64_t R,
     if (rc != L8_OK) return rc;
     return fold_colmax(w3, blocks, C, ca3, st);
   }
-  hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_kernel<NCHW, false>), dim3((unsigned)blocks), dim3(kGateBlock), 0, st,
+  hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_kernel<NCHW, false, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), 0, st,
                      (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,
                      (uint16_t *)g1, (uint16_t *)g3, ldg, (uint8_t *)q1, (uint8_t *)q3, ldq, s1, s3, (uint16_t *)nullptr,
                      (uint16_t *)nullptr, l8::scale_rule());
@@ -576,12 +579,12 @@ extern "C" int l8_swiglu_cast_rowwise(const void *h1, const void *h3, int64_t R,
   }
   hipStream_t st = (hipStream_t)stream;
   const int64_t nchw = ((C + 511) / 512 + kGateWaves - 1) / kGateWaves;
-#define L8_FWD(N) return launch_fwd<N>(h1, h3, R, C, ld1, ld3, h, ldh, q, ldq, scale, amax, col_amax, workspace, st)
+#define L8_FWD(...) return launch_fwd<__VA_ARGS__>(h1, h3, R, C, ld1, ld3, h, ldh, q, ldq, scale, amax, col_amax, workspace, st)
   if (nchw <= 1) L8_FWD(1);
   if (nchw <= 2) L8_FWD(2);
-  if (nchw <= 4) L8_FWD(4);
-  if (nchw <= 6) L8_FWD(6);
-  if (nchw <= 8) L8_FWD(8);
+  if (nchw <= 4) L8_FWD(2, 8);
+  if (nchw <= 6) L8_FWD(3, 8);
+  if (nchw <= 8) L8_FWD(4, 8);
 #undef L8_FWD
   return launch_fwd_wide(h1, h3, R, C, ld1, ld3, h, ldh, q, ldq, scale, amax, col_amax, workspace, st);
 }
@@ -608,13 +611,14 @@ extern "C" int l8_swiglu_bwd_cast_rowwise(const void *dh, const void *h1, const 
   }
   hipStream_t st = (hipStream_t)stream;
   const int64_t nchw = ((C + 511) / 512 + kGateWaves - 1) / kGateWaves;
-#define L8_BWD(N)                                                                                                  \
-  return launch_bwd<N>(dh, h1, h3, R, C, lddh, ld1, ld3, g1, g3, ldg, q1, q3, ldq, scale1, scale3, col_amax1, col_amax3, \
-                       workspace, st)
+#define L8_BWD(...)                                                                                                      \
+  return launch_bwd<__VA_ARGS__>(dh, h1, h3, R, C, lddh, ld1, ld3, g1, g3, ldg, q1, q3, ldq, scale1, scale3, col_amax1, \
+                                 col_amax3, workspace, st)
   if (nchw <= 1) L8_BWD(1);
   if (nchw <= 2) L8_BWD(2);
-  if (nchw <= 4) L8_BWD(4);
-  if (nchw <= 6) L8_BWD(6);
+  if (nchw <= 4) L8_BWD(2, 8);
+  if (nchw <= 6) L8_BWD(3, 8);
+  if (nchw <= 8) L8_BWD(2, 16);
 #undef L8_BWD
   return launch_bwd_wide(dh, h1, h3, R, C, lddh, ld1, ld3, g1, g3, ldg, q1, q3, ldq, scale1, scale3, col_amax1, col_amax3,
                          workspace, st);

@@ -104,6 +104,13 @@ def test_backward_gate_and_casts(shape, with_col):
     check_cast_of(g3, q3, s3, None, c3, "g3")
 
 
+@pytest.mark.parametrize("shape", [(3, 4104), (2, 8200), (3, 12288), (2, 12296), (3, 16384), (2, 16392), (515, 8184)])
+def test_gate_kernels_where_the_rows_take_more_waves(shape):
+    """The row lengths at which another kernel takes over, and more rows than workgroups."""
+    test_forward_gate_and_cast(shape, True)
+    test_backward_gate_and_casts(shape, True)
+
+
 def test_strided_inputs_and_nonfinite_rows():
     from lingua_amd import ops
     R, C = 12, 520
