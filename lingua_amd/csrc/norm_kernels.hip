@@ -17,7 +17,8 @@
 // can differ from the eager result in the last bf16 bit of an element now and
 // then (the tests bound it: at most one bf16 ulp, > 99.5 % identical).
 // Two layouts, as in the row-wise casts: a wavefront per row for short rows, a
-// 256-thread workgroup per row for the longer ones.
+// 256-thread workgroup per row for the longer ones; both add a row up in the same
+// order, so a row's result does not hang on the layout.
 #include "l8_common.h"
 
 namespace l8 {
@@ -112,17 +113,21 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_wave_kerne
   while (r < R) {
     const int64_t rn = r + stride;
     load_norm_row<NCH>(nxt, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
-    float ss = 0.0f;
+    // each chunk of 512 columns is summed for itself and the chunks are added in order, as the waves of a workgroup that
+    // shares a row add theirs: one order of summation, hence one result, in both layouts
+    float tot = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NCH; ++j)
+    for (int j = 0; j < NCH; ++j) {
+      float ss = 0.0f;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const float lo = __uint_as_float((uint32_t)cur[j][k] << 16), hi = __uint_as_float((uint32_t)cur[j][k] & 0xffff0000u);
         ss += lo * lo;
         ss += hi * hi;
       }
-    ss = wave_sum_f32(ss);
-    const float rinv = 1.0f / sqrtf(ss * inv_c + eps);
+      tot += wave_sum_f32(ss);
+    }
+    const float rinv = 1.0f / sqrtf(tot * inv_c + eps);
     const __amdgpu_buffer_rsrc_t rsY = make_rsrc(y + r * ldy, (uint32_t)C * 2u);
     uint32_t m = 0;
 #pragma unroll
@@ -279,16 +284,20 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_cast_rowwise_kernel(
 // Backward of the norm: with xhat = x * r and gh = gy * w,
 //   gx = (gh - xhat * mean(gh * xhat)) * r        (bf16)
 //   gw = sum over rows of gy * xhat               (fp32)
-// One workgroup per row again; the row products for gw are accumulated in
-// registers over all rows a workgroup sees and leave as one row of fp32
-// partial sums per workgroup, which rmsnorm_gw_fold_kernel adds up column by
-// column in a fixed order (no atomics: the result does not depend on timing).
-template <int NCHW, bool W_F32>
+// One workgroup per row, also for short rows; the row products for gw are
+// accumulated in registers over all rows a workgroup sees and leave as one row
+// of fp32 partial sums per workgroup, which rmsnorm_gw_fold_kernel adds up column
+// by column.  Which rows meet in a partial sum, and the order of every sum, hang
+// on the number of rows alone (no atomics: the result does not depend on timing).
+// Rows are requested AHEAD - 1 rows before they are used: a row of one chunk per
+// lane (up to 2048 columns) is too few bytes in flight for one row ahead.
+template <int NCHW, int AHEAD, bool W_F32>
 __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
     const uint16_t *__restrict__ gy, const uint16_t *__restrict__ x, const void *__restrict__ w,
     const float *__restrict__ rstd, int64_t R, int C, int64_t ldg, int64_t ldx, uint16_t *__restrict__ gx, int64_t ldgx,
     float *__restrict__ gw_partials) {
 #if defined(__HIP_DEVICE_COMPILE__)
+  static_assert(AHEAD % 2 == 0, "a buffer meets the same half of `red` every time");
   __shared__ float red[2][kNormWaves];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -301,58 +310,60 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) gwacc[j][e] = 0.0f;
   const float inv_c = 1.0f / (float)C;
-  v4i xc[NCHW], gc[NCHW], xn[NCHW], gn[NCHW];
-  float rinv = rstd[blockIdx.x];  // the grid is never larger than R
-  load_norm_row<NCHW>(xc, x, blockIdx.x, R, ldx, C, [&](int j) { return col_of(j); });
-  load_norm_row<NCHW>(gc, gy, blockIdx.x, R, ldg, C, [&](int j) { return col_of(j); });
-  int it = 0;
-  for (int64_t r = blockIdx.x; r < R; r += gridDim.x, ++it) {
-    const int64_t rn = r + gridDim.x;
-    const float rinv_n = rstd[rn < R ? rn : r];
-    load_norm_row<NCHW>(xn, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
-    load_norm_row<NCHW>(gn, gy, rn, R, ldg, C, [&](int j) { return col_of(j); });
-    auto xhat = [&](int j, int e) {
-      const uint32_t p = (uint32_t)xc[j][e >> 1];
-      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16)) * rinv;
-    };
-    auto grad = [&](int j, int e) {
-      const uint32_t p = (uint32_t)gc[j][e >> 1];
-      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
-    };
-    float dot = 0.0f;
+  v4i xb[AHEAD][NCHW], gb[AHEAD][NCHW];
+  float rb[AHEAD];
+  auto request = [&](int a, int64_t r) {  // a row beyond R: zeros, nothing is read
+    rb[a] = rstd[r < R ? r : 0];
+    load_norm_row<NCHW>(xb[a], x, r, R, ldx, C, [&](int j) { return col_of(j); });
+    load_norm_row<NCHW>(gb[a], gy, r, R, ldg, C, [&](int j) { return col_of(j); });
+  };
 #pragma unroll
-    for (int j = 0; j < NCHW; ++j)
+  for (int a = 0; a < AHEAD - 1; ++a) request(a, blockIdx.x + a * (int64_t)gridDim.x);
+  for (int64_t r0 = blockIdx.x; r0 < R; r0 += (int64_t)AHEAD * gridDim.x) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float ge = grad(j, e), xh = xhat(j, e);
-        gwacc[j][e] += ge * xh;
-        dot += (ge * wt.get(j, e)) * xh;
+    for (int a = 0; a < AHEAD; ++a) {
+      const int64_t r = r0 + a * (int64_t)gridDim.x;
+      if (r >= R) break;  // the same for the whole workgroup
+      request((a + AHEAD - 1) % AHEAD, r + (AHEAD - 1) * (int64_t)gridDim.x);
+      const v4i(&xc)[NCHW] = xb[a], (&gc)[NCHW] = gb[a];
+      const float rinv = rb[a];
+      auto xhat = [&](int j, int e) {
+        const uint32_t p = (uint32_t)xc[j][e >> 1];
+        return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16)) * rinv;
+      };
+      auto grad = [&](int j, int e) {
+        const uint32_t p = (uint32_t)gc[j][e >> 1];
+        return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
+      };
+      float dot = 0.0f;
+#pragma unroll
+      for (int j = 0; j < NCHW; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float ge = grad(j, e), xh = xhat(j, e);
+          gwacc[j][e] += ge * xh;
+          dot += (ge * wt.get(j, e)) * xh;
+        }
+      dot = wave_sum_f32(dot);
+      if (lane == 0) red[a & 1][wave] = dot;
+      __syncthreads();
+      float tot = 0.0f;
+#pragma unroll
+      for (int wv = 0; wv < kNormWaves; ++wv) tot += red[a & 1][wv];
+      const float c1 = tot * inv_c;
+      const __amdgpu_buffer_rsrc_t rsG = make_rsrc(gx + r * ldgx, (uint32_t)C * 2u);
+#pragma unroll
+      for (int j = 0; j < NCHW; ++j) {
+        v4i out;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t lo = bf16_rne_bits((grad(j, 2 * k) * wt.get(j, 2 * k) - xhat(j, 2 * k) * c1) * rinv);
+          const uint32_t hi = bf16_rne_bits((grad(j, 2 * k + 1) * wt.get(j, 2 * k + 1) - xhat(j, 2 * k + 1) * c1) * rinv);
+          out[k] = (int)(lo | (hi << 16));
+        }
+        store16_nt(rsG, (uint32_t)col_of(j) * 2u, out);
       }
-    dot = wave_sum_f32(dot);
-    if (lane == 0) red[it & 1][wave] = dot;
-    __syncthreads();
-    float tot = 0.0f;
-#pragma unroll
-    for (int wv = 0; wv < kNormWaves; ++wv) tot += red[it & 1][wv];
-    const float c1 = tot * inv_c;
-    const __amdgpu_buffer_rsrc_t rsG = make_rsrc(gx + r * ldgx, (uint32_t)C * 2u);
-#pragma unroll
-    for (int j = 0; j < NCHW; ++j) {
-      v4i out;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = bf16_rne_bits((grad(j, 2 * k) * wt.get(j, 2 * k) - xhat(j, 2 * k) * c1) * rinv);
-        const uint32_t hi = bf16_rne_bits((grad(j, 2 * k + 1) * wt.get(j, 2 * k + 1) - xhat(j, 2 * k + 1) * c1) * rinv);
-        out[k] = (int)(lo | (hi << 16));
-      }
-      store16_nt(rsG, (uint32_t)col_of(j) * 2u, out);
     }
-#pragma unroll
-    for (int j = 0; j < NCHW; ++j) {
-      xc[j] = xn[j];
-      gc[j] = gn[j];
-    }
-    rinv = rinv_n;
   }
 #pragma unroll
   for (int j = 0; j < NCHW; ++j) {
@@ -366,129 +377,49 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
 #endif
 }
 
-// Short rows: a wavefront per row, the next row's gy and x requested ahead; the row products for gw are accumulated per
-// lane over all rows of the wave and meet in LDS at the end, wave after wave (a fixed order).
-template <int NCH, bool W_F32>
-__global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_wave_kernel(
-    const uint16_t *__restrict__ gy, const uint16_t *__restrict__ x, const void *__restrict__ w,
-    const float *__restrict__ rstd, int64_t R, int C, int64_t ldg, int64_t ldx, uint16_t *__restrict__ gx, int64_t ldgx,
-    float *__restrict__ gw_partials) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  extern __shared__ __attribute__((aligned(16))) uint8_t dyn_lds[];  // [C] floats
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  auto col_of = [&](int j) { return j * 512 + lane * 8; };
-  NormWeights<NCH, W_F32> wt;
-  wt.load(w, C, [&](int j) { return col_of(j); });
-  float gwacc[NCH][8];
+// gw[c] = sum over the partial rows: eight sums of every eighth row, each in the order of the rows, added in order.
+// A workgroup owns 32 columns -- one 128-byte line of every partial row -- and passes them through LDS, 256 rows at a
+// time: 16 bytes per thread and load, the next 256 rows in flight under the additions, which come one after the other
+// but read LDS.  (With each addition waiting for its row from memory the fold of 512 rows of 2048 columns took 20 us.)
+constexpr int kGwCols = 32, kGwThreads = 1024, kGwRows = 256, kGwSums = 8;
+__global__ __launch_bounds__(kGwThreads) void rmsnorm_gw_fold_kernel(const float *__restrict__ partials, int n_slots, int C,
+                                                                     float *__restrict__ gw) {
+  constexpr int QUADS = kGwCols / 4, STEP = kGwThreads / QUADS, LOADS = kGwRows / STEP;  // threads to a row, rows to a load
+  __shared__ v4f rows[kGwRows][QUADS];
+  __shared__ float sums[kGwSums][kGwCols];
+  const int quad = threadIdx.x % QUADS, row = threadIdx.x / QUADS;
+  const int tx = threadIdx.x % kGwCols, ty = threadIdx.x / kGwCols;
+  const int col = blockIdx.x * kGwCols + quad * 4;
+  v4f part[LOADS];
+  auto request = [&](int s0) {  // without a branch around a load: a row beyond the last is the last again
 #pragma unroll
-  for (int j = 0; j < NCH; ++j)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) gwacc[j][e] = 0.0f;
-  const float inv_c = 1.0f / (float)C;
-  const int64_t stride = (int64_t)gridDim.x * kNormWaves;
-  int64_t r = (int64_t)blockIdx.x * kNormWaves + wave;
-  v4i xc[NCH], gc[NCH], xn[NCH], gn[NCH];
-  float rinv = r < R ? rstd[r] : 0.0f, rinv_n = 0.0f;
-  load_norm_row<NCH>(xc, x, r, R, ldx, C, [&](int j) { return col_of(j); });
-  load_norm_row<NCH>(gc, gy, r, R, ldg, C, [&](int j) { return col_of(j); });
-  while (r < R) {
-    const int64_t rn = r + stride;
-    rinv_n = rstd[rn < R ? rn : r];
-    load_norm_row<NCH>(xn, x, rn, R, ldx, C, [&](int j) { return col_of(j); });
-    load_norm_row<NCH>(gn, gy, rn, R, ldg, C, [&](int j) { return col_of(j); });
-    auto xhat = [&](int j, int e) {
-      const uint32_t p = (uint32_t)xc[j][e >> 1];
-      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16)) * rinv;
-    };
-    auto grad = [&](int j, int e) {
-      const uint32_t p = (uint32_t)gc[j][e >> 1];
-      return __uint_as_float((e & 1) ? (p & 0xffff0000u) : (p << 16));
-    };
-    float dot = 0.0f;
-#pragma unroll
-    for (int j = 0; j < NCH; ++j)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float ge = grad(j, e), xh = xhat(j, e);
-        gwacc[j][e] += ge * xh;
-        dot += (ge * wt.get(j, e)) * xh;
-      }
-    const float c1 = wave_sum_f32(dot) * inv_c;
-    const __amdgpu_buffer_rsrc_t rsG = make_rsrc(gx + r * ldgx, (uint32_t)C * 2u);
-#pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      v4i out;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t lo = bf16_rne_bits((grad(j, 2 * k) * wt.get(j, 2 * k) - xhat(j, 2 * k) * c1) * rinv);
-        const uint32_t hi = bf16_rne_bits((grad(j, 2 * k + 1) * wt.get(j, 2 * k + 1) - xhat(j, 2 * k + 1) * c1) * rinv);
-        out[k] = (int)(lo | (hi << 16));
-      }
-      store16_nt(rsG, (uint32_t)col_of(j) * 2u, out);
+    for (int i = 0; i < LOADS; ++i) {
+      const int sl = s0 + i * STEP + row;
+      part[i] = *(const v4f *)(partials + (int64_t)(sl < n_slots ? sl : n_slots - 1) * C + (col < C ? col : 0));
     }
+  };
+  if (n_slots > 0) request(0);
+  float s = 0.0f;
+  for (int s0 = 0; s0 < n_slots; s0 += kGwRows) {
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      xc[j] = xn[j];
-      gc[j] = gn[j];
-    }
-    rinv = rinv_n;
-    r = rn;
-  }
-  v4f *lds4 = (v4f *)dyn_lds;
-  for (int wv = 0; wv < kNormWaves; ++wv) {
-    if (wave == wv) {
-#pragma unroll
-      for (int j = 0; j < NCH; ++j) {
-        const int c = col_of(j);
-        if (c < C) {
-#pragma unroll
-          for (int half = 0; half < 2; ++half) {
-            v4f mine = {gwacc[j][4 * half], gwacc[j][4 * half + 1], gwacc[j][4 * half + 2], gwacc[j][4 * half + 3]};
-            if (wv > 0) mine = lds4[c / 4 + half] + mine;
-            if (wv == kNormWaves - 1) *(v4f *)(gw_partials + (int64_t)blockIdx.x * C + c + 4 * half) = mine;
-            else lds4[c / 4 + half] = mine;
-          }
-        }
-      }
+    for (int i = 0; i < LOADS; ++i) rows[i * STEP + row][quad] = part[i];
+    __syncthreads();
+    if (s0 + kGwRows < n_slots) request(s0 + kGwRows);
+    if (ty < kGwSums) {
+      const int n = n_slots - s0 < kGwRows ? n_slots - s0 : kGwRows;
+#pragma unroll 8
+      for (int sl = ty; sl < n; sl += kGwSums) s += reinterpret_cast<const float *>(&rows[sl][0])[tx];
     }
     __syncthreads();
   }
-#endif
-}
-
-// gw[c] = sum over the partial rows, in a fixed order.  A workgroup owns 32 columns -- one 128-byte line of every
-// partial row -- and its 1024 threads read 16 bytes each from 128 rows at a time, so that the few hundred rows are a
-// handful of loads per thread, all in flight together (with eight rows at a time the loads came one after the other:
-// 20 us for 512 rows of 2048 columns, now 4.8); the row groups then meet in LDS.
-constexpr int kGwCols = 32, kGwThreads = 1024, kGwGroups = kGwThreads / 8;
-__global__ __launch_bounds__(kGwThreads) void rmsnorm_gw_fold_kernel(const float *__restrict__ partials, int n_slots, int C,
-                                                                     float *__restrict__ gw) {
-  __shared__ v4f red[kGwGroups][8];
-  __shared__ float red2[8][kGwCols];
-  const int cc = threadIdx.x & 7, sg = threadIdx.x >> 3;
-  const int col = blockIdx.x * kGwCols + cc * 4;
-  v4f s = {0.0f, 0.0f, 0.0f, 0.0f};
-  if (col < C) {
-#pragma unroll 4
-    for (int sl = sg; sl < n_slots; sl += kGwGroups) s += *(const v4f *)(partials + (int64_t)sl * C + col);
-  }
-  red[sg][cc] = s;
+  if (ty < kGwSums) sums[ty][tx] = s;
   __syncthreads();
-  if (threadIdx.x < 256) {
-    const int c = threadIdx.x & 31, part = threadIdx.x >> 5;
-    float t = 0.0f;
+  const int c = blockIdx.x * kGwCols + tx;
+  if (ty == 0 && c < C) {
+    float t = sums[0][tx];
 #pragma unroll
-    for (int g = 0; g < kGwGroups / 8; ++g) t += reinterpret_cast<const float *>(&red[part * (kGwGroups / 8) + g][0])[c];
-    red2[part][c] = t;
-  }
-  __syncthreads();
-  if (threadIdx.x < kGwCols) {
-    float t = red2[0][threadIdx.x];
-#pragma unroll
-    for (int part = 1; part < 8; ++part) t += red2[part][threadIdx.x];
-    const int c = blockIdx.x * kGwCols + threadIdx.x;
-    if (c < C) gw[c] = t;
+    for (int k = 1; k < kGwSums; ++k) t += sums[k][tx];
+    gw[c] = t;
   }
 }
 
@@ -499,13 +430,15 @@ static int64_t norm_blocks(int64_t R) {
 
 constexpr int64_t kNormMaxC = 4 * kNormWaves * 512;  // 8192: the weights of a thread's columns live in registers
 
-// Which layout: a wavefront per row up to 2048 columns, a workgroup per row beyond (up to 8192), where a wave's row,
-// the row requested ahead, the weights and the column maxima or gw sums no longer fit 256 registers.  Inside a 1B-sized
-// step, [16384,2048], us: forward 59 (a workgroup per row, each row requested when its turn comes) -> 49 (next row
-// requested ahead) -> 34 (a wavefront per row: 168 MB at 4.9 TB/s); backward 45 -> 37 -> 35 (201 MB at 5.7 TB/s); the
-// fold of gw 20 -> 4.8.  [4093,4096], workgroup per row with the next row ahead: forward 25.5 -> 20.5, backward
-// 23.8 -> 20.5, fold 17.6 -> 4.9.  Four workgroups per compute unit instead of two: forward +-4 %, backward 7 % slower.
-// workgroups of the wavefront-per-row kernels (never more than norm_blocks(R), which the workspaces are sized for)
+// Which layout, forward: a wavefront per row up to 2048 columns, a workgroup per row beyond (up to 8192), where a wave's
+// row, the row requested ahead, the weights and the column maxima no longer fit 256 registers.  Inside a 1B-sized step,
+// [16384,2048], us: 59 (a workgroup per row, each row requested when its turn comes) -> 49 (next row requested ahead) ->
+// 34 (a wavefront per row: 168 MB at 4.9 TB/s); [4093,4096], workgroup per row with the next row ahead: 25.5 -> 20.5.
+// Backward: a workgroup per row, whose share of gw is a sum over rows 2 x (compute units) apart, on its own, back to
+// back, us: [16384,2048] 46.2 (no row ahead) -> 35.5 (three ahead: 201 MB at 5.7 TB/s; a wavefront per row the same),
+// [8192,1024] 20.3 -> 15.8, [64,2048] 4.3 -> 3.8, [4093,4096] 23.7 -> 21.8 (one ahead); the fold of gw 17 to 22 -> 4.
+// Four workgroups per compute unit instead of two: forward +-4 %, backward 7 % slower.
+// workgroups of the wavefront-per-row kernel (never more than norm_blocks(R), which the workspaces are sized for)
 static int64_t norm_wave_blocks(int64_t R) { return norm_blocks((R + kNormWaves - 1) / kNormWaves); }
 
 // N = chunks of 512 columns per wave (WAVE) or of 2048 per workgroup
@@ -528,16 +461,12 @@ static int launch_norm(const void *x, const void *w, int64_t R, int64_t C, int64
   return col_amax ? fold_colmax(ws, blocks, C, col_amax, st) : L8_OK;
 }
 
-template <bool WAVE, int N, bool W_F32>
+template <int N, bool W_F32>
 static int launch_norm_bwd(const void *gy, const void *x, const void *w, const float *rstd, int64_t R, int64_t C,
                            int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, float *gw, void *ws, hipStream_t st) {
-  const int64_t blocks = WAVE ? norm_wave_blocks(R) : norm_blocks(R);
-  auto go = [&](auto kernel, size_t lds) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kNormBlock), lds, st, (const uint16_t *)gy, (const uint16_t *)x, w,
-                       rstd, R, (int)C, ldg, ldx, (uint16_t *)gx, ldgx, (float *)ws);
-  };
-  if constexpr (WAVE) go(rmsnorm_bwd_wave_kernel<N, W_F32>, (size_t)C * 4);
-  else go(rmsnorm_bwd_kernel<N, W_F32>, 0);
+  const int64_t blocks = norm_blocks(R);
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<N, N == 1 ? 4 : 2, W_F32>), dim3((unsigned)blocks), dim3(kNormBlock), 0, st, (const uint16_t *)gy,
+                     (const uint16_t *)x, w, rstd, R, (int)C, ldg, ldx, (uint16_t *)gx, ldgx, (float *)ws);
   L8_HIP(hipGetLastError());
   hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + kGwCols - 1) / kGwCols)), dim3(kGwThreads), 0, st,
                      (const float *)ws, (int)blocks, (int)C, gw);
@@ -576,13 +505,13 @@ extern "C" int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int 
   L8_REQUIRE(workspace && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0,
              "l8_rmsnorm_bwd: needs a 16-byte aligned workspace of %lld bytes", (long long)need);
   hipStream_t st = (hipStream_t)stream;
-#define L8_NORM_BWD(WAVE, N)                                                                                              \
-  return w_is_f32 ? launch_norm_bwd<WAVE, N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)            \
-                  : launch_norm_bwd<WAVE, N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)
-  const int64_t nch = (C + 511) / 512, nchw = (nch + kNormWaves - 1) / kNormWaves;
-  if (nch <= 4) L8_NORM_BWD(true, 4);
-  if (nchw <= 2) L8_NORM_BWD(false, 2);
-  L8_NORM_BWD(false, 4);
+#define L8_NORM_BWD(N)                                                                                               \
+  return w_is_f32 ? launch_norm_bwd<N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)             \
+                  : launch_norm_bwd<N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)
+  const int64_t nchw = ((C + 511) / 512 + kNormWaves - 1) / kNormWaves;
+  if (nchw <= 1) L8_NORM_BWD(1);
+  if (nchw <= 2) L8_NORM_BWD(2);
+  L8_NORM_BWD(4);
 #undef L8_NORM_BWD
 }
 

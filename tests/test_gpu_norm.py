@@ -106,6 +106,46 @@ def test_either_side_of_the_layout_line(shape):
     assert rel_l2(gx, xa.grad) <= 1e-3 and rel_l2(gw, wa.grad) <= 1e-4
 
 
+@pytest.mark.parametrize("C", [16, 520, 1024, 2040, 2048])
+@pytest.mark.parametrize("R", [3, 700, 2051])
+def test_one_order_of_summation_in_every_layout(R, C):
+    """A row padded with zeros to four times its length takes the longest layout; with eps / 4 its mean is a quarter, so
+    rstd, y, gx and gw are exactly twice those of the short row -- bit for bit, if both add up in one order."""
+    from lingua_amd import ops
+    x, gy = (seeded_bf16((R, C), std=s, seed=R + C + i).cuda() for i, s in enumerate((2.0, 0.05)))
+    w = (1.0 + 0.1 * torch.randn(C, generator=torch.Generator().manual_seed(C))).cuda()
+    pad = lambda t: torch.nn.functional.pad(t, (0, 3 * C)).contiguous()
+    y, _, _, rstd = ops.rmsnorm_cast_rowwise(x, w, EPS)
+    y4, _, _, rstd4 = ops.rmsnorm_cast_rowwise(pad(x), pad(w), EPS / 4)
+    assert bits_equal(rstd4, 2 * rstd) and bits_equal(y4[:, :C].contiguous(), 2 * y)
+    gx, gw = ops.rmsnorm_bwd(gy, x, w, rstd)
+    gx4, gw4 = ops.rmsnorm_bwd(pad(gy), pad(x), pad(w), rstd4)
+    assert bits_equal(gx4[:, :C].contiguous(), 2 * gx) and bits_equal(gw4[:C].contiguous(), 2 * gw)
+
+
+@pytest.mark.parametrize("R,C", [(1, 8), (7, 40), (300, 2048), (1300, 72), (1027, 2056), (513, 4104)])
+def test_gw_is_added_up_in_the_stated_order(R, C):
+    """gw, bit for bit: row r belongs to partial sum r % (2 x compute units), each added up in the order of
+    the rows (products rounded first: the library is built without contraction); eight sums of every eighth partial sum,
+    then those eight in order."""
+    from lingua_amd import ops
+    x, gy = (seeded_bf16((R, C), std=s, seed=R * 3 + C + i) for i, s in enumerate((2.0, 0.05)))
+    rstd = torch.rand(R, 1, generator=torch.Generator().manual_seed(R)) + 0.5
+    slots = min(R, 2 * torch.cuda.get_device_properties(0).multi_processor_count)
+    part = torch.zeros(slots, C)
+    for r in range(0, R, slots):
+        xh = x[r:r + slots].float() * rstd[r:r + slots]
+        part[:xh.shape[0]] += gy[r:r + slots].float() * xh
+    sums = torch.zeros(8, C)
+    for s in range(slots):
+        sums[s % 8] += part[s]
+    want = sums[0]
+    for k in range(1, 8):
+        want = want + sums[k]
+    _, gw = ops.rmsnorm_bwd(gy.cuda(), x.cuda(), torch.ones(C, device="cuda"), rstd.cuda())
+    assert bits_equal(gw.cpu(), want)
+
+
 def test_argument_errors():
     from lingua_amd import ops
     x = seeded_bf16((4, 64)).cuda()
