@@ -373,7 +373,7 @@ def linear_infer(a, b_t, bias):
             x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
     w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
     ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, w_cast, w_cast is not None, None, config.gemm_algo)
-    if hit is None and x_cast is not None:
+    if hit is None and x_cast is not None and out.numel():   # nothing is quantised for a linear without outputs
         _fwd_cast.put(a, (*x_cast, None), b_t.data_ptr())
     return out
 

@@ -67,6 +67,17 @@ def test_linears_share_an_activation_and_see_it_change():
         float8.clear_cast_memos()
 
 
+def test_a_linear_without_outputs_leaves_no_quantised_activation():
+    """The next linear on the activation quantises it: nothing was written for the one before it."""
+    from lingua_amd import float8
+    none, some = make(256, 0, False), make(256, 272, False)
+    x = seeded_bf16((100, 256), seed=5).cuda()
+    with torch.no_grad():
+        assert none(x).shape == (100, 0) and not float8._fwd_cast.entries
+        assert rel_l2(some(x), oracle.linear_forward(x.cpu(), some.weight.detach().cpu())) <= 1e-3
+    float8.clear_cast_memos()
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
 @pytest.mark.parametrize("K", [16, 272, 4096, 4112, 8192, 8208, 12288, 12304])
 def test_weight_quantised_inside_the_product(M, K):

@@ -82,6 +82,33 @@ def test_linear_call_validates_its_arguments_on_the_host():
     assert lib.l8_linear_fwd(pack(qx=fake)) == -1 and lib.l8_linear_fwd(None) == -1
 
 
+@pytest.fixture
+def recorded_linear_calls(monkeypatch):
+    """The inference call of a linear on CPU tensors, its library call recorded instead of made."""
+    from lingua_amd import float8
+    calls = []
+
+    def linear_fwd(x, w, bias, y, x_cast=None, x_ready=False, w_cast=None, w_ready=False, *rest, **kw):
+        calls.append({"outputs": y.shape[-1], "x_cast": x_cast, "x_ready": x_ready})
+
+    monkeypatch.setattr(float8, "_check_operands", lambda a, b_t: None)
+    monkeypatch.setattr(ops, "linear_fwd", linear_fwd)
+    monkeypatch.setattr(ops, "current_stream_ptr", lambda index: 0)
+    float8.clear_cast_memos()
+    yield calls
+    float8.clear_cast_memos()
+
+
+def test_only_a_written_activation_cast_is_shared(recorded_linear_calls):
+    """Above 64 tokens linears share the quantised activation -- but not the memory that a linear without outputs, for
+    which the library has nothing to do, never wrote."""
+    from lingua_amd import float8
+    x = torch.zeros(80, 32, dtype=torch.bfloat16)
+    for outputs in (0, 48, 64):
+        float8.linear_infer(x, torch.zeros(outputs, 32, dtype=torch.bfloat16), None)
+    assert [(c["outputs"], c["x_ready"]) for c in recorded_linear_calls] == [(0, False), (48, False), (64, True)]
+
+
 def test_no_cpu_path():
     x = torch.zeros(4, 16, dtype=torch.bfloat16)
     with pytest.raises(RuntimeError, match="no CPU path"):
