@@ -369,8 +369,11 @@ def linear_infer(a, b_t, bias):
     x_cast = hit = None
     if config.share_input_casts:
         x_cast = hit = _fwd_cast.get(a, b_t.data_ptr())
-        if hit is None and tokens > _UNSHARED_TOKENS:
-            x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
+        if hit is None:
+            if tokens > _UNSHARED_TOKENS:
+                x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
+            else:   # nothing of its own to file, but an earlier activation (a prompt's, during generation) is not kept alive
+                _fwd_cast.clear(a)
     w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
     ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, w_cast, w_cast is not None, None, config.gemm_algo)
     if hit is None and x_cast is not None and out.numel():   # nothing is quantised for a linear without outputs

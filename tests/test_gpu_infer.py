@@ -78,6 +78,17 @@ def test_a_linear_without_outputs_leaves_no_quantised_activation():
     float8.clear_cast_memos()
 
 
+def test_a_prompts_activation_is_not_kept_during_generation():
+    """The memo holds the last activation alive; a call with few tokens, which shares none, lets go of it."""
+    from lingua_amd import float8
+    lin = make(256, 128, False)
+    with torch.no_grad():
+        lin(seeded_bf16((100, 256), seed=6).cuda())
+        assert len(float8._fwd_cast.entries) == 1
+        lin(seeded_bf16((1, 256), seed=7).cuda())
+        assert not float8._fwd_cast.entries
+
+
 @pytest.mark.parametrize("M", [1, 16, 17, 33, 64, 65])
 @pytest.mark.parametrize("K", [16, 272, 4096, 4112, 8192, 8208, 12288, 12304])
 def test_weight_quantised_inside_the_product(M, K):
