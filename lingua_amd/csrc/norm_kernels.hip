@@ -434,6 +434,9 @@ constexpr int64_t kNormMaxC = 4 * kNormWaves * 512;  // 8192: the weights of a t
 // row, the row requested ahead, the weights and the column maxima no longer fit 256 registers.  Inside a 1B-sized step,
 // [16384,2048], us: 59 (a workgroup per row, each row requested when its turn comes) -> 49 (next row requested ahead) ->
 // 34 (a wavefront per row: 168 MB at 4.9 TB/s); [4093,4096], workgroup per row with the next row ahead: 25.5 -> 20.5.
+// With no more rows than two per compute unit every row has a workgroup of its own, whose four waves share it: [1,2048]
+// 2.8 -> 2.5, [64,2048] 3.5 -> 3.0, [512,2048] 3.8 -> 3.5, but [768,2048] 4.1 / 4.3 and [2048,2048] 5.5 / 7.5; with
+// column maxima and their fold, of as many partial rows, 6.1 -> 4.7, 6.6 -> 5.2, 7.3 -> 7.1, 7.8 / 7.9, 9.9 / 11.3.
 // Backward: a workgroup per row, whose share of gw is a sum over rows 2 x (compute units) apart, on its own, back to
 // back, us: [16384,2048] 46.2 (no row ahead) -> 35.5 (three ahead: 201 MB at 5.7 TB/s; a wavefront per row the same),
 // [8192,1024] 20.3 -> 15.8, [64,2048] 4.3 -> 3.8, [4093,4096] 23.7 -> 21.8 (one ahead); the fold of gw 17 to 22 -> 4.
@@ -543,7 +546,8 @@ extern "C" int l8_rmsnorm_cast_rowwise(const void *x, const void *w, int w_is_f3
   return w_is_f32 ? launch_norm<WAVE, N, true>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)      \
                   : launch_norm<WAVE, N, false>(x, w, R, C, ldx, eps, y, ldy, q, ldq, scale, rstd, col_amax, workspace, st)
   const int64_t nch = (C + 511) / 512, nchw = (nch + kNormWaves - 1) / kNormWaves;
-  if (nch <= 4) L8_NORM(true, 4);
+  if (nch <= 4 && R > norm_blocks(R)) L8_NORM(true, 4);
+  if (nchw <= 1) L8_NORM(false, 1);
   if (nchw <= 2) L8_NORM(false, 2);
   L8_NORM(false, 4);
 #undef L8_NORM

@@ -107,9 +107,10 @@ def test_either_side_of_the_layout_line(shape):
 
 
 @pytest.mark.parametrize("C", [16, 520, 1024, 2040, 2048])
-@pytest.mark.parametrize("R", [3, 700, 2051])
+@pytest.mark.parametrize("R", [3, 512, 513, 700, 2051])
 def test_one_order_of_summation_in_every_layout(R, C):
-    """A row padded with zeros to four times its length takes the longest layout; with eps / 4 its mean is a quarter, so
+    """A workgroup per row for up to 512 rows (2 x compute units), then a wavefront per row up to 2048 columns.  A row padded
+    with zeros to four times its length takes the longest layout; with eps / 4 its mean is a quarter, so
     rstd, y, gx and gw are exactly twice those of the short row -- bit for bit, if both add up in one order."""
     from lingua_amd import ops
     x, gy = (seeded_bf16((R, C), std=s, seed=R + C + i).cuda() for i, s in enumerate((2.0, 0.05)))
