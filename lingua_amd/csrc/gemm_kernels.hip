@@ -1462,7 +1462,8 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // tiles on 256 compute units run 10-25 % faster than with 128x128 tiles, 128 tiles and fewer 15-45 % slower)
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  if (tiles(256, 256) * 16 >= cus * 9) return 12;
+  const bool big = tiles(256, 256) * 16 >= cus * 9;
+  if (big && M > kSkinnyMaxM) return 12;
   // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against the best tile: [20,2048].
   // [2048,2048] 4.2 / 7.5, [64,11008].[4096,11008] 18.9 / 28.8, [32,4096].[11008,4096] 14.6 / 13.5; from 48 tokens on
   // the 64 x 64 tiles win where there are enough of them ([48,4096].[11008,4096] 17.6 / 14.0, [40,4096].[8192,4096]
@@ -1472,7 +1473,12 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // 24.6 / 17.1, [16,5120].[9216,5120] 15.8 / 13.7, but [16,4096].[11008,4096] 10.9 / 12.5, [32,4096].[8192,4096] 10.6 / 11.8.
   const int64_t wide = tiles(32, 64);
   if (M > 8 && M <= 32 && (M > 16 || K > 4096) && wide * 16 >= cus * 9 && wide <= cus) return 22;
-  if (M <= 32 || (M <= kSkinnyMaxM && tiles(64, 64) * 16 < cus * 7)) return kSkinnyAlgo;
+  // A weight so wide that one row of big tiles would fill the chip gains nothing from them (they compute 256 rows): up to
+  // 16 tokens stay here, more go to the 128 x 128 tiles.  us, weight cold, skinny / 128 x 128 / 256 x 256: [1,4096].
+  // [36864,4096] 26 / 39 / 49, [16,4096].[36864,4096] 28 / 39 / 50, [32,4096].[36864,4096] 40 / 40 / 50, [64,4096].
+  // [36864,4096] 54 / 42 / 50, [1,4096].[128256,4096] 79 / 108 / 113, [16,4096].[128256,4096] 99 / 110 / 115,
+  // [32,4096].[128256,4096] 129 / 111 / 115, [64,4096].[128256,4096] 179 / 113 / 116.
+  if (M <= 16 || (M <= 32 && !big) || (M <= kSkinnyMaxM && tiles(64, 64) * 16 < cus * 7)) return kSkinnyAlgo;
   // Otherwise the smallest tile that gives no compute unit a second workgroup: these kernels are bound by their LDS
   // traffic and by what a K tile costs whatever its size, so more units at work are worth more than the larger tile's
   // economy.  us, 128 x 128 with two workgroups per unit (configuration 2) / chosen: [200,4096].[4096,4096] 19.1 / 8.9

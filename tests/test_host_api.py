@@ -82,6 +82,17 @@ def test_linear_call_validates_its_arguments_on_the_host():
     assert lib.l8_linear_fwd(pack(qx=fake)) == -1 and lib.l8_linear_fwd(None) == -1
 
 
+@pytest.mark.parametrize("M,N,K,name", [(1, 36608, 4096, "skinny"), (1, 36864, 4096, "skinny"), (16, 128256, 4096, "skinny"),
+                                        (17, 36608, 2048, "skinny"), (17, 36864, 2048, "2x2t_r5"), (32, 128256, 4096, "2x2t_r5"),
+                                        (64, 36864, 4096, "2x2t_r5"), (65, 36864, 4096, "stream"), (1, 1 << 20, 64, "skinny")])
+def test_few_tokens_take_no_big_tiles_however_wide_the_weight(M, N, K, name):
+    """Host arithmetic (256 compute units where there is no GPU): weights on either side of the width at which one row of
+    256 x 256 tiles fills the chip."""
+    if torch.cuda.is_available() and torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the sizes are for 256 compute units")
+    assert name in ops.gemm_pick(M, N, K)[1]
+
+
 @pytest.fixture
 def recorded_linear_calls(monkeypatch):
     """The inference call of a linear on CPU tensors, its library call recorded instead of made."""
