@@ -52,8 +52,9 @@ class _timed:
 
 
 # Raw handle of the calling thread's current stream on a device.  The public property builds a Python Stream object on
-# every call (2 us, as much as a launch); this is what PyTorch's own generated code calls.
-current_stream_ptr = torch._C._cuda_getCurrentRawStream
+# every call (2 us, as much as a launch); this is what PyTorch's own generated code calls.  A PyTorch built without GPU
+# support does not have it; there the package can be imported all the same.
+current_stream_ptr = getattr(torch._C, "_cuda_getCurrentRawStream", lambda index: torch.cuda.current_stream(index).cuda_stream)
 
 
 def _prep(t: torch.Tensor, what: str):

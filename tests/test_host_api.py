@@ -4,6 +4,8 @@ module mirror the reference interface (lingua/float8.py:134-191)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -118,6 +120,15 @@ def test_only_a_written_activation_cast_is_shared(recorded_linear_calls):
     for outputs in (0, 48, 64):
         float8.linear_infer(x, torch.zeros(outputs, 32, dtype=torch.bfloat16), None)
     assert [(c["outputs"], c["x_ready"]) for c in recorded_linear_calls] == [(0, False), (48, False), (64, True)]
+
+
+def test_package_imports_where_pytorch_has_no_gpu_support():
+    """Such a build lacks the private call that hands out raw streams; only a call on a GPU tensor may need it."""
+    code = ("import torch; del torch._C._cuda_getCurrentRawStream; import lingua_amd\n"
+            "try: lingua_amd.ops.cast_rowwise(torch.zeros(4, 16, dtype=torch.bfloat16))\n"
+            "except RuntimeError as e: print(e)")
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0 and "no CPU path" in done.stdout, done.stderr
 
 
 def test_no_cpu_path():
