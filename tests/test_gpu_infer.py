@@ -49,6 +49,29 @@ def test_inference_equals_the_training_forward(shape, bias, cached):
         float8.clear_cast_memos()
 
 
+@pytest.mark.parametrize("M,K,N", [(8, 1040, 11008), (32, 1040, 7104), (32, 1040, 11008), (16, 4112, 9216), (48, 1040, 11008),
+                                   (64, 1040, 16400), (17, 272, 36864), (64, 272, 36864)])
+def test_one_result_whoever_asks(M, K, N):
+    """Few tokens: with and without gradients, weight kept quantised or not, also where the product runs on another
+    kernel than the few-token one.  Values over all of e4m3's exponents, so that the order of a sum shows."""
+    from lingua_amd import float8
+    spread = lambda n, k, s: (seeded_bf16((n, k), seed=s).float() *
+                              torch.exp2(torch.randint(-7, 8, (n, k), generator=torch.Generator().manual_seed(s)).float())).to(torch.bfloat16)
+    lin = make(K, N, True)
+    with torch.no_grad():
+        lin.weight.copy_(spread(N, K, 1))
+    x = spread(M, K, 2).cuda()
+    want = lin(x.clone().requires_grad_(True)).detach()
+    old = float8.config.cache_weight_casts
+    try:
+        for float8.config.cache_weight_casts in (False, True):
+            with torch.no_grad():
+                assert torch.equal(lin(x).view(torch.int16), want.view(torch.int16))
+    finally:
+        float8.config.cache_weight_casts = old
+        float8.clear_cast_memos()
+
+
 def test_linears_share_an_activation_and_see_it_change():
     """Above 64 tokens w1 and w3 share one quantised copy; a write to the activation in between is seen, and another
     thread's default stream or a second model do not get it."""

@@ -77,6 +77,10 @@ def test_linear_call_validates_its_arguments_on_the_host():
     # up to 64 tokens the weight is quantised inside the product, up to 8 the tokens too: nothing to put anywhere
     assert 32 * 64 + 32 * 4 <= lib.l8_linear_fwd_workspace(pack(M=32)) < lib.l8_linear_fwd_workspace(pack(M=32, amax_w=fake))
     assert lib.l8_linear_fwd_workspace(pack(M=8)) == 0 < lib.l8_linear_fwd_workspace(pack(M=9))
+    # ... where the product of quantised operands is the same kernel, and with it the order of its sums
+    for M, N, K in ((32, 11008, 64), (16, 9216, 4112), (48, 11008, 64), (64, 16400, 64), (17, 36864, 64)):
+        assert not ops.gemm_pick(M, N, K)[1].startswith("skinny")
+        assert lib.l8_linear_fwd_workspace(pack(M=M, N=N, K=K, ldx=K, ldw=K, ldy=N)) >= M * K + M * 4 + N * K + N * 4
     assert lib.l8_linear_fwd(pack()) == -1 and "workspace" in _lib.last_error()
     assert lib.l8_linear_fwd(pack(M=-1)) == -1 and lib.l8_linear_fwd_workspace(pack(M=-1)) == -1
     assert lib.l8_linear_fwd(pack(x_ready=1)) == -1 and "x_ready" in _lib.last_error()
