@@ -64,6 +64,25 @@ static int check_fwd(const l8_linear_fwd_args *a) {
   return L8_OK;
 }
 
+// All that the casts and the product ask of their operands, so that a call is refused before any of them is enqueued.
+static int check_operands(const l8_linear_fwd_args &a) {
+  auto aligned = [](const void *p, uintptr_t n) { return (uintptr_t)p % n == 0; };
+  auto source = [&](const void *p, int64_t ld) { return p && a.K % 8 == 0 && ld % 8 == 0 && ld >= a.K && aligned(p, 16); };
+  if (!a.x_ready && a.M > 0 && a.K > 0)
+    L8_REQUIRE(source(a.x, a.ldx), "l8_linear_fwd: x must be 16-byte aligned, K=%lld and ldx=%lld multiples of 8, ldx >= K",
+               (long long)a.K, (long long)a.ldx);
+  if (!a.w_ready && a.N > 0 && a.K > 0)
+    L8_REQUIRE(source(a.w, a.ldw), "l8_linear_fwd: w must be 16-byte aligned, K=%lld and ldw=%lld multiples of 8, ldw >= K",
+               (long long)a.K, (long long)a.ldw);
+  if (a.M == 0 || a.N == 0) return L8_OK;
+  L8_REQUIRE(a.K > 0 && a.K % 16 == 0, "l8_linear_fwd: K=%lld must be positive and a multiple of 16", (long long)a.K);
+  L8_REQUIRE(a.M < (1LL << 31) && a.N < (1LL << 31) && a.K < (1LL << 31), "l8_linear_fwd: dimension too large");
+  L8_REQUIRE(aligned(a.qx, 16) && aligned(a.qw, 16), "l8_linear_fwd: qx and qw must be 16-byte aligned");
+  L8_REQUIRE(a.y && a.ldy >= a.N, "l8_linear_fwd: y is null, or ldy=%lld < N=%lld", (long long)a.ldy, (long long)a.N);
+  L8_REQUIRE(a.algo >= 0 && a.algo <= l8_gemm_algo_count(), "l8_linear_fwd: algo %lld out of range", (long long)a.algo);
+  return L8_OK;
+}
+
 extern "C" int64_t l8_linear_fwd_workspace(const l8_linear_fwd_args *a) {
   if (check_fwd(a) != L8_OK) return L8_EINVAL;
   Pieces ws{nullptr};
@@ -73,6 +92,7 @@ extern "C" int64_t l8_linear_fwd_workspace(const l8_linear_fwd_args *a) {
 
 extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
   int rc = check_fwd(a);
+  if (rc == L8_OK) rc = check_operands(*a);
   if (rc != L8_OK) return rc;
   Pieces ws{(uint8_t *)a->workspace};
   const LinearFwd t = plan(*a, ws);
@@ -87,14 +107,6 @@ extern "C" int l8_linear_fwd(const l8_linear_fwd_args *a) {
   } else if (cast_x) {
     rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, a->K, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
     if (rc != L8_OK) return rc;
-  }
-  if (t.x_on_the_way || t.w_on_the_way) {
-    L8_REQUIRE(a->w && a->y && a->K > 0 && a->K % 16 == 0 && a->ldw % 8 == 0 && a->ldw >= a->K && ((uintptr_t)a->w % 16) == 0 && a->ldy >= a->N,
-               "l8_linear_fwd: K=%lld must be a multiple of 16, ldw=%lld of 8 and >= K, w 16-byte aligned, ldy >= N", (long long)a->K, (long long)a->ldw);
-    if (t.x_on_the_way)
-      L8_REQUIRE(a->x && a->ldx % 8 == 0 && a->ldx >= a->K && ((uintptr_t)a->x % 16) == 0,
-                 "l8_linear_fwd: x must be 16-byte aligned, ldx=%lld a multiple of 8 and >= K", (long long)a->ldx);
-    if (!t.w_on_the_way) L8_REQUIRE(((uintptr_t)t.qw % 16) == 0, "l8_linear_fwd: qw must be 16-byte aligned");
   }
   if (cast_w && !together) {
     rc = l8_cast_rowwise(a->w, a->N, a->K, a->ldw, t.qw, a->K, t.sw, a->amax_w, nullptr, nullptr, 0, a->stream);

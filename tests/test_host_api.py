@@ -88,6 +88,22 @@ def test_linear_call_validates_its_arguments_on_the_host():
     assert lib.l8_linear_fwd(pack(qx=fake)) == -1 and lib.l8_linear_fwd(None) == -1
 
 
+@pytest.mark.parametrize("change,named", [
+    (dict(M=32, qx=(1 << 20) + 8, sx=1 << 20, x_ready=1), "qx"),          # few tokens: read in 16-byte pieces
+    (dict(qx=(1 << 20) + 8, sx=1 << 20), "qx"), (dict(qw=(1 << 20) + 8, sw=1 << 20, w_ready=1), "qw"),
+    (dict(x=(1 << 20) + 8), "x must"), (dict(w=(1 << 20) + 8), "w must"), (dict(w=0), "w must"), (dict(ldx=60), "ldx"), (dict(ldw=68), "ldw"),
+    (dict(K=72, ldx=72, ldw=72), "multiple of 16"), (dict(y=0), "y is null"), (dict(ldy=40), "ldy"), (dict(algo=99), "algo")])
+@pytest.mark.parametrize("M", [4, 32, 80])
+def test_linear_call_is_refused_before_anything_is_enqueued(M, change, named):
+    """An operand that the product cannot take is found before the casts: on a machine without a GPU the first launch
+    would answer with another error."""
+    lib = _lib.load()
+    fake = 1 << 20
+    base = dict(x=fake, M=M, K=64, ldx=64, w=fake, N=48, ldw=64, bias=0, y=fake, ldy=48, qx=0, sx=0, col=0, x_ready=0, qw=0,
+                sw=0, amax_w=0, w_ready=0, algo=0, ws=fake, ws_bytes=1 << 20, stream=0)
+    assert lib.l8_linear_fwd(ops._FWD.pack(*dict(base, **change).values())) == -1 and named in _lib.last_error()
+
+
 @pytest.mark.parametrize("M,N,K,name", [(1, 36608, 4096, "skinny"), (1, 36864, 4096, "skinny"), (16, 128256, 4096, "skinny"),
                                         (17, 36608, 2048, "skinny"), (17, 36864, 2048, "2x2t_r5"), (32, 128256, 4096, "2x2t_r5"),
                                         (64, 36864, 4096, "2x2t_r5"), (65, 36864, 4096, "stream"), (1, 1 << 20, 64, "skinny")])
