@@ -381,8 +381,9 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
     parts = []
     for qa, sa, out in zip(qas, sas, outs):
         parts += [qa.data_ptr(), qa.shape[0], sa.data_ptr(), out.data_ptr()]
-    code = _lib.load().l8_gemm_nt_multi(struct.pack(f"{len(parts)}q", *parts), len(qas), qb.data_ptr(), N, K, K, K, sb.data_ptr(),
-                                        SCALE_ROW, N, algo, st)
+    with _timed("gemm_nt_multi", 2 * sum(qa.shape[0] for qa in qas) * N * K, qb.device):
+        code = _lib.load().l8_gemm_nt_multi(struct.pack(f"{len(parts)}q", *parts), len(qas), qb.data_ptr(), N, K, K, K, sb.data_ptr(),
+                                            SCALE_ROW, N, algo, st)
     _lib.check(code, "l8_gemm_nt_multi")
     return outs
 

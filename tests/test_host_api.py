@@ -142,6 +142,43 @@ def test_only_a_written_activation_cast_is_shared(recorded_linear_calls):
     assert [(c["outputs"], c["x_ready"]) for c in recorded_linear_calls] == [(0, False), (48, False), (64, True)]
 
 
+class _RecordedLibrary:
+    """Stands in for the library: notes which entry is called, and between which devices' brackets."""
+
+    def __init__(self, monkeypatch):
+        self.calls, self.inside = [], None
+        outer = self
+
+        class timed:
+            def __init__(self, name, work, dev):
+                self.name, self.dev = name, dev
+
+            def __enter__(self):
+                outer.inside = (self.name, self.dev)
+
+            def __exit__(self, *exc):
+                outer.inside = None
+
+        monkeypatch.setattr(ops, "_timed", timed)
+        monkeypatch.setattr(ops, "_prep", lambda t, what: 0)
+        monkeypatch.setattr(_lib, "load", lambda: self)
+        monkeypatch.setattr(_lib, "check", lambda code, what: None)
+
+    def __getattr__(self, name):
+        if not name.startswith("l8_"):
+            raise AttributeError(name)
+        return lambda *args: self.calls.append((name, self.inside)) or 0
+
+
+def test_products_in_one_launch_run_on_their_operands_device(monkeypatch):
+    """The library launches on the current device and counts its compute units: like every launch, this one is made
+    with the tensors' device current."""
+    rec = _RecordedLibrary(monkeypatch)
+    qa, s = torch.zeros(16, 32, dtype=torch.float8_e4m3fn), torch.ones(16, 1)
+    ops.gemm_nt_multi((qa, qa), qa, (s, s), s)
+    assert rec.calls == [("l8_gemm_nt_multi", ("gemm_nt_multi", qa.device))]
+
+
 def test_package_imports_where_pytorch_has_no_gpu_support():
     """Such a build lacks the private call that hands out raw streams; only a call on a GPU tensor may need it."""
     code = ("import torch; del torch._C._cuda_getCurrentRawStream; import lingua_amd\n"
