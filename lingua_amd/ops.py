@@ -391,6 +391,15 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
 _FWD = struct.Struct("22q")   # l8_linear_fwd_args: eight bytes per member
 
 
+def _linear_fwd_call(members, x):
+    lib = _lib.load()
+    need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))
+    if need > 0:
+        ws = x.new_empty(need, dtype=torch.uint8)
+        members[19], members[20] = ws.data_ptr(), need
+    return lib.l8_linear_fwd(_FWD.pack(*members))
+
+
 def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y: torch.Tensor, x_cast=None, x_ready: bool = False,
                col_amax: Optional[torch.Tensor] = None, w_cast=None, w_ready: bool = False, amax_w: Optional[torch.Tensor] = None,
                algo: int = 0) -> None:
@@ -409,22 +418,16 @@ def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y
         bias = bias.contiguous()
     if M == 0 or N == 0:
         return
-    lib = _lib.load()
     members = [x.data_ptr(), M, K, _ld(x), w.data_ptr(), N, _ld(w), 0 if bias is None else bias.data_ptr(), y.data_ptr(), N,
                x_cast[0].data_ptr() if x_cast else 0, x_cast[1].data_ptr() if x_cast else 0,
                0 if col_amax is None else col_amax.data_ptr(), x_ready,
                w_cast[0].data_ptr() if w_cast else 0, w_cast[1].data_ptr() if w_cast else 0,
                0 if amax_w is None else amax_w.data_ptr(), w_ready, algo, 0, 0, st]
-    need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))
-    if need > 0:
-        ws = x.new_empty(need, dtype=torch.uint8)
-        members[19], members[20] = ws.data_ptr(), need
-    dev = x.device.index
-    if torch._C._cuda_getDevice() == dev:
-        code = lib.l8_linear_fwd(_FWD.pack(*members))
-    else:
-        with torch.cuda.device(dev):
-            code = lib.l8_linear_fwd(_FWD.pack(*members))
+    if torch._C._cuda_getDevice() == x.device.index:
+        code = _linear_fwd_call(members, x)
+    else:   # the size of the workspace is a question to that device too
+        with torch.cuda.device(x.device):
+            code = _linear_fwd_call(members, x)
     _lib.check(code, "l8_linear_fwd")
 
 

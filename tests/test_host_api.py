@@ -179,6 +179,27 @@ def test_products_in_one_launch_run_on_their_operands_device(monkeypatch):
     assert rec.calls == [("l8_gemm_nt_multi", ("gemm_nt_multi", qa.device))]
 
 
+def test_linear_call_asks_its_workspace_of_the_operands_device(monkeypatch):
+    """How much the call needs depends on the compute units of the device that it runs on."""
+    rec = _RecordedLibrary(monkeypatch)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)   # the operands' index is None: another one
+
+    class device:
+        def __init__(self, dev):
+            self.dev = dev
+
+        def __enter__(self):
+            rec.inside = ("device", self.dev)
+
+        def __exit__(self, *exc):
+            rec.inside = None
+
+    monkeypatch.setattr(torch.cuda, "device", device)
+    x, w, y = (torch.zeros(s, dtype=torch.bfloat16) for s in ((80, 32), (48, 32), (80, 48)))
+    ops.linear_fwd(x, w, None, y)
+    assert rec.calls == [(name, ("device", x.device)) for name in ("l8_linear_fwd_workspace", "l8_linear_fwd")]
+
+
 def test_package_imports_where_pytorch_has_no_gpu_support():
     """Such a build lacks the private call that hands out raw streams; only a call on a GPU tensor may need it."""
     code = ("import torch; del torch._C._cuda_getCurrentRawStream; import lingua_amd\n"
