@@ -17,11 +17,17 @@ SCALE_ROW = 1
 # Optional per-kernel timing: when `kernel_timer` is a list, every launch below
 # appends (kernel name, start event, end event, algorithmic work) where the
 # events are recorded on the stream the kernel runs on.  Work is flop for the
-# GEMM and compulsory bytes for the casts.  None (the default) records nothing.
+# products and compulsory bytes for the casts.  None (the default) records nothing.
 # `kernel_timer_names` (a set of kernel names, or None for all) limits the recording: every pair of events costs
 # the stream a little, which a caller timing a whole step may not want to pay for every launch.
 kernel_timer = None
 kernel_timer_names = None
+
+
+def timed_singly(*names) -> bool:
+    """Does the timer ask for kernels (by name, or for all) that calls which run several in one launch or from one library
+    call would hide?  Those calls then run them one by one.  A timer that names other kernels changes nothing."""
+    return kernel_timer is not None and (kernel_timer_names is None or not kernel_timer_names.isdisjoint(names))
 
 
 class _timed:
@@ -147,7 +153,7 @@ def cast_rowwise_many(xs, out=None):
     else:
         qs = [torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=dev) for x in xs]
         ss = [torch.empty((n, 1), dtype=torch.float32, device=dev) for n in rows]
-    if kernel_timer is not None:  # per-kernel figures are of the casts one by one
+    if timed_singly("cast_rowwise"):
         return [cast_rowwise(x, out_q=q, out_scale=s) for x, q, s in zip(xs, qs, ss)]
     amaxes = [torch.empty((n, 1), dtype=torch.bfloat16, device=dev) for n in rows]
     items = []
@@ -370,7 +376,7 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
     """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch where that fills the GPU better.  Dense fp8
     operands with one scale per row."""
     N, K = qb.shape
-    one = algo == 0 and len(qas) > 1 and kernel_timer is None and qb.is_contiguous() and sb.dtype == torch.float32 and sb.numel() == N and sb.is_contiguous()
+    one = algo == 0 and len(qas) > 1 and not timed_singly("gemm_nt") and qb.is_contiguous() and sb.dtype == torch.float32 and sb.numel() == N and sb.is_contiguous()
     for qa, sa in zip(qas, sas):
         one = (one and qa.dtype == qb.dtype == torch.float8_e4m3fn and qa.dim() == 2 and qa.shape[1] == K and qa.is_contiguous() and
                qa.device == qb.device and sa.dtype == torch.float32 and sa.numel() == qa.shape[0] and sa.is_contiguous())
@@ -423,10 +429,10 @@ def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y
                0 if col_amax is None else col_amax.data_ptr(), x_ready,
                w_cast[0].data_ptr() if w_cast else 0, w_cast[1].data_ptr() if w_cast else 0,
                0 if amax_w is None else amax_w.data_ptr(), w_ready, algo, 0, 0, st]
-    if torch._C._cuda_getDevice() == x.device.index:
+    if kernel_timer is None and torch._C._cuda_getDevice() == x.device.index:
         code = _linear_fwd_call(members, x)
     else:   # the size of the workspace is a question to that device too
-        with torch.cuda.device(x.device):
+        with _timed("linear_fwd", 2 * M * N * K, x.device):
             code = _linear_fwd_call(members, x)
     _lib.check(code, "l8_linear_fwd")
 

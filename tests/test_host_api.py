@@ -184,20 +184,28 @@ def test_linear_call_asks_its_workspace_of_the_operands_device(monkeypatch):
     rec = _RecordedLibrary(monkeypatch)
     monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)   # the operands' index is None: another one
 
-    class device:
-        def __init__(self, dev):
-            self.dev = dev
-
-        def __enter__(self):
-            rec.inside = ("device", self.dev)
-
-        def __exit__(self, *exc):
-            rec.inside = None
-
-    monkeypatch.setattr(torch.cuda, "device", device)
     x, w, y = (torch.zeros(s, dtype=torch.bfloat16) for s in ((80, 32), (48, 32), (80, 48)))
     ops.linear_fwd(x, w, None, y)
-    assert rec.calls == [(name, ("device", x.device)) for name in ("l8_linear_fwd_workspace", "l8_linear_fwd")]
+    assert rec.calls == [(name, ("linear_fwd", x.device)) for name in ("l8_linear_fwd_workspace", "l8_linear_fwd")]
+
+
+@pytest.mark.parametrize("names,singly", [({"swiglu_cast_rowwise"}, False), ({"gemm_nt_multi", "cast_rowwise_many", "linear_fwd"}, False),
+                                          ({"gemm_nt", "cast_rowwise"}, True), (None, True)])
+def test_a_kernel_timer_changes_only_what_it_asks_for(monkeypatch, recorded_linear_calls, names, singly):
+    """Calls that run several kernels in one launch take them one by one under a timer for those kernels, and as ever
+    under a timer for others."""
+    from lingua_amd import float8
+    rec = _RecordedLibrary(monkeypatch)
+    monkeypatch.setattr(ops, "kernel_timer", [])
+    monkeypatch.setattr(ops, "kernel_timer_names", names)
+    x, w = torch.zeros(80, 32, dtype=torch.bfloat16), torch.zeros(48, 32, dtype=torch.bfloat16)
+    qa, s = torch.zeros(16, 32, dtype=torch.float8_e4m3fn), torch.ones(16, 1)
+    ops.gemm_nt_multi((qa, qa), qa, (s, s), s)
+    ops.cast_rowwise_many((x, w))
+    assert [name for name, _ in rec.calls] == (["l8_gemm_nt_ws"] * 2 + ["l8_cast_rowwise"] * 2 if singly else
+                                               ["l8_gemm_nt_multi", "l8_cast_rowwise_many"])
+    float8.linear_infer(x, w, None)
+    assert len(recorded_linear_calls) == (0 if singly else 1)
 
 
 def test_package_imports_where_pytorch_has_no_gpu_support():
