@@ -160,3 +160,30 @@ def test_tokens_quantised_inside_the_product(M, K, kept):
     ops.linear_fwd(x, w, bias, got, w_cast=(qw, sw) if kept else None, w_ready=kept)
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and (M <= 4 or bool(torch.isnan(want[[2, M - 1]]).all()))
     assert torch.equal(torch.nan_to_num(got.float()), torch.nan_to_num(want.float()))
+
+
+@pytest.mark.parametrize("M,K,N", [(5, 272, 48), (40, 1040, 72), (64, 4112, 7168), (80, 272, 48), (1100, 2064, 80)])
+@pytest.mark.parametrize("give_qx", [False, True])
+@pytest.mark.parametrize("give_col", [False, True])
+@pytest.mark.parametrize("give_qw,give_amax", [(False, False), (False, True), (True, False), (True, True)])
+def test_what_the_linear_call_hands_out(M, K, N, give_qx, give_col, give_qw, give_amax):
+    """The quantised operands, the activation's column amaxes and the weight's row amaxes where they are asked for, few
+    tokens and many: the bits of the single entries, and the same y with or without them."""
+    from lingua_amd import ops
+    x, w = seeded_bf16((M, K), seed=M + K).cuda(), seeded_bf16((N, K), 0.02, seed=K).cuda()
+    bias = seeded_bf16((N,), seed=2).cuda()
+    want_col = torch.empty(K, device="cuda")
+    wqx, wsx, _ = ops.cast_rowwise(x, col_amax=want_col)
+    wqw, wsw, want_amax = ops.cast_rowwise(w)
+    want = ops.gemm_nt(wqx, wqw, wsx, wsw, bias)
+    fresh = lambda like: torch.full_like(like.view(torch.uint8), 0x55).view(like.dtype)
+    qx, sx, qw, sw, col, amax = (fresh(t) for t in (wqx, wsx, wqw, wsw, want_col, want_amax))
+    y = fresh(want)
+    ops.linear_fwd(x, w, bias, y, x_cast=(qx, sx) if give_qx else None, col_amax=col if give_col else None,
+                   w_cast=(qw, sw) if give_qw else None, amax_w=amax if give_amax else None)
+    same = lambda a, b: torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert same(y, want)
+    assert not give_qx or same(qx, wqx) and same(sx, wsx)
+    assert not give_col or same(col, want_col)
+    assert not give_qw or same(qw, wqw) and same(sw, wsw)
+    assert not give_amax or same(amax, want_amax)
