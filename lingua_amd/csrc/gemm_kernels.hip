@@ -1456,6 +1456,7 @@ extern "C" const char *l8_gemm_algo_name(int algo) {
 static int pick_plain_big(int64_t K) { return K >= 4096 ? 5 : 3; }
 
 static int pick_algo(int64_t M, int64_t N, int64_t K) {
+  if (M <= 8) return kSkinnyAlgo;  // whatever the chip: the smallest calls do not pay for asking
   // large problems: the persistent kernel (measured 2-11 % ahead of the plain ones on every shape with at
   // least one 256x256 tile per compute unit; groups of 4 tile rows ahead of groups of 8 by 1-3 %), also when
   // the big tiles leave up to 7/16 of the compute units idle (measured with K = 2048 .. 16384: 144 to 240
@@ -1472,7 +1473,7 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   // kernels the slower ones (every workgroup reads all of x): [32,4096].[11008,4096] 14.4 / 13.0, [32,5120].[14336,5120]
   // 24.6 / 17.1, [16,5120].[9216,5120] 15.8 / 13.7, but [16,4096].[11008,4096] 10.9 / 12.5, [32,4096].[8192,4096] 10.6 / 11.8.
   const int64_t wide = tiles(32, 64);
-  if (M > 8 && M <= 32 && (M > 16 || K > 4096) && wide * 16 >= cus * 9 && wide <= cus) return 22;
+  if (M <= 32 && (M > 16 || K > 4096) && wide * 16 >= cus * 9 && wide <= cus) return 22;
   // A weight so wide that one row of big tiles would fill the chip gains nothing from them (they compute 256 rows): up to
   // 16 tokens stay here, more go to the 128 x 128 tiles.  us, weight cold, skinny / 128 x 128 / 256 x 256: [1,4096].
   // [36864,4096] 26 / 39 / 49, [16,4096].[36864,4096] 28 / 39 / 50, [32,4096].[36864,4096] 40 / 40 / 50, [64,4096].

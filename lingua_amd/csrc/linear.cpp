@@ -32,11 +32,11 @@ static LinearFwd plan(const l8_linear_fwd_args &a, Pieces &ws) {
   // kernel adds up K in an order of its own, and a linear's result shall not hang on who wants its gradient or keeps its
   // weight quantised.  Where that product runs on tiles, one kernel would save at most a third: [17,4096].[11008,4096]
   // 35 / 27, [32,4096].[16384,4096] 50 / 36, but [32,5120].[14336,5120] 54 / 54, [64,4096].[11008,4096] 36 / 36.
-  const bool skinny = a.algo == 0 && a.M > 0 && a.N > 0 && a.K > 0 && l8_gemm_pick(a.M, a.N, a.K) == kSkinnyAlgo;
-  t.w_on_the_way = !a.qw && !a.amax_w && skinny && skinny_serves(a.M, a.N, a.K, a.K, a.ldw, 2);
+  auto skinny = [&] { return a.algo == 0 && a.M > 0 && a.N > 0 && a.K > 0 && l8_gemm_pick(a.M, a.N, a.K) == kSkinnyAlgo; };
+  t.w_on_the_way = !a.qw && !a.amax_w && skinny_serves(a.M, a.N, a.K, a.K, a.ldw, 2) && skinny();
   const int w_bytes = t.w_on_the_way ? 2 : 1;
-  t.x_on_the_way = !a.qx && !a.col_amax_x && skinny && skinny_quantises_x(a.M, a.N, a.K, a.ldx, w_bytes) &&
-                   (t.w_on_the_way || skinny_serves(a.M, a.N, a.K, a.ldx, a.K, 1));
+  t.x_on_the_way = !a.qx && !a.col_amax_x && skinny_quantises_x(a.M, a.N, a.K, a.ldx, w_bytes) &&
+                   (t.w_on_the_way || (skinny_serves(a.M, a.N, a.K, a.ldx, a.K, 1) && skinny()));
   if (!t.x_on_the_way) {
     t.qx = a.qx ? a.qx : ws.take(a.M * a.K);
     t.sx = a.qx ? a.sx : (float *)ws.take(a.M * 4);

@@ -357,7 +357,7 @@ _UNSHARED_TOKENS = 64
 def linear_infer(a, b_t, bias):
     """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
     both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same kernels and results as ``linear_forward``."""
-    if ops.timed_singly("cast_rowwise", "gemm_nt") or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
+    if (ops.kernel_timer is not None and ops.timed_singly("cast_rowwise", "gemm_nt")) or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
         return linear_forward(a.flatten(end_dim=-2), b_t, bias, False, config.gemm_algo)[0].unflatten(0, a.shape[:-1])
     shape = a.shape
     if a.dim() != 2:
@@ -372,7 +372,7 @@ def linear_infer(a, b_t, bias):
         if hit is None:
             if tokens > _UNSHARED_TOKENS:
                 x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
-            else:   # nothing of its own to file, but an earlier activation (a prompt's, during generation) is not kept alive
+            elif _fwd_cast.entries:   # nothing of its own to file, but an earlier activation (a prompt's) is not kept alive
                 _fwd_cast.clear(a)
     w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
     ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, w_cast, w_cast is not None, None, config.gemm_algo)

@@ -397,15 +397,6 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
 _FWD = struct.Struct("22q")   # l8_linear_fwd_args: eight bytes per member
 
 
-def _linear_fwd_call(members, x):
-    lib = _lib.load()
-    need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))
-    if need > 0:
-        ws = x.new_empty(need, dtype=torch.uint8)
-        members[19], members[20] = ws.data_ptr(), need
-    return lib.l8_linear_fwd(_FWD.pack(*members))
-
-
 def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y: torch.Tensor, x_cast=None, x_ready: bool = False,
                col_amax: Optional[torch.Tensor] = None, w_cast=None, w_ready: bool = False, amax_w: Optional[torch.Tensor] = None,
                algo: int = 0) -> None:
@@ -429,11 +420,19 @@ def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y
                0 if col_amax is None else col_amax.data_ptr(), x_ready,
                w_cast[0].data_ptr() if w_cast else 0, w_cast[1].data_ptr() if w_cast else 0,
                0 if amax_w is None else amax_w.data_ptr(), w_ready, algo, 0, 0, st]
-    if kernel_timer is None and torch._C._cuda_getDevice() == x.device.index:
-        code = _linear_fwd_call(members, x)
-    else:   # the size of the workspace is a question to that device too
-        with _timed("linear_fwd", 2 * M * N * K, x.device):
-            code = _linear_fwd_call(members, x)
+    lib, bracket = _lib.load(), None
+    if kernel_timer is not None or torch._C._cuda_getDevice() != x.device.index:   # else there is nothing to bracket
+        bracket = _timed("linear_fwd", 2 * M * N * K, x.device)
+        bracket.__enter__()
+    try:
+        need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))   # depends on the device's compute units
+        if need > 0:
+            ws = x.new_empty(need, dtype=torch.uint8)
+            members[19], members[20] = ws.data_ptr(), need
+        code = lib.l8_linear_fwd(_FWD.pack(*members))
+    finally:
+        if bracket is not None:
+            bracket.__exit__()
     _lib.check(code, "l8_linear_fwd")
 
 
