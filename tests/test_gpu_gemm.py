@@ -101,7 +101,8 @@ def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
                                                ((1536, 1500), 2048, 4112, False),
                                                ((2048, 2048, 2048), 2052, 128, None), ((2048, 0, 2048), 2048, 128, None)])
 def test_products_with_one_operand_in_one_launch(rows, N, K, together):
-    """Every product has the bits it has alone, in one launch or in several: last tile rows that are short, of different
+    """Every product has the bits it has alone -- in one launch those of the big tiles, which add up K in order, in several
+    those of the kernel that its own size picks: last tile rows that are short, of different
     lengths, one row alone in a tile; short column tiles; K tiles that are short, fewer than the ring; a workgroup's second
     tile in another product than its first; outputs (N % 8) and lists (an empty product) that cannot go together."""
     import struct

@@ -1,5 +1,5 @@
 """Inference passes: no autograd node, no column amaxes, one call of the library per linear -- and the very bytes of the
-training forward, whose kernels are the same."""
+training forward, whose product runs on the same kernel."""
 import pytest
 import torch
 
@@ -73,8 +73,8 @@ def test_one_result_whoever_asks(M, K, N):
 
 
 def test_linears_share_an_activation_and_see_it_change():
-    """Above 64 tokens w1 and w3 share one quantised copy; a write to the activation in between is seen, and another
-    thread's default stream or a second model do not get it."""
+    """Above 64 tokens w1 and w3 share one quantised copy, which a lookup from another stream does not get; a write to the
+    activation in between is seen."""
     from lingua_amd import float8
     w1, w3 = make(256, 128, False), make(256, 272, False)
     for tokens in (40, 100):
@@ -84,6 +84,12 @@ def test_linears_share_an_activation_and_see_it_change():
             assert rel_l2(w1(x), want[0]) <= 1e-3
             assert (len(float8._fwd_cast.entries) > 0) == (tokens > 64)
             assert rel_l2(w3(x), want[1]) <= 1e-3
+            if tokens > 64:
+                (entry,) = float8._fwd_cast.entries.values()
+                assert entry[3] == {w1.weight.data_ptr(), w3.weight.data_ptr()}   # who has used it
+                with torch.cuda.stream(torch.cuda.Stream()):
+                    assert float8._fwd_cast.get(x, "somebody else") is None
+                assert float8._fwd_cast.get(x, "somebody else") is not None
             w1(x)
             x.mul_(3.0)
             assert rel_l2(w3(x), oracle.linear_forward(x.cpu(), w3.weight.detach().cpu())) <= 1e-3

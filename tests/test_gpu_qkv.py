@@ -1,5 +1,6 @@
 """GPU tests of the single product for the attention projections (lingua/transformer.py:357-359 under
-lingua_amd.qkv.fuse_qkv): same bits as three separate Fp8Linear products, one GEMM launch in forward, and the
+lingua_amd.qkv.fuse_qkv): same bits as three separate Fp8Linear products (where their sizes pick kernels that
+add up K in one order), one GEMM launch in forward, and the
 right thing when the three linears are not called the way the reference's attention calls them."""
 import copy
 
