@@ -279,8 +279,8 @@ int l8_gemm_nt_add(const void *A, const void *B, int64_t M, int64_t N, int64_t K
                    const float *sa, int sa_mode, const float *sb, int sb_mode, void *C, int64_t ldc, int algo, void *stream);
 
 /* C_i [M_i,N] = bf16(A_i [M_i,K] . B^T * sa_i * sb) for n products with one B: the weight gradients of linears on one
- * activation (lingua/float8.py:123 once per linear).  One launch for two or three of them where that takes fewer rounds of
- * tiles over the chip, else as n calls of l8_gemm_nt.  sa_i fp32 [M_i]; lda and ldc are those of every A_i and C_i. */
+ * activation (lingua/float8.py:123 once per linear).  One launch of the 256 x 256 kernel for two or three of them where that
+ * takes fewer rounds of tiles over the chip, else as n calls of l8_gemm_nt.  sa_i fp32 [M_i]; lda and ldc are those of every A_i and C_i. */
 typedef struct {
   const void *A;
   int64_t M;
@@ -293,8 +293,10 @@ int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_
 int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t K);
 
 /* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
- * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; with a few
- * tokens, and neither qw nor amax_w asked for, the weight is quantised inside the product.  Every member is eight bytes
+ * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; where
+ * l8_gemm_pick names the few-token kernel, and neither qw nor amax_w is asked for, the weight (rows of up to 12288 columns)
+ * is quantised inside the product, up to 8 tokens of up to 4096 columns likewise.  All operands are checked before anything
+ * is enqueued: x and w as in l8_cast_rowwise, K a multiple of 16, qx and qw 16-byte aligned.  Every member is eight bytes
  * wide and in this order (a caller without C fills an array).
  *   x [M,K] bf16 (ldx), w [N,K] bf16 (ldw); bias bf16 [N] or NULL; y bf16 [M,N] (ldy)
  *   qx e4m3fn [M,K] dense + sx fp32 [M]: where the quantised x is wanted, NULL = in the workspace; with x_ready they
@@ -303,8 +305,8 @@ int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t 
  *   col_amax_x fp32 [K] or NULL: column amaxes of x (not with x_ready);  amax_w bf16 [N] or NULL: row amaxes of w (not with
  *      w_ready)
  *   algo  as in l8_gemm_nt (0 = library default)
- *   workspace  device scratch, 256-byte aligned, at least l8_linear_fwd_workspace(args) bytes (which depends on the shape and
- *      on which members are NULL, not on the other pointers' values) */
+ *   workspace  device scratch, 256-byte aligned, at least l8_linear_fwd_workspace(args) bytes (which depends on the shapes,
+ *      the strides, the current device and on which members are NULL, not on the other pointers' values) */
 typedef struct {
   const void *x;
   int64_t M, K, ldx;

@@ -356,7 +356,7 @@ _UNSHARED_TOKENS = 64
 
 def linear_infer(a, b_t, bias):
     """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
-    both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same kernels and results as ``linear_forward``."""
+    both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same results as ``linear_forward``."""
     if (ops.kernel_timer is not None and ops.timed_singly("cast_rowwise", "gemm_nt")) or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
         return linear_forward(a.flatten(end_dim=-2), b_t, bias, False, config.gemm_algo)[0].unflatten(0, a.shape[:-1])
     shape = a.shape

@@ -373,8 +373,9 @@ def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tens
 
 
 def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
-    """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch where that fills the GPU better.  Dense fp8
-    operands with one scale per row."""
+    """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch, on 256 x 256 tiles, where that fills the GPU
+    better (a product that alone is too small for those tiles may add up K in another order there).  Dense fp8 operands
+    with one scale per row."""
     N, K = qb.shape
     one = algo == 0 and len(qas) > 1 and not timed_singly("gemm_nt") and qb.is_contiguous() and sb.dtype == torch.float32 and sb.numel() == N and sb.is_contiguous()
     for qa, sa in zip(qas, sas):
@@ -400,7 +401,7 @@ _FWD = struct.Struct("22q")   # l8_linear_fwd_args: eight bytes per member
 def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y: torch.Tensor, x_cast=None, x_ready: bool = False,
                col_amax: Optional[torch.Tensor] = None, w_cast=None, w_ready: bool = False, amax_w: Optional[torch.Tensor] = None,
                algo: int = 0) -> None:
-    """y [M,N] (dense) = x @ w.T + bias with row-wise casts of both, in one call of the library: the same kernels as
+    """y [M,N] (dense) = x @ w.T + bias with row-wise casts of both, in one call of the library: the same results as
     ``cast_rowwise``, ``cast_rowwise``, ``gemm_nt``.  ``x_cast`` / ``w_cast`` = (q, scale), dense: where the quantised
     operand goes (None: a temporary), or with ``x_ready`` / ``w_ready`` where it comes from."""
     st = _prep(x, "linear_fwd")

@@ -7,8 +7,11 @@ share one quantised copy of ``x``; ``fuse_qkv`` additionally makes their three
 forward products one: the three weights are quantised row-wise straight into
 one ``[Nq+Nk+Nv, K]`` operand (no concatenation pass: the cast kernels write
 into row slices of it) and a single GEMM produces ``[T, Nq+Nk+Nv]``, of which
-the three linears return column slices.  Same recipe, same scales (every weight
-row keeps its own), so the same bits as three separate products.
+the three linears return column slices.  Same recipe, same bytes, same scales
+(every weight row keeps its own); the same bits as three separate products
+wherever the sizes pick kernels that add up K in one order.  Up to a few hundred
+tokens the narrow products can run on kernels that deal K out to groups of waves
+where the wide one does not: a last bit may differ then.
 
 Backward stays per linear (lingua/float8.py:99-131) but for its launches: the
 three dgrads have different row scales and are added up by their epilogues, the
