@@ -27,7 +27,7 @@ kernel_timer_names = None
 def timed_singly(*names) -> bool:
     """Does the timer ask for kernels (by name, or for all) that calls which run several in one launch or from one library
     call would hide?  Those calls then run them one by one.  A timer that names other kernels changes nothing."""
-    return kernel_timer is not None and (kernel_timer_names is None or not kernel_timer_names.isdisjoint(names))
+    return kernel_timer is not None and (kernel_timer_names is None or any(n in kernel_timer_names for n in names))
 
 
 class _timed:

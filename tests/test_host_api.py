@@ -190,7 +190,7 @@ def test_linear_call_asks_its_workspace_of_the_operands_device(monkeypatch):
 
 
 @pytest.mark.parametrize("names,singly", [({"swiglu_cast_rowwise"}, False), ({"gemm_nt_multi", "cast_rowwise_many", "linear_fwd"}, False),
-                                          ({"gemm_nt", "cast_rowwise"}, True), (None, True)])
+                                          ({"gemm_nt", "cast_rowwise"}, True), (["gemm_nt", "cast_rowwise"], True), (None, True)])
 def test_a_kernel_timer_changes_only_what_it_asks_for(monkeypatch, recorded_linear_calls, names, singly):
     """Calls that run several kernels in one launch take them one by one under a timer for those kernels, and as ever
     under a timer for others."""
