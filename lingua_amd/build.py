@@ -12,7 +12,7 @@ from concurrent.futures import ThreadPoolExecutor
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
 # LINGUA_FP8_LIB: where to put the library instead (a tuning variant beside the shipped one; `lingua_amd._lib` reads the
-# same variable); LINGUA_FP8_HIPCC_EXTRA: more hipcc flags for such a variant, e.g. "-DL8_STRADDLE=3 -DL8_READ_GROUPS=10".
+# same variable); LINGUA_FP8_HIPCC_EXTRA: more hipcc flags for such a variant, e.g. "-DL8_STRADDLE=3 -DL8_READ_GROUPS1=20".
 LIB_PATH = os.environ.get("LINGUA_FP8_LIB") or os.path.join(_HERE, "liblingua_fp8.so")
 SOURCES = ["api.cpp", "linear.cpp", "cast_kernels.hip", "gemm_kernels.hip", "swiglu_kernels.hip", "norm_kernels.hip", "skinny_kernels.hip"]
 

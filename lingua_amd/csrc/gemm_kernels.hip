@@ -119,9 +119,12 @@ L8_DEV void store16_aux(v4i data, __amdgpu_buffer_rsrc_t rs, uint32_t voff, int 
 #ifndef L8_STRADDLE
 #define L8_STRADDLE 2
 #endif
-// groups (of one MFMA each) of a half trip over which the persistent kernel issues the half's LDS reads
-#ifndef L8_READ_GROUPS
-#define L8_READ_GROUPS 13
+// groups (of one MFMA each) of the two halves of a trip over which the persistent kernel issues the half's LDS reads
+#ifndef L8_READ_GROUPS1
+#define L8_READ_GROUPS1 24
+#endif
+#ifndef L8_READ_GROUPS2
+#define L8_READ_GROUPS2 30
 #endif
 // L8_GEMM_PROF (compile-time, never set in the shipped build): the persistent kernel takes the `bias` pointer for
 // a buffer of 16 x uint64 per workgroup and records wall-clock ticks (100 MHz) at its start, after the prologue
@@ -598,18 +601,33 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 //
 // The C tile leaves straight from the accumulators, with no staging in LDS
 // (the ring stays in use by the panel stream) and no barrier:
-//   * the matrix cores compute D[i = m][j = n'] (A rows on the first port);
-//   * LDS row tn*32 + j of a wave's 128-row span of the B panel holds the
-//     global B row 4*g(j) + tn of that span, g(j) = 2*(j & 15) + (j >> 4) (the
-//     permutation is applied on the global-address side of the direct-to-LDS
-//     loads, which is free), so that lane j owns, at the same accumulator
-//     index of its four tn tiles, the four CONSECUTIVE output columns
-//     4*g(j) .. 4*g(j)+3, and lanes j / j+16 own neighbouring groups;
-//   * two v_permlane16_swap per pair of rows hand the lanes 0..15 of every 32
-//     the first row (their own four columns and their partners' four) and the
-//     lanes 16..31 the second: one 16-byte store per lane then covers 256
-//     contiguous bytes of a C row per 16 lanes (four rows per wave instruction,
-//     whole 128-byte lines).
+//   * the matrix cores compute D[i = m][j = n'] (A rows on the first port) in
+//     tiles of 16x16;
+//   * LDS row tn*16 + j of a wave's 128-row span of the B panel holds the
+//     global B row 8*j + tn of that span (the permutation is applied on the
+//     global-address side of the direct-to-LDS loads, which is free), so that
+//     lane j owns, at the same accumulator index of its eight tn tiles, the
+//     eight CONSECUTIVE output columns 8*j .. 8*j+7: 16 bytes of a C row, and
+//     one 16-byte store per lane covers 256 contiguous bytes of a row per 16
+//     lanes (four rows per wave instruction, whole 128-byte lines).
+//
+// The instruction is v_mfma_f32_16x16x128_f8f6f4, not 32x32x64: the same flop
+// per cycle for less power, and power is what sets this kernel's clock.  Matrix
+// instructions back to back on random operands, no memory traffic: 4.27 PFLOP/s
+// at 2.16 GHz against 3.98 at 1.97 (both 4.96 at 2.40 on zeros).  A K tile of
+// 128 bytes is then ONE step of 64 instructions, row by row of the wave's 8 x 8
+// tiles: the eight B fragments stay for the whole step, an A fragment for the
+// eight instructions of its row.
+// us, one launch behind the other on one box, 32x32x64 / this: [16384,11008] K =
+// 4096 502 / 490, [16384,4096] K = 11008 476 / 463, [11008,4096] K = 16384 500 /
+// 480, [16384,2048] K = 8192 187 / 180, [32768,8192] K = 2048 398 / 386.  A K tile
+// takes 2260 to 2310 cycles of the 2048 that its instructions need (2120 to 2190
+// before: a 32-cycle instruction hides less of what stands between two of them),
+// a C tile 5800 to 6300 (6700 before: no exchange of column groups between
+// lanes), at 1.6 to 1.85 GHz.  Cycles are not what bounds it: variants of the
+// loop's layout from 2260 to 2380 cycles took the same time, one of 3500 cycles
+// 20 % more.  Without the panel loads it runs at 2.2 GHz: they are the largest
+// consumer beside the matrix cores.
 // Work split: the tiles are dealt to the 8 XCDs in contiguous ranges of the
 // grouped order (as in the kernel above); inside an XCD, workgroup `loc`
 // takes tiles loc, loc + W, loc + 2W, ... of the range (W workgroups per XCD),
@@ -623,21 +641,17 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // MULTI: up to three products with one B (the weight gradients of linears on one activation) as one list of tiles.  On its
 // own [2048,16384].[2048,16384]^T has 64 tiles of 256 x 256, too few for this kernel, and [11008,4096] leaves a third of the
 // units without work in its last round; together they fill the rounds.
-template <int GROUP_M, bool HAS_BIAS, bool SK = false, int NW = 4, bool ADD = false, bool MULTI = false>
-__global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs p) {
+template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false>
+__global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  // NW = 4: one wave per SIMD, 128x128 per wave (the least LDS traffic per flop); NW = 8: two waves per SIMD,
-  // 64x128 per wave (while one of them waits -- for the port of the vector memory unit, for LDS, at the barrier --
-  // the other one's MFMAs keep the matrix core busy; half the stores per wave in the epilogue; 1.5 x the LDS reads)
-  static_assert(NW == 4 || NW == 8, "four or eight waves");
-  static_assert(!SK || NW == 4, "the shared-K exchange is written for four waves");
-  constexpr int BM = 256, BN = 256, BK = 128, TM = 16 / NW, TN = 4, R = 5;
-  constexpr int WROWS = TM * 32;  // rows of the tile per wave
+  // one wave per SIMD, 128x128 per wave: the least LDS traffic per flop
+  constexpr int BM = 256, BN = 256, BK = 128, NW = 4, TM = 8, TN = 8, R = 5;
+  constexpr int WROWS = TM * 16;  // rows of the tile per wave
   constexpr int UNIT = BM * BK;    // one ring slot: the A or the B panel of one K tile
   constexpr int NL = BM / 8 / NW;  // 1 KiB wave loads (8 rows x 128 B) per panel per wave
   constexpr int PEND = NL;         // in flight at the barrier of a trip: the unit requested in its first half
   constexpr int PEND0 = 2 * NL;    // prologue: K tile 1 may be in flight when K tile 0 is published
-  constexpr int N_STORES = TM * 4 * 2;  // store instructions per wave and C tile
+  constexpr int N_STORES = TM * 4;  // store instructions per wave and C tile
   static_assert(N_STORES + PEND <= 63, "vmcnt is a 6-bit counter");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
@@ -673,7 +687,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
   const int n_tail = !sk ? 0 : (helper ? (loc < r_tail ? (r_tail - loc + n_help - 1) / n_help : 0) : 1);  // pieces of this workgroup
   const int n_seg = sk ? n_rounds : (loc < cnt ? (cnt - loc + W - 1) / W : 0);                              // whole tiles
   if (n_seg + n_tail == 0) return;
-  [[maybe_unused]] uint64_t prof[24] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  [[maybe_unused]] uint64_t prof[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (L8_GEMM_PROF) {
     prof[0] = __builtin_amdgcn_s_memrealtime();
     prof[5] = __builtin_readcyclecounter();
@@ -732,15 +746,15 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
   // ---- global -> LDS load plan ----
   // lane l of a wave load fills LDS row l/8, position l%8 of an 8-row group; position p of LDS row r holds
   // chunk p ^ f(r), f(r) = (r & 7) ^ ((r >> 3) & 1).  Wave load i of a panel fills the LDS rows of group
-  // g = wave * NL + i.  For the A panel LDS row = tile row.  For the B panel LDS row r = span*128 + tn*32 + j
-  // holds tile row span*128 + 4*cg(j) + tn with cg(j) = 2*(j & 15) + (j >> 4): within a group (8 consecutive j)
-  // the rows are 8 apart, and the group's first row is span*128 + 64*(g & 1) + 4*((g >> 1) & 1) + (g%16)/4.
-  // The per-lane constants of the K loop (ten registers) are formed from an opaque copy of the lane number.  In the
+  // g = wave * NL + i.  For the A panel LDS row = tile row.  For the B panel LDS row r = span*128 + tn*16 + j
+  // holds tile row span*128 + 8*j + tn: within a group (8 consecutive j) the rows are 8 apart, and the group's
+  // first row is span*128 + 64*(g & 1) + (g%16)/2.
+  // The per-lane constants of the K loop (eight registers) are formed from an opaque copy of the lane number.  In the
   // instantiation that shares K ranges out they are formed afresh in front of every tile's K loop: there, values that
   // lived across the conversion of the C tile (the point of highest register pressure) were the ones the allocator
   // chose to spill, and it reloaded them inside the K loop.  The others have the registers to keep them (two hundred
   // cycles per tile with idle matrix cores otherwise).
-  uint32_t a_voff[2], b_voff[2], foff[2][2];
+  uint32_t a_voff[2], b_voff[2], foff[2];
   int chunk_even, chunk_odd;
   auto lane_consts = [&]() {
     int l = lane;
@@ -752,12 +766,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     a_voff[1] = (uint32_t)(lrow * (int)p.lda + chunk_odd);
     b_voff[0] = (uint32_t)(lrow * 8 * (int)p.ldb + chunk_even);
     b_voff[1] = (uint32_t)(lrow * 8 * (int)p.ldb + chunk_odd);
-    const int l31 = l & 31, h = l >> 5;
-    const int fr = (l31 & 7) ^ ((l31 >> 3) & 1);
+    const int l15 = l & 15, piece = l >> 4;  // fragment: lane l holds row l % 16, 16-byte chunks 2 (l / 16) and 2 (l / 16) + 1
+    const int fr = (l15 & 7) ^ (l15 >> 3);
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) foff[s][j] = l31 * BK + (((s * 4 + h * 2 + j) ^ fr) * 16);
+    for (int j = 0; j < 2; ++j) foff[j] = l15 * BK + (((piece * 2 + j) ^ fr) * 16);
   };
   lane_consts();
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem;
@@ -824,71 +836,54 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
                                                k0 + (wave * NL + i) * 8 * (int)p.lda, 0, 0);
     } else {
       const int g = wave * NL + i;  // 8-row group of the panel's LDS image
-      const int row = (g >> 4) * 128 + 64 * (g & 1) + 4 * ((g >> 1) & 1) + ((g & 15) >> 2);
+      const int row = (g >> 4) * 128 + 64 * (g & 1) + ((g & 15) >> 1);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsB, reinterpret_cast<lds_ptr_t>(dst), 16, b_voff[i & 1] | ((i & 1) ? m_odd : m_even),
                                                k0 + row * (int)p.ldb, 0, 0);
     }
   };
 
-  // ---- LDS -> register fragment plan (as in the kernel above) ----
-  const int a_base = wm * (TM * 32 * BK);
-  const int b_base = wn * (TN * 32 * BK);
+  // ---- LDS -> register fragment plan ----
+  const int a_base = wm * (WROWS * BK);
+  const int b_base = wn * (128 * BK);
   typedef const __attribute__((address_space(3))) v4i *lds_v4i_ptr;
-  auto frag_addrs = [&](int slot_a, int slot_b, int s, uint32_t (&ad)[4]) {
+  // LDS addresses of the two 16-byte pieces a lane reads of its A row (ad[0], ad[1]) and B row (ad[2], ad[3]); opaque
+  // additions, as in the kernel above
+  auto frag_addrs = [&](int slot_a, int slot_b, uint32_t (&ad)[4]) {
     const uint32_t sa = lds0 + slot_a * UNIT + a_base, sb = lds0 + slot_b * UNIT + b_base;
-    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[0]) : "s"(sa), "v"(foff[s][0]));
-    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[1]) : "s"(sa), "v"(foff[s][1]));
-    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[2]) : "s"(sb), "v"(foff[s][0]));
-    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[3]) : "s"(sb), "v"(foff[s][1]));
+    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[0]) : "s"(sa), "v"(foff[0]));
+    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[1]) : "s"(sa), "v"(foff[1]));
+    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[2]) : "s"(sb), "v"(foff[0]));
+    asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[3]) : "s"(sb), "v"(foff[1]));
   };
-  // fragment f, in the order the MFMAs need them: A0, B0 .. B(TN-1), A1 ..
-  auto read_one = [&](const uint32_t (&ad)[4], v8i (&af)[TM], v8i (&bf)[TN], int f) {
-    const bool is_a = f == 0 || f > TN;
-    const int t = f == 0 ? 0 : (f > TN ? f - TN : f - 1);
-    const v4i lo = *reinterpret_cast<lds_v4i_ptr>(ad[is_a ? 0 : 2] + t * (32 * BK));
-    const v4i hi = *reinterpret_cast<lds_v4i_ptr>(ad[is_a ? 1 : 3] + t * (32 * BK));
-    const v8i v = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-    if (is_a) af[t] = v;
-    else bf[t] = v;
+  // piece h of the fragment of tile t (16 rows) at the addresses of its lower and upper piece
+  auto read_piece = [&](const uint32_t *ad, v8i &f, int t, int h) {
+    const v4i v = *reinterpret_cast<lds_v4i_ptr>(ad[h] + t * (16 * BK));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f[h * 4 + k] = v[k];
   };
 
-  v16f acc[TM][TN];
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[tm][tn][v] = 0.0f;
-  // MFMA number idx of one 64-byte step, tm-major
-  auto mma_one = [&](v8i (&af)[TM], v8i (&bf)[TN], int idx) {
-    const int tm = idx / TN, tn = idx % TN;
-    acc[tm][tn] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[tm], bf[tn], acc[tm][tn], 0, 0, 0, 0, 0, 0);
-  };
+  v4f acc[TM][TN];
 
   // One accumulator element, fetched where it is used.  Written as assembly with an accumulator-register operand:
   // given plain reads, the register allocator moves the whole accumulator set into ordinary vector registers in
   // front of the conversion of the C tile and pays for it with spills inside the K loop.
   auto acc_read = [&](int tm, int tn, int i) -> float {
-    if constexpr (NW == 8) {
-      return acc[tm][tn][i];  // 128 accumulators: the allocator may keep them in ordinary registers
-    } else {
-      float x;
-      asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(acc[tm][tn][i]));
-      return x;
-    }
+    float x;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(acc[tm][tn][i]));
+    return x;
   };
   // ---- C tile straight from the accumulators ----
-  // acc[tm][tn][4*qd + e] of lane (l31, h) is C[m][n] with m = wm*WROWS + tm*32 + 8*qd + 4*h + e and
-  // n = wn*128 + 4*cg(l31) + tn (tile coordinates).  The host launches this kernel only when every lane pair's
-  // eight columns are in or out as a whole and its 16-byte store is aligned: N % 8 == 0, ldc % 8 == 0, C
-  // 16-byte aligned, row scales 16-byte and bias 8-byte aligned.
+  // acc[tm][tn][e] of lane l is C[m][n] with m = wm*WROWS + tm*16 + 4*(l / 16) + e and n = wn*128 + 8*(l % 16) + tn
+  // (tile coordinates).  The host launches this kernel only when every lane's eight columns are in or out as a whole
+  // and its 16-byte store is aligned: N % 8 == 0, ldc % 8 == 0, C 16-byte aligned, row scales 16-byte and bias
+  // 8-byte aligned.
   // The scales (and the bias) of a tile are requested before its K loop, a handful of registers per lane: lane l
-  // holds the A scales of tile rows wm*WROWS + l and (four waves) + 64 + l (handed to the lanes that need them by lane
-  // permutes at the end) and the B scales / bias of its own four columns.  Requested among the stores of the
+  // holds the A scales of tile rows wm*WROWS + l and + 64 + l (handed to the lanes that need them by lane permutes at
+  // the end) and the B scales / bias of its own eight columns.  Requested among the stores of the
   // tile they would make their consumer wait for every store ahead of them (the counter retires in order).
   int seg_sa[2] = {0, 0};
-  v4i seg_sb = {0, 0, 0, 0};
-  [[maybe_unused]] v2i seg_bias = {0, 0};
+  v4i seg_sb[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+  [[maybe_unused]] v4i seg_bias = {0, 0, 0, 0};
   // The descriptors cover the whole scale (bias) vectors and live as long as the kernel: a tile's requests then cost a
   // few address instructions (with a descriptor per tile, sixty scalar instructions at one per five cycles stood
   // between two tiles).  Rows past M and columns past N fall outside the range and read as zero; M, N < 2^29 here
@@ -905,8 +900,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     // epilogue needs them, so that none of them lives across a K loop
     int l = lane;
     asm volatile("" : "+v"(l));
-    const int l31 = l & 31;
-    const int cg = 2 * (l31 & 15) + (l31 >> 4);  // this lane's group of four output columns (of its wave's 32)
+    const int col = wn * 128 + 8 * (l & 15);  // this lane's eight output columns
     if (MULTI || p.sa_row) {
       __amdgpu_buffer_rsrc_t rs = rsSa;
       if constexpr (MULTI) {
@@ -914,16 +908,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
         rs = make_rsrc(t.sa, (uint32_t)t.M * 4u);
       }
       seg_sa[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + l) * 4, m0 * 4, 0);
-      if constexpr (TM == 4) seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
+      seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
     } else {
       seg_sa[0] = seg_sa[1] = sa_one;
     }
     if (p.sb_row) {
-      seg_sb = __builtin_amdgcn_raw_buffer_load_b128(rsSb, (wn * 128 + 4 * cg) * 4, n0 * 4, 0);
+      seg_sb[0] = __builtin_amdgcn_raw_buffer_load_b128(rsSb, col * 4, n0 * 4, 0);
+      seg_sb[1] = __builtin_amdgcn_raw_buffer_load_b128(rsSb, col * 4 + 16, n0 * 4, 0);
     } else {
-      seg_sb = v4i{sb_one, sb_one, sb_one, sb_one};
+      seg_sb[0] = seg_sb[1] = v4i{sb_one, sb_one, sb_one, sb_one};
     }
-    if constexpr (HAS_BIAS) seg_bias = __builtin_amdgcn_raw_buffer_load_b64(rsBias, (wn * 128 + 4 * cg) * 2, n0 * 2, 0);
+    if constexpr (HAS_BIAS) seg_bias = __builtin_amdgcn_raw_buffer_load_b128(rsBias, col * 2, n0 * 2, 0);
   };
   // (A compute unit drains its stores at about 16 bytes per clock: the 128 KiB of a C tile keep it busy for some
   // 8000 cycles, of which the conversion below hides about half.)
@@ -932,10 +927,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
   // Byte offset of piece i (of 64) of this wave in a slot.  The slots are 256 KiB apart and the workgroups of a
   // launch write theirs in step: the pieces are rotated by the slot number so that stores issued at the same time
   // do not all fall on the same memory channels.
-  [[maybe_unused]] auto piece_off = [&](int slot, int i) { return (wave * (TM * TN * 4) + ((i + slot * 5) & (TM * TN * 4 - 1))) * 1024; };
+  [[maybe_unused]] auto piece_off = [&](int slot, int i) { return (wave * (TM * TN) + ((i + slot * 5) & (TM * TN - 1))) * 1024; };
   [[maybe_unused]] __amdgpu_buffer_rsrc_t rs_p;
   [[maybe_unused]] int p_slot = 0;
-  constexpr int P_AHEAD = 3;  // groups / pieces of the partial sum requested ahead of their use (their latency is long)
   auto store_tile_as = [&](int m0, int n0, auto parts_tag, auto sbrow_tag) {
     constexpr bool PARTS = decltype(parts_tag)::value;
     // SB_ROW false: one scale for all columns; it is folded into the row scales (two multiplications per lane and
@@ -947,148 +941,102 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     asm volatile("" : "+s"(ldc2));
     int l = lane;
     asm volatile("" : "+v"(l));
-    const int l31 = l & 31, h = l >> 5;
-    int lane_col = wn * 128 + 8 * (l31 & 15);  // first of the eight columns this lane stores
+    const int quad = l >> 4;                // this lane's four rows of a tile of sixteen
+    int lane_col = wn * 128 + 8 * (l & 15);  // first of the eight columns this lane stores
     asm volatile("" : "+v"(lane_col));
     const GemmArgs::Part t = part_of(m0);
     const int64_t c_left = ((int64_t)(t.M - m0 - 1) * p.ldc + (p.N - n0)) * 2;
     const __amdgpu_buffer_rsrc_t rsC = make_rsrc(t.C + (int64_t)m0 * p.ldc + n0, c_left < 0x7fffffff ? (uint32_t)c_left : 0x7fffffffu);
-    float sbv[4];
-    [[maybe_unused]] float bv[4];
+    float sbv[TN];
+    [[maybe_unused]] float bv[TN];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) sbv[e] = __int_as_float(seg_sb[e]);
+    for (int e = 0; e < TN; ++e) sbv[e] = __int_as_float(seg_sb[e >> 2][e & 3]);
     if constexpr (HAS_BIAS) {
-      bv[0] = bf16_bits_to_f32((uint32_t)seg_bias[0] & 0xffffu);
-      bv[1] = bf16_bits_to_f32((uint32_t)seg_bias[0] >> 16);
-      bv[2] = bf16_bits_to_f32((uint32_t)seg_bias[1] & 0xffffu);
-      bv[3] = bf16_bits_to_f32((uint32_t)seg_bias[1] >> 16);
+#pragma unroll
+      for (int e = 0; e < TN; ++e) bv[e] = __uint_as_float(e & 1 ? (uint32_t)seg_bias[e >> 1] & 0xffff0000u : (uint32_t)seg_bias[e >> 1] << 16);
     }
-    // Row scale of tile row wm*WROWS + r: lane r % 64 of seg_sa[r / 64]; a lane needs r = tm*32 + 8*qd + 4*h + e.
-    // The lane permutes of the next (tm, qd) group are in flight while the current group is converted.  They are
-    // written as assembly for the immediate offset (as plain address arithmetic the 64 addresses were
-    // precomputed into 64 registers and spilled) and are waited for by hand: LDS operations return in order, so
+    // Row scale of tile row wm*WROWS + r: lane r % 64 of seg_sa[r / 64]; a lane needs r = tm*16 + 4*quad + e.
+    // The lane permutes of the next tm are in flight while the current one is converted.  They are
+    // written as assembly for the immediate offset (as plain address arithmetic their addresses were
+    // precomputed into a register each and spilled) and are waited for by hand: LDS operations return in order, so
     // "at most 4 outstanding" means that everything but the group requested last has arrived.
-    const int sa_addr = 16 * h;  // byte address of lane 4*h
+    const int sa_addr = 16 * quad;  // byte address of lane 4*quad
     const int sa_regs[2] = {SB_ROW ? seg_sa[0] : __float_as_int(__int_as_float(seg_sa[0]) * sbv[0]),
                             SB_ROW ? seg_sa[1] : __float_as_int(__int_as_float(seg_sa[1]) * sbv[0])};
     float sa_grp[2][4];
-    auto request_row_scales = [&](int g, float (&dst)[4]) {  // g = tm * 4 + qd
-      const int tm = g >> 2, qd = g & 3;
+    auto request_row_scales = [&](int tm, float (&dst)[4]) {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         asm volatile("ds_bpermute_b32 %0, %1, %2 offset:%3"
                      : "=v"(dst[e])
-                     : "v"(sa_addr), "v"(sa_regs[tm >> 1]), "n"(4 * ((tm & 1) * 32 + 8 * qd + e)));
+                     : "v"(sa_addr), "v"(sa_regs[tm >> 2]), "n"(4 * ((tm & 3) * 16 + e)));
     };
     request_row_scales(0, sa_grp[0]);
-    // partial sums of the group (tm, qd): one 16-byte piece per lane and accumulator, laid out as write_partial
-    // stores them; requested P_AHEAD groups ahead
-    [[maybe_unused]] v4f pbuf[P_AHEAD + 1][TN];
+    // partial sums of the tile row tm: one 16-byte piece per lane and accumulator, laid out as write_partial
+    // stores them; requested one tile row ahead
+    [[maybe_unused]] v4f pbuf[2][TN];
     [[maybe_unused]] const int p_voff = lane * 16;
-    [[maybe_unused]] auto request_parts = [&](int g, v4f (&dst)[TN]) {
-      const int tm = g >> 2, qd = g & 3;
+    [[maybe_unused]] auto request_parts = [&](int tm, v4f (&dst)[TN]) {
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn)
-        dst[tn] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(
-                                              rs_p, p_voff, piece_off(p_slot, (tm * TN + tn) * 4 + qd), kCoherent));
+        dst[tn] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(rs_p, p_voff, piece_off(p_slot, tm * TN + tn), kCoherent));
     };
-    if constexpr (PARTS) {
-#pragma unroll
-      for (int g = 0; g < P_AHEAD; ++g) request_parts(g, pbuf[g]);
-    }
-    // (the values of C that an ADD tile is added to, two 16-byte pieces per lane and row group)
-    constexpr int C_AHEAD = 4;
-    [[maybe_unused]] v4i cbuf[C_AHEAD + 1][2];
-    [[maybe_unused]] uint64_t tq0 = 0, tq1 = 0, tq2 = 0;
-    if (L8_GEMM_PROF) {
-      tq0 = __builtin_readcyclecounter();
-      __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0), lgkmcnt(0): the panel loads in flight
-      tq1 = __builtin_readcyclecounter();
-      prof[8] += tq1 - tq0;
-    }
-    // A store instruction costs the same whatever it carries, so lanes j and j+16 pair up: of two consecutive
-    // rows, lane j takes the first (its own four columns and its partner's four, 16 contiguous bytes) and lane
-    // j+16 the second.  One instruction then writes four rows x 256 bytes.  Lanes whose columns lie beyond N
-    // store nothing (N % 8 == 0 here: a lane pair is in or out as a whole).
-    const int par = l31 >> 4;
-    const uint32_t c_voff = (n0 + lane_col < p.N) ? (uint32_t)((4 * h + par) * ldc2 + lane_col * 2) : kOOB;
-    [[maybe_unused]] auto request_c = [&](int g, v4i (&dst)[2]) {
-      const int row = wm * WROWS + (g >> 2) * 32 + 8 * (g & 3);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) dst[i] = __builtin_amdgcn_raw_buffer_load_b128(rsC, c_voff, (row + 2 * i) * ldc2, 2 /* streaming */);
+    if constexpr (PARTS) request_parts(0, pbuf[0]);
+    // (the values of C that an ADD tile is added to, 16 bytes per lane and row)
+    constexpr int C_AHEAD = 8;
+    [[maybe_unused]] v4i cbuf[C_AHEAD + 1];
+    // Lanes whose columns lie beyond N store nothing (N % 8 == 0 here: a lane is in or out as a whole).
+    const uint32_t c_voff = (n0 + lane_col < p.N) ? (uint32_t)(4 * quad * ldc2 + lane_col * 2) : kOOB;
+    [[maybe_unused]] auto request_c = [&](int i, v4i &dst) {  // i = tm * 4 + e
+      dst = __builtin_amdgcn_raw_buffer_load_b128(rsC, c_voff, (wm * WROWS + (i >> 2) * 16 + (i & 3)) * ldc2, 2 /* streaming */);
     };
     if constexpr (ADD) {
 #pragma unroll
-      for (int g = 0; g < C_AHEAD; ++g) request_c(g, cbuf[g]);
-    }
-    if (L8_GEMM_PROF) {
-      __builtin_amdgcn_s_waitcnt(0x0070);  // the scales
-      tq2 = __builtin_readcyclecounter();
-      prof[9] += tq2 - tq1;
+      for (int i = 0; i < C_AHEAD; ++i) request_c(i, cbuf[i]);
     }
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
+      float(&sa_cur)[4] = sa_grp[tm & 1];
+      if constexpr (PARTS) {
+        if (tm + 1 < TM) request_parts(tm + 1, pbuf[(tm + 1) & 1]);
+      }
+      if (tm + 1 < TM) {
+        request_row_scales(tm + 1, sa_grp[(tm + 1) & 1]);
+        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(sa_cur[0]), "+v"(sa_cur[1]), "+v"(sa_cur[2]), "+v"(sa_cur[3]));
+      } else {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sa_cur[0]), "+v"(sa_cur[1]), "+v"(sa_cur[2]), "+v"(sa_cur[3]));
+      }
 #pragma unroll
-      for (int qd = 0; qd < 4; ++qd) {
-        const int row = wm * WROWS + tm * 32 + 8 * qd;  // + 4*h + e
-        const int g = tm * 4 + qd;
-        float(&sa_cur)[4] = sa_grp[g & 1];
-        if constexpr (PARTS) {
-          if (g + P_AHEAD < TM * 4) request_parts(g + P_AHEAD, pbuf[(g + P_AHEAD) % (P_AHEAD + 1)]);
-        }
+      for (int e = 0; e < 4; ++e) {
+        const int i = tm * 4 + e;
         if constexpr (ADD) {
-          if (g + C_AHEAD < TM * 4) request_c(g + C_AHEAD, cbuf[(g + C_AHEAD) % (C_AHEAD + 1)]);
+          if (i + C_AHEAD < TM * 4) request_c(i + C_AHEAD, cbuf[(i + C_AHEAD) % (C_AHEAD + 1)]);
         }
-        if (g + 1 < TM * 4) {
-          request_row_scales(g + 1, sa_grp[(g + 1) & 1]);
-          asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(sa_cur[0]), "+v"(sa_cur[1]), "+v"(sa_cur[2]), "+v"(sa_cur[3]));
-        } else {
-          asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(sa_cur[0]), "+v"(sa_cur[1]), "+v"(sa_cur[2]), "+v"(sa_cur[3]));
-        }
+        const float sa = sa_cur[e];
+        v4i out;
 #pragma unroll
-        for (int e2 = 0; e2 < 4; e2 += 2) {
-          int o[2][2];  // [row e2 / e2+1][low / high pair of columns]
+        for (int pair = 0; pair < TN / 2; ++pair) {
+          float v[2];
 #pragma unroll
-          for (int r = 0; r < 2; ++r) {
-            const float sa = sa_cur[e2 + r];
-            float v[4];
-#pragma unroll
-            for (int tn = 0; tn < TN; ++tn) {
-              float a = acc_read(tm, tn, 4 * qd + e2 + r);
-              if constexpr (PARTS) a = a + pbuf[g % (P_AHEAD + 1)][tn][e2 + r];  // ascending K
-              v[tn] = SB_ROW ? a * sa * sbv[tn] : a * sa;
-              if constexpr (HAS_BIAS) v[tn] += bv[tn];
-            }
-            typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-            const bf2 lo = {(__bf16)v[0], (__bf16)v[1]}, hi = {(__bf16)v[2], (__bf16)v[3]};
-            o[r][0] = __builtin_bit_cast(int, lo);
-            o[r][1] = __builtin_bit_cast(int, hi);
+          for (int k = 0; k < 2; ++k) {
+            const int tn = pair * 2 + k;
+            float a = acc_read(tm, tn, e);
+            if constexpr (PARTS) a = a + pbuf[tm & 1][tn][e];  // ascending K
+            v[k] = SB_ROW ? a * sa * sbv[tn] : a * sa;
+            if constexpr (HAS_BIAS) v[k] += bv[tn];
           }
-          // lanes 0..15 of every 32 hand over their second row and get their partners' first, lanes 16..31 the
-          // other way round: v_permlane16_swap exchanges the odd rows of 16 lanes of its first operand with the
-          // even rows of its second
-          const auto s0 = __builtin_amdgcn_permlane16_swap((unsigned)o[0][0], (unsigned)o[1][0], false, false);
-          const auto s1 = __builtin_amdgcn_permlane16_swap((unsigned)o[0][1], (unsigned)o[1][1], false, false);
-          v4i out = {(int)s0[0], (int)s1[0], (int)s0[1], (int)s1[1]};
-          if constexpr (ADD) out = add_bf16x8(out, cbuf[g % (C_AHEAD + 1)][e2 / 2]);
-          if (L8_GEMM_DIAG != 3 && !(L8_GEMM_DIAG == 8 && (qd & 1)))  // experiments: no stores (3), half of them (8)
-            store16(out, rsC, c_voff, (row + e2) * ldc2, 2 /* streaming */);
-          // one row pair at a time: left free, the scheduler reads a hundred accumulator registers ahead and the
-          // register pressure of this conversion makes the allocator spill values the K loop uses in every trip
-          __builtin_amdgcn_sched_barrier(0);
+          typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+          const bf2 b = {(__bf16)v[0], (__bf16)v[1]};
+          out[pair] = __builtin_bit_cast(int, b);
         }
+        if constexpr (ADD) out = add_bf16x8(out, cbuf[i % (C_AHEAD + 1)]);
+        if (L8_GEMM_DIAG != 3)  // experiment: no stores
+          store16(out, rsC, c_voff, (wm * WROWS + tm * 16 + e) * ldc2, 2 /* streaming */);
+        // one row at a time: left free, the scheduler reads a hundred accumulator registers ahead and the register
+        // pressure of this conversion makes the allocator spill values the K loop uses in every trip
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
-    if (L8_GEMM_PROF) {
-      tq0 = __builtin_readcyclecounter();
-      prof[10] += tq0 - tq2;
-    }
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[tm][tn][v] = 0.0f;
   };
 
   auto store_tile = [&](int m0, int n0, auto parts_tag) {
@@ -1097,8 +1045,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     // converted with a scalar scale" (which no launch takes) left their registers marked as awaited, and the first
     // write to one of them between two tiles got an s_waitcnt vmcnt(0) -- a wait for every store of the tile just
     // written, some 600 cycles with idle matrix cores.
-    if constexpr (HAS_BIAS) asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb), "v"(seg_bias));
-    else asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb));
+    if constexpr (HAS_BIAS) asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb[0]), "v"(seg_sb[1]), "v"(seg_bias));
+    else asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb[0]), "v"(seg_sb[1]));
     if (p.sb_row) store_tile_as(m0, n0, parts_tag, std::true_type{});
     else store_tile_as(m0, n0, parts_tag, std::false_type{});
   };
@@ -1119,19 +1067,10 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) {
-#pragma unroll
-        for (int qd = 0; qd < 4; ++qd) {
-          const v4f v = {acc_read(tm, tn, 4 * qd), acc_read(tm, tn, 4 * qd + 1), acc_read(tm, tn, 4 * qd + 2), acc_read(tm, tn, 4 * qd + 3)};
-          store16(__builtin_bit_cast(v4i, v), rs, voff, piece_off(slot, (tm * TN + tn) * 4 + qd), kCoherent);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        const v4f v = {acc_read(tm, tn, 0), acc_read(tm, tn, 1), acc_read(tm, tn, 2), acc_read(tm, tn, 3)};
+        store16(__builtin_bit_cast(v4i, v), rs, voff, piece_off(slot, tm * TN + tn), kCoherent);
+        if (tn & 1) __builtin_amdgcn_sched_barrier(0);
       }
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[tm][tn][v] = 0.0f;
     L8_WAIT_VM_LGKM0(0);  // this wave's part of the tile has reached the point of coherence
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -1151,11 +1090,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     return false;
   };
 
-  if (L8_GEMM_DIAG == 5 || L8_GEMM_DIAG == 6) {  // experiments: XCD x starts x/8 of a tile's duration late (5); workgroup loc of an XCD starts loc/256 of it late (6)
-    const uint64_t t_go = __builtin_amdgcn_s_memrealtime() + (L8_GEMM_DIAG == 5 ? (uint64_t)xcd * (uint64_t)KT * 17 : (uint64_t)loc * (uint64_t)KT * 17 / 32);  // ~1.36 us per K tile, 100 MHz ticks
-    while (__builtin_amdgcn_s_memrealtime() < t_go) __builtin_amdgcn_s_sleep(8);
-  }
-  // ---- prologue: K tiles 0 and 1 of the workgroup's stream requested, K tile 0 published, its first step read ----
+  // ---- prologue: K tiles 0 and 1 of the workgroup's stream requested, K tile 0 published, its first fragments read ----
   ld_open(0);
 #pragma unroll
   for (int u = 0; u < R - 1; ++u) {
@@ -1163,73 +1098,96 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     for (int i = 0; i < NL; ++i) load_one(u & 1, u, i);
     if (u & 1) ld_advance();
   }
-  v8i af0[TM], bf0[TN], af1[TM], bf1[TN];
-  uint32_t ad[4];
   L8_WAIT_VM_LGKM0(PEND0);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  frag_addrs(0, 1, 0, ad);
+  // One trip = one K tile = 64 MFMAs, row by row of the wave's 8 x 8 tiles.
+  //   first half : rows 0 .. 3, while the A fragments of rows 2 .. 7 are read and the A panel two K tiles ahead is
+  //                requested (into the slot that the previous barrier released);
+  //   barrier    : every wave has now read all of this K tile (lgkmcnt 0), and the next one has landed for every
+  //                wave (partial vmcnt wait);
+  //   second half: rows 4 .. 7, while the next K tile's eight B fragments and first two A fragments are read and
+  //                the matching B panel is requested into the A slot this K tile just released.
+  // A fragment lives for its row, the B fragments for the whole trip: two sets of them, in turn.  A wave issues in
+  // order and the matrix cores want an MFMA every 32 cycles, half a dozen issue slots, so a group is one MFMA with at
+  // most one LDS read and one panel load, and the scheduling fences keep the groups as they are laid out here.
+  constexpr int N_MMA = TM * TN, HALF = N_MMA / 2;
+  constexpr int A_EARLY = 2;                       // A fragments read in the trip before
+  constexpr int N_RD1 = 2 * (TM - A_EARLY), N_RD2 = 2 * (TN + A_EARLY);
+  constexpr int RD1_GROUPS = L8_READ_GROUPS1, RD2_GROUPS = L8_READ_GROUPS2;  // groups over which a half spreads its reads
+  static_assert(RD1_GROUPS < HALF - 4 && RD2_GROUPS <= HALF, "reads of the first half land before the barrier");
+  v8i af[TM], bf0[TN], bf1[TN];
+  uint32_t ad[4];
+  // read number r of the second half: B0, A0, B1, .. B7, A1, .. (the order of their use), two pieces each
+  auto read_next = [&](v8i (&bn)[TN], int r) {
+    const int f = r >> 1;
+    if (f == 0) read_piece(ad + 2, bn[0], 0, r & 1);
+    else if (f == 1) read_piece(ad, af[0], 0, r & 1);
+    else if (f <= TN) read_piece(ad + 2, bn[f - 1], f - 1, r & 1);
+    else read_piece(ad, af[f - TN], f - TN, r & 1);
+  };
+  frag_addrs(0, 1, ad);
 #pragma unroll
-  for (int f = 0; f < TM + TN; ++f) read_one(ad, af0, bf0, f);
-
-  // One trip = one K tile = two matrix-core steps of 64, laid out as in the kernel above: first half = MFMAs
-  // of step 0 + LDS reads of step 1 + requests for the A panel two K tiles ahead; barrier; second half =
-  // MFMAs of step 1 + LDS reads of the next K tile's step 0 + requests for the matching B panel.
-  constexpr int N_MMA = TM * TN, NF = TM + TN;
-  constexpr int STRADDLE = L8_STRADDLE < N_MMA - 2 ? L8_STRADDLE : 0;
-  constexpr int S1 = N_MMA - STRADDLE, S2 = N_MMA + STRADDLE;
+  for (int r = 0; r < N_RD2; ++r) read_next(bf0, r);
   int s0 = 0;  // ring slot of the A panel of the K tile being multiplied
-  // WAIT = the count of the wait in front of the barrier: everything older than the WAIT youngest requests must
-  // have landed.
-  // A wave issues in order and the matrix cores want an MFMA every 64 cycles, about a dozen issue slots: a group
-  // that carries more than that leaves them idle.  So nothing but its MFMA, LDS reads and panel loads goes into a
-  // group: the fragment addresses of a half are formed in the middle of the half before (ad_a for the first half,
-  // ad_b for the second), and the LDS reads of a half are all issued in its first RD groups, so that the wait for
-  // them at the end of the half (barrier, loop top) finds them landed.
-  constexpr int RD = L8_READ_GROUPS < S1 ? L8_READ_GROUPS : S1, G_ADDR = N_MMA / 2;
-  static_assert(RD >= NF / 2 && RD <= S1 && RD <= S2 - STRADDLE && G_ADDR < S1, "group layout");
-  uint32_t ad_a[4], ad_b[4];
-  frag_addrs(0, 1, 1, ad_a);
-  auto trip = [&](auto wait_tag) {
-    constexpr int WAIT = decltype(wait_tag)::value;
+  // FIRST: the first K tile of an output tile (the accumulators start from zero); `stores`: the stores of a C tile have
+  // been issued since the panels that the trip's barrier waits for were requested.  They are younger than the panels and
+  // the counter retires in order, so the count allows for them (waiting for the stores themselves would stall the start
+  // of every tile).
+  auto trip = [&](auto first_tag, bool stores, v8i (&bc)[TN], v8i (&bn)[TN]) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_tag)::value;
     const int slot_u1 = wrap(s0 + R - 1);
+    auto mma_one = [&](int i) __attribute__((always_inline)) {
+      const int tm = i / TN, tn = i % TN;
+      acc[tm][tn] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af[tm], bc[tn], FIRST ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : acc[tm][tn], 0, 0, 0, 0, 0, 0);
+    };
 #pragma unroll
-    for (int i = 0; i < S1; ++i) {
-      mma_one(af0, bf0, i);
-      if (i < RD) {
+    for (int i = 0; i < HALF; ++i) {
+      mma_one(i);
+      if (i < RD1_GROUPS) {
 #pragma unroll
-        for (int f = (NF * i) / RD; f < (NF * (i + 1)) / RD; ++f) read_one(ad_a, af1, bf1, f);
+        for (int r = (N_RD1 * i) / RD1_GROUPS; r < (N_RD1 * (i + 1)) / RD1_GROUPS; ++r) read_piece(ad, af[A_EARLY + r / 2], A_EARLY + r / 2, r & 1);
       }
 #pragma unroll
-      for (int j = (NL * i) / S1; j < (NL * (i + 1)) / S1; ++j) load_one(false, slot_u1, j);
-      if (i == G_ADDR) frag_addrs(wrap(s0 + 2), wrap(s0 + 3), 0, ad_b);
+      for (int j = (NL * i) / HALF; j < (NL * (i + 1)) / HALF; ++j) load_one(false, slot_u1, j);
+      if (i == RD1_GROUPS) frag_addrs(wrap(s0 + 2), wrap(s0 + 3), ad);
       __builtin_amdgcn_sched_barrier(0);
     }
-    L8_WAIT_VM_LGKM0(WAIT);
+    if (FIRST && stores) L8_WAIT_VM_LGKM0(N_STORES + PEND);
+    else L8_WAIT_VM_LGKM0(PEND);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < S2; ++i) {
-      if (i < STRADDLE) mma_one(af0, bf0, S1 + i);
-      else mma_one(af1, bf1, i - STRADDLE);
-      if (i >= STRADDLE && i - STRADDLE < RD) {
+    for (int i = 0; i < HALF; ++i) {
+      mma_one(HALF + i);
+      if (i < RD2_GROUPS) {
 #pragma unroll
-        for (int f = (NF * (i - STRADDLE)) / RD; f < (NF * (i - STRADDLE + 1)) / RD; ++f) read_one(ad_b, af0, bf0, f);
+        for (int r = (N_RD2 * i) / RD2_GROUPS; r < (N_RD2 * (i + 1)) / RD2_GROUPS; ++r) read_next(bn, r);
       }
 #pragma unroll
-      for (int j = (NL * i) / S2; j < (NL * (i + 1)) / S2; ++j) load_one(true, s0, j);
-      if (i == STRADDLE + G_ADDR) {
-        const int s_next = wrap(s0 + 2);
-        frag_addrs(s_next, wrap(s_next + 1), 1, ad_a);
-      }
+      for (int j = (NL * i) / HALF; j < (NL * (i + 1)) / HALF; ++j) load_one(true, s0, j);
       __builtin_amdgcn_sched_barrier(0);
     }
     ld_advance();
     s0 = wrap(s0 + 2);
   };
-  using std::integral_constant;
+  // n K tiles of one output tile.  Its first one finds its B fragments in bf0.
+  auto k_loop = [&](int n, bool stores) __attribute__((always_inline)) {
+    trip(std::true_type{}, stores, bf0, bf1);
+#pragma unroll 1
+    for (n -= 1; n >= 2; n -= 2) {
+      trip(std::false_type{}, false, bf1, bf0);
+      trip(std::false_type{}, false, bf0, bf1);
+    }
+    if (n) {
+      trip(std::false_type{}, false, bf1, bf0);
+    } else {  // an odd number of K tiles: the next tile's fragments are in the other set
+#pragma unroll
+      for (int t = 0; t < TN; ++t) bf0[t] = bf1[t];
+    }
+  };
 #pragma unroll 1
   for (int seg = 0; seg < n_seg; ++seg) {
     [[maybe_unused]] uint64_t t_loop = 0;
@@ -1240,37 +1198,9 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     int m0, n0;
     cursor_origin(cur_mul, m0, n0);
     cursor_step(cur_mul);
-    if (L8_GEMM_PROF && seg > 0) prof[17] += __builtin_readcyclecounter() - t_loop;
     if (SK && seg > 0) lane_consts();
-    if (L8_GEMM_PROF && seg > 0) {
-      asm volatile("" : "+v"(a_voff[0]), "+v"(b_voff[1]), "+v"(foff[1][1]));
-      prof[18] += __builtin_readcyclecounter() - t_loop;
-    }
     load_scales(m0, n0);
-    int kt = 0;
-    if (L8_GEMM_PROF && seg > 0) prof[16] += __builtin_readcyclecounter() - t_loop;  // tile origin, lane constants, scale requests
-    if (seg > 0) {
-      // The first barrier after the N_STORES stores of a C tile: they are younger than the panels waited for
-      // and the counter retires in order, so the count allows for them (waiting for the stores themselves would
-      // stall the start of every tile).
-      trip(integral_constant<int, N_STORES + PEND>{});
-      kt = 1;
-      if (L8_GEMM_PROF && !SK && KT > 4) {  // the first trips after a stored tile, one by one
-        const uint64_t ta = __builtin_readcyclecounter();
-        prof[12] += ta - t_loop;
-        trip(integral_constant<int, PEND>{});
-        const uint64_t tb = __builtin_readcyclecounter();
-        prof[13] += tb - ta;
-        trip(integral_constant<int, PEND>{});
-        const uint64_t tc = __builtin_readcyclecounter();
-        prof[14] += tc - tb;
-        trip(integral_constant<int, PEND>{});
-        prof[15] += __builtin_readcyclecounter() - tc;
-        kt = 4;
-      }
-    }
-#pragma unroll 1
-    for (; kt < KT; ++kt) trip(integral_constant<int, PEND>{});
+    k_loop(KT, seg > 0);
     if (L8_GEMM_PROF) {
       const uint64_t t = __builtin_readcyclecounter();
       prof[3] += t - t_loop;
@@ -1279,7 +1209,6 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     store_tile(m0, n0, std::false_type{});
     if (L8_GEMM_PROF) prof[4] += __builtin_readcyclecounter() - t_loop;
   }
-  if (L8_GEMM_PROF) prof[11] = __builtin_amdgcn_s_memrealtime();
   if constexpr (SK) {
     // ---- the workgroup's share of the tail ----
     bool after_store = true;  // the segment before ended with the N_STORES stores of a C tile (n_seg > 0 here)
@@ -1291,35 +1220,20 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
       const int slot = tt * 8 + xcd;
       lane_consts();
       if (owns) load_scales(m0, n0);
-      [[maybe_unused]] uint64_t t_a = 0, t_b = 0;
-      if (L8_GEMM_PROF) t_a = __builtin_readcyclecounter();
-      if (after_store) trip(integral_constant<int, N_STORES + PEND>{});
-      else trip(integral_constant<int, PEND>{});  // write_partial waited for everything in flight
-#pragma unroll 1
-      for (int kt = piece_kb + 1; kt < piece_ke; ++kt) trip(integral_constant<int, PEND>{});
-      if (L8_GEMM_PROF) {
-        t_b = __builtin_readcyclecounter();
-        prof[12] += t_b - t_a;
-      }
+      k_loop(piece_ke - piece_kb, after_store);  // write_partial waited for everything in flight
       if (!owns) {
         write_partial(slot);
         after_store = false;
-        if (L8_GEMM_PROF) prof[13] += __builtin_readcyclecounter() - t_b;
       } else {
         if (!wait_partial(slot)) {
           seg_sa[0] = seg_sa[1] = 0x7fc00000;  // every row scale a NaN
           // and the host can find out: one more tile poisoned, counted in the workspace (never reset by the library)
           if (threadIdx.x == 0) atomicAdd(p.sk_flags + kSkGaveUpWord, 1u);
         }
-        if (L8_GEMM_PROF) {
-          t_a = __builtin_readcyclecounter();
-          prof[14] += t_a - t_b;
-        }
         rs_p = partial_rsrc(slot);
         p_slot = slot;
         store_tile(m0, n0, std::true_type{});
         after_store = true;
-        if (L8_GEMM_PROF) prof[15] += __builtin_readcyclecounter() - t_a;
       }
     }
   }
@@ -1331,8 +1245,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_nt_stream_kernel(const GemmArgs 
     prof[6] = n_seg;
     prof[7] = ((uint64_t)__builtin_amdgcn_s_getreg(63508) << 32) | (uint32_t)__builtin_amdgcn_s_getreg(63492);  // XCC_ID, HW_ID
     if (threadIdx.x == 0 && p.dbg) {
-      uint64_t *d = p.dbg + (int64_t)blockIdx.x * 24;
-      for (int i = 0; i < 24; ++i) d[i] = prof[i];
+      uint64_t *d = p.dbg + (int64_t)blockIdx.x * 8;
+      for (int i = 0; i < 8; ++i) d[i] = prof[i];
     }
   }
 #else
@@ -1405,35 +1319,34 @@ template __global__ void gemm_nt_stream_kernel<8, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, true>(const GemmArgs);
-template __global__ void gemm_nt_stream_kernel<4, false, false, 4, true>(const GemmArgs);
-template __global__ void gemm_nt_stream_kernel<4, false, false, 4, false, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, true>(const GemmArgs);
-template __global__ void gemm_nt_stream_kernel<4, false, false, 8>(const GemmArgs);
 
 static_assert(kSkinnyAlgo == 17, "position in the list below");
 static const Algo kAlgos[] = {
     L8_ALGO_LIST(L8_ALGO_ROW)
     /* 11, 12: persistent 256x256 tiles, 4 waves, one panel stream across tiles, C stored from the accumulators */
-    {"stream_mt2x2w_4x4t_r5_g8", gemm_nt_stream_kernel<8, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<8, true>, nullptr, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g8", gemm_nt_stream_kernel<8, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<8, true>, gemm_nt_stream_kernel<4, false, false, true>, nullptr},
     {"stream_mt2x2w_4x4t_r5_g4", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>,
-     gemm_nt_stream_kernel<4, false, false, 4, true>, nullptr},
+     gemm_nt_stream_kernel<4, false, false, true>, nullptr},
     /* 13, 14: other shapes of the block of tiles resident on an XCD (2 x 16 and 16 x 2 instead of 4 x 8: 18 panels
        shared by 32 tiles instead of 12), kept for the traffic comparison */
-    {"stream_mt2x2w_4x4t_r5_g2", gemm_nt_stream_kernel<2, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<2, true>, nullptr, nullptr},
-    {"stream_mt2x2w_4x4t_r5_g16", gemm_nt_stream_kernel<16, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<16, true>, nullptr, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g2", gemm_nt_stream_kernel<2, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<2, true>, gemm_nt_stream_kernel<4, false, false, true>, nullptr},
+    {"stream_mt2x2w_4x4t_r5_g16", gemm_nt_stream_kernel<16, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<16, true>, gemm_nt_stream_kernel<4, false, false, true>, nullptr},
     /* 15: algo 12 that may share the K range of the last round's tiles out between workgroups (l8_gemm_nt_ws with
        a workspace; without one it is algo 12).  Measured neutral on the shapes it applies to: the part is
        power-limited, and the compute units that the plain split leaves idle in the last round let the busy ones
        clock higher, which recovers most of what the idle ones lose. */
     {"stream_mt2x2w_4x4t_r5_g4_sk", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>,
-     gemm_nt_stream_kernel<4, false, false, 4, true>, gemm_nt_stream_kernel<4, false, true>},
-    /* 16: algo 12 with eight waves (two per SIMD, 64x128 each), kept for the comparison: measured 1-2 % ahead of
-       algo 12 at K = 4096 and 2-4 % behind it at K >= 8192 (1.5 x the LDS reads); a product with a bias takes the
-       plain kernel (the bias instantiation would not fit the 256 registers of a wave without spills) */
-    {"stream_mt4x2w_2x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, 8>, 256, 256, 512, 5 * 256 * 128, true, nullptr, nullptr, nullptr},
+     gemm_nt_stream_kernel<4, false, false, true>, gemm_nt_stream_kernel<4, false, true>},
+    /* 16: was algo 12 with eight waves (two per SIMD), behind it since the fragments of a K tile take 192 registers;
+       the number stands for algo 12 */
+    {"stream_mt2x2w_4x4t_r5_g4", gemm_nt_stream_kernel<4, false>, 256, 256, 256, 5 * 256 * 128, true, gemm_nt_stream_kernel<4, true>,
+     gemm_nt_stream_kernel<4, false, false, true>, nullptr},
     /* 17: at most 64 tokens: 16 rows of B and all of A per workgroup, K split over its waves (skinny_kernels.hip) */
     {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr, nullptr},
     L8_SMALL_ALGO_LIST(L8_ALGO_ROW)
@@ -1713,7 +1626,7 @@ extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void
     return L8_OK;
   }
   constexpr int kLds = 5 * 256 * 128;
-  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, 4, false, true>;
+  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, false, true>;
   GemmArgs p{};
   p.A = (const uint8_t *)parts[0].A;
   p.B = (const uint8_t *)B;

@@ -42,6 +42,24 @@ def test_exact_small_integer_operands(algo):
         assert torch.equal(out.cpu().double(), want), (algo, M, N, K)
 
 
+@pytest.mark.parametrize("K", [16, 128, 144, 256, 272, 400, 528, 1152])
+@pytest.mark.parametrize("with_bias,scalar", [(False, False), (False, True), (True, False)])
+def test_persistent_kernel_carries_its_fragments_from_tile_to_tile(K, with_bias, scalar):
+    """One to nine K tiles per output tile (even and odd numbers of them leave the next tile's fragments in one or the other
+    register set, the last K tile short or whole) and 289 output tiles, so that some workgroups have two; ragged last tiles.
+    Integers in -1 .. 1 and powers of two for scales: the fp32 sums are exact, so is the one rounding to bf16."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(170 + K)
+    M, N = 4101, 4104
+    A, B = (torch.randint(-1, 2, (n, K), generator=g).float() for n in (M, N))
+    sa = torch.tensor([2.0 ** (i % 5 - 2) for i in range(M)]).reshape(M, 1).cuda()
+    sb = torch.tensor([2.0 ** (i % 3) for i in range(1 if scalar else N)]).reshape(-1, 1).cuda()
+    bias = torch.randint(-8, 9, (N,), generator=g).to(torch.bfloat16).cuda() if with_bias else None
+    out = ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa, sb, bias, algo=12)
+    want = (A.cuda() @ B.cuda().t()) * sa * sb.t() + (0 if bias is None else bias.float())   # fp32: exact here
+    assert torch.equal(out, want.to(torch.bfloat16))
+
+
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 48, 49, 64])
 def test_few_tokens_exact_on_integers_and_within_tolerance_of_the_oracle(M):
     """At most 64 tokens (the default's choice; 65 take a tile kernel): token tiles of 16 full and ragged, weight rows
