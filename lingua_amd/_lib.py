@@ -63,6 +63,7 @@ _RETURNS_I64 = {"l8_cast_rowwise_workspace", "l8_gemm_workspace", "l8_gemm_works
                 "l8_linear_fwd_workspace"}
 
 _lib = None
+_native = None    # the host extension, bound to the library's entries
 _lock = threading.Lock()
 _checked_devices = set()
 
@@ -86,6 +87,22 @@ def load():
                 fn.restype = ctypes.c_char_p if name in _RETURNS_STR else (_i64 if name in _RETURNS_I64 else _int)
             _lib = lib
     return _lib
+
+
+def native_for(index: int):
+    """The host extension, after ``require_device(index)``."""
+    global _native
+    if index not in _checked_devices:
+        require_device(index)
+    if _native is None:
+        try:
+            from . import _native as ext
+        except ImportError as e:
+            raise RuntimeError(f"the host extension is missing or was built for another PyTorch ({e}): build it with "
+                               "`python -m lingua_amd.build` (there is no fallback implementation)") from e
+        ext.bind(load()._handle)
+        _native = ext
+    return _native
 
 
 def last_error() -> str:

@@ -1,4 +1,4 @@
-"""Builds ``liblingua_fp8.so`` (gfx950 only) next to this file with hipcc.
+"""Builds ``liblingua_fp8.so`` (gfx950 only) next to this file with hipcc, and the host extension ``_native.so``.
 
 ``python -m lingua_amd.build`` or ``lingua_amd.build.build()``.  The library is
 built ahead of time, in-tree; nothing compiles at import or at first call.
@@ -7,6 +7,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -29,6 +30,20 @@ HIPCC_FLAGS = [
     "-Wall",
     "-Wno-unused-command-line-argument",
 ]
+
+
+NATIVE_PATH = os.path.join(_HERE, "_native.so")   # host path of the linear (csrc/native.cpp), a Python extension
+
+
+def _native_cmd():
+    """Compiles against the PyTorch that is installed, whose headers for ROCm ask for the two definitions."""
+    import torch
+    root = os.path.dirname(torch.__file__)
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               sysconfig.get_paths()["include"], os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include")]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{i}" for i in include),
+            os.path.join(CSRC, "native.cpp"), "-o", NATIVE_PATH, f"-L{os.path.join(root, 'lib')}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
 
 
 def _run(cmd, verbose):
@@ -93,6 +108,8 @@ def build(verbose: bool = False) -> str:
     objs = [os.path.join(obj_dir, os.path.splitext(src)[0] + ".o") for src in SOURCES]
     cmds = [[hipcc, *HIPCC_FLAGS, *extra, *(["-Rpass-analysis=kernel-resource-usage"] if src.endswith(".hip") else []),
              "-c", os.path.join(CSRC, src), "-o", obj] for src, obj in zip(SOURCES, objs)]
+    if not os.environ.get("LINGUA_FP8_LIB"):   # a tuning variant of the library is used through the same extension
+        cmds.append(_native_cmd())
     with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 1)) as pool:
         usages = list(pool.map(lambda c: _run(c, verbose), cmds))
     usage = {k: v for u in usages for k, v in u.items()}

@@ -42,7 +42,7 @@ from typing import Callable, Optional
 import torch
 from torch.autograd import forward_ad
 
-from . import ops
+from . import _lib, ops
 
 # avoid division by zero when calculating scale (same value as the reference)
 EPS = 1e-12
@@ -177,6 +177,8 @@ class _LastCast:
 
     @staticmethod
     def _key(t):
+        if t.is_cuda:
+            return _lib.native_for(t.get_device()).key(t)
         return (t.data_ptr(), t.shape, t.stride(), t.dtype, t.device, t._version, ops.current_stream_ptr(t.device.index))
 
     def get(self, t, user):
@@ -328,6 +330,12 @@ def _check_operands(a, b_t):
         raise RuntimeError(f"Fp8LinearFn: in_features ({a.shape[-1]}) and out_features ({b_t.shape[0]}) must be multiples of 16")
 
 
+def _native_call(a, gemm_algo) -> bool:
+    """May the host extension make the call?  Not where a timer wants to see the kernels one by one, nor for the tile
+    configuration that needs a workspace per stream."""
+    return ops.kernel_timer is None and a.is_cuda and gemm_algo != ops.GEMM_ALGO_SHARED_K
+
+
 def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
     """Forward of lingua/float8.py:85-96 on 2-D bf16 operands.  Returns ``(out, amax_b_t, a_col_amax | None)``:
     the two extra tensors are what backward needs beyond ``a`` and ``b_t``."""
@@ -335,6 +343,19 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
     # column amaxes of `a` fall out of the row-wise pass; wgrad wants them
     _bwd_cast.clear(a)
     hit = _fwd_cast.get(a, b_t.data_ptr()) if config.share_input_casts else None
+    if _native_call(a, gemm_algo):
+        ready = hit is not None and (hit[2] is not None or not need_wgrad_stats)
+        w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else (None, None, None)
+        res = _lib.native_for(a.get_device()).linear_fwd(
+            a, b_t, bias, *(hit[:2] if ready else (None, None)), ready, config.share_input_casts,
+            need_wgrad_stats and not ready, *w_cast[:2], w_cast[2] is None, gemm_algo)
+        if res is not None:
+            out, qa, sa, a_col_amax, amax_b_t = res
+            if ready:
+                a_col_amax = hit[2] if need_wgrad_stats else None
+            elif config.share_input_casts:
+                _fwd_cast.put(a, (qa, sa, a_col_amax), b_t.data_ptr())
+            return out, (amax_b_t if w_cast[2] is None else w_cast[2]), a_col_amax
     if hit is not None and (hit[2] is not None or not need_wgrad_stats):
         qa, sa, a_col_amax = hit
         if not need_wgrad_stats:
@@ -354,9 +375,39 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
 _UNSHARED_TOKENS = 64
 
 
+def _infer_native(a, b_t, bias):
+    """``linear_infer`` through the host extension, or None where its operands are not the plain ones."""
+    if a.dim() < 2 or b_t.dtype != torch.bfloat16 or not b_t.is_cuda:
+        return None
+    native = _lib.native_for(a.get_device())
+    if _bwd_cast.entries:
+        _bwd_cast.clear(a)
+    hit, rows, share = None, a, False
+    if config.share_input_casts:
+        few = a.numel() <= _UNSHARED_TOKENS * a.shape[-1]
+        if _fwd_cast.entries or not few:
+            rows = a if a.dim() == 2 else a.flatten(end_dim=-2)
+            hit = _fwd_cast.get(rows, b_t.data_ptr())
+            if hit is None and few:   # nothing of its own to file, but an earlier activation (a prompt's) is not kept alive
+                _fwd_cast.clear(rows)
+            share = hit is None and not few
+    qx, sx = (None, None) if hit is None else hit[:2]
+    qw, sw, _ = weight_cast_rowwise(b_t) if config.cache_weight_casts else (None, None, None)
+    res = native.linear_fwd(a, b_t, bias, qx, sx, hit is not None, share, False, qw, sw, False, config.gemm_algo)
+    if res is None:
+        return None
+    if share:
+        _fwd_cast.put(rows, (res[1], res[2], None), b_t.data_ptr())
+    return res[0]
+
+
 def linear_infer(a, b_t, bias):
     """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
     both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same results as ``linear_forward``."""
+    if _native_call(a, config.gemm_algo):
+        out = _infer_native(a, b_t, bias)
+        if out is not None:
+            return out
     if (ops.kernel_timer is not None and ops.timed_singly("cast_rowwise", "gemm_nt")) or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
         return linear_forward(a.flatten(end_dim=-2), b_t, bias, False, config.gemm_algo)[0].unflatten(0, a.shape[:-1])
     shape = a.shape
@@ -387,7 +438,9 @@ def input_cast_for_wgrad(a, a_col_amax, user):
     hit = _fwd_tcast.get(a, user) if config.share_input_casts else None
     if hit is not None:
         return hit
-    value = ops.cast_colwise_transposed(a, a_col_amax)
+    value = _lib.native_for(a.get_device()).cast_colwise_transposed(a, a_col_amax) if _native_call(a, 0) else None
+    if value is None:
+        value = ops.cast_colwise_transposed(a, a_col_amax)
     if config.share_input_casts:
         _fwd_tcast.put(a, value, user)
     return value
@@ -407,6 +460,22 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
     _fwd_tcast.clear(grad_out)
     if a is None and need_b and not (fp8_wgrad and a_tcast is not None):
         raise RuntimeError("Fp8LinearFn.backward: the bf16 input was not saved and no quantised copy stands in for it")
+
+    if (grad_a is None and wgrad_later is None and fp8_wgrad == need_b and _native_call(grad_out, gemm_algo) and
+            not torch.is_grad_enabled()):
+        hit = w_cast = None
+        if need_b and a_tcast is None and config.share_input_casts:
+            hit = _bwd_cast.get(a, b_t.data_ptr())
+        if need_a and config.cache_weight_casts:
+            w_cast = weight_cast_tensorwise_t(b_t, amax_b_t)
+        qat, sat = a_tcast or hit or (None, None)
+        res = _lib.native_for(grad_out.get_device()).linear_bwd(
+            grad_out, a if qat is None else None, b_t, amax_b_t, a_col_amax if qat is None else None, qat, sat, *(w_cast or (None, None)),
+            need_a, need_b, need_bias, gemm_algo)
+        if res is not None:
+            if need_b and qat is None and config.share_input_casts:
+                _bwd_cast.put(a, res[3:], b_t.data_ptr())
+            return res[:3]
 
     g_col_amax = None
     if need_a:
@@ -500,6 +569,8 @@ class Fp8Linear(torch.nn.Linear):
             out = fp8_linear(input.flatten(end_dim=-2), weight, bias)
         elif (torch.is_grad_enabled() and (input.requires_grad or weight.requires_grad or (bias is not None and bias.requires_grad))
               or not _plain_call()):
+            if input.dim() == 2:
+                return Fp8LinearFn.apply(input, weight, bias)
             out = Fp8LinearFn.apply(input.flatten(end_dim=-2), weight, bias)
         else:
             return linear_infer(input, weight, bias)
