@@ -330,6 +330,10 @@ typedef struct {
 } l8_linear_fwd_args;
 int64_t l8_linear_fwd_workspace(const l8_linear_fwd_args *args);
 int l8_linear_fwd(const l8_linear_fwd_args *args);
+/* The same with qx and qw (where they are not NULL) of row strides ldqx and ldqw, multiples of 16 and >= K, instead of
+ * dense.  Rows that start on 128-byte lines are what the products read fastest. */
+int64_t l8_linear_fwd_rows_workspace(const l8_linear_fwd_args *args, int64_t ldqx, int64_t ldqw);
+int l8_linear_fwd_rows(const l8_linear_fwd_args *args, int64_t ldqx, int64_t ldqw);
 
 #ifdef __cplusplus
 }

@@ -54,13 +54,15 @@ SIGNATURES = {
     "l8_rmsnorm_bwd_workspace": [_i64, _i64],
     "l8_linear_fwd": [ctypes.c_char_p],
     "l8_linear_fwd_workspace": [ctypes.c_char_p],
+    "l8_linear_fwd_rows": [ctypes.c_char_p, _i64, _i64],
+    "l8_linear_fwd_rows_workspace": [ctypes.c_char_p, _i64, _i64],
     "l8_gemm_algo_count": [],
     "l8_gemm_algo_name": [_int],
     "l8_gemm_pick": [_i64, _i64, _i64],
 }
 _RETURNS_STR = {"l8_last_error", "l8_gemm_algo_name"}
 _RETURNS_I64 = {"l8_cast_rowwise_workspace", "l8_gemm_workspace", "l8_gemm_workspace_gave_up_offset", "l8_swiglu_workspace", "l8_rmsnorm_workspace", "l8_rmsnorm_bwd_workspace",
-                "l8_linear_fwd_workspace"}
+                "l8_linear_fwd_workspace", "l8_linear_fwd_rows_workspace"}
 
 _lib = None
 _native = None    # the host extension, bound to the library's entries

@@ -26,7 +26,7 @@ using at::Tensor;
 struct Library {
 #define L8_ENTRY(name) decltype(&::name) name = nullptr;
 #define L8_ENTRIES(X)                                                                                                        \
-  X(l8_last_error) X(l8_linear_fwd) X(l8_linear_fwd_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
+  X(l8_last_error) X(l8_linear_fwd_rows) X(l8_linear_fwd_rows_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
   X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_col_amax) X(l8_gemm_nt)
   L8_ENTRIES(L8_ENTRY)
 #undef L8_ENTRY
@@ -68,6 +68,18 @@ bool dense(const Tensor &t, at::ScalarType type, int64_t n, int device) {
   return t.defined() && t.scalar_type() == type && t.layout() == at::kStrided && t.is_cuda() && t.get_device() == device && t.numel() == n && t.is_contiguous();
 }
 
+// A quantised operand handed in: rows x cols bytes, rows any stride apart (0: not one).
+int64_t fp8_rows(const Tensor &t, int64_t rows, int64_t cols, int device) {
+  if (!t.defined() || t.scalar_type() != at::kFloat8_e4m3fn || t.layout() != at::kStrided || !t.is_cuda() || t.get_device() != device ||
+      t.dim() != 2 || t.size(0) != rows || t.size(1) != cols || t.stride(1) != 1 || (rows > 1 && t.stride(0) < cols))
+    return 0;
+  return rows > 1 ? t.stride(0) : cols;
+}
+// A new one, its rows on 128-byte lines (figures in linear.cpp).
+Tensor empty_fp8(int64_t rows, int64_t cols, const at::TensorOptions &o) {
+  return at::empty_strided({rows, cols}, {(cols + 127) / 128 * 128, 1}, o.dtype(at::kFloat8_e4m3fn));
+}
+
 Tensor arg(PyObject *o) { return o == Py_None ? Tensor() : THPVariable_Unpack(o); }
 PyObject *wrap(const Tensor &t) {
   if (!t.defined()) Py_RETURN_NONE;
@@ -95,10 +107,8 @@ struct Space {
   void *p() const { return t.defined() ? t.mutable_data_ptr() : nullptr; }
 };
 
-constexpr at::ScalarType kFp8 = at::kFloat8_e4m3fn;
-
 // linear_fwd(x, w, bias, qx, sx, x_ready, want_qx, want_col, qw, sw, want_amax, algo) -> (y, qx, sx, col amax, w's row amax) or None.
-// The casts and the product of l8_linear_fwd.  qx / sx: x already quantised (x_ready); want_qx: hand the quantised x out.
+// The casts and the product of l8_linear_fwd_rows.  qx / sx: x already quantised (x_ready); want_qx: hand the quantised x out.
 PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 12) throw std::runtime_error("linear_fwd: 12 arguments");
@@ -114,8 +124,9 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       c10::hip::current_device() != device)
     Py_RETURN_NONE;
   const int64_t M = rx.rows, N = rw.rows, K = rx.cols;
-  if ((bias.defined() && !dense(bias, at::kBFloat16, N, device)) || (x_ready && !(dense(qx_in, kFp8, M * K, device) && dense(sx_in, at::kFloat, M, device))) ||
-      (qw.defined() && !(dense(qw, kFp8, N * K, device) && dense(sw, at::kFloat, N, device))))
+  int64_t ldqx = x_ready ? fp8_rows(qx_in, M, K, device) : K, ldqw = qw.defined() ? fp8_rows(qw, N, K, device) : K;
+  if ((bias.defined() && !dense(bias, at::kBFloat16, N, device)) || !ldqx || !ldqw || (x_ready && !dense(sx_in, at::kFloat, M, device)) ||
+      (qw.defined() && !dense(sw, at::kFloat, N, device)))
     Py_RETURN_NONE;
   Tensor y, qx, sx, col, amax;
   {
@@ -131,7 +142,8 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     qx = qx_in;
     sx = sx_in;
     if (!x_ready && want_qx) {
-      qx = at::empty({M, K}, o.dtype(kFp8));
+      qx = empty_fp8(M, K, o);
+      ldqx = qx.stride(0);
       sx = at::empty({M, 1}, o.dtype(at::kFloat));
     }
     if (want_col) col = at::empty({K}, o.dtype(at::kFloat));
@@ -147,10 +159,10 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (amax.defined()) a.amax_w = amax.mutable_data_ptr();
     a.algo = algo;
     a.stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-    const int64_t need = lib.l8_linear_fwd_workspace(&a);
+    const int64_t need = lib.l8_linear_fwd_rows_workspace(&a, ldqx, ldqw);
     const Space ws(x, need);  // a negative size is an error that the call below reports
     a.workspace = ws.p(), a.workspace_bytes = need > 0 ? need : 0;
-    check(lib.l8_linear_fwd(&a), "l8_linear_fwd");
+    check(lib.l8_linear_fwd_rows(&a, ldqx, ldqw), "l8_linear_fwd");
   }
   return tuple_of({y, qx, sx, col, amax});
   END_HANDLE_TH_ERRORS
@@ -160,9 +172,9 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
 void cast_colwise_t(const Tensor &like, const Rows &m, const Tensor &col, Tensor &q, Tensor &s, void *stream) {
   const auto o = like.options();
   const int64_t padded = (m.rows + 15) / 16 * 16;
-  q = at::empty({m.cols, padded}, o.dtype(kFp8));
+  q = empty_fp8(m.cols, padded, o);
   s = at::empty({m.cols, 1}, o.dtype(at::kFloat));
-  check(lib.l8_cast_colwise_transposed_pad(m.p, m.rows, m.cols, m.ld, col.const_data_ptr<float>(), q.mutable_data_ptr(), padded, padded,
+  check(lib.l8_cast_colwise_transposed_pad(m.p, m.rows, m.cols, m.ld, col.const_data_ptr<float>(), q.mutable_data_ptr(), q.stride(0), padded,
                                            s.mutable_data_ptr<float>(), stream), "l8_cast_colwise_transposed_pad");
 }
 
@@ -184,8 +196,8 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   const int64_t M = rg.rows, N = rg.cols, K = rw.cols, padded = (M + 15) / 16 * 16;
   if (rw.rows != N || N % 16 || K % 16 || !dense(amax, at::kBFloat16, N, device)) Py_RETURN_NONE;
   if (need_b && !qat_in.defined() && !(a.defined() && a.dim() == 2 && as_rows(a, device, ra) && ra.rows == M && ra.cols == K)) Py_RETURN_NONE;
-  if ((qat_in.defined() && !(dense(qat_in, kFp8, K * padded, device) && dense(sat_in, at::kFloat, K, device))) ||
-      (qwt_in.defined() && !(dense(qwt_in, kFp8, K * N, device) && dense(swt_in, at::kFloat, 1, device))) ||
+  if ((qat_in.defined() && !(fp8_rows(qat_in, K, padded, device) && dense(sat_in, at::kFloat, K, device))) ||
+      (qwt_in.defined() && !(fp8_rows(qwt_in, K, N, device) && dense(swt_in, at::kFloat, 1, device))) ||
       (a_col_in.defined() && !dense(a_col_in, at::kFloat, K, device)))
     Py_RETURN_NONE;
   Tensor ga, gb, gbias, qat = qat_in, sat = sat_in, qwt = qwt_in, swt = swt_in;
@@ -196,26 +208,26 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Tensor g_col;
     if (need_b) g_col = at::empty({N}, o.dtype(at::kFloat));
     if (need_a) {
-      Tensor qg = at::empty({M, N}, o.dtype(kFp8)), sg = at::empty({M, 1}, o.dtype(at::kFloat));
+      Tensor qg = empty_fp8(M, N, o), sg = at::empty({M, 1}, o.dtype(at::kFloat));
       const int64_t ws_bytes = need_b ? lib.l8_cast_rowwise_workspace(M, N) : 0;
       const Space ws(g, ws_bytes);
-      check(lib.l8_cast_rowwise(rg.p, M, N, rg.ld, qg.mutable_data_ptr(), N, sg.mutable_data_ptr<float>(), nullptr,
+      check(lib.l8_cast_rowwise(rg.p, M, N, rg.ld, qg.mutable_data_ptr(), qg.stride(0), sg.mutable_data_ptr<float>(), nullptr,
                                 need_b ? g_col.mutable_data_ptr<float>() : nullptr, ws.p(), ws_bytes, stream), "l8_cast_rowwise");
       if (!qwt.defined()) {
-        qwt = at::empty({K, N}, o.dtype(kFp8));
+        qwt = empty_fp8(K, N, o);
         swt = at::empty({1, 1}, o.dtype(at::kFloat));
         if (N % 8 == 0 && N <= 16384 && (reinterpret_cast<uintptr_t>(amax.const_data_ptr()) % 16) == 0) {
-          check(lib.l8_cast_tensorwise_t_rows(rw.p, N, K, rw.ld, amax.const_data_ptr(), N, qwt.mutable_data_ptr(), N, swt.mutable_data_ptr<float>(), stream),
+          check(lib.l8_cast_tensorwise_t_rows(rw.p, N, K, rw.ld, amax.const_data_ptr(), N, qwt.mutable_data_ptr(), qwt.stride(0), swt.mutable_data_ptr<float>(), stream),
                 "l8_cast_tensorwise_t_rows");
         } else {
           Tensor whole = at::empty({1, 1}, o);
           check(lib.l8_amax_reduce(amax.const_data_ptr(), N, whole.mutable_data_ptr(), stream), "l8_amax_reduce");
-          check(lib.l8_cast_tensorwise(rw.p, N, K, rw.ld, whole.const_data_ptr(), L8_AMAX_BF16, 1, qwt.mutable_data_ptr(), N, swt.mutable_data_ptr<float>(), stream),
+          check(lib.l8_cast_tensorwise(rw.p, N, K, rw.ld, whole.const_data_ptr(), L8_AMAX_BF16, 1, qwt.mutable_data_ptr(), qwt.stride(0), swt.mutable_data_ptr<float>(), stream),
                 "l8_cast_tensorwise");
         }
       }
       ga = at::empty({M, K}, o);
-      check(lib.l8_gemm_nt(qg.const_data_ptr(), qwt.const_data_ptr(), M, K, N, N, N, sg.const_data_ptr<float>(), L8_SCALE_ROW, swt.const_data_ptr<float>(),
+      check(lib.l8_gemm_nt(qg.const_data_ptr(), qwt.const_data_ptr(), M, K, N, qg.stride(0), qwt.stride(0), sg.const_data_ptr<float>(), L8_SCALE_ROW, swt.const_data_ptr<float>(),
                            L8_SCALE_SCALAR, nullptr, ga.mutable_data_ptr(), K, algo, stream), "l8_gemm_nt");
     } else if (need_b) {
       check(lib.l8_col_amax(rg.p, M, N, rg.ld, g_col.mutable_data_ptr<float>(), stream), "l8_col_amax");
@@ -232,7 +244,7 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
         cast_colwise_t(g, ra, a_col, qat, sat, stream);
       }
       gb = at::empty({N, K}, o);
-      check(lib.l8_gemm_nt(qgt.const_data_ptr(), qat.const_data_ptr(), N, K, padded, padded, padded, sgt.const_data_ptr<float>(), L8_SCALE_ROW,
+      check(lib.l8_gemm_nt(qgt.const_data_ptr(), qat.const_data_ptr(), N, K, padded, qgt.stride(0), qat.stride(0), sgt.const_data_ptr<float>(), L8_SCALE_ROW,
                            sat.const_data_ptr<float>(), L8_SCALE_ROW, nullptr, gb.mutable_data_ptr(), K, algo, stream), "l8_gemm_nt");
     }
     if (need_bias) gbias = at::sum(g, {0});

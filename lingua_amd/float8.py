@@ -104,8 +104,13 @@ def scale(t: torch.Tensor, amax_t: Optional[torch.Tensor] = None):
     for the fused kernel that finds the row amax in the same pass; only the
     sub-row-wise case always recomputes the group amaxes there.
     """
+    return _scale(t, amax_t, False)
+
+
+def _scale(t, amax_t, on_lines):
+    """``scale``; with ``on_lines`` for a product here: the copy's rows need not be dense."""
     if amax_t is None:
-        q, s, _ = ops.cast_rowwise(t)
+        q, s, _ = ops.cast_rowwise(t, on_lines=on_lines)
         return q, s
     g = _col_groups(t, amax_t)
     if g > 1:
@@ -118,8 +123,8 @@ def scale(t: torch.Tensor, amax_t: Optional[torch.Tensor] = None):
             ops.cast_rowwise(t[:, j * cs:(j + 1) * cs], out_q=q[:, j * cs:(j + 1) * cs], out_scale=s[:, j:j + 1])
         return q, s
     if amax_t.shape[0] == t.shape[0] and t.shape[0] != 1:
-        return ops.cast_rowwise_given_amax(t, amax_t)
-    return ops.cast_tensorwise(t, amax_t, transpose=False)
+        return ops.cast_rowwise_given_amax(t, amax_t, on_lines)
+    return ops.cast_tensorwise(t, amax_t, transpose=False, on_lines=on_lines)
 
 
 def matmul(first, amax_first, second_t, amax_second_t, bias, use_fast_accum: bool = True):
@@ -136,8 +141,8 @@ def matmul(first, amax_first, second_t, amax_second_t, bias, use_fast_accum: boo
     leaves the order of that sum to the all-reduce.
     """
     del use_fast_accum
-    q1, s1 = scale(first, amax_first)
-    q2, s2 = scale(second_t, amax_second_t)
+    q1, s1 = _scale(first, amax_first, True)
+    q2, s2 = _scale(second_t, amax_second_t, True)
     g1 = s1.shape[1] if s1.dim() == 2 else 1
     g2 = s2.shape[1] if s2.dim() == 2 else 1
     if g1 == 1 and g2 == 1:
@@ -252,7 +257,7 @@ class _WeightCasts:
         slot = self._slot(w) if config.cache_weight_casts else None
         if slot is not None and "row" in slot:
             return slot["row"]
-        value = ops.cast_rowwise(w)
+        value = ops.cast_rowwise(w, on_lines=True)
         if slot is not None:
             slot["row"] = value
         return value
@@ -261,7 +266,7 @@ class _WeightCasts:
         slot = self._slot(w) if config.cache_weight_casts else None
         if slot is not None and "tw" in slot:
             return slot["tw"]
-        value = ops.cast_tensorwise_t_rows(w, amax_rows)
+        value = ops.cast_tensorwise_t_rows(w, amax_rows, on_lines=True)
         if slot is not None:
             slot["tw"] = value
         return value
@@ -282,7 +287,7 @@ def weight_casts_rowwise(ws):
     """``weight_cast_rowwise`` of weights of one width that are quantised together."""
     if config.cache_weight_casts:
         return [_weight_casts.rowwise(w) for w in ws]
-    return ops.cast_rowwise_many(ws)
+    return ops.cast_rowwise_many(ws, on_lines=True)
 
 
 def weight_cast_tensorwise_t(w, amax_rows):
@@ -362,7 +367,7 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
             a_col_amax = None
     else:
         a_col_amax = torch.empty(a.shape[1], dtype=torch.float32, device=a.device) if need_wgrad_stats else None
-        qa, sa, _ = ops.cast_rowwise(a, col_amax=a_col_amax)
+        qa, sa, _ = ops.cast_rowwise(a, col_amax=a_col_amax, on_lines=True)
         if config.share_input_casts:
             _fwd_cast.put(a, (qa, sa, a_col_amax), b_t.data_ptr())
     qb, sb, amax_b_t = weight_cast_rowwise(b_t)
@@ -422,7 +427,7 @@ def linear_infer(a, b_t, bias):
         x_cast = hit = _fwd_cast.get(a, b_t.data_ptr())
         if hit is None:
             if tokens > _UNSHARED_TOKENS:
-                x_cast = (a.new_empty(a.shape, dtype=torch.float8_e4m3fn), a.new_empty((tokens, 1), dtype=torch.float32))
+                x_cast = (ops._empty_fp8(*a.shape, a.device, True), a.new_empty((tokens, 1), dtype=torch.float32))
             elif _fwd_cast.entries:   # nothing of its own to file, but an earlier activation (a prompt's) is not kept alive
                 _fwd_cast.clear(a)
     w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
@@ -440,7 +445,7 @@ def input_cast_for_wgrad(a, a_col_amax, user):
         return hit
     value = _lib.native_for(a.get_device()).cast_colwise_transposed(a, a_col_amax) if _native_call(a, 0) else None
     if value is None:
-        value = ops.cast_colwise_transposed(a, a_col_amax)
+        value = ops.cast_colwise_transposed(a, a_col_amax, on_lines=True)
     if config.share_input_casts:
         _fwd_tcast.put(a, value, user)
     return value
@@ -482,7 +487,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
         # grad_out row-wise, weight tensor-wise from the row amaxes saved in
         # forward, quantised straight into the [K,N] layout dgrad multiplies with
         g_col_amax = torch.empty(grad_out.shape[1], dtype=torch.float32, device=grad_out.device) if fp8_wgrad else None
-        qg, sg, _ = ops.cast_rowwise(grad_out, col_amax=g_col_amax)
+        qg, sg, _ = ops.cast_rowwise(grad_out, col_amax=g_col_amax, on_lines=True)
         qb, sb = weight_cast_tensorwise_t(b_t, amax_b_t)
         grad_a = ops.gemm_nt(qg, qb, sg, sb, None, algo=gemm_algo, out=grad_a, add=grad_a is not None)
 
@@ -490,7 +495,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
         if fp8_wgrad:
             if g_col_amax is None:
                 g_col_amax = ops.col_amax(grad_out)
-            qgt, sgt = ops.cast_colwise_transposed(grad_out, g_col_amax)
+            qgt, sgt = ops.cast_colwise_transposed(grad_out, g_col_amax, on_lines=True)
             hit = _bwd_cast.get(a, b_t.data_ptr()) if config.share_input_casts and a_tcast is None else None
             if a_tcast is not None:
                 qat, sat = a_tcast
@@ -499,7 +504,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
             else:
                 if a_col_amax is None:
                     a_col_amax = ops.col_amax(a)
-                qat, sat = ops.cast_colwise_transposed(a, a_col_amax)
+                qat, sat = ops.cast_colwise_transposed(a, a_col_amax, on_lines=True)
                 if config.share_input_casts:
                     _bwd_cast.put(a, (qat, sat), b_t.data_ptr())
             if wgrad_later is not None:

@@ -88,23 +88,37 @@ def _rows_2d(t: torch.Tensor, dtype, what: str) -> torch.Tensor:
     return t
 
 
+def _rows_apart(t: torch.Tensor) -> bool:
+    """Is each row dense, whatever lies between two of them?"""
+    return t.stride(1) == 1 and (t.shape[0] <= 1 or t.stride(0) >= t.shape[1])
+
+
 def _ld(t: torch.Tensor) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], 1)
 
 
+def _empty_fp8(rows: int, cols: int, device, on_lines: bool) -> torch.Tensor:
+    """A quantised operand; ``on_lines``: with rows that start on 128-byte lines, which the products read up to 1.6 times as
+    fast where they are bound by the L2's requests (figures at fp8_row_stride in csrc/linear.cpp)."""
+    if not on_lines or cols % 128 == 0:
+        return torch.empty((rows, cols), dtype=torch.float8_e4m3fn, device=device)
+    return torch.empty_strided((rows, cols), ((cols + 127) // 128 * 128, 1), dtype=torch.float8_e4m3fn, device=device)
+
+
 def cast_rowwise(x: torch.Tensor, col_amax: Optional[torch.Tensor] = None, want_q: bool = True,
-                 out_q: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None):
+                 out_q: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None, on_lines: bool = False):
     """Row-wise amax -> scale -> e4m3fn.  Returns (q [R,C] fp8 | None, scale [R,1] fp32, amax [R,1] bf16).
 
     ``col_amax`` (fp32 [C]) receives the column amaxes of x (overwritten).
     ``out_q`` (fp8 [R,C], unit column stride, row stride a multiple of 8) and ``out_scale`` (fp32 [R,1], any
-    strides) receive the results in place of fresh tensors: a column slice of a wider matrix is the use."""
+    strides) receive the results in place of fresh tensors: a column slice of a wider matrix is the use.
+    ``on_lines``: a fresh q has its rows on 128-byte lines instead of dense."""
     x = _rows_2d(x, torch.bfloat16, "cast_rowwise")
     st = _prep(x, "cast_rowwise")
     R, C = x.shape
     q = None
     if want_q:
-        q = out_q if out_q is not None else torch.empty((R, C), dtype=torch.float8_e4m3fn, device=x.device)
+        q = out_q if out_q is not None else _empty_fp8(R, C, x.device, on_lines)
         if q.dtype != torch.float8_e4m3fn or tuple(q.shape) != (R, C) or q.device != x.device or (q.numel() and q.stride(1) != 1):
             raise RuntimeError("cast_rowwise: out_q must be an e4m3fn [R,C] tensor on x's device with unit column stride")
     if out_scale is not None and (out_scale.dtype != torch.float32 or tuple(out_scale.shape) != (R, 1) or out_scale.device != x.device):
@@ -134,10 +148,10 @@ def cast_rowwise(x: torch.Tensor, col_amax: Optional[torch.Tensor] = None, want_
     return q, scale, amax
 
 
-def cast_rowwise_many(xs, out=None):
+def cast_rowwise_many(xs, out=None, on_lines: bool = False):
     """``cast_rowwise`` of several tensors of one width, in one launch where the library can.  ``out``: (q [sum of rows, C]
-    fp8, scale [sum of rows, 1] fp32), dense, that receives the results one below the other.  Returns a list of (q, scale,
-    amax) per tensor."""
+    fp8 with unit column stride, scale [sum of rows, 1] fp32, dense) that receives the results one below the other.
+    ``on_lines`` as in ``cast_rowwise``.  Returns a list of (q, scale, amax) per tensor."""
     xs = [_rows_2d(x, torch.bfloat16, "cast_rowwise_many") for x in xs]
     dev, C = xs[0].device, xs[0].shape[1]
     st = _prep(xs[0], "cast_rowwise_many")
@@ -146,19 +160,19 @@ def cast_rowwise_many(xs, out=None):
         raise RuntimeError("cast_rowwise_many: tensors of one width on one device required")
     if out is not None:
         q_all, s_all = out
-        if (q_all.dtype != torch.float8_e4m3fn or tuple(q_all.shape) != (sum(rows), C) or not q_all.is_contiguous() or q_all.device != dev or
+        if (q_all.dtype != torch.float8_e4m3fn or tuple(q_all.shape) != (sum(rows), C) or (q_all.numel() and q_all.stride(1) != 1) or q_all.device != dev or
                 s_all.dtype != torch.float32 or tuple(s_all.shape) != (sum(rows), 1) or not s_all.is_contiguous() or s_all.device != dev):
-            raise RuntimeError("cast_rowwise_many: out must be dense e4m3fn [rows,C] and fp32 [rows,1] tensors on the inputs' device")
+            raise RuntimeError("cast_rowwise_many: out must be e4m3fn [rows,C] (unit column stride) and dense fp32 [rows,1] tensors on the inputs' device")
         qs, ss = q_all.split(rows), s_all.split(rows)
     else:
-        qs = [torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=dev) for x in xs]
+        qs = [_empty_fp8(n, C, dev, on_lines) for n in rows]
         ss = [torch.empty((n, 1), dtype=torch.float32, device=dev) for n in rows]
     if timed_singly("cast_rowwise"):
         return [cast_rowwise(x, out_q=q, out_scale=s) for x, q, s in zip(xs, qs, ss)]
     amaxes = [torch.empty((n, 1), dtype=torch.bfloat16, device=dev) for n in rows]
     items = []
     for x, q, s, a in zip(xs, qs, ss, amaxes):
-        items += [x.data_ptr(), x.shape[0], _ld(x), q.data_ptr(), C, s.data_ptr(), a.data_ptr()]
+        items += [x.data_ptr(), x.shape[0], _ld(x), q.data_ptr(), _ld(q), s.data_ptr(), a.data_ptr()]
     with _timed("cast_rowwise_many", sum(rows) * (3 * C + 4), dev):
         code = _lib.load().l8_cast_rowwise_many(struct.pack(f"{len(items)}q", *items), len(xs), C, st)
     _lib.check(code, "l8_cast_rowwise_many")
@@ -181,17 +195,17 @@ def _amax_arg(amax: torch.Tensor, n: int, device, what: str):
     return amax.contiguous(), (AMAX_F32 if amax.dtype == torch.float32 else AMAX_BF16)
 
 
-def cast_rowwise_given_amax(x: torch.Tensor, amax: torch.Tensor):
+def cast_rowwise_given_amax(x: torch.Tensor, amax: torch.Tensor, on_lines: bool = False):
     """scale(x, amax) of lingua/float8.py:43-47 with a row amax [R,1] (bf16 or fp32) the caller supplies and that is
     used as given.  Returns (q [R,C] fp8, scale [R,1] fp32)."""
     x = _rows_2d(x, torch.bfloat16, "cast_rowwise_given_amax")
     st = _prep(x, "cast_rowwise_given_amax")
     R, C = x.shape
     amax, amax_dtype = _amax_arg(amax, R, x.device, "cast_rowwise_given_amax")
-    q = torch.empty((R, C), dtype=torch.float8_e4m3fn, device=x.device)
+    q = _empty_fp8(R, C, x.device, on_lines)
     scale = torch.empty((R, 1), dtype=torch.float32, device=x.device)
     with _timed("cast_rowwise_given_amax", R * C * 3 + 6 * R, x.device):
-        code = _lib.load().l8_cast_rowwise_given_amax(x.data_ptr(), R, C, _ld(x), amax.data_ptr(), amax_dtype, q.data_ptr(), C,
+        code = _lib.load().l8_cast_rowwise_given_amax(x.data_ptr(), R, C, _ld(x), amax.data_ptr(), amax_dtype, q.data_ptr(), _ld(q),
                                                       scale.data_ptr(), st)
     _lib.check(code, "l8_cast_rowwise_given_amax")
     return q, scale
@@ -222,18 +236,18 @@ def amax_reduce(amax: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def cast_tensorwise(x: torch.Tensor, amax: torch.Tensor, transpose: bool = False):
+def cast_tensorwise(x: torch.Tensor, amax: torch.Tensor, transpose: bool = False, on_lines: bool = False):
     """Tensor-wise scale -> e4m3fn with a device-resident amax scalar (bf16 or fp32).
     Returns (q [R,C] or [C,R] fp8, scale [1,1] fp32)."""
     x = _rows_2d(x, torch.bfloat16, "cast_tensorwise")
     st = _prep(x, "cast_tensorwise")
     amax, amax_dtype = _amax_arg(amax, 1, x.device, "cast_tensorwise")
     R, C = x.shape
-    q = torch.empty((C, R) if transpose else (R, C), dtype=torch.float8_e4m3fn, device=x.device)
+    q = _empty_fp8(*((C, R) if transpose else (R, C)), x.device, on_lines)
     scale = torch.empty((1, 1), dtype=torch.float32, device=x.device)
     with _timed("cast_tensorwise_t" if transpose else "cast_tensorwise", R * C * 3 + 4, x.device):
         code = _lib.load().l8_cast_tensorwise(x.data_ptr(), R, C, _ld(x), amax.data_ptr(), amax_dtype, int(transpose),
-                                              q.data_ptr(), max(q.shape[1], 1), scale.data_ptr(), st)
+                                              q.data_ptr(), _ld(q), scale.data_ptr(), st)
     _lib.check(code, "l8_cast_tensorwise")
     return q, scale
 
@@ -242,25 +256,25 @@ def cast_tensorwise(x: torch.Tensor, amax: torch.Tensor, transpose: bool = False
 _MAX_AMAX_ROWS = 16384
 
 
-def cast_tensorwise_t_rows(x: torch.Tensor, amax_rows: torch.Tensor):
+def cast_tensorwise_t_rows(x: torch.Tensor, amax_rows: torch.Tensor, on_lines: bool = False):
     """``cast_tensorwise(x, amax_reduce(amax_rows), transpose=True)``, in one launch where the list allows it."""
     x = _rows_2d(x, torch.bfloat16, "cast_tensorwise_t_rows")
     n = amax_rows.numel()
     if (amax_rows.dtype != torch.bfloat16 or amax_rows.device != x.device or not amax_rows.is_contiguous() or n % 8 or
             not 0 < n <= _MAX_AMAX_ROWS or amax_rows.data_ptr() % 16):
-        return cast_tensorwise(x, amax_reduce(amax_rows), transpose=True)
+        return cast_tensorwise(x, amax_reduce(amax_rows), transpose=True, on_lines=on_lines)
     st = _prep(x, "cast_tensorwise_t_rows")
     R, C = x.shape
-    q = torch.empty((C, R), dtype=torch.float8_e4m3fn, device=x.device)
+    q = _empty_fp8(C, R, x.device, on_lines)
     scale = torch.empty((1, 1), dtype=torch.float32, device=x.device)
     with _timed("cast_tensorwise_t", R * C * 3 + 2 * n + 4, x.device):
-        code = _lib.load().l8_cast_tensorwise_t_rows(x.data_ptr(), R, C, _ld(x), amax_rows.data_ptr(), n, q.data_ptr(), max(R, 1),
+        code = _lib.load().l8_cast_tensorwise_t_rows(x.data_ptr(), R, C, _ld(x), amax_rows.data_ptr(), n, q.data_ptr(), _ld(q),
                                                      scale.data_ptr(), st)
     _lib.check(code, "l8_cast_tensorwise_t_rows")
     return q, scale
 
 
-def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to: int = 16):
+def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to: int = 16, on_lines: bool = False):
     """scale(x.t().contiguous(), its row amax): returns (q [C,Rp] fp8, scale [C,1] fp32).
 
     Rp is R rounded up to a multiple of ``pad_to``; the padding columns hold
@@ -277,11 +291,11 @@ def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to:
         q = torch.zeros((C, pad_to), dtype=torch.uint8, device=x.device).view(torch.float8_e4m3fn)
         return q, (torch.clamp(col_amax_f32, min=1e-12) / 448.0).reshape(C, 1)
     Rp = (R + pad_to - 1) // pad_to * pad_to
-    q = torch.empty((C, Rp), dtype=torch.float8_e4m3fn, device=x.device)
+    q = _empty_fp8(C, Rp, x.device, on_lines)
     scale = torch.empty((C, 1), dtype=torch.float32, device=x.device)
     with _timed("cast_colwise_t", R * C * 3 + 4 * C, x.device):
         code = _lib.load().l8_cast_colwise_transposed_pad(x.data_ptr(), R, C, _ld(x), col_amax_f32.data_ptr(),
-                                                          q.data_ptr(), max(Rp, 1), Rp, scale.data_ptr(), st)
+                                                          q.data_ptr(), _ld(q), Rp, scale.data_ptr(), st)
     _lib.check(code, "l8_cast_colwise_transposed_pad")
     return q, scale
 
@@ -374,12 +388,12 @@ def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tens
 
 def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
     """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch, on 256 x 256 tiles, where that fills the GPU
-    better (a product that alone is too small for those tiles may add up K in another order there).  Dense fp8 operands
-    with one scale per row."""
+    better (a product that alone is too small for those tiles may add up K in another order there).  fp8 operands of one
+    row stride with one scale per row."""
     N, K = qb.shape
-    one = algo == 0 and len(qas) > 1 and not timed_singly("gemm_nt") and qb.is_contiguous() and sb.dtype == torch.float32 and sb.numel() == N and sb.is_contiguous()
+    one = algo == 0 and len(qas) > 1 and not timed_singly("gemm_nt") and _rows_apart(qb) and sb.dtype == torch.float32 and sb.numel() == N and sb.is_contiguous()
     for qa, sa in zip(qas, sas):
-        one = (one and qa.dtype == qb.dtype == torch.float8_e4m3fn and qa.dim() == 2 and qa.shape[1] == K and qa.is_contiguous() and
+        one = (one and qa.dtype == qb.dtype == torch.float8_e4m3fn and qa.dim() == 2 and qa.shape[1] == K and _rows_apart(qa) and _ld(qa) == _ld(qas[0]) and
                qa.device == qb.device and sa.dtype == torch.float32 and sa.numel() == qa.shape[0] and sa.is_contiguous())
     if not one:
         return [gemm_nt(qa, qb, sa, sb, None, algo=algo) for qa, sa in zip(qas, sas)]
@@ -389,7 +403,7 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
     for qa, sa, out in zip(qas, sas, outs):
         parts += [qa.data_ptr(), qa.shape[0], sa.data_ptr(), out.data_ptr()]
     with _timed("gemm_nt_multi", 2 * sum(qa.shape[0] for qa in qas) * N * K, qb.device):
-        code = _lib.load().l8_gemm_nt_multi(struct.pack(f"{len(parts)}q", *parts), len(qas), qb.data_ptr(), N, K, K, K, sb.data_ptr(),
+        code = _lib.load().l8_gemm_nt_multi(struct.pack(f"{len(parts)}q", *parts), len(qas), qb.data_ptr(), N, K, _ld(qas[0]), _ld(qb), sb.data_ptr(),
                                             SCALE_ROW, N, algo, st)
     _lib.check(code, "l8_gemm_nt_multi")
     return outs
@@ -402,8 +416,8 @@ def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y
                col_amax: Optional[torch.Tensor] = None, w_cast=None, w_ready: bool = False, amax_w: Optional[torch.Tensor] = None,
                algo: int = 0) -> None:
     """y [M,N] (dense) = x @ w.T + bias with row-wise casts of both, in one call of the library: the same results as
-    ``cast_rowwise``, ``cast_rowwise``, ``gemm_nt``.  ``x_cast`` / ``w_cast`` = (q, scale), dense: where the quantised
-    operand goes (None: a temporary), or with ``x_ready`` / ``w_ready`` where it comes from."""
+    ``cast_rowwise``, ``cast_rowwise``, ``gemm_nt``.  ``x_cast`` / ``w_cast`` = (q, scale), q with any row stride: where the
+    quantised operand goes (None: a temporary), or with ``x_ready`` / ``w_ready`` where it comes from."""
     st = _prep(x, "linear_fwd")
     x, w = _rows_2d(x, torch.bfloat16, "linear_fwd(x)"), _rows_2d(w, torch.bfloat16, "linear_fwd(w)")
     M, K = x.shape
@@ -425,12 +439,15 @@ def linear_fwd(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], y
     if kernel_timer is not None or torch._C._cuda_getDevice() != x.device.index:   # else there is nothing to bracket
         bracket = _timed("linear_fwd", 2 * M * N * K, x.device)
         bracket.__enter__()
+    ldq = [_ld(c[0]) if c else K for c in (x_cast, w_cast)]
+    dense = ldq == [K, K]
     try:
-        need = lib.l8_linear_fwd_workspace(_FWD.pack(*members))   # depends on the device's compute units
+        # depends on the device's compute units
+        need = lib.l8_linear_fwd_workspace(_FWD.pack(*members)) if dense else lib.l8_linear_fwd_rows_workspace(_FWD.pack(*members), *ldq)
         if need > 0:
             ws = x.new_empty(need, dtype=torch.uint8)
             members[19], members[20] = ws.data_ptr(), need
-        code = lib.l8_linear_fwd(_FWD.pack(*members))
+        code = lib.l8_linear_fwd(_FWD.pack(*members)) if dense else lib.l8_linear_fwd_rows(_FWD.pack(*members), *ldq)
     finally:
         if bracket is not None:
             bracket.__exit__()
@@ -475,7 +492,8 @@ def _swiglu_ws(R: int, C: int, device, halves: int):
     return (torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None), ws_bytes
 
 
-def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True, col_amax: Optional[torch.Tensor] = None):
+def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True, col_amax: Optional[torch.Tensor] = None,
+                        on_lines: bool = False):
     """h = bf16(bf16(silu(h1)) * h3) and its row-wise cast in one pass.
     Returns (h [R,C] bf16 | None, q [R,C] fp8, scale [R,1] fp32, amax [R,1] bf16); ``col_amax`` as in cast_rowwise."""
     h1 = _rows_2d(h1, torch.bfloat16, "swiglu_cast_rowwise(h1)")
@@ -486,7 +504,7 @@ def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True,
     R, C = h1.shape
     dev = h1.device
     h = torch.empty((R, C), dtype=torch.bfloat16, device=dev) if want_h else None
-    q = torch.empty((R, C), dtype=torch.float8_e4m3fn, device=dev)
+    q = _empty_fp8(R, C, dev, on_lines)
     scale = torch.empty((R, 1), dtype=torch.float32, device=dev)
     amax = torch.empty((R, 1), dtype=torch.bfloat16, device=dev)
     if col_amax is not None and (col_amax.dtype != torch.float32 or col_amax.numel() != C or not col_amax.is_contiguous()):
@@ -494,7 +512,7 @@ def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True,
     ws, ws_bytes = _swiglu_ws(R, C, dev, 1) if col_amax is not None else (None, 0)
     with _timed("swiglu_cast_rowwise", R * C * (5 + (2 if want_h else 0)) + 4 * R, dev):
         code = _lib.load().l8_swiglu_cast_rowwise(
-            h1.data_ptr(), h3.data_ptr(), R, C, _ld(h1), _ld(h3), h.data_ptr() if want_h else None, C, q.data_ptr(), C,
+            h1.data_ptr(), h3.data_ptr(), R, C, _ld(h1), _ld(h3), h.data_ptr() if want_h else None, C, q.data_ptr(), _ld(q),
             scale.data_ptr(), amax.data_ptr(), col_amax.data_ptr() if col_amax is not None else None,
             ws.data_ptr() if ws is not None else None, ws_bytes, st)
     _lib.check(code, "l8_swiglu_cast_rowwise")
@@ -502,7 +520,8 @@ def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True,
 
 
 def swiglu_bwd_cast_rowwise(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor,
-                            col_amax1: Optional[torch.Tensor] = None, col_amax3: Optional[torch.Tensor] = None):
+                            col_amax1: Optional[torch.Tensor] = None, col_amax3: Optional[torch.Tensor] = None,
+                            on_lines: bool = False):
     """Gradients of the SwiGLU gate and their row-wise casts in one pass.
     Returns (g1, g3 [R,C] bf16, q1, q3 [R,C] fp8, scale1, scale3 [R,1] fp32)."""
     dh = _rows_2d(dh, torch.bfloat16, "swiglu_bwd_cast_rowwise(dh)")
@@ -520,15 +539,14 @@ def swiglu_bwd_cast_rowwise(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor
             raise RuntimeError("swiglu_bwd_cast_rowwise: column amaxes must be contiguous fp32 tensors with C elements")
     g1 = torch.empty((R, C), dtype=torch.bfloat16, device=dev)
     g3 = torch.empty((R, C), dtype=torch.bfloat16, device=dev)
-    q1 = torch.empty((R, C), dtype=torch.float8_e4m3fn, device=dev)
-    q3 = torch.empty((R, C), dtype=torch.float8_e4m3fn, device=dev)
+    q1, q3 = _empty_fp8(R, C, dev, on_lines), _empty_fp8(R, C, dev, on_lines)
     s1 = torch.empty((R, 1), dtype=torch.float32, device=dev)
     s3 = torch.empty((R, 1), dtype=torch.float32, device=dev)
     ws, ws_bytes = _swiglu_ws(R, C, dev, 2) if col_amax1 is not None else (None, 0)
     with _timed("swiglu_bwd_cast_rowwise", R * C * 12 + 8 * R, dev):
         code = _lib.load().l8_swiglu_bwd_cast_rowwise(
             dh.data_ptr(), h1.data_ptr(), h3.data_ptr(), R, C, _ld(dh), _ld(h1), _ld(h3), g1.data_ptr(), g3.data_ptr(), C,
-            q1.data_ptr(), q3.data_ptr(), C, s1.data_ptr(), s3.data_ptr(),
+            q1.data_ptr(), q3.data_ptr(), _ld(q1), s1.data_ptr(), s3.data_ptr(),
             col_amax1.data_ptr() if col_amax1 is not None else None, col_amax3.data_ptr() if col_amax3 is not None else None,
             ws.data_ptr() if ws is not None else None, ws_bytes, st)
     _lib.check(code, "l8_swiglu_bwd_cast_rowwise")
@@ -536,7 +554,7 @@ def swiglu_bwd_cast_rowwise(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor
 
 
 def rmsnorm_cast_rowwise(x: torch.Tensor, weight: torch.Tensor, eps: float, want_q: bool = True,
-                         col_amax: Optional[torch.Tensor] = None, want_rstd: bool = True):
+                         col_amax: Optional[torch.Tensor] = None, want_rstd: bool = True, on_lines: bool = False):
     """y = bf16((f32(x) * rsqrt(mean(x^2) + eps)) * f32(weight)) and its row-wise cast in one pass.
     Returns (y [R,C] bf16, q [R,C] fp8 | None, scale [R,1] fp32 | None, rstd [R,1] fp32 | None)."""
     x = _rows_2d(x, torch.bfloat16, "rmsnorm_cast_rowwise")
@@ -549,7 +567,7 @@ def rmsnorm_cast_rowwise(x: torch.Tensor, weight: torch.Tensor, eps: float, want
     if col_amax is not None and (not want_q or col_amax.dtype != torch.float32 or col_amax.numel() != C or not col_amax.is_contiguous()):
         raise RuntimeError("rmsnorm_cast_rowwise: col_amax needs the cast and must be a contiguous fp32 tensor with C elements")
     y = torch.empty((R, C), dtype=torch.bfloat16, device=dev)
-    q = torch.empty((R, C), dtype=torch.float8_e4m3fn, device=dev) if want_q else None
+    q = _empty_fp8(R, C, dev, on_lines) if want_q else None
     scale = torch.empty((R, 1), dtype=torch.float32, device=dev) if want_q else None
     rstd = torch.empty((R, 1), dtype=torch.float32, device=dev) if want_rstd else None
     ws, ws_bytes = None, 0
@@ -559,7 +577,7 @@ def rmsnorm_cast_rowwise(x: torch.Tensor, weight: torch.Tensor, eps: float, want
     with _timed("rmsnorm_cast_rowwise", R * C * (4 + (1 if want_q else 0)) + 8 * R, dev):
         code = _lib.load().l8_rmsnorm_cast_rowwise(
             x.data_ptr(), weight.data_ptr(), int(weight.dtype == torch.float32), R, C, _ld(x), float(eps), y.data_ptr(), C,
-            q.data_ptr() if want_q else None, C, scale.data_ptr() if want_q else None,
+            q.data_ptr() if want_q else None, _ld(q) if want_q else C, scale.data_ptr() if want_q else None,
             rstd.data_ptr() if want_rstd else None, col_amax.data_ptr() if col_amax is not None else None,
             ws.data_ptr() if ws is not None else None, ws_bytes, st)
     _lib.check(code, "l8_rmsnorm_cast_rowwise")

@@ -51,12 +51,12 @@ class Fp8QKVFn(torch.autograd.Function):
                 x_col = None
         else:
             x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_stats else None
-            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col)
+            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
             if cfg.share_input_casts:
                 f8._fwd_cast.put(x, (qx, sx, x_col), ("qkv", wq.data_ptr()))
         K = x.shape[1]
         sizes = [w.shape[0] for w in ws]
-        qw = torch.empty((sum(sizes), K), dtype=torch.float8_e4m3fn, device=x.device)
+        qw = ops._empty_fp8(sum(sizes), K, x.device, True)
         sw = torch.empty((sum(sizes), 1), dtype=torch.float32, device=x.device)
         amaxes = [amax for _, _, amax in ops.cast_rowwise_many(ws, out=(qw, sw))]
         y = ops.gemm_nt(qx, qw, sx, sw, None, algo=cfg.gemm_algo)

@@ -47,13 +47,13 @@ class Fp8SwiGLUFn(torch.autograd.Function):
                 x_col = None
         else:
             x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_x_col else None
-            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col)
+            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
         (q1, s1, amax_w1), (q3, s3, amax_w3) = f8.weight_casts_rowwise((w1, w3))
         h1 = ops.gemm_nt(qx, q1, sx, s1, None, algo=algo)
         h3 = ops.gemm_nt(qx, q3, sx, s3, None, algo=algo)
         del qx, q1, q3
         h_col = torch.empty(w2.shape[1], dtype=torch.float32, device=x.device) if fp8_wgrad and w2.requires_grad else None
-        h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=w2.requires_grad, col_amax=h_col)
+        h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=w2.requires_grad, col_amax=h_col, on_lines=True)
         q2, s2, amax_w2 = f8.weight_cast_rowwise(w2)
         y = ops.gemm_nt(qh, q2, sh, s2, None, algo=algo)
 
@@ -88,7 +88,7 @@ class Fp8SwiGLUFn(torch.autograd.Function):
             return gx, gw1, gw3, gw2
 
         gy_col = torch.empty(D, dtype=torch.float32, device=dev) if fp8_wgrad and need_w2 else None
-        qgy, sgy, _ = ops.cast_rowwise(gy, col_amax=gy_col)
+        qgy, sgy, _ = ops.cast_rowwise(gy, col_amax=gy_col, on_lines=True)
         qw2t, sw2t = f8.weight_cast_tensorwise_t(w2, amax_w2)
         dh = ops.gemm_nt(qgy, qw2t, sgy, sw2t, None, algo=algo)
         del qgy, qw2t
@@ -98,7 +98,7 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         want_cols = fp8_wgrad and (need_w1 or need_w3)
         g1_col = torch.empty(F, dtype=torch.float32, device=dev) if want_cols else None
         g3_col = torch.empty(F, dtype=torch.float32, device=dev) if want_cols else None
-        g1, g3, qg1, qg3, sg1, sg3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, g1_col, g3_col)
+        g1, g3, qg1, qg3, sg1, sg3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, g1_col, g3_col, on_lines=True)
         del dh
         if need_x:
             qw1t, sw1t = f8.weight_cast_tensorwise_t(w1, amax_w1)
@@ -110,17 +110,17 @@ class Fp8SwiGLUFn(torch.autograd.Function):
             if fp8_wgrad:
                 if x_col is None:
                     x_col = ops.col_amax(x)
-                qxt, sxt = ops.cast_colwise_transposed(x, x_col)   # shared by both wgrads
+                qxt, sxt = ops.cast_colwise_transposed(x, x_col, on_lines=True)   # shared by both wgrads
                 if need_w1 and need_w3:
-                    q1, s1 = ops.cast_colwise_transposed(g1, g1_col)
+                    q1, s1 = ops.cast_colwise_transposed(g1, g1_col, on_lines=True)
                     del g1
-                    q3, s3 = ops.cast_colwise_transposed(g3, g3_col)
+                    q3, s3 = ops.cast_colwise_transposed(g3, g3_col, on_lines=True)
                     gw1, gw3 = ops.gemm_nt_multi((q1, q3), qxt, (s1, s3), sxt, algo=algo)
                 elif need_w1:
-                    qgt, sgt = ops.cast_colwise_transposed(g1, g1_col)
+                    qgt, sgt = ops.cast_colwise_transposed(g1, g1_col, on_lines=True)
                     gw1 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
                 else:
-                    qgt, sgt = ops.cast_colwise_transposed(g3, g3_col)
+                    qgt, sgt = ops.cast_colwise_transposed(g3, g3_col, on_lines=True)
                     gw3 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
             else:
                 gw1 = g1.t() @ x if need_w1 else None
@@ -136,8 +136,8 @@ def _wgrad(g, g_col, a, a_col, fp8_wgrad, algo):
         g_col = ops.col_amax(g)
     if a_col is None:
         a_col = ops.col_amax(a)
-    qgt, sgt = ops.cast_colwise_transposed(g, g_col)
-    qat, sat = ops.cast_colwise_transposed(a, a_col)
+    qgt, sgt = ops.cast_colwise_transposed(g, g_col, on_lines=True)
+    qat, sat = ops.cast_colwise_transposed(a, a_col, on_lines=True)
     return ops.gemm_nt(qgt, qat, sgt, sat, None, algo=algo)
 
 

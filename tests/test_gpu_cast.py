@@ -473,3 +473,39 @@ def test_several_operands_in_one_launch(C, rows):
             assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8))
             assert torch.equal(s.view(torch.int32), ws.view(torch.int32)) and torch.equal(a.view(torch.int16), wa.view(torch.int16))
     assert torch.equal(out[0].view(torch.uint8), torch.cat([w[0].view(torch.uint8) for w in want]))
+
+
+@pytest.mark.parametrize("R,C", [(33, 144), (1, 16), (130, 1040), (48, 256), (257, 4112)])
+def test_rows_on_lines_hold_what_dense_rows_hold(R, C):
+    """on_lines moves the rows of a quantised operand to 128-byte lines, nothing else: every cast's bytes and scales, and the
+    products that read them (one, several in one launch, a linear's forward in one call)."""
+    from lingua_amd import ops
+    x, w, h = (seeded_bf16((n, C), seed=n + C).cuda() for n in (R, 48, R))
+    amax, col = ops.cast_rowwise(x)[2], ops.col_amax(x)
+    wmax = ops.cast_rowwise(w)[2]
+    norm_w = torch.rand(C, device="cuda").to(torch.bfloat16)
+
+    def bits(t):
+        return t.contiguous().view({1: torch.uint8, 2: torch.int16, 4: torch.int32}[t.element_size()])
+
+    calls = [lambda on: ops.cast_rowwise(x, on_lines=on), lambda on: ops.cast_rowwise_given_amax(x, amax, on_lines=on),
+             lambda on: ops.cast_tensorwise(x, amax[:1], on_lines=on), lambda on: ops.cast_tensorwise(x, amax[:1], transpose=True, on_lines=on),
+             lambda on: ops.cast_tensorwise_t_rows(w, wmax, on_lines=on), lambda on: ops.cast_colwise_transposed(x, col, on_lines=on),
+             lambda on: [t for trio in ops.cast_rowwise_many((x, w), on_lines=on) for t in trio],
+             lambda on: ops.swiglu_cast_rowwise(x, h, on_lines=on), lambda on: ops.swiglu_bwd_cast_rowwise(x, x, h, on_lines=on),
+             lambda on: ops.rmsnorm_cast_rowwise(x, norm_w, 1e-5, on_lines=on) if C <= 8192 else ()]
+    for i, call in enumerate(calls):
+        for a, b in zip(call(False), call(True)):
+            assert a.shape == b.shape and torch.equal(bits(a), bits(b)), i
+            if b.dtype == torch.float8_e4m3fn and b.shape[0] > 1:
+                assert b.stride(0) % 128 == 0 and b.data_ptr() % 128 == 0 or i == 2
+    (q, s, _), (qw, sw, _) = ops.cast_rowwise(x), ops.cast_rowwise(w)
+    (ql, _, _), (qwl, _, _) = ops.cast_rowwise(x, on_lines=True), ops.cast_rowwise(w, on_lines=True)
+    want = ops.gemm_nt(q, qw, s, sw)
+    assert torch.equal(bits(ops.gemm_nt(ql, qwl, s, sw)), bits(want))
+    for a, b in zip(ops.gemm_nt_multi((q, q), qw, (s, s), sw), ops.gemm_nt_multi((ql, ql), qwl, (s, s), sw)):
+        assert torch.equal(bits(a), bits(b))
+    for x_cast, w_cast in (((ql, s), (qwl, sw)), ((ql, s), (qw, sw)), ((q, s), (qwl, sw))):
+        y = torch.empty_like(want)
+        ops.linear_fwd(x, w, None, y, x_cast=x_cast, x_ready=True, w_cast=w_cast, w_ready=True)
+        assert torch.equal(bits(y), bits(want))
