@@ -126,6 +126,10 @@ L8_DEV void store16_aux(v4i data, __amdgpu_buffer_rsrc_t rs, uint32_t voff, int 
 #ifndef L8_READ_GROUPS2
 #define L8_READ_GROUPS2 30
 #endif
+// ... and the number of a half tile's 32 MFMAs in front of the barrier of a trip
+#ifndef L8_HALF_TILE_BARRIER
+#define L8_HALF_TILE_BARRIER 10
+#endif
 // L8_GEMM_PROF (compile-time, never set in the shipped build): the persistent kernel takes the `bias` pointer for
 // a buffer of 16 x uint64 per workgroup and records wall-clock ticks (100 MHz) at its start, after the prologue
 // and at its end, and shader-clock cycles spent in the K loops and in the C-tile stores.
@@ -628,6 +632,14 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // loop's layout from 2260 to 2380 cycles took the same time, one of 3500 cycles
 // 20 % more.  Without the panel loads it runs at 2.2 GHz: they are the largest
 // consumer beside the matrix cores.
+//
+// BM x BN = 256 x 128 and 128 x 256 are half tiles for problems that whole ones
+// would spread over few units or an unlucky number of rounds.  A trip is 32
+// instructions per wave and wants 48 KiB through the L2 where a whole tile's 64
+// instructions want 64: it takes 1270 to 1360 cycles of the 1024 of its
+// instructions, 1075 without the panel loads.  The ring holds three whole K tiles,
+// and the barrier stands after the tenth instruction so that the 24 LDS reads of
+// a trip spread evenly (after the sixteenth: 1300 to 1385 cycles).
 // Work split: the tiles are dealt to the 8 XCDs in contiguous ranges of the
 // grouped order (as in the kernel above); inside an XCD, workgroup `loc`
 // takes tiles loc, loc + W, loc + 2W, ... of the range (W workgroups per XCD),
@@ -641,23 +653,33 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // MULTI: up to three products with one B (the weight gradients of linears on one activation) as one list of tiles.  On its
 // own [2048,16384].[2048,16384]^T has 64 tiles of 256 x 256, too few for this kernel, and [11008,4096] leaves a third of the
 // units without work in its last round; together they fill the rounds.
-template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false>
+template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false, int BM = 256, int BN = 256>
 __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  // one wave per SIMD, 128x128 per wave: the least LDS traffic per flop
-  constexpr int BM = 256, BN = 256, BK = 128, NW = 4, TM = 8, TN = 8, R = 5;
+  // one wave per SIMD, 128x128 per wave (the least LDS traffic per flop) or, in a half tile, 64x128
+  static_assert((BM == 256 && BN == 256) || (BM == 256 && BN == 128) || (BM == 128 && BN == 256), "whole or half tiles");
+  constexpr bool HALF_TILE = BM * BN == 32768;
+  static_assert(!SK || !HALF_TILE, "the shared-K exchange is written for whole tiles");
+  constexpr int BK = 128, NW = 4, TM = HALF_TILE ? 4 : 8, TN = 8, WN = BN / 128;
   constexpr int WROWS = TM * 16;  // rows of the tile per wave
-  constexpr int UNIT = BM * BK;    // one ring slot: the A or the B panel of one K tile
-  constexpr int NL = BM / 8 / NW;  // 1 KiB wave loads (8 rows x 128 B) per panel per wave
-  constexpr int PEND = NL;         // in flight at the barrier of a trip: the unit requested in its first half
-  constexpr int PEND0 = 2 * NL;    // prologue: K tile 1 may be in flight when K tile 0 is published
+  constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;                // the panels of one K tile
+  constexpr int NLA = BM / 8 / NW, NLB = BN / 8 / NW;                // 1 KiB wave loads (8 rows x 128 B) per panel per wave
+  // The LDS ring.  Whole tiles: five slots of one panel, 2.5 K tiles; panels are requested four ahead.  Half tiles: three
+  // slots of one K tile; five ahead.  A trip requests one panel before its barrier (into the slot that the barrier before
+  // released) and one behind it (into the slot that this K tile's A panel just left).
+  constexpr int R = HALF_TILE ? 3 : 5, UNIT = HALF_TILE ? A_BYTES + B_BYTES : A_BYTES;
+  constexpr int AHEAD = HALF_TILE ? 5 : 4;
+  constexpr bool U1_IS_B = AHEAD % 2 != 0;                           // the panel requested before the barrier
+  constexpr int NL1 = U1_IS_B ? NLB : NLA, NL2 = U1_IS_B ? NLA : NLB;
+  constexpr int PEND = HALF_TILE ? NLA + NLB : NLA;    // in flight at the barrier of a trip: what lies beyond the next K tile
+  constexpr int PEND0 = HALF_TILE ? 2 * NLA + NLB : NLA + NLB;  // prologue: K tile 1 and more may be in flight when K tile 0 is published
   constexpr int N_STORES = TM * 4;  // store instructions per wave and C tile
   static_assert(N_STORES + PEND <= 63, "vmcnt is a 6-bit counter");
   extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / WN, wn = wave % WN;
 
   // ---- this workgroup's tiles ----
   const int nb = p.tiles_m * p.tiles_n;
@@ -745,7 +767,7 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 
   // ---- global -> LDS load plan ----
   // lane l of a wave load fills LDS row l/8, position l%8 of an 8-row group; position p of LDS row r holds
-  // chunk p ^ f(r), f(r) = (r & 7) ^ ((r >> 3) & 1).  Wave load i of a panel fills the LDS rows of group
+  // chunk p ^ f(r), f(r) = (r & 7) ^ ((r >> 3) & 1).  Wave load i (of NL) of a panel fills the LDS rows of group
   // g = wave * NL + i.  For the A panel LDS row = tile row.  For the B panel LDS row r = span*128 + tn*16 + j
   // holds tile row span*128 + 8*j + tn: within a group (8 consecutive j) the rows are 8 apart, and the group's
   // first row is span*128 + 64*(g & 1) + (g%16)/2.
@@ -826,20 +848,25 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
       ld_open(++ld_seg);
     }
   };
-  // i-th wave load (of NL) of the A or B panel of the loader's K tile into ring slot `slot`
-  auto load_one = [&](bool is_b, int slot, int i) {
+  // i-th wave load of the A or B panel of the loader's K tile into the panel at LDS offset `at`
+  auto load_one = [&](bool is_b, int at, int i) {
     const int k0 = ld_kt * BK;
     const uint32_t m_even = (k0 + chunk_even < p.K) ? 0u : kOOB, m_odd = (k0 + chunk_odd < p.K) ? 0u : kOOB;
-    const uint32_t dst = lds0 + slot * UNIT + (wave * NL + i) * 1024;
+    const int g = wave * (is_b ? NLB : NLA) + i;  // 8-row group of the panel's LDS image
+    const uint32_t dst = lds0 + at + g * 1024;
     if (!is_b) {
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsA, reinterpret_cast<lds_ptr_t>(dst), 16, a_voff[i & 1] | ((i & 1) ? m_odd : m_even),
-                                               k0 + (wave * NL + i) * 8 * (int)p.lda, 0, 0);
+                                               k0 + g * 8 * (int)p.lda, 0, 0);
     } else {
-      const int g = wave * NL + i;  // 8-row group of the panel's LDS image
       const int row = (g >> 4) * 128 + 64 * (g & 1) + ((g & 15) >> 1);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsB, reinterpret_cast<lds_ptr_t>(dst), 16, b_voff[i & 1] | ((i & 1) ? m_odd : m_even),
                                                k0 + row * (int)p.ldb, 0, 0);
     }
+  };
+  // LDS offset of the panel of the K tile `ahead` beyond the one whose slot is s0 (whole tiles: a slot per panel)
+  auto panel_at = [&](int s0, int ahead, bool is_b) {
+    if constexpr (HALF_TILE) return wrap(s0 + ahead) * UNIT + (is_b ? A_BYTES : 0);
+    else return wrap(s0 + 2 * ahead + (is_b ? 1 : 0)) * UNIT;
   };
 
   // ---- LDS -> register fragment plan ----
@@ -848,8 +875,8 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   typedef const __attribute__((address_space(3))) v4i *lds_v4i_ptr;
   // LDS addresses of the two 16-byte pieces a lane reads of its A row (ad[0], ad[1]) and B row (ad[2], ad[3]); opaque
   // additions, as in the kernel above
-  auto frag_addrs = [&](int slot_a, int slot_b, uint32_t (&ad)[4]) {
-    const uint32_t sa = lds0 + slot_a * UNIT + a_base, sb = lds0 + slot_b * UNIT + b_base;
+  auto frag_addrs = [&](int panel_a, int panel_b, uint32_t (&ad)[4]) {
+    const uint32_t sa = lds0 + panel_a + a_base, sb = lds0 + panel_b + b_base;
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[0]) : "s"(sa), "v"(foff[0]));
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[1]) : "s"(sa), "v"(foff[1]));
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[2]) : "s"(sb), "v"(foff[0]));
@@ -908,7 +935,7 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
         rs = make_rsrc(t.sa, (uint32_t)t.M * 4u);
       }
       seg_sa[0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + l) * 4, m0 * 4, 0);
-      seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
+      if constexpr (TM > 4) seg_sa[1] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0);
     } else {
       seg_sa[0] = seg_sa[1] = sa_one;
     }
@@ -1090,36 +1117,38 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     return false;
   };
 
-  // ---- prologue: K tiles 0 and 1 of the workgroup's stream requested, K tile 0 published, its first fragments read ----
+  // ---- prologue: the first AHEAD panels of the workgroup's stream requested, K tile 0 published, its first fragments read ----
   ld_open(0);
 #pragma unroll
-  for (int u = 0; u < R - 1; ++u) {
+  for (int u = 0; u < AHEAD; ++u) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i) load_one(u & 1, u, i);
+    for (int i = 0; i < (u & 1 ? NLB : NLA); ++i) load_one(u & 1, panel_at(0, u >> 1, u & 1), i);
     if (u & 1) ld_advance();
   }
   L8_WAIT_VM_LGKM0(PEND0);
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  // One trip = one K tile = 64 MFMAs, row by row of the wave's 8 x 8 tiles.
-  //   first half : rows 0 .. 3, while the A fragments of rows 2 .. 7 are read and the A panel two K tiles ahead is
-  //                requested (into the slot that the previous barrier released);
+  // One trip = one K tile = TM x TN MFMAs, row by row of the wave's tiles.
+  //   before the barrier: the first BAR of them, while the A fragments that are not there yet are read and a panel is
+  //                requested;
   //   barrier    : every wave has now read all of this K tile (lgkmcnt 0), and the next one has landed for every
   //                wave (partial vmcnt wait);
-  //   second half: rows 4 .. 7, while the next K tile's eight B fragments and first two A fragments are read and
-  //                the matching B panel is requested into the A slot this K tile just released.
+  //   behind it  : the others, while the next K tile's eight B fragments and first two A fragments are read and
+  //                another panel is requested.
   // A fragment lives for its row, the B fragments for the whole trip: two sets of them, in turn.  A wave issues in
   // order and the matrix cores want an MFMA every 32 cycles, half a dozen issue slots, so a group is one MFMA with at
-  // most one LDS read and one panel load, and the scheduling fences keep the groups as they are laid out here.
-  constexpr int N_MMA = TM * TN, HALF = N_MMA / 2;
+  // most one LDS read (half tiles, which are bound by LDS: now and then two) and one panel load, and the scheduling fences
+  // keep the groups as they are laid out here.
+  constexpr int N_MMA = TM * TN, BAR = HALF_TILE ? L8_HALF_TILE_BARRIER : N_MMA / 2, REST = N_MMA - BAR;
   constexpr int A_EARLY = 2;                       // A fragments read in the trip before
   constexpr int N_RD1 = 2 * (TM - A_EARLY), N_RD2 = 2 * (TN + A_EARLY);
-  constexpr int RD1_GROUPS = L8_READ_GROUPS1, RD2_GROUPS = L8_READ_GROUPS2;  // groups over which a half spreads its reads
-  static_assert(RD1_GROUPS < HALF - 4 && RD2_GROUPS <= HALF, "reads of the first half land before the barrier");
+  // groups over which the reads before and behind the barrier are spread
+  constexpr int RD1_GROUPS = HALF_TILE ? BAR - 4 : L8_READ_GROUPS1, RD2_GROUPS = HALF_TILE ? REST - 2 : L8_READ_GROUPS2;
+  static_assert(RD1_GROUPS <= BAR - 4 && RD2_GROUPS <= REST, "reads before the barrier land before it");
   v8i af[TM], bf0[TN], bf1[TN];
   uint32_t ad[4];
-  // read number r of the second half: B0, A0, B1, .. B7, A1, .. (the order of their use), two pieces each
+  // read number r behind the barrier: B0, A0, B1, .. B7, A1, .. (the order of their use), two pieces each
   auto read_next = [&](v8i (&bn)[TN], int r) {
     const int f = r >> 1;
     if (f == 0) read_piece(ad + 2, bn[0], 0, r & 1);
@@ -1127,51 +1156,52 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     else if (f <= TN) read_piece(ad + 2, bn[f - 1], f - 1, r & 1);
     else read_piece(ad, af[f - TN], f - TN, r & 1);
   };
-  frag_addrs(0, 1, ad);
+  frag_addrs(panel_at(0, 0, false), panel_at(0, 0, true), ad);
 #pragma unroll
   for (int r = 0; r < N_RD2; ++r) read_next(bf0, r);
-  int s0 = 0;  // ring slot of the A panel of the K tile being multiplied
+  int s0 = 0;  // ring slot of the K tile being multiplied (whole tiles: of its A panel)
   // FIRST: the first K tile of an output tile (the accumulators start from zero); `stores`: the stores of a C tile have
   // been issued since the panels that the trip's barrier waits for were requested.  They are younger than the panels and
   // the counter retires in order, so the count allows for them (waiting for the stores themselves would stall the start
   // of every tile).
   auto trip = [&](auto first_tag, bool stores, v8i (&bc)[TN], v8i (&bn)[TN]) __attribute__((always_inline)) {
     constexpr bool FIRST = decltype(first_tag)::value;
-    const int slot_u1 = wrap(s0 + R - 1);
+    const int at1 = panel_at(s0, AHEAD / 2, U1_IS_B), at2 = panel_at(s0, 0, false);
     auto mma_one = [&](int i) __attribute__((always_inline)) {
       const int tm = i / TN, tn = i % TN;
       acc[tm][tn] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af[tm], bc[tn], FIRST ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : acc[tm][tn], 0, 0, 0, 0, 0, 0);
     };
 #pragma unroll
-    for (int i = 0; i < HALF; ++i) {
+    for (int i = 0; i < BAR; ++i) {
       mma_one(i);
       if (i < RD1_GROUPS) {
 #pragma unroll
         for (int r = (N_RD1 * i) / RD1_GROUPS; r < (N_RD1 * (i + 1)) / RD1_GROUPS; ++r) read_piece(ad, af[A_EARLY + r / 2], A_EARLY + r / 2, r & 1);
       }
 #pragma unroll
-      for (int j = (NL * i) / HALF; j < (NL * (i + 1)) / HALF; ++j) load_one(false, slot_u1, j);
-      if (i == RD1_GROUPS) frag_addrs(wrap(s0 + 2), wrap(s0 + 3), ad);
+      for (int j = (NL1 * i) / BAR; j < (NL1 * (i + 1)) / BAR; ++j) load_one(U1_IS_B, at1, j);
+      if (i == RD1_GROUPS) frag_addrs(panel_at(s0, 1, false), panel_at(s0, 1, true), ad);
       __builtin_amdgcn_sched_barrier(0);
     }
+    if (U1_IS_B) ld_advance();
     if (FIRST && stores) L8_WAIT_VM_LGKM0(N_STORES + PEND);
     else L8_WAIT_VM_LGKM0(PEND);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int i = 0; i < HALF; ++i) {
-      mma_one(HALF + i);
+    for (int i = 0; i < REST; ++i) {
+      mma_one(BAR + i);
       if (i < RD2_GROUPS) {
 #pragma unroll
         for (int r = (N_RD2 * i) / RD2_GROUPS; r < (N_RD2 * (i + 1)) / RD2_GROUPS; ++r) read_next(bn, r);
       }
 #pragma unroll
-      for (int j = (NL * i) / HALF; j < (NL * (i + 1)) / HALF; ++j) load_one(true, s0, j);
+      for (int j = (NL2 * i) / REST; j < (NL2 * (i + 1)) / REST; ++j) load_one(!U1_IS_B, at2, j);
       __builtin_amdgcn_sched_barrier(0);
     }
-    ld_advance();
-    s0 = wrap(s0 + 2);
+    if (!U1_IS_B) ld_advance();
+    s0 = wrap(s0 + (HALF_TILE ? 1 : 2));
   };
   // n K tiles of one output tile.  Its first one finds its B fragments in bf0.
   auto k_loop = [&](int n, bool stores) __attribute__((always_inline)) {
@@ -1351,6 +1381,11 @@ static const Algo kAlgos[] = {
     {"skinny_8w_16n", nullptr, 64, 16, 512, 0, false, nullptr, nullptr, nullptr},
     L8_SMALL_ALGO_LIST(L8_ALGO_ROW)
     L8_SPLIT_ALGO_LIST(L8_SPLIT_ALGO_ROW)
+    /* 23, 24: algo 12 on half tiles, for problems that whole ones would spread over too few compute units or rounds */
+    {"stream_mt4x1w_2x4t_r3_g4", gemm_nt_stream_kernel<4, false, false, false, false, 256, 128>, 256, 128, 256, 3 * 384 * 128, true,
+     gemm_nt_stream_kernel<4, true, false, false, false, 256, 128>, gemm_nt_stream_kernel<4, false, false, true, false, 256, 128>, nullptr},
+    {"stream_mt2x2w_2x4t_r3_g8", gemm_nt_stream_kernel<8, false, false, false, false, 128, 256>, 128, 256, 256, 3 * 384 * 128, true,
+     gemm_nt_stream_kernel<8, true, false, false, false, 128, 256>, gemm_nt_stream_kernel<8, false, false, true, false, 128, 256>, nullptr},
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
 
@@ -1370,14 +1405,9 @@ static int pick_plain_big(int64_t K) { return K >= 4096 ? 5 : 3; }
 
 static int pick_algo(int64_t M, int64_t N, int64_t K) {
   if (M <= 8) return kSkinnyAlgo;  // whatever the chip: the smallest calls do not pay for asking
-  // large problems: the persistent kernel (measured 2-11 % ahead of the plain ones on every shape with at
-  // least one 256x256 tile per compute unit; groups of 4 tile rows ahead of groups of 8 by 1-3 %), also when
-  // the big tiles leave up to 7/16 of the compute units idle (measured with K = 2048 .. 16384: 144 to 240
-  // tiles on 256 compute units run 10-25 % faster than with 128x128 tiles, 128 tiles and fewer 15-45 % slower)
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const bool big = tiles(256, 256) * 16 >= cus * 9;
-  if (big && M > kSkinnyMaxM) return 12;
+  const bool big = tiles(256, 256) * 16 >= cus * 9;  // 9/16 of the units have a 256 x 256 tile
   // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against the best tile: [20,2048].
   // [2048,2048] 4.2 / 7.5, [64,11008].[4096,11008] 18.9 / 28.8, [32,4096].[11008,4096] 14.6 / 13.5; from 48 tokens on
   // the 64 x 64 tiles win where there are enough of them ([48,4096].[11008,4096] 17.6 / 14.0, [40,4096].[8192,4096]
@@ -1403,7 +1433,26 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   if (tiles(64, 128) <= cus) return 19;
   if (tiles(128, 64) <= cus) return 20;
   if (tiles(128, 128) <= cus) return 18;
-  return 2;  // two 128 x 128 workgroups share a unit: [1500,1440].[3008,1440] 16.3, 20.9 with nine slots
+  // Barely more than that with a short reduction, or few rows: two 128 x 128 workgroups share a unit.  us, these / the half
+  // tiles below: [64,4096].[36864,4096] 42 / 44, [1500,1440].[3008,1440] 14.5 / 13.5 with rows on lines and 16.3 / 17 without;
+  // longer reductions [1884,4544].[2384,4544] 28.3 / 26.5, [3973,3488].[1072,3488] 25.0 / 21.9.
+  if (M <= kSkinnyMaxM || (!big && K <= 2048 && tiles(128, 128) * 8 <= cus * 9)) return 2;
+  // Beyond: the persistent kernel, on whole tiles or on half ones (of the two forms the one with fewer rounds).  It is
+  // bound by its rounds of one tile per unit, and a round of half tiles takes 0.59 of a round of whole ones (1300 against
+  // 2280 cycles per K tile: 1.5 times the bytes per flop through the L2, which then is what a trip waits for; with short
+  // reductions less, the C tile weighs more).  So half tiles where their rounds are at most 3/2 of the others', 5/3 up to
+  // K = 4096, 7/4 up to 2048.  us, 128 x 128 / half / whole: [4096,2048].[2048,2048] 19.9 / 18.4 / 26.0,
+  // [1645,9776].[4272,9776] 63.5 / 53.3 / 82.2, [502,11312].[9568,11312] 94.4 / 68.4 / 100.5, [3115,2336].[2752,2336] 31.5
+  // / 30.1 / 25.8 (286 half tiles are two rounds, 143 whole ones are one), [1566,1136].[9904,1136] 28.3 / 22.1 / 31.8,
+  // [1294,7392].[13664,7392] 142 / 126 / 138, [14991,4032].[2224,4032] 127 / 118 / 123 and [2710,8832].[14064,8832] 322 /
+  // 278 / 263 (5 against 3), [11181,1328].[3424,1328] 60.3 / 49.9 / 55.6, [5561,1664].[9104,1664] 92.8 / 81.0 / 88.4 (7
+  // rounds against 4), but [4093,4096]. [14336,4096] 204 / 169 / 163 (also 7 against 4), [6191,3568].[4016,3568] 88 / 83 /
+  // 73 (4 against 2).
+  auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
+  const int64_t whole = rounds(tiles(256, 256)), tall = rounds(tiles(256, 128)), wide2 = rounds(tiles(128, 256));
+  const int64_t half = wide2 < tall ? wide2 : tall;
+  if (half * 2 <= whole * 3 || (K <= 4096 && half * 3 <= whole * 5) || (K <= 2048 && half * 4 <= whole * 7)) return wide2 < tall ? 24 : 23;
+  return 12;
 }
 
 // Host arithmetic only: the tile configuration `algo = 0` resolves to for this problem on the current device when
@@ -1487,7 +1536,7 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
                     (sb_mode != L8_SCALE_ROW || ((uintptr_t)sb % 16) == 0) &&
                     (bias == nullptr || (((uintptr_t)bias % 8) == 0 && kAlgos[algo - 1].fn_bias != nullptr)) &&
                     (!add || kAlgos[algo - 1].fn_add != nullptr);
-    if (!ok) algo = pick_plain_big(K);
+    if (!ok) algo = kAlgos[algo - 1].bm * kAlgos[algo - 1].bn < 256 * 256 ? 2 : pick_plain_big(K);
   }
   if (algo == kSkinnyAlgo) {
     if (skinny_serves(M, N, K, lda, ldb, 1))

@@ -44,9 +44,11 @@ def test_exact_small_integer_operands(algo):
 
 @pytest.mark.parametrize("K", [16, 128, 144, 256, 272, 400, 528, 1152])
 @pytest.mark.parametrize("with_bias,scalar", [(False, False), (False, True), (True, False)])
-def test_persistent_kernel_carries_its_fragments_from_tile_to_tile(K, with_bias, scalar):
+@pytest.mark.parametrize("algo", [12, 23, 24])
+def test_persistent_kernel_carries_its_fragments_from_tile_to_tile(algo, K, with_bias, scalar):
     """One to nine K tiles per output tile (even and odd numbers of them leave the next tile's fragments in one or the other
-    register set, the last K tile short or whole) and 289 output tiles, so that some workgroups have two; ragged last tiles.
+    register set, the last K tile short or whole) and 289 whole or 561 half tiles, so that workgroups have one, two or three;
+    ragged last tiles.
     Integers in -1 .. 1 and powers of two for scales: the fp32 sums are exact, so is the one rounding to bf16."""
     from lingua_amd import ops
     g = torch.Generator().manual_seed(170 + K)
@@ -55,7 +57,7 @@ def test_persistent_kernel_carries_its_fragments_from_tile_to_tile(K, with_bias,
     sa = torch.tensor([2.0 ** (i % 5 - 2) for i in range(M)]).reshape(M, 1).cuda()
     sb = torch.tensor([2.0 ** (i % 3) for i in range(1 if scalar else N)]).reshape(-1, 1).cuda()
     bias = torch.randint(-8, 9, (N,), generator=g).to(torch.bfloat16).cuda() if with_bias else None
-    out = ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa, sb, bias, algo=12)
+    out = ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa, sb, bias, algo=algo)
     want = (A.cuda() @ B.cuda().t()) * sa * sb.t() + (0 if bias is None else bias.float())   # fp32: exact here
     assert torch.equal(out, want.to(torch.bfloat16))
 
@@ -85,7 +87,8 @@ def test_few_tokens_exact_on_integers_and_within_tolerance_of_the_oracle(M):
             assert rel_l2(out, oracle.gemm_nt(qa, qb, sa_, sb_, b_)) <= (TOL if M * N >= 5000 else 2.0 ** -8), (M, N, K)
 
 
-@pytest.mark.parametrize("algo,tile", [(18, (128, 128)), (19, (64, 128)), (20, (128, 64)), (21, (64, 64)), (22, (32, 64))])
+@pytest.mark.parametrize("algo,tile", [(18, (128, 128)), (19, (64, 128)), (20, (128, 64)), (21, (64, 64)), (22, (32, 64)), (23, (256, 128)),
+                                       (24, (128, 256))])
 def test_small_tiles_exact_on_integers_at_their_edges(algo, tile):
     """The configurations for problems of at most one workgroup per compute unit: tiles full, one short and one over,
     reductions from a ring that is never filled (K = 16; a second group of waves without a K tile) to one that wraps
@@ -106,7 +109,10 @@ def test_small_tiles_exact_on_integers_at_their_edges(algo, tile):
 @pytest.mark.parametrize("mnk,name", [((200, 4096, 4096), "1x1t"), ((1021, 2048, 2048), "1x2t"), ((512, 4096, 4096), "1x2t"),
                                       ((2176, 960, 256), "2x1t"), ((2048, 2048, 4096), "2x2t_r9"), ((1500, 3008, 1440), "2x2t_r5"),
                                       ((64, 11008, 4096), "mt2x2w_1x1t"), ((32, 11008, 4096), "mt1x2w_1x1t"), ((16, 11008, 4096), "skinny"),
-                                      ((9, 9216, 5120), "mt1x2w_1x1t"), ((8, 9216, 5120), "skinny"), ((32, 16448, 4096), "skinny"), ((16384, 2048, 2048), "stream")])
+                                      ((9, 9216, 5120), "mt1x2w_1x1t"), ((8, 9216, 5120), "skinny"), ((32, 16448, 4096), "skinny"), ((16384, 2048, 2048), "stream"),
+                                      ((4096, 2048, 2048), "mt4x1w_2x4t"), ((4165, 1920, 2832), "mt4x1w_2x4t"), ((3115, 2752, 2336), "mt2x2w_4x4t"),
+                                      ((1566, 9904, 1136), "mt2x2w_2x4t"), ((5561, 9104, 1664), "mt4x1w_2x4t"), ((5561, 9104, 4096), "mt2x2w_4x4t"),
+                                      ((64, 36864, 4096), "2x2t_r5"), ((65, 36864, 4096), "mt2x2w_2x4t")])
 def test_tile_chosen_by_how_many_workgroups_it_makes(mnk, name):
     from lingua_amd import ops
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:
