@@ -87,6 +87,21 @@ typedef struct {
 int l8_cast_rowwise_many(const l8_cast_rowwise_item *items, int64_t n, int64_t C, void *stream);
 int64_t l8_cast_rowwise_workspace(int64_t R, int64_t C);
 
+/* l8_cast_rowwise with column amaxes for n operands (of any widths), each with a workspace of its own; up to three folds of
+ * partial column maxima share a launch. */
+typedef struct {
+  const void *x;
+  int64_t R, C, ldx;
+  void *q;
+  int64_t ldq;
+  float *scale;
+  void *amax;
+  float *col_amax;
+  void *workspace;
+  int64_t workspace_bytes;
+} l8_cast_rowwise_cols_item;
+int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items, int64_t n, void *stream);
+
 /* l8_cast_rowwise for callers that cannot allocate device memory (code under HIP graph capture, tight
  * serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference, whose ATen ops
  * allocate freely.  Same arguments and results as l8_cast_rowwise without the workspace: the partial
@@ -158,6 +173,21 @@ int l8_cast_colwise_transposed(const void *x, int64_t R, int64_t C, int64_t ldx,
 int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t C, int64_t ldx,
                                    const float *col_amax,
                                    void *q, int64_t ldq, int64_t Rp, float *scale, void *stream);
+
+/* Transposed casts of n operands: with col_amax as l8_cast_colwise_transposed_pad, with amax_rows (bf16, n_amax of them) as
+ * l8_cast_tensorwise_t_rows; exactly one of the two is set.  Neighbours of one kind share a launch, up to four.  All operands
+ * are checked before anything is enqueued; none may be empty. */
+typedef struct {
+  const void *x;
+  int64_t R, C, ldx;
+  const float *col_amax;
+  const void *amax_rows;
+  int64_t n_amax;
+  void *q;
+  int64_t ldq, Rp;
+  float *scale;
+} l8_cast_transposed_item;
+int l8_cast_transposed_many(const l8_cast_transposed_item *items, int64_t n, void *stream);
 
 /* Scaled fp8 product, both operands reduction-contiguous ("NT"):
  *   C[m,n] = bf16( (sum_k A[m,k]*B[n,k]) * sa[m or 0] * sb[n or 0] + bias[n] )

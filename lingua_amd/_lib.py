@@ -27,6 +27,8 @@ SIGNATURES = {
     "l8_cast_rowwise": [_p, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p],
     "l8_cast_rowwise_many": [_p, _i64, _i64, _p],
     "l8_cast_rowwise_workspace": [_i64, _i64],
+    "l8_cast_rowwise_cols_many": [_p, _i64, _p],
+    "l8_cast_transposed_many": [_p, _i64, _p],
     "l8_cast_rowwise_noalloc": [_p, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _p],
     "l8_cast_rowwise_given_amax": [_p, _i64, _i64, _i64, _p, _int, _p, _i64, _p, _p],
     "l8_col_amax": [_p, _i64, _i64, _i64, _p, _p],

@@ -303,9 +303,18 @@ __global__ __launch_bounds__(kRowBlock, (NCHW <= 4 ? 4 : (NCHW <= 8 ? 2 : 1))) v
 // read by a launch that lasts microseconds); the 128 row groups then meet in LDS.  One launch, no atomics,
 // nothing to zero beforehand.
 constexpr int kFoldCols = 64, kFoldThreads = 1024, kFoldRowGroups = kFoldThreads / 8;
-__global__ __launch_bounds__(kFoldThreads) void colmax_fold_kernel(const uint16_t *__restrict__ partials,
-                                                                   int n_slots, int C,
-                                                                   uint32_t *__restrict__ col_amax) {
+// Tensors that are folded together (row y of the grid is one) share the launch: the fold of one is microseconds of latency
+// on a few workgroups.  us, casts with their folds, one by one / together: four [16384,2048] 92.2 / 85.0, four [3290,1392]
+// 42.7 / 34.2, [493,4832] and two [493,6784] 33.1 / 25.3.
+struct FoldOperands {
+  FoldOperand op[kMaxFolds];
+};
+__global__ __launch_bounds__(kFoldThreads) void colmax_fold_kernel(const FoldOperands list) {
+  const FoldOperand &o = list.op[blockIdx.y];
+  const uint16_t *__restrict__ partials = (const uint16_t *)o.partials;
+  uint32_t *__restrict__ col_amax = (uint32_t *)o.col_amax;
+  const int n_slots = (int)o.slots, C = (int)o.C;
+  if ((int)blockIdx.x * kFoldCols >= C) return;
   __shared__ v4i red[kFoldRowGroups][8];
   __shared__ uint32_t red2[8][32];
   const int cc = threadIdx.x & 7;   // which 8 columns (16 bytes) of the 64
@@ -550,12 +559,46 @@ constexpr int64_t kMaxAmaxRows = 16384;           // longest list that every wor
 
 // Columns R .. Rp - 1 of q are zeros: what a reduction over the tokens pads them to.  The rows are whole 16-byte pieces
 // then, also for an odd number of tokens: [4093,14336] 36.1 -> 33.9 us, [4093,4096] 13.6 -> 12.4, and no fill in front (5).
-template <AmaxFrom FROM, int TC, int TU>
-__global__ __launch_bounds__(256) void cast_transposed_kernel(
-    const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, const void *__restrict__ amax_scalar, int amax_f32,
-    const uint32_t *__restrict__ col_amax, const uint16_t *__restrict__ amax_rows, int n_amax, uint8_t *__restrict__ q,
-    int64_t ldq, int64_t Rp, float *__restrict__ scale, int vec_store, int scale_rule) {
+//
+// Several tensors go through one launch as one list of tiles (the output gradients of linears on one activation and that
+// activation; their weights): each alone fills and drains the chip in a few microseconds.  us, one by one / together:
+// four [16384,2048] 79.6 / 68.0, [4093,4096] and two [4093,14336] 79.4 / 69.2, two [1021,2048] 5.8 / 3.9, four [3290,1392] 22.7 /
+// 15.2, [16384,2048] and two [16384,8192] 173.9 / 165.3; weights: three [2048,2048] 11.8 / 7.5, two [14336,4096] 69.6 / 64.4.
+struct TransposedOperand {
+  const uint16_t *x;
+  int64_t R, ldx;
+  const void *amax;             // scalar, column amaxes or row amaxes, as FROM says
+  uint8_t *q;
+  int64_t ldq, Rp;
+  float *scale;
+  int C, n_amax, vec_store;     // n_amax: length of the list of row amaxes, or 1 for an fp32 scalar
+  int first;                    // first workgroup of the launch; the operands are in order, unused ones start beyond the last
+};
+constexpr int kMaxTransposed = 4;
+struct TransposedOperands {
+  TransposedOperand op[kMaxTransposed];
+};
+template <AmaxFrom FROM, int TC, int TU, bool MANY = false>
+__global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditional_t<MANY, TransposedOperands, TransposedOperand> list, int scale_rule) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only
+  int which = 0;
+  if constexpr (MANY) {
+#pragma unroll
+    for (int i = 1; i < kMaxTransposed; ++i) which += (int)blockIdx.x >= list.op[i].first ? 1 : 0;
+  }
+  const TransposedOperand &op = [&]() -> const TransposedOperand & {
+    if constexpr (MANY) return list.op[which];
+    else return list;
+  }();
+  const uint16_t *const __restrict__ x = op.x;
+  const int64_t R = op.R, ldx = op.ldx, ldq = op.ldq, Rp = op.Rp;
+  const int C = op.C, n_amax = op.n_amax, vec_store = op.vec_store, amax_f32 = FROM == AmaxFrom::kScalar ? n_amax : 0;
+  const uint32_t *const __restrict__ col_amax = (const uint32_t *)op.amax;
+  const uint16_t *const __restrict__ amax_rows = (const uint16_t *)op.amax;
+  const void *const __restrict__ amax_scalar = op.amax;
+  uint8_t *const __restrict__ q = op.q;
+  float *const __restrict__ scale = op.scale;
+  const unsigned block = blockIdx.x - (MANY ? (unsigned)op.first : 0u);
   using T = TransposeTile<TC, TU>;
   constexpr bool PER_COL = FROM == AmaxFrom::kColumns, ROWS = FROM == AmaxFrom::kRows;
   constexpr int kTC = T::kTC, kCCH = T::kCCH, kRG = T::kRG, kTU = T::kTU, kTR = T::kTR, kTStride = T::kTStride;
@@ -572,8 +615,8 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
   // column blocks (wide bands of the input rows).
   const int nct = (C + kTC - 1) / kTC;
   const int64_t nrt = (Rp + kTR - 1) / kTR;
-  const int cb = (int)(blockIdx.x % nct);
-  const int64_t rt = (blockIdx.x / nct + cb) % nrt;
+  const int cb = (int)(block % nct);
+  const int64_t rt = (block / nct + cb) % nrt;
   const int64_t r0 = rt * kTR;
   const int c0 = cb * kTC;
   const int cc = t % kCCH;  // which 8-column chunk of the tile
@@ -659,7 +702,7 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(
     const float rc = recip_exact(s);
 #pragma unroll
     for (int j = 0; j < 8; ++j) rcp[j] = rc;
-    if (blockIdx.x == 0 && t == 0) scale[0] = s;
+    if (block == 0 && t == 0) scale[0] = s;
   }
 
   // convert and transpose inside the thread: column j <- rows 0..3 of each unit
@@ -753,11 +796,21 @@ static int64_t rowwise_blocks(int64_t R, int64_t C, bool colmax) {
   return 0;
 }
 
-int fold_colmax(const void *partials, int64_t slots, int64_t C, float *col_amax, hipStream_t st) {
-  hipLaunchKernelGGL(colmax_fold_kernel, dim3((unsigned)((C + kFoldCols - 1) / kFoldCols)), dim3(kFoldThreads), 0, st,
-                     (const uint16_t *)partials, (int)slots, (int)C, (uint32_t *)col_amax);
+int fold_colmax_many(const FoldOperand *ops, int n, hipStream_t st) {
+  FoldOperands list{};
+  int64_t widest = 0;
+  for (int i = 0; i < n; ++i) {
+    list.op[i] = ops[i];
+    if (ops[i].C > widest) widest = ops[i].C;
+  }
+  hipLaunchKernelGGL(colmax_fold_kernel, dim3((unsigned)((widest + kFoldCols - 1) / kFoldCols), (unsigned)n), dim3(kFoldThreads), 0, st, list);
   L8_HIP(hipGetLastError());
   return L8_OK;
+}
+
+int fold_colmax(const void *partials, int64_t slots, int64_t C, float *col_amax, hipStream_t st) {
+  const FoldOperand one{partials, col_amax, slots, C};
+  return fold_colmax_many(&one, 1, st);
 }
 
 static int zero_u32(void *p, int64_t n, hipStream_t st) {
@@ -775,7 +828,7 @@ static int launch_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx, void
     hipLaunchKernelGGL((cast_rowwise_kernel<NCH, true>), dim3((unsigned)blocks), dim3(kRowBlock), lds, st,
                        (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule(), 0);
     L8_HIP(hipGetLastError());
-    return fold_colmax(ws, blocks, C, col_amax, st);
+    return L8_OK;  // the caller folds
   }
   hipLaunchKernelGGL((cast_rowwise_kernel<NCH, false>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
                      (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule(), 0);
@@ -791,7 +844,7 @@ static int launch_rowwise_wg(const void *x, int64_t R, int64_t C, int64_t ldx, v
     hipLaunchKernelGGL((cast_rowwise_wg_kernel<NCHW, true>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
                        (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)ws, l8::scale_rule(), 0);
     L8_HIP(hipGetLastError());
-    return fold_colmax(ws, blocks, C, col_amax, st);
+    return L8_OK;  // the caller folds
   }
   hipLaunchKernelGGL((cast_rowwise_wg_kernel<NCHW, false>), dim3((unsigned)blocks), dim3(kRowBlock), 0, st,
                      (const uint16_t *)x, R, (int)C, ldx, (uint8_t *)q, ldq, scale, (uint16_t *)amax, (uint16_t *)nullptr, l8::scale_rule(), 0);
@@ -856,9 +909,21 @@ extern "C" int64_t l8_cast_rowwise_workspace(int64_t R, int64_t C) {
 
 // Argument checks and dispatch shared by l8_cast_rowwise and l8_cast_rowwise_noalloc; `what` names the
 // entry point in error messages.  `workspace` holds at least l8_cast_rowwise_workspace(R, C) bytes when
-// col_amax is given (checked by the callers).
+// col_amax is given (checked by the callers).  The partial column maxima are left to be folded where `fold` is given (and
+// there are any: else its width is 0), and folded otherwise.
+static int launch_rowwise_any(const char *what, const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq,
+                              float *scale, void *amax, float *col_amax, void *workspace, hipStream_t st);
 static int cast_rowwise_impl(const char *what, const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq,
-                             float *scale, void *amax, float *col_amax, void *workspace, hipStream_t st) {
+                             float *scale, void *amax, float *col_amax, void *workspace, hipStream_t st, FoldOperand *fold = nullptr) {
+  const int rc = launch_rowwise_any(what, x, R, C, ldx, q, ldq, scale, amax, col_amax, workspace, st);
+  const int64_t slots = rc == L8_OK && col_amax ? rowwise_blocks(R, C, true) : 0;
+  if (fold) *fold = {workspace, col_amax, slots, slots ? C : 0};
+  else if (slots) return fold_colmax(workspace, slots, C, col_amax, st);
+  return rc;
+}
+
+static int launch_rowwise_any(const char *what, const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq,
+                              float *scale, void *amax, float *col_amax, void *workspace, hipStream_t st) {
   L8_REQUIRE(x != nullptr, "%s: x is null", what);
   L8_REQUIRE((q == nullptr) || (scale != nullptr), "%s: q given without scale", what);
   L8_REQUIRE(C % 8 == 0 && ldx % 8 == 0 && ldx >= C, "%s: C=%lld and ldx=%lld must be multiples of 8, ldx >= C", what,
@@ -899,6 +964,31 @@ extern "C" int l8_cast_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx,
                (long long)need);
   }
   return cast_rowwise_impl("l8_cast_rowwise", x, R, C, ldx, q, ldq, scale, amax, col_amax, workspace, (hipStream_t)stream);
+}
+
+extern "C" int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items, int64_t n, void *stream) {
+  L8_REQUIRE(n >= 0 && (n == 0 || items), "l8_cast_rowwise_cols_many: null items, or a negative count");
+  for (int64_t i = 0; i < n; ++i) {
+    const l8_cast_rowwise_cols_item &t = items[i];
+    L8_REQUIRE(t.R >= 0 && t.C >= 0 && t.col_amax, "l8_cast_rowwise_cols_many: negative shape, or no column amaxes asked for");
+    const int64_t need = l8_cast_rowwise_workspace(t.R, t.C);
+    L8_REQUIRE(need == 0 || (t.workspace != nullptr && t.workspace_bytes >= need && aligned(t.workspace, 16)),
+               "l8_cast_rowwise_cols_many: needs a 16-byte aligned workspace of %lld bytes (l8_cast_rowwise_workspace) per operand", (long long)need);
+  }
+  FoldOperand folds[kMaxFolds];
+  int pending = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const l8_cast_rowwise_cols_item &t = items[i];
+    if (t.R == 0 || t.C == 0) continue;
+    int rc = cast_rowwise_impl("l8_cast_rowwise_cols_many", t.x, t.R, t.C, t.ldx, t.q, t.ldq, t.scale, t.amax, t.col_amax, t.workspace,
+                               (hipStream_t)stream, &folds[pending]);
+    if (rc == L8_OK && folds[pending].C > 0 && ++pending == kMaxFolds) {
+      rc = fold_colmax_many(folds, pending, (hipStream_t)stream);
+      pending = 0;
+    }
+    if (rc != L8_OK) return rc;
+  }
+  return pending ? fold_colmax_many(folds, pending, (hipStream_t)stream) : L8_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -1019,34 +1109,56 @@ struct TransposedCast {
   float *scale;
 };
 
+// `n` casts of one kind (all from column amaxes, all from row amaxes, or one from a scalar) as one list of tiles.
 template <int TC, int TU>
-static int launch_transposed_tile(const TransposedCast &a, hipStream_t st) {
+static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st) {
   using T = TransposeTile<TC, TU>;
   static_assert(T::kTR <= kMaxTileRows, "the row-stride limit assumes no taller tile");
-  const int64_t gx = ((a.C + T::kTC - 1) / T::kTC) * ((a.Rp + T::kTR - 1) / T::kTR);
-  L8_REQUIRE(gx < (1LL << 31), "transposed cast: shape too large (%lld x %lld)", (long long)a.R, (long long)a.C);
-  const int vec = (a.ldq % 16 == 0 && aligned(a.q, 16)) ? 1 : 0;
-  auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)gx), dim3(256), 0, st, (const uint16_t *)a.x, a.R, (int)a.C, a.ldx, a.amax, a.amax_f32,
-                       (const uint32_t *)a.col_amax, (const uint16_t *)a.amax_rows, (int)a.n_amax, (uint8_t *)a.q, a.ldq, a.Rp, a.scale,
-                       vec, l8::scale_rule());
+  TransposedOperands list{};
+  int64_t gx = 0;
+  for (int i = 0; i < kMaxTransposed; ++i) {
+    if (i >= n) {
+      list.op[i].first = INT32_MAX;
+      continue;
+    }
+    const TransposedCast &t = a[i];
+    const void *amax = t.col_amax ? (const void *)t.col_amax : t.amax_rows ? t.amax_rows : t.amax;
+    list.op[i] = {(const uint16_t *)t.x, t.R, t.ldx, amax, (uint8_t *)t.q, t.ldq, t.Rp, t.scale, (int)t.C,
+                  t.amax_rows ? (int)t.n_amax : t.amax_f32, (t.ldq % 16 == 0 && aligned(t.q, 16)) ? 1 : 0, (int)gx};
+    gx += ((t.C + T::kTC - 1) / T::kTC) * ((t.Rp + T::kTR - 1) / T::kTR);
+    L8_REQUIRE(gx < INT32_MAX, "transposed cast: shape too large (%lld x %lld)", (long long)t.R, (long long)t.C);
+  }
+  auto go = [&](auto kernel, const auto &what) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gx), dim3(256), 0, st, what, l8::scale_rule());
   };
-  if (a.col_amax) go(cast_transposed_kernel<AmaxFrom::kColumns, TC, TU>);
-  else if (a.amax_rows) go(cast_transposed_kernel<AmaxFrom::kRows, TC, TU>);
-  else go(cast_transposed_kernel<AmaxFrom::kScalar, TC, TU>);
+  if (n > 1) {
+    if (a[0].col_amax) go(cast_transposed_kernel<AmaxFrom::kColumns, TC, TU, true>, list);
+    else go(cast_transposed_kernel<AmaxFrom::kRows, TC, TU, true>, list);
+  } else if (a[0].col_amax) {
+    go(cast_transposed_kernel<AmaxFrom::kColumns, TC, TU>, list.op[0]);
+  } else if (a[0].amax_rows) {
+    go(cast_transposed_kernel<AmaxFrom::kRows, TC, TU>, list.op[0]);
+  } else {
+    go(cast_transposed_kernel<AmaxFrom::kScalar, TC, TU>, list.op[0]);
+  }
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
 
-static int launch_transposed(const TransposedCast &a, hipStream_t st) {
-  // a tile's rows within 1 GiB: then no sum of a lane's offset (up to twice the tile) and a row's scalar offset wraps
-  L8_REQUIRE((int64_t)kMaxTileRows * a.ldx * 2 < (1LL << 30), "transposed cast: row stride too large (%lld elements)", (long long)a.ldx);
-  const int64_t tiles128 = ((a.C + 127) / 128) * ((a.R + 127) / 128);
+static int launch_transposed(const TransposedCast *a, int n, hipStream_t st) {
+  int64_t tiles128 = 0;
+  bool large = true;
+  for (int i = 0; i < n; ++i) {
+    // a tile's rows within 1 GiB: then no sum of a lane's offset (up to twice the tile) and a row's scalar offset wraps
+    L8_REQUIRE((int64_t)kMaxTileRows * a[i].ldx * 2 < (1LL << 30), "transposed cast: row stride too large (%lld elements)", (long long)a[i].ldx);
+    tiles128 += ((a[i].C + 127) / 128) * ((a[i].R + 127) / 128);
+    large = large && a[i].R >= 16384 && a[i].C >= 8192;
+  }
   if (tiles128 < 4 * (int64_t)num_cus())  // too few 128 x 128 tiles for four workgroups per compute unit
-    return launch_transposed_tile<64, 1>(a, st);
-  if (a.R >= 16384 && a.C >= 8192)  // the large activations: see the note on the tile shapes
-    return launch_transposed_tile<128, 4>(a, st);
-  return launch_transposed_tile<128, 2>(a, st);
+    return launch_transposed_tile<64, 1>(a, n, st);
+  if (large)  // the large activations: see the note on the tile shapes
+    return launch_transposed_tile<128, 4>(a, n, st);
+  return launch_transposed_tile<128, 2>(a, n, st);
 }
 
 static int check_transposed(const char *what, const TransposedCast &a) {
@@ -1070,7 +1182,8 @@ extern "C" int l8_cast_tensorwise(const void *x, int64_t R, int64_t C, int64_t l
   hipStream_t st = (hipStream_t)stream;
   if (transpose) {
     L8_REQUIRE(ldq >= R, "l8_cast_tensorwise: transposed output needs ldq >= R");
-    return launch_transposed(TransposedCast{x, R, C, ldx, amax, amax_dtype, nullptr, nullptr, 0, q, ldq, R, scale}, st);
+    const TransposedCast a{x, R, C, ldx, amax, amax_dtype == L8_AMAX_F32, nullptr, nullptr, 0, q, ldq, R, scale};
+    return launch_transposed(&a, 1, st);
   }
   L8_REQUIRE(ldq >= C && ldq % 8 == 0 && aligned(q, 8), "l8_cast_tensorwise: q must be 8-byte aligned with ldq %% 8 == 0, ldq >= C");
   const int64_t total = R * (C / 8);
@@ -1093,7 +1206,7 @@ extern "C" int l8_cast_tensorwise_t_rows(const void *x, int64_t R, int64_t C, in
   if (R == 0 || C == 0) return L8_OK;
   const TransposedCast a{x, R, C, ldx, nullptr, 0, nullptr, amax_rows, n, q, ldq, R, scale};
   const int rc = check_transposed("l8_cast_tensorwise_t_rows", a);
-  return rc == L8_OK ? launch_transposed(a, (hipStream_t)stream) : rc;
+  return rc == L8_OK ? launch_transposed(&a, 1, (hipStream_t)stream) : rc;
 }
 
 static int cast_colwise(const char *what, const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax, void *q,
@@ -1104,7 +1217,7 @@ static int cast_colwise(const char *what, const void *x, int64_t R, int64_t C, i
   L8_REQUIRE(R > 0, "%s: R must be positive when C > 0", what);
   const TransposedCast a{x, R, C, ldx, nullptr, 0, col_amax, nullptr, 0, q, ldq, Rp, scale};
   const int rc = check_transposed(what, a);
-  return rc == L8_OK ? launch_transposed(a, (hipStream_t)stream) : rc;
+  return rc == L8_OK ? launch_transposed(&a, 1, (hipStream_t)stream) : rc;
 }
 
 extern "C" int l8_cast_colwise_transposed(const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax,
@@ -1115,4 +1228,30 @@ extern "C" int l8_cast_colwise_transposed(const void *x, int64_t R, int64_t C, i
 extern "C" int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t C, int64_t ldx, const float *col_amax,
                                               void *q, int64_t ldq, int64_t Rp, float *scale, void *stream) {
   return cast_colwise("l8_cast_colwise_transposed_pad", x, R, C, ldx, col_amax, q, ldq, Rp, scale, stream);
+}
+
+extern "C" int l8_cast_transposed_many(const l8_cast_transposed_item *items, int64_t n, void *stream) {
+  L8_REQUIRE(n >= 0 && (n == 0 || items), "l8_cast_transposed_many: null items, or a negative count");
+  TransposedCast casts[kMaxTransposed];
+  for (int64_t i = 0; i < n; ++i) {  // all are checked before any of them is enqueued
+    const l8_cast_transposed_item &t = items[i];
+    L8_REQUIRE(t.R > 0 && t.C > 0 && t.scale && (t.col_amax != nullptr) != (t.amax_rows != nullptr),
+               "l8_cast_transposed_many: operands with rows, a scale and either column amaxes or row amaxes required");
+    L8_REQUIRE(!t.amax_rows || (t.n_amax >= 8 && t.n_amax <= kMaxAmaxRows && t.n_amax % 8 == 0 && aligned(t.amax_rows, 16)),
+               "l8_cast_transposed_many: 16-byte aligned row amaxes, a multiple of 8 of them and at most %lld, required", (long long)kMaxAmaxRows);
+    const int rc = check_transposed("l8_cast_transposed_many", TransposedCast{t.x, t.R, t.C, t.ldx, nullptr, 0, t.col_amax, t.amax_rows, t.n_amax, t.q, t.ldq, t.Rp, t.scale});
+    if (rc != L8_OK) return rc;
+    L8_REQUIRE((int64_t)kMaxTileRows * t.ldx * 2 < (1LL << 30), "l8_cast_transposed_many: row stride too large (%lld elements)", (long long)t.ldx);
+  }
+  for (int64_t i = 0; i < n;) {  // runs of one kind
+    int run = 0;
+    for (; i < n && run < kMaxTransposed; ++i, ++run) {
+      const l8_cast_transposed_item &t = items[i];
+      if (run && (t.col_amax != nullptr) != (casts[0].col_amax != nullptr)) break;
+      casts[run] = TransposedCast{t.x, t.R, t.C, t.ldx, nullptr, 0, t.col_amax, t.amax_rows, t.n_amax, t.q, t.ldq, t.Rp, t.scale};
+    }
+    const int rc = launch_transposed(casts, run, (hipStream_t)stream);
+    if (rc != L8_OK) return rc;
+  }
+  return L8_OK;
 }

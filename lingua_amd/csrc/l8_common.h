@@ -38,6 +38,14 @@ int device_slot();
 // Folds partial column maxima [slots, C] (bf16, one row per workgroup of a
 // row-wise kernel) into col_amax[C] (fp32 bit patterns, overwritten).  Defined in cast_kernels.hip.
 int fold_colmax(const void *partials, int64_t slots, int64_t C, float *col_amax, hipStream_t st);
+// The same for up to kMaxFolds tensors in one launch.
+constexpr int kMaxFolds = 3;
+struct FoldOperand {
+  const void *partials;
+  float *col_amax;
+  int64_t slots, C;
+};
+int fold_colmax_many(const FoldOperand *ops, int n, hipStream_t st);
 
 // Looks up, for the current device, the address of the static scratch array of l8_cast_rowwise_noalloc.
 // Defined in cast_kernels.hip; l8_device_check calls it so that the look-up happens at set-up.

@@ -27,7 +27,7 @@ struct Library {
 #define L8_ENTRY(name) decltype(&::name) name = nullptr;
 #define L8_ENTRIES(X)                                                                                                        \
   X(l8_last_error) X(l8_linear_fwd_rows) X(l8_linear_fwd_rows_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
-  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_col_amax) X(l8_gemm_nt)
+  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_gemm_nt)
   L8_ENTRIES(L8_ENTRY)
 #undef L8_ENTRY
 } lib;
@@ -234,14 +234,20 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     if (need_b) {
       Tensor qgt, sgt;
-      cast_colwise_t(g, rg, g_col, qgt, sgt, stream);
-      if (!qat.defined()) {
+      if (qat.defined()) {
+        cast_colwise_t(g, rg, g_col, qgt, sgt, stream);
+      } else {
         Tensor a_col = a_col_in;
         if (!a_col.defined()) {
           a_col = at::empty({K}, o.dtype(at::kFloat));
           check(lib.l8_col_amax(ra.p, M, K, ra.ld, a_col.mutable_data_ptr<float>(), stream), "l8_col_amax");
         }
-        cast_colwise_t(g, ra, a_col, qat, sat, stream);
+        qgt = empty_fp8(N, padded, o), sgt = at::empty({N, 1}, o.dtype(at::kFloat));
+        qat = empty_fp8(K, padded, o), sat = at::empty({K, 1}, o.dtype(at::kFloat));
+        const l8_cast_transposed_item both[2] = {
+            {rg.p, M, N, rg.ld, g_col.const_data_ptr<float>(), nullptr, 0, qgt.mutable_data_ptr(), qgt.stride(0), padded, sgt.mutable_data_ptr<float>()},
+            {ra.p, M, K, ra.ld, a_col.const_data_ptr<float>(), nullptr, 0, qat.mutable_data_ptr(), qat.stride(0), padded, sat.mutable_data_ptr<float>()}};
+        check(lib.l8_cast_transposed_many(both, 2, stream), "l8_cast_transposed_many");
       }
       gb = at::empty({N, K}, o);
       check(lib.l8_gemm_nt(qgt.const_data_ptr(), qat.const_data_ptr(), N, K, padded, qgt.stride(0), qat.stride(0), sgt.const_data_ptr<float>(), L8_SCALE_ROW,

@@ -479,15 +479,14 @@ static int launch_bwd_wide(const void *dh, const void *h1, const void *h3, int64
     static bool done[kMaxDev] = {};
     uint16_t *w1 = (uint16_t *)ws, *w3 = w1 + blocks * C;
     const size_t lds = (size_t)C * 4;
-    int rc = allow_lds(swiglu_bwd_cast_rowwise_wide_kernel<true>, lds, done);
+    const int rc = allow_lds(swiglu_bwd_cast_rowwise_wide_kernel<true>, lds, done);
     if (rc != L8_OK) return rc;
     hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_wide_kernel<true>), dim3((unsigned)blocks), dim3(kWideBlock), lds, st,
                        (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,
                        (uint16_t *)g1, (uint16_t *)g3, ldg, (uint8_t *)q1, (uint8_t *)q3, ldq, s1, s3, w1, w3, l8::scale_rule());
     L8_HIP(hipGetLastError());
-    rc = fold_colmax(w1, blocks, C, ca1, st);
-    if (rc != L8_OK) return rc;
-    return fold_colmax(w3, blocks, C, ca3, st);
+    const FoldOperand both[2] = {{w1, ca1, blocks, C}, {w3, ca3, blocks, C}};
+    return fold_colmax_many(both, 2, st);
   }
   hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_wide_kernel<false>), dim3((unsigned)blocks), dim3(kWideBlock), 0, st,
                      (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,
@@ -535,9 +534,8 @@ static int launch_bwd(const void *dh, const void *h1, const void *h3, int64_t R,
                        (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,
                        (uint16_t *)g1, (uint16_t *)g3, ldg, (uint8_t *)q1, (uint8_t *)q3, ldq, s1, s3, w1, w3, l8::scale_rule());
     L8_HIP(hipGetLastError());
-    const int rc = fold_colmax(w1, blocks, C, ca1, st);
-    if (rc != L8_OK) return rc;
-    return fold_colmax(w3, blocks, C, ca3, st);
+    const FoldOperand both[2] = {{w1, ca1, blocks, C}, {w3, ca3, blocks, C}};
+    return fold_colmax_many(both, 2, st);
   }
   hipLaunchKernelGGL((swiglu_bwd_cast_rowwise_kernel<NCHW, false, WAVES>), dim3((unsigned)blocks), dim3(WAVES * 64), 0, st,
                      (const uint16_t *)dh, (const uint16_t *)h1, (const uint16_t *)h3, R, (int)C, lddh, ld1, ld3,

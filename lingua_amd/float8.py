@@ -296,6 +296,13 @@ def weight_cast_tensorwise_t(w, amax_rows):
     return _weight_casts.tensorwise_t(w, amax_rows)
 
 
+def weight_casts_tensorwise_t(ws, amaxes):
+    """``weight_cast_tensorwise_t`` of weights that are quantised together."""
+    if config.cache_weight_casts:
+        return [_weight_casts.tensorwise_t(w, amax) for w, amax in zip(ws, amaxes)]
+    return ops.cast_transposed_many(list(zip(ws, amaxes)), on_lines=True)
+
+
 def clear_cast_memos() -> None:
     """Forget the shared activation casts.  The memos trust the tensor's version counter, exactly as
     autograd's check of saved tensors does: every PyTorch in-place op and every ``out=`` write of
@@ -452,12 +459,10 @@ def input_cast_for_wgrad(a, a_col_amax, user):
 
 
 def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b: bool, need_bias: bool,
-                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None, grad_a=None, wgrad_later=None):
+                    fp8_wgrad: bool, gemm_algo: int, a_tcast=None, grad_a=None):
     """Backward of lingua/float8.py:99-131 (fp8 wgrad optional).  Returns ``(grad_a, grad_b, grad_bias)`` with
     ``None`` where not needed.  ``a_tcast`` = ``(qat [K,M], sat [K,1])`` made in forward stands in for ``a``
-    (then ``a`` may be None; fp8 wgrad only).  ``grad_a``: a gradient of ``a`` that this one is added to, in place.
-    ``wgrad_later``: a list that receives the operands ``(qgt, sgt, qat, sat)`` of the fp8 wgrad product in the place of
-    ``grad_b``, which then is ``None``."""
+    (then ``a`` may be None; fp8 wgrad only).  ``grad_a``: a gradient of ``a`` that this one is added to, in place."""
     if grad_out.dtype != torch.bfloat16:
         raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {grad_out.dtype}")
     fp8_wgrad = fp8_wgrad and need_b
@@ -466,7 +471,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
     if a is None and need_b and not (fp8_wgrad and a_tcast is not None):
         raise RuntimeError("Fp8LinearFn.backward: the bf16 input was not saved and no quantised copy stands in for it")
 
-    if (grad_a is None and wgrad_later is None and fp8_wgrad == need_b and _native_call(grad_out, gemm_algo) and
+    if (grad_a is None and fp8_wgrad == need_b and _native_call(grad_out, gemm_algo) and
             not torch.is_grad_enabled()):
         hit = w_cast = None
         if need_b and a_tcast is None and config.share_input_casts:
@@ -507,11 +512,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
                 qat, sat = ops.cast_colwise_transposed(a, a_col_amax, on_lines=True)
                 if config.share_input_casts:
                     _bwd_cast.put(a, (qat, sat), b_t.data_ptr())
-            if wgrad_later is not None:
-                wgrad_later.append((qgt, sgt, qat, sat))
-                grad_b = None
-            else:
-                grad_b = ops.gemm_nt(qgt, qat, sgt, sat, None, algo=gemm_algo)
+            grad_b = ops.gemm_nt(qgt, qat, sgt, sat, None, algo=gemm_algo)
         else:
             grad_b = grad_out.t() @ a
     else:
@@ -519,6 +520,43 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
 
     grad_bias = grad_out.sum(dim=0) if need_bias else None
     return grad_a, grad_b, grad_bias
+
+
+def shared_input_backward(grads, a, ws, amaxes, a_col_amax, need_a: bool, need_ws, gemm_algo: int):
+    """Backward of linears on one activation ``a`` without biases, fp8 weight gradients, as ``linear_backward`` of each in turn
+    computes it: ``(grad_a, [grad_w ...])``.  Casts of one kind share a launch, and so do the weight gradients."""
+    for g in grads:
+        if g.dtype != torch.bfloat16:
+            raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {g.dtype}")
+    _fwd_cast.clear(a)
+    _fwd_tcast.clear(a)
+    grad_a, cols = None, [None] * len(grads)
+    if need_a:
+        which = [i for i, need in enumerate(need_ws) if need]
+        quantised = dict(zip(which, ops.cast_rowwise_cols_many([grads[i] for i in which], on_lines=True))) if which else {}
+        for i, g in enumerate(grads):   # a gradient whose weight does not learn needs no column amaxes
+            if i not in quantised:
+                quantised[i] = (*ops.cast_rowwise(g, on_lines=True)[:2], None)
+        for i, (qwt, swt) in enumerate(weight_casts_tensorwise_t(ws, amaxes)):
+            qg, sg, cols[i] = quantised[i]
+            grad_a = ops.gemm_nt(qg, qwt, sg, swt, None, algo=gemm_algo, out=grad_a, add=grad_a is not None)
+        del quantised
+    learning = [i for i, need in enumerate(need_ws) if need]
+    grad_ws = [None] * len(grads)
+    if learning:
+        casts = [(grads[i], cols[i] if cols[i] is not None else ops.col_amax(grads[i])) for i in learning]
+        user = ws[learning[0]].data_ptr()
+        hit = _bwd_cast.get(a, user) if config.share_input_casts else None
+        if hit is None:
+            casts.append((a, a_col_amax if a_col_amax is not None else ops.col_amax(a)))
+        qts = ops.cast_transposed_many(casts, on_lines=True)
+        if hit is None:
+            hit = qts.pop()
+            if config.share_input_casts:
+                _bwd_cast.put(a, hit, user)
+        for i, gw in zip(learning, ops.gemm_nt_multi([q for q, _ in qts], hit[0], [s for _, s in qts], hit[1], algo=gemm_algo)):
+            grad_ws[i] = gw
+    return grad_a, grad_ws
 
 
 class Fp8LinearFn(torch.autograd.Function):

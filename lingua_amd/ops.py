@@ -182,6 +182,39 @@ def cast_rowwise_many(xs, out=None, on_lines: bool = False):
     return list(zip(qs, ss, amaxes))
 
 
+def cast_rowwise_cols_many(xs, on_lines: bool = False):
+    """``cast_rowwise`` with column amaxes of several tensors; the folds behind the casts share a launch.  Returns a list of
+    (q, scale, column amaxes) per tensor."""
+    if len(xs) == 1 or timed_singly("cast_rowwise"):
+        out = []
+        for x in xs:
+            col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device)
+            q, s, _ = cast_rowwise(x, col_amax=col, on_lines=on_lines)
+            out.append((q, s, col))
+        return out
+    xs = [_rows_2d(x, torch.bfloat16, "cast_rowwise_cols_many") for x in xs]
+    dev, lib = xs[0].device, _lib.load()
+    st = _prep(xs[0], "cast_rowwise_cols_many")
+    if any(x.device != dev for x in xs):
+        raise RuntimeError("cast_rowwise_cols_many: tensors on one device required")
+    out, items = [], []
+    with _timed("cast_rowwise_many", sum(x.shape[0] * (3 * x.shape[1] + 4) + 4 * x.shape[1] for x in xs), dev):
+        # (how much workspace depends on the device's compute units)
+        sizes = [lib.l8_cast_rowwise_workspace(*x.shape) for x in xs]
+        at = [sum((s + 255) // 256 * 256 for s in sizes[:i]) for i in range(len(xs))]
+        ws = torch.empty(at[-1] + sizes[-1] + 16, dtype=torch.uint8, device=dev)
+        base = ws.data_ptr()
+        for x, size, off in zip(xs, sizes, at):
+            R, C = x.shape
+            q, s = _empty_fp8(R, C, dev, on_lines), torch.empty((R, 1), dtype=torch.float32, device=dev)
+            col = torch.empty(C, dtype=torch.float32, device=dev)
+            out.append((q, s, col))
+            items += [x.data_ptr(), R, C, _ld(x), q.data_ptr(), _ld(q), s.data_ptr(), 0, col.data_ptr(), base + off, size]
+        code = lib.l8_cast_rowwise_cols_many(struct.pack(f"{len(items)}q", *items), len(xs), st)
+    _lib.check(code, "l8_cast_rowwise_cols_many")
+    return out
+
+
 AMAX_BF16, AMAX_F32 = 0, 1
 
 
@@ -298,6 +331,42 @@ def cast_colwise_transposed(x: torch.Tensor, col_amax_f32: torch.Tensor, pad_to:
                                                           q.data_ptr(), _ld(q), Rp, scale.data_ptr(), st)
     _lib.check(code, "l8_cast_colwise_transposed_pad")
     return q, scale
+
+
+def cast_transposed_many(casts, on_lines: bool = False):
+    """``cast_colwise_transposed(x, col_amax)`` and ``cast_tensorwise_t_rows(x, amax_rows)`` of several tensors, neighbours of
+    one kind in one launch.  ``casts``: (x, amaxes) pairs; fp32 amaxes are column amaxes, bf16 ones a weight's row amaxes.
+    Returns a list of (q, scale)."""
+    def one(x, amax):
+        return (cast_tensorwise_t_rows if amax.dtype == torch.bfloat16 else cast_colwise_transposed)(x, amax, on_lines=on_lines)
+
+    dev = casts[0][0].device
+    together = len(casts) > 1 and not timed_singly("cast_tensorwise_t", "cast_colwise_t")
+    for x, amax in casts:
+        n = amax.numel()
+        together = (together and x.dim() == 2 and x.numel() > 0 and x.device == dev == amax.device and amax.is_contiguous() and
+                    (amax.dtype == torch.float32 and n == x.shape[1] or amax.dtype == torch.bfloat16 and n % 8 == 0 and
+                     0 < n <= _MAX_AMAX_ROWS and amax.data_ptr() % 16 == 0))
+    if not together:
+        return [one(x, amax) for x, amax in casts]
+    st = _prep(casts[0][0], "cast_transposed_many")
+    out, items, work, keep = [], [], 0, []
+    for x, amax in casts:
+        x = _rows_2d(x, torch.bfloat16, "cast_transposed_many")
+        keep.append(x)
+        R, C = x.shape
+        rows = amax.dtype == torch.bfloat16
+        Rp = R if rows else (R + 15) // 16 * 16
+        q = _empty_fp8(C, Rp, dev, on_lines)
+        s = torch.empty((1 if rows else C, 1), dtype=torch.float32, device=dev)
+        out.append((q, s))
+        p = amax.data_ptr()
+        items += [x.data_ptr(), R, C, _ld(x), 0 if rows else p, p if rows else 0, amax.numel() if rows else 0, q.data_ptr(), _ld(q), Rp, s.data_ptr()]
+        work += R * C * 3
+    with _timed("cast_transposed_many", work, dev):
+        code = _lib.load().l8_cast_transposed_many(struct.pack(f"{len(items)}q", *items), len(casts), st)
+    _lib.check(code, "l8_cast_transposed_many")
+    return out
 
 
 # Tile configuration that may share the K range of the last round's tiles out (opt-in: measured neutral), and its

@@ -74,19 +74,17 @@ class Fp8QKVFn(torch.autograd.Function):
         saved = ctx.saved_tensors
         x, ws, amaxes = saved[0], saved[1:4], saved[4:7]
         x_col = saved[7] if ctx.has_col else None
-        gx, gws, later, which = None, [None, None, None], [], []
-        for i, g in enumerate(grads):
-            if g is None or not (ctx.need[0] or ctx.need[1 + i]):
-                continue
-            # the wgrads share the quantised x and wait for one launch
-            gx, gws[i], _ = f8.linear_backward(g.contiguous(), x, ws[i], amaxes[i], x_col, ctx.need[0], ctx.need[1 + i], False,
-                                               ctx.fp8_wgrad, ctx.gemm_algo, a_tcast=later[0][2:] if later else None, grad_a=gx,
-                                               wgrad_later=later)
-            which += [i] * (len(later) - len(which))
-        if later:
-            qgts, sgts, (qat, *_), (sat, *_) = zip(*later)
-            for i, gw in zip(which, ops.gemm_nt_multi(qgts, qat, sgts, sat, algo=ctx.gemm_algo)):
+        gx, gws = None, [None, None, None]
+        live = [i for i, g in enumerate(grads) if g is not None and (ctx.need[0] or ctx.need[1 + i])]
+        if ctx.fp8_wgrad and live:
+            gx, some = f8.shared_input_backward([grads[i].contiguous() for i in live], x, [ws[i] for i in live], [amaxes[i] for i in live],
+                                                x_col, ctx.need[0], [ctx.need[1 + i] for i in live], ctx.gemm_algo)
+            for i, gw in zip(live, some):
                 gws[i] = gw
+        else:
+            for i in live:
+                gx, gws[i], _ = f8.linear_backward(grads[i].contiguous(), x, ws[i], amaxes[i], x_col, ctx.need[0], ctx.need[1 + i], False,
+                                                   ctx.fp8_wgrad, ctx.gemm_algo, grad_a=gx)
         return (gx, *gws)
 
 

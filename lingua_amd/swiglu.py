@@ -101,27 +101,19 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         g1, g3, qg1, qg3, sg1, sg3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, g1_col, g3_col, on_lines=True)
         del dh
         if need_x:
-            qw1t, sw1t = f8.weight_cast_tensorwise_t(w1, amax_w1)
+            (qw1t, sw1t), (qw3t, sw3t) = f8.weight_casts_tensorwise_t((w1, w3), (amax_w1, amax_w3))
             gx = ops.gemm_nt(qg1, qw1t, sg1, sw1t, None, algo=algo)
-            qw3t, sw3t = f8.weight_cast_tensorwise_t(w3, amax_w3)
             ops.gemm_nt(qg3, qw3t, sg3, sw3t, None, algo=algo, out=gx, add=True)
         del qg1, qg3
         if need_w1 or need_w3:
             if fp8_wgrad:
                 if x_col is None:
                     x_col = ops.col_amax(x)
-                qxt, sxt = ops.cast_colwise_transposed(x, x_col, on_lines=True)   # shared by both wgrads
-                if need_w1 and need_w3:
-                    q1, s1 = ops.cast_colwise_transposed(g1, g1_col, on_lines=True)
-                    del g1
-                    q3, s3 = ops.cast_colwise_transposed(g3, g3_col, on_lines=True)
-                    gw1, gw3 = ops.gemm_nt_multi((q1, q3), qxt, (s1, s3), sxt, algo=algo)
-                elif need_w1:
-                    qgt, sgt = ops.cast_colwise_transposed(g1, g1_col, on_lines=True)
-                    gw1 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
-                else:
-                    qgt, sgt = ops.cast_colwise_transposed(g3, g3_col, on_lines=True)
-                    gw3 = ops.gemm_nt(qgt, qxt, sgt, sxt, None, algo=algo)
+                wanted = [(g, col) for g, col, need in ((g1, g1_col, need_w1), (g3, g3_col, need_w3)) if need]
+                (qxt, sxt), *qgs = ops.cast_transposed_many([(x, x_col)] + wanted, on_lines=True)   # x for both wgrads
+                del g1, g3, wanted
+                gws = iter(ops.gemm_nt_multi([q for q, _ in qgs], qxt, [s for _, s in qgs], sxt, algo=algo))
+                gw1, gw3 = (next(gws) if need else None for need in (need_w1, need_w3))
             else:
                 gw1 = g1.t() @ x if need_w1 else None
                 gw3 = g3.t() @ x if need_w3 else None
@@ -136,8 +128,7 @@ def _wgrad(g, g_col, a, a_col, fp8_wgrad, algo):
         g_col = ops.col_amax(g)
     if a_col is None:
         a_col = ops.col_amax(a)
-    qgt, sgt = ops.cast_colwise_transposed(g, g_col, on_lines=True)
-    qat, sat = ops.cast_colwise_transposed(a, a_col, on_lines=True)
+    (qgt, sgt), (qat, sat) = ops.cast_transposed_many([(g, g_col), (a, a_col)], on_lines=True)
     return ops.gemm_nt(qgt, qat, sgt, sat, None, algo=algo)
 
 

@@ -509,3 +509,47 @@ def test_rows_on_lines_hold_what_dense_rows_hold(R, C):
         y = torch.empty_like(want)
         ops.linear_fwd(x, w, None, y, x_cast=x_cast, x_ready=True, w_cast=w_cast, w_ready=True)
         assert torch.equal(bits(y), bits(want))
+
+
+def _many_inputs(shapes, seed):
+    """Odd sizes, one with a row stride, one with an infinity and a NaN."""
+    xs = []
+    for i, (R, C) in enumerate(shapes):
+        wide = seeded_bf16((R, C + 8), seed=seed + i).cuda()
+        xs.append(wide[:, :C] if i == 1 else wide[:, :C].contiguous())
+    xs[0][0, 0], xs[0][-1, -1] = float("inf"), float("nan")
+    return xs
+
+
+@pytest.mark.parametrize("shapes", [[(33, 144), (257, 16), (1, 8)], [(130, 2056), (130, 520), (130, 520), (130, 2056)],
+                                    [(1021, 1040)] * 5, [(520, 4112), (516, 8200)], [(16400, 8200), (16384, 8192)]])
+def test_several_transposed_casts_in_one_launch_equal_single_ones(shapes):
+    """Column-wise ones of several widths and heights (more than a launch takes; small, ordinary and large tiles), then
+    tensor-wise ones with their row amaxes, then both kinds mixed; bytes, scales and the zero padding."""
+    from lingua_amd import ops
+    xs = _many_inputs(shapes, 31)
+    cols = [ops.col_amax(x) for x in xs]
+
+    def compare(casts, want):
+        for (q, s), (wq, ws) in zip(ops.cast_transposed_many(casts), want):
+            assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(s.view(torch.int32), ws.view(torch.int32))
+
+    compare(list(zip(xs, cols)), [ops.cast_colwise_transposed(x, c) for x, c in zip(xs, cols)])
+    ws = [x[:x.shape[0] // 8 * 8] for x in xs if x.shape[0] >= 8]
+    amaxes = [ops.cast_rowwise(w)[2] for w in ws]
+    compare(list(zip(ws, amaxes)), [ops.cast_tensorwise_t_rows(w, a) for w, a in zip(ws, amaxes)])
+    compare([(xs[0], cols[0]), (ws[0], amaxes[0]), (ws[-1], amaxes[-1]), (xs[1], cols[1])],
+            [ops.cast_colwise_transposed(xs[0], cols[0]), ops.cast_tensorwise_t_rows(ws[0], amaxes[0]),
+             ops.cast_tensorwise_t_rows(ws[-1], amaxes[-1]), ops.cast_colwise_transposed(xs[1], cols[1])])
+
+
+@pytest.mark.parametrize("shapes", [[(33, 144), (257, 16)], [(1, 8), (2, 2048), (700, 2056), (64, 4104)], [(40, 33024), (3, 64), (5, 24)]])
+def test_several_row_casts_with_column_amaxes_equal_single_ones(shapes):
+    """Folds of different widths and lengths in one launch, more than a launch takes, and rows that leave nothing to fold."""
+    from lingua_amd import ops
+    xs = _many_inputs(shapes, 47)
+    for x, (q, s, col) in zip(xs, ops.cast_rowwise_cols_many(xs)):
+        want = torch.full((x.shape[1],), -1.0, device="cuda")
+        wq, ws, _ = ops.cast_rowwise(x, col_amax=want)
+        assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(s.view(torch.int32), ws.view(torch.int32))
+        assert torch.equal(col.view(torch.int32), want.view(torch.int32))
