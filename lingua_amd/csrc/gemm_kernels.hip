@@ -157,6 +157,24 @@ L8_DEV v4i add_bf16x8(v4i a, v4i b) {
 #define L8_WAIT_VM_LGKM0(n) \
   __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (0x7 << 4) | (0x0 << 8) | ((((n) >> 4) & 0x3) << 14))
 
+// R > 5, the small tiles: the deep form of the main loop.  The fragments of a whole K tile are in registers before its trip
+// begins, read during the trip before; a slot is given away one trip later than above, when the MFMAs that used it have been
+// issued, so that no wave waits for LDS at the barrier; and the ring holds as many whole K tiles as fit.  us, before (nine
+// slots of one panel) / now: [2048,16384].[2048,16384] 65.3 / 60.2, [700,11008].[4096,11008] 40.7 / 37.7, [512,4096].[4096,4096]
+// 15.0 / 13.9, [493,6784].[4832,6784] 26.8 / 24.8, [1021,2048].[2048,2048] 9.8 / 9.4, [333,2048].[8192,2048] 12.0 / 11.5.  What
+// bounds them now is the way from the L2 to LDS: 33 to 38 bytes per clock and unit with every one of these tiles (and with
+// the half tiles below), whatever the depth; touching the L2 two to ten K tiles ahead cost a tenth and gained nothing.
+//
+// s_waitcnt for vmcnt <= n alone
+#define L8_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (0x7 << 4) | (0xF << 8) | ((((n) >> 4) & 0x3) << 14))
+
+// Whole K tiles of a BM x BN problem that the LDS holds for each of KS groups of waves (six are enough).
+constexpr int deep_slots(int bm, int bn, int ks) {
+  const int n = 160 * 1024 / (ks * (bm + bn) * 128);
+  return n < 6 ? n : 6;
+}
+constexpr int plain_lds(int bm, int bn, int r, int ks) { return ks * (r > 5 ? deep_slots(bm, bn, ks) * (bm + bn) : r * (bm > bn ? bm : bn)) * 128; }
+
 // KS > 1: KS groups of WM x WN waves, each with a ring of its own, take K tiles in turn (group g the tiles g, g + KS, ..)
 // and add their accumulators at the end, in the order of the groups.
 template <int WM, int WN, int TM, int TN, int R, int GROUP_M, int PF, int KS = 1>
@@ -166,6 +184,8 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   constexpr int NW = WM * WN;
   constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;
   constexpr int UNIT = A_BYTES > B_BYTES ? A_BYTES : B_BYTES;  // one ring slot holds an A or a B panel of one K tile
+  constexpr bool DEEP = R > 5;
+  constexpr int NS = deep_slots(BM, BN, KS), RING = DEEP ? NS * (A_BYTES + B_BYTES) : R * UNIT;  // of one group of waves
   static_assert((BM / 8) % NW == 0 && (BN / 8) % NW == 0, "tile rows must split evenly over waves");
   constexpr int NA = BM / 8 / NW, NB = BN / 8 / NW;  // 1 KiB wave loads (8 rows x 128 B) per panel per wave
   // L2 touches (PF > 0): one lane per panel row, every wave covers 64 rows per instruction
@@ -247,7 +267,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   const int chunk_even = (lpos ^ lrow) * 16, chunk_odd = (lpos ^ lrow ^ 1) * 16;  // byte offset in the row, by parity of g
 
   const int KT = (p.K + BK * KS - 1) / (BK * KS);  // trips
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem + group * (R * UNIT);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem + group * RING;
   auto wrap = [](int slot) { return slot >= R ? slot - R : slot; };  // slot in [0, 2R)
   // Units are issued in the order A(0), B(0), A(1), B(1), ...; unit u lives in
   // ring slot u % R (the callers keep the slot numbers as running scalars).
@@ -255,13 +275,13 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   // uniform; K tiles at or beyond the end, rows beyond M / N and chunks beyond
   // K use an out-of-range offset, which the buffer unit turns into zeros in LDS.
   // load_one: i-th vector-memory instruction (of IA or IB) of the unit of K
-  // tile kt (A or B panel) into ring slot `slot`: first the L2 touches, then
+  // tile kt (A or B panel) to LDS offset `at`: first the L2 touches, then
   // the 1 KiB panel loads.
-  auto load_one = [&](bool is_b, int kt, int slot, int i) {
+  auto load_one = [&](bool is_b, int kt, int at, int i) {
     const int k0 = (kt * KS + group) * BK;
     const uint32_t m_even = (k0 + chunk_even < p.K) ? 0u : kOOB, m_odd = (k0 + chunk_odd < p.K) ? 0u : kOOB;
     if (!is_b) {
-      const uint32_t dst = lds0 + slot * UNIT + wave * (NA * 1024);
+      const uint32_t dst = lds0 + at + wave * (NA * 1024);
       // a touched dword lands in this wave's own part of the slot and is
       // overwritten by the panel loads that follow (a wave's loads return in order)
       if (i < PFA)
@@ -272,7 +292,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
                                                  a_voff[(i - PFA) & 1] | (((i - PFA) & 1) ? m_odd : m_even),
                                                  k0 + a_srow + (i - PFA) * a_lda8, 0, 0);
     } else {
-      const uint32_t dst = lds0 + slot * UNIT + wave * (NB * 1024);
+      const uint32_t dst = lds0 + at + wave * (NB * 1024);
       if (i < PFB)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsB, reinterpret_cast<lds_ptr_t>(dst), 4,
                                                  pfb_voff[i < PFB ? i : 0] | ((k0 + PF * KS * BK < p.K) ? 0u : kOOB), k0 + PF * KS * BK, 0, 0);
@@ -295,12 +315,12 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   const int b_base = wn * (TN * 32 * BK);
 
   // LDS addresses of the two 16-byte pieces a lane reads of its row, for step s
-  // of the K tile whose panels sit in slots slot_a / slot_b.  The additions are
+  // of the K tile whose panels sit at LDS offsets at_a / at_b.  The additions are
   // opaque to the compiler on purpose: it would otherwise keep a register per
   // (slot, piece) combination alive across the loop.
   typedef const __attribute__((address_space(3))) v4i *lds_v4i_ptr;
-  auto frag_addrs = [&](int slot_a, int slot_b, int s, uint32_t (&ad)[4]) {
-    const uint32_t sa = lds0 + slot_a * UNIT + a_base, sb = lds0 + slot_b * UNIT + b_base;
+  auto frag_addrs = [&](int at_a, int at_b, int s, uint32_t (&ad)[4]) {
+    const uint32_t sa = lds0 + at_a + a_base, sb = lds0 + at_b + b_base;
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[0]) : "s"(sa), "v"(foff[s][0]));
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[1]) : "s"(sa), "v"(foff[s][1]));
     asm volatile("v_add_u32 %0, %1, %2" : "=v"(ad[2]) : "s"(sb), "v"(foff[s][0]));
@@ -337,10 +357,75 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   // of them after the barrier would keep the waves queueing at the
   // vector-memory port instead of issuing MFMAs.
   //   prologue: units 0 .. R-2 in flight, K tile 0 published, its first half read
+  if constexpr (DEEP) {
+    // Trip kt: K tile kt + 1 has landed for every wave behind the barrier (a partial wait for its own loads in front of it);
+    // MFMAs on K tile kt, whose fragments were requested in the trip before, beside the reads of kt + 1 and the loads of
+    // kt + NS - 1, which go where kt - 1 was: every wave has issued the MFMAs of kt - 1, so its reads are done.
+    constexpr int KTILE = A_BYTES + B_BYTES, LOADS = IA + IB, N_MMA = 2 * TM * TN, N_RD = 4 * (TM + TN);
+    constexpr int PEND_D = (NS - 3) * LOADS;
+    static_assert(NS >= 4 && (NS - 2) * LOADS <= 63, "vmcnt is a 6-bit counter");
+    struct Frags { v8i a[2][TM], b[2][TN]; };
+    auto slot_after = [](int slot, int n) { return slot + n >= NS ? slot + n - NS : slot + n; };
+    auto load_tile_part = [&](int kt, int slot, int j) {
+      if (j < IA) load_one(false, kt, slot * KTILE, j);
+      else load_one(true, kt, slot * KTILE + A_BYTES, j - IA);
+    };
+    // piece r of a K tile's fragments: step by step, in the order the MFMAs need them
+    auto read_part = [&](const uint32_t (&ad)[2][4], Frags &f, int r) __attribute__((always_inline)) {
+      const int step = r / (2 * (TM + TN)), q = (r % (2 * (TM + TN))) >> 1, h = r & 1;
+      const bool is_b = q == 0 || q > TM;
+      const int t = q == 0 ? 0 : (q > TM ? q - TM : q - 1);
+      const v4i v = *reinterpret_cast<lds_v4i_ptr>(ad[step][(is_b ? 2 : 0) + h] + t * (32 * BK));
+      v8i &d = is_b ? f.b[step][t] : f.a[step][t];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) d[h * 4 + k] = v[k];
+    };
+    Frags f0, f1;
+    uint32_t ad[2][4];
+#pragma unroll
+    for (int u = 0; u < NS - 1; ++u)
+#pragma unroll
+      for (int j = 0; j < LOADS; ++j) load_tile_part(u, u, j);
+    L8_WAIT_VM((NS - 2) * LOADS);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    frag_addrs(0, A_BYTES, 0, ad[0]);
+    frag_addrs(0, A_BYTES, 1, ad[1]);
+#pragma unroll
+    for (int r = 0; r < N_RD; ++r) read_part(ad, f0, r);
+    int slot = 0;  // of K tile kt
+    auto trip = [&](int kt, Frags &cur, Frags &nxt) __attribute__((always_inline)) {
+      L8_WAIT_VM(PEND_D);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      const int next = slot_after(slot, 1), free = slot_after(slot, NS - 1);
+      frag_addrs(next * KTILE, next * KTILE + A_BYTES, 0, ad[0]);
+      frag_addrs(next * KTILE, next * KTILE + A_BYTES, 1, ad[1]);
+#pragma unroll
+      for (int i = 0; i < N_MMA; ++i) {
+        mma_one(cur.a[i / (TM * TN)], cur.b[i / (TM * TN)], i % (TM * TN));
+#pragma unroll
+        for (int r = (N_RD * i) / N_MMA; r < (N_RD * (i + 1)) / N_MMA; ++r) read_part(ad, nxt, r);
+#pragma unroll
+        for (int j = (LOADS * i) / N_MMA; j < (LOADS * (i + 1)) / N_MMA; ++j) load_tile_part(kt + NS - 1, free, j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      slot = next;
+    };
+    int kt = 0;
+#pragma unroll 1
+    for (; kt + 2 <= KT; kt += 2) {
+      trip(kt, f0, f1);
+      trip(kt + 1, f1, f0);
+    }
+    if (kt < KT) trip(kt, f0, f1);
+  } else {
 #pragma unroll
   for (int u = 0; u < R - 1; ++u) {
 #pragma unroll
-    for (int i = 0; i < ((u & 1) ? IB : IA); ++i) load_one(u & 1, u >> 1, u, i);
+    for (int i = 0; i < ((u & 1) ? IB : IA); ++i) load_one(u & 1, u >> 1, u * UNIT, i);
   }
   v8i af0[TM], bf0[TN], af1[TM], bf1[TN];
   uint32_t ad[4];
@@ -348,7 +433,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  frag_addrs(0, 1, 0, ad);
+  frag_addrs(0, UNIT, 0, ad);
 #pragma unroll
   for (int f = 0; f < TM + TN; ++f) read_one(ad, af0, bf0, f);
 
@@ -372,7 +457,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   int s0 = 0;  // ring slot of unit 2kt
   for (int kt = 0; kt < KT; ++kt) {
     const int slot_u1 = wrap(s0 + R - 1);  // unit 2kt+R-1 reuses the slot of unit 2kt-1
-    frag_addrs(s0, wrap(s0 + 1), 1, ad);
+    frag_addrs(s0 * UNIT, wrap(s0 + 1) * UNIT, 1, ad);
 #pragma unroll
     for (int i = 0; i < S1; ++i) {
       if (L8_GEMM_DIAG != 2 && L8_GEMM_DIAG != 4) {
@@ -382,7 +467,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
       }
       if (L8_GEMM_DIAG != 1) {
 #pragma unroll
-        for (int j = (I1 * i) / S1; j < (I1 * (i + 1)) / S1; ++j) load_one(U1_IS_B, kt + (R - 1) / 2, slot_u1, j);
+        for (int j = (I1 * i) / S1; j < (I1 * (i + 1)) / S1; ++j) load_one(U1_IS_B, kt + (R - 1) / 2, slot_u1 * UNIT, j);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -392,7 +477,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
     asm volatile("" ::: "memory");
     // the last MFMAs of the first half are issued after the barrier: they need
     // registers only and keep the matrix cores busy while the waves regroup
-    frag_addrs(wrap(s0 + 2), wrap(s0 + 3), 0, ad);
+    frag_addrs(wrap(s0 + 2) * UNIT, wrap(s0 + 3) * UNIT, 0, ad);
 #pragma unroll
     for (int i = 0; i < S2; ++i) {
       if (L8_GEMM_DIAG != 2 && L8_GEMM_DIAG != 4) {
@@ -405,11 +490,12 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
       }
       if (L8_GEMM_DIAG != 1) {
 #pragma unroll
-        for (int j = (I2 * i) / S2; j < (I2 * (i + 1)) / S2; ++j) load_one(U2_IS_B, kt + R / 2, s0, j);
+        for (int j = (I2 * i) / S2; j < (I2 * (i + 1)) / S2; ++j) load_one(U2_IS_B, kt + R / 2, s0 * UNIT, j);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
     s0 = wrap(s0 + 2);
+  }
   }
   // ---- epilogue ----
   // All scales of this wave's part of the tile are requested in one batch,
@@ -445,7 +531,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   __builtin_amdgcn_s_barrier();
   if constexpr (KS > 1) {
     // every group's ring is idle: the others leave their sums in theirs, the first group adds them to its own
-    static_assert(BM * BN * 4 <= R * UNIT, "a group's sums must fit in its ring");
+    static_assert(BM * BN * 4 <= RING, "a group's sums must fit in its ring");
     typedef __attribute__((address_space(3))) v4f *lds_v4f_ptr;
     constexpr int PIECE = NW * 64 * 16;
     const uint32_t mine = lds0 + (wave * 64 + lane) * 16;
@@ -472,7 +558,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
           for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
             for (int qd = 0; qd < 4; ++qd) {
-              const v4f t = *reinterpret_cast<lds_v4f_ptr>(mine + g * (R * UNIT) + ((tn * TM + tm) * 4 + qd) * PIECE);
+              const v4f t = *reinterpret_cast<lds_v4f_ptr>(mine + g * RING + ((tn * TM + tm) * 4 + qd) * PIECE);
 #pragma unroll
               for (int e = 0; e < 4; ++e) acc[tn][tm][qd * 4 + e] += t[e];
             }
@@ -488,7 +574,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   // leaves as whole rows: one store instruction covers 1 KiB of consecutive
   // bytes of C per row pair.
   constexpr int C_ROW = BN * 2 + 16;  // staged row pitch in bytes
-  static_assert(BM * C_ROW <= R * UNIT, "the C tile must fit in the ring");
+  static_assert(BM * C_ROW <= KS * RING, "the C tile must fit in the ring");
   typedef __attribute__((address_space(3))) v4i *lds_v4i_wptr;
   auto convert_and_stage = [&](auto has_bias) {
     constexpr bool HAS_BIAS = decltype(has_bias)::value;
@@ -1335,14 +1421,13 @@ L8_SMALL_ALGO_LIST(L8_INSTANTIATE)
   template __global__ void gemm_nt_kernel<WM, WN, TM, TN, R, GM, 0, KS>(const GemmArgs);
 L8_SPLIT_ALGO_LIST(L8_SPLIT_INSTANTIATE)
 
-#define L8_MAX2(a, b) ((a) > (b) ? (a) : (b))
 #define L8_ALGO_ROW(WM, WN, TM, TN, R, GM, PF)                                                                \
   {"mt" #WM "x" #WN "w_" #TM "x" #TN "t_r" #R "_g" #GM "_pf" #PF, gemm_nt_kernel<WM, WN, TM, TN, R, GM, PF>, \
-   WM * TM * 32, WN * TN * 32, WM * WN * 64, R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr, nullptr},
+   WM * TM * 32, WN * TN * 32, WM * WN * 64, plain_lds(WM * TM * 32, WN * TN * 32, R, 1), false, nullptr, nullptr, nullptr},
 
 #define L8_SPLIT_ALGO_ROW(WM, WN, TM, TN, R, GM, KS)                                                               \
   {"mt" #WM "x" #WN "w_" #TM "x" #TN "t_r" #R "_g" #GM "_ks" #KS, gemm_nt_kernel<WM, WN, TM, TN, R, GM, 0, KS>, \
-   WM * TM * 32, WN * TN * 32, WM * WN * KS * 64, KS * R * L8_MAX2(WM * TM * 32, WN * TN * 32) * 128, false, nullptr, nullptr, nullptr},
+   WM * TM * 32, WN * TN * 32, WM * WN * KS * 64, plain_lds(WM * TM * 32, WN * TN * 32, R, KS), false, nullptr, nullptr, nullptr},
 
 template __global__ void gemm_nt_stream_kernel<8, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<8, true>(const GemmArgs);
