@@ -293,6 +293,10 @@ int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int w_is_f32, c
                    int64_t R, int64_t C, int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, float *gw,
                    void *workspace, int64_t workspace_bytes, void *stream);
 int64_t l8_rmsnorm_bwd_workspace(int64_t R, int64_t C);
+/* The same with gw in fp32 (gw_is_f32) or rounded to bf16, as autograd hands it to a bf16 weight. */
+int l8_rmsnorm_bwd_as(const void *gy, const void *x, const void *w, int w_is_f32, const float *rstd,
+                      int64_t R, int64_t C, int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, void *gw, int gw_is_f32,
+                      void *workspace, int64_t workspace_bytes, void *stream);
 
 int l8_gemm_algo_count(void);
 /* human-readable description of tile configuration `algo` (1-based), or NULL */

@@ -54,6 +54,7 @@ SIGNATURES = {
     "l8_rmsnorm_workspace": [_i64, _i64],
     "l8_rmsnorm_bwd": [_p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _p, _i64, _p],
     "l8_rmsnorm_bwd_workspace": [_i64, _i64],
+    "l8_rmsnorm_bwd_as": [_p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _int, _p, _i64, _p],
     "l8_linear_fwd": [ctypes.c_char_p],
     "l8_linear_fwd_workspace": [ctypes.c_char_p],
     "l8_linear_fwd_rows": [ctypes.c_char_p, _i64, _i64],

@@ -381,9 +381,10 @@ __global__ __launch_bounds__(kNormBlock, 2) void rmsnorm_bwd_kernel(
 // A workgroup owns 32 columns -- one 128-byte line of every partial row -- and passes them through LDS, 256 rows at a
 // time: 16 bytes per thread and load, the next 256 rows in flight under the additions, which come one after the other
 // but read LDS.  (With each addition waiting for its row from memory the fold of 512 rows of 2048 columns took 20 us.)
+// gw leaves as fp32 or, for a bf16 weight, rounded: a conversion of its own was a launch of 4 to 5 us for a few KiB.
 constexpr int kGwCols = 32, kGwThreads = 1024, kGwRows = 256, kGwSums = 8;
 __global__ __launch_bounds__(kGwThreads) void rmsnorm_gw_fold_kernel(const float *__restrict__ partials, int n_slots, int C,
-                                                                     float *__restrict__ gw) {
+                                                                     void *__restrict__ gw, int gw_f32) {
   constexpr int QUADS = kGwCols / 4, STEP = kGwThreads / QUADS, LOADS = kGwRows / STEP;  // threads to a row, rows to a load
   __shared__ v4f rows[kGwRows][QUADS];
   __shared__ float sums[kGwSums][kGwCols];
@@ -419,7 +420,8 @@ __global__ __launch_bounds__(kGwThreads) void rmsnorm_gw_fold_kernel(const float
     float t = sums[0][tx];
 #pragma unroll
     for (int k = 1; k < kGwSums; ++k) t += sums[k][tx];
-    gw[c] = t;
+    if (gw_f32) ((float *)gw)[c] = t;
+    else ((uint16_t *)gw)[c] = (uint16_t)bf16_rne_bits(t);
   }
 }
 
@@ -466,13 +468,13 @@ static int launch_norm(const void *x, const void *w, int64_t R, int64_t C, int64
 
 template <int N, bool W_F32>
 static int launch_norm_bwd(const void *gy, const void *x, const void *w, const float *rstd, int64_t R, int64_t C,
-                           int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, float *gw, void *ws, hipStream_t st) {
+                           int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, void *gw, int gw_f32, void *ws, hipStream_t st) {
   const int64_t blocks = norm_blocks(R);
   hipLaunchKernelGGL((rmsnorm_bwd_kernel<N, N == 1 ? 4 : 2, W_F32>), dim3((unsigned)blocks), dim3(kNormBlock), 0, st, (const uint16_t *)gy,
                      (const uint16_t *)x, w, rstd, R, (int)C, ldg, ldx, (uint16_t *)gx, ldgx, (float *)ws);
   L8_HIP(hipGetLastError());
   hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + kGwCols - 1) / kGwCols)), dim3(kGwThreads), 0, st,
-                     (const float *)ws, (int)blocks, (int)C, gw);
+                     (const float *)ws, (int)blocks, (int)C, gw, gw_f32);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
@@ -489,12 +491,18 @@ extern "C" int64_t l8_rmsnorm_bwd_workspace(int64_t R, int64_t C) {
 extern "C" int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int w_is_f32, const float *rstd, int64_t R,
                               int64_t C, int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, float *gw, void *workspace,
                               int64_t workspace_bytes, void *stream) {
+  return l8_rmsnorm_bwd_as(gy, x, w, w_is_f32, rstd, R, C, ldg, ldx, gx, ldgx, gw, 1, workspace, workspace_bytes, stream);
+}
+
+extern "C" int l8_rmsnorm_bwd_as(const void *gy, const void *x, const void *w, int w_is_f32, const float *rstd, int64_t R,
+                                 int64_t C, int64_t ldg, int64_t ldx, void *gx, int64_t ldgx, void *gw, int gw_is_f32, void *workspace,
+                                 int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_rmsnorm_bwd: negative shape R=%lld C=%lld", (long long)R, (long long)C);
   if (C == 0) return L8_OK;
   L8_REQUIRE(gw, "l8_rmsnorm_bwd: null pointer");
   if (R == 0) {  // no rows: gw = 0, written by the fold kernel over zero partial rows
     hipLaunchKernelGGL(rmsnorm_gw_fold_kernel, dim3((unsigned)((C + kGwCols - 1) / kGwCols)), dim3(kGwThreads), 0, (hipStream_t)stream,
-                       (const float *)nullptr, 0, (int)C, gw);
+                       (const float *)nullptr, 0, (int)C, gw, gw_is_f32);
     L8_HIP(hipGetLastError());
     return L8_OK;
   }
@@ -509,8 +517,8 @@ extern "C" int l8_rmsnorm_bwd(const void *gy, const void *x, const void *w, int 
              "l8_rmsnorm_bwd: needs a 16-byte aligned workspace of %lld bytes", (long long)need);
   hipStream_t st = (hipStream_t)stream;
 #define L8_NORM_BWD(N)                                                                                               \
-  return w_is_f32 ? launch_norm_bwd<N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)             \
-                  : launch_norm_bwd<N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, workspace, st)
+  return w_is_f32 ? launch_norm_bwd<N, true>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, gw_is_f32, workspace, st)  \
+                  : launch_norm_bwd<N, false>(gy, x, w, rstd, R, C, ldg, ldx, gx, ldgx, gw, gw_is_f32, workspace, st)
   const int64_t nchw = ((C + 511) / 512 + kNormWaves - 1) / kNormWaves;
   if (nchw <= 1) L8_NORM_BWD(1);
   if (nchw <= 2) L8_NORM_BWD(2);

@@ -38,9 +38,9 @@ class Fp8RMSNormFn(torch.autograd.Function):
         x2d, weight, rstd = ctx.saved_tensors
         if gy.dtype != torch.bfloat16:
             raise RuntimeError(f"Fp8RMSNorm.backward: bf16 grad_out required, got {gy.dtype}")
-        gx2d, gw = ops.rmsnorm_bwd(gy.flatten(end_dim=-2), x2d, weight, rstd)
+        gx2d, gw = ops.rmsnorm_bwd(gy.flatten(end_dim=-2), x2d, weight, rstd, gw_dtype=weight.dtype)
         gx = gx2d.reshape(ctx.x_shape) if ctx.needs_input_grad[0] else None
-        return gx, (gw.to(weight.dtype) if ctx.needs_input_grad[1] else None), None, None
+        return gx, (gw if ctx.needs_input_grad[1] else None), None, None
 
 
 class Fp8RMSNorm(torch.nn.Module):

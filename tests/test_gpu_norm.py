@@ -308,3 +308,17 @@ def test_fused_feed_forward_takes_the_norm_output_already_quantised():
 def test_norm_cast_under_the_gpu_division_rule(gpu_division_rule):
     for shape in [(5, 264), (300, 1000), (17, 4096), (9, 8192)]:
         test_norm_and_cast(shape, torch.bfloat16, True)
+
+
+@pytest.mark.parametrize("R,C", [(0, 64), (1, 8), (700, 2056), (1025, 2048), (33, 8192)])
+def test_weight_gradient_rounded_by_the_fold_is_the_fp32_one_rounded(R, C):
+    """bf16 from the fold kernel has the bits of a conversion of its fp32 result: no rows, fewer and more of them than
+    workgroups, columns that do not fill a workgroup."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(R + C)
+    gy, x = ((torch.randn(R, C, generator=g)).to(torch.bfloat16).cuda() for _ in range(2))
+    w, rstd = torch.rand(C, generator=g).to(torch.bfloat16).cuda(), torch.rand(R, 1, generator=g).cuda()
+    gx32, gw32 = ops.rmsnorm_bwd(gy, x, w, rstd)
+    gx16, gw16 = ops.rmsnorm_bwd(gy, x, w, rstd, gw_dtype=torch.bfloat16)
+    assert gw32.dtype == torch.float32 and torch.equal(gx32.view(torch.int16), gx16.view(torch.int16))
+    assert torch.equal(gw32.to(torch.bfloat16).view(torch.int16), gw16.view(torch.int16))
