@@ -136,6 +136,12 @@ int l8_cast_rowwise_given_amax(const void *x, int64_t R, int64_t C, int64_t ldx,
 /* Column amax on its own: col_amax fp32 [C] is overwritten, as above. */
 int l8_col_amax(const void *x, int64_t R, int64_t C, int64_t ldx, float *col_amax, void *stream);
 
+/* Column sums: out bf16 [C] = bf16(sum over the rows of f32(x)), x bf16 [R,C] (ldx): the bias gradient (lingua/float8.py:127).
+ * Summed in fp32 in an order that depends on the shape and the device's compute units.  Requires C % 8 == 0, ldx % 8 == 0, x
+ * 16-byte aligned and a workspace of l8_col_sum_workspace(R, C) bytes. */
+int64_t l8_col_sum_workspace(int64_t R, int64_t C);
+int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void *out, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* bf16 amax[n] -> bf16 amax_out[1] = max, NaN propagating.
  * Replaces lingua/float8.py:115 (tensor amax of the weight from the row
  * amaxes saved by forward). */

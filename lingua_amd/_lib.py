@@ -32,6 +32,8 @@ SIGNATURES = {
     "l8_cast_rowwise_noalloc": [_p, _i64, _i64, _i64, _p, _i64, _p, _p, _p, _p],
     "l8_cast_rowwise_given_amax": [_p, _i64, _i64, _i64, _p, _int, _p, _i64, _p, _p],
     "l8_col_amax": [_p, _i64, _i64, _i64, _p, _p],
+    "l8_col_sum": [_p, _i64, _i64, _i64, _p, _p, _i64, _p],
+    "l8_col_sum_workspace": [_i64, _i64],
     "l8_amax_reduce": [_p, _i64, _p, _p],
     "l8_cast_tensorwise": [_p, _i64, _i64, _i64, _p, _int, _int, _p, _i64, _p, _p],
     "l8_cast_tensorwise_t_rows": [_p, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p],
@@ -65,7 +67,7 @@ SIGNATURES = {
 }
 _RETURNS_STR = {"l8_last_error", "l8_gemm_algo_name"}
 _RETURNS_I64 = {"l8_cast_rowwise_workspace", "l8_gemm_workspace", "l8_gemm_workspace_gave_up_offset", "l8_swiglu_workspace", "l8_rmsnorm_workspace", "l8_rmsnorm_bwd_workspace",
-                "l8_linear_fwd_workspace", "l8_linear_fwd_rows_workspace"}
+                "l8_linear_fwd_workspace", "l8_linear_fwd_rows_workspace", "l8_col_sum_workspace"}
 
 _lib = None
 _native = None    # the host extension, bound to the library's entries

@@ -431,6 +431,53 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const uint16_t *__restric
 }
 
 // bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
+// ---------------------------------------------------------------------------
+// Column sums of bf16 x (the bias gradient, lingua/float8.py:127), in fp32, rounded to bf16 once.  Bound by memory from a few
+// thousand rows on, by latency below: a workgroup owns 128 columns -- two lines of every row, which 64 columns read at the same
+// rate up to 4096 columns and 10 % slower beyond, and 256 half as fast at [16384,2048] -- and a slab of rows, read 16 at a time
+// with eight loads in flight per thread.  Slabs until there are four workgroups per unit, of at least 128 rows; several slabs
+// leave fp32 partial sums that the second kernel adds in their order.  The order of every sum hangs on the shape and the number
+// of compute units.  us, PyTorch's sum / this, back to back: [256,1024] 9.2 / 4.3, [1021,2048] 11.6 / 5.2, [1801,11040] 88 / 12,
+// [4096,4096] 19.8 / 9.4, [5580,12176] 369 / 33, [16384,2048] 28 / 16, [16384,11008] 69 / 68 (a copy's rate: 64)
+// ---------------------------------------------------------------------------
+constexpr int kSumCols = 128, kSumThreads = 256, kSumRows = kSumThreads / (kSumCols / 8);
+__global__ __launch_bounds__(kSumThreads) void col_sum_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx,
+                                                              int64_t slab, float *__restrict__ partials, uint16_t *__restrict__ out) {
+  __shared__ float sums[kSumRows][kSumCols + 1];
+  const int cc = threadIdx.x % (kSumCols / 8), rg = threadIdx.x / (kSumCols / 8);
+  const int col = blockIdx.x * kSumCols + cc * 8;
+  const int64_t r1 = ((int64_t)blockIdx.y + 1) * slab < R ? ((int64_t)blockIdx.y + 1) * slab : R;
+  float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  if (col < C) {
+    const uint16_t *at = x + col;
+#pragma unroll 8
+    for (int64_t r = (int64_t)blockIdx.y * slab + rg; r < r1; r += kSumRows) {
+      const v4i v = *(const v4i *)(at + r * ldx);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] += __uint_as_float((e & 1) ? ((uint32_t)v[e >> 1] & 0xffff0000u) : ((uint32_t)v[e >> 1] << 16));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sums[rg][cc * 8 + e] = s[e];
+  __syncthreads();
+  if (threadIdx.x >= kSumCols) return;
+  float t = sums[0][threadIdx.x];
+#pragma unroll
+  for (int k = 1; k < kSumRows; ++k) t += sums[k][threadIdx.x];
+  const int c = blockIdx.x * kSumCols + threadIdx.x;
+  if (c >= C) return;
+  if (out) out[c] = (uint16_t)bf16_rne_bits(t);
+  else partials[(int64_t)blockIdx.y * C + c] = t;
+}
+__global__ __launch_bounds__(256) void col_sum_fold_kernel(const float *__restrict__ partials, int slabs, int C, uint16_t *__restrict__ out) {
+  const int c = blockIdx.x * 256 + threadIdx.x;
+  if (c >= C) return;
+  float t = 0.0f;
+#pragma unroll 8
+  for (int s = 0; s < slabs; ++s) t += partials[(int64_t)s * C + c];
+  out[c] = (uint16_t)bf16_rne_bits(t);
+}
+
 __global__ __launch_bounds__(1024) void amax_reduce_kernel(const uint16_t *__restrict__ amax, int64_t n,
                                                            uint16_t *__restrict__ out) {
   __shared__ uint32_t red[16];
@@ -964,6 +1011,42 @@ extern "C" int l8_cast_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx,
                (long long)need);
   }
   return cast_rowwise_impl("l8_cast_rowwise", x, R, C, ldx, q, ldq, scale, amax, col_amax, workspace, (hipStream_t)stream);
+}
+
+// slabs of rows, and rows of a slab
+static int64_t col_sum_slabs(int64_t R, int64_t C, int64_t *slab) {
+  const int64_t cols = (C + kSumCols - 1) / kSumCols;
+  int64_t n = (4 * (int64_t)num_cus() + cols - 1) / cols;
+  if (n > (R + 127) / 128) n = (R + 127) / 128;
+  if (n < 1) n = 1;
+  *slab = (R + n - 1) / n;
+  return *slab > 0 ? (R + *slab - 1) / *slab : 1;
+}
+
+extern "C" int64_t l8_col_sum_workspace(int64_t R, int64_t C) {
+  if (R <= 0 || C <= 0) return 0;
+  int64_t slab;
+  const int64_t n = col_sum_slabs(R, C, &slab);
+  return n > 1 ? n * C * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void *out, void *workspace, int64_t workspace_bytes, void *stream) {
+  L8_REQUIRE(R >= 0 && C >= 0, "l8_col_sum: negative shape");
+  if (C == 0) return L8_OK;
+  L8_REQUIRE(out && (R == 0 || x), "l8_col_sum: null pointer");
+  L8_REQUIRE(C % 8 == 0 && ldx % 8 == 0 && ldx >= C && aligned(x, 16) && C < (1LL << 31), "l8_col_sum: C, ldx multiples of 8 and x 16-byte aligned required");
+  const int64_t need = l8_col_sum_workspace(R, C);
+  L8_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned(workspace, 4)), "l8_col_sum: needs a workspace of %lld bytes (l8_col_sum_workspace)", (long long)need);
+  int64_t slab;
+  const int64_t n = col_sum_slabs(R, C, &slab);
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(col_sum_kernel, dim3((unsigned)((C + kSumCols - 1) / kSumCols), (unsigned)n), dim3(kSumThreads), 0, st, (const uint16_t *)x, R, (int)C,
+                     ldx, slab, (float *)workspace, n > 1 ? nullptr : (uint16_t *)out);
+  L8_HIP(hipGetLastError());
+  if (n == 1) return L8_OK;
+  hipLaunchKernelGGL(col_sum_fold_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, (const float *)workspace, (int)n, (int)C, (uint16_t *)out);
+  L8_HIP(hipGetLastError());
+  return L8_OK;
 }
 
 extern "C" int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items, int64_t n, void *stream) {

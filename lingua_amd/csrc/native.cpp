@@ -27,7 +27,7 @@ struct Library {
 #define L8_ENTRY(name) decltype(&::name) name = nullptr;
 #define L8_ENTRIES(X)                                                                                                        \
   X(l8_last_error) X(l8_linear_fwd_rows) X(l8_linear_fwd_rows_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
-  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_gemm_nt)
+  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_col_sum) X(l8_col_sum_workspace) X(l8_gemm_nt)
   L8_ENTRIES(L8_ENTRY)
 #undef L8_ENTRY
 } lib;
@@ -194,7 +194,9 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   Rows rg, rw, ra;
   if (g.dim() != 2 || w.dim() != 2 || !as_rows(g, device, rg) || !as_rows(w, device, rw) || c10::hip::current_device() != device) Py_RETURN_NONE;
   const int64_t M = rg.rows, N = rg.cols, K = rw.cols, padded = (M + 15) / 16 * 16;
-  if (rw.rows != N || N % 16 || K % 16 || !dense(amax, at::kBFloat16, N, device)) Py_RETURN_NONE;
+  if (rw.rows != N || N % 16 || K % 16 || !dense(amax, at::kBFloat16, N, device) ||
+      (need_bias && (rg.ld % 8 || reinterpret_cast<uintptr_t>(rg.p) % 16)))
+    Py_RETURN_NONE;
   if (need_b && !qat_in.defined() && !(a.defined() && a.dim() == 2 && as_rows(a, device, ra) && ra.rows == M && ra.cols == K)) Py_RETURN_NONE;
   if ((qat_in.defined() && !(fp8_rows(qat_in, K, padded, device) && dense(sat_in, at::kFloat, K, device))) ||
       (qwt_in.defined() && !(fp8_rows(qwt_in, K, N, device) && dense(swt_in, at::kFloat, 1, device))) ||
@@ -253,7 +255,12 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       check(lib.l8_gemm_nt(qgt.const_data_ptr(), qat.const_data_ptr(), N, K, padded, qgt.stride(0), qat.stride(0), sgt.const_data_ptr<float>(), L8_SCALE_ROW,
                            sat.const_data_ptr<float>(), L8_SCALE_ROW, nullptr, gb.mutable_data_ptr(), K, algo, stream), "l8_gemm_nt");
     }
-    if (need_bias) gbias = at::sum(g, {0});
+    if (need_bias) {
+      gbias = at::empty({N}, o);
+      const int64_t ws_bytes = lib.l8_col_sum_workspace(M, N);
+      const Space ws(g, ws_bytes);
+      check(lib.l8_col_sum(rg.p, M, N, rg.ld, gbias.mutable_data_ptr(), ws.p(), ws_bytes, stream), "l8_col_sum");
+    }
   }
   return tuple_of({ga, gb, gbias, qat, sat});
   END_HANDLE_TH_ERRORS

@@ -93,6 +93,10 @@ def _rows_apart(t: torch.Tensor) -> bool:
     return t.stride(1) == 1 and (t.shape[0] <= 1 or t.stride(0) >= t.shape[1])
 
 
+def rows_on_16_bytes(t: torch.Tensor) -> bool:
+    return t.data_ptr() % 16 == 0 and t.shape[1] * t.element_size() % 16 == 0 and (not _rows_apart(t) or _ld(t) * t.element_size() % 16 == 0)
+
+
 def _ld(t: torch.Tensor) -> int:
     return t.stride(0) if t.shape[0] > 1 else max(t.shape[1], 1)
 
@@ -253,6 +257,20 @@ def col_amax(x: torch.Tensor) -> torch.Tensor:
     with _timed("col_amax", R * C * 2 + 4 * C, x.device):
         code = _lib.load().l8_col_amax(x.data_ptr(), R, C, _ld(x), out.data_ptr(), st)
     _lib.check(code, "l8_col_amax")
+    return out
+
+
+def col_sum(x: torch.Tensor) -> torch.Tensor:
+    """bf16 [C] column sums of bf16 x [R,C], added up in fp32."""
+    x = _rows_2d(x, torch.bfloat16, "col_sum")
+    st = _prep(x, "col_sum")
+    R, C = x.shape
+    out = torch.empty(C, dtype=torch.bfloat16, device=x.device)
+    with _timed("col_sum", R * C * 2 + 2 * C, x.device):
+        need = _lib.load().l8_col_sum_workspace(R, C)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+        code = _lib.load().l8_col_sum(x.data_ptr(), R, C, _ld(x), out.data_ptr(), ws.data_ptr(), need, st)
+    _lib.check(code, "l8_col_sum")
     return out
 
 

@@ -553,3 +553,34 @@ def test_several_row_casts_with_column_amaxes_equal_single_ones(shapes):
         wq, ws, _ = ops.cast_rowwise(x, col_amax=want)
         assert torch.equal(q.view(torch.uint8), wq.view(torch.uint8)) and torch.equal(s.view(torch.int32), ws.view(torch.int32))
         assert torch.equal(col.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("R,C", [(0, 16), (1, 8), (127, 72), (128, 64), (129, 2048), (1021, 2048), (4100, 520), (20000, 48)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_column_sums(R, C, strided):
+    """One slab and several, the last one short, columns that do not fill a workgroup, a row stride.  Integers of magnitude up
+    to 8: sums below 2^24 are exact in fp32, whatever their order, so the result is the exact sum rounded once; then normal
+    values against the sum in 64 bits: at most R roundings of fp32 on top of the one to bf16; an infinity and a NaN stay."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(R + C)
+    wide = torch.randint(-8, 9, (R, C + 8), generator=g).to(torch.bfloat16).cuda()
+    x = wide[:, :C] if strided else wide[:, :C].contiguous()
+    assert torch.equal(ops.col_sum(x), x.double().sum(0).to(torch.bfloat16))
+    x = torch.randn(R, C, generator=g).to(torch.bfloat16).cuda()
+    want, mag = x.double().sum(0), x.double().abs().sum(0)
+    assert bool(((ops.col_sum(x).double() - want).abs() <= want.abs() * 2.0 ** -8 + mag * R * 2.0 ** -24).all())
+    if R > 1:
+        x[0, 0], x[R - 1, 1] = float("inf"), float("nan")
+        got = ops.col_sum(x)
+        assert bool(torch.isinf(got[0])) and bool(torch.isnan(got[1])) and bool(torch.isfinite(got[2:]).all())
+
+
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_bias_gradient_of_rows_off_16_byte_lines(shift):
+    """Only the bias learns, and the gradient's rows start off 16-byte lines, or not at all on a common one."""
+    from lingua_amd.float8 import linear_backward
+    g = torch.Generator().manual_seed(3)
+    wide = torch.randint(-8, 9, (130, 64 + shift), generator=g).to(torch.bfloat16).cuda()
+    got = linear_backward(wide[:, shift:], None, torch.zeros(64, 32, dtype=torch.bfloat16, device="cuda"),
+                          torch.zeros(64, dtype=torch.bfloat16, device="cuda"), None, False, False, True, False, 0)
+    assert got[0] is None and got[1] is None and torch.equal(got[2], wide[:, shift:].double().sum(0).to(torch.bfloat16))
