@@ -2,7 +2,7 @@
 //
 // What generation and short prompts call (lingua/float8.py:85-96 with M in the tens): every weight byte is used for a
 // handful of tokens, so the weight's bytes per second are all that counts, and a 128 x 128 tile leaves most of the chip
-// without work ([32,4096] . [11008,4096]^T has 86 of them).  Here a workgroup owns 16 weight rows and ALL tokens:
+// without work ([32,4096] . [11008,4096]^T has 86 of them).  Here a workgroup owns 16 weight rows (or 32) and ALL tokens:
 //
 //   * its eight waves split K between them (step s of 128 elements goes to wave s % 8), so that even a [2048,2048] weight
 //     puts a thousand waves to work, each with all of its few loads in flight, and no wave waits for another;
@@ -48,22 +48,23 @@ L8_DEV uint32_t dpp_row_max(uint32_t v) {
 L8_DEV int tile_pos(int r, int c) { return r * kSkStep + ((c ^ (r & 7) ^ ((r >> 3) & 1)) * 16); }
 #endif
 
-// MT tiles of 16 tokens, U steps of a wave requested together.
+// MT tiles of 16 tokens, NT of 16 weight rows, U steps of a wave requested together.
 // SW > 0: the weight comes in bf16, at most SW steps per wave are held in registers.
 // SX > 0: x comes in bf16 (one tile of tokens), at most SX steps per wave are held in registers.
-template <int MT, int U, int SW, int SX>
+template <int MT, int NT, int U, int SW, int SX>
 __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && (MT > 2 || SX > 0)) || SX > 4 ? 2 : 4)) void linear_skinny_kernel(const SkinnyArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   constexpr bool QW = SW > 0, QX = SX > 0;
+  static_assert(NT == 1 || (!QW && !QX), "one tile of weight rows is quantised");
   static_assert(!QX || (MT == 1 && (QW ? SW == SX : U == SX)), "x is quantised for one tile of tokens");
   constexpr int kBuf = 2 * kSkTile;  // a wave's two tile buffers: weight rows, tokens
-  constexpr int kRed = MT * 64 * 16;
+  constexpr int kRed = MT * NT * 64 * 16;
   __shared__ __attribute__((aligned(16))) uint8_t lds[kSkWaves * (kBuf > kRed ? kBuf : kRed)];
   __shared__ uint32_t amax_w[kSkWaves][16], amax_x[kSkWaves][16];
   __shared__ float scale_w[16], scale_x[16];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int n0 = blockIdx.x * 16;
+  const int n0 = blockIdx.x * (16 * NT);
   const int KT = (p.K + kSkStep - 1) / kSkStep;
   constexpr uint32_t kBeyond = 0x80000000u;  // an offset no descriptor covers: the load returns zeros
   constexpr int EW = QW ? 2 : 1, EX = QX ? 2 : 1;  // bytes per element of the weight and of x
@@ -98,16 +99,16 @@ __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && (MT > 2 || SX > 0)) || 
     a = __builtin_amdgcn_raw_buffer_load_b128(rsX, (int)off, 0, 0);
     b = __builtin_amdgcn_raw_buffer_load_b128(rsX, (int)off, 8 * (int)p.ldx, 0);
   };
-  auto load_w = [&](int s, v4i &a, v4i &b) {
+  auto load_w = [&](int s, int nt, v4i &a, v4i &b) {
     const int k = s * kSkStep + lchunk * 16;
-    const uint32_t off = (uint32_t)(lrow * (int)p.ldw + k) | mask(k);
+    const uint32_t off = (uint32_t)((nt * 16 + lrow) * (int)p.ldw + k) | mask(k);
     a = load16_nt(rsW, off, 0);
     b = load16_nt(rsW, off, (uint32_t)(8 * (int)p.ldw));
   };
 
-  v4f acc[MT];
+  v4f acc[NT * MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) acc[mt] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int t = 0; t < NT * MT; ++t) acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
   auto mma = [&](v8i wf, v8i xf, v4f c) { return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf, c, 0, 0, 0, 0, 0, 0); };
 
   // Row j * 4 + qrow of a tile held as raw[..][j]: its maximum over this wave's share of K, and 1 / scale from all waves'.
@@ -190,7 +191,7 @@ __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && (MT > 2 || SX > 0)) || 
   } else if constexpr (QX) {
     v4i wa[U], wb[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) load_w(wave + u * kSkWaves, wa[u], wb[u]);
+    for (int u = 0; u < U; ++u) load_w(wave + u * kSkWaves, 0, wa[u], wb[u]);
     row_maxima(xraw, amax_x, p.M);
     __syncthreads();
     row_scales(amax_x, scale_x, xrecip, p.M);
@@ -201,35 +202,43 @@ __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && (MT > 2 || SX > 0)) || 
     }
   } else {
     for (int s0 = wave; s0 < KT; s0 += kSkWaves * U) {
-      v4i wa[U], wb[U], xa[U][MT], xb[U][MT];
+      v4i wa[U][NT], wb[U][NT], xa[U][MT], xb[U][MT];
 #pragma unroll
       for (int u = 0; u < U; ++u)  // the weight first: its bytes come from HBM, the tokens' from the L2
-        load_w(s0 + u * kSkWaves, wa[u], wb[u]);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) load_w(s0 + u * kSkWaves, nt, wa[u][nt], wb[u][nt]);
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) load_x(s0 + u * kSkWaves, mt, xa[u][mt], xb[u][mt]);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const v8i wf = turn(wbuf, wa[u], wb[u]);
+        v8i wf[NT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt] = mma(wf, turn(xbuf, xa[u][mt], xb[u][mt]), acc[mt]);
+        for (int nt = 0; nt < NT; ++nt) wf[nt] = turn(wbuf, wa[u][nt], wb[u][nt]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+          const v8i xf = turn(xbuf, xa[u][mt], xb[u][mt]);
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) acc[nt * MT + mt] = mma(wf[nt], xf, acc[nt * MT + mt]);
+        }
       }
     }
   }
 
   // ---- the waves' partial tiles, added in the order of the waves ----
   __syncthreads();  // the tile buffers become the array of partial tiles
-  v4f(*red)[MT][64] = reinterpret_cast<v4f(*)[MT][64]>(lds);
+  static_assert(NT * MT <= kSkWaves, "a wave adds up one tile");
+  v4f(*red)[NT * MT][64] = reinterpret_cast<v4f(*)[NT * MT][64]>(lds);
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) red[wave][mt][lane] = acc[mt];
+  for (int t = 0; t < NT * MT; ++t) red[wave][t][lane] = acc[t];
   __syncthreads();
-  if (wave >= MT) return;
+  if (wave >= NT * MT) return;
   v4f sum = red[0][wave][lane];
 #pragma unroll
   for (int v = 1; v < kSkWaves; ++v) sum += red[v][wave][lane];
-  // lane: token (lane & 15) of token tile `wave`, weight rows 4 * (lane >> 4) .. + 3
-  const int m = wave * 16 + frow, nl = fpiece * 4, n = n0 + nl;
+  // lane: token (lane & 15) of token tile wave % MT, rows 4 * (lane >> 4) .. + 3 of weight tile wave / MT
+  const int m = wave % MT * 16 + frow, nl = wave / MT * 16 + fpiece * 4, n = n0 + nl;
   if (m >= p.M || n >= p.N) return;
   const float sa = QX ? scale_x[frow] : p.sx_row ? p.sx[m] : p.sx[0];
   float v[4];
@@ -256,9 +265,9 @@ __global__ __launch_bounds__(kSkBlock, (SW > 4 || (SW && (MT > 2 || SX > 0)) || 
 #endif
 }
 
-template <int MT, int U, int SW, int SX>
+template <int MT, int NT, int U, int SW, int SX>
 static int skinny_go(const SkinnyArgs &p, hipStream_t st) {
-  hipLaunchKernelGGL((linear_skinny_kernel<MT, U, SW, SX>), dim3((unsigned)((p.N + 15) / 16)), dim3(kSkBlock), 0, st, p);
+  hipLaunchKernelGGL((linear_skinny_kernel<MT, NT, U, SW, SX>), dim3((unsigned)((p.N + 16 * NT - 1) / (16 * NT))), dim3(kSkBlock), 0, st, p);
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
@@ -287,27 +296,44 @@ bool skinny_quantises_x(int64_t M, int64_t N, int64_t K, int64_t ldx, int w_byte
 // [11008,4096] 10.6 / 9.3 (4.8 TB/s; 19.4 with 128 x 128 tiles); two token tiles U = 1 / 2 / 4: [32,11008].[4096,11008]
 // 14.0 / 14.8 / 14.9 (43.9 with tiles), [32,4096].[4096,4096] 7.1 / 7.2 / 6.7, [17,2048].[8192,2048] 6.1 / 5.8 / 7.4; four
 // token tiles U = 1 / 2: [64,4096].[11008,4096] 19.8 / 20.7 (19.6), [64,14336].[4096,14336] 23.6 / 24.3 (57.4).
+//
+// Two tiles of weight rows per workgroup (NT): a compute unit takes in some 25 bytes per clock, weight and tokens together, and
+// every workgroup reads all tokens; so what counts is rounds of one workgroup per unit, times the rows that each reads.  Twice the
+// rows need half the rounds of tokens, and above 16 rows per unit 257 tiles are no longer two rounds for little more than one's
+// work.  Sums, their order and the results are the same.  us, weights cold, one tile / two: [1,8960].[5120,8960] 12.9 / 10.9,
+// [1,5120].[12800,5120] 16.1 / 13.6, [16,4096].[14336,4096] 13.4 / 12.0, [32,8960].[5120,8960] 19.8 / 14.5, [32,4096].[8192,4096]
+// 11.8 / 9.8, [64,6752].[6000,6752] 21.0 / 15.8; where the rule says one: [1,8192].[2560,8192] 6.6 / 8.8, [64,8192].[2560,8192]
+// 12.5 / 14.9, [8,3648].[10496,3648] 8.4 / 9.4.  Beyond four rounds 16 tokens or fewer keep HBM busy either way and gain nothing:
+// [16,4096].[20480,4096] 16.9 / 18.1, [1,4096].[24576,4096] 18.0 / 19.3, but [32,4096].[32000,4096] 35.3 / 27.8.  U there, 2 / 4: three or four steps [16,4096].[8192,4096] 9.2 / 8.1, else
+// [1,2048].[6400,2048] 4.8 / 5.6, [16,8960].[5120,8960] 12.9 / 13.8; two token tiles 1 / 2: [32,6752].[6000,6752] 11.8 / 13.2.
 int skinny_linear(const SkinnyArgs &p, bool w_is_bf16, bool x_is_bf16, hipStream_t st) {
   const int mt = (p.M + 15) / 16;
   const int steps = (p.K + kSkStep * kSkWaves - 1) / (kSkStep * kSkWaves);  // of a wave
   if (x_is_bf16) {
-    if (w_is_bf16) return steps <= 2 ? skinny_go<1, 1, 2, 2>(p, st) : skinny_go<1, 1, 4, 4>(p, st);
-    return steps <= 2 ? skinny_go<1, 2, 0, 2>(p, st) : skinny_go<1, 4, 0, 4>(p, st);
+    if (w_is_bf16) return steps <= 2 ? skinny_go<1, 1, 1, 2, 2>(p, st) : skinny_go<1, 1, 1, 4, 4>(p, st);
+    return steps <= 2 ? skinny_go<1, 1, 2, 0, 2>(p, st) : skinny_go<1, 1, 4, 0, 4>(p, st);
   }
   if (w_is_bf16) {
 #define L8_SKINNY_Q(MT)                                 \
-  if (steps <= 4) return skinny_go<MT, 1, 4, 0>(p, st); \
-  if (steps <= 8) return skinny_go<MT, 1, 8, 0>(p, st); \
-  return skinny_go<MT, 1, kSkinnyMaxQuantSteps, 0>(p, st)
+  if (steps <= 4) return skinny_go<MT, 1, 1, 4, 0>(p, st); \
+  if (steps <= 8) return skinny_go<MT, 1, 1, 8, 0>(p, st); \
+  return skinny_go<MT, 1, 1, kSkinnyMaxQuantSteps, 0>(p, st)
     if (mt == 1) { L8_SKINNY_Q(1); }
     if (mt == 2) { L8_SKINNY_Q(2); }
     L8_SKINNY_Q(4);
 #undef L8_SKINNY_Q
   }
-  if (mt == 1) return steps <= 2 ? skinny_go<1, 2, 0, 0>(p, st) : skinny_go<1, 4, 0, 0>(p, st);
-  if (mt == 2) return steps <= 2 ? skinny_go<2, 2, 0, 0>(p, st) : skinny_go<2, 1, 0, 0>(p, st);
-  if (mt == 3) return skinny_go<3, 1, 0, 0>(p, st);
-  return skinny_go<4, 1, 0, 0>(p, st);
+  const int64_t cus = num_cus(), t16 = ((int64_t)p.N + 15) / 16, t32 = ((int64_t)p.N + 31) / 32;
+  if ((p.M > 16 || t16 <= 4 * cus) && (t32 + cus - 1) / cus * (32 + p.M) < (t16 + cus - 1) / cus * (16 + p.M) && 32 * p.ldw + p.K < (1LL << 31)) {
+    if (mt == 1) return steps == 3 || steps == 4 ? skinny_go<1, 2, 4, 0, 0>(p, st) : skinny_go<1, 2, 2, 0, 0>(p, st);
+    if (mt == 2) return skinny_go<2, 2, 1, 0, 0>(p, st);
+    if (mt == 3) return skinny_go<3, 2, 1, 0, 0>(p, st);
+    return skinny_go<4, 2, 1, 0, 0>(p, st);
+  }
+  if (mt == 1) return steps <= 2 ? skinny_go<1, 1, 2, 0, 0>(p, st) : skinny_go<1, 1, 4, 0, 0>(p, st);
+  if (mt == 2) return steps <= 2 ? skinny_go<2, 1, 2, 0, 0>(p, st) : skinny_go<2, 1, 1, 0, 0>(p, st);
+  if (mt == 3) return skinny_go<3, 1, 1, 0, 0>(p, st);
+  return skinny_go<4, 1, 1, 0, 0>(p, st);
 }
 
 }  // namespace l8

@@ -421,3 +421,27 @@ def test_against_the_scaled_mm_call_the_reference_makes(mnk):
     rows = torch.arange(0, M, max(1, M // 32))[:32]
     want = oracle.gemm_nt(qa[rows.cuda()].cpu().view(torch.uint8), qb.cpu().view(torch.uint8), sa[rows.cuda()].cpu(), sb.cpu())
     assert rel_l2(ref[rows.cuda()], want) <= TOL and rel_l2(out[rows.cuda()], want) <= TOL
+
+
+@pytest.mark.parametrize("M,extra,K", [(1, 16, 2048), (8, 21, 3072), (9, 5, 16), (16, 16, 4096), (17, 40, 272), (32, 1, 9008), (33, 16, 1040),
+                                       (48, 37, 2064), (49, 16, 128), (64, 100, 4112), (64, 16, 9008)])
+@pytest.mark.parametrize("mode", ["plain", "bias", "add"])
+def test_two_tiles_of_weight_rows_per_workgroup(M, extra, K, mode):
+    """Just beyond one tile of 16 weight rows per compute unit, where the skinny kernels take 32 rows per workgroup: bit by bit
+    what they give for the two halves of the weight (16 rows per workgroup), the last workgroup short of rows or not."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(M * K + extra)
+    N = 16 * torch.cuda.get_device_properties(0).multi_processor_count + extra
+    half = N // 2 // 16 * 16
+    qa, qb = (torch.randint(-8, 9, (r, K), generator=g).float().cuda().to(torch.float8_e4m3fn) for r in (M, N))
+    sa, sb = (torch.rand(r, 1, generator=g).cuda() + 0.5 for r in (M, N))
+    bias = torch.randn(N, generator=g).bfloat16().cuda() if mode == "bias" else None
+    out = torch.randn(M, N, generator=g).bfloat16().cuda()
+    parts = [out[:, :half].contiguous(), out[:, half:].contiguous()]
+    y = ops.gemm_nt(qa, qb, sa, sb, bias, algo=17, out=out, add=mode == "add")
+    for part, rows in zip(parts, (slice(0, half), slice(half, N))):
+        want = ops.gemm_nt(qa, qb[rows], sa, sb[rows], bias[rows].contiguous() if bias is not None else None, algo=17, out=part, add=mode == "add")
+        assert torch.equal(y[:, rows], want)
+    if mode == "plain":   # products of integers up to 8 add up exactly in fp32
+        want = qa.double() @ qb.double().t() * sa.double() * sb.double().t()
+        assert bool(((y.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20)).all())
