@@ -436,13 +436,16 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const uint16_t *__restric
 // thousand rows on, by latency below: a workgroup owns 128 columns -- two lines of every row, which 64 columns read at the same
 // rate up to 4096 columns and 10 % slower beyond, and 256 half as fast at [16384,2048] -- and a slab of rows, read 16 at a time
 // with eight loads in flight per thread.  Slabs until there are four workgroups per unit, of at least 128 rows; several slabs
-// leave fp32 partial sums that the second kernel adds in their order.  The order of every sum hangs on the shape and the number
-// of compute units.  us, PyTorch's sum / this, back to back: [256,1024] 9.2 / 4.3, [1021,2048] 11.6 / 5.2, [1801,11040] 88 / 12,
+// leave fp32 partial sums that the second kernel adds in their order.  Up to 1024 rows one slab, by twice the threads: a launch less
+// ([512,4096] 5.2 / 3.1, [1021,2048] 5.2 / 5.0, [1024,11008] 7.6 / 5.8; [2048,2048] as one slab of 512 threads 6.5 against 4.9).  The order of every sum
+// hangs on the shape and the number of compute units.  us, PyTorch's sum / this, back to back: [256,1024] 9.2 / 2.6, [1021,2048] 11.6 / 5.0, [1801,11040] 88 / 12,
 // [4096,4096] 19.8 / 9.4, [5580,12176] 369 / 33, [16384,2048] 28 / 16, [16384,11008] 69 / 68 (a copy's rate: 64)
 // ---------------------------------------------------------------------------
-constexpr int kSumCols = 128, kSumThreads = 256, kSumRows = kSumThreads / (kSumCols / 8);
-__global__ __launch_bounds__(kSumThreads) void col_sum_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx,
-                                                              int64_t slab, float *__restrict__ partials, uint16_t *__restrict__ out) {
+constexpr int kSumCols = 128, kSumOneSlab = 1024;
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void col_sum_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx,
+                                                          int64_t slab, float *__restrict__ partials, uint16_t *__restrict__ out) {
+  constexpr int kSumRows = THREADS / (kSumCols / 8);
   __shared__ float sums[kSumRows][kSumCols + 1];
   const int cc = threadIdx.x % (kSumCols / 8), rg = threadIdx.x / (kSumCols / 8);
   const int col = blockIdx.x * kSumCols + cc * 8;
@@ -1018,7 +1021,7 @@ static int64_t col_sum_slabs(int64_t R, int64_t C, int64_t *slab) {
   const int64_t cols = (C + kSumCols - 1) / kSumCols;
   int64_t n = (4 * (int64_t)num_cus() + cols - 1) / cols;
   if (n > (R + 127) / 128) n = (R + 127) / 128;
-  if (n < 1) n = 1;
+  if (n < 1 || R <= kSumOneSlab) n = 1;
   *slab = (R + n - 1) / n;
   return *slab > 0 ? (R + *slab - 1) / *slab : 1;
 }
@@ -1040,10 +1043,14 @@ extern "C" int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void
   int64_t slab;
   const int64_t n = col_sum_slabs(R, C, &slab);
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(col_sum_kernel, dim3((unsigned)((C + kSumCols - 1) / kSumCols), (unsigned)n), dim3(kSumThreads), 0, st, (const uint16_t *)x, R, (int)C,
-                     ldx, slab, (float *)workspace, n > 1 ? nullptr : (uint16_t *)out);
+  const dim3 grid((unsigned)((C + kSumCols - 1) / kSumCols), (unsigned)n);
+  if (n == 1) {
+    hipLaunchKernelGGL(col_sum_kernel<512>, grid, dim3(512), 0, st, (const uint16_t *)x, R, (int)C, ldx, slab, nullptr, (uint16_t *)out);
+    L8_HIP(hipGetLastError());
+    return L8_OK;
+  }
+  hipLaunchKernelGGL(col_sum_kernel<256>, grid, dim3(256), 0, st, (const uint16_t *)x, R, (int)C, ldx, slab, (float *)workspace, nullptr);
   L8_HIP(hipGetLastError());
-  if (n == 1) return L8_OK;
   hipLaunchKernelGGL(col_sum_fold_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, (const float *)workspace, (int)n, (int)C, (uint16_t *)out);
   L8_HIP(hipGetLastError());
   return L8_OK;

@@ -555,7 +555,7 @@ def test_several_row_casts_with_column_amaxes_equal_single_ones(shapes):
         assert torch.equal(col.view(torch.int32), want.view(torch.int32))
 
 
-@pytest.mark.parametrize("R,C", [(0, 16), (1, 8), (127, 72), (128, 64), (129, 2048), (1021, 2048), (4100, 520), (20000, 48)])
+@pytest.mark.parametrize("R,C", [(0, 16), (1, 8), (127, 72), (128, 64), (129, 2048), (1021, 2048), (1024, 136), (1025, 136), (4100, 520), (20000, 48)])
 @pytest.mark.parametrize("strided", [False, True])
 def test_column_sums(R, C, strided):
     """One slab and several, the last one short, columns that do not fill a workgroup, a row stride.  Integers of magnitude up
