@@ -64,7 +64,7 @@ int l8_get_scale_rule(void);
  *   amax     bf16 [R] row amax, NaN propagating     (may be NULL)
  *   col_amax fp32 [C] (may be NULL): receives the column amaxes of x (as
  *            non-negative float bit patterns; overwritten, nothing to
- *            initialise), so that a later l8_cast_colwise_transposed() needs
+ *            initialise; zeros if R is 0), so that a later l8_cast_colwise_transposed() needs
  *            no pass of its own to find them.
  *   workspace  device scratch of at least l8_cast_rowwise_workspace(R, C)
  *            bytes, 16-byte aligned; needed only with col_amax (per-workgroup

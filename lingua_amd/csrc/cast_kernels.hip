@@ -869,6 +869,8 @@ static int zero_u32(void *p, int64_t n, hipStream_t st) {
   return L8_OK;
 }
 
+int empty_col_amax(float *col_amax, int64_t C, hipStream_t st) { return col_amax && C > 0 ? zero_u32(col_amax, C, st) : L8_OK; }
+
 template <int NCH>
 static int launch_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq, float *scale,
                           void *amax, float *col_amax, void *ws, hipStream_t st) {
@@ -1006,7 +1008,7 @@ static int launch_rowwise_any(const char *what, const void *x, int64_t R, int64_
 extern "C" int l8_cast_rowwise(const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq, float *scale,
                                void *amax, float *col_amax, void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_cast_rowwise: negative shape R=%lld C=%lld", (long long)R, (long long)C);
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) return empty_col_amax(col_amax, C, (hipStream_t)stream);
   if (col_amax) {
     const int64_t need = l8_cast_rowwise_workspace(R, C);
     L8_REQUIRE(need == 0 || (workspace != nullptr && workspace_bytes >= need && aligned(workspace, 16)),
@@ -1069,7 +1071,11 @@ extern "C" int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items,
   int pending = 0;
   for (int64_t i = 0; i < n; ++i) {
     const l8_cast_rowwise_cols_item &t = items[i];
-    if (t.R == 0 || t.C == 0) continue;
+    if (t.R == 0 || t.C == 0) {
+      const int rc = empty_col_amax(t.col_amax, t.C, (hipStream_t)stream);
+      if (rc != L8_OK) return rc;
+      continue;
+    }
     int rc = cast_rowwise_impl("l8_cast_rowwise_cols_many", t.x, t.R, t.C, t.ldx, t.q, t.ldq, t.scale, t.amax, t.col_amax, t.workspace,
                                (hipStream_t)stream, &folds[pending]);
     if (rc == L8_OK && folds[pending].C > 0 && ++pending == kMaxFolds) {
@@ -1119,7 +1125,7 @@ int l8::noalloc_setup_current_device() {
 extern "C" int l8_cast_rowwise_noalloc(const void *x, int64_t R, int64_t C, int64_t ldx, void *q, int64_t ldq,
                                        float *scale, void *amax, float *col_amax, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_cast_rowwise_noalloc: negative shape R=%lld C=%lld", (long long)R, (long long)C);
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) return empty_col_amax(col_amax, C, (hipStream_t)stream);
   void *ws = nullptr;
   if (col_amax) {
     const int64_t need = l8_cast_rowwise_workspace(R, C);
@@ -1157,7 +1163,7 @@ extern "C" int l8_cast_rowwise_given_amax(const void *x, int64_t R, int64_t C, i
 
 extern "C" int l8_col_amax(const void *x, int64_t R, int64_t C, int64_t ldx, float *col_amax, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_col_amax: negative shape");
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) return empty_col_amax(col_amax, C, (hipStream_t)stream);
   L8_REQUIRE(x && col_amax, "l8_col_amax: null pointer");
   L8_REQUIRE(C % 8 == 0 && ldx % 8 == 0 && ldx >= C && aligned(x, 16), "l8_col_amax: C, ldx multiples of 8 and x 16-byte aligned required");
   L8_REQUIRE(C < (1LL << 31), "l8_col_amax: C too large");

@@ -47,6 +47,10 @@ struct FoldOperand {
 };
 int fold_colmax_many(const FoldOperand *ops, int n, hipStream_t st);
 
+// Column amaxes (if asked for) of an operand without rows: zeros, the maximum of nothing, so that the scales made of them
+// are finite and the products with the operand's copy are the zeros of an empty sum.  Defined in cast_kernels.hip.
+int empty_col_amax(float *col_amax, int64_t C, hipStream_t st);
+
 // Looks up, for the current device, the address of the static scratch array of l8_cast_rowwise_noalloc.
 // Defined in cast_kernels.hip; l8_device_check calls it so that the look-up happens at set-up.
 int noalloc_setup_current_device();

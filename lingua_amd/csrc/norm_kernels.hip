@@ -535,7 +535,7 @@ extern "C" int l8_rmsnorm_cast_rowwise(const void *x, const void *w, int w_is_f3
                                        void *y, int64_t ldy, void *q, int64_t ldq, float *scale, float *rstd,
                                        float *col_amax, void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_rmsnorm_cast_rowwise: negative shape R=%lld C=%lld", (long long)R, (long long)C);
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) return empty_col_amax(col_amax, C, (hipStream_t)stream);
   L8_REQUIRE(x && w && y, "l8_rmsnorm_cast_rowwise: null pointer");
   L8_REQUIRE((q == nullptr) == (scale == nullptr), "l8_rmsnorm_cast_rowwise: pass q and scale together");
   L8_REQUIRE(C % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 && ldx >= C && ldy >= C && (!q || (ldq % 8 == 0 && ldq >= C)),

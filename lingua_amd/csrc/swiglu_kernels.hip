@@ -560,7 +560,7 @@ extern "C" int l8_swiglu_cast_rowwise(const void *h1, const void *h3, int64_t R,
                                       int64_t ldh, void *q, int64_t ldq, float *scale, void *amax, float *col_amax,
                                       void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_swiglu_cast_rowwise: negative shape R=%lld C=%lld", (long long)R, (long long)C);
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) return empty_col_amax(col_amax, C, (hipStream_t)stream);
   L8_REQUIRE(h1 && h3 && q && scale, "l8_swiglu_cast_rowwise: null pointer");
   L8_REQUIRE(C % 8 == 0 && ld1 % 8 == 0 && ld3 % 8 == 0 && ld1 >= C && ld3 >= C,
              "l8_swiglu_cast_rowwise: C=%lld, ld1=%lld, ld3=%lld must be multiples of 8 and ld >= C", (long long)C,
@@ -592,7 +592,10 @@ extern "C" int l8_swiglu_bwd_cast_rowwise(const void *dh, const void *h1, const 
                                           int64_t ldq, float *scale1, float *scale3, float *col_amax1, float *col_amax3,
                                           void *workspace, int64_t workspace_bytes, void *stream) {
   L8_REQUIRE(R >= 0 && C >= 0, "l8_swiglu_bwd_cast_rowwise: negative shape R=%lld C=%lld", (long long)R, (long long)C);
-  if (R == 0 || C == 0) return L8_OK;
+  if (R == 0 || C == 0) {
+    const int rc = empty_col_amax(col_amax1, C, (hipStream_t)stream);
+    return rc == L8_OK ? empty_col_amax(col_amax3, C, (hipStream_t)stream) : rc;
+  }
   L8_REQUIRE(dh && h1 && h3 && g1 && g3 && q1 && q3 && scale1 && scale3, "l8_swiglu_bwd_cast_rowwise: null pointer");
   L8_REQUIRE((col_amax1 == nullptr) == (col_amax3 == nullptr), "l8_swiglu_bwd_cast_rowwise: pass both column amaxes or neither");
   L8_REQUIRE(C % 8 == 0 && lddh % 8 == 0 && ld1 % 8 == 0 && ld3 % 8 == 0 && ldg % 8 == 0 && ldq % 8 == 0,

@@ -555,6 +555,58 @@ def test_several_row_casts_with_column_amaxes_equal_single_ones(shapes):
         assert torch.equal(col.view(torch.int32), want.view(torch.int32))
 
 
+@pytest.fixture
+def new_memory_is_nan():
+    """Memory that PyTorch hands out unwritten holds NaNs instead of whatever was there."""
+    torch.use_deterministic_algorithms(True)
+    assert torch.utils.deterministic.fill_uninitialized_memory
+    yield
+    torch.use_deterministic_algorithms(False)
+
+
+def test_column_amaxes_of_nothing_are_zeros(new_memory_is_nan):
+    """Operands without rows: every kernel that reports column amaxes writes them (the scales that are made of them multiply
+    the zeros of an empty sum), alone and beside an operand that has rows."""
+    from lingua_amd import _lib, ops
+    C = 272
+    x = torch.empty((0, C), dtype=torch.bfloat16, device="cuda")
+    one = torch.ones((1, C), dtype=torch.bfloat16, device="cuda")
+    got = [torch.empty(C, device="cuda") for _ in range(6)]
+    assert bool(torch.isnan(torch.stack(got)).all())
+    ops.cast_rowwise(x, col_amax=got[0])
+    ops.swiglu_cast_rowwise(x, x, col_amax=got[1])
+    ops.swiglu_bwd_cast_rowwise(x, x, x, got[2], got[3])
+    ops.rmsnorm_cast_rowwise(x, one[0], 1e-5, col_amax=got[4])
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(_lib.load().l8_cast_rowwise_noalloc(0, 0, C, C, 0, C, 0, 0, got[5].data_ptr(), stream), "l8_cast_rowwise_noalloc")
+    got.append(ops.col_amax(x))
+    many = [col for _, _, col in ops.cast_rowwise_cols_many([x, one, x])]
+    assert bool((torch.stack(got + [many[0], many[2]]) == 0).all()) and bool((many[1] == 1).all())
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_weight_gradients_of_an_empty_batch_are_zeros(new_memory_is_nan, fused):
+    """No tokens through linears on one activation, each for itself and as one product."""
+    from lingua_amd import convert_linears_to_fp8, float8
+    from lingua_amd.qkv import fuse_qkv
+
+    class Block(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.wq, self.wk, self.wv = (torch.nn.Linear(64, n, bias=False, device="cuda", dtype=torch.bfloat16) for n in (64, 32, 32))
+            for p in self.parameters():
+                torch.nn.init.constant_(p, 0.5)
+
+    float8.clear_cast_memos()
+    block = convert_linears_to_fp8(Block(), "rowwise", "w[qkv]")
+    if fused:
+        block = fuse_qkv(block, "^$")
+    x = torch.zeros((0, 64), dtype=torch.bfloat16, device="cuda", requires_grad=True)
+    sum(y.sum() for y in (block.wq(x), block.wk(x), block.wv(x))).backward()
+    assert x.grad.shape == x.shape
+    assert all(bool((w.weight.grad == 0).all()) for w in (block.wq, block.wk, block.wv))
+
+
 @pytest.mark.parametrize("R,C", [(0, 16), (1, 8), (127, 72), (128, 64), (129, 2048), (1021, 2048), (1024, 136), (1025, 136), (4100, 520), (20000, 48)])
 @pytest.mark.parametrize("strided", [False, True])
 def test_column_sums(R, C, strided):
