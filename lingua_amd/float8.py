@@ -387,59 +387,46 @@ def linear_forward(a, b_t, bias, need_wgrad_stats: bool, gemm_algo: int):
 _UNSHARED_TOKENS = 64
 
 
-def _infer_native(a, b_t, bias):
-    """``linear_infer`` through the host extension, or None where its operands are not the plain ones."""
-    if a.dim() < 2 or b_t.dtype != torch.bfloat16 or not b_t.is_cuda:
-        return None
-    native = _lib.native_for(a.get_device())
+def linear_infer(a, b_t, bias):
+    """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
+    both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same results as ``linear_forward``."""
+    # (the extension takes contiguous leading dimensions as they are)
+    native = (_native_call(a, config.gemm_algo) and (a.dim() == 2 or a.dim() > 2 and a.is_contiguous()) and
+              b_t.dtype == torch.bfloat16 and b_t.is_cuda)
+    shape = a.shape
+    if not native:
+        if a.dim() != 2:
+            a = a.flatten(end_dim=-2)
+        if (ops.kernel_timer is not None and ops.timed_singly("cast_rowwise", "gemm_nt")) or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
+            return linear_forward(a, b_t, bias, False, config.gemm_algo)[0].unflatten(0, shape[:-1])
+        _check_operands(a, b_t)
     if _bwd_cast.entries:
         _bwd_cast.clear(a)
     hit, rows, share = None, a, False
     if config.share_input_casts:
-        few = a.numel() <= _UNSHARED_TOKENS * a.shape[-1]
+        few = a.numel() <= _UNSHARED_TOKENS * shape[-1]
         if _fwd_cast.entries or not few:
             rows = a if a.dim() == 2 else a.flatten(end_dim=-2)
-            hit = _fwd_cast.get(rows, b_t.data_ptr())
+            hit = _fwd_cast.get(rows, b_t.data_ptr())   # answers a linear once: both forms below go by this answer
             if hit is None and few:   # nothing of its own to file, but an earlier activation (a prompt's) is not kept alive
                 _fwd_cast.clear(rows)
             share = hit is None and not few
-    qx, sx = (None, None) if hit is None else hit[:2]
     qw, sw, _ = weight_cast_rowwise(b_t) if config.cache_weight_casts else (None, None, None)
-    res = native.linear_fwd(a, b_t, bias, qx, sx, hit is not None, share, False, qw, sw, False, config.gemm_algo)
-    if res is None:
-        return None
-    if share:
-        _fwd_cast.put(rows, (res[1], res[2], None), b_t.data_ptr())
-    return res[0]
-
-
-def linear_infer(a, b_t, bias):
-    """Forward without anything backward would need: no column amaxes, no autograd node, and one call of the library for
-    both casts and the product.  ``a`` is [..., K]; returns [..., N].  Same results as ``linear_forward``."""
-    if _native_call(a, config.gemm_algo):
-        out = _infer_native(a, b_t, bias)
-        if out is not None:
-            return out
-    if (ops.kernel_timer is not None and ops.timed_singly("cast_rowwise", "gemm_nt")) or config.gemm_algo == ops.GEMM_ALGO_SHARED_K:
-        return linear_forward(a.flatten(end_dim=-2), b_t, bias, False, config.gemm_algo)[0].unflatten(0, a.shape[:-1])
-    shape = a.shape
-    if a.dim() != 2:
-        a = a.flatten(end_dim=-2)
-    _check_operands(a, b_t)
-    _bwd_cast.clear(a)
-    tokens = a.shape[0]
+    if native:
+        qx, sx = (None, None) if hit is None else hit[:2]
+        res = _lib.native_for(a.get_device()).linear_fwd(a, b_t, bias, qx, sx, hit is not None, share, False, qw, sw, False, config.gemm_algo)
+        if res is not None:
+            if share:
+                _fwd_cast.put(rows, (res[1], res[2], None), b_t.data_ptr())
+            return res[0]
+        a = rows if rows.dim() == 2 else rows.flatten(end_dim=-2)
+        _check_operands(a, b_t)
     out = a.new_empty(shape[:-1] + b_t.shape[:1])
-    x_cast = hit = None
-    if config.share_input_casts:
-        x_cast = hit = _fwd_cast.get(a, b_t.data_ptr())
-        if hit is None:
-            if tokens > _UNSHARED_TOKENS:
-                x_cast = (ops._empty_fp8(*a.shape, a.device, True), a.new_empty((tokens, 1), dtype=torch.float32))
-            elif _fwd_cast.entries:   # nothing of its own to file, but an earlier activation (a prompt's) is not kept alive
-                _fwd_cast.clear(a)
-    w_cast = weight_cast_rowwise(b_t) if config.cache_weight_casts else None
-    ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, w_cast, w_cast is not None, None, config.gemm_algo)
-    if hit is None and x_cast is not None and out.numel():   # nothing is quantised for a linear without outputs
+    x_cast = hit
+    if share:
+        x_cast = (ops._empty_fp8(*a.shape, a.device, True), a.new_empty((a.shape[0], 1), dtype=torch.float32))
+    ops.linear_fwd(a, b_t, bias, out, x_cast, hit is not None, None, None if qw is None else (qw, sw), qw is not None, None, config.gemm_algo)
+    if share and out.numel():   # nothing is quantised for a linear without outputs
         _fwd_cast.put(a, (*x_cast, None), b_t.data_ptr())
     return out
 

@@ -114,6 +114,32 @@ def test_inference_pass_has_the_bits_of_the_python_form(form, monkeypatch, token
     _same(*results)
 
 
+@pytest.mark.parametrize("kind", ["slice", "transposed", "bias view"])
+def test_inference_on_operands_the_extension_leaves_shares_the_cast(form, monkeypatch, kind):
+    """Two linears on one activation quantise it once also where the extension does not take the call: three dimensions with
+    gaps (flattened without a copy, and with one: then each linear has an activation of its own), and a strided bias."""
+    from lingua_amd import float8
+    (a, g), (b, _) = _layer(256, 128, True, 3), _layer(256, 64, True, 4)
+    x = _input((2, 80, 256), kind == "slice", g)
+    if kind == "transposed":
+        x = x.transpose(0, 1)
+    if kind == "bias view":
+        for lin in (a, b):
+            wide = torch.zeros(2 * lin.bias.numel(), dtype=torch.bfloat16, device="cuda")
+            wide[::2] = lin.bias.detach()
+            lin.bias = torch.nn.Parameter(wide[::2])
+    filed = []
+    put = float8._fwd_cast.put
+    monkeypatch.setattr(float8._fwd_cast, "put", lambda *args: filed.append(args) or put(*args))
+    form(True)
+    with torch.no_grad():
+        out = [a(x), b(x)]
+    assert len(filed) == (2 if kind == "transposed" else 1)
+    form(False)
+    with torch.no_grad():
+        _same(out, [a(x), b(x)])
+
+
 def test_what_the_python_form_refuses_stays_refused(form):
     lin, g = _layer(64, 48, False, 1)
     x = torch.randn(33, 64, generator=g).cuda()
