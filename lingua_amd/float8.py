@@ -458,14 +458,12 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
     if a is None and need_b and not (fp8_wgrad and a_tcast is not None):
         raise RuntimeError("Fp8LinearFn.backward: the bf16 input was not saved and no quantised copy stands in for it")
 
+    # the memo answers a linear once: both forms below go by this answer
+    hit = _bwd_cast.get(a, b_t.data_ptr()) if fp8_wgrad and a_tcast is None and config.share_input_casts else None
+    qat, sat = a_tcast or hit or (None, None)
     if (grad_a is None and fp8_wgrad == need_b and _native_call(grad_out, gemm_algo) and
             not torch.is_grad_enabled()):
-        hit = w_cast = None
-        if need_b and a_tcast is None and config.share_input_casts:
-            hit = _bwd_cast.get(a, b_t.data_ptr())
-        if need_a and config.cache_weight_casts:
-            w_cast = weight_cast_tensorwise_t(b_t, amax_b_t)
-        qat, sat = a_tcast or hit or (None, None)
+        w_cast = weight_cast_tensorwise_t(b_t, amax_b_t) if need_a and config.cache_weight_casts else None
         res = _lib.native_for(grad_out.get_device()).linear_bwd(
             grad_out, a if qat is None else None, b_t, amax_b_t, a_col_amax if qat is None else None, qat, sat, *(w_cast or (None, None)),
             need_a, need_b, need_bias, gemm_algo)
@@ -488,12 +486,7 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
             if g_col_amax is None:
                 g_col_amax = ops.col_amax(grad_out)
             qgt, sgt = ops.cast_colwise_transposed(grad_out, g_col_amax, on_lines=True)
-            hit = _bwd_cast.get(a, b_t.data_ptr()) if config.share_input_casts and a_tcast is None else None
-            if a_tcast is not None:
-                qat, sat = a_tcast
-            elif hit is not None:
-                qat, sat = hit
-            else:
+            if qat is None:
                 if a_col_amax is None:
                     a_col_amax = ops.col_amax(a)
                 qat, sat = ops.cast_colwise_transposed(a, a_col_amax, on_lines=True)

@@ -171,6 +171,24 @@ def test_gradients_that_need_a_copy_take_the_python_form(form):
     _same(*results)
 
 
+def test_weight_gradients_beside_such_gradients_share_the_input_cast(form, monkeypatch):
+    """Two linears on one activation quantise it along its tokens once, whichever form their gradients take."""
+    from lingua_amd import float8
+    results = []
+    for on in (False, True):
+        (a, g), (b, _) = _layer(64, 48, False, 9), _layer(64, 32, False, 10)
+        x = _input((40, 64), False, g).requires_grad_(True)
+        form(on)
+        filed = []
+        with monkeypatch.context() as m:
+            put = float8._bwd_cast.put
+            m.setattr(float8._bwd_cast, "put", lambda *args: filed.append(args[0]) or put(*args))
+            (a(x).sum() + b(x).sum()).backward()
+        assert len(filed) == 1
+        results.append([x.grad, a.weight.grad, b.weight.grad])
+    _same(*results)
+
+
 def test_key_tells_tensors_apart_as_the_tuple_did():
     from lingua_amd import _lib
     key = _lib.native_for(0).key
