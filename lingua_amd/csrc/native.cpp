@@ -85,6 +85,11 @@ PyObject *wrap(const Tensor &t) {
   if (!t.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(t);
 }
+bool truth(PyObject *o) {  // as `if` takes it: a switch of the configuration may hold any number
+  const int t = PyObject_IsTrue(o);
+  if (t < 0) throw python_error();
+  return t != 0;
+}
 bool tensors(PyObject *const *args, int n) {  // Tensor, Parameter or None, and no mode that wants to see what is done to them
   for (int i = 0; i < n; ++i)
     if (args[i] != Py_None && !plain_type(args[i])) return false;
@@ -115,7 +120,7 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!tensors(args, 5) || !tensors(args + 8, 2) || args[0] == Py_None || args[1] == Py_None) Py_RETURN_NONE;
   const Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]);
   const Tensor bias = arg(args[2]), qx_in = arg(args[3]), sx_in = arg(args[4]), qw = arg(args[8]), sw = arg(args[9]);
-  const bool x_ready = args[5] == Py_True, want_qx = args[6] == Py_True, want_col = args[7] == Py_True, want_amax = args[10] == Py_True;
+  const bool x_ready = truth(args[5]), want_qx = truth(args[6]), want_col = truth(args[7]), want_amax = truth(args[10]);
   const int64_t algo = PyLong_AsLongLong(args[11]);
   if (!x.is_cuda()) Py_RETURN_NONE;
   const int device = x.get_device();
@@ -187,7 +192,7 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (!tensors(args, 9) || args[0] == Py_None || args[2] == Py_None || args[3] == Py_None) Py_RETURN_NONE;
   const Tensor &g = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[2]), &amax = THPVariable_Unpack(args[3]);
   const Tensor a = arg(args[1]), a_col_in = arg(args[4]), qat_in = arg(args[5]), sat_in = arg(args[6]), qwt_in = arg(args[7]), swt_in = arg(args[8]);
-  const bool need_a = args[9] == Py_True, need_b = args[10] == Py_True, need_bias = args[11] == Py_True;
+  const bool need_a = truth(args[9]), need_b = truth(args[10]), need_bias = truth(args[11]);
   const int algo = (int)PyLong_AsLongLong(args[12]);
   if (!g.is_cuda()) Py_RETURN_NONE;
   const int device = g.get_device();

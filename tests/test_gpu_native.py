@@ -140,6 +140,24 @@ def test_inference_on_operands_the_extension_leaves_shares_the_cast(form, monkey
         _same(out, [a(x), b(x)])
 
 
+def test_switches_count_as_true_where_python_takes_them_so(form, monkeypatch):
+    """A configuration read from a file may hold 1 for True."""
+    from lingua_amd import float8
+    results = []
+    for yes in (True, 1):
+        for name in ("share_input_casts", "fp8_wgrad"):
+            monkeypatch.setattr(float8.config, name, yes)
+        (a, g), (b, _) = _layer(64, 48, True, 9), _layer(64, 32, True, 10)
+        x = _input((80, 64), False, g).requires_grad_(True)
+        made = form(True)
+        (torch.cat([a(x), b(x)], dim=1) ** 2).sum().backward()
+        with torch.no_grad():
+            out = [a(x), b(x)]
+        assert made.made == 6
+        results.append([*out, x.grad, a.weight.grad, b.weight.grad, a.bias.grad, b.bias.grad])
+    _same(*results)
+
+
 def test_what_the_python_form_refuses_stays_refused(form):
     lin, g = _layer(64, 48, False, 1)
     x = torch.randn(33, 64, generator=g).cuda()
