@@ -1488,11 +1488,14 @@ extern "C" const char *l8_gemm_algo_name(int algo) {
 // tile, which eight waves share out over twice as many wave slots, weighs more than the K loop
 static int pick_plain_big(int64_t K) { return K >= 4096 ? 5 : 3; }
 
+// 9/16 of the units have a 256 x 256 tile
+static bool fills_with_big_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256) * 16 >= (int64_t)num_cus() * 9; }
+
 static int pick_algo(int64_t M, int64_t N, int64_t K) {
   if (M <= 8) return kSkinnyAlgo;  // whatever the chip: the smallest calls do not pay for asking
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
-  const bool big = tiles(256, 256) * 16 >= cus * 9;  // 9/16 of the units have a 256 x 256 tile
+  const bool big = fills_with_big_tiles(M, N);
   // A few tokens: the weight's bytes are what counts (skinny_kernels.hip).  us, against the best tile: [20,2048].
   // [2048,2048] 4.2 / 7.5, [64,11008].[4096,11008] 18.9 / 28.8, [32,4096].[11008,4096] 14.6 / 13.5; from 48 tokens on
   // the 64 x 64 tiles win where there are enough of them ([48,4096].[11008,4096] 17.6 / 14.0, [40,4096].[8192,4096]
@@ -1610,7 +1613,12 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
              "l8_gemm_nt: bad scale mode");
   L8_REQUIRE(M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31), "l8_gemm_nt: dimension too large");
   L8_REQUIRE(algo >= 0 && algo <= kNumAlgos, "l8_gemm_nt: algo %d out of range 0..%d", algo, kNumAlgos);
-  if (algo == 0) algo = pick_algo(M, N, K);
+  const bool chosen = algo == 0;
+  if (chosen) algo = pick_algo(M, N, K);
+  // Rows so far apart that 256 of them pass the 32-bit offsets below: a problem of middling size, which taller tiles would
+  // only serve faster, takes 128 x 128 ones and is refused where 128 rows are too many.
+  if (chosen && kAlgos[algo - 1].persistent && !fills_with_big_tiles(M, N) && (256 * lda + K >= (1LL << 31) || 256 * ldb + K >= (1LL << 31)))
+    algo = 2;
   if (kAlgos[algo - 1].persistent) {
     // the persistent kernel stores 16 aligned bytes (eight columns) per lane and reads the row scales 16 bytes
     // at a time; operands that do not allow that go to the plain kernel with the same tile shape

@@ -207,6 +207,21 @@ def test_random_operands_vs_oracle(algo):
             assert rel_l2(out, want) <= TOL, (algo, M, N, K)
 
 
+def test_rows_so_far_apart_that_only_the_smaller_tiles_can_address_them():
+    """256 rows of A 8 MiB apart pass the 32-bit offsets of a tile, 128 do not: a problem whose choice may fall on taller tiles
+    is computed all the same, on the smaller ones.  Integers of magnitude up to 4: the sums are exact."""
+    from lingua_amd import _lib, ops
+    M, N, K, lda = 130, 16640, 2064, 1 << 23
+    g = torch.Generator().manual_seed(3)
+    qa = torch.randint(-4, 5, (M, K), generator=g).float().cuda().to(torch.float8_e4m3fn)
+    qb = torch.randint(-4, 5, (N, K), generator=g).float().cuda().to(torch.float8_e4m3fn)
+    sa, sb = torch.ones(M, 1, device="cuda"), torch.ones(N, 1, device="cuda")
+    assert _lib.load().l8_gemm_pick(M, N, K) in (23, 24)
+    far = torch.empty_strided((M, K), (lda, 1), dtype=torch.float8_e4m3fn, device="cuda")
+    far.view(torch.uint8).copy_(qa.view(torch.uint8))
+    assert torch.equal(ops.gemm_nt(far, qb, sa, sb), ops.gemm_nt(qa, qb, sa, sb))
+
+
 def test_output_leading_dimension_and_unaligned_n():
     from lingua_amd import ops
     g = torch.Generator().manual_seed(9)
