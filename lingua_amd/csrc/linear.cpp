@@ -89,7 +89,8 @@ static int check_operands(const l8_linear_fwd_args &a, int64_t ldqx, int64_t ldq
   L8_REQUIRE(a.K > 0 && a.K % 16 == 0, "l8_linear_fwd: K=%lld must be positive and a multiple of 16", (long long)a.K);
   L8_REQUIRE(a.M < (1LL << 31) && a.N < (1LL << 31) && a.K < (1LL << 31), "l8_linear_fwd: dimension too large");
   L8_REQUIRE(aligned(a.qx, 16) && aligned(a.qw, 16), "l8_linear_fwd: qx and qw must be 16-byte aligned");
-  L8_REQUIRE(ldqx >= a.K && ldqw >= a.K && ldqx % 16 == 0 && ldqw % 16 == 0, "l8_linear_fwd: ldqx=%lld and ldqw=%lld must be multiples of 16, >= K",
+  auto rows = [&](const void *q, int64_t ld) { return !q || (ld >= a.K && ld % 16 == 0); };
+  L8_REQUIRE(rows(a.qx, ldqx) && rows(a.qw, ldqw), "l8_linear_fwd: ldqx=%lld and ldqw=%lld must be multiples of 16, >= K",
              (long long)ldqx, (long long)ldqw);
   L8_REQUIRE(a.y && a.ldy >= a.N, "l8_linear_fwd: y is null, or ldy=%lld < N=%lld", (long long)a.ldy, (long long)a.N);
   L8_REQUIRE(a.algo >= 0 && a.algo <= l8_gemm_algo_count(), "l8_linear_fwd: algo %lld out of range", (long long)a.algo);

@@ -86,6 +86,11 @@ def test_linear_call_validates_its_arguments_on_the_host():
     assert lib.l8_linear_fwd(pack(x_ready=1)) == -1 and "x_ready" in _lib.last_error()
     assert lib.l8_linear_fwd(pack(w_ready=1)) == -1 and "w_ready" in _lib.last_error()
     assert lib.l8_linear_fwd(pack(qx=fake)) == -1 and lib.l8_linear_fwd(None) == -1
+    # a row stride counts where its operand is given
+    assert lib.l8_linear_fwd_rows(pack(), 0, 0) == -1 and "workspace" in _lib.last_error()
+    assert lib.l8_linear_fwd_rows(pack(qx=fake, sx=fake), 128, 0) == -1 and "workspace" in _lib.last_error()
+    for given, ldqx, ldqw in ((dict(qx=fake, sx=fake), 48, 128), (dict(qx=fake, sx=fake), 72, 128), (dict(qw=fake, sw=fake), 128, 48)):
+        assert lib.l8_linear_fwd_rows(pack(**given), ldqx, ldqw) == -1 and "ldqx" in _lib.last_error()
 
 
 @pytest.mark.parametrize("change,named", [
