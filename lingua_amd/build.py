@@ -47,7 +47,7 @@ def _native_cmd():
 
 
 def _run(cmd, verbose):
-    """Runs one hipcc command; returns the register / scratch figures of the kernels it compiled
+    """Runs one compiler command; returns the register / scratch figures of the kernels it compiled
     ({mangled name: {"VGPRs": n, "AGPRs": n, "ScratchSize": bytes per lane, "VGPRs Spill": n, "SGPRs Spill": n}})."""
     if verbose:
         print(" ".join(cmd), flush=True)
@@ -67,7 +67,7 @@ def _run(cmd, verbose):
         rest.append(line)
     err = "\n".join(rest)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed ({res.returncode}):\n{err}")
+        raise RuntimeError(f"{os.path.basename(cmd[0])} failed ({res.returncode}):\n{err}")
     if verbose and err.strip():
         print(err, file=sys.stderr)
     return usage
@@ -100,7 +100,9 @@ def _check_usage(usage) -> None:
 
 
 def build(verbose: bool = False) -> str:
-    """Compiles every source (in parallel, one object each) and links the shared library."""
+    """Compiles every source (in parallel, one object each) and links the shared library; beside that the host extension.
+    The library needs hipcc alone: it is linked also where the extension cannot be compiled (no g++, no PyTorch for ROCm),
+    which is reported afterwards."""
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     extra = os.environ.get("LINGUA_FP8_HIPCC_EXTRA", "").split()
     obj_dir = OBJ_DIR if not os.environ.get("LINGUA_FP8_LIB") else os.path.join(OBJ_DIR, os.path.splitext(os.path.basename(LIB_PATH))[0])
@@ -108,16 +110,19 @@ def build(verbose: bool = False) -> str:
     objs = [os.path.join(obj_dir, os.path.splitext(src)[0] + ".o") for src in SOURCES]
     cmds = [[hipcc, *HIPCC_FLAGS, *extra, *(["-Rpass-analysis=kernel-resource-usage"] if src.endswith(".hip") else []),
              "-c", os.path.join(CSRC, src), "-o", obj] for src, obj in zip(SOURCES, objs)]
-    if not os.environ.get("LINGUA_FP8_LIB"):   # a tuning variant of the library is used through the same extension
-        cmds.append(_native_cmd())
-    with ThreadPoolExecutor(max_workers=min(len(cmds), os.cpu_count() or 1)) as pool:
+    with ThreadPoolExecutor(max_workers=min(len(cmds) + 1, os.cpu_count() or 1)) as pool:
+        native = None
+        if not os.environ.get("LINGUA_FP8_LIB") or not os.path.exists(NATIVE_PATH):   # (a tuning variant is used through the same extension)
+            native = pool.submit(lambda: _run(_native_cmd(), verbose))
         usages = list(pool.map(lambda c: _run(c, verbose), cmds))
-    usage = {k: v for u in usages for k, v in u.items()}
-    with open(os.path.join(obj_dir, "resource_usage.txt"), "w") as f:
-        for name in sorted(usage):
-            f.write(f"{name} {usage[name]}\n")
-    _check_usage(usage)
-    _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs], verbose)
+        usage = {k: v for u in usages for k, v in u.items()}
+        with open(os.path.join(obj_dir, "resource_usage.txt"), "w") as f:
+            for name in sorted(usage):
+                f.write(f"{name} {usage[name]}\n")
+        _check_usage(usage)
+        _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs], verbose)
+        if native is not None:
+            native.result()
     return LIB_PATH
 
 

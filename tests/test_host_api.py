@@ -413,6 +413,41 @@ def test_build_refuses_a_persistent_gemm_kernel_that_uses_scratch():
             assert "gemm_nt_stream_kernel" + inst in text, inst
 
 
+@pytest.mark.parametrize("variant", [False, True])
+@pytest.mark.parametrize("there", [False, True])
+@pytest.mark.parametrize("compiles", [False, True])
+def test_build_links_the_library_whatever_becomes_of_the_host_extension(monkeypatch, tmp_path, variant, there, compiles):
+    """The library needs hipcc alone.  The extension is compiled with every build of the shipped library and, where it is
+    missing, with a tuning variant's; that it cannot be is an error, but one that leaves the library linked."""
+    from lingua_amd import build
+    ran = []
+
+    def run(cmd, verbose):
+        ran.append("native" if "native.cpp" in cmd[-1] else "link" if "-shared" in cmd else "object")
+        if ran[-1] == "native" and not compiles:
+            raise RuntimeError("g++ failed")
+        return {}
+
+    monkeypatch.setattr(build, "_run", run)
+    monkeypatch.setattr(build, "_native_cmd", lambda: ["g++", "native.cpp"])
+    monkeypatch.setattr(build, "_check_usage", lambda usage: None)
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path))
+    monkeypatch.setattr(build, "NATIVE_PATH", str(tmp_path / "_native.so"))
+    if there:
+        (tmp_path / "_native.so").touch()
+    if variant:
+        monkeypatch.setenv("LINGUA_FP8_LIB", str(tmp_path / "variant.so"))
+    else:
+        monkeypatch.delenv("LINGUA_FP8_LIB", raising=False)
+    tried = not (variant and there)
+    if tried and not compiles:
+        with pytest.raises(RuntimeError, match="failed"):
+            build.build()
+    else:
+        build.build()
+    assert ran.count("link") == 1 and ran.count("native") == tried
+
+
 def test_converter_drops_compiled_code_like_the_reference():
     """lingua/float8.py:187 resets the dynamo code caches after the swap ("force re-compile everything"): a
     module compiled before the conversion is traced again by its next call.  Runs on the CPU with a filter that
