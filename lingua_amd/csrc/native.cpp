@@ -75,9 +75,9 @@ int64_t fp8_rows(const Tensor &t, int64_t rows, int64_t cols, int device) {
     return 0;
   return rows > 1 ? t.stride(0) : cols;
 }
-// A new one, its rows on 128-byte lines (figures in linear.cpp).
-Tensor empty_fp8(int64_t rows, int64_t cols, const at::TensorOptions &o) {
-  return at::empty_strided({rows, cols}, {(cols + 127) / 128 * 128, 1}, o.dtype(at::kFloat8_e4m3fn));
+// A new one, its rows on 128-byte lines (figures in linear.cpp) or dense.
+Tensor empty_fp8(int64_t rows, int64_t cols, const at::TensorOptions &o, bool on_lines = true) {
+  return at::empty_strided({rows, cols}, {on_lines ? (cols + 127) / 128 * 128 : cols, 1}, o.dtype(at::kFloat8_e4m3fn));
 }
 
 Tensor arg(PyObject *o) { return o == Py_None ? Tensor() : THPVariable_Unpack(o); }
@@ -174,10 +174,10 @@ PyObject *linear_fwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // A matrix quantised along its rows' direction, padded to 16 of them, in the layout that the weight gradient multiplies with.
-void cast_colwise_t(const Tensor &like, const Rows &m, const Tensor &col, Tensor &q, Tensor &s, void *stream) {
+void cast_colwise_t(const Tensor &like, const Rows &m, const Tensor &col, bool on_lines, Tensor &q, Tensor &s, void *stream) {
   const auto o = like.options();
   const int64_t padded = (m.rows + 15) / 16 * 16;
-  q = empty_fp8(m.cols, padded, o);
+  q = empty_fp8(m.cols, padded, o, on_lines);
   s = at::empty({m.cols, 1}, o.dtype(at::kFloat));
   check(lib.l8_cast_colwise_transposed_pad(m.p, m.rows, m.cols, m.ld, col.const_data_ptr<float>(), q.mutable_data_ptr(), q.stride(0), padded,
                                            s.mutable_data_ptr<float>(), stream), "l8_cast_colwise_transposed_pad");
@@ -242,7 +242,7 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (need_b) {
       Tensor qgt, sgt;
       if (qat.defined()) {
-        cast_colwise_t(g, rg, g_col, qgt, sgt, stream);
+        cast_colwise_t(g, rg, g_col, true, qgt, sgt, stream);
       } else {
         Tensor a_col = a_col_in;
         if (!a_col.defined()) {
@@ -271,20 +271,21 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// cast_colwise_transposed(a, col amax) -> (q, s) or None, as in lingua_amd.ops
+// cast_colwise_transposed(a, col amax, on_lines) -> (q, s) or None, as in lingua_amd.ops
 PyObject *cast_colwise_transposed(PyObject *, PyObject *const *args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 2) throw std::runtime_error("cast_colwise_transposed: 2 arguments");
+  if (n != 3) throw std::runtime_error("cast_colwise_transposed: 3 arguments");
   if (!tensors(args, 2) || args[0] == Py_None || args[1] == Py_None) Py_RETURN_NONE;
   const Tensor &a = THPVariable_Unpack(args[0]), &col = THPVariable_Unpack(args[1]);
   if (!a.is_cuda()) Py_RETURN_NONE;
   const int device = a.get_device();
   Rows ra;
   if (a.dim() != 2 || !as_rows(a, device, ra) || !dense(col, at::kFloat, ra.cols, device) || c10::hip::current_device() != device) Py_RETURN_NONE;
+  const bool on_lines = truth(args[2]);
   Tensor q, s;
   {
     pybind11::gil_scoped_release no_gil;
-    cast_colwise_t(a, ra, col, q, s, c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream());
+    cast_colwise_t(a, ra, col, on_lines, q, s, c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream());
   }
   return tuple_of({q, s});
   END_HANDLE_TH_ERRORS

@@ -64,11 +64,12 @@ class Fp8Config:
     use_custom_ops: bool = False
     # with fp8_wgrad: quantise the input along the token dimension already in
     # forward and keep that e4m3 [K,M] copy (+ K scales) for wgrad instead of the
-    # bf16 input: half the bytes held between forward and backward, the same
-    # kernels and the same results (plain autograd.Function route only)
+    # bf16 input: half the bytes held between forward and backward (M rounded up
+    # to 16, and to 128 where that adds at most an eighth), the same kernels and
+    # the same results (plain autograd.Function route only)
     save_fp8_input: bool = False
     # keep the quantised copies of every weight (row-wise for forward, tensor-wise transposed for dgrad:
-    # 2 bytes per parameter) until the weight's version counter moves, so that micro-batches between two
+    # 2 bytes per parameter, 2.25 for widths off 128) until the weight's version counter moves, so that micro-batches between two
     # optimizer steps (gradient accumulation) and evaluation passes quantise each weight once
     cache_weight_casts: bool = False
 
@@ -228,8 +229,8 @@ class _WeightCasts:
     """Quantised copies of weights, one slot per live weight tensor, valid while pointer, shape, strides, dtype,
     version counter and stream are what they were (an optimizer step advances the version).  A slot holds the
     weight by weak reference only and goes away with it, so the cache never holds more than two bytes per
-    parameter of the ``Fp8Linear`` weights that are alive, and a deleted model releases its copies.  Used only
-    with ``config.cache_weight_casts``."""
+    parameter of the ``Fp8Linear`` weights that are alive (and an eighth of that for rows on 128-byte lines), and a
+    deleted model releases its copies.  Used only with ``config.cache_weight_casts``."""
 
     def __init__(self):
         self.entries = {}   # id(weight) -> {"ref": weakref to the weight, "key": ..., "row": ..., "tw": ...}
@@ -257,7 +258,7 @@ class _WeightCasts:
         slot = self._slot(w) if config.cache_weight_casts else None
         if slot is not None and "row" in slot:
             return slot["row"]
-        value = ops.cast_rowwise(w, on_lines=True)
+        value = ops.cast_rowwise(w, on_lines=slot is None or ops.keeps_on_lines(w.shape[1]))
         if slot is not None:
             slot["row"] = value
         return value
@@ -266,7 +267,7 @@ class _WeightCasts:
         slot = self._slot(w) if config.cache_weight_casts else None
         if slot is not None and "tw" in slot:
             return slot["tw"]
-        value = ops.cast_tensorwise_t_rows(w, amax_rows, on_lines=True)
+        value = ops.cast_tensorwise_t_rows(w, amax_rows, on_lines=slot is None or ops.keeps_on_lines(w.shape[0]))
         if slot is not None:
             slot["tw"] = value
         return value
@@ -437,9 +438,10 @@ def input_cast_for_wgrad(a, a_col_amax, user):
     hit = _fwd_tcast.get(a, user) if config.share_input_casts else None
     if hit is not None:
         return hit
-    value = _lib.native_for(a.get_device()).cast_colwise_transposed(a, a_col_amax) if _native_call(a, 0) else None
+    on_lines = ops.keeps_on_lines((a.shape[0] + 15) // 16 * 16)
+    value = _lib.native_for(a.get_device()).cast_colwise_transposed(a, a_col_amax, on_lines) if _native_call(a, 0) else None
     if value is None:
-        value = ops.cast_colwise_transposed(a, a_col_amax, on_lines=True)
+        value = ops.cast_colwise_transposed(a, a_col_amax, on_lines=on_lines)
     if config.share_input_casts:
         _fwd_tcast.put(a, value, user)
     return value

@@ -109,6 +109,12 @@ def _empty_fp8(rows: int, cols: int, device, on_lines: bool) -> torch.Tensor:
     return torch.empty_strided((rows, cols), ((cols + 127) // 128 * 128, 1), dtype=torch.float8_e4m3fn, device=device)
 
 
+def keeps_on_lines(cols: int) -> bool:
+    """Do copies that are kept between calls have their rows on 128-byte lines?  Where that adds at most an eighth to them;
+    shorter rows stay dense (16 bytes would become 128)."""
+    return -cols % 128 * 8 <= cols
+
+
 def cast_rowwise(x: torch.Tensor, col_amax: Optional[torch.Tensor] = None, want_q: bool = True,
                  out_q: Optional[torch.Tensor] = None, out_scale: Optional[torch.Tensor] = None, on_lines: bool = False):
     """Row-wise amax -> scale -> e4m3fn.  Returns (q [R,C] fp8 | None, scale [R,1] fp32, amax [R,1] bf16).

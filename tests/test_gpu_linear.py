@@ -607,6 +607,30 @@ def test_weight_casts_kept_between_optimizer_steps():
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))
 
 
+@pytest.mark.parametrize("native", [True, False])
+@pytest.mark.parametrize("tokens,K,N", [(1, 16, 48), (16, 112, 128), (130, 272, 144), (900, 1040, 912), (1021, 2048, 1024)])
+def test_what_is_kept_between_calls_is_at_most_an_eighth_larger_than_its_bytes(monkeypatch, native, tokens, K, N):
+    """Weights kept quantised and the quantised input kept for backward: short rows are not spread to 128-byte lines."""
+    from lingua_amd import Fp8Linear, float8
+    monkeypatch.setattr(float8.config, "cache_weight_casts", True)
+    monkeypatch.setattr(float8.config, "save_fp8_input", True)
+    if not native:
+        monkeypatch.setattr(float8, "_native_call", lambda a, algo: False)
+    float8.clear_cast_memos()
+    lin = Fp8Linear(K, N, bias=False, device="cuda", dtype=torch.bfloat16)
+    x = seeded_bf16((tokens, K), seed=5).cuda().requires_grad_(True)
+    y = lin(x)
+    saved = [t for t in y.grad_fn.saved_tensors if t.dtype == torch.float8_e4m3fn]
+    y.backward(seeded_bf16((tokens, N), seed=6).cuda())
+    slot = float8._weight_casts.entries[id(lin.weight)]
+    kept = saved + [slot["row"][0], slot["tw"][0]]
+    assert len(kept) == 3
+    for q in kept:
+        assert q.untyped_storage().nbytes() * 8 <= q.numel() * 9
+    assert saved[0].numel() == K * ((tokens + 15) // 16 * 16)
+    float8.clear_cast_memos()
+
+
 def test_large_linear_with_bias_vs_oracle():
     """nn.Linear(4096, 4096, bias=True) on 4096 tokens: 256 tiles, so forward takes the persistent kernel's bias
     instantiation; forward (lingua/float8.py:65-73 with the bias fused), dgrad and fp8 wgrad against the oracle on
