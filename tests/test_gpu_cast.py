@@ -478,7 +478,7 @@ def test_several_operands_in_one_launch(C, rows):
 @pytest.mark.parametrize("R,C", [(33, 144), (1, 16), (130, 1040), (48, 256), (257, 4112)])
 def test_rows_on_lines_hold_what_dense_rows_hold(R, C):
     """on_lines moves the rows of a quantised operand to 128-byte lines, nothing else: every cast's bytes and scales, and the
-    products that read them (one, several in one launch, a linear's forward in one call)."""
+    products that read them (one, several with one operand, a linear's forward in one call)."""
     from lingua_amd import ops
     x, w, h = (seeded_bf16((n, C), seed=n + C).cuda() for n in (R, 48, R))
     amax, col = ops.cast_rowwise(x)[2], ops.col_amax(x)

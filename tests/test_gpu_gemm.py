@@ -144,9 +144,42 @@ def test_products_with_one_operand_in_one_launch(rows, N, K, together):
         assert out.shape == want.shape and torch.equal(out.view(torch.int16), want.view(torch.int16))
 
 
+def spread(q, ld):
+    """q with its rows `ld` bytes apart and NaN codes between them."""
+    wide = torch.full((q.shape[0], ld), 0x7f, dtype=torch.uint8, device="cuda")
+    wide[:, :q.shape[1]] = q.view(torch.uint8)
+    return wide.view(torch.float8_e4m3fn)[:, :q.shape[1]]
+
+
+@pytest.mark.parametrize("rows,N,K", [((2008, 2048, 520), 2048, 272), ((1536, 1500), 2048, 400), ((2817, 2900, 3070), 2200, 1040)])
+def test_products_in_one_launch_with_rows_apart(rows, N, K):
+    """Operands whose rows are further apart than they are long, one distance for A and another for B, have the bits of dense
+    ones and no byte from between the rows; operands of different distances go one by one."""
+    import struct
+    from lingua_amd import _lib, ops
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        parts = [v for m in rows for v in (0, m, 0, 0)]
+        assert _lib.load().l8_gemm_multi_pays(struct.pack(f"{len(parts)}q", *parts), len(rows), N, K)
+    g = torch.Generator().manual_seed(970 + N)
+    qb = random_fp8_bytes((N, K), g).cuda().view(torch.float8_e4m3fn)
+    sb = (torch.rand(N, 1, generator=g) + 0.5).cuda()
+    qas = [random_fp8_bytes((m, K), g).cuda().view(torch.float8_e4m3fn) for m in rows]
+    sas = [(torch.rand(m, 1, generator=g) + 0.5).cuda() for m in rows]
+    lines = (K + 127) // 128 * 128
+    want = ops.gemm_nt_multi(qas, qb, sas, sb)
+    for ldas, ldb in (([lines] * len(rows), lines), ([lines + 16] * len(rows), K), ([K] * len(rows), lines)):
+        got = ops.gemm_nt_multi([spread(q, ld) for q, ld in zip(qas, ldas)], spread(qb, ldb), sas, sb)
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(got, want))
+    got = ops.gemm_nt_multi([spread(q, lines + 16 * i) for i, q in enumerate(qas)], spread(qb, lines), sas, sb)
+    for qa, sa, out in zip(qas, sas, got):
+        assert torch.equal(out.view(torch.int16), ops.gemm_nt(qa, qb, sa, sb).view(torch.int16))
+
+
 @pytest.mark.parametrize("algo,mnk", [(0, (40, 52, 272)), (2, (130, 200, 144)), (2, (256, 256, 128)), (12, (256, 256, 128)),
                                       (12, (300, 520, 400)), (12, (4136, 4104, 272)), (11, (520, 264, 144)), (17, (33, 50, 1040)),
-                                      (18, (128, 128, 256)), (21, (65, 70, 128)), (22, (32, 64, 400))])
+                                      (18, (128, 128, 256)), (21, (65, 70, 128)), (22, (32, 64, 400)), (14, (520, 264, 144)),
+                                      (23, (256, 128, 128)), (23, (300, 520, 400)), (23, (4136, 4104, 272)), (23, (4136, 4104, 128)),
+                                      (24, (128, 256, 128)), (24, (300, 520, 400)), (24, (4136, 4104, 272)), (24, (4136, 4104, 128))])
 def test_product_added_to_what_the_output_holds(algo, mnk):
     """add=True leaves the bits of out.add_(product): every kernel's epilogue (interior and ragged tiles, a workgroup's
     second tile, a configuration without an add of its own), an output with a row stride, nothing written beside it."""
