@@ -90,9 +90,9 @@ bool truth(PyObject *o) {  // as `if` takes it: a switch of the configuration ma
   if (t < 0) throw python_error();
   return t != 0;
 }
-bool tensors(PyObject *const *args, int n) {  // Tensor, Parameter or None, and no mode that wants to see what is done to them
+bool tensors(PyObject *const *args, int n) {  // Tensor or Parameter with memory of its own (not a batch under vmap) or None, and no mode that wants to see what is done to them
   for (int i = 0; i < n; ++i)
-    if (args[i] != Py_None && !plain_type(args[i])) return false;
+    if (args[i] != Py_None && !(plain_type(args[i]) && THPVariable_Unpack(args[i]).has_storage())) return false;
   return !c10::impl::dispatch_mode_enabled();
 }
 PyObject *tuple_of(std::initializer_list<Tensor> ts) {

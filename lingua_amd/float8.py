@@ -501,8 +501,9 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
         grad_b = None
 
     grad_bias = None
-    if need_bias:   # a backward pass that is itself differentiated, and rows off 16-byte lines, need PyTorch's sum
-        own = grad_out.is_cuda and not torch.is_grad_enabled() and ops.rows_on_16_bytes(grad_out)
+    if need_bias:   # a backward pass that is itself differentiated, a batch of gradients and rows off 16-byte lines need PyTorch's sum
+        own = (grad_out.is_cuda and not torch.is_grad_enabled() and type(grad_out) is torch.Tensor and
+               torch._C._has_storage(grad_out) and ops.rows_on_16_bytes(grad_out))
         grad_bias = ops.col_sum(grad_out) if own else grad_out.sum(dim=0)
     return grad_a, grad_b, grad_bias
 

@@ -189,6 +189,19 @@ def test_gradients_that_need_a_copy_take_the_python_form(form):
     _same(*results)
 
 
+@pytest.mark.parametrize("on", [False, True])
+def test_bias_gradients_of_a_batch_of_output_gradients(form, on):
+    """A linear of which the bias alone learns has vectorised gradients (is_grads_batched): no kernel sees its backward pass."""
+    lin, g = _layer(64, 48, True, 9)
+    lin.weight.requires_grad_(False)
+    x = _input((40, 64), False, g)
+    form(on)
+    y = lin(x)
+    grads = torch.randn(3, 40, 48, generator=g).to(torch.bfloat16).cuda()
+    batch, = torch.autograd.grad(y, lin.bias, grads, is_grads_batched=True)
+    _same([batch], [grads.sum(dim=1)])
+
+
 def test_weight_gradients_beside_such_gradients_share_the_input_cast(form, monkeypatch):
     """Two linears on one activation quantise it along its tokens once, whichever form their gradients take."""
     from lingua_amd import float8
