@@ -430,14 +430,15 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const uint16_t *__restric
   }
 }
 
-// bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
 // ---------------------------------------------------------------------------
 // Column sums of bf16 x (the bias gradient, lingua/float8.py:127), in fp32, rounded to bf16 once.  Bound by memory from a few
 // thousand rows on, by latency below: a workgroup owns 128 columns -- two lines of every row, which 64 columns read at the same
 // rate up to 4096 columns and 10 % slower beyond, and 256 half as fast at [16384,2048] -- and a slab of rows, read 16 at a time
-// with eight loads in flight per thread.  Slabs until there are four workgroups per unit, of at least 128 rows; several slabs
-// leave fp32 partial sums that the second kernel adds in their order.  Up to 1024 rows one slab, by twice the threads: a launch less
-// ([512,4096] 5.2 / 3.1, [1021,2048] 5.2 / 5.0, [1024,11008] 7.6 / 5.8; [2048,2048] as one slab of 512 threads 6.5 against 4.9).  The order of every sum
+// with eight loads in flight per thread.  Slabs until there are four workgroups per unit, one per 128 rows begun at most and of
+// equal heights; several slabs leave fp32 partial sums that the second kernel adds in their order.  Up to 1024 rows one slab, by
+// twice the threads: a launch less ([512,4096] 5.2 / 3.1, [1021,2048] 5.2 / 5.0, [1024,11008] 7.6 / 5.8; [2048,2048] as one slab of
+// 512 threads 6.5 against 4.9).  From HBM its few workgroups take longer, with two launches to enqueue / with one [400,4096]
+// 8.4 / 5.9, [700,4096] 9.8 / 8.0, [1021,4096] 8.6 / 10.5, [1021,11008] 11.1 / 10.9: even at the limit.  The order of every sum
 // hangs on the shape and the number of compute units.  us, PyTorch's sum / this, back to back: [256,1024] 9.2 / 2.6, [1021,2048] 11.6 / 5.0, [1801,11040] 88 / 12,
 // [4096,4096] 19.8 / 9.4, [5580,12176] 369 / 33, [16384,2048] 28 / 16, [16384,11008] 69 / 68 (a copy's rate: 64)
 // ---------------------------------------------------------------------------
@@ -481,6 +482,7 @@ __global__ __launch_bounds__(256) void col_sum_fold_kernel(const float *__restri
   out[c] = (uint16_t)bf16_rne_bits(t);
 }
 
+// bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
 __global__ __launch_bounds__(1024) void amax_reduce_kernel(const uint16_t *__restrict__ amax, int64_t n,
                                                            uint16_t *__restrict__ out) {
   __shared__ uint32_t red[16];

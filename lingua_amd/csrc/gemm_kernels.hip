@@ -89,8 +89,8 @@ typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
 // 16-byte-per-lane buffer store with a scalar-register offset, followed by two wait states.  A vector-ALU write to
 // one of the store's data registers right behind it can reach the register before the store has read it: with two
-// waves per SIMD the eight-wave kernel stored, now and then, the next row pair's values in 4 of 64 lanes (found by
-// the exact-integer tests; two wait states cure it, which is what the compiler's hazard recognizer inserts behind
+// waves per SIMD a form of the persistent kernel with eight waves stored, now and then, the next row pair's values in
+// 4 of 64 lanes (found by the exact-integer tests; two wait states cure it, which is what the compiler's hazard recognizer inserts behind
 // stores of more than 8 bytes -- except behind buffer stores whose soffset is a register, like these, which an old
 // rule exempts).  Every such store in this file goes through here.
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1397,16 +1397,19 @@ struct Algo {
   X(2, 2, 4, 4, 5, 16, 0) /* 9: algo 1 with groups of 16                      */ \
   X(2, 4, 4, 2, 5, 8, 0)  /* 10: algo 3 with taller groups                    */
 
-// 18 .. 20: small problems, one workgroup per compute unit or fewer: a ring of 9 slots (3.5 K tiles ahead instead of 1.5;
-// a second workgroup has no use for the LDS) and smaller tiles where 128 x 128 ones would be too few
+// (R, and the _r of a name: 5 is the ring of five panels; beyond that it only says that the loop is the deep one, whose
+// ring holds as many whole K tiles as the LDS does -- deep_slots.  The t of a name counts 32x32 pieces of a wave's tile,
+// also in the persistent kernels, whose instruction is 16x16.)
+// 18 .. 20: small problems, one workgroup per compute unit or fewer: the deep loop (five K tiles in the ring for 128x128, six
+// for the smaller ones; a second workgroup has no use for the LDS) and smaller tiles where 128 x 128 ones would be too few
 #define L8_SMALL_ALGO_LIST(X)                         \
   X(2, 2, 2, 2, 9, 4, 0) /* 18: 128x128            */ \
   X(2, 2, 1, 2, 9, 4, 0) /* 19: 64x128             */ \
   X(2, 2, 2, 1, 9, 4, 0) /* 20: 128x64             */
 
 // X(WM, WN, TM, TN, R, GROUP_M, KS): the smallest tiles, K tiles dealt to two groups of waves with a ring each.  A trip
-// costs them 310 ns whatever they load (wait, barrier, LDS reads, one or two matrix instructions in a row; a ring of 13 or
-// 19 slots changed nothing), so two trips run side by side.  us, weight just written, one group / two / four:
+// costs them 310 ns whatever they load (wait, barrier, LDS reads, one or two matrix instructions in a row; a deeper ring
+// changed nothing), so two trips run side by side.  us, before the deep loop, weight just written, one group / two / four:
 // [333,8192].[2048,8192] 19.5 / 14.6 / 16.7, [100,11008].[4096,11008] 24.9 / 18.7 / 22.2, [200,4096].[4096,4096] 11.2 / 8.9 /
 // 9.3.  Larger tiles gain nothing: 128x128 [700,11008].[4096,11008] 39.2 / 39.7, 64x128 [1021,2048].[2048,2048] cold 9.3 / 9.9.
 #define L8_SPLIT_ALGO_LIST(X)                         \
@@ -1513,10 +1516,11 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   if (M <= 16 || (M <= 32 && !big) || (M <= kSkinnyMaxM && tiles(64, 64) * 16 < cus * 7)) return kSkinnyAlgo;
   // Otherwise the smallest tile that gives no compute unit a second workgroup: these kernels are bound by their LDS
   // traffic and by what a K tile costs whatever its size, so more units at work are worth more than the larger tile's
-  // economy.  us, 128 x 128 with two workgroups per unit (configuration 2) / chosen: [200,4096].[4096,4096] 19.1 / 8.9
-  // (64 x 64), [333,8192].[2048,8192] 32.8 / 14.6 (64 x 64), [1021,2048].[2048,2048] 12.3 / 9.3 (64 x 128),
-  // [512,4096].[4096,4096] 19.7 / 14.7 (128 x 64), [700,11008].[4096,11008] 67.2 / 49.5 (128 x 128, 9 slots),
-  // [2048,16384].[2048,16384] 86.8 / 72.1 (the same).
+  // economy.  us, operands of several problems in turn, 128 x 128 with two workgroups per unit (configuration 2) / 128 x 128 /
+  // 64 x 128 / 128 x 64 / 64 x 64: [200,4096].[4096,4096] 18.9 / 15.0 / 11.8 / 12.1 / 9.8, [333,8192].[2048,8192] 32.6 / 25.6 /
+  // 19.8 / 20.7 / 15.4, [1021,2048].[2048,2048] 12.4 / 11.1 / 9.8 / 10.0 / 12.9, [512,4096].[4096,4096] 19.3 / 16.0 / 13.7 / 13.8 /
+  // 18.6, [1392,3280].[1392,3280] 17.1 / 14.7 / 12.4 / 12.5 / 16.8, [333,2048].[8192,2048] 12.5 / 10.9 / 16.2 / 15.7 / 18.5,
+  // [700,11008].[4096,11008] 65.9 / 50.8 / 71.4 / 64.7 / 69.7, [2048,16384].[2048,16384] 87.6 / 75.0 / 99.9 / 98.5 / 128.3.
   if (tiles(64, 64) <= cus) return 21;
   if (tiles(64, 128) <= cus) return 19;
   if (tiles(128, 64) <= cus) return 20;
