@@ -274,6 +274,25 @@ int l8_swiglu_bwd_cast_rowwise(const void *dh, const void *h1, const void *h3, i
                                float *col_amax1, float *col_amax3,
                                void *workspace, int64_t workspace_bytes, void *stream);
 
+/* The same without g1 and g3 (C <= 16384), for a caller whose weight gradients take them from
+ * l8_swiglu_bwd_cast_transposed. */
+int l8_swiglu_bwd_cast_rowwise_q(const void *dh, const void *h1, const void *h3, int64_t R, int64_t C,
+                                 int64_t lddh, int64_t ld1, int64_t ld3, void *q1, void *q3, int64_t ldq,
+                                 float *scale1, float *scale3, float *col_amax1, float *col_amax3,
+                                 void *workspace, int64_t workspace_bytes, void *stream);
+
+/* The gate's two gradients and its output, quantised per column and written transposed: what
+ * l8_cast_colwise_transposed_pad writes for g1, g3 (of l8_swiglu_bwd_cast_rowwise) and h (of
+ * l8_swiglu_cast_rowwise), bit for bit, without any of the three in memory.
+ *   dh, h1, h3 bf16 [R,C];  col_amax1, col_amax3, col_amaxh fp32 [C]: column amaxes of g1, g3 and h
+ *   q1, q3, qh e4m3 [C,Rp], rows ldq >= Rp bytes apart; columns R .. Rp - 1 are zeros;  scale1, scale3, scaleh fp32 [C]
+ * Requires C % 8 == 0, bf16 leading dimensions % 8 == 0 and below 2 Mi. */
+int l8_swiglu_bwd_cast_transposed(const void *dh, const void *h1, const void *h3, int64_t R, int64_t C,
+                                  int64_t lddh, int64_t ld1, int64_t ld3,
+                                  const float *col_amax1, const float *col_amax3, const float *col_amaxh,
+                                  void *q1, void *q3, void *qh, int64_t ldq, int64_t Rp,
+                                  float *scale1, float *scale3, float *scaleh, void *stream);
+
 /* RMSNorm fused with the row-wise cast of its output.
  * Replaces RMSNorm.forward of lingua/transformer.py:283-289 (x.float(), x*x, mean, rsqrt, two
  * multiplies, type_as: seven eager kernels) followed by the cast of that output in the forward of

@@ -52,6 +52,8 @@ SIGNATURES = {
     "l8_swiglu_workspace": [_i64, _i64],
     "l8_swiglu_bwd_cast_rowwise": [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _p, _i64, _p, _p, _p, _p,
                                    _p, _i64, _p],
+    "l8_swiglu_bwd_cast_rowwise_q": [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _i64, _p, _p, _p, _p, _p, _i64, _p],
+    "l8_swiglu_bwd_cast_transposed": [_p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _i64, _p, _p, _p, _p],
     "l8_rmsnorm_cast_rowwise": [_p, _p, _int, _i64, _i64, _i64, ctypes.c_float, _p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p],
     "l8_rmsnorm_workspace": [_i64, _i64],
     "l8_rmsnorm_bwd": [_p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _p, _i64, _p],

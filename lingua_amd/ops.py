@@ -614,9 +614,10 @@ def swiglu_cast_rowwise(h1: torch.Tensor, h3: torch.Tensor, want_h: bool = True,
 
 def swiglu_bwd_cast_rowwise(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor,
                             col_amax1: Optional[torch.Tensor] = None, col_amax3: Optional[torch.Tensor] = None,
-                            on_lines: bool = False):
+                            on_lines: bool = False, want_g: bool = True):
     """Gradients of the SwiGLU gate and their row-wise casts in one pass.
-    Returns (g1, g3 [R,C] bf16, q1, q3 [R,C] fp8, scale1, scale3 [R,1] fp32)."""
+    Returns (g1, g3 [R,C] bf16, q1, q3 [R,C] fp8, scale1, scale3 [R,1] fp32); without ``want_g`` (C <= 16384) g1 and g3
+    are None."""
     dh = _rows_2d(dh, torch.bfloat16, "swiglu_bwd_cast_rowwise(dh)")
     h1 = _rows_2d(h1, torch.bfloat16, "swiglu_bwd_cast_rowwise(h1)")
     h3 = _rows_2d(h3, torch.bfloat16, "swiglu_bwd_cast_rowwise(h3)")
@@ -630,20 +631,52 @@ def swiglu_bwd_cast_rowwise(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor
     for ca in (col_amax1, col_amax3):
         if ca is not None and (ca.dtype != torch.float32 or ca.numel() != C or not ca.is_contiguous()):
             raise RuntimeError("swiglu_bwd_cast_rowwise: column amaxes must be contiguous fp32 tensors with C elements")
-    g1 = torch.empty((R, C), dtype=torch.bfloat16, device=dev)
-    g3 = torch.empty((R, C), dtype=torch.bfloat16, device=dev)
+    g1 = torch.empty((R, C), dtype=torch.bfloat16, device=dev) if want_g else None
+    g3 = torch.empty((R, C), dtype=torch.bfloat16, device=dev) if want_g else None
     q1, q3 = _empty_fp8(R, C, dev, on_lines), _empty_fp8(R, C, dev, on_lines)
     s1 = torch.empty((R, 1), dtype=torch.float32, device=dev)
     s3 = torch.empty((R, 1), dtype=torch.float32, device=dev)
     ws, ws_bytes = _swiglu_ws(R, C, dev, 2) if col_amax1 is not None else (None, 0)
-    with _timed("swiglu_bwd_cast_rowwise", R * C * 12 + 8 * R, dev):
-        code = _lib.load().l8_swiglu_bwd_cast_rowwise(
-            dh.data_ptr(), h1.data_ptr(), h3.data_ptr(), R, C, _ld(dh), _ld(h1), _ld(h3), g1.data_ptr(), g3.data_ptr(), C,
-            q1.data_ptr(), q3.data_ptr(), _ld(q1), s1.data_ptr(), s3.data_ptr(),
-            col_amax1.data_ptr() if col_amax1 is not None else None, col_amax3.data_ptr() if col_amax3 is not None else None,
-            ws.data_ptr() if ws is not None else None, ws_bytes, st)
+    results = (q1.data_ptr(), q3.data_ptr(), _ld(q1), s1.data_ptr(), s3.data_ptr(),
+               col_amax1.data_ptr() if col_amax1 is not None else None, col_amax3.data_ptr() if col_amax3 is not None else None,
+               ws.data_ptr() if ws is not None else None, ws_bytes, st)
+    operands = (dh.data_ptr(), h1.data_ptr(), h3.data_ptr(), R, C, _ld(dh), _ld(h1), _ld(h3))
+    with _timed("swiglu_bwd_cast_rowwise", R * C * (12 if want_g else 8) + 8 * R, dev):
+        if want_g:
+            code = _lib.load().l8_swiglu_bwd_cast_rowwise(*operands, g1.data_ptr(), g3.data_ptr(), C, *results)
+        else:
+            code = _lib.load().l8_swiglu_bwd_cast_rowwise_q(*operands, *results)
     _lib.check(code, "l8_swiglu_bwd_cast_rowwise")
     return g1, g3, q1, q3, s1, s3
+
+
+# Widest gate whose gradients need not be stored; see l8_swiglu_bwd_cast_rowwise_q.
+GATE_MAX_COLUMNS = 16384
+
+
+def swiglu_bwd_cast_transposed(dh: torch.Tensor, h1: torch.Tensor, h3: torch.Tensor, col_amax1: torch.Tensor,
+                               col_amax3: torch.Tensor, col_amax_h: torch.Tensor, on_lines: bool = False):
+    """``cast_colwise_transposed`` of the gate's gradients g1 and g3 and of its output h, all three made from dh, h1 and h3:
+    ``[(q1, scale1), (q3, scale3), (qh, scale_h)]``.  The column amaxes are those of g1, g3 and h (fp32 [C])."""
+    dh = _rows_2d(dh, torch.bfloat16, "swiglu_bwd_cast_transposed(dh)")
+    h1 = _rows_2d(h1, torch.bfloat16, "swiglu_bwd_cast_transposed(h1)")
+    h3 = _rows_2d(h3, torch.bfloat16, "swiglu_bwd_cast_transposed(h3)")
+    if not (dh.shape == h1.shape == h3.shape) or not (dh.device == h1.device == h3.device):
+        raise RuntimeError("swiglu_bwd_cast_transposed: dh, h1 and h3 must have the same shape and device")
+    st = _prep(dh, "swiglu_bwd_cast_transposed")
+    R, C = dh.shape
+    cols = (col_amax1, col_amax3, col_amax_h)
+    if R == 0 or any(ca.dtype != torch.float32 or ca.numel() != C or ca.device != dh.device or not ca.is_contiguous() for ca in cols):
+        raise RuntimeError("swiglu_bwd_cast_transposed: rows, and contiguous fp32 column amaxes with C elements, required")
+    Rp = (R + 15) // 16 * 16
+    qs = [_empty_fp8(C, Rp, dh.device, on_lines) for _ in range(3)]
+    ss = [torch.empty((C, 1), dtype=torch.float32, device=dh.device) for _ in range(3)]
+    with _timed("swiglu_bwd_cast_transposed", R * C * 9 + 24 * C, dh.device):
+        code = _lib.load().l8_swiglu_bwd_cast_transposed(
+            dh.data_ptr(), h1.data_ptr(), h3.data_ptr(), R, C, _ld(dh), _ld(h1), _ld(h3), *(ca.data_ptr() for ca in cols),
+            *(q.data_ptr() for q in qs), _ld(qs[0]), Rp, *(s.data_ptr() for s in ss), st)
+    _lib.check(code, "l8_swiglu_bwd_cast_transposed")
+    return list(zip(qs, ss))
 
 
 def rmsnorm_cast_rowwise(x: torch.Tensor, weight: torch.Tensor, eps: float, want_q: bool = True,

@@ -53,12 +53,17 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         h3 = ops.gemm_nt(qx, q3, sx, s3, None, algo=algo)
         del qx, q1, q3
         h_col = torch.empty(w2.shape[1], dtype=torch.float32, device=x.device) if fp8_wgrad and w2.requires_grad else None
-        h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=w2.requires_grad, col_amax=h_col, on_lines=True)
+        # where every weight learns, backward makes the operands of the three weight gradients that come out of the gate
+        # from h1, h3 and the gradient of h in one pass, and h itself is not kept
+        regate = (fp8_wgrad and w1.requires_grad and w3.requires_grad and w2.requires_grad and x.shape[0] > 0 and
+                  h1.shape[1] <= ops.GATE_MAX_COLUMNS)
+        h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=w2.requires_grad and not regate, col_amax=h_col, on_lines=True)
         q2, s2, amax_w2 = f8.weight_cast_rowwise(w2)
         y = ops.gemm_nt(qh, q2, sh, s2, None, algo=algo)
 
         ctx.fp8_wgrad, ctx.gemm_algo = fp8_wgrad, algo
         ctx.need = (x.requires_grad, w1.requires_grad, w3.requires_grad, w2.requires_grad)
+        ctx.regate = regate
         ctx.opt = (h is not None, x_col is not None, h_col is not None)
         saved = [x, w1, w3, w2, h1, h3, amax_w1, amax_w3, amax_w2]
         saved += [t for t in (h, x_col, h_col) if t is not None]
@@ -92,20 +97,30 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         qw2t, sw2t = f8.weight_cast_tensorwise_t(w2, amax_w2)
         dh = ops.gemm_nt(qgy, qw2t, sgy, sw2t, None, algo=algo)
         del qgy, qw2t
-        if need_w2:
+        regate = ctx.regate
+        if need_w2 and not regate:
             gw2 = _wgrad(gy, gy_col, h, h_col, fp8_wgrad, algo)
 
         want_cols = fp8_wgrad and (need_w1 or need_w3)
         g1_col = torch.empty(F, dtype=torch.float32, device=dev) if want_cols else None
         g3_col = torch.empty(F, dtype=torch.float32, device=dev) if want_cols else None
-        g1, g3, qg1, qg3, sg1, sg3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, g1_col, g3_col, on_lines=True)
-        del dh
+        g1, g3, qg1, qg3, sg1, sg3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, g1_col, g3_col, on_lines=True, want_g=not regate)
+        if not regate:
+            del dh
         if need_x:
             (qw1t, sw1t), (qw3t, sw3t) = f8.weight_casts_tensorwise_t((w1, w3), (amax_w1, amax_w3))
             gx = ops.gemm_nt(qg1, qw1t, sg1, sw1t, None, algo=algo)
             ops.gemm_nt(qg3, qw3t, sg3, sw3t, None, algo=algo, out=gx, add=True)
         del qg1, qg3
-        if need_w1 or need_w3:
+        if regate:
+            if x_col is None:
+                x_col = ops.col_amax(x)
+            (qxt, sxt), (qgyt, sgyt) = ops.cast_transposed_many([(x, x_col), (gy, gy_col)], on_lines=True)
+            (qg1t, sg1t), (qg3t, sg3t), (qht, sht) = ops.swiglu_bwd_cast_transposed(dh, h1, h3, g1_col, g3_col, h_col, on_lines=True)
+            del dh
+            gw1, gw3 = ops.gemm_nt_multi([qg1t, qg3t], qxt, [sg1t, sg3t], sxt, algo=algo)
+            gw2 = ops.gemm_nt(qgyt, qht, sgyt, sht, None, algo=algo)
+        elif need_w1 or need_w3:
             if fp8_wgrad:
                 if x_col is None:
                     x_col = ops.col_amax(x)

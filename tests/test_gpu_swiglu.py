@@ -299,3 +299,33 @@ def test_gate_casts_under_the_gpu_division_rule(gpu_division_rule):
     for shape in [(5, 264), (33, 4096), (21, 11008), (3, 32768)]:
         test_forward_gate_and_cast(shape, True)
         test_backward_gate_and_casts(shape, True)
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (5, 264), (127, 64), (128, 72), (129, 128), (300, 1000), (1021, 520), (21, 11008), (9, 16384)])
+@pytest.mark.parametrize("poison", [False, True])
+def test_transposed_operands_made_from_the_gate(shape, poison):
+    """g1, g3 and h quantised per column and transposed, without any of them in memory: the bytes and scales of the transposed
+    casts of the stored copies, at the edges of the 64 x 128 tiles, with rows apart, and where a column's amax is not finite."""
+    from lingua_amd import ops
+    R, C = shape
+    big = [seeded_bf16((R, C + 8 * (i + 1)), std=std, seed=R + C + i).cuda() for i, std in enumerate((0.01, 2.0, 1.5))]
+    dh, h1, h3 = (b[:, 8 * i:8 * i + C] for i, b in enumerate(big))
+    if poison:
+        h3[R // 2, C // 2] = float("inf")
+        h1[R - 1, C - 1] = float("nan")
+        dh[0, 1] = float("-inf")
+    cols = [torch.empty(C, dtype=torch.float32, device="cuda") for _ in range(3)]
+    h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, col_amax=cols[2])
+    g1, g3, q1, q3, s1, s3 = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, cols[0], cols[1])
+    got = ops.swiglu_bwd_cast_transposed(dh, h1, h3, *cols)
+    for (q, s), stored, col in zip(got, (g1, g3, h), cols):
+        q0, s0 = ops.cast_colwise_transposed(stored, col)
+        assert q.shape == q0.shape and torch.equal(q.view(torch.uint8), q0.view(torch.uint8))
+        assert bits_equal(s.cpu(), s0.cpu())
+    # the row-wise pass without g1 and g3: the same bytes, scales and column amaxes
+    again = [torch.empty_like(c) for c in cols[:2]]
+    n1, n3, *rest = ops.swiglu_bwd_cast_rowwise(dh, h1, h3, *again, want_g=False)
+    assert n1 is None and n3 is None
+    for a, b in zip(rest, (q1, q3, s1, s3)):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    assert all(bits_equal(a.cpu(), c.cpu()) for a, c in zip(again, cols))
