@@ -351,6 +351,17 @@ int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_
 /* Host arithmetic only: would l8_gemm_nt_multi launch these once (aligned operands, n = 2 or 3 assumed; reads M alone)? */
 int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t K);
 
+/* C [M,N] = bf16(sum over i of A_i [M,K_i] . B_i [N,K_i]^T * sa_i * sb_i): the gradient of an activation that several linears
+ * read (lingua/float8.py:119 once per linear, added up by autograd).  sa_i fp32 [M], sb_i one fp32.  Two or three products
+ * that 256 x 256 tiles serve, none shorter than 512 and shorter than 8192 on average, run as one whose sum is rounded once;
+ * else as l8_gemm_nt of the first and l8_gemm_nt_add of the others, rounded per product. */
+typedef struct {
+  const void *A, *B;
+  int64_t K, lda, ldb;
+  const float *sa, *sb;
+} l8_gemm_term;
+int l8_gemm_nt_sum(const l8_gemm_term *terms, int64_t n, int64_t M, int64_t N, void *C, int64_t ldc, int algo, void *stream);
+
 /* Forward of one linear in one call, lingua/float8.py:85-96: x and w quantised row-wise, y = bf16(product * scales + bias).
  * The results of l8_cast_rowwise(x), l8_cast_rowwise(w), l8_gemm_nt, with their temporaries in `workspace`; where
  * l8_gemm_pick names the few-token kernel, and neither qw nor amax_w is asked for, the weight (rows of up to 12288 columns)

@@ -43,6 +43,7 @@ SIGNATURES = {
     "l8_gemm_nt_ws": [_p, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _p, _p, _i64, _int, _p, _i64, _p],
     "l8_gemm_nt_add": [_p, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _p, _int, _p, _i64, _int, _p],
     "l8_gemm_nt_multi": [_p, _i64, _p, _i64, _i64, _i64, _i64, _p, _int, _i64, _int, _p],
+    "l8_gemm_nt_sum": [_p, _i64, _i64, _i64, _p, _i64, _int, _p],
     "l8_gemm_multi_pays": [_p, _i64, _i64, _i64],
     "l8_gemm_workspace": [],
     "l8_gemm_workspace_gave_up_offset": [],

@@ -80,6 +80,15 @@ struct GemmArgs {
     uint16_t *C;
     int first, M;
   } part[2];
+  // SUM kernels: further products whose sum with the first one is C.  A, B, K, lda, ldb, sa (one per row) and sb (one) above
+  // are the first one's.
+  struct Term {
+    const uint8_t *A, *B;
+    const float *sa, *sb;
+    int64_t lda, ldb;
+    int K;
+  } term[2];
+  int terms;  // how many of them
 };
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
@@ -739,13 +748,21 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // MULTI: up to three products with one B (the weight gradients of linears on one activation) as one list of tiles.  On its
 // own [2048,16384].[2048,16384]^T has 64 tiles of 256 x 256, too few for this kernel, and [11008,4096] leaves a third of the
 // units without work in its last round; together they fill the rounds.
-template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false, int BM = 256, int BN = 256>
+//
+// SUM: C = A0.B0^T + A1.B1^T (+ A2.B2^T), each with row scales for A and one scale for B (the gradient of an activation that
+// several linears read), as one K loop over all of them: the stream of panels runs on from the last K tile of one product
+// into the first of the next.  The accumulators hold multiples of the present product's scale, so at a change of products
+// they are multiplied by the quotient of the old one and the new, row by row, under the matrix instructions of the new
+// product's first K tile (768 vector instructions beside its 64: 2.5 us per change of two rounds of tiles).  C is rounded and
+// written once, where ADD reads it back and rounds it per product.
+template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false, int BM = 256, int BN = 256, bool SUM = false>
 __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // one wave per SIMD, 128x128 per wave (the least LDS traffic per flop) or, in a half tile, 64x128
   static_assert((BM == 256 && BN == 256) || (BM == 256 && BN == 128) || (BM == 128 && BN == 256), "whole or half tiles");
   constexpr bool HALF_TILE = BM * BN == 32768;
   static_assert(!SK || !HALF_TILE, "the shared-K exchange is written for whole tiles");
+  static_assert(!SUM || !(HAS_BIAS || SK || ADD || MULTI || HALF_TILE), "a sum of products is a kernel of its own");
   constexpr int BK = 128, NW = 4, TM = HALF_TILE ? 4 : 8, TN = 8, WN = BN / 128;
   constexpr int WROWS = TM * 16;  // rows of the tile per wave
   constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;                // the panels of one K tile
@@ -864,16 +881,20 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   // cycles per tile with idle matrix cores otherwise).
   uint32_t a_voff[2], b_voff[2], foff[2];
   int chunk_even, chunk_odd;
+  int ld_K = p.K;  // the loader's reduction length (SUM: the present product's)
+  auto row_offsets = [&](int lrow, int lda, int ldb) {
+    a_voff[0] = (uint32_t)(lrow * lda + chunk_even);
+    a_voff[1] = (uint32_t)(lrow * lda + chunk_odd);
+    b_voff[0] = (uint32_t)(lrow * 8 * ldb + chunk_even);
+    b_voff[1] = (uint32_t)(lrow * 8 * ldb + chunk_odd);
+  };
   auto lane_consts = [&]() {
     int l = lane;
     asm volatile("" : "+v"(l));
     const int lrow = l >> 3, lpos = l & 7;
     chunk_even = (lpos ^ lrow) * 16;
     chunk_odd = (lpos ^ lrow ^ 1) * 16;
-    a_voff[0] = (uint32_t)(lrow * (int)p.lda + chunk_even);
-    a_voff[1] = (uint32_t)(lrow * (int)p.lda + chunk_odd);
-    b_voff[0] = (uint32_t)(lrow * 8 * (int)p.ldb + chunk_even);
-    b_voff[1] = (uint32_t)(lrow * 8 * (int)p.ldb + chunk_odd);
+    row_offsets(lrow, (int)p.lda, (int)p.ldb);
     const int l15 = l & 15, piece = l >> 4;  // fragment: lane l holds row l % 16, 16-byte chunks 2 (l / 16) and 2 (l / 16) + 1
     const int fr = (l15 & 7) ^ (l15 >> 3);
 #pragma unroll
@@ -903,10 +924,45 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 
   // loader cursor: the K tile whose panels are requested next (two K tiles ahead of the one being multiplied)
   int ld_seg = 0, ld_kt = 0;
-  [[maybe_unused]] int ld_ke = KT;  // SK: the loader's piece ends here
+  [[maybe_unused]] int ld_ke = KT;  // SK: the loader's piece ends here; SUM: its product
+  [[maybe_unused]] int ld_term = 0, ld_m0 = 0, ld_n0 = 0;  // SUM: its product and tile
+  // SUM: row and K offset of the load before; row offsets of this wave's first A and B row group, and the steps from group to group
+  [[maybe_unused]] int ld_off = 0, ld_a0 = 0, ld_step_a = 0, ld_b0 = 0, ld_step_b = 0, ld_back_b = 0;
   __amdgpu_buffer_rsrc_t ld_rsA, ld_rsB;
   auto ld_open = [&](int seg) {
-    if (seg < n_seg + n_tail) {
+    if (SUM && seg < n_seg) {
+      if (ld_term == 0) {
+        cursor_origin(cur_ld, ld_m0, ld_n0);
+        cursor_step(cur_ld);
+      }
+      GemmArgs::Term t = {p.A, p.B, p.sa, p.sb, p.lda, p.ldb, p.K};
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {  // member by member: a copy of the whole would live in scratch memory
+        const bool here = ld_term == i + 1;
+        t.A = here ? p.term[i].A : t.A;
+        t.B = here ? p.term[i].B : t.B;
+        t.lda = here ? p.term[i].lda : t.lda;
+        t.ldb = here ? p.term[i].ldb : t.ldb;
+        t.K = here ? p.term[i].K : t.K;
+      }
+      ld_K = t.K;
+      ld_ke = (t.K + BK - 1) / BK;
+      int l = lane;
+      asm volatile("" : "+v"(l));
+      row_offsets(l >> 3, (int)t.lda, (int)t.ldb);
+      // (opaque: kept in registers, not formed again in every trip)
+      const int gb = wave * NLB;
+      ld_step_a = 8 * (int)t.lda;
+      ld_a0 = wave * NLA * ld_step_a;
+      ld_step_b = 64 * (int)t.ldb;
+      ld_back_b = -63 * (int)t.ldb;
+      ld_b0 = ((gb >> 4) * 128 + 64 * (gb & 1) + ((gb & 15) >> 1)) * (int)t.ldb;
+      asm volatile("" : "+s"(ld_step_a), "+s"(ld_a0), "+s"(ld_step_b), "+s"(ld_back_b), "+s"(ld_b0));
+      const int64_t a_left = (int64_t)(p.M - ld_m0 - 1) * t.lda + t.K;
+      const int64_t b_left = (int64_t)(p.N - ld_n0 - 1) * t.ldb + t.K;
+      ld_rsA = make_rsrc(t.A + (int64_t)ld_m0 * t.lda, a_left < 0x7fffffff ? (uint32_t)a_left : 0x7fffffffu);
+      ld_rsB = make_rsrc(t.B + (int64_t)ld_n0 * t.ldb, b_left < 0x7fffffff ? (uint32_t)b_left : 0x7fffffffu);
+    } else if (seg < n_seg + n_tail) {
       int m0, n0;
       if (!SK || seg < n_seg) {
         cursor_origin(cur_ld, m0, n0);  // ld_open is called for seg = 0, 1, 2, ... in turn
@@ -925,28 +981,40 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     } else {  // past the last tile: every load is out of range and fills its LDS bytes with zeros
       ld_rsA = make_rsrc(p.A, 0);
       ld_rsB = make_rsrc(p.B, 0);
-      if (SK) ld_ke = 0x7fffffff;
+      if (SK || SUM) ld_ke = 0x7fffffff;
     }
   };
   auto ld_advance = [&]() {
-    if (++ld_kt == (SK ? ld_ke : KT)) {
+    if (++ld_kt == (SK || SUM ? ld_ke : KT)) {
       ld_kt = 0;
-      ld_open(++ld_seg);
+      if (SUM) {
+        if (++ld_term > p.terms) {
+          ld_term = 0;
+          ++ld_seg;
+        }
+        ld_open(ld_seg);
+      } else {
+        ld_open(++ld_seg);
+      }
     }
   };
   // i-th wave load of the A or B panel of the loader's K tile into the panel at LDS offset `at`
   auto load_one = [&](bool is_b, int at, int i) {
     const int k0 = ld_kt * BK;
-    const uint32_t m_even = (k0 + chunk_even < p.K) ? 0u : kOOB, m_odd = (k0 + chunk_odd < p.K) ? 0u : kOOB;
+    const uint32_t m_even = (k0 + chunk_even < ld_K) ? 0u : kOOB, m_odd = (k0 + chunk_odd < ld_K) ? 0u : kOOB;
     const int g = wave * (is_b ? NLB : NLA) + i;  // 8-row group of the panel's LDS image
     const uint32_t dst = lds0 + at + g * 1024;
+    // SUM: row offsets change with the product, so a load's is formed from the one before (one addition, as many as K's
+    // offset takes otherwise), not kept in scalar registers
     if (!is_b) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsA, reinterpret_cast<lds_ptr_t>(dst), 16, a_voff[i & 1] | ((i & 1) ? m_odd : m_even),
-                                               k0 + g * 8 * (int)p.lda, 0, 0);
+      int at_row = k0 + g * 8 * (int)p.lda;
+      if constexpr (SUM) at_row = ld_off = i == 0 ? k0 + ld_a0 : ld_off + ld_step_a;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsA, reinterpret_cast<lds_ptr_t>(dst), 16, a_voff[i & 1] | ((i & 1) ? m_odd : m_even), at_row, 0, 0);
     } else {
       const int row = (g >> 4) * 128 + 64 * (g & 1) + ((g & 15) >> 1);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsB, reinterpret_cast<lds_ptr_t>(dst), 16, b_voff[i & 1] | ((i & 1) ? m_odd : m_even),
-                                               k0 + row * (int)p.ldb, 0, 0);
+      int at_row = k0 + row * (int)p.ldb;
+      if constexpr (SUM) at_row = ld_off = i == 0 ? k0 + ld_b0 : ld_off + ((i & 1) ? ld_step_b : ld_back_b);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ld_rsB, reinterpret_cast<lds_ptr_t>(dst), 16, b_voff[i & 1] | ((i & 1) ? m_odd : m_even), at_row, 0, 0);
     }
   };
   // LDS offset of the panel of the K tile `ahead` beyond the one whose slot is s0 (whole tiles: a slot per panel)
@@ -1008,6 +1076,12 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   // and the K loop of the next, it was a vector load whose result was copied at once: a wait for every store)
   const int sa_one = MULTI || p.sa_row ? 0 : __builtin_amdgcn_readfirstlane(__float_as_int(p.sa[0]));
   const int sb_one = p.sb_row ? 0 : __builtin_amdgcn_readfirstlane(__float_as_int(p.sb[0]));
+  [[maybe_unused]] int sb_term[2] = {0, 0};
+  if constexpr (SUM) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+      if (t < p.terms) sb_term[t] = __builtin_amdgcn_readfirstlane(__float_as_int(p.term[t].sb[0]));
+  }
   auto load_scales = [&](int m0, int n0) {
     // lane-derived values are formed afresh from an opaque copy of the lane number wherever a tile's prologue or
     // epilogue needs them, so that none of them lives across a K loop
@@ -1160,8 +1234,12 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     // written, some 600 cycles with idle matrix cores.
     if constexpr (HAS_BIAS) asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb[0]), "v"(seg_sb[1]), "v"(seg_bias));
     else asm volatile("" : : "v"(seg_sa[0]), "v"(seg_sa[1]), "v"(seg_sb[0]), "v"(seg_sb[1]));
-    if (p.sb_row) store_tile_as(m0, n0, parts_tag, std::true_type{});
-    else store_tile_as(m0, n0, parts_tag, std::false_type{});
+    if constexpr (SUM) {
+      store_tile_as(m0, n0, parts_tag, std::false_type{});
+    } else {
+      if (p.sb_row) store_tile_as(m0, n0, parts_tag, std::true_type{});
+      else store_tile_as(m0, n0, parts_tag, std::false_type{});
+    }
   };
 
   // ---- SK: exchange of partial sums for tiles whose K range is shared out ----
@@ -1250,8 +1328,19 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   // been issued since the panels that the trip's barrier waits for were requested.  They are younger than the panels and
   // the counter retires in order, so the count allows for them (waiting for the stores themselves would stall the start
   // of every tile).
-  auto trip = [&](auto first_tag, bool stores, v8i (&bc)[TN], v8i (&bn)[TN]) __attribute__((always_inline)) {
-    constexpr bool FIRST = decltype(first_tag)::value;
+  // RESCALE (SUM): the first K tile of a further product.  ratio holds what the accumulators' rows are multiplied by, a value
+  // per accumulator index; tile i + 1 is rescaled under the instruction of tile i.
+  [[maybe_unused]] float ratio[SUM ? TM * 4 : 1];
+  [[maybe_unused]] auto rescale = [&](int i) __attribute__((always_inline)) {
+    const int tm = i / TN, tn = i % TN;
+    v4f n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) n[e] = acc_read(tm, tn, e) * ratio[SUM ? tm * 4 + e : 0];
+    acc[tm][tn] = n;
+  };
+  auto trip = [&](auto first_tag, bool stores, v8i (&bc)[TN], v8i (&bn)[TN], auto rescale_tag) __attribute__((always_inline)) {
+    constexpr bool FIRST = decltype(first_tag)::value, RESCALE = decltype(rescale_tag)::value;
+    if constexpr (RESCALE) rescale(0);
     const int at1 = panel_at(s0, AHEAD / 2, U1_IS_B), at2 = panel_at(s0, 0, false);
     auto mma_one = [&](int i) __attribute__((always_inline)) {
       const int tm = i / TN, tn = i % TN;
@@ -1260,13 +1349,18 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < BAR; ++i) {
       mma_one(i);
+      if constexpr (RESCALE) rescale(i + 1);
       if (i < RD1_GROUPS) {
 #pragma unroll
         for (int r = (N_RD1 * i) / RD1_GROUPS; r < (N_RD1 * (i + 1)) / RD1_GROUPS; ++r) read_piece(ad, af[A_EARLY + r / 2], A_EARLY + r / 2, r & 1);
       }
 #pragma unroll
       for (int j = (NL1 * i) / BAR; j < (NL1 * (i + 1)) / BAR; ++j) load_one(U1_IS_B, at1, j);
-      if (i == RD1_GROUPS) frag_addrs(panel_at(s0, 1, false), panel_at(s0, 1, true), ad);
+      if (i == RD1_GROUPS) {
+        int slot = s0;
+        if constexpr (SUM) asm volatile("" : "+s"(slot));  // (else these addresses are formed in front of the second instruction)
+        frag_addrs(panel_at(slot, 1, false), panel_at(slot, 1, true), ad);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
     if (U1_IS_B) ld_advance();
@@ -1278,6 +1372,9 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #pragma unroll
     for (int i = 0; i < REST; ++i) {
       mma_one(BAR + i);
+      if constexpr (RESCALE) {
+        if (i + 1 < REST) rescale(BAR + i + 1);
+      }
       if (i < RD2_GROUPS) {
 #pragma unroll
         for (int r = (N_RD2 * i) / RD2_GROUPS; r < (N_RD2 * (i + 1)) / RD2_GROUPS; ++r) read_next(bn, r);
@@ -1290,15 +1387,17 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     s0 = wrap(s0 + (HALF_TILE ? 1 : 2));
   };
   // n K tiles of one output tile.  Its first one finds its B fragments in bf0.
-  auto k_loop = [&](int n, bool stores) __attribute__((always_inline)) {
-    trip(std::true_type{}, stores, bf0, bf1);
+  auto k_loop = [&](int n, bool stores, bool further = false) __attribute__((always_inline)) {
+    constexpr std::false_type no{};
+    if (SUM && further) trip(no, false, bf0, bf1, std::integral_constant<bool, SUM>{});
+    else trip(std::true_type{}, stores, bf0, bf1, no);
 #pragma unroll 1
     for (n -= 1; n >= 2; n -= 2) {
-      trip(std::false_type{}, false, bf1, bf0);
-      trip(std::false_type{}, false, bf0, bf1);
+      trip(no, false, bf1, bf0, no);
+      trip(no, false, bf0, bf1, no);
     }
     if (n) {
-      trip(std::false_type{}, false, bf1, bf0);
+      trip(no, false, bf1, bf0, no);
     } else {  // an odd number of K tiles: the next tile's fragments are in the other set
 #pragma unroll
       for (int t = 0; t < TN; ++t) bf0[t] = bf1[t];
@@ -1315,8 +1414,54 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     cursor_origin(cur_mul, m0, n0);
     cursor_step(cur_mul);
     if (SK && seg > 0) lane_consts();
-    load_scales(m0, n0);
-    k_loop(KT, seg > 0);
+    if constexpr (SUM) {
+      // A product's unit is the scale of its row times that of its B; all units of the tile's rows are requested here, lane l
+      // holding those of rows wm*WROWS + l and + 64 + l.  A product much finer than what it is added to (2^90, where its
+      // largest sum is below 2^-56 of the other's smallest step) is counted in units that keep the quotient finite.
+      int l = lane;
+      asm volatile("" : "+v"(l));
+      int bits[3][2];
+#pragma unroll
+      for (int t = 0; t < 3; ++t) {
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(t == 0 ? p.sa : p.term[t ? t - 1 : 0].sa, t <= p.terms ? (uint32_t)p.M * 4u : 0u);
+        bits[t][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + l) * 4, m0 * 4, 0);
+        bits[t][1] = TM > 4 ? __builtin_amdgcn_raw_buffer_load_b32(rs, (wm * WROWS + 64 + l) * 4, m0 * 4, 0) : 0;
+      }
+      k_loop(KT, seg > 0);
+      float unit[2] = {__int_as_float(bits[0][0]) * __int_as_float(sb_one), __int_as_float(bits[0][1]) * __int_as_float(sb_one)};
+      auto go_on = [&](int t) __attribute__((always_inline)) {
+        int quot[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const float least = unit[h] * 0x1p-90f;
+          float next = __int_as_float(bits[1][h]) * __int_as_float(t == 1 ? sb_term[0] : sb_term[1]);
+          next = next < least ? least : next;  // (a NaN stays)
+          quot[h] = __float_as_int(unit[h] / next);
+          unit[h] = next;
+        }
+        int at = lane;
+        asm volatile("" : "+v"(at));
+        const int from = 16 * (at >> 4);
+#pragma unroll
+        for (int i = 0; i < TM * 4; ++i)
+          ratio[i] = __int_as_float(__builtin_amdgcn_ds_bpermute(from + 4 * (((i >> 2) & 3) * 16 + (i & 3)), quot[i >> 4]));
+        k_loop((p.term[t - 1].K + BK - 1) / BK, false, true);
+      };
+#pragma unroll 1
+      for (int t = 1; t <= p.terms; ++t) {
+        if (t == 2) {
+          bits[1][0] = bits[2][0];
+          bits[1][1] = bits[2][1];
+        }
+        go_on(t);
+      }
+      seg_sa[0] = __float_as_int(unit[0]);
+      seg_sa[1] = __float_as_int(unit[1]);
+      seg_sb[0][0] = __float_as_int(1.0f);
+    } else {
+      load_scales(m0, n0);
+      k_loop(KT, seg > 0);
+    }
     if (L8_GEMM_PROF) {
       const uint64_t t = __builtin_readcyclecounter();
       prof[3] += t - t_loop;
@@ -1439,6 +1584,7 @@ template __global__ void gemm_nt_stream_kernel<4, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, false, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, false, false, 256, 256, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
@@ -1794,6 +1940,70 @@ extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void
     first += (parts[i].M + 255) / 256 * 256;
     if (i + 1 < n) p.part[i] = {(const uint8_t *)parts[i + 1].A, parts[i + 1].sa, (uint16_t *)parts[i + 1].C, (int)first, (int)parts[i + 1].M};
     else p.part[i] = {p.A, p.sa, p.C, 0x7fffffff, p.M};
+  }
+  static std::atomic<bool> attr_done[kMaxDev] = {};  // idempotent; a race only repeats the call
+  const int slot = device_slot();
+  if (slot < 0 || !attr_done[slot]) {
+    L8_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
+    if (slot >= 0) attr_done[slot] = true;
+  }
+  hipLaunchKernelGGL(fn, dim3((unsigned)persistent_grid((int64_t)p.tiles_m * p.tiles_n)), dim3(256), kLds, (hipStream_t)stream, p);
+  L8_HIP(hipGetLastError());
+  return L8_OK;
+}
+
+// The sum of products as one K loop, or as one product that the others are added to?  As one it saves, per product after the
+// first, the conversion of a C tile and its way to memory and back, and pays 2000 cycles per tile for the change of scales.
+// Bound by the matrix cores' power either way: beyond K = 8192 per product what is saved no longer shows.  us, one by one /
+// as one: 3 x [16384,2048] K = 2048 194.8 / 157.4, K = 2048 + 512 + 512 125.9 / 84.2, 2 x K = 512 58.4 / 39.6, K = 4096 197.7 / 176.6,
+// K = 5632 254 / 234, K = 8192 355.5 / 352.5 and, on another machine, 382.9 / 387.5; 2 x [16384,4096] K = 4096 384.6 / 349.4,
+// K = 6144 540.8 / 511.9, K = 11008 924 / 922; 2 x [8192,5120] K = 7168 431 / 399; 2 x [4093,4096] K = 14336 298 / 290 and,
+// on another machine, 311 / 323.  Against 64 bits the sum is 1.7e-3 off (one rounding to bf16), before 2.4e-3 with two products
+// and 2.9e-3 with three.
+static bool sum_in_one(const l8_gemm_term *terms, int64_t n, int64_t M, int64_t N, const void *C, int64_t ldc) {
+  if (n < 2 || n > 3 || M <= 0 || N <= 0 || M >= (1LL << 29) || N >= (1LL << 29) || N % 8 || ldc % 8 || ldc < N || ldc >= (1LL << 22) || ((uintptr_t)C % 16)) return false;
+  int64_t K = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    const l8_gemm_term &t = terms[i];
+    if (!t.A || !t.B || !t.sa || !t.sb || t.K < 512 || t.K % 16 || t.lda % 16 || t.ldb % 16 || t.lda < t.K || t.ldb < t.K ||
+        256 * t.lda + t.K >= (1LL << 31) || 256 * t.ldb + t.K >= (1LL << 31) || ((uintptr_t)t.A % 16) || ((uintptr_t)t.B % 16))
+      return false;
+    K += t.K;
+  }
+  return K < n * 8192 && ((M + 255) / 256) * ((N + 255) / 256) < (1LL << 31) && pick_algo(M, N, K) == 12;
+}
+
+extern "C" int l8_gemm_nt_sum(const l8_gemm_term *terms, int64_t n, int64_t M, int64_t N, void *C, int64_t ldc, int algo, void *stream) {
+  L8_REQUIRE(n >= 1 && terms, "l8_gemm_nt_sum: no terms");
+  if (algo != 0 || !sum_in_one(terms, n, M, N, C, ldc)) {
+    for (int64_t i = 0; i < n; ++i) {
+      const l8_gemm_term &t = terms[i];
+      const int rc = gemm_nt_impl(t.A, t.B, M, N, t.K, t.lda, t.ldb, t.sa, L8_SCALE_ROW, t.sb, L8_SCALE_SCALAR, nullptr, C, ldc, i > 0, algo, nullptr, 0, stream);
+      if (rc != L8_OK) return rc;
+    }
+    return L8_OK;
+  }
+  constexpr int kLds = 5 * 256 * 128;
+  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, false, false, 256, 256, true>;
+  GemmArgs p{};
+  p.A = (const uint8_t *)terms[0].A;
+  p.B = (const uint8_t *)terms[0].B;
+  p.M = (int)M;
+  p.N = (int)N;
+  p.K = (int)terms[0].K;
+  p.lda = terms[0].lda;
+  p.ldb = terms[0].ldb;
+  p.ldc = ldc;
+  p.sa = terms[0].sa;
+  p.sb = terms[0].sb;
+  p.sa_row = 1;
+  p.C = (uint16_t *)C;
+  p.tiles_m = (int)((M + 255) / 256);
+  p.tiles_n = (int)((N + 255) / 256);
+  p.terms = (int)n - 1;
+  for (int i = 0; i < 2; ++i) {
+    const l8_gemm_term &t = terms[i + 1 < n ? i + 1 : 0];
+    p.term[i] = {(const uint8_t *)t.A, (const uint8_t *)t.B, t.sa, t.sb, t.lda, t.ldb, (int)t.K};
   }
   static std::atomic<bool> attr_done[kMaxDev] = {};  // idempotent; a race only repeats the call
   const int slot = device_slot();

@@ -510,7 +510,8 @@ def linear_backward(grad_out, a, b_t, amax_b_t, a_col_amax, need_a: bool, need_b
 
 def shared_input_backward(grads, a, ws, amaxes, a_col_amax, need_a: bool, need_ws, gemm_algo: int):
     """Backward of linears on one activation ``a`` without biases, fp8 weight gradients, as ``linear_backward`` of each in turn
-    computes it: ``(grad_a, [grad_w ...])``.  Casts of one kind share a launch, and so do the weight gradients."""
+    computes it: ``(grad_a, [grad_w ...])``.  Casts of one kind share a launch, and so do the weight gradients; the sum of the
+    input gradients is rounded once instead of per linear where ``ops.gemm_nt_sum`` makes one product of them."""
     for g in grads:
         if g.dtype != torch.bfloat16:
             raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {g.dtype}")
@@ -523,9 +524,10 @@ def shared_input_backward(grads, a, ws, amaxes, a_col_amax, need_a: bool, need_w
         for i, g in enumerate(grads):   # a gradient whose weight does not learn needs no column amaxes
             if i not in quantised:
                 quantised[i] = (*ops.cast_rowwise(g, on_lines=True)[:2], None)
-        for i, (qwt, swt) in enumerate(weight_casts_tensorwise_t(ws, amaxes)):
-            qg, sg, cols[i] = quantised[i]
-            grad_a = ops.gemm_nt(qg, qwt, sg, swt, None, algo=gemm_algo, out=grad_a, add=grad_a is not None)
+        qwts, swts = zip(*weight_casts_tensorwise_t(ws, amaxes))
+        qgs, sgs, cols = (list(t) for t in zip(*(quantised[i] for i in range(len(grads)))))
+        grad_a = ops.gemm_nt_sum(qgs, qwts, sgs, swts, algo=gemm_algo)
+        del qgs, qwts
         del quantised
     learning = [i for i, need in enumerate(need_ws) if need]
     grad_ws = [None] * len(grads)

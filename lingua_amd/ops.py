@@ -502,6 +502,32 @@ def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
     return outs
 
 
+def gemm_nt_sum(qas, qbs, sas, sbs, algo: int = 0) -> torch.Tensor:
+    """bf16 [M,N] sum of ``gemm_nt(qa, qb, sa, sb)`` over products of one shape [M,N]: in one launch and rounded once where
+    the library can, else added up product by product (``gemm_nt(..., add=True)``).  Row scales sa, one scale sb each."""
+    M, N = qas[0].shape[0], qbs[0].shape[0]
+    dev = qas[0].device
+    one = algo == 0 and M > 0 and N > 0 and len(qas) > 1 and not timed_singly("gemm_nt")
+    for qa, qb, sa, sb in zip(qas, qbs, sas, sbs):
+        one = (one and qa.dtype == qb.dtype == torch.float8_e4m3fn and qa.dim() == qb.dim() == 2 and qa.shape == (M, qb.shape[1]) and
+               qb.shape[0] == N and _rows_apart(qa) and _rows_apart(qb) and qa.device == qb.device == dev and
+               sa.dtype == sb.dtype == torch.float32 and sa.numel() == M and sb.numel() == 1 and sa.is_contiguous())
+    if not one:
+        out = None
+        for qa, qb, sa, sb in zip(qas, qbs, sas, sbs):
+            out = gemm_nt(qa, qb, sa, sb, None, algo=algo, out=out, add=out is not None)
+        return out
+    st = _prep(qas[0], "gemm_nt_sum")
+    out = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
+    terms = []
+    for qa, qb, sa, sb in zip(qas, qbs, sas, sbs):
+        terms += [qa.data_ptr(), qb.data_ptr(), qa.shape[1], _ld(qa), _ld(qb), sa.data_ptr(), sb.data_ptr()]
+    with _timed("gemm_nt_sum", 2 * M * N * sum(qa.shape[1] for qa in qas), dev):
+        code = _lib.load().l8_gemm_nt_sum(struct.pack(f"{len(terms)}q", *terms), len(qas), M, N, out.data_ptr(), N, algo, st)
+    _lib.check(code, "l8_gemm_nt_sum")
+    return out
+
+
 _FWD = struct.Struct("22q")   # l8_linear_fwd_args: eight bytes per member
 
 

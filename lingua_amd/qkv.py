@@ -14,9 +14,9 @@ tokens the narrow products can run on kernels that deal K out to groups of waves
 where the wide one does not: a last bit may differ then.
 
 Backward stays per linear (lingua/float8.py:99-131) but for its launches: the
-three dgrads have different row scales and are added up by their epilogues, the
-three wgrads share the token-dimension copy of ``x`` and run as one list of
-tiles.
+three dgrads have different row scales and are one sum of products, rounded
+once, where large tiles serve them, else added up by their epilogues; the three
+wgrads share the token-dimension copy of ``x`` and run as one list of tiles.
 
 Nothing changes in the attention module or in the state dict: ``wq`` computes
 all three products when it is called and keeps the other two for ``wk`` and

@@ -109,8 +109,7 @@ class Fp8SwiGLUFn(torch.autograd.Function):
             del dh
         if need_x:
             (qw1t, sw1t), (qw3t, sw3t) = f8.weight_casts_tensorwise_t((w1, w3), (amax_w1, amax_w3))
-            gx = ops.gemm_nt(qg1, qw1t, sg1, sw1t, None, algo=algo)
-            ops.gemm_nt(qg3, qw3t, sg3, sw3t, None, algo=algo, out=gx, add=True)
+            gx = ops.gemm_nt_sum((qg1, qg3), (qw1t, qw3t), (sg1, sg3), (sw1t, sw3t), algo=algo)
         del qg1, qg3
         if regate:
             if x_col is None:

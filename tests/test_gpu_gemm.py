@@ -198,6 +198,80 @@ def test_product_added_to_what_the_output_holds(algo, mnk):
         ops.gemm_nt(qa, qb, sa, sb, algo=algo, add=True)
 
 
+def sum_of_products(terms):
+    from lingua_amd import ops
+    return ops.gemm_nt_sum(*zip(*terms))
+
+
+def one_by_one(terms):
+    from lingua_amd import ops
+    out = None
+    for qa, qb, sa, sb in terms:
+        out = ops.gemm_nt(qa, qb, sa, sb, out=out, add=out is not None)
+    return out
+
+
+# (two tiles per workgroup and one, K tiles even and odd in number, whole and short, rows on lines and apart)
+@pytest.mark.parametrize("M,N,Ks", [(4093, 8184, (512, 512)), (4093, 8184, (528, 1152, 656)), (3590, 3592, (640, 2064)), (3590, 3592, (1040, 512, 768))])
+def test_sum_of_products_is_rounded_once(M, N, Ks):
+    """Integers in -1 .. 1 and powers of two for scales: the fp32 sums are exact, whichever product's scale they are counted in,
+    so the result is the one rounding to bf16 of the exact sum."""
+    from lingua_amd import _lib
+    assert _lib.load().l8_gemm_pick(M, N, sum(Ks)) == 12
+    g = torch.Generator().manual_seed(M + len(Ks))
+    terms, want = [], 0
+    for i, K in enumerate(Ks):
+        A, B = (torch.randint(-1, 2, (n, K), generator=g).float().cuda() for n in (M, N))
+        sa = torch.tensor([2.0 ** ((r * (i + 3)) % 5 - 2) for r in range(M)]).reshape(M, 1).cuda()
+        sb = torch.tensor([[2.0 ** (1 - i)]]).cuda()
+        want = want + (A.double() @ B.double().t()) * sa.double() * sb.double()
+        terms.append((spread(fp8(A).view(torch.uint8), K + 16 * i).view(torch.float8_e4m3fn), fp8(B), sa, sb))
+    assert torch.equal(sum_of_products(terms).view(torch.int16), want.float().to(torch.bfloat16).view(torch.int16))
+
+
+def test_sum_of_products_whose_scales_lie_far_apart():
+    """Rows whose products differ by up to 2^150 in scale, rows of zeros with the smallest scale, rows whose scale is infinite or
+    NaN: what adding one product to the other gives, but for its roundings to bf16 (2^-9 of either product and of the sum)."""
+    M, N, K = 3590, 3592, 528
+    g = torch.Generator().manual_seed(77)
+    qs = [random_fp8_bytes(s, g).cuda().view(torch.float8_e4m3fn) for s in ((M, K), (N, K), (M, K), (N, K))]
+    s0, s1 = (torch.rand(M, 1, generator=g) + 0.5 for _ in range(2))
+    tiny = 1e-12 / 448
+    for r, (a, b) in enumerate([(1e20, 1e-25), (1e-25, 1e20), (1.0, tiny), (tiny, 1.0), (1.0, float("inf")), (float("nan"), 1.0),
+                                (1.0, float("nan")), (float("inf"), 1.0), (1e20, 1.0), (tiny, tiny)]):
+        s0[r * 131], s1[r * 131] = a, b
+    # the casts give such a scale to rows that hold an infinity or a NaN, whose bytes are NaN codes: the whole row of results is NaN
+    for q, rows in ((qs[0], (5, 7)), (qs[2], (4, 6))):
+        for r in rows:
+            q.view(torch.uint8)[r * 131, 9] = 0x7f
+    qs[2].view(torch.uint8)[2 * 131] = 0
+    qs[0].view(torch.uint8)[3 * 131] = 0
+    terms = [(qs[0], qs[1], s0.cuda(), torch.tensor([[0.25]]).cuda()), (qs[2], qs[3], s1.cuda(), torch.tensor([[3.0]]).cuda())]
+    got, want = sum_of_products(terms).float().cpu(), one_by_one(terms).float().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    parts = sum(one_by_one([t]).float().abs().cpu() for t in terms)
+    fine = torch.isfinite(want)
+    bound = parts * 2.0 ** -7
+    # (a sum of cancelling terms in fp32: K * 2^-24 of the largest term that a row can hold)
+    floor = torch.maximum(s0 * 0.25, s1 * 3.0) * (448.0 ** 2 * K * K * 2.0 ** -24)
+    assert ((got - want).abs()[fine] <= (bound + floor.expand_as(bound))[fine]).all()
+
+
+def test_sum_of_products_that_one_loop_does_not_serve():
+    """Sizes for smaller tiles, reductions too short or too long, a tile configuration asked for: added one by one, the same bits."""
+    from lingua_amd import ops
+    for M, N, Ks, algo in ((150, 256, (512, 528), 0), (3590, 3592, (512, 496), 0), (2304, 4096, (16384, 512), 0), (3590, 3592, (512, 512), 12)):
+        g = torch.Generator().manual_seed(M + N)
+        terms = []
+        for K in Ks:
+            qa, qb = (random_fp8_bytes((n, K), g).cuda().view(torch.float8_e4m3fn) for n in (M, N))
+            terms.append((qa, qb, (torch.rand(M, 1, generator=g) + 0.5).cuda(), (torch.rand(1, 1, generator=g) + 0.5).cuda()))
+        want = None
+        for t in terms:
+            want = ops.gemm_nt(*t, algo=algo, out=want, add=want is not None)
+        assert torch.equal(ops.gemm_nt_sum(*zip(*terms), algo=algo).view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("algo", [0, 1, 2, 3, 11, 15])
 def test_k_indexing_with_one_hot_operands(algo):
     # B[n] is one-hot at k = pi(n): C[m,n] = A[m, pi(n)] exactly, for any K (tails included)
