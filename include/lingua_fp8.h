@@ -405,6 +405,42 @@ int l8_linear_fwd(const l8_linear_fwd_args *args);
 int64_t l8_linear_fwd_rows_workspace(const l8_linear_fwd_args *args, int64_t ldqx, int64_t ldqw);
 int l8_linear_fwd_rows(const l8_linear_fwd_args *args, int64_t ldqx, int64_t ldqw);
 
+/* All casts of a linear's backward pass (lingua/float8.py:106-118 and the fp8 weight gradient's), for shapes where
+ * l8_linear_bwd_casts_pays(M, N, K): two launches.  The results of
+ *   l8_cast_rowwise(g, with column amaxes), l8_cast_colwise_transposed_pad(g, those),
+ *   l8_cast_colwise_transposed_pad(a, a_col) and l8_cast_tensorwise_t_rows(w, amax_w),
+ * g [M,N], a [M,K], w [N,K] bf16; qgt [N,Mp], qat [K,Mp], qwt [K,N], rows ldq.. bytes apart.  qat NULL: a is not wanted,
+ * qwt NULL: w is not.  amax_w bf16 [N], 16-byte aligned, N % 8 == 0.  The workspace needs l8_cast_rowwise_workspace(M, N) bytes. */
+typedef struct {
+  const void *g;
+  int64_t M, N, ldg;
+  void *qg;
+  int64_t ldqg;
+  float *sg;
+  void *qgt;
+  int64_t ldqgt;
+  float *sgt;
+  int64_t Mp;
+  const void *a;
+  int64_t K, lda;
+  const float *a_col;
+  void *qat;
+  int64_t ldqat;
+  float *sat;
+  const void *w;
+  int64_t ldw;
+  const void *amax_w;
+  void *qwt;
+  int64_t ldqwt;
+  float *swt;
+  void *workspace;
+  int64_t workspace_bytes;
+  void *stream;
+} l8_linear_bwd_casts_args;
+int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *args);
+/* Host arithmetic only. */
+int l8_linear_bwd_casts_pays(int64_t M, int64_t N, int64_t K);
+
 #ifdef __cplusplus
 }
 #endif

@@ -74,21 +74,52 @@ L8_DEV RowOperand operand_of(const RowOperands &list, int64_t r) {
 }
 #endif
 
-// MANY: the operands come from `list`, R counts the rows of all of them and x .. amax_out are not used.
-template <int NCH, bool COLMAX, bool MANY = false>
+// With column maxima a workgroup collects them of one operand, so each operand has workgroups of its own, in proportion to
+// its rows: what one launch leaves in partial rows is then shared out, where each of several launches leaves as many.  us,
+// one by one / together, with the folds (one each / one): three [16384,2048] 69.3 / 54.5 (5.5 TB/s), [16384,4096] 114 / 101,
+// [4096,4096] 48.8 / 31.4, [1021,2048] 19.3 / 8.8, two [300,2048] 11.8 / 6.5; an activation and a weight without column maxima
+// [1021,2048] and [2048,2048] 15.9 / 13.8, [4096,2048] and [2048,2048] 21.0 / 17.7, [16384,4096] and [11008,4096] 59.4 / 56.7.
+struct RowGroup {
+  const uint16_t *x;
+  int64_t R, ldx;
+  uint8_t *q;
+  int64_t ldq;
+  float *scale;
+  uint16_t *amax, *partials;  // either may be null
+  int first, blocks;          // its workgroups; the operands are in order, unused ones start beyond the last
+};
+struct RowGroups {
+  RowGroup op[kMaxRowOperands];
+};
+
+// MANY without column maxima: the operands come from `list`, R counts the rows of all of them and x .. amax_out are not used.
+// With them: everything but C comes from `list`.
+template <bool COLMAX, bool MANY>
+using RowList = std::conditional_t<MANY, std::conditional_t<COLMAX, RowGroups, RowOperands>, int>;
+template <int NCH, bool COLMAX, bool MANY_OPERANDS = false>
 __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
     const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint8_t *__restrict__ q, int64_t ldq,
     float *__restrict__ scale, uint16_t *__restrict__ amax_out, uint16_t *__restrict__ col_partials, int scale_rule,
-    const std::conditional_t<MANY, RowOperands, int> list) {
+    const RowList<COLMAX, MANY_OPERANDS> list) {
 #if defined(__HIP_DEVICE_COMPILE__)  // buffer descriptors exist in the device pass only
+  constexpr bool GROUPS = MANY_OPERANDS && COLMAX, MANY = MANY_OPERANDS && !COLMAX;
+  int block = blockIdx.x, blocks = gridDim.x;
+  if constexpr (GROUPS) {
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxRowOperands; ++i) which += block >= list.op[i].first ? 1 : 0;
+    const RowGroup &op = list.op[which];
+    x = op.x, R = op.R, ldx = op.ldx, q = op.q, ldq = op.ldq, scale = op.scale, amax_out = op.amax, col_partials = op.partials;
+    block -= op.first, blocks = op.blocks;
+  }
   extern __shared__ uint32_t lds_colmax[];  // [C/2] packed bf16 pairs when COLMAX
   // the next row is prefetched into a second register set unless that would
   // push the wave beyond 256 VGPRs (two waves per SIMD are worth more)
   constexpr bool PREFETCH = COLMAX ? (NCH <= 8) : (NCH <= 24);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // in a scalar register: the row descriptors hang on it
-  const int64_t wave_stride = (int64_t)gridDim.x * kRowWaves;
-  int64_t r = (int64_t)blockIdx.x * kRowWaves + wave;
+  const int64_t wave_stride = (int64_t)blocks * kRowWaves;
+  int64_t r = (int64_t)block * kRowWaves + wave;
   auto load = [&](auto &buf, int64_t row) {
     constexpr int N = sizeof(buf) / sizeof(buf[0]);
     if constexpr (MANY) {
@@ -167,7 +198,7 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
     r = rn;
   }
 
-  if (COLMAX) {
+  if (COLMAX && (!GROUPS || col_partials)) {
     // merge the four waves' column maxima through LDS, one wave after the other
     // (packed pairs, plain reads and writes), then write this workgroup's row of
     // the partial-maxima array; a second small kernel folds the rows.  (Global
@@ -185,7 +216,7 @@ __global__ __launch_bounds__(kRowBlock, 2) void cast_rowwise_kernel(
 #pragma unroll
               for (int k = 0; k < 4; ++k) mine[k] = (int)pk_absmax_u16((uint32_t)old[k], (uint32_t)mine[k]);
             }
-            if (w == kRowWaves - 1) *(v4i *)(col_partials + (int64_t)blockIdx.x * C + c) = mine;
+            if (w == kRowWaves - 1) *(v4i *)(col_partials + (int64_t)block * C + c) = mine;
             else lds4[c / 8] = mine;
           }
         }
@@ -602,11 +633,12 @@ struct TransposeTile {
 };
 constexpr int kMaxTileRows = 256;                 // no tile is taller (bounds the row stride the host accepts)
 
-// Where the scale comes from: one amax, a column amax each, or one amax that every workgroup finds among the row amaxes
+// Where the scale comes from: one amax, a column amax each -- or the partial maxima that the row-wise cast's workgroups left
+// of them, while these are few --, or one amax that every workgroup finds among the row amaxes
 // (a few kilobytes from the L2 under the tile's loads, where a reduction of its own is a launch).  Weights inside a forward
 // + backward, us, reduction + cast / this: [2048,2048] 4.7 + 4.7 / 5.2, [4096,14336] 4.8 + 33.6 / 34.7, [14336,4096]
 // 7.5 + 34.0 / 36.8.
-enum class AmaxFrom { kScalar, kColumns, kRows };
+enum class AmaxFrom { kScalar, kColumns, kRows, kPartials };
 constexpr int64_t kMaxAmaxRows = 16384;           // longest list that every workgroup reads
 
 // Columns R .. Rp - 1 of q are zeros: what a reduction over the tokens pads them to.  The rows are whole 16-byte pieces
@@ -623,25 +655,24 @@ struct TransposedOperand {
   uint8_t *q;
   int64_t ldq, Rp;
   float *scale;
-  int C, n_amax, vec_store;     // n_amax: length of the list of row amaxes, or 1 for an fp32 scalar
+  int C, n_amax, vec_store;     // n_amax: length of the list of row amaxes, rows of partial maxima, or 1 for an fp32 scalar
   int first;                    // first workgroup of the launch; the operands are in order, unused ones start beyond the last
+  AmaxFrom from;                // read by the kernel for operands of several kinds
 };
 constexpr int kMaxTransposed = 4;
 struct TransposedOperands {
   TransposedOperand op[kMaxTransposed];
 };
-template <AmaxFrom FROM, int TC, int TU, bool MANY = false>
-__global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditional_t<MANY, TransposedOperands, TransposedOperand> list, int scale_rule) {
+// LDS of a workgroup
+template <int TC, int TU>
+struct TransposeShared {
+  __attribute__((aligned(16))) uint8_t tile[TransposeTile<TC, TU>::kTC * TransposeTile<TC, TU>::kTStride];
+  float recips[TC];
+  uint32_t wave_amax[4], amaxes[TC];
+};
 #if defined(__HIP_DEVICE_COMPILE__)  // the buffer-resource type exists in the device pass only
-  int which = 0;
-  if constexpr (MANY) {
-#pragma unroll
-    for (int i = 1; i < kMaxTransposed; ++i) which += (int)blockIdx.x >= list.op[i].first ? 1 : 0;
-  }
-  const TransposedOperand &op = [&]() -> const TransposedOperand & {
-    if constexpr (MANY) return list.op[which];
-    else return list;
-  }();
+template <AmaxFrom FROM, int TC, int TU>
+L8_DEV void transpose_tile(const TransposedOperand &op, unsigned block, int scale_rule, TransposeShared<TC, TU> &lds) {
   const uint16_t *const __restrict__ x = op.x;
   const int64_t R = op.R, ldx = op.ldx, ldq = op.ldq, Rp = op.Rp;
   const int C = op.C, n_amax = op.n_amax, vec_store = op.vec_store, amax_f32 = FROM == AmaxFrom::kScalar ? n_amax : 0;
@@ -650,13 +681,12 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
   const void *const __restrict__ amax_scalar = op.amax;
   uint8_t *const __restrict__ q = op.q;
   float *const __restrict__ scale = op.scale;
-  const unsigned block = blockIdx.x - (MANY ? (unsigned)op.first : 0u);
   using T = TransposeTile<TC, TU>;
-  constexpr bool PER_COL = FROM == AmaxFrom::kColumns, ROWS = FROM == AmaxFrom::kRows;
+  constexpr bool ROWS = FROM == AmaxFrom::kRows, PARTIALS = FROM == AmaxFrom::kPartials, PER_COL = FROM == AmaxFrom::kColumns || PARTIALS;
   constexpr int kTC = T::kTC, kCCH = T::kCCH, kRG = T::kRG, kTU = T::kTU, kTR = T::kTR, kTStride = T::kTStride;
-  __shared__ __attribute__((aligned(16))) uint8_t tile[kTC * kTStride];
-  __shared__ float recips[kTC];
-  __shared__ uint32_t wave_amax[4];
+  uint8_t *const tile = lds.tile;
+  float *const recips = lds.recips;
+  uint32_t *const wave_amax = lds.wave_amax;
   const int t = threadIdx.x;
   // Workgroup w takes column block w % nct and row tile (w / nct + w % nct) % nrt:
   // a diagonal walk.  The workgroups resident at one time then touch addresses
@@ -681,6 +711,7 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
   // around each load the compiler waited for all of them after the fifth and again before the division.)
   uint32_t amax_lo = 0, amax_hi = 0;
   v4i listed[ROWS ? 4 : 1];
+  [[maybe_unused]] v4i parts[PARTIALS ? 8 : 1], part_max = {0, 0, 0, 0};
   if constexpr (ROWS) {
     const __amdgpu_buffer_rsrc_t rsList = make_rsrc(amax_rows, (uint32_t)n_amax * 2u);  // zeros beyond the list
     for (int i0 = t * 8;; i0 += 4 * 256 * 8) {
@@ -691,6 +722,19 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
       for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int w = 0; w < 4; ++w) amax_lo = pk_absmax_u16(amax_lo, (uint32_t)listed[k][w]);
+    }
+  } else if constexpr (PARTIALS) {
+    // this thread's 8 columns in every kRG-th partial row
+    const __amdgpu_buffer_rsrc_t rsPart = make_rsrc(op.amax, (uint32_t)n_amax * (uint32_t)C * 2u);  // zeros beyond the last row
+    const uint32_t at = c < C ? (uint32_t)c * 2u : 0x80000000u;
+    for (int i0 = rg;; i0 += 8 * kRG) {
+#pragma unroll
+      for (int k = 0; k < 8; ++k) parts[k] = __builtin_amdgcn_raw_buffer_load_b128(rsPart, (int)(at + (uint32_t)(i0 + k * kRG) * (uint32_t)C * 2u), 0, 0);
+      if (i0 - rg + 8 * kRG >= n_amax) break;  // the last eight stay in flight under the tile's loads
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) part_max[w] = (int)pk_absmax_u16((uint32_t)part_max[w], (uint32_t)parts[k][w]);
     }
   } else if (PER_COL) {
     const __amdgpu_buffer_rsrc_t rsAmax = make_rsrc(col_amax, (uint32_t)C * 4u);
@@ -720,6 +764,30 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
     for (int i = 0; i < 4; ++i)
       in[u][i] = load16_nt(rsX, voff, (u * kRG * 4 + i) * row_bytes);
 
+  if constexpr (PARTIALS) {
+    // the columns' maxima over the kRG groups of partial rows meet in the tile's memory
+    static_assert(kRG % 8 == 0 && kRG * kTC * 2 + 8 * kTC * 2 <= kTC * kTStride, "the maxima fit the tile's memory");
+    uint32_t *const groups = (uint32_t *)tile, *const eighths = groups + kRG * (kTC / 2);  // [kRG][kTC / 2], [8][kTC / 2] pairs of columns
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) part_max[w] = (int)pk_absmax_u16((uint32_t)part_max[w], (uint32_t)parts[k][w]);
+    *(v4i *)(groups + rg * (kTC / 2) + cc * 4) = part_max;
+    __syncthreads();
+    for (int i = t; i < 8 * (kTC / 2); i += 256) {
+      const int pair = i % (kTC / 2), part = i / (kTC / 2);
+      uint32_t m = 0;
+#pragma unroll
+      for (int g = 0; g < kRG / 8; ++g) m = pk_absmax_u16(m, groups[(part * (kRG / 8) + g) * (kTC / 2) + pair]);
+      eighths[part * (kTC / 2) + pair] = m;
+    }
+    __syncthreads();
+    uint32_t m = 0;
+#pragma unroll
+    for (int part = 0; part < 8; ++part) m = pk_absmax_u16(m, eighths[part * (kTC / 2) + (t % kTC) / 2]);
+    amax_lo = (t & 1) ? m & 0xffff0000u : m << 16;  // bf16 -> fp32 bit patterns
+    if (t < kTC) lds.amaxes[t] = amax_lo;
+  }
   if (PER_COL) {
     // every wave computes the 64 scales (a branch around the division would pull the amax's load into it, behind
     // the tile's loads); the first one keeps them
@@ -785,7 +853,8 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
       float rc;
       if (PER_COL) {
         if (recips[cc * 8 + j] == recips[cc * 8 + j]) continue;
-        rc = recip_exact(scale_from_amax_bits32(col_amax[c + j < C ? c + j : 0], scale_rule));
+        const uint32_t bits = PARTIALS ? lds.amaxes[cc * 8 + j] : col_amax[c + j < C ? c + j : 0];
+        rc = recip_exact(scale_from_amax_bits32(bits, scale_rule));
       } else {
         rc = rcp[0];
       }
@@ -818,6 +887,43 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
       }
     }
   }
+}
+#endif
+
+// MANY: the operands come from a list, all of one kind.
+template <AmaxFrom FROM, int TC, int TU, bool MANY = false>
+__global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditional_t<MANY, TransposedOperands, TransposedOperand> list, int scale_rule) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ TransposeShared<TC, TU> lds;
+  if constexpr (MANY) {
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kMaxTransposed; ++i) which += (int)blockIdx.x >= list.op[i].first ? 1 : 0;
+    const TransposedOperand &op = list.op[which];
+    transpose_tile<FROM, TC, TU>(op, blockIdx.x - (unsigned)op.first, scale_rule, lds);
+  } else {
+    transpose_tile<FROM, TC, TU>(list, blockIdx.x, scale_rule, lds);
+  }
+#endif
+}
+
+// Operands of several kinds: the weight (row amaxes), the output gradient (partial maxima, or column amaxes) and the
+// activation (column amaxes) of a linear's backward pass while each is small.  Bound by what a launch costs: us, all casts of
+// the pass, five launches / two: M = 1021 N = K = 2048 14.4 / 10.6, 256 1024 1024 10.8 / 6.9, 1000 3008 2000 19.6 / 17.7,
+// 256 8192 1024 17.3 / 14.3; and as many calls less for the host, which such a pass waits for: forward + backward of the first,
+// with a bias, 143 -> 77.
+template <int TC, int TU>
+__global__ __launch_bounds__(256) void cast_transposed_mixed_kernel(const TransposedOperands list, int scale_rule) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __shared__ TransposeShared<TC, TU> lds;
+  int which = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxTransposed; ++i) which += (int)blockIdx.x >= list.op[i].first ? 1 : 0;
+  const TransposedOperand &op = list.op[which];
+  const unsigned block = blockIdx.x - (unsigned)op.first;
+  if (op.from == AmaxFrom::kRows) transpose_tile<AmaxFrom::kRows, TC, TU>(op, block, scale_rule, lds);
+  else if (op.from == AmaxFrom::kPartials) transpose_tile<AmaxFrom::kPartials, TC, TU>(op, block, scale_rule, lds);
+  else transpose_tile<AmaxFrom::kColumns, TC, TU>(op, block, scale_rule, lds);
 #endif
 }
 
@@ -905,6 +1011,36 @@ static int launch_rowwise_wg(const void *x, int64_t R, int64_t C, int64_t ldx, v
   L8_HIP(hipGetLastError());
   return L8_OK;
 }
+
+// Operands of one width in one launch, those with partials collecting column maxima; their folds (operand i's slots in
+// slots[i], at most rowwise_blocks of it) are left to the caller.
+static int cast_rowwise_groups(const l8_cast_rowwise_cols_item *items, int n, int64_t C, int64_t *slots, hipStream_t st) {
+  RowGroups list{};
+  int64_t rows = 0, first = 0;
+  for (int i = 0; i < n; ++i) rows += items[i].R;
+  const int64_t all = rowwise_blocks(rows, C, true);
+  for (int i = 0; i < kMaxRowOperands; ++i) {
+    if (i >= n) {
+      list.op[i].first = INT32_MAX;
+      continue;
+    }
+    const l8_cast_rowwise_cols_item &t = items[i];
+    const int64_t most = rowwise_blocks(t.R, C, true), share = all * t.R / rows;
+    slots[i] = share < 1 ? 1 : share < most ? share : most;
+    list.op[i] = {(const uint16_t *)t.x, t.R, t.ldx, (uint8_t *)t.q, t.ldq, t.scale, (uint16_t *)t.amax,
+                  t.col_amax ? (uint16_t *)t.workspace : nullptr, (int)first, (int)slots[i]};
+    first += slots[i];
+  }
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)first), dim3(kRowBlock), (size_t)C * sizeof(uint16_t), st, nullptr, 0, (int)C, 0, nullptr, 0,
+                       nullptr, nullptr, nullptr, l8::scale_rule(), list);
+  };
+  if (C <= 4 * 512) go(cast_rowwise_kernel<4, true, true>);
+  else go(cast_rowwise_kernel<8, true, true>);
+  L8_HIP(hipGetLastError());
+  return L8_OK;
+}
+constexpr int64_t kMaxGroupColumns = 8 * 512;  // a wavefront per row
 
 static int cast_rowwise_many(const l8_cast_rowwise_item *items, int n, int64_t C, hipStream_t st) {
   RowOperands list{};
@@ -1060,6 +1196,19 @@ extern "C" int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void
   return L8_OK;
 }
 
+static bool group_serves(const l8_cast_rowwise_cols_item &t, int64_t C) {
+  return t.C == C && many_serves(l8_cast_rowwise_item{t.x, t.R, t.ldx, t.q, t.ldq, t.scale, t.amax}, C);
+}
+
+int l8::cast_rowwise_pair(const l8_cast_rowwise_cols_item *two, hipStream_t st, bool *served) {
+  const int64_t C = two[0].C;
+  *served = C > 0 && C <= kMaxGroupColumns && group_serves(two[0], C) && group_serves(two[1], C);
+  if (!*served) return L8_OK;
+  int64_t slots[kMaxRowOperands];
+  const int rc = cast_rowwise_groups(two, 2, C, slots, st);
+  return rc == L8_OK ? fold_colmax(two[0].workspace, slots[0], C, two[0].col_amax, st) : rc;
+}
+
 extern "C" int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items, int64_t n, void *stream) {
   L8_REQUIRE(n >= 0 && (n == 0 || items), "l8_cast_rowwise_cols_many: null items, or a negative count");
   for (int64_t i = 0; i < n; ++i) {
@@ -1071,22 +1220,44 @@ extern "C" int l8_cast_rowwise_cols_many(const l8_cast_rowwise_cols_item *items,
   }
   FoldOperand folds[kMaxFolds];
   int pending = 0;
-  for (int64_t i = 0; i < n; ++i) {
+  auto flush = [&]() {
+    const int rc = pending ? fold_colmax_many(folds, pending, (hipStream_t)stream) : L8_OK;
+    pending = 0;
+    return rc;
+  };
+  for (int64_t i = 0; i < n;) {
     const l8_cast_rowwise_cols_item &t = items[i];
     if (t.R == 0 || t.C == 0) {
       const int rc = empty_col_amax(t.col_amax, t.C, (hipStream_t)stream);
       if (rc != L8_OK) return rc;
+      ++i;
       continue;
     }
-    int rc = cast_rowwise_impl("l8_cast_rowwise_cols_many", t.x, t.R, t.C, t.ldx, t.q, t.ldq, t.scale, t.amax, t.col_amax, t.workspace,
-                               (hipStream_t)stream, &folds[pending]);
-    if (rc == L8_OK && folds[pending].C > 0 && ++pending == kMaxFolds) {
-      rc = fold_colmax_many(folds, pending, (hipStream_t)stream);
-      pending = 0;
+    int run = 0;  // neighbours of one width that one launch can serve
+    while (i + run < n && run < kMaxRowOperands && t.C <= kMaxGroupColumns && group_serves(items[i + run], t.C)) ++run;
+    if (run > 1) {
+      if (pending + run > kMaxFolds) {
+        const int rc = flush();
+        if (rc != L8_OK) return rc;
+      }
+      int64_t slots[kMaxRowOperands];
+      const int rc = cast_rowwise_groups(items + i, run, t.C, slots, (hipStream_t)stream);
+      if (rc != L8_OK) return rc;
+      for (int k = 0; k < run; ++k) folds[pending++] = {items[i + k].workspace, items[i + k].col_amax, slots[k], t.C};
+      i += run;
+    } else {
+      int rc = cast_rowwise_impl("l8_cast_rowwise_cols_many", t.x, t.R, t.C, t.ldx, t.q, t.ldq, t.scale, t.amax, t.col_amax, t.workspace,
+                                 (hipStream_t)stream, &folds[pending]);
+      if (rc != L8_OK) return rc;
+      if (folds[pending].C > 0) ++pending;
+      ++i;
     }
-    if (rc != L8_OK) return rc;
+    if (pending == kMaxFolds) {
+      const int rc = flush();
+      if (rc != L8_OK) return rc;
+    }
   }
-  return pending ? fold_colmax_many(folds, pending, (hipStream_t)stream) : L8_OK;
+  return flush();
 }
 
 // ---------------------------------------------------------------------------
@@ -1207,9 +1378,10 @@ struct TransposedCast {
   float *scale;
 };
 
-// `n` casts of one kind (all from column amaxes, all from row amaxes, or one from a scalar) as one list of tiles.
+// `n` casts of one kind (all from column amaxes, all from row amaxes, or one from a scalar) as one list of tiles; with
+// `partials` (one per cast; those with slots stand in for column amaxes) of any kinds but the scalar.
 template <int TC, int TU>
-static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st) {
+static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st, const FoldOperand *partials = nullptr) {
   using T = TransposeTile<TC, TU>;
   static_assert(T::kTR <= kMaxTileRows, "the row-stride limit assumes no taller tile");
   TransposedOperands list{};
@@ -1222,13 +1394,26 @@ static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st
     const TransposedCast &t = a[i];
     const void *amax = t.col_amax ? (const void *)t.col_amax : t.amax_rows ? t.amax_rows : t.amax;
     list.op[i] = {(const uint16_t *)t.x, t.R, t.ldx, amax, (uint8_t *)t.q, t.ldq, t.Rp, t.scale, (int)t.C,
-                  t.amax_rows ? (int)t.n_amax : t.amax_f32, (t.ldq % 16 == 0 && aligned(t.q, 16)) ? 1 : 0, (int)gx};
+                  t.amax_rows ? (int)t.n_amax : t.amax_f32, (t.ldq % 16 == 0 && aligned(t.q, 16)) ? 1 : 0, (int)gx,
+                  t.col_amax ? AmaxFrom::kColumns : t.amax_rows ? AmaxFrom::kRows : AmaxFrom::kScalar};
+    if (partials && partials[i].slots) {
+      list.op[i].amax = partials[i].partials;
+      list.op[i].n_amax = (int)partials[i].slots;
+      list.op[i].from = AmaxFrom::kPartials;
+    }
     gx += ((t.C + T::kTC - 1) / T::kTC) * ((t.Rp + T::kTR - 1) / T::kTR);
     L8_REQUIRE(gx < INT32_MAX, "transposed cast: shape too large (%lld x %lld)", (long long)t.R, (long long)t.C);
   }
   auto go = [&](auto kernel, const auto &what) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)gx), dim3(256), 0, st, what, l8::scale_rule());
   };
+  if constexpr (TC == 64) {
+    if (partials) {
+      go(cast_transposed_mixed_kernel<TC, TU>, list);
+      L8_HIP(hipGetLastError());
+      return L8_OK;
+    }
+  }
   if (n > 1) {
     if (a[0].col_amax) go(cast_transposed_kernel<AmaxFrom::kColumns, TC, TU, true>, list);
     else go(cast_transposed_kernel<AmaxFrom::kRows, TC, TU, true>, list);
@@ -1257,6 +1442,18 @@ static int launch_transposed(const TransposedCast *a, int n, hipStream_t st) {
   if (large)  // the large activations: see the note on the tile shapes
     return launch_transposed_tile<128, 4>(a, n, st);
   return launch_transposed_tile<128, 2>(a, n, st);
+}
+
+// Up to this many partial rows a transposed cast's workgroup reads them itself (32 KB of its 64 columns from the L2, beside
+// 16 KB of its own operand) instead of waiting for a launch that folds them.
+constexpr int64_t kMaxReadPartials = 256;
+
+static bool bwd_casts_together(int64_t M, int64_t N, int64_t K) {
+  auto tiles = [](int64_t rows, int64_t cols) { return ((cols + 127) / 128) * ((rows + 127) / 128); };
+  const int64_t slots = rowwise_blocks(M, N, true);
+  // (in launch_transposed's terms: 64-column tiles)
+  return M > 0 && N > 0 && K > 0 && N % 8 == 0 && N <= kMaxAmaxRows && slots > 0 && slots <= kMaxReadPartials &&
+         tiles(M, N) + tiles(N, K) + tiles(M, K) < 4 * (int64_t)num_cus();
 }
 
 static int check_transposed(const char *what, const TransposedCast &a) {
@@ -1327,6 +1524,33 @@ extern "C" int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t 
                                               void *q, int64_t ldq, int64_t Rp, float *scale, void *stream) {
   return cast_colwise("l8_cast_colwise_transposed_pad", x, R, C, ldx, col_amax, q, ldq, Rp, scale, stream);
 }
+
+extern "C" int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *p) {
+  L8_REQUIRE(p && bwd_casts_together(p->M, p->N, p->K), "l8_linear_bwd_casts: null arguments, or a shape that l8_linear_bwd_casts_pays does not name");
+  const l8_linear_bwd_casts_args &a = *p;
+  hipStream_t st = (hipStream_t)a.stream;
+  L8_REQUIRE(a.g && a.qg && a.sg && a.qgt && a.sgt && (a.qwt == nullptr || (a.w && a.amax_w && a.swt && aligned(a.amax_w, 16))) &&
+                 (a.qat == nullptr || (a.a && a.a_col && a.sat)), "l8_linear_bwd_casts: null or misaligned pointer");
+  const int64_t need = l8_cast_rowwise_workspace(a.M, a.N);
+  L8_REQUIRE(a.workspace && a.workspace_bytes >= need && aligned(a.workspace, 16), "l8_linear_bwd_casts: needs a 16-byte aligned workspace of %lld bytes", (long long)need);
+  TransposedCast casts[3];
+  FoldOperand partials[3] = {};
+  int n = 0;
+  casts[n] = {a.g, a.M, a.N, a.ldg, nullptr, 0, nullptr, nullptr, 0, a.qgt, a.ldqgt, a.Mp, a.sgt};
+  partials[n++] = {a.workspace, nullptr, rowwise_blocks(a.M, a.N, true), a.N};
+  if (a.qat) casts[n++] = {a.a, a.M, a.K, a.lda, nullptr, 0, a.a_col, nullptr, 0, a.qat, a.ldqat, a.Mp, a.sat};
+  if (a.qwt) casts[n++] = {a.w, a.N, a.K, a.ldw, nullptr, 0, nullptr, a.amax_w, a.N, a.qwt, a.ldqwt, a.N, a.swt};
+  for (int i = 0; i < n; ++i) {
+    const int rc = check_transposed("l8_linear_bwd_casts", casts[i]);
+    if (rc != L8_OK) return rc;
+    L8_REQUIRE((int64_t)kMaxTileRows * casts[i].ldx * 2 < (1LL << 30), "l8_linear_bwd_casts: row stride too large (%lld elements)", (long long)casts[i].ldx);
+  }
+  // (the column amaxes' place is not written: the partial maxima stay in the workspace for the casts behind)
+  const int rc = launch_rowwise_any("l8_linear_bwd_casts", a.g, a.M, a.N, a.ldg, a.qg, a.ldqg, a.sg, nullptr, (float *)a.workspace, a.workspace, st);
+  return rc == L8_OK ? launch_transposed_tile<64, 1>(casts, n, st, partials) : rc;
+}
+
+extern "C" int l8_linear_bwd_casts_pays(int64_t M, int64_t N, int64_t K) { return bwd_casts_together(M, N, K) ? 1 : 0; }
 
 extern "C" int l8_cast_transposed_many(const l8_cast_transposed_item *items, int64_t n, void *stream) {
   L8_REQUIRE(n >= 0 && (n == 0 || items), "l8_cast_transposed_many: null items, or a negative count");

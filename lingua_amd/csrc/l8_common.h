@@ -47,6 +47,11 @@ struct FoldOperand {
 };
 int fold_colmax_many(const FoldOperand *ops, int n, hipStream_t st);
 
+// Row-wise casts of two operands of one width in one launch, the first with column amaxes (workspace of
+// l8_cast_rowwise_workspace bytes), the second without.  *served: whether the kernel takes operands like these (else nothing
+// is enqueued).  Defined in cast_kernels.hip.
+int cast_rowwise_pair(const l8_cast_rowwise_cols_item *two, hipStream_t st, bool *served);
+
 // Column amaxes (if asked for) of an operand without rows: zeros, the maximum of nothing, so that the scales made of them
 // are finite and the products with the operand's copy are the zeros of an empty sum.  Defined in cast_kernels.hip.
 int empty_col_amax(float *col_amax, int64_t C, hipStream_t st);

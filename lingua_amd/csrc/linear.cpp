@@ -117,12 +117,18 @@ extern "C" int l8_linear_fwd_rows(const l8_linear_fwd_args *a, int64_t ldqx, int
   L8_REQUIRE(ws.used <= a->workspace_bytes && ((uintptr_t)a->workspace % 256) == 0,
              "l8_linear_fwd: needs a 256-byte aligned workspace of %lld bytes", (long long)ws.used);
   const bool cast_x = !a->x_ready && !t.x_on_the_way, cast_w = !t.w_on_the_way && !a->w_ready;
-  const bool together = cast_x && cast_w && !a->col_amax_x;
-  if (together) {
+  bool together = cast_x && cast_w && !a->col_amax_x;
+  if (cast_x && cast_w && a->col_amax_x) {
+    const l8_cast_rowwise_cols_item two[2] = {{a->x, a->M, a->K, a->ldx, t.qx, t.ldqx, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes},
+                                              {a->w, a->N, a->K, a->ldw, t.qw, t.ldqw, t.sw, a->amax_w, nullptr, nullptr, 0}};
+    rc = cast_rowwise_pair(two, (hipStream_t)a->stream, &together);
+    if (rc != L8_OK) return rc;
+  } else if (together) {
     const l8_cast_rowwise_item items[2] = {{a->x, a->M, a->ldx, t.qx, t.ldqx, t.sx, nullptr}, {a->w, a->N, a->ldw, t.qw, t.ldqw, t.sw, a->amax_w}};
     rc = l8_cast_rowwise_many(items, 2, a->K, a->stream);
     if (rc != L8_OK) return rc;
-  } else if (cast_x) {
+  }
+  if (cast_x && !together) {
     rc = l8_cast_rowwise(a->x, a->M, a->K, a->ldx, t.qx, t.ldqx, t.sx, nullptr, a->col_amax_x, t.col_ws, t.col_ws_bytes, a->stream);
     if (rc != L8_OK) return rc;
   }

@@ -27,7 +27,7 @@ struct Library {
 #define L8_ENTRY(name) decltype(&::name) name = nullptr;
 #define L8_ENTRIES(X)                                                                                                        \
   X(l8_last_error) X(l8_linear_fwd_rows) X(l8_linear_fwd_rows_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
-  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_col_sum) X(l8_col_sum_workspace) X(l8_gemm_nt)
+  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_col_sum) X(l8_col_sum_workspace) X(l8_gemm_nt) X(l8_linear_bwd_casts) X(l8_linear_bwd_casts_pays)
   L8_ENTRIES(L8_ENTRY)
 #undef L8_ENTRY
 } lib;
@@ -212,10 +212,35 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
     pybind11::gil_scoped_release no_gil;
     const auto o = g.options();
     void *stream = c10::hip::getCurrentHIPStream((c10::DeviceIndex)device).stream();
-    Tensor g_col;
-    if (need_b) g_col = at::empty({N}, o.dtype(at::kFloat));
-    if (need_a) {
-      Tensor qg = empty_fp8(M, N, o), sg = at::empty({M, 1}, o.dtype(at::kFloat));
+    Tensor g_col, qg, sg, qgt, sgt;
+    // the casts of a small pass in two launches
+    const bool together = need_a && need_b && !(need_b && !qat.defined() && !a_col_in.defined()) &&
+                          (reinterpret_cast<uintptr_t>(amax.const_data_ptr()) % 16) == 0 && lib.l8_linear_bwd_casts_pays(M, N, K);
+    if (together) {
+      l8_linear_bwd_casts_args c{};
+      qg = empty_fp8(M, N, o), sg = at::empty({M, 1}, o.dtype(at::kFloat));
+      qgt = empty_fp8(N, padded, o), sgt = at::empty({N, 1}, o.dtype(at::kFloat));
+      c.g = rg.p, c.M = M, c.N = N, c.ldg = rg.ld, c.K = K, c.Mp = padded, c.stream = stream;
+      c.qg = qg.mutable_data_ptr(), c.ldqg = qg.stride(0), c.sg = sg.mutable_data_ptr<float>();
+      c.qgt = qgt.mutable_data_ptr(), c.ldqgt = qgt.stride(0), c.sgt = sgt.mutable_data_ptr<float>();
+      if (!qat.defined()) {
+        qat = empty_fp8(K, padded, o), sat = at::empty({K, 1}, o.dtype(at::kFloat));
+        c.a = ra.p, c.lda = ra.ld, c.a_col = a_col_in.const_data_ptr<float>();
+        c.qat = qat.mutable_data_ptr(), c.ldqat = qat.stride(0), c.sat = sat.mutable_data_ptr<float>();
+      }
+      if (!qwt.defined()) {
+        qwt = empty_fp8(K, N, o), swt = at::empty({1, 1}, o.dtype(at::kFloat));
+        c.w = rw.p, c.ldw = rw.ld, c.amax_w = amax.const_data_ptr();
+        c.qwt = qwt.mutable_data_ptr(), c.ldqwt = qwt.stride(0), c.swt = swt.mutable_data_ptr<float>();
+      }
+      c.workspace_bytes = lib.l8_cast_rowwise_workspace(M, N);
+      const Space ws(g, c.workspace_bytes);
+      c.workspace = ws.p();
+      check(lib.l8_linear_bwd_casts(&c), "l8_linear_bwd_casts");
+    }
+    if (need_b && !together) g_col = at::empty({N}, o.dtype(at::kFloat));
+    if (need_a && !together) {
+      qg = empty_fp8(M, N, o), sg = at::empty({M, 1}, o.dtype(at::kFloat));
       const int64_t ws_bytes = need_b ? lib.l8_cast_rowwise_workspace(M, N) : 0;
       const Space ws(g, ws_bytes);
       check(lib.l8_cast_rowwise(rg.p, M, N, rg.ld, qg.mutable_data_ptr(), qg.stride(0), sg.mutable_data_ptr<float>(), nullptr,
@@ -233,6 +258,8 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
                 "l8_cast_tensorwise");
         }
       }
+    }
+    if (need_a) {
       ga = at::empty({M, K}, o);
       check(lib.l8_gemm_nt(qg.const_data_ptr(), qwt.const_data_ptr(), M, K, N, qg.stride(0), qwt.stride(0), sg.const_data_ptr<float>(), L8_SCALE_ROW, swt.const_data_ptr<float>(),
                            L8_SCALE_SCALAR, nullptr, ga.mutable_data_ptr(), K, algo, stream), "l8_gemm_nt");
@@ -240,8 +267,8 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       check(lib.l8_col_amax(rg.p, M, N, rg.ld, g_col.mutable_data_ptr<float>(), stream), "l8_col_amax");
     }
     if (need_b) {
-      Tensor qgt, sgt;
-      if (qat.defined()) {
+      if (together) {   // made above
+      } else if (qat.defined()) {
         cast_colwise_t(g, rg, g_col, true, qgt, sgt, stream);
       } else {
         Tensor a_col = a_col_in;

@@ -636,3 +636,62 @@ def test_bias_gradient_of_rows_off_16_byte_lines(shift):
     got = linear_backward(wide[:, shift:], None, torch.zeros(64, 32, dtype=torch.bfloat16, device="cuda"),
                           torch.zeros(64, dtype=torch.bfloat16, device="cuda"), None, False, False, True, False, 0)
     assert got[0] is None and got[1] is None and torch.equal(got[2], wide[:, shift:].double().sum(0).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows,C", [((1, 3, 5), 8), ((600, 2, 4093), 520), ((1021, 1021), 2048), ((33, 700, 5), 2056), ((4, 2100), 4096), ((9, 40), 4104)])
+@pytest.mark.parametrize("poison", [False, True])
+def test_column_amaxes_of_several_operands_in_one_launch(rows, C, poison):
+    """Operands that share a launch (and, of other widths, those that do not): bytes, scales and column amaxes of the casts one
+    by one, each with workgroups of its own whatever its share of the rows."""
+    from lingua_amd import ops
+    xs = [seeded_bf16((r, C + 8 * i), std=10.0 ** (i - 1), seed=r + i).cuda()[:, :C] for i, r in enumerate(rows)]
+    if poison:
+        xs[0][0, C // 2] = float("inf")
+        xs[1][rows[1] - 1, C - 1] = float("nan")
+    xs.append(seeded_bf16((5, 16), seed=3).cuda())
+    for x, (q, s, col) in zip(xs, ops.cast_rowwise_cols_many(xs)):
+        col0 = torch.empty_like(col)
+        q0, s0, _ = ops.cast_rowwise(x, col_amax=col0)
+        assert torch.equal(q.view(torch.uint8), q0.view(torch.uint8)) and bits_equal(s.cpu(), s0.cpu()) and bits_equal(col.cpu(), col0.cpu())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (5, 72, 200), (127, 64, 128), (129, 528, 48), (1021, 2048, 2048), (1024, 256, 2048), (256, 8192, 1024)])
+@pytest.mark.parametrize("poison", [False, True])
+def test_casts_of_a_backward_pass_in_two_launches(M, N, K, poison):
+    """l8_linear_bwd_casts against the casts one by one: up to 256 rows of partial column maxima are read by the workgroups of the
+    transposed cast, each of its three operands at tile edges, with rows apart, with column amaxes that are not finite."""
+    import struct
+    from lingua_amd import _lib, ops
+    lib = _lib.load()
+    assert lib.l8_linear_bwd_casts_pays(M, N, K) and not lib.l8_linear_bwd_casts_pays(1025, N, K)
+    g, a, w = (seeded_bf16((r, c + 8), std=s, seed=r + c).cuda()[:, :c] for r, c, s in ((M, N, 1e-2), (M, K, 1.0), (N, K, 0.02)))
+    if poison:
+        g[M // 2, N // 2] = float("inf")
+        g[M - 1, 0] = float("nan")
+        a[0, K - 1] = float("nan")
+    Mp = (M + 15) // 16 * 16
+    g_col, a_col = (torch.empty(c, dtype=torch.float32, device="cuda") for c in (N, K))
+    qg0, sg0, _ = ops.cast_rowwise(g, col_amax=g_col)
+    ops.cast_rowwise(a, col_amax=a_col)
+    _, _, amax_w = ops.cast_rowwise(w)
+    want = [(qg0, sg0), ops.cast_colwise_transposed(g, g_col), ops.cast_colwise_transposed(a, a_col),
+            ops.cast_tensorwise(w, ops.amax_reduce(amax_w), transpose=True)]
+    for parts in (3, 2, 1):     # gradient, activation and weight; the weight or the activation ready
+        got = [(torch.full((r, c + 16), 0x55, dtype=torch.uint8, device="cuda")[:, :c], torch.empty(n, dtype=torch.float32, device="cuda"))
+               for r, c, n in ((M, N, M), (N, Mp, N), (K, Mp, K), (K, N, 1))]
+        need = lib.l8_cast_rowwise_workspace(M, N)
+        ws = torch.empty(need + 16, dtype=torch.uint8, device="cuda")
+        p = [t.data_ptr() for pair in got for t in pair]
+        ld = [q.stride(0) for q, _ in got]
+        with_a, with_w = parts != 1, parts != 2
+        args = [g.data_ptr(), M, N, g.stride(0), p[0], ld[0], p[1], p[2], ld[1], p[3], Mp,
+                a.data_ptr(), K, a.stride(0), a_col.data_ptr(), p[4] if with_a else 0, ld[2], p[5],
+                w.data_ptr(), w.stride(0), amax_w.data_ptr(), p[6] if with_w else 0, ld[3], p[7],
+                ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream]
+        _lib.check(lib.l8_linear_bwd_casts(struct.pack("27q", *args)), "l8_linear_bwd_casts")
+        for i, ((q, s), (q0, s0)) in enumerate(zip(got, want)):
+            if (i == 2 and not with_a) or (i == 3 and not with_w):
+                assert (q == 0x55).all()
+                continue
+            assert torch.equal(q, q0.view(torch.uint8)), i
+            assert bits_equal(s.cpu(), s0.cpu().reshape(-1)), i
