@@ -275,6 +275,45 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   }
   const int chunk_even = (lpos ^ lrow) * 16, chunk_odd = (lpos ^ lrow ^ 1) * 16;  // byte offset in the row, by parity of g
 
+  // ---- scales and bias ----
+  // The small tiles request them in front of their panels: loads retire in order, so they are there when the K loop starts,
+  // and the partial waits below count as before.  Requested behind the loop, with a branch around each load, a product of a
+  // few microseconds ended in the latency of loads that wait for one another.  us, operands cold, before / now: [1021,2048].
+  // [2048,2048] with a bias 12.4 / 9.8, without 10.0 / 9.6; [32,4096].[11008,4096] 16.2 / 14.3 and 14.7 / 14.3; [128,1024].
+  // [1024,1024] without 6.0 / 5.6.  Two 128 x 128 workgroups on a unit cover for each other: there the registers are worth more
+  // (requested early [64,4096].[36864,4096] 46.4 -> 46.9).
+  constexpr bool EARLY = DEEP;
+  const int l31 = lane & 31, h = lane >> 5;
+  float sav[TM], sb_all;
+  float sbv[TN][4][4];  // of the 16 n per 32-column tile that this lane holds before the half-wave swap
+  v2i biasv[TN][4];
+  const bool bias_vec = p.bias && ((uintptr_t)p.bias & 7) == 0 && p.N % 2 == 0;  // whole dwords up to column N
+  auto scales = [&]() __attribute__((always_inline)) {
+    const int m_left = p.M - m0 < BM ? p.M - m0 : BM, n_left = p.N - n0 < BN ? p.N - n0 : BN;
+    const __amdgpu_buffer_rsrc_t rsSa = make_rsrc(p.sa + (p.sa_row ? m0 : 0), p.sa_row ? m_left * 4 : 4);
+    const __amdgpu_buffer_rsrc_t rsSb = make_rsrc(p.sb + (p.sb_row ? n0 : 0), p.sb_row ? n_left * 4 : 4);
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+      sav[tm] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsSa, p.sa_row ? ((wm * TM + tm) * 32 + l31) * 4 : 0, 0, 0));
+    sb_all = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsSb, 0, 0, 0));  // the one scale, if it is one
+#pragma unroll
+    for (int i = 0; i < TN * 4; ++i) {
+      const v4i t = __builtin_amdgcn_raw_buffer_load_b128(rsSb, ((wn * TN + i / 4) * 32 + 8 * (i % 4) + 4 * h) * 4, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sbv[i / 4][i % 4][e] = __uint_as_float((uint32_t)t[e]);
+    }
+    if (bias_vec) {
+      const __amdgpu_buffer_rsrc_t rsBias = make_rsrc(p.bias + n0, n_left * 2);
+#pragma unroll
+      for (int i = 0; i < TN * 4; ++i)
+        biasv[i / 4][i % 4] = __builtin_amdgcn_raw_buffer_load_b64(rsBias, ((wn * TN + i / 4) * 32 + 8 * (i % 4) + 4 * h) * 2, 0, 0);
+    }
+  };
+  if constexpr (EARLY) {
+    if (group == 0) scales();
+    asm volatile("" ::: "memory");
+  }
+
   const int KT = (p.K + BK * KS - 1) / (BK * KS);  // trips
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr_t)smem + group * RING;
   auto wrap = [](int slot) { return slot >= R ? slot - R : slot; };  // slot in [0, 2R)
@@ -313,7 +352,6 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   };
 
   // ---- LDS -> register fragment plan ----
-  const int l31 = lane & 31, h = lane >> 5;
   const int fr = (l31 & 7) ^ ((l31 >> 3) & 1);
   uint32_t foff[2][2];
 #pragma unroll
@@ -507,33 +545,22 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   }
   }
   // ---- epilogue ----
-  // All scales of this wave's part of the tile are requested in one batch,
-  // before the wait that drains the ring: one memory latency in total,
-  // overlapped with that wait, instead of one per 32-column tile.
-  const float sa_s = p.sa[0], sb_s = p.sb[0];
-  float sav[TM];
+  if constexpr (!EARLY) scales();  // one memory latency, under the wait that drains the ring
+  if (!p.sb_row) {
 #pragma unroll
-  for (int tm = 0; tm < TM; ++tm) {
-    const int m = m0 + (wm * TM + tm) * 32 + l31;
-    sav[tm] = p.sa_row ? (m < p.M ? p.sa[m] : 0.0f) : sa_s;
+    for (int i = 0; i < TN * 16; ++i) sbv[i / 16][i / 4 % 4][i % 4] = sb_all;
   }
-  // scales of the 16 n per 32-column tile that this lane holds before the half-wave swap
-  float sbv[TN][4][4];
-  const bool sb_vec = p.sb_row && (((uintptr_t)p.sb & 15) == 0);
+  if (p.bias && !bias_vec) {  // element by element
+    const __amdgpu_buffer_rsrc_t rsBias = make_rsrc(p.bias + n0, (p.N - n0 < BN ? p.N - n0 : BN) * 2);
 #pragma unroll
-  for (int tn = 0; tn < TN; ++tn)
+    for (int i = 0; i < TN * 4; ++i) {
+      uint32_t b[4];
 #pragma unroll
-    for (int qd = 0; qd < 4; ++qd) {
-      const int nq = n0 + (wn * TN + tn) * 32 + 8 * qd + 4 * h;  // four consecutive n
-      if (sb_vec && nq + 4 <= p.N) {
-        const v4f t = *(const v4f *)(p.sb + nq);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sbv[tn][qd][e] = t[e];
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) sbv[tn][qd][e] = p.sb_row ? (nq + e < p.N ? p.sb[nq + e] : 0.0f) : sb_s;
-      }
+      for (int e = 0; e < 4; ++e)
+        b[e] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rsBias, ((wn * TN + i / 4) * 32 + 8 * (i % 4) + 4 * h + e) * 2, 0, 0);
+      biasv[i / 4][i % 4] = v2i{(int)(b[0] | b[1] << 16), (int)(b[2] | b[3] << 16)};
     }
+  }
   // every wave's tail loads (out of range, zero-filling) and LDS reads are done
   // before the ring is reused as the staging area of the C tile
   L8_WAIT_VM_LGKM0(0);
@@ -589,17 +616,6 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
     constexpr bool HAS_BIAS = decltype(has_bias)::value;
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) {
-    // the bias (rare: the linears of the model have none) is fetched per 32-column tile
-    float biasv[4][4];
-    if constexpr (HAS_BIAS) {
-#pragma unroll
-      for (int qd = 0; qd < 4; ++qd)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int n = n0 + (wn * TN + tn) * 32 + 8 * qd + 4 * h + e;
-          biasv[qd][e] = n < p.N ? bf16_bits_to_f32(p.bias[n]) : 0.0f;
-        }
-    }
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       const float sa = sav[tm];
@@ -610,7 +626,7 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           v[e] = acc[tn][tm][qd * 4 + e] * sa * sbv[tn][qd][e];
-          if constexpr (HAS_BIAS) v[e] += biasv[qd][e];
+          if constexpr (HAS_BIAS) v[e] += bf16_bits_to_f32(((uint32_t)biasv[tn][qd][e >> 1] >> (16 * (e & 1))) & 0xffffu);
         }
         typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
         bf2 lo = {(__bf16)v[0], (__bf16)v[1]}, hi = {(__bf16)v[2], (__bf16)v[3]};
