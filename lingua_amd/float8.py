@@ -517,6 +517,16 @@ def shared_input_backward(grads, a, ws, amaxes, a_col_amax, need_a: bool, need_w
             raise RuntimeError(f"Fp8LinearFn.backward: bf16 grad_out required, got {g.dtype}")
     _fwd_cast.clear(a)
     _fwd_tcast.clear(a)
+    # the memo answers once: both forms below go by this answer
+    learning = [i for i, need in enumerate(need_ws) if need]
+    user = ws[learning[0]].data_ptr() if learning else None
+    hit = _bwd_cast.get(a, user) if learning and config.share_input_casts else None
+    if need_a and len(learning) == len(ws) and not config.cache_weight_casts and _native_call(a, gemm_algo) and not torch.is_grad_enabled():
+        res = _lib.native_for(a.get_device()).shared_bwd(tuple(grads), a, tuple(ws), tuple(amaxes), a_col_amax, *(hit or (None, None)), gemm_algo)
+        if res is not None:
+            if hit is None and config.share_input_casts:
+                _bwd_cast.put(a, res[1:3], user)
+            return res[0], list(res[3:])
     grad_a, cols = None, [None] * len(grads)
     if need_a:
         which = [i for i, need in enumerate(need_ws) if need]
@@ -529,12 +539,9 @@ def shared_input_backward(grads, a, ws, amaxes, a_col_amax, need_a: bool, need_w
         grad_a = ops.gemm_nt_sum(qgs, qwts, sgs, swts, algo=gemm_algo)
         del qgs, qwts
         del quantised
-    learning = [i for i, need in enumerate(need_ws) if need]
     grad_ws = [None] * len(grads)
     if learning:
         casts = [(grads[i], cols[i] if cols[i] is not None else ops.col_amax(grads[i])) for i in learning]
-        user = ws[learning[0]].data_ptr()
-        hit = _bwd_cast.get(a, user) if config.share_input_casts else None
         if hit is None:
             casts.append((a, a_col_amax if a_col_amax is not None else ops.col_amax(a)))
         qts = ops.cast_transposed_many(casts, on_lines=True)

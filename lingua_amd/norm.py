@@ -15,8 +15,8 @@ import re
 
 import torch
 
+from . import _lib, ops
 from . import float8 as f8
-from . import ops
 
 
 class Fp8RMSNormFn(torch.autograd.Function):
@@ -25,8 +25,13 @@ class Fp8RMSNormFn(torch.autograd.Function):
         if x.dtype != torch.bfloat16:
             raise RuntimeError(f"Fp8RMSNorm: bf16 activations required, got {x.dtype}")
         x2d = x.flatten(end_dim=-2)
-        col = torch.empty(x2d.shape[1], dtype=torch.float32, device=x.device) if (training and f8.config.fp8_wgrad) else None
-        y2d, q, s, rstd = ops.rmsnorm_cast_rowwise(x2d, weight, eps, want_q=True, col_amax=col, want_rstd=True, on_lines=True)
+        want_col, res = bool(training and f8.config.fp8_wgrad), None
+        if f8._native_call(x2d, 0):
+            res = _lib.native_for(x2d.get_device()).rmsnorm_fwd(x2d, weight, eps, want_col)
+        if res is None:
+            col = torch.empty(x2d.shape[1], dtype=torch.float32, device=x.device) if want_col else None
+            res = (*ops.rmsnorm_cast_rowwise(x2d, weight, eps, want_q=True, col_amax=col, want_rstd=True, on_lines=True), col)
+        y2d, q, s, rstd, col = res
         if f8.config.share_input_casts:
             f8._fwd_cast.put(y2d, (q, s, col), "rmsnorm")
         ctx.save_for_backward(x2d, weight, rstd)
@@ -38,7 +43,10 @@ class Fp8RMSNormFn(torch.autograd.Function):
         x2d, weight, rstd = ctx.saved_tensors
         if gy.dtype != torch.bfloat16:
             raise RuntimeError(f"Fp8RMSNorm.backward: bf16 grad_out required, got {gy.dtype}")
-        gx2d, gw = ops.rmsnorm_bwd(gy.flatten(end_dim=-2), x2d, weight, rstd, gw_dtype=weight.dtype)
+        gy2d, res = gy.flatten(end_dim=-2), None
+        if f8._native_call(gy2d, 0):
+            res = _lib.native_for(gy2d.get_device()).rmsnorm_bwd(gy2d, x2d, weight, rstd)
+        gx2d, gw = ops.rmsnorm_bwd(gy2d, x2d, weight, rstd, gw_dtype=weight.dtype) if res is None else res
         gx = gx2d.reshape(ctx.x_shape) if ctx.needs_input_grad[0] else None
         return gx, (gw if ctx.needs_input_grad[1] else None), None, None
 

@@ -28,8 +28,8 @@ import re
 
 import torch
 
+from . import _lib, ops
 from . import float8 as f8
-from . import ops
 
 
 class Fp8QKVFn(torch.autograd.Function):
@@ -44,22 +44,34 @@ class Fp8QKVFn(torch.autograd.Function):
         cfg = f8.config
         need_stats = cfg.fp8_wgrad and any(w.requires_grad for w in ws)
         f8._bwd_cast.clear(x)
-        hit = f8._fwd_cast.get(x, ("qkv", wq.data_ptr())) if cfg.share_input_casts else None
-        if hit is not None and (hit[2] is not None or not need_stats):
-            qx, sx, x_col = hit
-            if not need_stats:
-                x_col = None
-        else:
-            x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_stats else None
-            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
-            if cfg.share_input_casts:
-                f8._fwd_cast.put(x, (qx, sx, x_col), ("qkv", wq.data_ptr()))
-        K = x.shape[1]
+        user = ("qkv", wq.data_ptr())
+        hit = f8._fwd_cast.get(x, user) if cfg.share_input_casts else None
+        if hit is not None and hit[2] is None and need_stats:
+            hit = None
+        res = None
+        if x.dim() == 2 and f8._native_call(x, cfg.gemm_algo):
+            res = _lib.native_for(x.get_device()).qkv_fwd(x, wq, wk, wv, *(hit[:2] if hit else (None, None)), need_stats, cfg.gemm_algo)
         sizes = [w.shape[0] for w in ws]
-        qw = ops._empty_fp8(sum(sizes), K, x.device, True)
-        sw = torch.empty((sum(sizes), 1), dtype=torch.float32, device=x.device)
-        amaxes = [amax for _, _, amax in ops.cast_rowwise_many(ws, out=(qw, sw))]
-        y = ops.gemm_nt(qx, qw, sx, sw, None, algo=cfg.gemm_algo)
+        if res is not None:
+            y, *amaxes, qx, sx, x_col = res
+            if hit is not None:
+                x_col = hit[2] if need_stats else None
+            elif cfg.share_input_casts:
+                f8._fwd_cast.put(x, (qx, sx, x_col), user)
+        else:
+            if hit is not None:
+                qx, sx, x_col = hit
+                if not need_stats:
+                    x_col = None
+            else:
+                x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_stats else None
+                qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
+                if cfg.share_input_casts:
+                    f8._fwd_cast.put(x, (qx, sx, x_col), user)
+            qw = ops._empty_fp8(sum(sizes), x.shape[1], x.device, True)
+            sw = torch.empty((sum(sizes), 1), dtype=torch.float32, device=x.device)
+            amaxes = [amax for _, _, amax in ops.cast_rowwise_many(ws, out=(qw, sw))]
+            y = ops.gemm_nt(qx, qw, sx, sw, None, algo=cfg.gemm_algo)
         ctx.fp8_wgrad, ctx.gemm_algo, ctx.has_col = cfg.fp8_wgrad, cfg.gemm_algo, x_col is not None
         ctx.need = (x.requires_grad,) + tuple(w.requires_grad for w in ws)
         ctx.save_for_backward(x, *ws, *amaxes, *([x_col] if x_col is not None else []))

@@ -22,8 +22,8 @@ from typing import Optional
 
 import torch
 
+from . import _lib, ops
 from . import float8 as f8
-from . import ops
 
 
 class Fp8SwiGLUFn(torch.autograd.Function):
@@ -41,25 +41,36 @@ class Fp8SwiGLUFn(torch.autograd.Function):
         # an Fp8RMSNorm in front of this block has filed its output already quantised (with its column amaxes when
         # it ran in training mode): take that copy instead of quantising the activation a second time
         hit = f8._fwd_cast.get(x, ("swiglu", w1.data_ptr())) if cfg.share_input_casts else None
-        if hit is not None and (hit[2] is not None or not need_x_col):
-            qx, sx, x_col = hit
-            if not need_x_col:
-                x_col = None
-        else:
-            x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_x_col else None
-            qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
-        (q1, s1, amax_w1), (q3, s3, amax_w3) = f8.weight_casts_rowwise((w1, w3))
-        h1 = ops.gemm_nt(qx, q1, sx, s1, None, algo=algo)
-        h3 = ops.gemm_nt(qx, q3, sx, s3, None, algo=algo)
-        del qx, q1, q3
-        h_col = torch.empty(w2.shape[1], dtype=torch.float32, device=x.device) if fp8_wgrad and w2.requires_grad else None
+        if hit is not None and hit[2] is None and need_x_col:
+            hit = None
         # where every weight learns, backward makes the operands of the three weight gradients that come out of the gate
         # from h1, h3 and the gradient of h in one pass, and h itself is not kept
         regate = (fp8_wgrad and w1.requires_grad and w3.requires_grad and w2.requires_grad and x.shape[0] > 0 and
-                  h1.shape[1] <= ops.GATE_MAX_COLUMNS)
-        h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=w2.requires_grad and not regate, col_amax=h_col, on_lines=True)
-        q2, s2, amax_w2 = f8.weight_cast_rowwise(w2)
-        y = ops.gemm_nt(qh, q2, sh, s2, None, algo=algo)
+                  w1.shape[0] <= ops.GATE_MAX_COLUMNS)
+        want_h, need_h_col = w2.requires_grad and not regate, fp8_wgrad and w2.requires_grad
+        res = None
+        if not cfg.cache_weight_casts and f8._native_call(x, algo):
+            res = _lib.native_for(x.get_device()).swiglu_fwd(x, w1, w3, w2, *(hit[:2] if hit else (None, None)), need_x_col, need_h_col, want_h, algo)
+        if res is not None:
+            y, h1, h3, amax_w1, amax_w3, amax_w2, h, x_col, h_col = res
+            if hit is not None:
+                x_col = hit[2] if need_x_col else None
+        else:
+            if hit is not None:
+                qx, sx, x_col = hit
+                if not need_x_col:
+                    x_col = None
+            else:
+                x_col = torch.empty(x.shape[1], dtype=torch.float32, device=x.device) if need_x_col else None
+                qx, sx, _ = ops.cast_rowwise(x, col_amax=x_col, on_lines=True)
+            (q1, s1, amax_w1), (q3, s3, amax_w3) = f8.weight_casts_rowwise((w1, w3))
+            h1 = ops.gemm_nt(qx, q1, sx, s1, None, algo=algo)
+            h3 = ops.gemm_nt(qx, q3, sx, s3, None, algo=algo)
+            del qx, q1, q3
+            h_col = torch.empty(w2.shape[1], dtype=torch.float32, device=x.device) if need_h_col else None
+            h, qh, sh, _ = ops.swiglu_cast_rowwise(h1, h3, want_h=want_h, col_amax=h_col, on_lines=True)
+            q2, s2, amax_w2 = f8.weight_cast_rowwise(w2)
+            y = ops.gemm_nt(qh, q2, sh, s2, None, algo=algo)
 
         ctx.fp8_wgrad, ctx.gemm_algo = fp8_wgrad, algo
         ctx.need = (x.requires_grad, w1.requires_grad, w3.requires_grad, w2.requires_grad)
@@ -91,6 +102,12 @@ class Fp8SwiGLUFn(torch.autograd.Function):
             if need_w2:
                 gw2 = _wgrad(gy, None, h, h_col, fp8_wgrad, algo)
             return gx, gw1, gw3, gw2
+
+        if (ctx.regate and need_x and x_col is not None and not f8.config.cache_weight_casts and f8._native_call(gy, algo) and
+                not torch.is_grad_enabled()):
+            res = _lib.native_for(gy.get_device()).swiglu_bwd(gy, x, w1, w3, w2, h1, h3, amax_w1, amax_w3, amax_w2, x_col, h_col, algo)
+            if res is not None:
+                return res
 
         gy_col = torch.empty(D, dtype=torch.float32, device=dev) if fp8_wgrad and need_w2 else None
         qgy, sgy, _ = ops.cast_rowwise(gy, col_amax=gy_col, on_lines=True)
