@@ -514,11 +514,25 @@ __global__ __launch_bounds__(256) void col_sum_fold_kernel(const float *__restri
 }
 
 // bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
+// Bound by latencies: sixteen bytes per lane and load where the list is aligned, one round trip up to 32768 values.  us, two
+// bytes per load / sixteen: 4691 values 2.1 / 2.05, 16384 3.0 / 2.0, 28465 4.2 / 2.25.
 __global__ __launch_bounds__(1024) void amax_reduce_kernel(const uint16_t *__restrict__ amax, int64_t n,
                                                            uint16_t *__restrict__ out) {
   __shared__ uint32_t red[16];
   uint32_t m = 0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) m = max(m, (uint32_t)(amax[i] & 0x7fffu));
+  int64_t done = 0;
+  if (((uintptr_t)amax & 15) == 0) {
+    done = n / 8 * 8;
+    uint32_t pk = 0;
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i < n / 8; i += 1024) {
+      const v4i v = ((const v4i *)amax)[i];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) pk = pk_absmax_u16(pk, (uint32_t)v[k]);
+    }
+    m = max(pk & 0xffffu, pk >> 16);
+  }
+  for (int64_t i = done + threadIdx.x; i < n; i += 1024) m = max(m, (uint32_t)(amax[i] & 0x7fffu));
   m = wave_max_u32(m);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();

@@ -695,3 +695,15 @@ def test_casts_of_a_backward_pass_in_two_launches(M, N, K, poison):
                 continue
             assert torch.equal(q, q0.view(torch.uint8)), i
             assert bits_equal(s.cpu(), s0.cpu().reshape(-1)), i
+
+
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 1023, 8191, 8192, 32769, 65537])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_amax_reduce_edges(n, offset):
+    """Lists around one load per lane and one round of loads, on and off 16-byte lines, the maximum in each end; a NaN wins."""
+    from lingua_amd import ops
+    v = torch.rand(n + offset, generator=torch.Generator().manual_seed(n)).bfloat16()
+    for at, value in ((offset, -3.0), (n + offset - 1, 5.0), (offset + n // 2, float("nan"))):
+        v[at] = value
+        got = ops.amax_reduce(v.cuda()[offset:])
+        assert torch.equal(got.cpu().reshape(()), v[offset:].abs().max()) or (value != value and bool(got.isnan()))
