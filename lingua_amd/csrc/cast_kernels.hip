@@ -466,18 +466,20 @@ __global__ __launch_bounds__(256) void col_amax_kernel(const uint16_t *__restric
 // thousand rows on, by latency below: a workgroup owns 128 columns -- two lines of every row, which 64 columns read at the same
 // rate up to 4096 columns and 10 % slower beyond, and 256 half as fast at [16384,2048] -- and a slab of rows, read 16 at a time
 // with eight loads in flight per thread.  Slabs until there are four workgroups per unit, one per 128 rows begun at most and of
-// equal heights; several slabs leave fp32 partial sums that the second kernel adds in their order.  Up to 1024 rows one slab, by
-// twice the threads: a launch less ([512,4096] 5.2 / 3.1, [1021,2048] 5.2 / 5.0, [1024,11008] 7.6 / 5.8; [2048,2048] as one slab of
-// 512 threads 6.5 against 4.9).  From HBM its few workgroups take longer, with two launches to enqueue / with one [400,4096]
-// 8.4 / 5.9, [700,4096] 9.8 / 8.0, [1021,4096] 8.6 / 10.5, [1021,11008] 11.1 / 10.9: even at the limit.  The order of every sum
-// hangs on the shape and the number of compute units.  us, PyTorch's sum / this, back to back: [256,1024] 9.2 / 2.6, [1021,2048] 11.6 / 5.0, [1801,11040] 88 / 12,
-// [4096,4096] 19.8 / 9.4, [5580,12176] 369 / 33, [16384,2048] 28 / 16, [16384,11008] 69 / 68 (a copy's rate: 64)
+// equal heights; several slabs leave fp32 partial sums that the second kernel adds in their order.  The order of every sum
+// hangs on the shape and the number of compute units.  us, PyTorch's sum / this, back to back: [4096,4096] 19.8 / 9.4,
+// [5580,12176] 369 / 33, [16384,2048] 28 / 16, [16384,11008] 69 / 68 (a copy's rate: 64).
+//
+// Up to 2048 rows one launch whose workgroups own 32 columns and every row: a unit takes in some 40 bytes per clock, so what
+// counts is how many of them read.  us, from HBM, slabs (of 1024 rows, then; one launch up to there) / 128 columns per workgroup
+// of 1024 threads / 64 / 32: [400,4096] 4.7 / 4.6 / 3.6 / 3.3, [1021,2048] 7.7 / 7.0 / 6.0 / 4.1, [1021,4096] 11.1 / 10.8 / 9.1 /
+// 6.2, [1801,2048] 10.3 / 12.3 / 9.1 / 8.1, [1801,11040] 13.3 / 15.4 / 11.6 / 12.1; [3000,4096] 12.1 / 20.6 / 15.0 / 13.2.
 // ---------------------------------------------------------------------------
-constexpr int kSumCols = 128, kSumOneSlab = 1024;
-template <int THREADS>
-__global__ __launch_bounds__(THREADS) void col_sum_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx,
+constexpr int kSumCols = 128, kSumThreads = 256, kWholeCols = 32;
+constexpr int64_t kSumWhole = 2048;
+__global__ __launch_bounds__(kSumThreads) void col_sum_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx,
                                                           int64_t slab, float *__restrict__ partials, uint16_t *__restrict__ out) {
-  constexpr int kSumRows = THREADS / (kSumCols / 8);
+  constexpr int kSumRows = kSumThreads / (kSumCols / 8);
   __shared__ float sums[kSumRows][kSumCols + 1];
   const int cc = threadIdx.x % (kSumCols / 8), rg = threadIdx.x / (kSumCols / 8);
   const int col = blockIdx.x * kSumCols + cc * 8;
@@ -511,6 +513,38 @@ __global__ __launch_bounds__(256) void col_sum_fold_kernel(const float *__restri
 #pragma unroll 8
   for (int s = 0; s < slabs; ++s) t += partials[(int64_t)s * C + c];
   out[c] = (uint16_t)bf16_rne_bits(t);
+}
+
+// One launch.  Workgroups of one XCD take neighbouring columns: 64 bytes of a row are half a line.
+__global__ __launch_bounds__(1024) void col_sum_whole_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint16_t *__restrict__ out) {
+  constexpr int COLS = kWholeCols, kGroups = 1024 / (COLS / 8), kParts = 1024 / COLS;
+  __shared__ float sums[kGroups][COLS + 1];
+  __shared__ float parts[kParts][COLS];
+  const int n = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+  const int c0 = ((n >> 3) * xcd + (xcd < (n & 7) ? xcd : n & 7) + loc) * COLS;
+  const int cc = threadIdx.x % (COLS / 8), rg = threadIdx.x / (COLS / 8), col = c0 + cc * 8;
+  float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  if (col < C) {
+#pragma unroll 8
+    for (int64_t r = rg; r < R; r += kGroups) {
+      const v4i v = *(const v4i *)(x + r * ldx + col);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s[e] += __uint_as_float((e & 1) ? ((uint32_t)v[e >> 1] & 0xffff0000u) : ((uint32_t)v[e >> 1] << 16));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sums[rg][cc * 8 + e] = s[e];
+  __syncthreads();
+  const int c = threadIdx.x % COLS, part = threadIdx.x / COLS;
+  float t = sums[part * (kGroups / kParts)][c];
+#pragma unroll
+  for (int k = 1; k < kGroups / kParts; ++k) t += sums[part * (kGroups / kParts) + k][c];
+  parts[part][c] = t;
+  __syncthreads();
+  if (part > 0 || c0 + c >= C) return;
+#pragma unroll
+  for (int k = 1; k < kParts; ++k) t += parts[k][c];
+  out[c0 + c] = (uint16_t)bf16_rne_bits(t);
 }
 
 // bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
@@ -1175,7 +1209,7 @@ static int64_t col_sum_slabs(int64_t R, int64_t C, int64_t *slab) {
   const int64_t cols = (C + kSumCols - 1) / kSumCols;
   int64_t n = (4 * (int64_t)num_cus() + cols - 1) / cols;
   if (n > (R + 127) / 128) n = (R + 127) / 128;
-  if (n < 1 || R <= kSumOneSlab) n = 1;
+  if (n < 1 || R <= kSumWhole) n = 1;
   *slab = (R + n - 1) / n;
   return *slab > 0 ? (R + *slab - 1) / *slab : 1;
 }
@@ -1197,14 +1231,15 @@ extern "C" int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void
   int64_t slab;
   const int64_t n = col_sum_slabs(R, C, &slab);
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid((unsigned)((C + kSumCols - 1) / kSumCols), (unsigned)n);
-  if (n == 1) {
-    hipLaunchKernelGGL(col_sum_kernel<512>, grid, dim3(512), 0, st, (const uint16_t *)x, R, (int)C, ldx, slab, nullptr, (uint16_t *)out);
+  if (R <= kSumWhole) {
+    hipLaunchKernelGGL(col_sum_whole_kernel, dim3((unsigned)((C + kWholeCols - 1) / kWholeCols)), dim3(1024), 0, st, (const uint16_t *)x, R, (int)C, ldx, (uint16_t *)out);
     L8_HIP(hipGetLastError());
     return L8_OK;
   }
-  hipLaunchKernelGGL(col_sum_kernel<256>, grid, dim3(256), 0, st, (const uint16_t *)x, R, (int)C, ldx, slab, (float *)workspace, nullptr);
+  hipLaunchKernelGGL(col_sum_kernel, dim3((unsigned)((C + kSumCols - 1) / kSumCols), (unsigned)n), dim3(kSumThreads), 0, st, (const uint16_t *)x, R, (int)C, ldx,
+                     slab, (float *)workspace, n == 1 ? (uint16_t *)out : nullptr);
   L8_HIP(hipGetLastError());
+  if (n == 1) return L8_OK;
   hipLaunchKernelGGL(col_sum_fold_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, (const float *)workspace, (int)n, (int)C, (uint16_t *)out);
   L8_HIP(hipGetLastError());
   return L8_OK;

@@ -707,3 +707,10 @@ def test_amax_reduce_edges(n, offset):
         v[at] = value
         got = ops.amax_reduce(v.cuda()[offset:])
         assert torch.equal(got.cpu().reshape(()), v[offset:].abs().max()) or (value != value and bool(got.isnan()))
+
+
+@pytest.mark.parametrize("R,C", [(255, 32), (256, 40), (257, 24), (2047, 264), (2048, 40), (2049, 40), (2100, 264)])
+def test_column_sums_around_the_one_launch(R, C):
+    """Rows around one per thread and around the last that one launch takes, columns that end inside a workgroup's 32."""
+    test_column_sums(R, C, False)
+    test_column_sums(R, C, True)
