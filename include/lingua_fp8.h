@@ -438,6 +438,8 @@ typedef struct {
   void *stream;
 } l8_linear_bwd_casts_args;
 int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *args);
+/* The same, and l8_col_sum of g into bias_grad (bf16 [N], or NULL: not wanted). */
+int l8_linear_bwd_casts_bias(const l8_linear_bwd_casts_args *args, void *bias_grad);
 /* Host arithmetic only. */
 int l8_linear_bwd_casts_pays(int64_t M, int64_t N, int64_t K);
 

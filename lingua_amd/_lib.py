@@ -65,6 +65,7 @@ SIGNATURES = {
     "l8_linear_fwd_rows": [ctypes.c_char_p, _i64, _i64],
     "l8_linear_fwd_rows_workspace": [ctypes.c_char_p, _i64, _i64],
     "l8_linear_bwd_casts": [ctypes.c_char_p],
+    "l8_linear_bwd_casts_bias": [ctypes.c_char_p, _p],
     "l8_linear_bwd_casts_pays": [_i64, _i64, _i64],
     "l8_gemm_algo_count": [],
     "l8_gemm_algo_name": [_int],

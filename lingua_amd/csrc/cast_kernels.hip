@@ -515,36 +515,73 @@ __global__ __launch_bounds__(256) void col_sum_fold_kernel(const float *__restri
   out[c] = (uint16_t)bf16_rne_bits(t);
 }
 
-// One launch.  Workgroups of one XCD take neighbouring columns: 64 bytes of a row are half a line.
-__global__ __launch_bounds__(1024) void col_sum_whole_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint16_t *__restrict__ out) {
-  constexpr int COLS = kWholeCols, kGroups = 1024 / (COLS / 8), kParts = 1024 / COLS;
-  __shared__ float sums[kGroups][COLS + 1];
-  __shared__ float parts[kParts][COLS];
-  const int n = gridDim.x, xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
+// Sums of all rows of COLS columns by one workgroup, the same bits for every number of threads and columns: row r belongs to group
+// r % 256, eight groups to a part.  Workgroup `block` of n; those of one XCD take neighbouring columns (64 bytes of a row are
+// half a line).
+constexpr int kWholeGroups = 256, kWholeParts = kWholeGroups / 8;
+template <int THREADS, int COLS>
+struct WholeSums {
+  float groups[THREADS / (COLS / 8)][COLS + 1];
+  float parts[kWholeParts][COLS];
+};
+template <int THREADS, int COLS>
+L8_DEV void sum_columns(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint16_t *__restrict__ out, int block, int n, WholeSums<THREADS, COLS> &lds) {
+  constexpr int kLanes = COLS / 8, kHeld = THREADS / kLanes, kPasses = kWholeGroups / kHeld;  // groups of rows that the threads hold at once
+  const int t = threadIdx.x, xcd = block & 7, loc = block >> 3;
   const int c0 = ((n >> 3) * xcd + (xcd < (n & 7) ? xcd : n & 7) + loc) * COLS;
-  const int cc = threadIdx.x % (COLS / 8), rg = threadIdx.x / (COLS / 8), col = c0 + cc * 8;
-  float s[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  if (col < C) {
+  const int cc = t % kLanes, col = c0 + cc * 8;
+  float s[kPasses][8] = {};
+  if (kPasses == 1 && col < C) {
 #pragma unroll 8
-    for (int64_t r = rg; r < R; r += kGroups) {
+    for (int64_t r = t / kLanes; r < R; r += kWholeGroups) {
       const v4i v = *(const v4i *)(x + r * ldx + col);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s[e] += __uint_as_float((e & 1) ? ((uint32_t)v[e >> 1] & 0xffff0000u) : ((uint32_t)v[e >> 1] << 16));
+      for (int e = 0; e < 8; ++e) s[0][e] += __uint_as_float((e & 1) ? ((uint32_t)v[e >> 1] & 0xffff0000u) : ((uint32_t)v[e >> 1] << 16));
+    }
+  } else if (col < C) {
+    // eight rows are requested together, without branches; beyond the last one they are that one again, and count as zeros
+    constexpr int kBatch = 8 / kPasses;
+    for (int64_t r0 = t / kLanes; r0 - t / kLanes < R; r0 += kBatch * kWholeGroups) {
+      v4i v[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int64_t r = r0 + (i / kPasses) * kWholeGroups + (i % kPasses) * kHeld;
+        v[i] = *(const v4i *)(x + (r < R ? r : R - 1) * ldx + col);
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const bool in = r0 + (i / kPasses) * kWholeGroups + (i % kPasses) * kHeld < R;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const uint32_t w = in ? (uint32_t)v[i][e >> 1] : 0u;
+          s[i % kPasses][e] += __uint_as_float((e & 1) ? w & 0xffff0000u : w << 16);
+        }
+      }
     }
   }
+  const int c = t % COLS, part = t / COLS;
+  float sum = 0.0f;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) sums[rg][cc * 8 + e] = s[e];
-  __syncthreads();
-  const int c = threadIdx.x % COLS, part = threadIdx.x / COLS;
-  float t = sums[part * (kGroups / kParts)][c];
+  for (int j = 0; j < kPasses; ++j) {
+    if (j) __syncthreads();
 #pragma unroll
-  for (int k = 1; k < kGroups / kParts; ++k) t += sums[part * (kGroups / kParts) + k][c];
-  parts[part][c] = t;
+    for (int e = 0; e < 8; ++e) lds.groups[t / kLanes][cc * 8 + e] = s[j][e];
+    __syncthreads();
+    float u = lds.groups[part * 8][c];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) u += lds.groups[part * 8 + k][c];
+    lds.parts[j * (THREADS / COLS) + part][c] = u;
+    if (j == 0) sum = u;
+  }
   __syncthreads();
   if (part > 0 || c0 + c >= C) return;
 #pragma unroll
-  for (int k = 1; k < kParts; ++k) t += parts[k][c];
-  out[c0 + c] = (uint16_t)bf16_rne_bits(t);
+  for (int k = 1; k < kWholeParts; ++k) sum += lds.parts[k][c];
+  out[c0 + c] = (uint16_t)bf16_rne_bits(sum);
+}
+__global__ __launch_bounds__(1024) void col_sum_whole_kernel(const uint16_t *__restrict__ x, int64_t R, int C, int64_t ldx, uint16_t *__restrict__ out) {
+  __shared__ WholeSums<1024, kWholeCols> lds;
+  sum_columns<1024, kWholeCols>(x, R, C, ldx, out, blockIdx.x, gridDim.x, lds);
 }
 
 // bf16 amax[n] -> bf16 amax_out[1]; one workgroup of 1024 threads.
@@ -960,15 +997,34 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
 // the pass, five launches / two: M = 1021 N = K = 2048 14.4 / 10.6, 256 1024 1024 10.8 / 6.9, 1000 3008 2000 19.6 / 17.7,
 // 256 8192 1024 17.3 / 14.3; and as many calls less for the host, which such a pass waits for: forward + backward of the first,
 // with a bias, 143 -> 77.
+// The first workgroups make the bias gradient, if there is one, 16 columns each (32 on 64 workgroups were the last to finish).
+// us at M = 1021 N = K = 2048: 7.5 and a launch of 5.9 for the sums / 10.0 together.
+constexpr int kMixedCols = 16;
+struct MixedOperands {
+  TransposedOperands list;
+  const uint16_t *sum_x;
+  int64_t sum_rows, sum_ld;
+  uint16_t *sums;
+  int sum_cols, sum_blocks;
+};
 template <int TC, int TU>
-__global__ __launch_bounds__(256) void cast_transposed_mixed_kernel(const TransposedOperands list, int scale_rule) {
+__global__ __launch_bounds__(256) void cast_transposed_mixed_kernel(const MixedOperands p, int scale_rule) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  __shared__ TransposeShared<TC, TU> lds;
+  __shared__ union {
+    TransposeShared<TC, TU> cast;
+    WholeSums<256, kMixedCols> sum;
+  } shared;
+  if ((int)blockIdx.x < p.sum_blocks) {
+    sum_columns<256, kMixedCols>(p.sum_x, p.sum_rows, p.sum_cols, p.sum_ld, p.sums, blockIdx.x, p.sum_blocks, shared.sum);
+    return;
+  }
+  TransposeShared<TC, TU> &lds = shared.cast;
+  const int at = (int)blockIdx.x - p.sum_blocks;
   int which = 0;
 #pragma unroll
-  for (int i = 1; i < kMaxTransposed; ++i) which += (int)blockIdx.x >= list.op[i].first ? 1 : 0;
-  const TransposedOperand &op = list.op[which];
-  const unsigned block = blockIdx.x - (unsigned)op.first;
+  for (int i = 1; i < kMaxTransposed; ++i) which += at >= p.list.op[i].first ? 1 : 0;
+  const TransposedOperand &op = p.list.op[which];
+  const unsigned block = (unsigned)(at - op.first);
   if (op.from == AmaxFrom::kRows) transpose_tile<AmaxFrom::kRows, TC, TU>(op, block, scale_rule, lds);
   else if (op.from == AmaxFrom::kPartials) transpose_tile<AmaxFrom::kPartials, TC, TU>(op, block, scale_rule, lds);
   else transpose_tile<AmaxFrom::kColumns, TC, TU>(op, block, scale_rule, lds);
@@ -1430,7 +1486,7 @@ struct TransposedCast {
 // `n` casts of one kind (all from column amaxes, all from row amaxes, or one from a scalar) as one list of tiles; with
 // `partials` (one per cast; those with slots stand in for column amaxes) of any kinds but the scalar.
 template <int TC, int TU>
-static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st, const FoldOperand *partials = nullptr) {
+static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st, const FoldOperand *partials = nullptr, void *sums = nullptr) {
   using T = TransposeTile<TC, TU>;
   static_assert(T::kTR <= kMaxTileRows, "the row-stride limit assumes no taller tile");
   TransposedOperands list{};
@@ -1458,7 +1514,10 @@ static int launch_transposed_tile(const TransposedCast *a, int n, hipStream_t st
   };
   if constexpr (TC == 64) {
     if (partials) {
-      go(cast_transposed_mixed_kernel<TC, TU>, list);
+      MixedOperands mixed{list, (const uint16_t *)a[0].x, a[0].R, a[0].ldx, (uint16_t *)sums, (int)a[0].C, 0};
+      if (sums) mixed.sum_blocks = (int)((a[0].C + kMixedCols - 1) / kMixedCols);
+      gx += mixed.sum_blocks;
+      go(cast_transposed_mixed_kernel<TC, TU>, mixed);
       L8_HIP(hipGetLastError());
       return L8_OK;
     }
@@ -1574,7 +1633,9 @@ extern "C" int l8_cast_colwise_transposed_pad(const void *x, int64_t R, int64_t 
   return cast_colwise("l8_cast_colwise_transposed_pad", x, R, C, ldx, col_amax, q, ldq, Rp, scale, stream);
 }
 
-extern "C" int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *p) {
+extern "C" int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *p) { return l8_linear_bwd_casts_bias(p, nullptr); }
+
+extern "C" int l8_linear_bwd_casts_bias(const l8_linear_bwd_casts_args *p, void *bias_grad) {
   L8_REQUIRE(p && bwd_casts_together(p->M, p->N, p->K), "l8_linear_bwd_casts: null arguments, or a shape that l8_linear_bwd_casts_pays does not name");
   const l8_linear_bwd_casts_args &a = *p;
   hipStream_t st = (hipStream_t)a.stream;
@@ -1596,7 +1657,7 @@ extern "C" int l8_linear_bwd_casts(const l8_linear_bwd_casts_args *p) {
   }
   // (the column amaxes' place is not written: the partial maxima stay in the workspace for the casts behind)
   const int rc = launch_rowwise_any("l8_linear_bwd_casts", a.g, a.M, a.N, a.ldg, a.qg, a.ldqg, a.sg, nullptr, (float *)a.workspace, a.workspace, st);
-  return rc == L8_OK ? launch_transposed_tile<64, 1>(casts, n, st, partials) : rc;
+  return rc == L8_OK ? launch_transposed_tile<64, 1>(casts, n, st, partials, bias_grad) : rc;
 }
 
 extern "C" int l8_linear_bwd_casts_pays(int64_t M, int64_t N, int64_t K) { return bwd_casts_together(M, N, K) ? 1 : 0; }

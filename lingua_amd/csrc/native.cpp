@@ -27,7 +27,7 @@ struct Library {
 #define L8_ENTRY(name) decltype(&::name) name = nullptr;
 #define L8_ENTRIES(X)                                                                                                        \
   X(l8_last_error) X(l8_linear_fwd_rows) X(l8_linear_fwd_rows_workspace) X(l8_cast_rowwise) X(l8_cast_rowwise_workspace)               \
-  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_col_sum) X(l8_col_sum_workspace) X(l8_gemm_nt) X(l8_linear_bwd_casts) X(l8_linear_bwd_casts_pays)  \
+  X(l8_cast_tensorwise) X(l8_cast_tensorwise_t_rows) X(l8_amax_reduce) X(l8_cast_colwise_transposed_pad) X(l8_cast_transposed_many) X(l8_col_amax) X(l8_col_sum) X(l8_col_sum_workspace) X(l8_gemm_nt) X(l8_linear_bwd_casts_bias) X(l8_linear_bwd_casts_pays)  \
   X(l8_cast_rowwise_many) X(l8_cast_rowwise_cols_many) X(l8_gemm_nt_multi) X(l8_gemm_nt_sum) X(l8_rmsnorm_cast_rowwise)            \
   X(l8_rmsnorm_workspace) X(l8_rmsnorm_bwd_as) X(l8_rmsnorm_bwd_workspace) X(l8_swiglu_cast_rowwise) X(l8_swiglu_workspace)        \
   X(l8_swiglu_bwd_cast_rowwise_q) X(l8_swiglu_bwd_cast_transposed)
@@ -239,7 +239,8 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       c.workspace_bytes = lib.l8_cast_rowwise_workspace(M, N);
       const Space ws(g, c.workspace_bytes);
       c.workspace = ws.p();
-      check(lib.l8_linear_bwd_casts(&c), "l8_linear_bwd_casts");
+      if (need_bias) gbias = at::empty({N}, o);
+      check(lib.l8_linear_bwd_casts_bias(&c, need_bias ? gbias.mutable_data_ptr() : nullptr), "l8_linear_bwd_casts");
     }
     if (need_b && !together) g_col = at::empty({N}, o.dtype(at::kFloat));
     if (need_a && !together) {
@@ -290,7 +291,7 @@ PyObject *linear_bwd(PyObject *, PyObject *const *args, Py_ssize_t n) {
       check(lib.l8_gemm_nt(qgt.const_data_ptr(), qat.const_data_ptr(), N, K, padded, qgt.stride(0), qat.stride(0), sgt.const_data_ptr<float>(), L8_SCALE_ROW,
                            sat.const_data_ptr<float>(), L8_SCALE_ROW, nullptr, gb.mutable_data_ptr(), K, algo, stream), "l8_gemm_nt");
     }
-    if (need_bias) {
+    if (need_bias && !together) {
       gbias = at::empty({N}, o);
       const int64_t ws_bytes = lib.l8_col_sum_workspace(M, N);
       const Space ws(g, ws_bytes);

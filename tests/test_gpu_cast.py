@@ -714,3 +714,29 @@ def test_column_sums_around_the_one_launch(R, C):
     """Rows around one per thread and around the last that one launch takes, columns that end inside a workgroup's 32."""
     test_column_sums(R, C, False)
     test_column_sums(R, C, True)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (63, 32, 128), (65, 40, 48), (257, 72, 64), (1021, 2048, 2048), (1024, 264, 2048)])
+def test_bias_gradient_beside_the_casts_of_a_backward_pass(M, N, K):
+    """l8_linear_bwd_casts_bias: the bits of l8_col_sum, rows around one per thread and columns that end inside a workgroup's,
+    and the casts' bits with and without it."""
+    import struct
+    from lingua_amd import _lib, ops
+    lib = _lib.load()
+    g, a, w = (seeded_bf16((r, c + 8), std=s, seed=r + c).cuda()[:, :c] for r, c, s in ((M, N, 1e-2), (M, K, 1.0), (N, K, 0.02)))
+    Mp, need = (M + 15) // 16 * 16, lib.l8_cast_rowwise_workspace(M, N)
+    a_col, amax_w = ops.col_amax(a), ops.cast_rowwise(w)[2]
+    results = []
+    for wanted in (False, True):
+        q = [torch.full((r, c), 0x55, dtype=torch.uint8, device="cuda") for r, c in ((M, N), (N, Mp), (K, Mp), (K, N))]
+        s = [torch.zeros(n, device="cuda") for n in (M, N, K, 1)]
+        ws = torch.empty(need + 16, dtype=torch.uint8, device="cuda")
+        sums = torch.full((N,), 7.0, dtype=torch.bfloat16, device="cuda")
+        args = [g.data_ptr(), M, N, g.stride(0), q[0].data_ptr(), N, s[0].data_ptr(), q[1].data_ptr(), Mp, s[1].data_ptr(), Mp,
+                a.data_ptr(), K, a.stride(0), a_col.data_ptr(), q[2].data_ptr(), Mp, s[2].data_ptr(),
+                w.data_ptr(), w.stride(0), amax_w.data_ptr(), q[3].data_ptr(), N, s[3].data_ptr(),
+                ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream]
+        _lib.check(lib.l8_linear_bwd_casts_bias(struct.pack("27q", *args), sums.data_ptr() if wanted else None), "l8_linear_bwd_casts_bias")
+        assert torch.equal(sums, ops.col_sum(g) if wanted else torch.full_like(sums, 7.0))
+        results.append(q + s)
+    assert all(torch.equal(x, y) for x, y in zip(*results))
