@@ -775,18 +775,19 @@ template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MU
 __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // one wave per SIMD, 128x128 per wave (the least LDS traffic per flop) or, in a half tile, 64x128
-  static_assert((BM == 256 && BN == 256) || (BM == 256 && BN == 128) || (BM == 128 && BN == 256), "whole or half tiles");
+  static_assert(((BM == 256 || BM == 192) && BN == 256) || (BM == 256 && BN == 128) || (BM == 128 && BN == 256), "whole, three-quarter or half tiles");
   constexpr bool HALF_TILE = BM * BN == 32768;
-  static_assert(!SK || !HALF_TILE, "the shared-K exchange is written for whole tiles");
-  static_assert(!SUM || !(HAS_BIAS || SK || ADD || MULTI || HALF_TILE), "a sum of products is a kernel of its own");
-  constexpr int BK = 128, NW = 4, TM = HALF_TILE ? 4 : 8, TN = 8, WN = BN / 128;
+  static_assert(!SK || (BM == 256 && !HALF_TILE), "the shared-K exchange is written for whole tiles");
+  static_assert(!(SUM || MULTI) || (BM == 256 && !HALF_TILE), "lists and sums of products are made of whole tiles");
+  static_assert(!SUM || !(HAS_BIAS || SK || ADD || MULTI), "a sum of products is a kernel of its own");
+  constexpr int BK = 128, NW = 4, TM = HALF_TILE ? 4 : BM / 32, TN = 8, WN = BN / 128;
   constexpr int WROWS = TM * 16;  // rows of the tile per wave
   constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;                // the panels of one K tile
   constexpr int NLA = BM / 8 / NW, NLB = BN / 8 / NW;                // 1 KiB wave loads (8 rows x 128 B) per panel per wave
   // The LDS ring.  Whole tiles: five slots of one panel, 2.5 K tiles; panels are requested four ahead.  Half tiles: three
   // slots of one K tile; five ahead.  A trip requests one panel before its barrier (into the slot that the barrier before
   // released) and one behind it (into the slot that this K tile's A panel just left).
-  constexpr int R = HALF_TILE ? 3 : 5, UNIT = HALF_TILE ? A_BYTES + B_BYTES : A_BYTES;
+  constexpr int R = HALF_TILE ? 3 : 5, UNIT = HALF_TILE ? A_BYTES + B_BYTES : B_BYTES;  // (A_BYTES <= B_BYTES)
   constexpr int AHEAD = HALF_TILE ? 5 : 4;
   constexpr bool U1_IS_B = AHEAD % 2 != 0;                           // the panel requested before the barrier
   constexpr int NL1 = U1_IS_B ? NLB : NLA, NL2 = U1_IS_B ? NLA : NLB;
@@ -1324,7 +1325,7 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   constexpr int A_EARLY = 2;                       // A fragments read in the trip before
   constexpr int N_RD1 = 2 * (TM - A_EARLY), N_RD2 = 2 * (TN + A_EARLY);
   // groups over which the reads before and behind the barrier are spread
-  constexpr int RD1_GROUPS = HALF_TILE ? BAR - 4 : L8_READ_GROUPS1, RD2_GROUPS = HALF_TILE ? REST - 2 : L8_READ_GROUPS2;
+  constexpr int RD1_GROUPS = HALF_TILE ? BAR - 4 : L8_READ_GROUPS1 * TM / 8, RD2_GROUPS = HALF_TILE ? REST - 2 : L8_READ_GROUPS2 * TM / 8;
   static_assert(RD1_GROUPS <= BAR - 4 && RD2_GROUPS <= REST, "reads before the barrier land before it");
   v8i af[TM], bf0[TN], bf1[TN];
   uint32_t ad[4];
@@ -1636,6 +1637,9 @@ static const Algo kAlgos[] = {
      gemm_nt_stream_kernel<4, true, false, false, false, 256, 128>, gemm_nt_stream_kernel<4, false, false, true, false, 256, 128>, nullptr},
     {"stream_mt2x2w_2x4t_r3_g8", gemm_nt_stream_kernel<8, false, false, false, false, 128, 256>, 128, 256, 256, 3 * 384 * 128, true,
      gemm_nt_stream_kernel<8, true, false, false, false, 128, 256>, gemm_nt_stream_kernel<8, false, false, true, false, 128, 256>, nullptr},
+    /* 25: algo 12 on three quarters of a tile, for problems that leave whole ones' last round nearly empty */
+    {"stream_mt2x2w_3x4t_r5_g4", gemm_nt_stream_kernel<4, false, false, false, false, 192, 256>, 192, 256, 256, 5 * 256 * 128, true,
+     gemm_nt_stream_kernel<4, true, false, false, false, 192, 256>, gemm_nt_stream_kernel<4, false, false, true, false, 192, 256>, nullptr},
 };
 constexpr int kNumAlgos = sizeof(kAlgos) / sizeof(kAlgos[0]);
 
@@ -1656,7 +1660,7 @@ static int pick_plain_big(int64_t K) { return K >= 4096 ? 5 : 3; }
 // 9/16 of the units have a 256 x 256 tile
 static bool fills_with_big_tiles(int64_t M, int64_t N) { return ((M + 255) / 256) * ((N + 255) / 256) * 16 >= (int64_t)num_cus() * 9; }
 
-static int pick_algo(int64_t M, int64_t N, int64_t K) {
+static int pick_algo(int64_t M, int64_t N, int64_t K, bool three_quarters = true) {
   if (M <= 8) return kSkinnyAlgo;  // whatever the chip: the smallest calls do not pay for asking
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
@@ -1705,6 +1709,17 @@ static int pick_algo(int64_t M, int64_t N, int64_t K) {
   auto rounds = [&](int64_t t) { return (t + cus - 1) / cus; };
   const int64_t whole = rounds(tiles(256, 256)), tall = rounds(tiles(256, 128)), wide2 = rounds(tiles(128, 256));
   const int64_t half = wide2 < tall ? wide2 : tall;
+  // Three quarters of a tile (192 x 256) where whole ones would leave more than that of their rounds idle: where they need no
+  // more rounds, each of 0.87 .. 0.93 of the time (a K tile is 1536 cycles of matrix instructions instead of 2048, its loads
+  // and the C tile's conversion shrink less), and half tiles not so few that they are ahead.  A round more is never made up
+  // for.  us, whole / half / three quarters: [3000,3600] K = 512 13.7 / - / 11.9, 4096 42.0 / 46.9 / 36.8, 11008 106 / - / 100,
+  // [2800,5120].[3072,5120] 46.5 / - / 40.6, [180,2048].[65536,2048] 36.9 / - / 32.4, [520,1024].[16384,1024] 15.7 / - / 12.9,
+  // [1801,2912].[11040,2912] 65.4 / 67.8 / 56.8, [1676,4128].[9360,4128] 91 / 97 / 82, [4800,9216].[4864,9216] 172 / 173 / 161,
+  // [12288,1024].[2048,1024] 30.3 / 28.5 / 27.2, [5000,4096].[6656,4096] - / 121 / 107; but [3290,1392].[3904,1392] (two rounds
+  // against one) 21.2 / - / 30.3, [4093,4096].[14336,4096] (five against four) 168 / 184 / 176, [300,4096].[36864,4096] (two
+  // rounds of half tiles) - / 59.6 / 76.6, [3115,2752].[2336,2752] (one) 30.4 / 23.3 / 24.8.
+  const int64_t quarters = rounds(tiles(192, 256));
+  if (three_quarters && big && quarters <= whole && half * 5 > quarters * 7) return 25;
   if (half * 2 <= whole * 3 || (K <= 4096 && half * 3 <= whole * 5) || (K <= 2048 && half * 4 <= whole * 7)) return wide2 < tall ? 24 : 23;
   return 12;
 }
@@ -1986,7 +2001,7 @@ static bool sum_in_one(const l8_gemm_term *terms, int64_t n, int64_t M, int64_t 
       return false;
     K += t.K;
   }
-  return K < n * 8192 && ((M + 255) / 256) * ((N + 255) / 256) < (1LL << 31) && pick_algo(M, N, K) == 12;
+  return K < n * 8192 && ((M + 255) / 256) * ((N + 255) / 256) < (1LL << 31) && pick_algo(M, N, K, false) == 12;
 }
 
 extern "C" int l8_gemm_nt_sum(const l8_gemm_term *terms, int64_t n, int64_t M, int64_t N, void *C, int64_t ldc, int algo, void *stream) {

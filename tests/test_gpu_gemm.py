@@ -567,3 +567,26 @@ def test_two_tiles_of_weight_rows_per_workgroup(M, extra, K, mode):
     if mode == "plain":   # products of integers up to 8 add up exactly in fp32
         want = qa.double() @ qb.double().t() * sa.double() * sb.double().t()
         assert bool(((y.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2.0 ** -20)).all())
+
+
+@pytest.mark.parametrize("K", [16, 128, 144, 256, 400, 1152])
+@pytest.mark.parametrize("with_bias,scalar", [(False, False), (False, True), (True, False)])
+def test_three_quarter_tiles_carry_their_fragments(K, with_bias, scalar):
+    """Tiles of 192 rows (22 x 17 of them here, the last row of tiles short): one to nine K tiles, one or two tiles per workgroup."""
+    test_persistent_kernel_carries_its_fragments_from_tile_to_tile(25, K, with_bias, scalar)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 16), (95, 256, 128), (97, 264, 144), (192, 128, 4096), (193, 520, 272), (575, 1000, 528)])
+def test_three_quarter_tiles_at_their_edges(M, N, K):
+    """Rows around a wave's 96 and a tile's 192, columns off 256, a C with rows apart, and a sum added to C: exact integers."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(M + N)
+    A, B = (torch.randint(-1, 2, (n, K), generator=g).float() for n in (M, N))
+    sa = torch.tensor([2.0 ** (i % 5 - 2) for i in range(M)]).reshape(M, 1)
+    sb = torch.tensor([2.0 ** (i % 3) for i in range(N)]).reshape(N, 1)
+    want = ((A.double() @ B.double().t()) * sa.double() * sb.double().t()).to(torch.bfloat16)
+    for add in (False, True):
+        wide = torch.full((M, N + 8), 1.0, dtype=torch.bfloat16, device="cuda")
+        ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa.cuda(), sb.cuda(), algo=25, out=wide[:, :N], add=add)
+        assert torch.equal(wide[:, :N].cpu(), (want.float() + 1.0).to(torch.bfloat16) if add else want)
+        assert bool((wide[:, N:] == 1.0).all())
