@@ -778,7 +778,7 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   static_assert(((BM == 256 || BM == 192) && BN == 256) || (BM == 256 && BN == 128) || (BM == 128 && BN == 256), "whole, three-quarter or half tiles");
   constexpr bool HALF_TILE = BM * BN == 32768;
   static_assert(!SK || (BM == 256 && !HALF_TILE), "the shared-K exchange is written for whole tiles");
-  static_assert(!(SUM || MULTI) || (BM == 256 && !HALF_TILE), "lists and sums of products are made of whole tiles");
+  static_assert(!(SUM || MULTI) || !HALF_TILE, "lists and sums of products are made of whole or three-quarter tiles");
   static_assert(!SUM || !(HAS_BIAS || SK || ADD || MULTI), "a sum of products is a kernel of its own");
   constexpr int BK = 128, NW = 4, TM = HALF_TILE ? 4 : BM / 32, TN = 8, WN = BN / 128;
   constexpr int WROWS = TM * 16;  // rows of the tile per wave
@@ -1602,6 +1602,8 @@ template __global__ void gemm_nt_stream_kernel<4, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, false, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<4, false, false, false, false, 256, 256, true>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, false, true, 192, 256>(const GemmArgs);
+template __global__ void gemm_nt_stream_kernel<4, false, false, false, false, 192, 256, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, false>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<2, true>(const GemmArgs);
 template __global__ void gemm_nt_stream_kernel<16, false>(const GemmArgs);
@@ -1926,6 +1928,17 @@ extern "C" int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t 
   return tiles * 32 >= (int64_t)num_cus() * (K > 4096 ? 13 : 12);
 }
 
+// Rows of the list's tiles: three quarters of a whole one by the rule of single products (pick_algo).
+static int64_t multi_tile_rows(const l8_gemm_part *parts, int64_t n, int64_t N) {
+  const int64_t cus = num_cus();
+  int64_t whole = 0, quarters = 0;
+  for (int64_t i = 0; i < n; ++i) {
+    whole += (parts[i].M + 255) / 256 * ((N + 255) / 256);
+    quarters += (parts[i].M + 191) / 192 * ((N + 255) / 256);
+  }
+  return whole * 16 >= cus * 9 && (quarters + cus - 1) / cus <= (whole + cus - 1) / cus ? 192 : 256;
+}
+
 extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_t N, int64_t K, int64_t lda, int64_t ldb,
                                 const float *sb, int sb_mode, int64_t ldc, int algo, void *stream) {
   L8_REQUIRE(n >= 0 && (n == 0 || parts), "l8_gemm_nt_multi: null list or negative count");
@@ -1949,7 +1962,10 @@ extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void
     return L8_OK;
   }
   constexpr int kLds = 5 * 256 * 128;
-  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, false, true>;
+  const int64_t bm = multi_tile_rows(parts, n, N);
+  const gemm_fn fn = bm == 256 ? gemm_nt_stream_kernel<4, false, false, false, true> : gemm_nt_stream_kernel<4, false, false, false, true, 192, 256>;
+  tile_rows = 0;
+  for (int64_t i = 0; i < n; ++i) tile_rows += (parts[i].M + bm - 1) / bm;
   GemmArgs p{};
   p.A = (const uint8_t *)parts[0].A;
   p.B = (const uint8_t *)B;
@@ -1968,15 +1984,15 @@ extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void
   p.tiles_n = (int)((N + 255) / 256);
   int64_t first = 0;
   for (int i = 0; i < 2; ++i) {
-    first += (parts[i].M + 255) / 256 * 256;
+    first += (parts[i].M + bm - 1) / bm * bm;
     if (i + 1 < n) p.part[i] = {(const uint8_t *)parts[i + 1].A, parts[i + 1].sa, (uint16_t *)parts[i + 1].C, (int)first, (int)parts[i + 1].M};
     else p.part[i] = {p.A, p.sa, p.C, 0x7fffffff, p.M};
   }
-  static std::atomic<bool> attr_done[kMaxDev] = {};  // idempotent; a race only repeats the call
+  static std::atomic<bool> attr_done[2][kMaxDev] = {};  // idempotent; a race only repeats the call
   const int slot = device_slot();
-  if (slot < 0 || !attr_done[slot]) {
+  if (slot < 0 || !attr_done[bm == 256][slot]) {
     L8_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
-    if (slot >= 0) attr_done[slot] = true;
+    if (slot >= 0) attr_done[bm == 256][slot] = true;
   }
   hipLaunchKernelGGL(fn, dim3((unsigned)persistent_grid((int64_t)p.tiles_m * p.tiles_n)), dim3(256), kLds, (hipStream_t)stream, p);
   L8_HIP(hipGetLastError());
@@ -2015,7 +2031,10 @@ extern "C" int l8_gemm_nt_sum(const l8_gemm_term *terms, int64_t n, int64_t M, i
     return L8_OK;
   }
   constexpr int kLds = 5 * 256 * 128;
-  const gemm_fn fn = gemm_nt_stream_kernel<4, false, false, false, false, 256, 256, true>;
+  int64_t K = 0;
+  for (int64_t i = 0; i < n; ++i) K += terms[i].K;
+  const int64_t bm = pick_algo(M, N, K) == 25 ? 192 : 256;
+  const gemm_fn fn = bm == 256 ? gemm_nt_stream_kernel<4, false, false, false, false, 256, 256, true> : gemm_nt_stream_kernel<4, false, false, false, false, 192, 256, true>;
   GemmArgs p{};
   p.A = (const uint8_t *)terms[0].A;
   p.B = (const uint8_t *)terms[0].B;
@@ -2029,18 +2048,18 @@ extern "C" int l8_gemm_nt_sum(const l8_gemm_term *terms, int64_t n, int64_t M, i
   p.sb = terms[0].sb;
   p.sa_row = 1;
   p.C = (uint16_t *)C;
-  p.tiles_m = (int)((M + 255) / 256);
+  p.tiles_m = (int)((M + bm - 1) / bm);
   p.tiles_n = (int)((N + 255) / 256);
   p.terms = (int)n - 1;
   for (int i = 0; i < 2; ++i) {
     const l8_gemm_term &t = terms[i + 1 < n ? i + 1 : 0];
     p.term[i] = {(const uint8_t *)t.A, (const uint8_t *)t.B, t.sa, t.sb, t.lda, t.ldb, (int)t.K};
   }
-  static std::atomic<bool> attr_done[kMaxDev] = {};  // idempotent; a race only repeats the call
+  static std::atomic<bool> attr_done[2][kMaxDev] = {};  // idempotent; a race only repeats the call
   const int slot = device_slot();
-  if (slot < 0 || !attr_done[slot]) {
+  if (slot < 0 || !attr_done[bm == 256][slot]) {
     L8_HIP(hipFuncSetAttribute((const void *)fn, hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
-    if (slot >= 0) attr_done[slot] = true;
+    if (slot >= 0) attr_done[bm == 256][slot] = true;
   }
   hipLaunchKernelGGL(fn, dim3((unsigned)persistent_grid((int64_t)p.tiles_m * p.tiles_n)), dim3(256), kLds, (hipStream_t)stream, p);
   L8_HIP(hipGetLastError());

@@ -590,3 +590,37 @@ def test_three_quarter_tiles_at_their_edges(M, N, K):
         ops.gemm_nt(fp8(A).cuda(), fp8(B).cuda(), sa.cuda(), sb.cuda(), algo=25, out=wide[:, :N], add=add)
         assert torch.equal(wide[:, :N].cpu(), (want.float() + 1.0).to(torch.bfloat16) if add else want)
         assert bool((wide[:, N:] == 1.0).all())
+
+
+@pytest.mark.parametrize("Ks", [(512, 512), (528, 1152, 656)])
+def test_sum_of_products_on_three_quarter_tiles(Ks):
+    """As on whole tiles: exact sums, one rounding, whichever product's scale they are counted in."""
+    from lingua_amd import _lib, ops
+    M, N = 2990, 3592
+    assert _lib.load().l8_gemm_pick(M, N, sum(Ks)) == 25
+    g = torch.Generator().manual_seed(len(Ks))
+    terms, want = [], 0
+    for i, K in enumerate(Ks):
+        A, B = (torch.randint(-1, 2, (n, K), generator=g).float().cuda() for n in (M, N))
+        sa = torch.tensor([2.0 ** ((r * (i + 3)) % 5 - 2) for r in range(M)]).reshape(M, 1).cuda()
+        sb = torch.tensor([[2.0 ** (1 - i)]]).cuda()
+        want = want + (A.double() @ B.double().t()) * sa.double() * sb.double()
+        terms.append((fp8(A), fp8(B), sa, sb))
+    got = ops.gemm_nt_sum(*zip(*terms))
+    assert torch.equal(got.view(torch.int16), want.float().to(torch.bfloat16).view(torch.int16))
+
+
+@pytest.mark.parametrize("K", [16, 272, 1152])
+@pytest.mark.parametrize("rows", [(2000, 500, 500), (1930, 960), (200, 2400, 390)])
+def test_list_of_products_on_three_quarter_tiles(rows, K):
+    """Products with one B whose tiles of 192 rows start where the one before ends, the last tile of each short; exact integers."""
+    from lingua_amd import ops
+    N = 3600
+    g = torch.Generator().manual_seed(K)
+    B = torch.randint(-1, 2, (N, K), generator=g).float().cuda()
+    sb = torch.tensor([2.0 ** (i % 3) for i in range(N)]).reshape(N, 1).cuda()
+    As = [torch.randint(-1, 2, (m, K), generator=g).float().cuda() for m in rows]
+    sas = [torch.tensor([2.0 ** (i % 5 - 2) for i in range(m)]).reshape(m, 1).cuda() for m in rows]
+    got = ops.gemm_nt_multi([fp8(A) for A in As], fp8(B), sas, sb)
+    for A, sa, y in zip(As, sas, got):
+        assert torch.equal(y, ((A.double() @ B.double().t()) * sa.double() * sb.double().t()).to(torch.bfloat16))
