@@ -740,3 +740,21 @@ def test_bias_gradient_beside_the_casts_of_a_backward_pass(M, N, K):
         assert torch.equal(sums, ops.col_sum(g) if wanted else torch.full_like(sums, 7.0))
         results.append(q + s)
     assert all(torch.equal(x, y) for x, y in zip(*results))
+
+
+@pytest.mark.parametrize("C", [512, 520, 1024, 2048, 2056, 4096, 4104])
+@pytest.mark.parametrize("R", [1, 3, 512, 513])
+def test_few_rows_have_the_bits_of_many(R, C):
+    """The kernels for up to 512 rows and for more, around the widths where the loads per lane change, with and without the
+    bytes: the rows of a small cast are those of a large one."""
+    from lingua_amd import ops
+    x = seeded_bf16((600, C + 8), std=1.0, seed=C).cuda()[:, :C]
+    x[R - 1, C - 1], x[0, 0] = float("inf"), 300.0
+    if R > 2:
+        x[1, C // 2] = float("nan")
+        x[2] = 0.0
+    q0, s0, a0 = ops.cast_rowwise(x)
+    q, s, a = ops.cast_rowwise(x[:R])
+    assert torch.equal(q.view(torch.uint8), q0.view(torch.uint8)[:R])
+    assert bits_equal(s.cpu(), s0[:R].cpu()) and bits_equal(a.cpu(), a0[:R].cpu())
+    assert bits_equal(ops.cast_rowwise(x[:R], want_q=False)[2].cpu(), a.cpu())
