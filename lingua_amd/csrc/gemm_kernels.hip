@@ -1798,6 +1798,8 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
   L8_REQUIRE(algo >= 0 && algo <= kNumAlgos, "l8_gemm_nt: algo %d out of range 0..%d", algo, kNumAlgos);
   const bool chosen = algo == 0;
   if (chosen) algo = pick_algo(M, N, K);
+  // (rows so far apart that whole tiles are refused below are refused, not served by the shorter ones)
+  if (chosen && algo == 25 && 256 * lda + K >= (1LL << 31)) algo = pick_algo(M, N, K, false);
   // Rows so far apart that 256 of them pass the 32-bit offsets below: a problem of middling size, which taller tiles would
   // only serve faster, takes 128 x 128 ones and is refused where 128 rows are too many.
   if (chosen && kAlgos[algo - 1].persistent && !fills_with_big_tiles(M, N) && (256 * lda + K >= (1LL << 31) || 256 * ldb + K >= (1LL << 31)))
@@ -1812,7 +1814,10 @@ static int gemm_nt_impl(const void *A, const void *B, int64_t M, int64_t N, int6
                     (sb_mode != L8_SCALE_ROW || ((uintptr_t)sb % 16) == 0) &&
                     (bias == nullptr || (((uintptr_t)bias % 8) == 0 && kAlgos[algo - 1].fn_bias != nullptr)) &&
                     (!add || kAlgos[algo - 1].fn_add != nullptr);
-    if (!ok) algo = kAlgos[algo - 1].bm * kAlgos[algo - 1].bn < 256 * 256 ? 2 : pick_plain_big(K);
+    if (!ok) {
+      if (algo == 25) algo = chosen ? pick_algo(M, N, K, false) : 12;
+      algo = kAlgos[algo - 1].bm * kAlgos[algo - 1].bn < 256 * 256 ? 2 : pick_plain_big(K);
+    }
   }
   if (algo == kSkinnyAlgo) {
     if (skinny_serves(M, N, K, lda, ldb, 1))

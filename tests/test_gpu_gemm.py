@@ -624,3 +624,16 @@ def test_list_of_products_on_three_quarter_tiles(rows, K):
     got = ops.gemm_nt_multi([fp8(A) for A in As], fp8(B), sas, sb)
     for A, sa, y in zip(As, sas, got):
         assert torch.equal(y, ((A.double() @ B.double().t()) * sa.double() * sb.double().t()).to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("algo", [0, 25])
+def test_outputs_that_three_quarter_tiles_cannot_store(algo):
+    """N off 8 columns, and a C whose rows start off 16 bytes: computed by the plain kernel.  Exact integers."""
+    from lingua_amd import ops
+    g = torch.Generator().manual_seed(9)
+    for M, N, pad in ((2990, 3593, 0), (2990, 3592, 4)):
+        A, B = (torch.randint(-1, 2, (n, 144), generator=g).float().cuda() for n in (M, N))
+        one = torch.ones(1, 1, device="cuda")
+        wide = torch.zeros((M, N + pad), dtype=torch.bfloat16, device="cuda")
+        ops.gemm_nt(fp8(A), fp8(B), one, one, algo=algo, out=wide[:, :N])
+        assert torch.equal(wide[:, :N].float(), A @ B.t()) and not bool(wide[:, N:].any())

@@ -539,3 +539,15 @@ def test_a_named_library_that_is_not_there_fails_loudly():
     env = dict(os.environ, LINGUA_FP8_LIB="/nonexistent/libl8_variant.so", PYTHONPATH=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     out = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=120)
     assert "RuntimeError" in out.stdout and "/nonexistent/libl8_variant.so" in out.stdout, out.stdout + out.stderr
+
+
+def test_rows_too_far_apart_for_whole_tiles_stay_refused():
+    """256 rows 8 MiB apart pass the 32-bit offsets of a tile; 192 do not, but a large problem is refused whichever of the two its
+    size chooses (host checks only: nothing is enqueued)."""
+    lib = _lib.load()
+    fake, far = 1 << 20, 1 << 23
+    if not torch.cuda.is_available():
+        assert lib.l8_gemm_pick(3000, 3600, 4096) == 25
+    for M, N in ((3000, 3600), (4096, 4096)):
+        assert lib.l8_gemm_nt(fake, fake, M, N, 4096, far, 4096, fake, 1, fake, 1, None, fake, N, 0, None) == -1
+        assert "leading dimension" in _lib.last_error()
