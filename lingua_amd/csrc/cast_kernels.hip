@@ -1316,8 +1316,9 @@ extern "C" int l8_col_sum(const void *x, int64_t R, int64_t C, int64_t ldx, void
   return L8_OK;
 }
 
+// (C % 8: a chunk across column C would reach the next workgroup's partial row)
 static bool group_serves(const l8_cast_rowwise_cols_item &t, int64_t C) {
-  return t.C == C && many_serves(l8_cast_rowwise_item{t.x, t.R, t.ldx, t.q, t.ldq, t.scale, t.amax}, C);
+  return t.C == C && C % 8 == 0 && many_serves(l8_cast_rowwise_item{t.x, t.R, t.ldx, t.q, t.ldq, t.scale, t.amax}, C);
 }
 
 int l8::cast_rowwise_pair(const l8_cast_rowwise_cols_item *two, hipStream_t st, bool *served) {

@@ -4,6 +4,7 @@ module mirror the reference interface (lingua/float8.py:134-191)."""
 import ctypes
 import os
 import re
+import struct
 import subprocess
 import sys
 
@@ -56,6 +57,19 @@ def test_argument_validation_happens_before_launch():
     assert lib.l8_cast_rowwise(fake, 64, 1024, 1024, fake, 1024, fake, None, fake, None, 0, None) == -1
     assert "workspace" in _lib.last_error()
     assert lib.l8_gemm_nt(None, None, 0, 4, 16, 16, 16, None, 1, None, 1, None, None, 4, 0, None) == 0
+
+
+def test_column_amaxes_of_several_operands_are_refused_where_those_of_one_are():
+    """Neighbours that one launch could take: a width that is no multiple of 8, pointers and strides that are.  Refused before
+    anything is enqueued: on a machine without a GPU the first launch would answer with another error."""
+    lib = _lib.load()
+    fake = 1 << 20
+    for C in (12, 2044):
+        item = (fake, 8, C, (C + 15) // 16 * 16, fake, (C + 15) // 16 * 16, fake, 0, fake, fake, 1 << 30)
+        assert lib.l8_cast_rowwise(*item, None) == -1 and "multiples of 8" in _lib.last_error()
+        for n in (1, 2, 3):
+            assert lib.l8_cast_rowwise_cols_many(struct.pack(f"{11 * n}q", *item * n), n, None) == -1
+            assert f"C={C}" in _lib.last_error() and "multiples of 8" in _lib.last_error()
 
 
 def test_linear_call_validates_its_arguments_on_the_host():
