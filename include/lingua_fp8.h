@@ -353,8 +353,9 @@ int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t 
 
 /* C [M,N] = bf16(sum over i of A_i [M,K_i] . B_i [N,K_i]^T * sa_i * sb_i): the gradient of an activation that several linears
  * read (lingua/float8.py:119 once per linear, added up by autograd).  sa_i fp32 [M], sb_i one fp32.  Two or three products
- * that 256 x 256 tiles serve, none shorter than 512 and shorter than 8192 on average, run as one whose sum is rounded once;
- * else as l8_gemm_nt of the first and l8_gemm_nt_add of the others, rounded per product. */
+ * that 256 x 256 tiles serve, none shorter than 512 and shorter than 8192 on average, run as one whose sum is rounded once,
+ * but for rows whose finite scales sa_i * sb_i lie more than 2^90 apart or beyond the normal fp32 numbers; these, and all rows
+ * else, as l8_gemm_nt of the first and l8_gemm_nt_add of the others, rounded per product. */
 typedef struct {
   const void *A, *B;
   int64_t K, lda, ldb;

@@ -771,6 +771,82 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
 // they are multiplied by the quotient of the old one and the new, row by row, under the matrix instructions of the new
 // product's first K tile (768 vector instructions beside its 64: 2.5 us per change of two rounds of tiles).  C is rounded and
 // written once, where ADD reads it back and rounds it per product.
+//
+// A sum of products is below 2^33 units and no finer than 2^-18, so units within 2^90 of one another keep what the
+// accumulators hold between 2^-108 and 2^125, however often they are rescaled.  A row whose units lie further apart (or beyond
+// fp32's normal numbers) would overflow on the way or lose a product that is alone in its column: such rows are computed
+// again behind the loop, product by product, each rounded and added as l8_gemm_nt_add does: there no accumulators are live
+// (a second conversion of the tile beside the first spills 250 registers).  Looking at the units costs a launch 0.3 .. 0.5 us:
+// 2 x [16384,2048] K = 512 38.1 -> 38.6, 3 x [16384,2048] K = 2048 140.8 -> 141.4.  (Rows with a scale that is infinite or NaN
+// stay: the casts give such a scale to rows whose every product is NaN.)
+#if defined(__HIP_DEVICE_COMPILE__)
+L8_DEV bool units_apart(float a, float b, float c) {
+  const float least = fminf(fminf(fabsf(a), fabsf(b)), fabsf(c)), largest = fmaxf(fmaxf(fabsf(a), fabsf(b)), fabsf(c));
+  return !(least >= 0x1p-126f && largest < INFINITY && largest <= least * 0x1p90f);
+}
+
+// 16 rows from m on, 128 columns from n on, of a sum of products, the rows with units far apart alone: one wave, operands
+// straight from memory.  The instruction and the order of K are those of the kernel below.
+L8_DEV void sum_rows_one_by_one(const GemmArgs &p, int m, int n) {
+  int lane = threadIdx.x & 63;
+  const int l15 = lane & 15, quad = lane >> 4;
+  const float sb[3] = {p.sb[0], p.term[0].sb[0], p.terms > 1 ? p.term[1].sb[0] : p.sb[0]};  // (two products at least)
+  float sa[4][3];
+  bool redo[4], any = false;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int row = m + 4 * quad + e;
+    const int at = row < p.M ? row : p.M - 1;
+    redo[e] = row < p.M;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      sa[e][t] = t == 0 ? p.sa[at] : t <= p.terms ? p.term[t ? t - 1 : 0].sa[at] : sa[e][0];
+      redo[e] = redo[e] && fabsf(sa[e][t]) < INFINITY && fabsf(sb[t]) < INFINITY;
+    }
+    redo[e] = redo[e] && units_apart(sa[e][0] * sb[0], sa[e][1] * sb[1], sa[e][2] * sb[2]);
+    any |= redo[e];
+  }
+  if (__ballot(any) == 0) return;
+#pragma unroll 1
+  for (int c = n; c < n + 128 && c < p.N; c += 16) {
+    v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int t = 0; t <= p.terms; ++t) {
+      const uint8_t *A = t == 0 ? p.A : p.term[t - 1].A, *B = t == 0 ? p.B : p.term[t - 1].B;
+      const int64_t lda = t == 0 ? p.lda : p.term[t - 1].lda, ldb = t == 0 ? p.ldb : p.term[t - 1].ldb;
+      const int K = t == 0 ? p.K : p.term[t - 1].K;
+      // rows at or beyond M (N) start beyond the descriptor's end and read as zeros
+      const int64_t a_left = (int64_t)(p.M - m - 1) * lda + K, b_left = (int64_t)(p.N - c - 1) * ldb + K;
+      const __amdgpu_buffer_rsrc_t rsA = make_rsrc(A + (int64_t)m * lda, a_left < 0x7fffffff ? (uint32_t)a_left : 0x7fffffffu);
+      const __amdgpu_buffer_rsrc_t rsB = make_rsrc(B + (int64_t)c * ldb, b_left < 0x7fffffff ? (uint32_t)b_left : 0x7fffffffu);
+      v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+      for (int k0 = 0; k0 < K; k0 += 128) {
+        v8i a, b;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int k = k0 + quad * 32 + h * 16;  // K is a multiple of 16
+          const v4i va = __builtin_amdgcn_raw_buffer_load_b128(rsA, k < K ? l15 * (int)lda + k : (int)kOOB, 0, 0);
+          const v4i vb = __builtin_amdgcn_raw_buffer_load_b128(rsB, k < K ? l15 * (int)ldb + k : (int)kOOB, 0, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) a[h * 4 + i] = va[i], b[h * 4 + i] = vb[i];
+        }
+        acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, acc, 0, 0, 0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float a = t == 0 ? sa[e][0] : t == 1 ? sa[e][1] : sa[e][2], b = t == 0 ? sb[0] : t == 1 ? sb[1] : sb[2];
+        const float part = (float)(__bf16)(acc[e] * (a * b));
+        sum[e] = t == 0 ? part : (float)(__bf16)(sum[e] + part);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (redo[e] && c + l15 < p.N) ((__bf16 *)p.C)[(int64_t)(m + 4 * quad + e) * p.ldc + c + l15] = (__bf16)sum[e];
+  }
+}
+#endif
+
 template <int GROUP_M, bool HAS_BIAS, bool SK = false, bool ADD = false, bool MULTI = false, int BM = 256, int BN = 256, bool SUM = false>
 __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1420,6 +1496,7 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
       for (int t = 0; t < TN; ++t) bf0[t] = bf1[t];
     }
   };
+  [[maybe_unused]] int again = 0;  // SUM: this lane has seen a row with units far apart
 #pragma unroll 1
   for (int seg = 0; seg < n_seg; ++seg) {
     [[maybe_unused]] uint64_t t_loop = 0;
@@ -1432,9 +1509,8 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
     cursor_step(cur_mul);
     if (SK && seg > 0) lane_consts();
     if constexpr (SUM) {
-      // A product's unit is the scale of its row times that of its B; all units of the tile's rows are requested here, lane l
-      // holding those of rows wm*WROWS + l and + 64 + l.  A product much finer than what it is added to (2^90, where its
-      // largest sum is below 2^-56 of the other's smallest step) is counted in units that keep the quotient finite.
+      // A product's unit is the scale of its row times that of its B; all row scales of the tile are requested here, lane l
+      // holding those of rows wm*WROWS + l and + 64 + l.
       int l = lane;
       asm volatile("" : "+v"(l));
       int bits[3][2];
@@ -1446,13 +1522,19 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
       }
       k_loop(KT, seg > 0);
       float unit[2] = {__int_as_float(bits[0][0]) * __int_as_float(sb_one), __int_as_float(bits[0][1]) * __int_as_float(sb_one)};
+      const int rows = (p.M - m0 < BM ? p.M - m0 : BM) - wm * WROWS;  // of this wave, and maybe of the one below
+#pragma unroll
+      for (int h = 0; h < (TM > 4 ? 2 : 1); ++h) {
+        int row = lane;
+        asm volatile("" : "+v"(row));
+        const float next = __int_as_float(bits[1][h]) * __int_as_float(sb_term[0]), last = __int_as_float(bits[2][h]) * __int_as_float(sb_term[1]);
+        again |= row + 64 * h < rows && units_apart(unit[h], next, p.terms > 1 ? last : next);
+      }
       auto go_on = [&](int t) __attribute__((always_inline)) {
         int quot[2];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-          const float least = unit[h] * 0x1p-90f;
-          float next = __int_as_float(bits[1][h]) * __int_as_float(t == 1 ? sb_term[0] : sb_term[1]);
-          next = next < least ? least : next;  // (a NaN stays)
+          const float next = __int_as_float(bits[1][h]) * __int_as_float(t == 1 ? sb_term[0] : sb_term[1]);
           quot[h] = __float_as_int(unit[h] / next);
           unit[h] = next;
         }
@@ -1517,6 +1599,18 @@ __global__ __launch_bounds__(256) void gemm_nt_stream_kernel(const GemmArgs p) {
   }
   // the tail requests (out of range, zero filling) must have landed before the workgroup's LDS is released
   L8_WAIT_VM_LGKM0(0);
+  if constexpr (SUM) {
+    if (__ballot(again != 0) != 0) {
+#pragma unroll 1
+      for (int seg = 0; seg < n_seg; ++seg) {
+        int m0, n0;
+        tile_at(first + loc + seg * W, m0, n0);
+#pragma unroll 1
+        for (int tm = 0; tm < TM; ++tm)
+          if (m0 + wm * WROWS + tm * 16 < p.M) sum_rows_one_by_one(p, m0 + wm * WROWS + tm * 16, n0 + wn * 128);
+      }
+    }
+  }
   if (L8_GEMM_PROF) {
     prof[2] = __builtin_amdgcn_s_memrealtime();
     prof[5] = __builtin_readcyclecounter() - prof[5];

@@ -257,6 +257,37 @@ def test_sum_of_products_whose_scales_lie_far_apart():
     assert ((got - want).abs()[fine] <= (bound + floor.expand_as(bound))[fine]).all()
 
 
+@pytest.mark.parametrize("M,N,Ks,algo", [(3590, 3592, (528, 656), 12), (3590, 3592, (528, 1040, 656), 12), (4093, 8184, (512, 528, 1152), 12), (2990, 3592, (528, 656, 784), 25)])
+def test_sum_of_products_in_rows_that_no_one_scale_serves(M, N, Ks, algo):
+    """Rows in which the products' scales fall or rise by 2^60 and more, once or twice, pass fp32's range on either side or are
+    zero or negative, columns in which the coarse product is exactly zero: such rows have the bits of the products added one by
+    one, all others those that they have without such rows beside them."""
+    from lingua_amd import _lib
+    assert _lib.load().l8_gemm_pick(M, N, sum(Ks)) == algo
+    g = torch.Generator().manual_seed(M + len(Ks))
+    qs = [tuple(random_fp8_bytes((n, K), g).cuda() for n in (M, N)) for K in Ks]
+    scales = [torch.rand(M, 1, generator=g) + 0.5 for _ in Ks]
+    plain = [s.clone() for s in scales]
+    odd = [(1e20, 1.0, 1e-25), (1.0, 2.0 ** -60, 2.0 ** -120), (2.0 ** 45, 1e-12 / 448, 1e-12 / 448 / 4096), (1e-25, 1.0, 1e20), (1e20, 1e-25, 1e20),
+           (1e-25, 1e20, 1e-25), (1e35, 1e-5, 1.0), (1e-38, 1e-38, 1e-38), (0.0, 1.0, 1.0), (1.0, 0.0, 0.0), (0.0, 0.0, 0.0), (-1e20, 1.0, 1e-25)]
+    rows = [min(i * (M // len(odd)) + 17 * (i % 4), M - 1) for i in range(len(odd) - 1)] + [M - 1]
+    for r, values in zip(rows, odd):
+        for s, v in zip(scales, values):
+            s[r] = v
+    qs[0][1][5::37] = 0  # columns in which the first product is zero, and of these every second one in which the second is
+    qs[1][1][5::74] = 0
+    qs[0][0][rows[0]] = 0
+
+    def terms(sas):
+        return [(spread(a, a.shape[1] + 32 * i), b.view(torch.float8_e4m3fn), s.cuda(), torch.tensor([[0.75 + i]]).cuda()) for i, ((a, b), s) in enumerate(zip(qs, sas))]
+    got, want, beside = sum_of_products(terms(scales)), one_by_one(terms(scales)), sum_of_products(terms(plain))
+    assert torch.equal(got[rows].view(torch.int16), want[rows].view(torch.int16))
+    assert torch.isfinite(got[rows[0]]).all()
+    got[rows] = 0
+    beside[rows] = 0
+    assert torch.equal(got.view(torch.int16), beside.view(torch.int16))
+
+
 def test_sum_of_products_that_one_loop_does_not_serve():
     """Sizes for smaller tiles, reductions too short or too long, a tile configuration asked for: added one by one, the same bits."""
     from lingua_amd import ops
