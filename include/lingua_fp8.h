@@ -350,6 +350,8 @@ int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void *B, int64_
                      const float *sb, int sb_mode, int64_t ldc, int algo, void *stream);
 /* Host arithmetic only: would l8_gemm_nt_multi launch these once (aligned operands, n = 2 or 3 assumed; reads M alone)? */
 int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t N, int64_t K);
+/* Host arithmetic only: rows of the tiles of such a launch, 256 or 192 (reads M alone). */
+int l8_gemm_multi_tile_rows(const l8_gemm_part *parts, int64_t n, int64_t N);
 
 /* C [M,N] = bf16(sum over i of A_i [M,K_i] . B_i [N,K_i]^T * sa_i * sb_i): the gradient of an activation that several linears
  * read (lingua/float8.py:119 once per linear, added up by autograd).  sa_i fp32 [M], sb_i one fp32.  Two or three products

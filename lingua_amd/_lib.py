@@ -45,6 +45,7 @@ SIGNATURES = {
     "l8_gemm_nt_multi": [_p, _i64, _p, _i64, _i64, _i64, _i64, _p, _int, _i64, _int, _p],
     "l8_gemm_nt_sum": [_p, _i64, _i64, _i64, _p, _i64, _int, _p],
     "l8_gemm_multi_pays": [_p, _i64, _i64, _i64],
+    "l8_gemm_multi_tile_rows": [_p, _i64, _i64],
     "l8_gemm_workspace": [],
     "l8_gemm_workspace_gave_up_offset": [],
     "l8_gemm_set_wait_limit": [_int],

@@ -2027,8 +2027,8 @@ extern "C" int l8_gemm_multi_pays(const l8_gemm_part *parts, int64_t n, int64_t 
   return tiles * 32 >= (int64_t)num_cus() * (K > 4096 ? 13 : 12);
 }
 
-// Rows of the list's tiles: three quarters of a whole one by the rule of single products (pick_algo).
-static int64_t multi_tile_rows(const l8_gemm_part *parts, int64_t n, int64_t N) {
+// Three quarters of a whole tile by the rule of single products (pick_algo).
+extern "C" int l8_gemm_multi_tile_rows(const l8_gemm_part *parts, int64_t n, int64_t N) {
   const int64_t cus = num_cus();
   int64_t whole = 0, quarters = 0;
   for (int64_t i = 0; i < n; ++i) {
@@ -2061,7 +2061,7 @@ extern "C" int l8_gemm_nt_multi(const l8_gemm_part *parts, int64_t n, const void
     return L8_OK;
   }
   constexpr int kLds = 5 * 256 * 128;
-  const int64_t bm = multi_tile_rows(parts, n, N);
+  const int64_t bm = l8_gemm_multi_tile_rows(parts, n, N);
   const gemm_fn fn = bm == 256 ? gemm_nt_stream_kernel<4, false, false, false, true> : gemm_nt_stream_kernel<4, false, false, false, true, 192, 256>;
   tile_rows = 0;
   for (int64_t i = 0; i < n; ++i) tile_rows += (parts[i].M + bm - 1) / bm;

@@ -642,11 +642,15 @@ def test_sum_of_products_on_three_quarter_tiles(Ks):
 
 
 @pytest.mark.parametrize("K", [16, 272, 1152])
-@pytest.mark.parametrize("rows", [(2000, 500, 500), (1930, 960), (200, 2400, 390)])
-def test_list_of_products_on_three_quarter_tiles(rows, K):
-    """Products with one B whose tiles of 192 rows start where the one before ends, the last tile of each short; exact integers."""
-    from lingua_amd import ops
-    N = 3600
+@pytest.mark.parametrize("rows,N,tile_rows", [((2000, 500, 500), 3600, 192), ((1930, 960), 3600, 192), ((200, 2400, 390), 3600, 256), ((200, 2400, 390), 3328, 192)])
+def test_list_of_products_on_three_quarter_tiles(rows, N, tile_rows, K):
+    """Products with one B whose tiles of 192 rows start where the one before ends, the last tile of each short, the first one
+    barely longer than a tile; and a list that these would give a second round.  Exact integers."""
+    import struct
+    from lingua_amd import _lib, ops
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        parts = struct.pack(f"{4 * len(rows)}q", *(v for m in rows for v in (0, m, 0, 0)))
+        assert _lib.load().l8_gemm_multi_pays(parts, len(rows), N, K) and _lib.load().l8_gemm_multi_tile_rows(parts, len(rows), N) == tile_rows
     g = torch.Generator().manual_seed(K)
     B = torch.randint(-1, 2, (N, K), generator=g).float().cuda()
     sb = torch.tensor([2.0 ** (i % 3) for i in range(N)]).reshape(N, 1).cuda()
