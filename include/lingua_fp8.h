@@ -338,8 +338,9 @@ int l8_gemm_nt_add(const void *A, const void *B, int64_t M, int64_t N, int64_t K
                    const float *sa, int sa_mode, const float *sb, int sb_mode, void *C, int64_t ldc, int algo, void *stream);
 
 /* C_i [M_i,N] = bf16(A_i [M_i,K] . B^T * sa_i * sb) for n products with one B: the weight gradients of linears on one
- * activation (lingua/float8.py:123 once per linear).  One launch of the 256 x 256 kernel for two or three of them where that
- * takes fewer rounds of tiles over the chip, else as n calls of l8_gemm_nt.  sa_i fp32 [M_i]; lda and ldc are those of every A_i and C_i. */
+ * activation (lingua/float8.py:123 once per linear).  One launch on tiles of 256 x 256 or 192 x 256 for two or three of them
+ * where that takes fewer rounds of tiles over the chip, else as n calls of l8_gemm_nt.  sa_i fp32 [M_i]; lda and ldc are those
+ * of every A_i and C_i. */
 typedef struct {
   const void *A;
   int64_t M;
@@ -355,7 +356,7 @@ int l8_gemm_multi_tile_rows(const l8_gemm_part *parts, int64_t n, int64_t N);
 
 /* C [M,N] = bf16(sum over i of A_i [M,K_i] . B_i [N,K_i]^T * sa_i * sb_i): the gradient of an activation that several linears
  * read (lingua/float8.py:119 once per linear, added up by autograd).  sa_i fp32 [M], sb_i one fp32.  Two or three products
- * that 256 x 256 tiles serve, none shorter than 512 and shorter than 8192 on average, run as one whose sum is rounded once,
+ * that tiles of 256 x 256 or 192 x 256 serve, none shorter than 512 and shorter than 8192 on average, run as one whose sum is rounded once,
  * but for rows whose finite scales sa_i * sb_i lie more than 2^90 apart or beyond the normal fp32 numbers; these, and all rows
  * else, as l8_gemm_nt of the first and l8_gemm_nt_add of the others, rounded per product. */
 typedef struct {

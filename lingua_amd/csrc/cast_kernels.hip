@@ -996,7 +996,8 @@ __global__ __launch_bounds__(256) void cast_transposed_kernel(const std::conditi
 // activation (column amaxes) of a linear's backward pass while each is small.  Bound by what a launch costs: us, all casts of
 // the pass, five launches / two: M = 1021 N = K = 2048 14.4 / 10.6, 256 1024 1024 10.8 / 6.9, 1000 3008 2000 19.6 / 17.7,
 // 256 8192 1024 17.3 / 14.3; and as many calls less for the host, which such a pass waits for: forward + backward of the first,
-// with a bias, 143 -> 77.
+// with a bias, 140 -> 126 (with the sums in one launch and the products' early scales; an empty autograd function takes 66 .. 72
+// of it, and where the host is at the faster of its two levels the whole pass takes 70 .. 77).
 // The first workgroups make the bias gradient, if there is one, 16 columns each (32 on 64 workgroups were the last to finish).
 // us at M = 1021 N = K = 2048: 7.5 and a launch of 5.9 for the sums / 10.0 together.
 constexpr int kMixedCols = 16;
@@ -1569,7 +1570,8 @@ static int launch_transposed(const TransposedCast *a, int n, hipStream_t st) {
 }
 
 // Up to this many partial rows a transposed cast's workgroup reads them itself (32 KB of its 64 columns from the L2, beside
-// 16 KB of its own operand) instead of waiting for a launch that folds them.
+// 16 KB of its own operand) instead of waiting for a launch that folds them: what 1024 rows leave, or 256 beyond 4096 columns
+// (rowwise_blocks).
 constexpr int64_t kMaxReadPartials = 256;
 
 static bool bwd_casts_together(int64_t M, int64_t N, int64_t K) {

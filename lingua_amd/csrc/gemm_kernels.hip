@@ -73,7 +73,7 @@ struct GemmArgs {
   uint32_t sk_epoch;  // value that marks a flag as set in THIS launch (never 0; flags are never cleared)
   int sk_wait_limit;  // polls of a flag before the waiting workgroup gives up and poisons its tile
   // MULTI kernels: products with the same B, one below the other.  A, sa, C and M above are the first one's; a further one
-  // starts at tile row first / 256 of the launch, an unused one beyond the last.
+  // starts at row `first` of the launch, a multiple of the tiles' BM, an unused one beyond the last.
   struct Part {
     const uint8_t *A;
     const float *sa;
@@ -279,8 +279,8 @@ __global__ __launch_bounds__(WM *WN *KS * 64) void gemm_nt_kernel(const GemmArgs
   // The small tiles request them in front of their panels: loads retire in order, so they are there when the K loop starts,
   // and the partial waits below count as before.  Requested behind the loop, with a branch around each load, a product of a
   // few microseconds ended in the latency of loads that wait for one another.  us, operands cold, before / now: [1021,2048].
-  // [2048,2048] with a bias 12.4 / 9.8, without 10.0 / 9.6; [32,4096].[11008,4096] 16.2 / 14.3 and 14.7 / 14.3; [128,1024].
-  // [1024,1024] without 6.0 / 5.6.  Two 128 x 128 workgroups on a unit cover for each other: there the registers are worth more
+  // [2048,2048] with a bias 12.4 / 9.6, without 9.8 / 9.3; [32,4096].[11008,4096] 16.1 / 14.1 and 14.6 / 14.1; [128,1024].
+  // [1024,1024] without 5.8 / 5.3.  Two 128 x 128 workgroups on a unit cover for each other: there the registers are worth more
   // (requested early [64,4096].[36864,4096] 46.4 -> 46.9).
   constexpr bool EARLY = DEEP;
   const int l31 = lane & 31, h = lane >> 5;

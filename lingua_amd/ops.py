@@ -480,7 +480,7 @@ def gemm_nt(qa: torch.Tensor, qb: torch.Tensor, sa: torch.Tensor, sb: torch.Tens
 
 
 def gemm_nt_multi(qas, qb: torch.Tensor, sas, sb: torch.Tensor, algo: int = 0):
-    """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch, on 256 x 256 tiles, where that fills the GPU
+    """``[gemm_nt(qa, qb, sa, sb) for qa, sa in zip(qas, sas)]`` in one launch, on large tiles, where that fills the GPU
     better (a product that alone is too small for those tiles may add up K in another order there).  fp8 operands of one
     row stride with one scale per row."""
     N, K = qb.shape
